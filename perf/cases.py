@@ -2,10 +2,11 @@
 
 Every case serves a batch of requests once: the prompts go in (in one step or in portions), then every request is continued token by
 token with tokens that are given - the replay of a trace, so that a pass does the same work and gives the same numbers every time it is
-run.  Outputs: the logits behind the prompts, the greedy tokens of every decode step, the logits of the last step, and, where the
-case samples, the sampled tokens.
+run.  Every step's greedy tokens are asked for (and, where the case samples, a sampled one), as a server does.  Outputs: the logits behind
+the prompts and those of the last step, which read everything that the steps between left in the caches and states.  The tokens are no
+outputs: the largest logits of a random model lie closer together than a rounding moves them.
 
-Sizes are those of the repository's own benchmark configurations.  Qwen3-4B / 8B run at full depth, the Qwen3.5-4B hybrid with three rounds of
+Sizes are those of the repository's own benchmark configurations.  Qwen3-4B / 8B run at full depth, the Qwen3.5-4B hybrid with two rounds of
 its layer pattern (at full depth a random hybrid turns bf16 roundings into a tenth of its logits); the other families at their benchmark's
 layer sizes with one round of their layer pattern (every kind of layer once or twice).
 
@@ -40,7 +41,7 @@ FAMILY = {
     "zofadra": (ZofadraEngine, bench_zofadra.SIZES, bench_zofadra.zofadra_config, 5),
     "sopanex": (SopanexEngine, bench_sopanex.SIZES, bench_sopanex.sopanex_config, 2),
 }
-WEIGHT_STD = 0.02
+WEIGHT_STD = {"qwen3-4b": 0.006, "qwen3-8b": 0.006, "qwen3.5-4b": 0.02}
 
 
 def _case(name, model, requests, prompt, new, size="", dtype="bfloat16", ragged=False, portion=0, sample=False):
@@ -114,7 +115,7 @@ def _config(case):
     if case["model"] in QWEN:
         cfg = dict(QWEN[case["model"]])
         if "layer_types" in cfg:
-            cfg.update(num_hidden_layers=12, layer_types=cfg["layer_types"][:12])
+            cfg.update(num_hidden_layers=8, layer_types=cfg["layer_types"][:8])
         return cfg
     _, sizes, make, layers = FAMILY[case["model"]]
     cfg = make(sizes[case["size"]])
@@ -375,7 +376,7 @@ def _checkpoint(case, seed):
         out[name] = t.view(shape)
         layer, _, expert = name.partition(".mlp.e")
         if expert and not expert.startswith("0."):
-            t.mul_(0.125).add_(out["%s.mlp.e0.%s" % (layer, expert.split(".")[1])].view(-1))
+            t.mul_(0.03125).add_(out["%s.mlp.e0.%s" % (layer, expert.split(".")[1])].view(-1))
         if case["model"] == "sopanex" and name.endswith(".correction"):
             real = cfg["layers"][0]["mlp"]["router"]["experts"]
             t[real:].fill_(-10.0)
@@ -391,10 +392,10 @@ def prepare(case, seed):
     room = sum((len(p) + new + 15) // 16 + 1 for p in prompts)
     if case["model"] == "qwen3.5-4b":
         eng = Qwen35Engine(cfg, num_kv_pages=room + 8, max_batch_size=n, max_positions=longest + new + 16)
-        eng.fill_synthetic(seed=seed, std=WEIGHT_STD)
+        eng.fill_synthetic(seed=seed, std=WEIGHT_STD[case["model"]])
     elif case["model"] in QWEN:
         eng = Qwen3Engine(cfg, num_kv_pages=room + 8, max_batch_size=8 if n <= 8 else 32, decode_mode=1, max_positions=longest + new + 16)
-        eng.fill_synthetic(seed=seed, std=WEIGHT_STD)
+        eng.fill_synthetic(seed=seed, std=WEIGHT_STD[case["model"]])
     else:
         eng = FAMILY[case["model"]][0](cfg, max_tokens=16 * room, max_requests=n, dtype=case["dtype"])
         flat, tensors = _checkpoint(case, seed)
@@ -413,28 +414,21 @@ def run(state):
     case, eng, prompts, given = state["case"], state["engine"], state["prompts"], state["given"]
     new, out = case["new"], {}
     rids = [eng.new_request() for _ in prompts]
-    tokens, sampled = [], []
     if case["model"] == "qwen3.5-4b":
-        first = [eng.prefill(r, p, want_logits=True) for r, p in zip(rids, prompts)]
-        tokens.append([t for t, _ in first])
-        out["prompt_logits"] = np.stack([lg for _, lg in first])
+        out["prompt_logits"] = np.stack([eng.prefill(r, p, want_logits=True)[1] for r, p in zip(rids, prompts)])
         for s in range(new - 1):
-            tokens.append(eng.decode(rids, given[s]))
-        tk, out["logits"] = eng.decode(rids, given[new - 1], want_logits=True)
-        tokens.append(tk)
+            eng.decode(rids, given[s])
+        out["logits"] = eng.decode(rids, given[new - 1], want_logits=True)[1]
     elif case["model"] in QWEN:
-        tk, lg = eng.prefill(rids, prompts, return_logits=True)
-        tokens.append(tk)
-        out["prompt_logits"] = _bf16(lg)
+        out["prompt_logits"] = _bf16(eng.prefill(rids, prompts, return_logits=True)[1])
         for s in range(new):
             if s == new - 1:
-                tk, lg = eng.decode(rids, given[s], return_logits=True)
-                out["logits"] = _bf16(lg)
+                out["logits"] = _bf16(eng.decode(rids, given[s], return_logits=True)[1])
             else:
-                tk = eng.decode(rids, given[s])
-            tokens.append(tk)
+                eng.decode(rids, given[s])
             if case["sample"]:
-                sampled.append([eng.sample(c, 0.8, 50, 0.95, u) for c, u in enumerate(state["uniform"][s])])
+                for c, u in enumerate(state["uniform"][s]):
+                    eng.sample(c, 0.8, 50, 0.95, u)
     else:
         portion = case["portion"] or max(map(len, prompts))
         done = [0] * len(prompts)
@@ -450,19 +444,14 @@ def run(state):
                     if done[i] == len(p):
                         last.append((i, row - 1))
             res = eng.step(entries, want=[r for _, r in last], logits=bool(last), tokens=bool(last))
-            for (i, _), lg, tk in zip(last, *(res or ((), ()))):
-                ends[i] = (lg, tk)
-        out["prompt_logits"] = np.stack([ends[i][0] for i in range(len(prompts))])
-        tokens.append([ends[i][1] for i in range(len(prompts))])
+            for (i, _), lg in zip(last, res[0] if last else ()):
+                ends[i] = lg
+        out["prompt_logits"] = np.stack([ends[i] for i in range(len(prompts))])
         for s in range(new - 1):
-            tokens.append(eng.step([(r, [t]) for r, t in zip(rids, given[s])], logits=False, tokens=True))
-        out["logits"], tk = eng.step([(r, [t]) for r, t in zip(rids, given[new - 1])], logits=True, tokens=True)
-        tokens.append(tk)
+            eng.step([(r, [t]) for r, t in zip(rids, given[s])], logits=False, tokens=True)
+        out["logits"] = eng.step([(r, [t]) for r, t in zip(rids, given[new - 1])], logits=True, tokens=True)[0]
     for r in rids:
         eng.drop_request(r)
-    out["tokens"] = np.asarray(tokens, dtype=np.int32)
-    if case["sample"]:
-        out["sampled"] = np.asarray(sampled, dtype=np.int32)
     return out
 
 
@@ -560,19 +549,15 @@ def work(case):
     return {"bytes": nbytes, "flops": flops}
 
 
-# about four times the error of the logits against `exact`, the largest of the listed cases and of a hundred drawn ones: values in bf16 along
-# 36 layers (12 hybrid ones) or 2 .. 5 layers; a router's near tie that a rounding turns moves a whole row (duguzen, ramalix, sopanex)
-REL = {"qwen3-4b": 0.18, "qwen3-8b": 0.24, "qwen3.5-4b": 0.24, "duguzen": 0.06, "feruzen": 0.03, "ramalix": 0.1, "kukulorn": 0.036,
-       "zofadra": 0.06, "sopanex": 0.04}
+# four times the error of the logits against `exact`, the largest of the listed cases and of a hundred drawn ones, and no more than three
+# hundredths: values in bf16 along 36 layers (8 hybrid ones) or 2 .. 5 layers; a router's near tie that a rounding turns moves a whole row
+# (duguzen, ramalix, sopanex)
+REL = {"qwen3-4b": 0.03, "qwen3-8b": 0.03, "qwen3.5-4b": 0.03, "duguzen": 0.03, "feruzen": 0.026, "ramalix": 0.03, "kukulorn": 0.03,
+       "zofadra": 0.03, "sopanex": 0.03}
 
 
 def tolerance(case):
-    """differ: greedy (and sampled) tokens of a random model, whose largest logits lie close together - within the rounding of the bf16 row
-    that the choice is made from - so that a quarter of them turn in the deepest model; few tokens make coarse shares."""
-    turns = 2.0 / ((case["new"] + 1) * case["requests"])
-    if case["dtype"] == "float32":
-        return {"rel": 2e-5, "differ": min(0.9, 0.05 + turns)}
-    return {"rel": REL[case["model"]], "differ": min(0.9, 0.25 + turns)}
+    return {"rel": 2e-5 if case["dtype"] == "float32" else REL[case["model"]]}
 
 
 # ------------------------------------------------------------------ the same numbers in 64 bits, plain torch
@@ -597,11 +582,12 @@ def _synthetic(index, seed, std, mean, single=False):
 class _SyntheticWeights:
     """tensors of a seeded Qwen engine, drawn in the engine's order"""
 
-    def __init__(self, seed):
-        self.base, self.count = seed * 1000003, 0
+    def __init__(self, seed, std):
+        self.base, self.count, self.std = seed * 1000003, 0, std
 
-    def next(self, rows, cols=1, std=WEIGHT_STD, mean=0.0, single=False):
+    def next(self, rows, cols=1, std=None, mean=0.0, single=False):
         self.count += 1
+        std = self.std if std is None else std
         return functools.partial(self._values, self.base + self.count, rows, cols, std, mean, single)
 
     @staticmethod
@@ -687,10 +673,10 @@ def _spread(x, heads):
     return x.repeat_interleave(heads // x.shape[1], 1)
 
 
-def _exact_qwen3(cfg, seed, seqs):
+def _exact_qwen3(cfg, seed, std, seqs):
     H, I, L, V, hd = (cfg[k] for k in ("hidden_size", "intermediate_size", "num_hidden_layers", "vocab_size", "head_dim"))
     Hq, G, eps = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["rms_norm_eps"]
-    w = _SyntheticWeights(seed)
+    w = _SyntheticWeights(seed, std)
     embed = w.next(V, H)
     head = embed if cfg["tie_word_embeddings"] else w.next(V, H)
     final = w.next(H, std=0.1, mean=1.0)()
@@ -714,12 +700,12 @@ def _exact_qwen3(cfg, seed, seqs):
     return (_rms(x, eps) * final).split(lens), lambda rows: rows @ head().T
 
 
-def _exact_qwen35(cfg, seed, seqs):
+def _exact_qwen35(cfg, seed, std, seqs):
     H, I, V, hd = (cfg[k] for k in ("hidden_size", "intermediate_size", "vocab_size", "head_dim"))
     Hq, G, eps = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["rms_norm_eps"]
     kh, vh, taps = cfg["linear_num_key_heads"], cfg["linear_num_value_heads"], cfg["linear_conv_kernel_dim"]
     C, Z = (2 * kh + vh) * 128, vh * 128
-    w = _SyntheticWeights(seed)
+    w = _SyntheticWeights(seed, std)
     embed = w.next(V, H)
     final = w.next(H, std=0.1)()
     freqs = _frequencies(int(hd * cfg["partial_rotary_factor"]), cfg["rope_theta"])
@@ -1065,7 +1051,7 @@ def exact(case, seed):
     prompts, given, _ = _tokens(case, seed)
     seqs = [p + [row[i] for row in given] for i, p in enumerate(prompts)]
     if case["model"] in QWEN:
-        rows, head = (_exact_qwen35 if case["model"] == "qwen3.5-4b" else _exact_qwen3)(cfg, seed, seqs)
+        rows, head = (_exact_qwen35 if case["model"] == "qwen3.5-4b" else _exact_qwen3)(cfg, seed, WEIGHT_STD[case["model"]], seqs)
     else:
         flat, tensors = _checkpoint(case, seed)
         w = _Named(tensors)
@@ -1076,10 +1062,7 @@ def exact(case, seed):
         def head(r):
             lg = w.lin(r, done[0][1])
             return cap * torch.tanh(lg / cap) if cap else lg
-    # rows that were asked for: the end of the prompt and every continued token
-    lg = head(torch.cat([r[len(p) - 1:] for r, p in zip(rows, prompts)])).view(len(seqs), case["new"] + 1, -1)
-    out = {"prompt_logits": lg[:, 0].cpu().numpy(), "logits": lg[:, -1].cpu().numpy(),
-           "tokens": lg.argmax(-1).T.to(torch.int32).cpu().numpy()}
-    if case["sample"]:
-        out["sampled"] = None
-    return out
+    # rows that were asked for: the end of the prompt and the last continued token
+    at_prompt = head(torch.stack([r[len(p) - 1] for r, p in zip(rows, prompts)]))
+    at_end = head(torch.stack([r[-1] for r in rows]))
+    return {"prompt_logits": at_prompt.cpu().numpy(), "logits": at_end.cpu().numpy()}
