@@ -51,9 +51,10 @@ pegainfer_status_t pegainfer_silu_mul_rows(const void* gate_up, void* out, int32
  * Grouped form: a device-side table of row tiles, each of <= 64 (or 128: tile_rows_cap) consecutive POSITIONS of a sorted list that belong to
  * one group (expert); positions map to x / y rows through x_row_index / y_row_index (NULL = identity).  Tiles beyond
  * *n_tiles exit; the grid is max_tiles wide.
- * Three kernels behind one entry: an fp32-FMA tile kernel (any sizes and strides, both storage types), a matrix-core tile
- * kernel (bf16 weights with contiguous k in 16-byte chunks; an fp32 x is rounded to bf16 as it is staged) and a few-rows
- * form that streams the weights once (<= 8 rows per tile: decode).  In each the k order of an output is fixed, so a row's
+ * Kernels behind one entry: an fp32-FMA tile kernel (any sizes and strides, both storage types), a matrix-core tile
+ * kernel (bf16 weights with contiguous k in 16-byte chunks; an fp32 x is rounded to bf16 as it is staged) and two few-rows
+ * forms that stream the weights once (decode): bf16 weights on the matrix cores (<= 16 rows per tile; an fp32 x enters in three exact
+ * parts), fp32 weights by FMA (<= 8 rows).  In each the k order of an output is fixed, so a row's
  * result does not depend on what else is in the launch; which kernel runs depends on the launch's shape. */
 enum { PEGAINFER_EPI_NONE = 0, PEGAINFER_EPI_RELU_SQ = 1, PEGAINFER_EPI_SIGMOID_GATE = 2, PEGAINFER_EPI_GELU_ERF = 3 };
 typedef struct {

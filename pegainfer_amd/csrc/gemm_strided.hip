@@ -225,7 +225,7 @@ static void mfma_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   else gemm_strided_mfma_kernel<TX, TY, TG, 64><<<grid, 256, 0, s>>>(d);
 }
 
-// ------------------------------------------------------------------ few-rows form (decode)
+// ------------------------------------------------------------------ few-rows form (decode), fp32 weights or one fp32 row
 // At most R rows per tile (a decode step's tokens, or the pairs one expert received): the weights are streamed once with
 // 16-byte loads, the rows wait in LDS as fp32 (2048 k values at a time), a wave owns one output at a time (lanes over k, butterfly sum), 32 outputs per
 // workgroup - or 8 (OUT) when 32 would leave most of the chip without a workgroup (a matrix of a few thousand outputs).  fp32
@@ -354,6 +354,192 @@ static void rows_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   else kern<<<grid, 256, lds, s>>>(d);
 }
 
+// ------------------------------------------------------------------ few-rows form on the matrix cores (bf16 weights, decode)
+// At most 16 rows per tile; bound by the stream of weights.  A wave takes OB blocks of 16 outputs, wk waves share a block's K (wave
+// j the 64-wide pieces j, j + wk, ... of k; wk follows from K alone), their partial sums meet in LDS in wave order: an output's k order is
+// fixed by K.  One load instruction covers 8 outputs x 128 bytes: lane = output (lane >> 1) & 7, 16-byte chunk 2 (lane >> 4) + (lane & 1).
+// Taken unpermuted as an A operand, row 2 r + h holds output r's chunks of parity h, so the product with the x chunks of parity h is
+// right in the rows of that parity and discarded in the others (the same layout as gemm_skinny.h).  x comes straight from memory - a tile's
+// rows are few and stay in the caches - a chunk of pieces ahead, as the weights do: 16 KB of weights in flight per wave.
+// fp32 rows enter as three bf16 parts of 8 bits each, cut off rather than rounded: their sum IS the value, every product is exact
+// and the sums stay in fp32.
+// Against the FMA form (eight rows in LDS, four weight loads in flight per wave): 17 experts of 2048 x 2048 with 24 pairs 51 -> 15.6 us
+// (4.6 TB/s) up and, with the output matrix of 65 536 x 2048 and 8 rows among them, 79 -> 26 us on average; 32 768 x 1024 with 8 fp32
+// rows 61 -> 18.7 us; 4 experts of 2048 x 2560 and one row each 15.1 -> 13.4 us.
+__device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, bf16x8_t (&o)[3]) {
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t part[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t hi[2], mid[2], lo[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float x = v[2 * i + e];
+      hi[e] = __builtin_bit_cast(uint32_t, x) & 0xFFFF0000u;
+      // an infinity has no remainder (x - x would be NaN)
+      const float r1 = (hi[e] & 0x7FFFFFFFu) == 0x7F800000u ? 0.f : x - __builtin_bit_cast(float, hi[e]);
+      mid[e] = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+      lo[e] = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, mid[e]));
+    }
+    part[0][i] = (hi[0] >> 16) | hi[1];
+    part[1][i] = (mid[0] >> 16) | mid[1];
+    part[2][i] = (lo[0] >> 16) | (lo[1] & 0xFFFF0000u);
+  }
+#pragma unroll
+  for (int s = 0; s < 3; ++s) o[s] = __builtin_bit_cast(bf16x8_t, u32x4{part[s][0], part[s][1], part[s][2], part[s][3]});
+}
+
+// 8 values of x as they are fetched, and as operands
+template <typename TX>
+struct RowPiece;
+template <>
+struct RowPiece<uint16_t> {
+  static constexpr int kParts = 1;
+  u32x4 v;
+  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const u32x4*>(p); }
+  __device__ __forceinline__ void zero() { v = u32x4{0u, 0u, 0u, 0u}; }
+  __device__ __forceinline__ void parts(bf16x8_t (&o)[1]) const { o[0] = __builtin_bit_cast(bf16x8_t, v); }
+};
+template <>
+struct RowPiece<float> {
+  static constexpr int kParts = 3;
+  f32x4 a, b;
+  __device__ __forceinline__ void load(const float* p) { a = *reinterpret_cast<const f32x4*>(p); b = *reinterpret_cast<const f32x4*>(p + 4); }
+  __device__ __forceinline__ void zero() { a = f32x4{0.f, 0.f, 0.f, 0.f}; b = a; }
+  __device__ __forceinline__ void parts(bf16x8_t (&o)[3]) const { split3(a, b, o); }
+};
+
+constexpr int kRowsMax = 16;   // token rows of a tile of the matrix-core few-rows form
+
+template <typename TX, typename TY, typename TG, int OB>
+__global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc d, int wk) {
+  constexpr int CH = OB == 1 && sizeof(TX) == 2 ? 4 : 2;      // 64-wide pieces per register set
+  constexpr int NP = RowPiece<TX>::kParts;
+  __shared__ f32x4 red[4][OB][64];
+  int g, row0, nrows;
+  if (d.tile_group) {
+    if ((int)blockIdx.x >= *d.n_tiles) return;
+    g = d.tile_group[blockIdx.x];
+    row0 = d.tile_row0[blockIdx.x];
+    nrows = min(kRowsMax, d.tile_rows[blockIdx.x]);
+  } else {
+    g = blockIdx.z;
+    row0 = blockIdx.x * kRowsMax;
+    nrows = min(kRowsMax, d.rows - row0);
+  }
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
+  const int per_wg = 4 / wk * OB * 16;                        // outputs of a workgroup
+  const int blk = wave / wk, ks = wave - blk * wk;
+  const int m0 = blockIdx.y * per_wg + blk * OB * 16;
+  const TX* X = static_cast<const TX*>(d.x) + (int64_t)g * d.x_group_stride;
+  const uint16_t* W = static_cast<const uint16_t*>(d.w) + (int64_t)g * d.w_group_stride;
+  const int tok = row0 + min(l15, nrows - 1);                 // absent rows repeat the last one; they are never stored
+  const TX* xp = X + (int64_t)(d.x_row_index ? d.x_row_index[tok] : tok) * d.x_row_stride + gq * 16;
+  const int pchunk = 2 * gq + (lane & 1);
+  const uint16_t* wp[OB][2];
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      wp[o][h] = W + (int64_t)min(m0 + o * 16 + h * 8 + ((lane >> 1) & 7), d.m - 1) * d.w_m_stride + pchunk * 8;
+  const int K = d.k, np = (K + 63) >> 6, mine = ks < np ? (np - ks + wk - 1) / wk : 0;   // pieces of k; those of this wave
+  f32x4 acc[OB][2][2];
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[o][q >> 1][q & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Set { RowPiece<TX> x[CH][2]; u32x4 w[CH][OB][2]; } A, B;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  auto issue = [&](int i0, Set& s) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (i0 + c >= mine) continue;
+      const int k = (ks + (i0 + c) * wk) * 64;
+      if (k + 64 <= K) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) s.x[c][h].load(xp + k + h * 8);
+#pragma unroll
+        for (int o = 0; o < OB; ++o)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) s.w[c][o][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[o][h] + k));
+      } else {                                                // the last piece of a K that is no multiple of 64 (it is one of 8)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (k + gq * 16 + h * 8 < K) s.x[c][h].load(xp + k + h * 8);
+          else s.x[c][h].zero();
+        }
+#pragma unroll
+        for (int o = 0; o < OB; ++o)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) s.w[c][o][h] = k + pchunk * 8 < K ? *reinterpret_cast<const u32x4*>(wp[o][h] + k) : zero;
+      }
+    }
+  };
+  auto compute = [&](int i0, const Set& s) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (i0 + c >= mine) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        bf16x8_t xf[NP];
+        s.x[c][h].parts(xf);
+#pragma unroll
+        for (int q = NP - 1; q >= 0; --q)                     // the smallest part first
+#pragma unroll
+          for (int o = 0; o < OB; ++o)
+#pragma unroll
+            for (int rh = 0; rh < 2; ++rh)
+              acc[o][rh][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, s.w[c][o][rh]), xf[q], acc[o][rh][h], 0, 0, 0);
+      }
+    }
+  };
+  issue(0, A);
+  if (CH < mine) issue(CH, B);
+  for (int i0 = 0; i0 < mine; i0 += 2 * CH) {
+    compute(i0, A);
+    if (i0 + 2 * CH < mine) issue(i0 + 2 * CH, A);
+    if (i0 + CH >= mine) break;
+    compute(i0 + CH, B);
+    if (i0 + 3 * CH < mine) issue(i0 + 3 * CH, B);
+  }
+  // slot i of lane ln: output (i >> 1) * 8 + 2 (ln >> 4) + (i & 1) of the block, row ln & 15
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+    red[wave][o][lane] = f32x4{acc[o][0][0][0] + acc[o][0][1][1], acc[o][0][0][2] + acc[o][0][1][3],
+                               acc[o][1][0][0] + acc[o][1][1][1], acc[o][1][0][2] + acc[o][1][1][3]};
+  __syncthreads();
+  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
+  const float* part = reinterpret_cast<const float*>(red);
+  for (int e = tid; e < per_wg * 16; e += 256) {              // consecutive threads: consecutive outputs of one row
+    const int out = e % per_wg, r = e / per_wg;
+    const int m = blockIdx.y * per_wg + out;
+    if (r >= nrows || m >= d.m) continue;
+    const int b = out / (OB * 16), o = (out >> 4) % OB, j = out & 15;
+    const int at = (o * 64 + ((j & 7) >> 1) * 16 + r) * 4 + (j >> 3) * 2 + (j & 1);
+    float v = part[b * wk * OB * 256 + at];
+    for (int w = 1; w < wk; ++w) v += part[(b * wk + w) * OB * 256 + at];
+    const int p = row0 + r;
+    if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+    else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
+    else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
+      v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)(d.x_row_index ? d.x_row_index[p] : p) * d.gate_row_stride + g));
+    st(Y + (int64_t)(d.y_row_index ? d.y_row_index[p] : p) * d.y_row_stride + m, v);
+  }
+}
+
+template <typename TX, typename TY, typename TG>
+static void rows_mfma_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
+  const int np = ceil_div(d.k, 64), wk = np >= 8 ? 4 : np >= 4 ? 2 : 1;
+  // the tiles that a table's bound allows for and that are empty come last: an even grid width would send the others' workgroups, in
+  // their round robin over the XCDs, to some of the eight only
+  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, kRowsMax), groups = d.tile_group ? 1 : d.groups;
+  const int blocks = ceil_div(d.m, 16 * (4 / wk));
+  // two blocks of outputs per wave (each x piece used twice) where that still gives every compute unit two workgroups
+  const bool two = (long)row_tiles * groups * blocks >= 4L * device_cus();
+  if (two) gemm_rows_mfma_kernel<TX, TY, TG, 2><<<dim3(row_tiles, ceil_div(blocks, 2), groups), 256, 0, s>>>(d, wk);
+  else gemm_rows_mfma_kernel<TX, TY, TG, 1><<<dim3(row_tiles, blocks, groups), 256, 0, s>>>(d, wk);
+}
+
 static inline bool chunks_ok(const pegainfer_gemm_desc& d) {
   auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   return d.w_k_stride == 1 && (d.k & 7) == 0 && (d.x_row_stride & 7) == 0 && (d.x_group_stride & 7) == 0 &&
@@ -365,13 +551,25 @@ static bool gemm_strided_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   dim3 grid(d.tile_group ? d.max_tiles : ceil_div(d.rows, GT), ceil_div(d.m, GM), d.tile_group ? 1 : d.groups);
   const bool gate32 = d.gate_dtype == kDtF32;
   if (!d.plain && chunks_ok(d)) {
-    // few rows per tile: stream the weights once (both storage types, fp32 arithmetic)
+    // few rows per tile: stream the weights once
     const int tr = d.tile_group ? (d.max_tile_rows > 0 ? d.max_tile_rows : (d.tile_rows_cap > 0 ? d.tile_rows_cap : GT)) : d.rows;
+    if constexpr (std::is_same<TW, uint16_t>::value) {
+      // one fp32 row stays on the FMA form: splitting it costs more than the matrix cores give (a 65 536 x 2048 matrix: 49 us against 57)
+      if (tr <= kRowsMax && !(tr == 1 && std::is_same<TX, float>::value)) {
+        if (gate32) rows_mfma_launch<TX, TY, float>(d, s);
+        else rows_mfma_launch<TX, TY, uint16_t>(d, s);
+        return true;
+      }
+    }
+    constexpr bool kWide = std::is_same<TW, float>::value;    // bf16 weights reach the FMA form with one row only
     const int R = tr <= 1 ? 1 : tr <= 4 ? 4 : tr <= 8 ? 8 : 0;
     if (R && (size_t)R * d.k * sizeof(float) <= 150 * 1024) {
-      if (gate32) { if (R == 1) rows_form_launch<TX, TW, TY, float, 1>(d, s); else if (R == 4) rows_form_launch<TX, TW, TY, float, 4>(d, s); else rows_form_launch<TX, TW, TY, float, 8>(d, s); }
-      else { if (R == 1) rows_form_launch<TX, TW, TY, uint16_t, 1>(d, s); else if (R == 4) rows_form_launch<TX, TW, TY, uint16_t, 4>(d, s); else rows_form_launch<TX, TW, TY, uint16_t, 8>(d, s); }
-      return true;
+      if (R == 1) { if (gate32) rows_form_launch<TX, TW, TY, float, 1>(d, s); else rows_form_launch<TX, TW, TY, uint16_t, 1>(d, s); return true; }
+      if constexpr (kWide) {
+        if (gate32) { if (R == 4) rows_form_launch<TX, TW, TY, float, 4>(d, s); else rows_form_launch<TX, TW, TY, float, 8>(d, s); }
+        else { if (R == 4) rows_form_launch<TX, TW, TY, uint16_t, 4>(d, s); else rows_form_launch<TX, TW, TY, uint16_t, 8>(d, s); }
+        return true;
+      }
     }
     if constexpr (std::is_same<TW, uint16_t>::value) {   // bf16 weights: the matrix cores
       if (gate32) mfma_form_launch<TX, TY, float>(d, s);

@@ -1071,7 +1071,8 @@ struct Model {
     d.m = 2 * ff; d.k = D;
     d.x_row_stride = D; d.w_m_stride = D; d.w_k_stride = 1; d.w_group_stride = (int64_t)2 * ff * D;
     d.y_row_stride = 2 * ff;
-    d.tile_group = t_group; d.tile_row0 = t_row0; d.tile_rows = t_rows; d.n_tiles = n_tiles; d.max_tiles = (P + per_tile - 1) / per_tile + f.experts;
+    d.tile_group = t_group; d.tile_row0 = t_row0; d.tile_rows = t_rows; d.n_tiles = n_tiles;
+    d.max_tiles = std::min(P, (P + per_tile - 1) / per_tile + f.experts);   // every tile holds a pair
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
     d.max_tile_rows = std::min(T, 64);   // a row chooses distinct experts: an expert never gets more pairs than there are rows

@@ -349,6 +349,32 @@ def test_strided_gemm_forms_agree(dtype):
     assert (outs[0].double() - ref).abs().max() < 1e-4 and (outs[1].double() - ref).abs().max() < 1e-4
 
 
+@pytest.mark.parametrize("x_type", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,M,K", [(1, 16, 8), (2, 33, 72), (3, 48, 200), (16, 17, 256), (5, 100, 520), (15, 64, 512), (9, 31, 2056),
+                                   (8, 40000, 64), (16, 20011, 136), (17, 40, 64)])
+def test_few_rows_on_the_matrix_cores(T, M, K, x_type):
+    """Row counts up to the form's sixteen and the first beyond, outputs that are no multiple of a block of 16, k that ends inside a piece of 64,
+    one, two and four waves per block, one and two blocks per wave.  Products are exact (an fp32 x is not rounded: parts of it sum to it), so
+    the error is that of fp32 sums: half an ulp of the running sum per addition, at most K / 2 of them in a row."""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(T * 1000 + K)
+    x, w = torch.randn(T, K, generator=g), C.bf16_round(torch.randn(M, K, generator=g))
+    x[0, :4] *= 2.0 ** 60                       # far apart: the small parts must not reach the large row's neighbours
+    if x_type == torch.bfloat16 or T > 16:      # the tile form that takes over beyond 16 rows rounds an fp32 x
+        x = C.bf16_round(x)
+    got = B.linear(x.to(x_type).cuda(), w.bfloat16().cuda(), out_dtype=torch.float32).cpu().double()
+    scale = x.double().abs() @ w.double().abs().T
+    assert ((got - x.double() @ w.double().T).abs() <= (K / 2 + 16) * 2.0 ** -24 * scale).all()
+
+
+def test_few_rows_keep_infinities():
+    from pegainfer_amd import ops_blocks as B
+    x, w = torch.ones(3, 64), torch.ones(16, 64)
+    x[0, 5], x[1, 7], x[2, 9] = float("inf"), float("nan"), 3.4e38
+    got = B.linear(x.cuda(), w.bfloat16().cuda(), out_dtype=torch.float32).cpu()
+    assert torch.isinf(got[0]).all() and torch.isnan(got[1]).all() and torch.isfinite(got[2]).all()
+
+
 def test_grouped_gemm_over_128_row_tiles():
     from pegainfer_amd import ops_blocks as B
     g = torch.Generator().manual_seed(11)
