@@ -367,6 +367,35 @@ def test_few_rows_on_the_matrix_cores(T, M, K, x_type):
     assert ((got - x.double() @ w.double().T).abs() <= (K / 2 + 16) * 2.0 ** -24 * scale).all()
 
 
+@pytest.mark.parametrize("T,M,K", [(9, 1, 8), (32, 64, 64), (33, 63, 72), (64, 65, 136), (65, 17, 1032), (130, 4200, 64), (4200, 130, 40)])
+def test_fp32_tiles_on_the_matrix_cores(T, M, K):
+    """32- and 64-row tiles, rows and outputs that end inside a tile, k that ends inside a slice of 64; fp32 products and sums: at most K / 4
+    additions of four products each in a row, half an ulp of the running sum per addition and product."""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(T + M + K)
+    x, w = torch.randn(T, K, generator=g), torch.randn(M, K, generator=g)
+    got = B.linear(x.cuda(), w.cuda(), out_dtype=torch.float32).cpu().double()
+    bound = (K + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((got - x.double() @ w.double().T).abs() <= bound).all()
+
+
+def test_fp32_tiles_over_a_tile_table():
+    """gathered rows, a table whose last tile of an expert is partly filled, outputs scattered by pair"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(5)
+    rows, top, E, d, ff = 150, 2, 3, 72, 100
+    expert = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(rows)]).int()
+    pos_pair, pos_row, tg, t0, tr, nt, max_tiles = B.route_sort(expert.cuda(), E)
+    x, w = torch.randn(rows, d, generator=g), torch.randn(E, ff, d, generator=g)
+    xd, wd, y = x.cuda(), w.cuda(), torch.zeros(rows * top, ff, device="cuda")
+    B.gemm_strided(B.GemmDesc(x=xd.data_ptr(), w=wd.data_ptr(), y=y.data_ptr(), x_dtype=1, w_dtype=1, y_dtype=1, m=ff, k=d, x_row_stride=d,
+                              w_m_stride=d, w_k_stride=1, w_group_stride=ff * d, y_row_stride=ff, tile_group=tg.data_ptr(),
+                              tile_row0=t0.data_ptr(), tile_rows=tr.data_ptr(), n_tiles=nt.data_ptr(), max_tiles=max_tiles,
+                              x_row_index=pos_row.data_ptr(), y_row_index=pos_pair.data_ptr()))
+    ref = torch.bmm(x.double().repeat_interleave(top, 0)[:, None], w.double()[expert.reshape(-1).long()].transpose(1, 2).contiguous())[:, 0]
+    assert (y.cpu().double() - ref).abs().max() < (d + 8) * 2.0 ** -24 * d * 16
+
+
 def test_few_rows_keep_infinities():
     from pegainfer_amd import ops_blocks as B
     x, w = torch.ones(3, 64), torch.ones(16, 64)
