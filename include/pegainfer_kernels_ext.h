@@ -160,6 +160,9 @@ void pegainfer_debug_streamk(int32_t on);
 // call (the value heads of a key head meet there to shift the shared q / k conv windows once; the words reset themselves), may be
 // shared by every layer and request of one stream.
 int32_t pegainfer_linear_attn_decode_fused(const Half* x_qkv, const Half* conv_weight, Half* conv_state, const Half* b_proj, const Half* a_proj, const Half* dt_bias, const float* A_log, float* state, const float* norm_weight, const Half* gate, Half* out, int32_t num_key_heads, int32_t num_value_heads, int32_t key_dim, int32_t val_dim, int32_t kernel_size, float eps, int32_t* tickets, pegainfer_stream_t stream);
+// The same for a batch of requests in one launch (16 at a time): request i's rows lie i strides (elements) behind the first one's, its conv
+// windows and state are conv_state[i] and state[i] (host arrays of device pointers, read during the call); tickets: batch_size x num_key_heads.
+int32_t pegainfer_linear_attn_decode_fused_batch(const Half* x_qkv, int64_t x_stride, const Half* conv_weight, Half* const* conv_state, const Half* b_proj, const Half* a_proj, int64_t ba_stride, const Half* dt_bias, const float* A_log, float* const* state, const float* norm_weight, const Half* gate, int64_t gate_stride, Half* out, int64_t out_stride, int32_t batch_size, int32_t num_key_heads, int32_t num_value_heads, int32_t key_dim, int32_t val_dim, int32_t kernel_size, float eps, int32_t* tickets, pegainfer_stream_t stream);
 
 /* Partition-KV decode attention at head_dim 256 (Qwen3.5 full-attention layers).  No counterpart in ffi.rs (its
  * hd256 decode symbol is non-partition only, ffi.rs:1286-1306); arguments and scratch contract are exactly those of

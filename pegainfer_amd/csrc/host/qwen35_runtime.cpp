@@ -100,7 +100,7 @@ struct Model35 {
        *q_attn = nullptr, *k_attn = nullptr, *v_attn = nullptr, *attn_out = nullptr, *qkv = nullptr,
        *qkv_conv = nullptr, *z = nullptr, *b_proj = nullptr, *a_proj = nullptr, *gdr_out = nullptr,
        *normed_gated = nullptr, *gate_out = nullptr, *up_out = nullptr, *act_out = nullptr, *mlp_out = nullptr,
-       *logits = nullptr, *wide = nullptr;  // wide: one token's stacked projection output (fused path)
+       *logits = nullptr, *wide = nullptr;  // wide: stacked projection outputs of up to kFusedBatch tokens (fused path)
   int32_t* tokens_out_d = nullptr;
   uint8_t* top1_state = nullptr;
   int32_t* tokens_out_host = nullptr;
@@ -119,7 +119,8 @@ struct Model35 {
   Half* split_tmp_v = nullptr;
   float* split_tmp_s = nullptr;
   int32_t* merge_ctr = nullptr;  // in-launch split-KV merge tickets, zeroed at the head of every step
-  int32_t* lin_ticket = nullptr; // pegainfer_linear_attn_decode_fused: one self-resetting word per key head (zero at allocation)
+  static constexpr int kFusedBatch = 2;   // decode batches whose projections the fused GEMVs take with the unfused calls' bits
+  int32_t* lin_ticket = nullptr; // pegainfer_linear_attn_decode_fused*: one self-resetting word per request and key head (zero at allocation)
   hipGraphExec_t graph = nullptr;
   std::vector<int> graph_ids;   // request ids of the captured step, then the attention path
   std::vector<std::pair<std::vector<int>, hipGraphExec_t>> graph_cache;   // parked execs of other keys (<= 8)
@@ -235,9 +236,9 @@ struct Model35 {
         dalloc(&mlp_out, bs * H) || dalloc(&logits, bs * (size_t)V) ||
         dalloc(&top1_state, bs * 16) || dalloc(&start_pos_d, 1) || dalloc(&probs_scratch, (size_t)V) || dalloc(&top1_value, 1) ||
         dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1) ||
-        dalloc(&wide, (size_t)std::max(C + Z + 2 * vh, 2 * q_dim + 2 * kv_dim)) ||
+        dalloc(&wide, (size_t)kFusedBatch * std::max(C + Z + 2 * vh, 2 * q_dim + 2 * kv_dim)) ||
         dalloc(&split_tmp_v, bs * pq::kSplitMaxChunksPerRequest * q_dim) ||
-        dalloc(&split_tmp_s, bs * pq::kSplitMaxChunksPerRequest * Hq) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&lin_ticket, (size_t)kh) || dalloc(&pf_last, H) ||
+        dalloc(&split_tmp_s, bs * pq::kSplitMaxChunksPerRequest * Hq) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&lin_ticket, bs * (size_t)kh) || dalloc(&pf_last, H) ||
         dalloc(&pf_last_normed, H) || dalloc(&pf_logits, V))
       return -1;
     auto al = [](size_t x) { return (x + 63) & ~size_t(63); };
@@ -575,13 +576,15 @@ struct Model35 {
         G(ly.in_b, normed, b_proj, vh, bs, H);
         G(ly.in_a, normed, a_proj, vh, bs, H);
         // per slot (batch_decode.rs:315-345); the reference copies each column out and back, the kernels take
-        // the column pointers directly - same kernels, same bits
-        for (int i = 0; i < bs; ++i) {
-          conv1d_prefill_cuda(qkv + (size_t)i * C, ly.conv_w, rs[i]->conv[lin], qkv_conv + (size_t)i * C, C, 1, convK, S());
-          gated_delta_rule_decode_cuda(qkv_conv + (size_t)i * C, b_proj + (size_t)i * vh, a_proj + (size_t)i * vh,
-                                       ly.dt_bias, ly.a_log, rs[i]->state[lin], gdr_out + (size_t)i * Z, kh, vh, LK, LK, S());
+        // the column pointers directly - same kernels, same bits.  decode_mode 1: the slots' three calls in one launch, same bits
+        if (decode_mode != 1 || !linattn_fused || linattn(ly, rs, lin, bs, qkv, C, b_proj, a_proj, vh, z, Z)) {
+          for (int i = 0; i < bs; ++i) {
+            conv1d_prefill_cuda(qkv + (size_t)i * C, ly.conv_w, rs[i]->conv[lin], qkv_conv + (size_t)i * C, C, 1, convK, S());
+            gated_delta_rule_decode_cuda(qkv_conv + (size_t)i * C, b_proj + (size_t)i * vh, a_proj + (size_t)i * vh,
+                                         ly.dt_bias, ly.a_log, rs[i]->state[lin], gdr_out + (size_t)i * Z, kh, vh, LK, LK, S());
+          }
+          rms_norm_gated_cuda(gdr_out, ly.norm_w, z, normed_gated, bs * vh, LK, eps, S());
         }
-        rms_norm_gated_cuda(gdr_out, ly.norm_w, z, normed_gated, bs * vh, LK, eps, S());
         G(ly.out_proj, normed_gated, attn_res, H, bs, Z);
         ++lin;
       }
@@ -597,16 +600,28 @@ struct Model35 {
     return 0;
   }
 
-  // bs == 1 fused step (decode_mode 1): 8-10 launches per layer instead of 16-17, every result bit-identical to
+  // conv step + gated delta rule + gated norm of every slot in one launch (csrc/qwen35.hip); != 0: a shape that the kernel does not take,
+  // nothing was launched
+  int linattn(const Layer35& ly, const std::vector<Request35*>& rs, int lin, int bs, const Half* x, int64_t x_stride, const Half* b,
+              const Half* a, int64_t ba_stride, const Half* gate, int64_t gate_stride) {
+    std::vector<Half*> conv(bs);
+    std::vector<float*> state(bs);
+    for (int i = 0; i < bs; ++i) { conv[i] = rs[i]->conv[lin]; state[i] = rs[i]->state[lin]; }
+    return pegainfer_linear_attn_decode_fused_batch(x, x_stride, ly.conv_w, conv.data(), b, a, ba_stride, ly.dt_bias, ly.a_log, state.data(),
+                                                    ly.norm_w, gate, gate_stride, normed_gated, Z, bs, kh, vh, LK, LK, convK, eps, lin_ticket, S());
+  }
+
+  // Fused step of one or two requests (decode_mode 1): 5 launches per linear-attention layer instead of 16-18, every result bit-identical to
   // decode_kernels().  The two norms and both residual adds ride in GEMV prologues (pegainfer_gemv_fused_ex with the
   // Qwen3.5 rounding points), SwiGLU in the gate|up GEMV epilogue, and the stacked qkv|z|b|a / q|k|v / gate|up
-  // weights are streamed by one GEMV each.  Batches > 1 use the reference-order path (the consumers of the
-  // stacked outputs take contiguous [bs, dim] tensors in the reference ABI).
-  int decode_kernels_fused1(Request35* r, bool split) {
+  // weights are streamed by one GEMV each (two requests: q, k and v of a full-attention layer by one each, their consumers take
+  // contiguous [bs, dim] tensors in the reference ABI).  Two columns are as far as the dot2 GEMV of the unfused calls goes; larger
+  // batches keep the reference order around the one-launch token mixer.
+  int decode_kernels_fused(int bs, const std::vector<Request35*>& rs, bool split) {
     auto md = [&](size_t off) { return reinterpret_cast<int32_t*>(meta_dev + off); };
     // a kernel node, not a memset node (csrc/elementwise.hip: pegainfer_zero_words)
     if (split && pegainfer_zero_words(merge_ctr, (int32_t)((size_t)max_bs * Hkv * 32), S())) { set_error("pegainfer_zero_words failed"); return -1; }
-    if (embedding_batched_cuda(embed, reinterpret_cast<uint32_t*>(meta_dev + m_tok), hidden, H, 1, S())) {
+    if (embedding_batched_cuda(embed, reinterpret_cast<uint32_t*>(meta_dev + m_tok), hidden, H, bs, S())) {
       set_error("embedding failed"); return -1;
     }
     const float sm = 1.0f / std::sqrt((float)D);
@@ -616,61 +631,72 @@ struct Model35 {
     int lin = 0, full = 0, rc = 0;
     for (const Layer35& ly : layers) {
       if (ly.full) {
-        rc = pegainfer_gemv_fused_ex(ly.q_proj, cur, wide, 2 * q_dim + 2 * kv_dim, 1, H, resid, ly.ln1,
-                                     resid ? nxt : nullptr, eps, 0, OFF | (resid ? RSUM : 0), S());
-        if (resid) std::swap(cur, nxt);
-        if (resid && tap_layer(lin + full - 1, cur, 1)) return -1;   // cur = the previous layer's output
-        Half *qf = wide, *kk = wide + 2 * q_dim, *vv = kk + kv_dim;   // [q|gate per head | k | v] of this token
+        Half *qf = wide, *kk, *vv;
+        if (bs == 1) {   // [q|gate per head | k | v] of this token
+          rc = pegainfer_gemv_fused_ex(ly.q_proj, cur, wide, 2 * q_dim + 2 * kv_dim, 1, H, resid, ly.ln1,
+                                       resid ? nxt : nullptr, eps, 0, OFF | (resid ? RSUM : 0), S());
+          kk = wide + 2 * q_dim;
+          vv = kk + kv_dim;
+          if (resid) std::swap(cur, nxt);
+        } else {         // k and v norm the sum that the q call has left (the norm reads the rounded sum in any case)
+          qf = q_full; kk = k_attn; vv = v_attn;
+          rc = pegainfer_gemv_fused_ex(ly.q_proj, cur, qf, 2 * q_dim, bs, H, resid, ly.ln1, resid ? nxt : nullptr, eps, 0,
+                                       OFF | (resid ? RSUM : 0), S());
+          if (resid) std::swap(cur, nxt);
+          if (!rc) rc = pegainfer_gemv_fused_ex(ly.k_proj, cur, kk, kv_dim, bs, H, nullptr, ly.ln1, nullptr, eps, 0, OFF, S());
+          if (!rc) rc = pegainfer_gemv_fused_ex(ly.v_proj, cur, vv, kv_dim, bs, H, nullptr, ly.ln1, nullptr, eps, 0, OFF, S());
+        }
+        if (resid && tap_layer(lin + full - 1, cur, bs)) return -1;   // cur = the previous layer's output
         if (!rc) {
           qk_norm_partial_rope_batched_decode_hd256_cuda(qf, kk, ly.q_norm, ly.k_norm, cos, sin, md(m_pos), q_attn, Hq,
-                                                         Hkv, 1, rotary, eps, S());
+                                                         Hkv, bs, rotary, eps, S());
           rc = paged_kv_scatter_cuda(kv_buffer, layout.k_offset(full), layout.v_offset(full), md(m_pages), md(m_indptr),
-                                     md(m_lpl), kk, vv, md(m_ri), md(m_pos), 1, Hkv, D, layout.page_size,
+                                     md(m_lpl), kk, vv, md(m_ri), md(m_pos), bs, Hkv, D, layout.page_size,
                                      layout.page_stride, kv_dim, D, S());
         }
         if (!rc && split)
           rc = pegainfer_paged_attention_decode_split_kv_hd256(
               q_attn, attn_out, kv_buffer, layout.k_offset(full), layout.v_offset(full), md(m_pages), md(m_indptr),
               md(m_lpl), md(m_sri), md(m_skt), md(m_skc), md(m_soi), meta_dev + m_sva, split_tmp_v, split_tmp_s, Hq, Hkv,
-              D, layout.page_size, 1, split_slots, layout.page_stride, sm, merge_ctr, S());
+              D, layout.page_size, bs, split_slots, layout.page_stride, sm, merge_ctr, S());
         else if (!rc)
           rc = paged_attention_decode_cuda_hd256(q_attn, attn_out, kv_buffer, layout.k_offset(full), layout.v_offset(full),
                                                  md(m_pages), md(m_indptr), md(m_lpl), md(m_ri), md(m_kti), md(m_kcs), Hq,
-                                                 Hkv, D, layout.page_size, 1, layout.page_stride, sm, S());
+                                                 Hkv, D, layout.page_size, bs, layout.page_stride, sm, S());
         if (rc) { set_error("fused full-attention layer failed"); return -1; }
-        attention_gate_batch_hd256_cuda(qf, attn_out, Hq, 1, S());
-        gemm_graphsafe_cuda(ly.o_proj, attn_out, attn_res, H, 1, q_dim, S());
+        attention_gate_batch_hd256_cuda(qf, attn_out, Hq, bs, S());
+        G(ly.o_proj, attn_out, attn_res, H, bs, q_dim);
         ++full;
       } else {
-        rc = pegainfer_gemv_fused_ex(ly.in_qkv, cur, wide, C + Z + 2 * vh, 1, H, resid, ly.ln1, resid ? nxt : nullptr,
+        const int W = C + Z + 2 * vh;
+        rc = pegainfer_gemv_fused_ex(ly.in_qkv, cur, wide, W, bs, H, resid, ly.ln1, resid ? nxt : nullptr,
                                      eps, 0, OFF | (resid ? RSUM : 0), S());
         if (rc) { set_error("fused linear-attention projection failed"); return -1; }
         if (resid) std::swap(cur, nxt);
-        if (resid && tap_layer(lin + full - 1, cur, 1)) return -1;
-        // (round 6) conv step + gated delta rule + gated norm in ONE launch (one workgroup per key head, same bits:
-        // csrc/qwen35.hip); PEGAINFER_LINATTN_FUSED=0, or a shape that kernel does not take, runs the three calls
-        if (!linattn_fused ||
-            pegainfer_linear_attn_decode_fused(wide, ly.conv_w, r->conv[lin], wide + C + Z, wide + C + Z + vh, ly.dt_bias,
-                                               ly.a_log, r->state[lin], ly.norm_w, wide + C, normed_gated, kh, vh, LK, LK,
-                                               convK, eps, lin_ticket, S()) != 0) {
-          conv1d_prefill_cuda(wide, ly.conv_w, r->conv[lin], qkv_conv, C, 1, convK, S());
-          gated_delta_rule_decode_cuda(qkv_conv, wide + C + Z, wide + C + Z + vh, ly.dt_bias, ly.a_log, r->state[lin],
-                                       gdr_out, kh, vh, LK, LK, S());
-          rms_norm_gated_cuda(gdr_out, ly.norm_w, wide + C, normed_gated, vh, LK, eps, S());
+        if (resid && tap_layer(lin + full - 1, cur, bs)) return -1;
+        // PEGAINFER_LINATTN_FUSED=0, or a shape that the one-launch kernel does not take, runs the three calls
+        if (!linattn_fused || linattn(ly, rs, lin, bs, wide, W, wide + C + Z, wide + C + Z + vh, W, wide + C, W)) {
+          for (int i = 0; i < bs; ++i) {
+            Half* row = wide + (size_t)i * W;
+            conv1d_prefill_cuda(row, ly.conv_w, rs[i]->conv[lin], qkv_conv, C, 1, convK, S());
+            gated_delta_rule_decode_cuda(qkv_conv, row + C + Z, row + C + Z + vh, ly.dt_bias, ly.a_log, rs[i]->state[lin],
+                                         gdr_out, kh, vh, LK, LK, S());
+            rms_norm_gated_cuda(gdr_out, ly.norm_w, row + C, normed_gated + (size_t)i * Z, vh, LK, eps, S());
+          }
         }
-        gemm_graphsafe_cuda(ly.out_proj, normed_gated, attn_res, H, 1, Z, S());
+        G(ly.out_proj, normed_gated, attn_res, H, bs, Z);
         ++lin;
       }
       // mid = bf16(cur + attn_res) -> nxt; act = silu_mul(gate, up) of norm_offset(mid)
-      rc = pegainfer_gemv_fused_ex(ly.gate, cur, act_out, 2 * I, 1, H, attn_res, ly.ln2, nxt, eps, I, OFF | RSUM | SILU2, S());
+      rc = pegainfer_gemv_fused_ex(ly.gate, cur, act_out, 2 * I, bs, H, attn_res, ly.ln2, nxt, eps, I, OFF | RSUM | SILU2, S());
       if (rc) { set_error("fused gate|up GEMV failed"); return -1; }
       std::swap(cur, nxt);
-      gemm_graphsafe_cuda(ly.down, act_out, mlp_out, H, 1, I, S());
+      G(ly.down, act_out, mlp_out, H, bs, I);
       resid = mlp_out;
     }
-    rc = pegainfer_gemv_fused_ex(embed, cur, logits, V, 1, H, resid, final_norm, nxt, eps, 0, OFF | RSUM, S());
-    if (!rc) rc = tap_layer(L - 1, nxt, 1);
-    if (rc || pegainfer_batched_top1(logits, V, 1, V, top1_state, tokens_out_d, S())) { set_error("fused lm_head failed"); return -1; }
+    rc = pegainfer_gemv_fused_ex(embed, cur, logits, V, bs, H, resid, final_norm, nxt, eps, 0, OFF | RSUM, S());
+    if (!rc) rc = tap_layer(L - 1, nxt, bs);
+    if (rc || pegainfer_batched_top1(logits, V, bs, V, top1_state, tokens_out_d, S())) { set_error("fused lm_head failed"); return -1; }
     return 0;
   }
   // bench.py roofline: the dominant kernel of the fused bs = 1 step - the gate|up GEMV with the residual add + (1 + w)
@@ -694,7 +720,7 @@ struct Model35 {
     return ms / iters;
   }
   int run_decode_kernels(int n, const std::vector<Request35*>& rs, bool split) {
-    if (decode_mode == 1 && n == 1 && (H & 7) == 0) return decode_kernels_fused1(rs[0], split);
+    if (decode_mode == 1 && n <= kFusedBatch && (H & 7) == 0) return decode_kernels_fused(n, rs, split);
     return decode_kernels(n, rs, split);
   }
 

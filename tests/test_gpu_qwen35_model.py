@@ -144,6 +144,34 @@ def test_qwen35_graph_eager_batch_and_handoff(built_libs, golden35):
     eng.close()
 
 
+@pytest.mark.parametrize("n", [2, 3])
+@pytest.mark.parametrize("split", [0, 1])
+def test_qwen35_fused_batch_decode_bitwise_equals_reference_sequence(built_libs, golden35, split, n, monkeypatch):
+    """Two requests (stacked projections, fused prologues, one launch for the token mixers of both) and three (reference order around
+    that launch) == the reference-order op sequence, logits bit for bit; the contexts differ and one request joins late, so windows,
+    states and tickets of several requests are told apart."""
+    meta, _ = golden35
+    runs = []
+    for mode in ("0", "1"):
+        monkeypatch.setenv("PEGAINFER_Q35_DECODE_MODE", mode)
+        eng = make_engine(meta, split_policy=split)
+        rids, toks, rows = [], [], []
+        for i in range(n):
+            r = eng.new_request()
+            toks.append(eng.prefill(r, meta["cases"][i % len(meta["cases"])]["prompt_tokens"] + [7] * i))
+            rids.append(r)
+            o, lg = eng.decode(rids, toks, want_logits=True)
+            rows.append(lg.copy())
+            toks = [int(t) for t in o]
+        for _ in range(6):
+            o, lg = eng.decode(rids, toks, want_logits=True)
+            rows.append(lg.copy())
+            toks = [int(t) for t in o]
+        runs.append(np.concatenate(rows))
+        eng.close()
+    assert np.array_equal(runs[0].view(np.uint32), runs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("split", [0, 1])
 def test_qwen35_fused_decode_bitwise_equals_reference_sequence(built_libs, golden35, split, monkeypatch):
     """bs = 1 fused step (stacked-projection GEMVs with the norm / residual-add prologues and the SwiGLU epilogue in
