@@ -183,6 +183,29 @@ __device__ __forceinline__ float attn_score(const AttnForm& form, float dot, flo
   return sc;
 }
 
+// cap * tanh(x / cap) of eight scores in fp32: an odd series where tanh is nearly its argument (next term below 3e-7 of it), beyond it
+// 1 - 2 / (e^2u + 1), which runs into +-1 without an infinity in between.  Scores of a wave that all lie below 0.35 cap take the series alone.
+__device__ __forceinline__ void soft_cap8(f32x4 (&x)[2], float cap, float inv_cap) {
+  float u[8], small[8];
+  bool near = true;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    u[i] = x[i >> 2][i & 3] * inv_cap;
+    const float u2 = u[i] * u[i];
+    near = near && u2 < 0.1225f;
+    small[i] = u[i] * fmaf(u2, fmaf(u2, fmaf(u2, fmaf(u2, 0.021869489f, -0.053968254f), 0.13333333f), -0.33333333f), 1.0f);
+  }
+  if (!__all(near)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float big = fmaf(-2.0f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(u[i] * 2.8853900818f) + 1.0f), 1.0f);
+      if (!(u[i] * u[i] < 0.1225f)) small[i] = big;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i >> 2][i & 3] = cap * small[i];
+}
+
 // A row's softmax states (one per map) turned into its output: the sink joins every denominator, the maps are combined, the
 // head is normed, `factor` comes last.  The wave holds the row: lane l has columns l, l + 64, ...
 template <typename A, int MAPS>
@@ -685,13 +708,24 @@ static size_t mfma_attention_lds(int maps, int dim, int ncb) {
 }
 
 // Prompts: the same attention with 16 RG rows per workgroup (32 or 64), for a bf16 cache, one map, sizes in multiples of 8.
-// Two waves per 16 rows, each on 32 of a tile's 64 keys, two softmax streams per row folded once at the end.  The next tile is on its way
-// while one is multiplied: its values are requested into registers a whole tile ahead (its page numbers two tiles ahead, through LDS)
-// and land in the other half of a double buffer, so a tile costs one barrier.  Products on v_mfma_f32_16x16x32_bf16: S^T = K Q^T leaves
-// lane l with the scores of row l % 16, and O^T = V^T P^T takes them as they are - which of its 32 keys sits in which place of the product
-// is free, so a lane's two runs of four keys are its eight places - and leaves the outputs of row l % 16 in the same lane: the running
-// maximum's factors need no exchange.  Values lie transposed in LDS as pairs of keys (dword: column, key pair), the pair number XORed with
-// bits of the column: writes along a row and reads along 16 columns both spread over the banks.
+// Two waves per 16 rows, each on 32 of a tile's 64 keys, two softmax streams per row folded once at the end.  Keys and values travel by
+// LDS-DMA into a ring of S tiles, row-major, requested S - 1 tiles ahead (their page numbers one tile further, in scalar registers: a vector
+// load beside the DMAs could only be waited for together with them): a tile costs one barrier and a counted wait, no LDS writes.  A row's 16-byte chunks are XORed with bits of its number (the DMA
+// fetches the chunk that belongs in its place), so 16 rows of one column lie in 16 different bank groups.
+// Products on v_mfma_f32_16x16x32_bf16: S^T = K Q^T leaves lane l with the scores of row l % 16, and O^T = V^T P^T takes them as they
+// are - which of its 32 keys sits in which place of the product is free, so a lane's two runs of four keys are its eight places (the
+// value fragments come from ds_read_b64_tr_b16 of the same row-major tile) - and leaves the outputs of row l % 16 in the same lane.  The
+// running maximum follows only when a score passes it by more than 2^8: weights up to 256 keep their relative precision, and a tile
+// without a jump needs no exchange between lanes; the row sums stay per lane until the end.
+// Bound by each wave's chain through a tile (LDS reads, products, weights, products) at two waves per SIMD.  1024 rows x 16 heads of 128: 28 us
+// causal (153 TFLOP/s), 86 us behind 3072 cached tokens, 103 us with a cap - against 39, 131 and 160 us with both tiles
+// passing through registers, values transposed on the way, scores shaped one by one and the maximum exchanged in every tile.
+template <int P, int RG>
+struct RowsShape {
+  static constexpr int N = RG * 128, CH = P / 8, S = P == 256 || RG == 2 ? 2 : 3;   // threads, chunks of a row, tiles in the ring
+  static constexpr int kTile = kAttKeys * P * 2;                                  // bytes of a key (or value) tile
+  static constexpr int kLoads = 2 * (kTile / 1024) / (2 * RG);                    // DMA instructions per wave and tile
+};
 template <int P, int RG>
 __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     const float* __restrict__ q, const uint16_t* __restrict__ cache, int64_t page_stride, int64_t k_cache_off, int64_t v_cache_off,
@@ -701,11 +735,9 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     const int32_t* __restrict__ tile_qh0, const int32_t* __restrict__ tile_nqh, uint16_t* __restrict__ out, int64_t out_stride,
     AttnForm form) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
-  constexpr int N = RG * 128, NCB = P / 16, CH = P / 8, KS = P + 8, KU = 64 * CH / N, VU = (32 * CH + N - 1) / N;
-  constexpr float kLog2e = 1.44269504088896341f;
-  uint16_t* s_k = reinterpret_cast<uint16_t*>(smraw);                 // [2][64][KS]
-  uint32_t* s_v = reinterpret_cast<uint32_t*>(s_k + 2 * kAttKeys * KS);   // [2][P][32]
-  __shared__ int s_pg[2][kAttKeys];
+  typedef RowsShape<P, RG> Sh;
+  constexpr int N = Sh::N, NCB = P / 16, CH = Sh::CH, S = Sh::S;     // LDS: ring [S][keys | values][64][P]
+  constexpr float kLog2e = 1.44269504088896341f, kJump = 8.0f;
   const int tile = gridDim.x - 1 - blockIdx.x, g = blockIdx.y;        // the longest rows of keys first
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, lg = lane >> 4;
   const int rg = wave % RG, kh = wave / RG;
@@ -726,7 +758,10 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   const int rpos = mine ? positions[row0 + lr / nqh] : -1, rlo = mine ? attn_row_lo(form, rpos) : 0;
   const int rqh = g * per_group + qh0 + (mine ? lr % nqh : 0);
   const float rsl = form.dist_slope ? form.dist_slope[rqh] : 0.f;
-  const int last = rg * 16 < nrows ? positions[row0 + min(rg * 16 + 15, nrows - 1) / nqh] : -1;    // uniform: no later key concerns the wave
+  const float inv_cap = form.softcap > 0.f ? 1.0f / form.softcap : 0.f;
+  // uniform: no key after `last` concerns the wave; keys of [all_lo, all_hi] are seen by all of its rows, without a look at each
+  const int last = rg * 16 < nrows ? positions[row0 + min(rg * 16 + 15, nrows - 1) / nqh] : -1;
+  const int all_lo = last >= 0 ? attn_row_lo(form, last) : 0, all_hi = rg * 16 + 15 < nrows ? positions[row0 + rg * 16 / nqh] : -1;
   bf16x8_t qf[P / 32];
   {
     const float* qr = q + ((int64_t)(row0 + (mine ? lr / nqh : 0)) * H + rqh) * dim;
@@ -738,133 +773,187 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
       qf[st] = __builtin_bit_cast(bf16x8_t, u32x4{pack_bf2(t[0], t[1]), pack_bf2(t[2], t[3]), pack_bf2(t[4], t[5]), pack_bf2(t[6], t[7])});
     }
   }
-  for (int i = tid; i < 2 * kAttKeys * KS / 8; i += N) reinterpret_cast<u32x4*>(s_k)[i] = u32x4{0u, 0u, 0u, 0u};   // columns past dim stay zero
-  u32x4 rk[KU], rv[VU][2];
-  auto page_of = [&](int k0) { return k0 + tid < kmax ? pages[(k0 + tid) / page_size] : 0; };      // threads 0 .. 63
-  auto request = [&](int k0, int b) {      // the tile's values into registers; keys past the context's end as zeros
-    const u32x4 zero = {0u, 0u, 0u, 0u};
+  if (dim < P || vdim < P) {       // chunks past a row's end are never fetched: they stay zero
+    for (int i = tid; i < S * 2 * Sh::kTile / 16; i += N) reinterpret_cast<u32x4*>(smraw)[i] = u32x4{0u, 0u, 0u, 0u};
+  }
+  // swizzle of row j: CH 16 - its low four bits; CH 8 - two rows share 256 bytes, the three bits above the lowest
+  auto swz = [](int j) { return CH == 8 ? (j >> 1) & 7 : j & 15; };
+  // a wave's DMA instructions: kLoads / 2 of the key tile, as many of the value tile; lane l fills the 16 bytes l of a run of 64
+  constexpr int kHalf = Sh::kLoads / 2;
+  int src_j[kHalf], src_c[kHalf], off_k[kHalf], off_v[kHalf];
+  // the rows of one instruction share a page and lie at the same place in it for every tile (pages of 16: always)
+  const bool even = page_size % (64 / CH) == 0 && kAttKeys % page_size == 0;
 #pragma unroll
-    for (int i = 0; i < KU; ++i) {
-      const int c = (tid % CH) * 8, j = tid / CH + (N / CH) * i, p = k0 + j;
-      rk[i] = zero;
-      if (p < kmax && c < dim) {
-        const int64_t slot = (int64_t)(p % page_size) * G + g;
-        const uint16_t* pg = cache + (int64_t)s_pg[b][j] * page_stride;
-        rk[i] = *reinterpret_cast<const u32x4*>(c < kw ? pg + k_cache_off + slot * kw + c : pg + v_cache_off + slot * vdim + c);
-      }
-    }
+  for (int i = 0; i < kHalf; ++i) {
+    const int unit = (wave * kHalf + i) * 64 + lane;
+    src_j[i] = unit / CH;
+    src_c[i] = ((unit % CH) ^ swz(src_j[i])) * 8;
+    const int slot = (src_j[i] % page_size) * G + g;
+    off_k[i] = src_c[i] < kw ? slot * kw + src_c[i] : slot * vdim + src_c[i];
+    off_v[i] = slot * vdim + src_c[i];
+  }
+  const uint16_t *kbase = cache + k_cache_off, *vbase = cache + v_cache_off;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr_t)smraw;
+  auto dma = [&](const uint16_t* src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :: "v"(src), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+  };
+  // page numbers of a tile's instructions, uniform over the wave (even pages)
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  auto page_numbers = [&](int k0, int (&pn)[kHalf]) {
 #pragma unroll
-    for (int i = 0; i < VU; ++i) {
-      const int unit = tid + N * i, c = (unit % CH) * 8, jp = unit / CH;
+    for (int i = 0; i < kHalf; ++i) pn[i] = even ? pages[min(k0 + (wave_u * kHalf + i) * (64 / CH), kmax - 1) / page_size] : 0;
+  };
+  // kLoads instructions per wave, whatever the tile: keys past the end fetch the last key's row again
+  auto fetch = [&](int i, int64_t page, int ok, int ov, int stage) {
+    const int c = src_c[i];
+    const uint32_t dst = ring + (uint32_t)(stage * 2 * Sh::kTile + (wave_u * kHalf + i) * 1024);
+    if (c < dim) dma((c < kw ? kbase : vbase) + page + ok, dst);
+    if (c < vdim) dma(vbase + page + ov, dst + Sh::kTile);
+  };
+  auto fetch_at = [&](int i, int p, int page, int stage) {     // the general form: a key's own page and place
+    const int slot = (p % page_size) * G + g, c = src_c[i];
+    fetch(i, (int64_t)page * page_stride, c < kw ? slot * kw + c : slot * vdim + c, slot * vdim + c, stage);
+  };
+  auto request = [&](int k0, const int (&pn)[kHalf], int stage) {
+    if (even && k0 + kAttKeys <= kmax) {             // uniform; paths of their own: a vector load of page numbers would be waited for in both
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int j = 2 * jp + t, p = k0 + j;
-        rv[i][t] = zero;
-        if (jp < 32 && p < kmax && c < vdim)
-          rv[i][t] = *reinterpret_cast<const u32x4*>(cache + (int64_t)s_pg[b][j] * page_stride + v_cache_off + ((int64_t)(p % page_size) * G + g) * vdim + c);
+      for (int i = 0; i < kHalf; ++i) fetch(i, (int64_t)pn[i] * page_stride, off_k[i], off_v[i], stage);
+    } else if (even) {
+#pragma unroll
+      for (int i = 0; i < kHalf; ++i) fetch_at(i, min(k0 + src_j[i], kmax - 1), pn[i], stage);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kHalf; ++i) {
+        const int p = min(k0 + src_j[i], kmax - 1);
+        fetch_at(i, p, pages[p / page_size], stage);
       }
     }
   };
-  auto v_at = [](int col, int jp) { return col * 32 + (jp ^ (((col ^ (col >> 3)) & 7) << 2)); };
-  auto land = [&](int b) {
-    uint16_t* kb = s_k + b * kAttKeys * KS;
-    uint32_t* vb = s_v + b * P * 32;
-#pragma unroll
-    for (int i = 0; i < KU; ++i) {
-      const int c = (tid % CH) * 8, j = tid / CH + (N / CH) * i;
-      if (c < dim) *reinterpret_cast<u32x4*>(kb + j * KS + c) = rk[i];
-    }
-#pragma unroll
-    for (int i = 0; i < VU; ++i) {
-      const int unit = tid + N * i, c = (unit % CH) * 8, jp = unit / CH;
-      if (jp < 32) {
-        const uint32_t a[4] = {rv[i][0].x, rv[i][0].y, rv[i][0].z, rv[i][0].w}, d[4] = {rv[i][1].x, rv[i][1].y, rv[i][1].z, rv[i][1].w};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          vb[v_at(c + 2 * u, jp)] = (a[u] & 0xFFFFu) | (d[u] << 16);
-          vb[v_at(c + 2 * u + 1, jp)] = (a[u] >> 16) | (d[u] & 0xFFFF0000u);
-        }
-      }
-    }
-  };
-  float mrun = -INFINITY, lrun = 0.f;
+  float mrun = -INFINITY, lrun = 0.f;                 // log2 units; lrun: this lane's part of the row sum
   f32x4 o[NCB];
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) o[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int k0, int b) {
+  const int krow = 32 * kh + l15, vrow = 32 * kh + 4 * lg + (l15 >> 2);
+  // byte addresses inside a tile: swz(row + 16) = swz(row) for both row widths, so the second half of the keys lies 16 rows on
+  const uint32_t ka = (uint32_t)(krow * P * 2 + ((lg ^ swz(krow)) << 4));
+  const uint32_t va = (uint32_t)(vrow * P * 2 + ((((l15 & 3) >> 1) ^ swz(vrow)) << 4) + (l15 & 1) * 8);
+  auto multiply = [&](int k0, int stage) {
     const int kb = k0 + 32 * kh;
     if (kb > last || kb >= kmax) return;             // uniform over the wave
-    const uint16_t* ka = s_k + b * kAttKeys * KS + (32 * kh + l15) * KS + lg * 8;
+    const unsigned char* kt = smraw + stage * 2 * Sh::kTile;
     f32x4 sc[2] = {};
 #pragma unroll
     for (int st = 0; st < P / 32; ++st)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(ka + 16 * t * KS + st * 32)),
-                                                         qf[st], sc[t], 0, 0, 0);
-    float tmax = -INFINITY;
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(kt + 16 * t * P * 2 + (ka ^ (uint32_t)(st << 6)))), qf[st], sc[t], 0, 0, 0);
+    // dot products -> scores times log2(e); each option in a pass of its own: one uniform branch per tile, its loads in flight together
+    const int dist = rpos - kb - 4 * lg;             // of this lane's key (t, r): dist - 16 t - r
+    const bool options = form.softcap > 0.f || form.dist_bias || form.dist_slope;
+    const float f0 = options ? scale : scale * kLog2e;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kp = kb + 16 * t + 4 * lg + r;
-        sc[t][r] = kp <= rpos && (kp >= rlo || kp < form.keep_first) ? attn_score(form, sc[t][r], scale, rpos, kp, rqh, H, rsl) : -INFINITY;
-        tmax = fmaxf(tmax, sc[t][r]);
-      }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-    const float mnew = fmaxf(mrun, tmax), mref = mnew == -INFINITY ? 0.f : mnew;
-    const float corr = __builtin_amdgcn_exp2f((mrun - mref) * kLog2e);           // a row that has met no key yet: 0, and nothing to scale
+      for (int r = 0; r < 4; ++r) sc[t][r] *= f0;
+    if (form.softcap > 0.f) soft_cap8(sc, form.softcap, inv_cap);
+    if (form.dist_bias) {
+      float bias[2][4];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bias[t][r] = form.dist_bias[(int64_t)max(0, min(dist - 16 * t - r, form.n_dist - 1)) * H + rqh];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[t][r] += bias[t][r];
+    }
+    if (form.dist_slope) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[t][r] = fmaf(-rsl, (float)(dist - 16 * t - r), sc[t][r]);
+    }
+    if (options) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[t][r] *= kLog2e;
+    }
+    if (kb < all_lo || kb + 31 > all_hi) {           // uniform: some row of the wave does not see some of these keys
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int kp = kb + 16 * t + 4 * lg + r;
+          if (!(kp <= rpos && (kp >= rlo || kp < form.keep_first))) sc[t][r] = -INFINITY;
+        }
+    }
+    float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])), fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
+    if (__any(!(tmax <= mrun + kJump))) {            // uniform; the first keys of a row always, a NaN too
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+      const float mnew = fmaxf(mrun, tmax);
+      const float corr = __builtin_amdgcn_exp2f(mrun - (mnew == -INFINITY ? 0.f : mnew));   // a row that has met no key yet: 0, and nothing to scale
+      lrun *= corr;
+#pragma unroll
+      for (int cb = 0; cb < NCB; ++cb) { o[cb].x *= corr; o[cb].y *= corr; o[cb].z *= corr; o[cb].w *= corr; }
+      mrun = mnew;
+    }
+    const float mref = mrun == -INFINITY ? 0.f : mrun;
     uint32_t pb[4];
     float psum = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        const uint32_t w = pack_bf2(__builtin_amdgcn_exp2f((sc[t][r] - mref) * kLog2e), __builtin_amdgcn_exp2f((sc[t][r + 1] - mref) * kLog2e));
+        const uint32_t w = pack_bf2(__builtin_amdgcn_exp2f(sc[t][r] - mref), __builtin_amdgcn_exp2f(sc[t][r + 1] - mref));
         pb[2 * t + (r >> 1)] = w;
         psum += bf_lo(w) + bf_hi(w);                 // the sum of the weights as they are multiplied
       }
-    psum += __shfl_xor(psum, 16, kWave);
-    psum += __shfl_xor(psum, 32, kWave);
-    lrun = lrun * corr + psum;
-    if (__any(mnew != mrun)) {
-#pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) { o[cb].x *= corr; o[cb].y *= corr; o[cb].z *= corr; o[cb].w *= corr; }
-    }
-    mrun = mnew;
+    lrun += psum;
     const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, u32x4{pb[0], pb[1], pb[2], pb[3]});
-    const uint32_t* vb = s_v + b * P * 32;
+    typedef v4s_t __attribute__((address_space(3)))* lds_v4_t;
+    const uint32_t vt = ring + (uint32_t)(stage * 2 * Sh::kTile + Sh::kTile);
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
-      const int col = 16 * cb + l15, jp = 16 * kh + 2 * lg;
-      const u32x2 v0 = *reinterpret_cast<const u32x2*>(vb + v_at(col, jp)), v1 = *reinterpret_cast<const u32x2*>(vb + v_at(col, jp + 8));
+      const uint32_t at = vt + (va ^ (uint32_t)(cb << 5));
+      const u32x2 v0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)at));
+      const u32x2 v1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)(at + 16 * P * 2)));
       o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, u32x4{v0.x, v0.y, v1.x, v1.y}), pf, o[cb], 0, 0, 0);
     }
   };
-  int k0 = kfirst, k1 = next_tile(k0);
-  if (tid < kAttKeys) {
-    s_pg[0][tid] = page_of(k0);
-    s_pg[1][tid] = page_of(k1);
+  int k[S + 1];                                      // k[i]: the tile i ahead
+  k[0] = kfirst;
+#pragma unroll
+  for (int i = 1; i <= S; ++i) k[i] = next_tile(k[i - 1]);
+  int pn[kHalf];
+  __syncthreads();                                   // the zeros are in LDS
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i) {
+    page_numbers(k[i], pn);
+    request(k[i], pn, i);
   }
-  __syncthreads();
-  request(k0, 0);
-  land(0);
-  __syncthreads();
-  request(k1, 1);
-  for (int b = 0;; b ^= 1) {
-    const int k2 = next_tile(k1);
-    const int pg = tid < kAttKeys ? page_of(k2) : 0;
-    multiply(k0, b);
-    if (k1 >= kmax) break;                           // uniform over the workgroup
-    land(b ^ 1);
-    if (tid < kAttKeys) s_pg[b][tid] = pg;
-    __syncthreads();
-    k0 = k1;
-    k1 = k2;
-    request(k1, b);                                  // k1 may lie past the end: zeros, no access
+  page_numbers(k[S - 1], pn);
+  int stage = 0;
+  while (true) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * Sh::kLoads) : "memory");   // this wave's part of tile k[0] has landed
+    __syncthreads();                                 // everybody's has; the stage of the tile before is free
+    request(k[S - 1], pn, stage == 0 ? S - 1 : stage - 1);
+    page_numbers(k[S], pn);
+    multiply(k[0], stage);
+    if (k[1] >= kmax) break;                         // uniform over the workgroup
+#pragma unroll
+    for (int i = 0; i < S; ++i) k[i] = k[i + 1];
+    k[S] = next_tile(k[S]);
+    stage = stage + 1 == S ? 0 : stage + 1;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in the memory that is reused below
   __syncthreads();                                   // the tiles' LDS is free
+  lrun += __shfl_xor(lrun, 16, kWave);
+  lrun += __shfl_xor(lrun, 32, kWave);
   f32x4* f_o = reinterpret_cast<f32x4*>(smraw);      // [RG][NCB][64]
   float* f_ml = reinterpret_cast<float*>(f_o + RG * NCB * 64);        // [RG][64][2]
   if (kh == 1) {
@@ -878,11 +967,11 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   const float m1 = f_ml[(rg * 64 + lane) * 2], l1 = f_ml[(rg * 64 + lane) * 2 + 1];
   float mall = fmaxf(mrun, m1), sink = -INFINITY;
   if (form.sink && mine) {
-    sink = bf2f(static_cast<const uint16_t*>(form.sink)[rqh]);
+    sink = bf2f(static_cast<const uint16_t*>(form.sink)[rqh]) * kLog2e;
     mall = fmaxf(mall, sink);
   }
-  const float w0 = mrun == -INFINITY ? 0.f : expf(mrun - mall), w1 = m1 == -INFINITY ? 0.f : expf(m1 - mall);
-  const float l = lrun * w0 + l1 * w1 + (sink == -INFINITY ? 0.f : expf(sink - mall));
+  const float w0 = mrun == -INFINITY ? 0.f : exp2f(mrun - mall), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - mall);
+  const float l = lrun * w0 + l1 * w1 + (sink == -INFINITY ? 0.f : exp2f(sink - mall));
   const float i0 = w0 / l, i1 = w1 / l;
   float ss = 0.f;
 #pragma unroll
@@ -918,8 +1007,10 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     st4(dst + c, v);
   }
 }
-static size_t rows_attention_lds(int p, int rg) {
-  return std::max((size_t)2 * kAttKeys * (p + 8) * 2 + (size_t)2 * p * 32 * 4, (size_t)rg * 64 * (p / 16 * 16 + 8));
+template <int P, int RG>
+static constexpr size_t rows_attention_lds() {
+  typedef RowsShape<P, RG> Sh;
+  return std::max((size_t)Sh::S * 2 * Sh::kTile, (size_t)RG * 64 * (P + 8));
 }
 
 // The states that the splits of a tile have left, brought to their common maximum and summed in split order, then finished like
@@ -1147,8 +1238,7 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
         !host_aligned16(out) || !host_aligned16(q) || !host_aligned16(cache) || k_cache_off % 8 ||
         !pegainfer_paged_attention_rows_ok(dim, vdim, opt->shared_tail, page_stride, v_cache_off, page_size))
       return PK_BAD;
-    auto launch = [&](auto kern, int p, int rg) {
-      const size_t lds = rows_attention_lds(p, rg);
+    auto launch = [&](auto kern, size_t lds, int rg) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         ok = false;
         return;
@@ -1160,9 +1250,9 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
     auto by_size = [&](auto rg) {
       constexpr int RG = decltype(rg)::value;
       const int most = std::max(dim, vdim);
-      if (most <= 64) launch(paged_attention_rows_kernel<64, RG>, 64, RG);
-      else if (most <= 128) launch(paged_attention_rows_kernel<128, RG>, 128, RG);
-      else launch(paged_attention_rows_kernel<256, RG>, 256, RG);
+      if (most <= 64) launch(paged_attention_rows_kernel<64, RG>, rows_attention_lds<64, RG>(), RG);
+      else if (most <= 128) launch(paged_attention_rows_kernel<128, RG>, rows_attention_lds<128, RG>(), RG);
+      else launch(paged_attention_rows_kernel<256, RG>, rows_attention_lds<256, RG>(), RG);
     };
     if (opt->tile_rows == 64) by_size(std::integral_constant<int, 4>());
     else by_size(std::integral_constant<int, 2>());

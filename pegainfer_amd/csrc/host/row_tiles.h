@@ -1,0 +1,45 @@
+// Row tiles of the paged attention launches (pegainfer_paged_attention_opt): a tile is a run of token rows of one entry times a run of the
+// query heads of one key/value head.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+namespace ptiles {
+
+constexpr int kGroupRows = 16;      // (token, query head) rows of one workgroup of the general attention kernels
+// A step whose 64- (32-) row tiles give so many workgroups takes those; below, 16-row tiles whose keys are dealt to several workgroups have more
+// of them.  16 heads over 4 key/value heads of 128, 16 / 32 / 64 rows: 1024 tokens 82 / 38 / 28 us, 128 tokens (32 workgroups of 64 rows)
+// 14.5 / 10.4 / 10.2 us, behind 2048 cached tokens 128 / 55 / 45 us.
+constexpr int kWideGroups = 32;
+
+inline size_t count(const int32_t* lens, int n, int per, int rows) {
+  const int tpt = std::max(1, rows / per), cuts = (per + rows - 1) / rows;
+  size_t c = 0;
+  for (int i = 0; i < n; ++i) c += (size_t)((lens[i] + tpt - 1) / tpt) * cuts;
+  return c;
+}
+// rows of a tile for a step of prompts: the widest tiles that still fill the chip (kv: key/value heads of the launch; <= 0: the launch
+// takes no wide tiles) and are at least half full
+inline int wide_rows(const int32_t* lens, int n, int T, int per, int kv) {
+  for (int rows : {64, 32}) {
+    const long tiles = (long)count(lens, n, per, rows);
+    if (tiles * kv >= kWideGroups && (long)T * per * 2 >= tiles * rows) return rows;
+  }
+  return kGroupRows;
+}
+// the table's four columns, `tiles` (= count()) values each: first token row, tokens, first query head, query heads
+inline void cut(const int32_t* lens, int n, int per, int rows, size_t tiles, int32_t* table) {
+  int32_t *row0 = table, *ntok = row0 + tiles, *qh0 = ntok + tiles, *nqh = qh0 + tiles;
+  const int tpt = std::max(1, rows / per);
+  size_t at = 0;
+  int r0 = 0;
+  for (int i = 0; i < n; r0 += lens[i++])
+    for (int t0 = 0; t0 < lens[i]; t0 += tpt)
+      for (int q0 = 0; q0 < per; q0 += rows, ++at) {
+        row0[at] = r0 + t0; ntok[at] = std::min(tpt, lens[i] - t0); qh0[at] = q0; nqh[at] = std::min(rows, per - q0);
+      }
+}
+
+}  // namespace ptiles

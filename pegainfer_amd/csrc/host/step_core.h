@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "row_tiles.h"
 #include "seq_state.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
@@ -75,8 +76,7 @@ inline bool ends_with(const std::string& s, const char* suf) {
 }
 
 constexpr int kPageSize = 16;       // tokens per cache page, as in the other runtimes
-constexpr int kGroupRows = 16;      // (token, query head) rows of one workgroup of the paged attention
-constexpr int kWideGroups = 256;    // a step whose 64- (32-) row tiles give so many workgroups takes those
+using ptiles::kGroupRows;
 constexpr int kFlatRows = 64;       // flattened (token, head) rows of one workgroup of the latent attention
 
 // A table of row tiles on the device.  Group tiles: runs of tokens of one entry times a run of the query heads of one key/value
@@ -321,7 +321,7 @@ class StepModel {
     std::vector<std::pair<size_t, int>> group_at, flat_at;    // (offset, tiles)
     std::vector<int> group_rows;
     for (auto& gt : group_sets) {
-      const int rows = gt.wide_kv > 0 && !plain_kernels ? wide_rows(lens, n, (int)T, gt) : kGroupRows;
+      const int rows = plain_kernels ? kGroupRows : ptiles::wide_rows(lens, n, (int)T, gt.per, gt.wide_kv);
       group_rows.push_back(rows);
       group_at.push_back(put_group_tiles(&mb, lens, n, gt.per, rows));
     }
@@ -685,26 +685,11 @@ class StepModel {
     for (auto& c : cols) mb->insert(mb->end(), c.begin(), c.end());
     return {at, (int)cols[0].size()};
   }
-  // the widest tiles that still fill the chip and are at least half full
-  static int wide_rows(const int32_t* lens, int n, int T, const GroupSet& g) {
-    for (int rows : {64, 32}) {
-      const int tpt = std::max(1, rows / g.per), cuts = (g.per + rows - 1) / rows;
-      long tiles = 0;
-      for (int i = 0; i < n; ++i) tiles += (long)((lens[i] + tpt - 1) / tpt) * cuts;
-      if (tiles * g.wide_kv >= kWideGroups && (long)T * g.per * 2 >= tiles * rows) return rows;
-    }
-    return kGroupRows;
-  }
   static std::pair<size_t, int> put_group_tiles(std::vector<int32_t>* mb, const int32_t* lens, int n, int per, int rows) {
-    std::vector<std::vector<int32_t>> c(4);
-    auto add = [&](int row0, int ntok, int qh0, int nqh) { c[0].push_back(row0); c[1].push_back(ntok); c[2].push_back(qh0); c[3].push_back(nqh); };
-    int r0 = 0;
-    for (int i = 0; i < n; r0 += lens[i++]) {
-      const int tpt = std::max(1, rows / per);
-      for (int t0 = 0; t0 < lens[i]; t0 += tpt)
-        for (int q0 = 0; q0 < per; q0 += rows) add(r0 + t0, std::min(tpt, lens[i] - t0), q0, std::min(rows, per - q0));
-    }
-    return put_columns(mb, c);
+    const size_t at = mb->size(), tiles = ptiles::count(lens, n, per, rows);
+    mb->resize(at + 4 * tiles);
+    ptiles::cut(lens, n, per, rows, tiles, mb->data() + at);
+    return {at, (int)tiles};
   }
   static std::pair<size_t, int> put_flat_tiles(std::vector<int32_t>* mb, const int32_t* lens, int n, int heads) {
     std::vector<std::vector<int32_t>> c(2);

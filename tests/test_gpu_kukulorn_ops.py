@@ -413,3 +413,51 @@ def test_an_old_write_is_kept_by_a_slow_head_and_forgotten_by_a_fast_one():
         y = torch.cat(ys).cpu()
         assert abs(float(y[202, 0]) - 50.0 * math.exp(-0.001 * 200)) < 1e-3 and abs(float(y[202, P])) < 1e-30
         assert abs(float(y[2, P]) - 50.0) < 1e-4 and float(y[1].abs().max()) == 0.0
+
+
+FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
+         "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
+         "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
+
+
+@pytest.mark.parametrize("tile_rows", [32, 64])
+@pytest.mark.parametrize("dim,vdim,page", [(24, 40, 16), (64, 64, 8), (72, 128, 5), (128, 128, 16), (136, 256, 32), (256, 72, 16)])
+@pytest.mark.parametrize("form", FORMS)
+def test_wide_tiles_take_every_form(form, dim, vdim, page, tile_rows):
+    """The kernel for prompts against the fp32-FMA kernel on the same bf16 cache: every option, rows of one and two halves of 256 bytes and more,
+    rows whose last chunks are padding, pages that hold a whole number of a DMA's rows and pages that do not, entries that end around a
+    64-key tile, a portion behind a cached prefix.  The matrix cores see q and the weights in bf16 (2^-9 each, relative); a score of size s moves by
+    2^-9 s and with it its weight: 2^-7 of the largest value covers s up to 4 at these scales."""
+    from pegainfer_amd import ops_blocks as B
+    import ctypes
+    o = FORMS[form]
+    g = torch.Generator().manual_seed(dim * 7 + vdim + page)
+    H, G = 6, 2
+    lens, past = [1, 63, 64, 65, 130, 7], [0, 0, 0, 3, 0, 140]
+    T = sum(lens)
+    need = [-(-(a + b) // page) for a, b in zip(lens, past)]
+    order = torch.randperm(sum(need), generator=g).int()
+    indptr = torch.tensor([0] + np.cumsum(need).tolist(), dtype=torch.int32)
+    stride = (page * G * (dim + vdim) + 7) // 8 * 8
+    v_off = page * G * dim
+    cache = torch.randn(sum(need) * stride, generator=g).bfloat16().cuda()
+    q = torch.randn(T, H, dim, generator=g).cuda()
+    pos = torch.cat([torch.arange(b, a + b) for a, b in zip(lens, past)]).int().cuda()
+    ent = torch.cat([torch.full((a,), i) for i, a in enumerate(lens)]).int().cuda()
+    ind, ids = indptr.cuda(), order.cuda()
+    sink, bias = torch.randn(H, generator=g).bfloat16().cuda(), torch.randn(max(1, o.get("bias", 1)), H, generator=g).cuda()
+    slope, gate = torch.rand(H, generator=g).cuda() * 0.1, torch.randn(T, H * vdim, generator=g).bfloat16().cuda()
+    outs = []
+    for rows, plain in ((16, 1), (tile_rows, 0)):
+        t = B.attention_tiles(lens, H // G, "cuda", rows)
+        out = torch.full((T, H * vdim), float("nan"), dtype=torch.bfloat16, device="cuda")
+        a = B.AttnOptions(softcap=o.get("softcap", 0.0), window=o.get("window", 0), keep_first=o.get("keep_first", 0), block=o.get("block", 0),
+                          dist_bias=bias.data_ptr() if "bias" in o else None, n_dist=o.get("bias", 0), dist_slope=slope.data_ptr() if "slope" in o else None,
+                          sink=sink.data_ptr() if "sink" in o else None, head_norm=int(o.get("norm", False)), norm_eps=1e-6,
+                          gate=gate.data_ptr() if "gate" in o else None, gate_stride=H * vdim, gate_kind=o.get("gate", 0), n_split=1, plain=plain,
+                          tile_rows=rows if rows > 16 else 0)
+        B._chk(B.ffi.lib().pegainfer_paged_attention_opt(
+            q.data_ptr(), cache.data_ptr(), stride, 0, v_off, page, pos.data_ptr(), ent.data_ptr(), ind.data_ptr(), ids.data_ptr(), H, G, dim, vdim,
+            dim ** -0.5, 1.0, *(c.data_ptr() for c in t), t[0].numel(), out.data_ptr(), out.stride(0), ctypes.addressof(a), 0, B._stream()), "attention")
+        outs.append(out.float().cpu())
+    assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * outs[0].abs().max()
