@@ -138,9 +138,10 @@ pegainfer_status_t pegainfer_latent_prep_form(const pegainfer_latent_prep_desc* 
  * A row's keys are cut into splits of split_keys (<= 0: 1024) that run in parallel and are merged in split order;
  * workspace: fp32 scratch of pegainfer_latent_attention_workspace(...) floats (NULL allowed when that is 0).
  * Two forms.  tile_row0 == NULL: the plain form, any sizes, bf16 or fp32 cache, fp32 arithmetic throughout.
- * tile_row0 != NULL: the matrix-core form for a bf16 cache (pegainfer_latent_attention_tiled_ok says whether the sizes fit):
+ * tile_row0 != NULL: the matrix-core form (pegainfer_latent_attention_tiled_ok says whether the sizes fit):
  * the flattened rows t * heads + h are cut by the caller into n_tiles runs of <= 64 rows that stay inside one request
- * (tile_row0[i], tile_rows[i]); q and the softmax weights are rounded to bf16 where they enter the matrix cores. */
+ * (tile_row0[i], tile_rows[i]).  With a bf16 cache q and the softmax weights are rounded to bf16 where they enter the matrix
+ * cores; with an fp32 cache everything stays fp32. */
 int64_t pegainfer_latent_attention_workspace(int32_t n_tokens, int32_t heads, int32_t rank, int32_t max_kv_len,
                                              int32_t split_keys);
 int32_t pegainfer_latent_attention_tiled_ok(int32_t rank, int32_t rot, int64_t page_stride, int64_t layer_off, int32_t dtype);

@@ -12,11 +12,15 @@
 //
 //   latent_prep_kernel        RMS-norm of the latent, rotation of the shared key part and of the query's rotated part (halves or
 //                             neighbours), cache write; RMS-norm of a query latent (each part optional)
-//   latent_attn_kernel        one workgroup per (token, head, key split): 256 keys per round, scores by one thread per
+//   latent_attn_kernel        any sizes: one workgroup per (token, head, key split), 256 keys per round, scores by one thread per
 //                             key, online softmax, value accumulation by one thread per latent dimension
+//   latent_attn_mfma_kernel   bf16 cache, tiles of up to 64 (token, head) rows of one request: a wave per 16 rows
+//   latent_attn_few_kernel    tiles of a few rows of a bf16 cache, any tile of an fp32 one: four waves per 16 or 32 rows
 //   latent_attn_merge_kernel  combines the key splits of a row (log-sum-exp weights), fixed split order
 // A row's result depends on its own query, position and cache entries only.  With contiguous splits the split count is a
 // function of the row's key count alone; with dealt splits it also depends on the step's shape (rounding only).
+#include <type_traits>
+
 #include "common.h"
 #include "typed.h"
 #include "pegainfer_kernels_blocks.h"
@@ -115,7 +119,22 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrep<A> a, float
   }
 }
 
-// partial layout per (row = t * H + h, split): [m, l, acc[rank]] fp32
+// What a split of a row leaves for the merge, all fp32: the rows' accumulators ([row][split][rank]; row = t * H + h), and behind
+// them [row][split][maximum, sum], so that the accumulators of a rank that is a multiple of four lie on 16 bytes.
+struct LatentPartial {
+  float *acc, *max_sum;      // of one (row, split), or of a row's first split
+  int r;
+  __device__ __forceinline__ LatentPartial(float* base, int64_t slots, int rank, int64_t slot)
+      : acc(base + slot * rank), max_sum(base + slots * rank + 2 * slot), r(rank) {}
+  __device__ __forceinline__ LatentPartial(const float* base, int64_t slots, int rank, int64_t slot)
+      : LatentPartial(const_cast<float*>(base), slots, rank, slot) {}
+  __device__ __forceinline__ f32x4 load(int split, int d, bool vec) const {
+    const float* p = acc + (int64_t)split * r + d;
+    if (vec) return *reinterpret_cast<const f32x4*>(p);
+    return f32x4{p[0], d + 1 < r ? p[1] : 0.f, d + 2 < r ? p[2] : 0.f, d + 3 < r ? p[3] : 0.f};
+  }
+};
+
 template <typename A>
 __global__ __launch_bounds__(256) void latent_attn_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
                                                           const A* __restrict__ cache, int64_t page_stride,
@@ -175,39 +194,65 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const float* __restric
       if (d < r) o_lat[((int64_t)t * H + h) * r + d] = acc[k] * inv;
     }
   } else {
-    float* part = partial + (((int64_t)t * H + h) * max_splits + split) * (r + 2);
-    if (tid == 0) { part[0] = m; part[1] = l; }
+    const LatentPartial part(partial, (int64_t)gridDim.x * H * max_splits, r, ((int64_t)t * H + h) * max_splits + split);
+    if (tid == 0) { part.max_sum[0] = m; part.max_sum[1] = l; }
 #pragma unroll
     for (int k = 0; k < kLatAcc; ++k) {
       const int d = tid + k * 256;
-      if (d < r) part[2 + d] = acc[k];
+      if (d < r) part.acc[d] = acc[k];
     }
   }
 }
 
+// Four waves per row, each with every fourth split and all of the row's latent dims, four splits' loads in flight per lane; the waves'
+// sums meet in LDS in wave order.  (A thread per dim that walked the splits one after another: 16 rows of 512 dims over 29 splits,
+// 4 tokens, 9.1 us; now 6.0 us.)
 __global__ __launch_bounds__(256) void latent_attn_merge_kernel(float* __restrict__ o_lat, const float* __restrict__ partial,
                                                                 const int32_t* __restrict__ positions, int H, int r,
                                                                 int max_splits, LatentCut cut) {
-  extern __shared__ float wsm[];   // [n_splits] weights exp(m_s - m) / l
-  __shared__ float red[4];
-  const int t = blockIdx.x, h = blockIdx.y;
+  extern __shared__ __attribute__((aligned(16))) float wsm[];   // [3][256] sums of waves 1 .. 3, then [n_splits] weights exp(m_s - m)
+  const int t = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n_splits = cut.splits_of(positions[t] + 1, max_splits);
   if (n_splits <= 1) return;
-  const float* part = partial + ((int64_t)t * H + h) * max_splits * (r + 2);
-  // the splits' maxima and sums are read in parallel (one thread each), combined in split order
-  float mloc = -INFINITY;
-  for (int s = threadIdx.x; s < n_splits; s += 256) mloc = fmaxf(mloc, part[(int64_t)s * (r + 2)]);
-  const float m = block_max256(mloc, red);
-  for (int s = threadIdx.x; s < n_splits; s += 256) wsm[s] = expf(part[(int64_t)s * (r + 2)] - m);
-  __syncthreads();
+  const LatentPartial part(partial, (int64_t)gridDim.x * H * max_splits, r, ((int64_t)t * H + h) * max_splits);
+  float* weight = wsm + 3 * 256;
+  float m = -INFINITY;                      // every wave reads the splits' maxima and sums itself
+  for (int s = lane; s < n_splits; s += 64) m = fmaxf(m, part.max_sum[2 * s]);
+  m = wave_max(m);
   float l = 0.f;
-  for (int s = 0; s < n_splits; ++s) l += part[(int64_t)s * (r + 2) + 1] * wsm[s];
-  const float inv = 1.0f / l;
-  for (int d = threadIdx.x; d < r; d += 256) {
-    float a = 0.f;
-#pragma unroll 4
-    for (int s = 0; s < n_splits; ++s) a = fmaf(part[(int64_t)s * (r + 2) + 2 + d], wsm[s], a);
-    o_lat[((int64_t)t * H + h) * r + d] = a * inv;
+  for (int s = lane; s < n_splits; s += 64) {
+    const float w = expf(part.max_sum[2 * s] - m);
+    l = fmaf(part.max_sum[2 * s + 1], w, l);
+    if (wave == 0) weight[s] = w;
+  }
+  const float inv = 1.0f / wave_sum(l);
+  __syncthreads();
+  const bool vec = (r & 3) == 0;
+  for (int d0 = 0; d0 < r; d0 += 256) {
+    const int d = d0 + lane * 4;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    if (d < r) {
+      int s = wave;
+      for (; s + 12 < n_splits; s += 16) {
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = part.load(s + 4 * u, d, vec);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a += v[u] * weight[s + 4 * u];
+      }
+      for (; s < n_splits; s += 4) a += part.load(s, d, vec) * weight[s];
+    }
+    if (wave > 0) *reinterpret_cast<f32x4*>(wsm + (wave - 1) * 256 + lane * 4) = a;
+    __syncthreads();
+    if (wave == 0 && d < r) {
+#pragma unroll
+      for (int w = 0; w < 3; ++w) a += *reinterpret_cast<const f32x4*>(wsm + w * 256 + lane * 4);
+      float* o = o_lat + ((int64_t)t * H + h) * r + d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (d + e < r) o[e] = a[e] * inv;
+    }
+    __syncthreads();
   }
 }
 
@@ -238,8 +283,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
                                                                const int32_t* __restrict__ page_ids,
                                                                const int32_t* __restrict__ tile_row0,
                                                                const int32_t* __restrict__ tile_rows, int H, int r, int dr,
-                                                               float scale, float* __restrict__ partial, int max_splits,
-                                                               LatentCut cut) {
+                                                               float scale, float* __restrict__ partial, int n_tokens,
+                                                               int max_splits, LatentCut cut) {
   extern __shared__ __align__(16) uint8_t lat_smem[];
   typedef short v4s_t __attribute__((ext_vector_type(4)));
   const int E = r + dr, Epad = (E + 31) & ~31;
@@ -392,31 +437,302 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
       if (dd < r) *reinterpret_cast<f32x4*>(o_lat + grow * r + dd) = o[d] * inv;
     }
   } else if (split < own_splits) {
-    float* part = partial + (grow * max_splits + split) * (r + 2);
-    if (g == 0) { part[0] = m; part[1] = l; }
+    const LatentPartial part(partial, (int64_t)n_tokens * H * max_splits, r, grow * max_splits + split);
+    if (g == 0) { part.max_sum[0] = m; part.max_sum[1] = l; }
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
       const int dd = d * 16 + 4 * g;
-      if (dd < r) { part[2 + dd] = o[d][0]; part[3 + dd] = o[d][1]; part[4 + dd] = o[d][2]; part[5 + dd] = o[d][3]; }
+      if (dd < r) *reinterpret_cast<f32x4*>(part.acc + dd) = o[d];
     }
   }
 }
 
-template <int ND>
-static void latent_attn_mfma_launch(const float* qc, float* o_lat, const uint16_t* cache, int64_t page_stride, int64_t layer_off,
-                                    int page_size, const int32_t* positions, const int32_t* token_req,
-                                    const int32_t* page_indptr, const int32_t* page_ids, const int32_t* tile_row0,
-                                    const int32_t* tile_rows, int n_tiles, int H, int r, int dr, float scale, float* ws, int sp,
-                                    LatentCut cut, hipStream_t s) {
-  const int Epad = (r + dr + 31) & ~31;
-  const int lds = (kTileRows + kTileKeys) * (Epad + 8) * 2;
-  auto kern = &latent_attn_mfma_kernel<ND>;
-  static const bool once = (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                160 * 1024), true);
-  (void)once;
-  kern<<<dim3(n_tiles, sp), 256, lds, s>>>(qc, o_lat, cache, page_stride, layer_off, page_size, positions, token_req, page_indptr,
-                                           page_ids, tile_row0, tile_rows, H, r, dr, scale, ws, sp, cut);
+// ------------------------------------------------------------------ few-rows form (decoding, and every tile of an fp32 cache)
+// The form above gives each wave sixteen rows of its own: a decoded token's sixteen heads then keep one wave of four busy, alone on its
+// SIMD, with 2 x 18 dependent products for the scores and 64 transposed reads for the values of every key tile.  Here the four waves share
+// the same 16 RB rows: wave w takes every fourth block of the entry for the scores (the four parts meet in LDS, added in wave order),
+// eight threads per row take the softmax of the tile, and wave w takes every fourth block of latent dims of the values.  Queries
+// stay in registers (a wave's own quarter of the entry), so LDS holds the key tile and the tile's scores alone.
+// The fp32 instance works on v_mfma_f32_16x16x4_f32: lane (l15, g) fetches four neighbouring values at 4 g of a 16-wide block with one
+// 16-byte read, and product e of the block takes value e of every lane - both operands numbered alike; its weights stay fp32.
+// Bound by the latency of one pass through scores, softmax and values (three barriers per tile of 32 keys), not by memory.
+// With the merge, 16 heads of 512 + 64 and 4 requests of 500 to 900 keys in splits of 32: 17.1 (the form above) -> 15.9 us, 32 requests
+// 53.6 -> 35.0 us.  In fp32, where a workgroup took one head and a thread one key: 8 heads of 256 + 64, two requests of up to 300 keys
+// 54 -> 14 us, their 470 prompt tokens 228 -> 66 us.
+template <typename A, int ND, int RB>
+__global__ __launch_bounds__(256) void latent_attn_few_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
+                                                              const A* __restrict__ cache, int64_t page_stride, int64_t layer_off,
+                                                              int page_size, const int32_t* __restrict__ positions,
+                                                              const int32_t* __restrict__ token_req,
+                                                              const int32_t* __restrict__ page_indptr,
+                                                              const int32_t* __restrict__ page_ids,
+                                                              const int32_t* __restrict__ tile_row0,
+                                                              const int32_t* __restrict__ tile_rows, int H, int r, int dr, float scale,
+                                                              float* __restrict__ partial, int n_tokens, int max_splits, LatentCut cut) {
+  typedef short v4s_t __attribute__((ext_vector_type(4)));
+  constexpr bool F32 = std::is_same<A, float>::value;
+  constexpr int kRows = 16 * RB;
+  constexpr int kPer = 16 / (int)sizeof(A);               // values of a 16-byte chunk
+  constexpr int KB = F32 ? 16 : 32;                       // width of a score block
+  constexpr int kMaxE = ND <= 4 ? 384 : 640;              // widest entry of this instance (latent_few_shape)
+  constexpr int NB = (kMaxE / KB + 3) / 4;                // blocks of a wave at most
+  constexpr int NP = kTileKeys * kMaxE / kPer / 256;      // chunks of a key tile per thread
+  constexpr int kSStride = kTileKeys + 4;
+  extern __shared__ __align__(16) uint8_t lat_smem[];
+  const int E = r + dr, Epad = (E + KB - 1) / KB * KB, cs = Epad + kPer;      // a row's LDS stride: 16 bytes past a multiple of 64
+  A* Ck = reinterpret_cast<A*>(lat_smem);                                      // [32][cs]
+  float* S = reinterpret_cast<float*>(Ck + kTileKeys * cs);                    // [4][kRows][kSStride] parts of the scores
+  A* P = reinterpret_cast<A*>(S + 4 * kRows * kSStride);                       // [kRows][kSStride] weights
+  float* s_row = reinterpret_cast<float*>(P + kRows * kSStride);               // [kRows] rescale of the tile, at the end 1 / sum
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  const int tile = blockIdx.x, sub = blockIdx.z, split = blockIdx.y;
+  const int cnt = min(kRows, tile_rows[tile] - sub * kRows);
+  if (cnt <= 0) return;
+  const int row0 = tile_row0[tile] + sub * kRows;
+  const int t_first = row0 / H, t_last = (row0 + cnt - 1) / H;
+  const int pmax = positions[t_last];
+  const int j_lo = split * cut.grain;
+  if (j_lo > pmax) return;
+  const int j_hi = cut.end_of(split, pmax + 1), j_step = cut.step(kTileKeys, max_splits);
+  const int32_t* pages = page_ids + page_indptr[token_req[t_first]];
+  const int nchunk = E / kPer, tile_chunks = kTileKeys * nchunk;
+  u32x4 pre[NP];
+  int ck_kk[NP], ck_el[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int c = tid + i * 256;
+    ck_kk[i] = c < tile_chunks ? c / nchunk : -1;
+    ck_el[i] = c < tile_chunks ? (c - ck_kk[i] * nchunk) * kPer : 0;
+  }
+  const int pshift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if (ck_kk[i] >= 0) {
+        const int j = min(j0 + ck_kk[i], j_hi - 1);
+        const int pg = pshift >= 0 ? j >> pshift : j / page_size;
+        const int slot = pshift >= 0 ? j & (page_size - 1) : j - pg * page_size;
+        pre[i] = *reinterpret_cast<const u32x4*>(cache + (int64_t)pages[pg] * page_stride + layer_off + (int64_t)slot * E + ck_el[i]);
+      }
+    }
+  };
+  fetch(j_lo);
+  // this wave's blocks of the queries: fp32 values 4 g .. of a block of 16, or bf16 values 8 g .. of a block of 32
+  const int blocks = Epad / KB;
+  u32x4 q[RB][NB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      q[rb][b] = u32x4{0u, 0u, 0u, 0u};
+      const int k = (wave + 4 * b) * KB + g * kPer, row = rb * 16 + l15;
+      if (row < cnt && k < E) {
+        const float* src = qc + (int64_t)(row0 + row) * E + k;
+        if constexpr (F32) q[rb][b] = *reinterpret_cast<const u32x4*>(src);
+        else {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(src), c = *reinterpret_cast<const f32x4*>(src + 4);
+          q[rb][b] = u32x4{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(c.x, c.y), pack_bf2(c.z, c.w)};
+        }
+      }
+    }
+  for (int i = tid; i < kTileKeys * (Epad - E); i += 256) Ck[(i / (Epad - E)) * cs + E + i % (Epad - E)] = 0;
+  // softmax: eight threads per row, four keys each
+  const int my_row = tid >> 3, my_key = 4 * (tid & 7);
+  const bool sm_live = my_row < cnt;                       // whole groups of eight lanes
+  const int pq = sm_live ? positions[(row0 + my_row) / H] : -1;
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[RB][ND];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[rb][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int j0 = j_lo; j0 < j_hi; j0 += j_step) {
+    __syncthreads();                                       // the previous tile's values are read
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (ck_kk[i] >= 0) *reinterpret_cast<u32x4*>(Ck + ck_kk[i] * cs + ck_el[i]) = pre[i];
+    __syncthreads();
+    if (j0 + j_step < j_hi) fetch(j0 + j_step);
+    {
+      f32x4 s[RB][2];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) s[rb][0] = s[rb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        if (wave + 4 * b >= blocks) break;
+        const A* kp = Ck + l15 * cs + (wave + 4 * b) * KB + g * kPer;
+        const u32x4 k0 = *reinterpret_cast<const u32x4*>(kp), k1 = *reinterpret_cast<const u32x4*>(kp + 16 * cs);
+        if constexpr (F32) {
+          const f32x4 f0 = __builtin_bit_cast(f32x4, k0), f1 = __builtin_bit_cast(f32x4, k1);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+              const f32x4 qv = __builtin_bit_cast(f32x4, q[rb][b]);
+              s[rb][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(f0[e], qv[e], s[rb][0], 0, 0, 0);
+              s[rb][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f1[e], qv[e], s[rb][1], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) {
+            const bf16x8_t qv = __builtin_bit_cast(bf16x8_t, q[rb][b]);
+            s[rb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, k0), qv, s[rb][0], 0, 0, 0);
+            s[rb][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, k1), qv, s[rb][1], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          *reinterpret_cast<f32x4*>(S + (wave * kRows + rb * 16 + l15) * kSStride + 16 * kb + 4 * g) = s[rb][kb];
+    }
+    __syncthreads();
+    if (my_row < kRows) {                                  // whole waves
+      f32x4 v = *reinterpret_cast<const f32x4*>(S + my_row * kSStride + my_key);
+#pragma unroll
+      for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(S + (w * kRows + my_row) * kSStride + my_key);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = j0 + my_key + e;
+        v[e] = j <= pq && j < j_hi ? v[e] * scale : -INFINITY;
+        mx = fmaxf(mx, v[e]);
+      }
+#pragma unroll
+      for (int x = 1; x < 8; x <<= 1) mx = fmaxf(mx, __shfl_xor(mx, x, kWave));
+      const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float corr = F32 ? expf(m - m_use) : __expf(m - m_use);
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = F32 ? expf(v[e] - m_use) : bf16_round_f(__expf(v[e] - m_use));   // the sum uses the weights as the matrix core sees them
+        sum += v[e];
+      }
+#pragma unroll
+      for (int x = 1; x < 8; x <<= 1) sum += __shfl_xor(sum, x, kWave);
+      l = l * corr + sum;
+      m = m_new;
+      if constexpr (F32) *reinterpret_cast<f32x4*>(P + my_row * kSStride + my_key) = v;
+      else *reinterpret_cast<u32x2*>(P + my_row * kSStride + my_key) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      if ((tid & 7) == 0) s_row[my_row] = corr;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const float corr = s_row[rb * 16 + l15];
+      if (__any(corr != 1.0f)) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) o[rb][d] *= corr;
+      }
+    }
+    if constexpr (F32) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        f32x4 p[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) p[rb] = *reinterpret_cast<const f32x4*>(P + (rb * 16 + l15) * kSStride + 16 * kb + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int d = 0; d < ND; ++d) {
+            const int dd = (wave + 4 * d) * 16;
+            if (dd >= r) break;
+            const float c = Ck[(16 * kb + 4 * g + e) * cs + dd + l15];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) o[rb][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(c, p[rb][e], o[rb][d], 0, 0, 0);
+          }
+      }
+    } else {
+      bf16x8_t p[RB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const A* pp = P + (rb * 16 + l15) * kSStride + 4 * g;
+        const u32x2 a = *reinterpret_cast<const u32x2*>(pp), b = *reinterpret_cast<const u32x2*>(pp + 16);
+        p[rb] = __builtin_bit_cast(bf16x8_t, u32x4{a.x, a.y, b.x, b.y});
+      }
+      const __attribute__((address_space(3))) uint16_t* ck3 =
+          (const __attribute__((address_space(3))) uint16_t*)(Ck) + (4 * g + (l15 >> 2)) * cs + 4 * (l15 & 3);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const int dd = (wave + 4 * d) * 16;
+        if (dd >= r) break;
+        const v4s_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + dd));
+        const v4s_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + dd + 16 * cs));
+        const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
+        const bf16x8_t cv = __builtin_bit_cast(bf16x8_t, u32x4{w0.x, w0.y, w1.x, w1.y});
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) o[rb][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cv, p[rb], o[rb][d], 0, 0, 0);
+      }
+    }
+  }
+  const int64_t slots = (int64_t)n_tokens * H * max_splits;
+  __syncthreads();                                         // the last tile's rescales are read
+  if (sm_live && (tid & 7) == 0) s_row[my_row] = 1.0f / l;
+  __syncthreads();
+  if (sm_live && (tid & 7) == 0 && cut.splits_of(pq + 1, max_splits) > max(1, split)) {
+    const LatentPartial part(partial, slots, r, (int64_t)(row0 + my_row) * max_splits + split);
+    part.max_sum[0] = m;
+    part.max_sum[1] = l;
+  }
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int row = rb * 16 + l15;
+    if (row >= cnt) continue;
+    const int own_splits = cut.splits_of(positions[(row0 + row) / H] + 1, max_splits);
+    if (split >= own_splits) continue;
+    const bool whole = own_splits == 1;
+    const float inv = whole ? s_row[row] : 1.0f;
+    float* dst = whole ? o_lat + (int64_t)(row0 + row) * r
+                       : LatentPartial(partial, slots, r, (int64_t)(row0 + row) * max_splits + split).acc;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const int dd = (wave + 4 * d) * 16 + 4 * g;
+      if (dd < r) *reinterpret_cast<f32x4*>(dst + dd) = o[rb][d] * inv;
+    }
+  }
 }
+
+// One call's tiled form.  An fp32 cache always takes the few-rows form.  A bf16 cache takes it when the tiles hold no more than 16 rows
+// on average, measured against the 64-row form (512 + 64, splits of 32, with the merge): 4 requests of 16 heads 15.9 / 17.1 us,
+// 32 of them 35.0 / 53.6; at 32 rows per tile there is nothing between them (20.0 / 20.3, 37.8 / 37.5), at 64 the other is faster
+// (35.7 / 30.0, a prompt of 1800 tokens 303 / 257).
+struct LatentCall {
+  const float* qc; float* o_lat;
+  const void* cache; int64_t page_stride, layer_off; int page_size;
+  const int32_t *positions, *token_req, *page_indptr, *page_ids, *tile_row0, *tile_rows;
+  int n_tiles, H, r, dr; float scale; float* ws; int n_tokens, sp; LatentCut cut; hipStream_t s;
+
+  template <typename A, typename K>
+  void run(K kern, int subs, size_t lds) const {
+    if (lds > 48 * 1024)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    kern<<<dim3(n_tiles, sp, subs), 256, lds, s>>>(qc, o_lat, static_cast<const A*>(cache), page_stride, layer_off, page_size, positions, token_req,
+                                           page_indptr, page_ids, tile_row0, tile_rows, H, r, dr, scale, ws, n_tokens, sp, cut);
+  }
+  template <int ND>
+  void wide() const {
+    const int Epad = (r + dr + 31) & ~31;
+    run<uint16_t>(&latent_attn_mfma_kernel<ND>, 1, (size_t)(kTileRows + kTileKeys) * (Epad + 8) * 2);
+  }
+  template <typename A, int ND, int RB>
+  void few_rows() const {
+    constexpr int kRows = 16 * RB, KB = std::is_same<A, float>::value ? 16 : 32;
+    const size_t cs = (r + dr + KB - 1) / KB * KB + 16 / sizeof(A);
+    // the parts of a tile past its rows come last: between the others they would take those from some of the XCDs' turns
+    run<A>(&latent_attn_few_kernel<A, ND, RB>, kTileRows / kRows,
+           (kTileKeys * cs + kRows * (kTileKeys + 4)) * sizeof(A) + (4 * kRows * (kTileKeys + 4) + kRows) * sizeof(float));
+  }
+  bool narrow() const { return (int64_t)n_tokens * H <= 16 * (int64_t)n_tiles; }
+  template <typename A>
+  void few() const {
+    const bool small = r <= 256 && r + dr <= 384;
+    if constexpr (std::is_same<A, float>::value) {
+      if (!narrow()) return small ? few_rows<A, 4, 2>() : few_rows<A, 8, 2>();
+    }
+    small ? few_rows<A, 4, 1>() : few_rows<A, 8, 1>();
+  }
+};
 
 static inline int latent_split_keys(int split_keys) { return split_keys > 0 ? split_keys : kLatSplitKeys; }
 static inline int latent_max_splits(int max_kv_len, int split_keys) {
@@ -477,9 +793,10 @@ int64_t pegainfer_latent_attention_workspace(int32_t n_tokens, int32_t heads, in
 }
 
 int32_t pegainfer_latent_attention_tiled_ok(int32_t rank, int32_t rot, int64_t page_stride, int64_t layer_off, int32_t dtype) {
-  const int Epad = (rank + rot + 31) & ~31;
-  return dtype == kDtBf16 && rank % 16 == 0 && rank <= 512 && rot % 8 == 0 && page_stride % 8 == 0 && layer_off % 8 == 0 &&
-         kTileKeys * ((rank + rot) / 8) <= kLatPrefetch * 256 && (kTileRows + kTileKeys) * (Epad + 8) * 2 <= 160 * 1024;
+  // the entry's limit is the key tile's: 640 values (20 chunks of 16 bytes per thread in fp32, kLatPrefetch in bf16)
+  const int chunk = dtype == kDtF32 ? 4 : 8;
+  return (dtype == kDtBf16 || dtype == kDtF32) && rank % 16 == 0 && rank <= 512 && rot % chunk == 0 && rank + rot <= 640 &&
+         page_stride % chunk == 0 && layer_off % chunk == 0;
 }
 
 // one launch (and its merge) with the keys cut as `cut` says into `sp` splits at most
@@ -495,14 +812,14 @@ static pegainfer_status_t latent_attention_launch(const float* qc, float* o_lat,
     if (!tile_rows || n_tiles <= 0 || !pegainfer_latent_attention_tiled_ok(rank, rot, page_stride, layer_off, dtype) ||
         (reinterpret_cast<uintptr_t>(cache) & 15u))
       return (pegainfer_status_t)hipErrorInvalidValue;
-    const uint16_t* c = static_cast<const uint16_t*>(cache);
-#define LAT_LAUNCH(ND) latent_attn_mfma_launch<ND>(qc, o_lat, c, page_stride, layer_off, page_size, positions, token_req, page_indptr, \
-                                                   page_ids, tile_row0, tile_rows, n_tiles, heads, rank, rot, scale, workspace, sp, cut, s)
-    if (rank <= 64) LAT_LAUNCH(4);
-    else if (rank <= 128) LAT_LAUNCH(8);
-    else if (rank <= 256) LAT_LAUNCH(16);
-    else LAT_LAUNCH(32);
-#undef LAT_LAUNCH
+    const LatentCall c{qc, o_lat, cache, page_stride, layer_off, page_size, positions, token_req, page_indptr, page_ids, tile_row0, tile_rows,
+                       n_tiles, heads, rank, rot, scale, workspace, n_tokens, sp, cut, s};
+    if (dtype == kDtF32) c.few<float>();
+    else if (c.narrow()) c.few<uint16_t>();
+    else if (rank <= 64) c.wide<4>();
+    else if (rank <= 128) c.wide<8>();
+    else if (rank <= 256) c.wide<16>();
+    else c.wide<32>();
   } else {
     if (rank > kLatAcc * 256) return (pegainfer_status_t)hipErrorInvalidValue;
     const size_t smem = (size_t)(rank + rot + kLatKeys) * sizeof(float);
@@ -516,7 +833,7 @@ static pegainfer_status_t latent_attention_launch(const float* qc, float* o_lat,
         }))
       return (pegainfer_status_t)hipErrorInvalidValue;
   }
-  if (sp > 1) latent_attn_merge_kernel<<<dim3(n_tokens, heads), 256, (size_t)sp * sizeof(float), s>>>(o_lat, workspace, positions, heads, rank, sp, cut);
+  if (sp > 1) latent_attn_merge_kernel<<<dim3(n_tokens, heads), 256, (3 * 256 + (size_t)sp) * sizeof(float), s>>>(o_lat, workspace, positions, heads, rank, sp, cut);
   return (pegainfer_status_t)hipGetLastError();
 }
 

@@ -285,6 +285,48 @@ def test_latent_attention_matrix_core_form(shape, split_keys):
     assert float((o - plain).abs().mean()) < 2e-3
 
 
+@pytest.mark.parametrize("split_keys", [0, 32, -3])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("shape", [(8, 256, 64, [1, 1, 1]), (16, 512, 64, [1, 1]), (3, 16, 8, [5, 1, 9]), (40, 512, 128, [1]), (5, 272, 24, [3, 13, 1]),
+                                   (24, 64, 0, [1, 1]), (64, 128, 64, [3])])
+def test_latent_attention_few_rows_form(shape, dtype, split_keys):
+    """tiles of a few rows (and any tile of an fp32 cache): one to four blocks of sixteen rows, entries that end inside a block, portions
+    deep inside a context; split_keys < 0: the keys dealt to that many workgroups.  In fp32 the sums of at most 640 products of about
+    one each and of 300 weights stay within 2e-5; q and the weights are rounded to bf16 in the other instance."""
+    from pegainfer_amd import ops_blocks as B
+    H, r, dr, lens = shape
+    g = torch.Generator().manual_seed(H * 10 + r)
+    E, ps = r + dr, 16
+    starts = [0, 290, 33][:len(lens)]
+    ctx = [s + n for s, n in zip(starts, lens)]
+    ent = [C.bf16_round(torch.randn(n, E, generator=g) * 0.7) for n in ctx]
+    npages = [(n + ps - 1) // ps for n in ctx]
+    pool = torch.full((sum(npages), ps, E), float("nan"))                  # slots past an entry's context are never used
+    order = np.random.default_rng(H).permutation(sum(npages))
+    page_lists, at = [], 0
+    for e, k in zip(ent, npages):
+        page_lists.append([int(x) for x in order[at:at + k]])
+        at += k
+        for j in range(len(e)):
+            pool[page_lists[-1][j // ps], j % ps] = e[j]
+    pos = [s + k for s, n in zip(starts, lens) for k in range(n)]
+    req = [i for i, n in enumerate(lens) for _ in range(n)]
+    qc = torch.randn(len(pos), H, E, generator=g) / E ** 0.5
+    indptr = torch.tensor(np.cumsum([0] + npages).astype(np.int32)).cuda()
+    ids = torch.tensor(sum(page_lists, []), dtype=torch.int32).cuda()
+    cache, tiles = dev(pool, DT[dtype]), B.row_tiles(lens, H)
+    if split_keys < 0:
+        o = B.latent_attention_dealt(dev(qc), cache, ps * E, 0, ps, B.Ragged(lens, starts=starts), indptr, ids, r, dr, 2.0, n_split=-split_keys, tiles=tiles)
+    else:
+        o = B.latent_attention(dev(qc), cache, ps * E, 0, ps, torch.tensor(pos, dtype=torch.int32).cuda(),
+                               torch.tensor(req, dtype=torch.int32).cuda(), indptr, ids, r, dr, 2.0, max(ctx), split_keys=split_keys, tiles=tiles)
+    tol = 2e-5 if dtype == "float32" else 2.5e-2
+    for i in range(len(pos)):
+        e = ent[req[i]][:pos[i] + 1].double()
+        ref = torch.softmax(torch.einsum("he,je->hj", qc[i].double(), e) * 2.0, -1) @ e[:, :r]
+        assert (o[i].cpu().double() - ref).abs().max() < tol, (i, pos[i], float((o[i].cpu().double() - ref).abs().max()))
+
+
 def ffi_ok(B, r, dr, page_stride):
     from pegainfer_amd import ffi
     return ffi.lib().pegainfer_latent_attention_tiled_ok(r, dr, page_stride, 0, 0) == 1
