@@ -19,6 +19,11 @@ extern "C" {
  * extract_vec + flashinfer_top1_cuda + sync + D2H: executor.rs:324-328, ops/sampling.rs:122-168).
  * state_scratch: rows*16 bytes, zeroed once by the caller, left zeroed.  Ties -> lowest index. */
 pegainfer_status_t pegainfer_batched_top1(const Half* logits, int32_t vocab_size, int32_t rows, int64_t row_stride, uint8_t* state_scratch, int32_t* out_tokens, pegainfer_stream_t stream);
+/* gpu_sample_flashinfer_cuda's draw (same token from the same logits, filters and seed) over many workgroups.  scratch:
+ * pegainfer_sample_scratch_bytes(vocab_size) bytes on 16 bytes, any contents; its first vocab_size floats hold the probabilities
+ * afterwards.  One call at a time per scratch. */
+int64_t pegainfer_sample_scratch_bytes(int32_t vocab_size);
+pegainfer_status_t pegainfer_sample(const Half* logits, void* scratch, uint8_t* valid_scratch, int32_t* output, int32_t vocab_size, float inv_temperature, int32_t top_k, float top_p, uint64_t seed, pegainfer_stream_t stream);
 
 /* Decode GEMM (T <= 64 token columns, weights streamed once) with optional prologue / epilogue fused in; same
  * accumulation cores as gemm_graphsafe_cuda (dot2 GEMV at T <= 2, skinny MFMA GEMM at 3 <= T <= 16, the tiled

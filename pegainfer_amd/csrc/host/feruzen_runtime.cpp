@@ -152,7 +152,7 @@ struct Model {
   int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
   uint8_t *meta_host = nullptr, *meta_dev = nullptr;
-  float* probs_scratch = nullptr;
+  uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -381,7 +381,7 @@ struct Model {
     if (any_fast && (dalloc(&split_tmp_v, (size_t)max_requests * pq::kSplitMaxChunksPerRequest * (size_t)std::max(1, mx_q)) ||
                      dalloc(&split_tmp_s, (size_t)max_requests * pq::kSplitMaxChunksPerRequest * (size_t)std::max(1, mx_q))))
       return -1;
-    if (dalloc(&probs_scratch, (size_t)V) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
+    if (dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
         dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1))
       return -1;
     return 0;
@@ -1094,7 +1094,7 @@ struct Model {
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      gpu_sample_flashinfer_cuda(lg, probs_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S());
+      FZ_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
     }
     FZ_HIP(hipStreamSynchronize(stream));
     FZ_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));

@@ -168,7 +168,7 @@ struct Model {
   int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
   uint8_t *meta_host = nullptr, *meta_dev = nullptr;
-  float* probs_scratch = nullptr;
+  uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -398,7 +398,7 @@ struct Model {
     requests.assign((size_t)max_requests, KvState());
     if (dalloc_a(&cache, (size_t)num_pages * (size_t)page_stride)) return -1;
     if (dalloc(&state, (size_t)max_requests * (size_t)std::max<int64_t>(1, state_layout.floats_per_slot()))) return -1;
-    if (dalloc(&probs_scratch, (size_t)V) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
+    if (dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
         dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1))
       return -1;
     return 0;
@@ -1020,7 +1020,7 @@ struct Model {
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      gpu_sample_flashinfer_cuda(lg, probs_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S());
+      KK_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
     }
     KK_HIP(hipStreamSynchronize(stream));
     KK_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));

@@ -107,7 +107,7 @@ struct Model35 {
   // per-request sampling / logprobs over the LAST step's logits (ops/sampling.rs:109-170, executor.rs:400-434)
   const Half* last_logits = nullptr;
   int last_rows = 0;
-  float* probs_scratch = nullptr;
+  uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -234,7 +234,7 @@ struct Model35 {
         dalloc(&a_proj, bs * vh) || dalloc(&gdr_out, bs * Z) || dalloc(&normed_gated, bs * Z) ||
         dalloc(&gate_out, bs * I) || dalloc(&up_out, bs * I) || dalloc(&act_out, bs * I) ||
         dalloc(&mlp_out, bs * H) || dalloc(&logits, bs * (size_t)V) ||
-        dalloc(&top1_state, bs * 16) || dalloc(&start_pos_d, 1) || dalloc(&probs_scratch, (size_t)V) || dalloc(&top1_value, 1) ||
+        dalloc(&top1_state, bs * 16) || dalloc(&start_pos_d, 1) || dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) ||
         dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1) ||
         dalloc(&wide, (size_t)kFusedBatch * std::max(C + Z + 2 * vh, 2 * q_dim + 2 * kv_dim)) ||
         dalloc(&split_tmp_v, bs * pq::kSplitMaxChunksPerRequest * q_dim) ||
@@ -919,8 +919,8 @@ struct Model35 {
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      gpu_sample_flashinfer_cuda(lg, probs_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
-                                 (uint64_t)bits, S());
+      P35_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
+                                          (uint64_t)bits, S()));
     }
     P35_HIP(hipStreamSynchronize(stream));
     P35_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));

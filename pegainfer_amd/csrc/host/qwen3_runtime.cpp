@@ -119,7 +119,7 @@ struct Model {
   bool oproj_plan = false;   // this step's split plan keeps the padding slots the fused launch needs (single request, <= 2304 tokens)
   int oproj_fallbacks = 0;
   // sampling scratch (ops/sampling.rs)
-  float* probs_scratch = nullptr;
+  uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t* row_states = nullptr;
   uint8_t* valid_scratch = nullptr;
@@ -227,7 +227,7 @@ struct Model {
         dalloc(&mlp_act, bs * I) || dalloc(&mlp_out, bs * H) || dalloc(&hidden, bs * H) ||
         dalloc(&hidden2, bs * H) || dalloc(&qkv_out, bs * (size_t)(q_dim + 2 * kv_dim)) ||
         dalloc(&logits, bs * (size_t)V) || dalloc(&split_tmp_v, slots * q_dim) || dalloc(&split_tmp_s, slots * Hq) ||
-        dalloc(&top1_state, bs * 16) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&probs_scratch, (size_t)V) ||
+        dalloc(&top1_state, bs * 16) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) ||
         dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) ||
         dalloc(&sample_out_d, 1))
       return -1;
@@ -1356,8 +1356,8 @@ struct Model {
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      gpu_sample_flashinfer_cuda(lg, probs_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
-                                 (uint64_t)bits, S());
+      PQ_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
+                                          (uint64_t)bits, S()));
     }
     PQ_HIP(hipStreamSynchronize(stream));
     PQ_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));

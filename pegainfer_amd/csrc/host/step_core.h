@@ -171,7 +171,7 @@ class StepModel {
     last_token.assign((size_t)max_requests, -1);
     if (dalloc_a(&cache, (size_t)num_pages * (size_t)page_stride)) return -1;
     if (dalloc(&state, (size_t)max_requests * (size_t)std::max<int64_t>(1, state_layout.floats_per_slot()))) return -1;
-    return dalloc(&probs_scratch, (size_t)V) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
+    return dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
            dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1) ? -1 : 0;
   }
 
@@ -399,7 +399,7 @@ class StepModel {
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      gpu_sample_flashinfer_cuda(lg, probs_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S());
+      PSTEP_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
     }
     PSTEP_HIP(hipStreamSynchronize(stream));
     PSTEP_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));
@@ -612,7 +612,8 @@ class StepModel {
   Half *logits16 = nullptr, *top1_value = nullptr;
   int32_t *tokens_d = nullptr, *sample_out_d = nullptr;
   uint8_t *top1_state = nullptr, *row_states = nullptr, *valid_scratch = nullptr;
-  float *probs_scratch = nullptr, *tap = nullptr;
+  float* tap = nullptr;
+  uint8_t* sample_scratch = nullptr;
   int last_rows = 0, tap_rows = 0;
   std::vector<float> lp_row;
 

@@ -661,3 +661,31 @@ def test_sampling_distribution(P):
             renorm = np.where(keep, ref, 0) / ref[keep].sum()
             freq = np.bincount(draws, minlength=n) / len(draws)
             assert np.abs(freq - renorm).max() < 0.08
+
+
+@pytest.mark.parametrize("n", [257, 24575, 24576, 24577, 32768, 65541, 151936, 262144 + 4, 300007])
+def test_sampling_over_many_workgroups_is_the_same_draw(P, n):
+    """pegainfer_sample against the one-workgroup kernel: same probabilities bit for bit and the same token, for every filter, for rows
+    off 16 bytes, one dominant value, equal values, infinities and no number at all; the scratch holds garbage before each call"""
+    import torch
+    from pegainfer_amd import ffi
+    L, g = ffi.lib(), torch.Generator().manual_seed(n)
+    s = torch.cuda.current_stream().cuda_stream
+    base = torch.randn(n + 8, generator=g) * 3.0
+    forms = {"random": base, "one": torch.where(torch.arange(n + 8) == n // 2, 60.0, base), "equal": torch.zeros(n + 8),
+             "cut": torch.where(torch.arange(n + 8) % 3 == 0, float("-inf"), base), "inf": torch.where(torch.arange(n + 8) == 5, float("inf"), base),
+             "none": torch.full((n + 8,), float("nan"))}
+    out = torch.zeros(2, dtype=torch.int32, device="cuda")
+    valid = torch.zeros(1, dtype=torch.uint8, device="cuda")
+    for name, x in forms.items():
+        for shift in (0, 1):
+            lg = x.to(torch.bfloat16).cuda()[shift:shift + n]
+            for i, (inv_t, k, p) in enumerate([(1.25, 50, 0.95), (1.0, -1, 0.9), (0.7, 20, 1.0), (1.0, -1, 1.0), (1.0, n, 1e-6), (2.0, 1, 0.5), (1.0, 3000, 0.999)]):
+                seed = 1000 * n + 17 * i + shift
+                ref = torch.zeros(n, dtype=torch.float32, device="cuda")
+                scratch = torch.full((int(L.pegainfer_sample_scratch_bytes(n)),), 0xA5, dtype=torch.uint8, device="cuda")
+                L.gpu_sample_flashinfer_cuda(lg.data_ptr(), ref.data_ptr(), valid.data_ptr(), out.data_ptr(), n, inv_t, k, p, seed, s)
+                assert L.pegainfer_sample(lg.data_ptr(), scratch.data_ptr(), valid.data_ptr(), out[1:].data_ptr(), n, inv_t, k, p, seed, s) == 0
+                got = scratch[:4 * n].view(torch.int32)
+                assert torch.equal(got, ref.view(torch.int32)), (name, shift, i)
+                assert int(out[0]) == int(out[1]), (name, shift, i, out.tolist())
