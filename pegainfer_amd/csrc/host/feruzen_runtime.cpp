@@ -1039,10 +1039,13 @@ struct Model {
     const MlpCfg& f = c.mlp;
     const int ff = f.glu.ff, P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
+    const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && ff % 8 == 0 ? 128 : 64;
     if (T > 8 || f.experts > 1024) {   // many rows (or more experts than the selection kernel's four rows hold in LDS): one
                                        // workgroup per row does logits and selection
       FZ_K(pegainfer_route_topk(xb, w.router, nullptr, route_e, route_w, D, f.experts, 1, 1, f.top, T, PEGAINFER_SCORE_SOFTMAX, dtype, S()));
-    } else {       // few rows (decoding): the few-rows GEMM streams the router with the whole chip into fp32 logits, then the selection
+      FZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
+    } else {       // few rows (decoding): the few-rows GEMM streams the router with the whole chip into fp32 logits, then selection and
+                   // sort in one launch
       pegainfer_gemm_desc r{};
       r.x = xb; r.w = w.router; r.y = route_logits;
       r.x_dtype = r.w_dtype = dtype; r.y_dtype = PEGAINFER_DTYPE_F32;
@@ -1050,10 +1053,14 @@ struct Model {
       r.x_row_stride = D; r.w_m_stride = D; r.w_k_stride = 1; r.y_row_stride = f.experts;
       r.plain = plain_kernels;
       FZ_K(pegainfer_gemm_strided(&r, S()));
-      FZ_K(pegainfer_route_from_logits(route_logits, nullptr, route_e, route_w, f.experts, 1, 1, f.top, T, PEGAINFER_SCORE_SOFTMAX, dtype, S()));
+      pegainfer_route_plan_desc q{};
+      q.logits = route_logits; q.logits_stride = f.experts; q.out_expert = route_e; q.out_weight = route_w;
+      q.experts = f.experts; q.n_groups = q.keep_groups = 1; q.top = f.top; q.rows = T; q.score_kind = PEGAINFER_SCORE_SOFTMAX; q.factor = 1.0f;
+      q.sort_experts = f.experts; q.pos_pair = pos_pair; q.pos_row = pos_row;
+      q.tile_group = t_group; q.tile_row0 = t_row0; q.tile_rows = t_rows; q.n_tiles = n_tiles;
+      q.max_tiles = max_tiles; q.rows_per_tile = per_tile; q.dtype = dtype;
+      FZ_K(pegainfer_route_plan(&q, S()));
     }
-    const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && ff % 8 == 0 ? 128 : 64;
-    FZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
     pegainfer_gemm_desc d{};
     d.x = xb; d.w = w.gate_up_e; d.y = gu_e;
     d.x_dtype = d.w_dtype = d.y_dtype = dtype;

@@ -1061,10 +1061,15 @@ struct Model {
     const int ff = f.ff, P = T * f.top, E1 = f.experts + 1;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     if (linear_strided(w.router, hb, dtype, D, route_logits, PEGAINFER_DTYPE_F32, E1, T, D)) return -1;
-    RX_K(pegainfer_route_from_logits_ex(route_logits, E1, nullptr, route_e, route_w, f.experts, f.groups, f.keep, f.top, T,
-                                        PEGAINFER_SCORE_SOFTMAX, PEGAINFER_GROUP_MAX, 1, dtype, S()));
     const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && ff % 8 == 0 ? 128 : 64;
-    RX_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
+    pegainfer_route_plan_desc r{};      // selection and sort: one launch for few rows
+    r.logits = route_logits; r.logits_stride = E1; r.out_expert = route_e; r.out_weight = route_w;
+    r.experts = f.experts; r.n_groups = f.groups; r.keep_groups = f.keep; r.top = f.top; r.rows = T;
+    r.score_kind = PEGAINFER_SCORE_SOFTMAX; r.group_kind = PEGAINFER_GROUP_MAX; r.renorm = 1; r.factor = 1.0f;
+    r.sort_experts = f.experts; r.pos_pair = pos_pair; r.pos_row = pos_row;
+    r.tile_group = t_group; r.tile_row0 = t_row0; r.tile_rows = t_rows; r.n_tiles = n_tiles;
+    r.max_tiles = max_tiles; r.rows_per_tile = per_tile; r.dtype = dtype;
+    RX_K(pegainfer_route_plan(&r, S()));
     pegainfer_gemm_desc d{};
     d.x = hb; d.w = w.gate_up_e; d.y = gu_e;
     d.x_dtype = d.w_dtype = d.y_dtype = dtype;

@@ -148,6 +148,36 @@ def test_router_chooses_by_corrected_and_weighs_by_plain_scores(dtype, rows, E, 
         assert sorted(covered) == list(range(n_real))
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17])
+@pytest.mark.parametrize("E,top", [(1, 1), (9, 9), (63, 5), (64, 64), (65, 4), (130, 70), (200, 3)])
+def test_router_at_the_edges_of_a_wave_with_ties_and_experts_out_of_reach(E, top, rows):
+    """values from a coarse grid (ties go to the lower index), corrections of minus infinity and no number (never chosen: expert 0 with
+    weight 0 fills the place), and the sort of the choices over one, two and four runs of 64 experts"""
+    g = torch.Generator().manual_seed(E)
+    z = torch.randint(-4, 5, (rows, E), generator=g).float() / 2
+    corr = torch.randint(-1, 2, (E,), generator=g).float() * 4
+    if E > 8:
+        corr[3], corr[5] = float("-inf"), float("nan")
+    for renorm, factor in ((True, 1.0), (False, 1.0), (False, 2.5), (True, 0.5)):
+        e, wt, s = B().route_plan(z.cuda(), E, top, E, correction=corr.cuda(), score="sigmoid", renorm=renorm, factor=factor, dtype=torch.float32)
+        e, wt = e.cpu(), wt.cpu().double()
+        for r in range(rows):
+            sc = torch.sigmoid(z[r].double())
+            order = sorted((i for i in range(E) if (sc[i] + corr[i]) > float("-inf")), key=lambda i: (-float(sc[i] + corr[i]), i))[:top]
+            w = torch.tensor([float(sc[i]) for i in order] + [0.0] * (top - len(order)), dtype=torch.float64)
+            if renorm:
+                w = w / (w.sum() + 1e-20)
+            assert e[r].tolist() == order + [0] * (top - len(order)), (r, renorm)
+            assert float((wt[r] - w * factor).abs().max()) < 1e-5
+        pp, nt, seen = s["pos_pair"].cpu(), int(s["n_tiles"]), []
+        assert sorted(pp.tolist()) == list(range(rows * top))
+        for t in range(nt):
+            x, r0, n = (int(s[k][t]) for k in ("tile_group", "tile_row0", "tile_rows"))
+            assert all(int(e.view(-1)[int(pp[i])]) == x for i in range(r0, r0 + n)) and 0 < n <= 64
+            seen += list(range(r0, r0 + n))
+        assert seen == list(range(rows * top))
+
+
 @BOTH
 @pytest.mark.parametrize("rows,d", [(3, 50), (20, 300), (260, 72)])
 def test_identity_experts_give_their_input(dtype, rows, d):
