@@ -500,6 +500,34 @@ typedef struct {
 int32_t pegainfer_decay_attention_chunked_ok(int32_t dim, int32_t vdim);
 int64_t pegainfer_decay_attention_workspace(int32_t n_chunks, int32_t heads, int32_t dim, int32_t vdim);
 pegainfer_status_t pegainfer_decay_attention(const pegainfer_decay_attention_desc* d, pegainfer_stream_t stream);
+/* The state-space scan with the entries of the tables in chunks of <= PEGAINFER_DECAY_CHUNK tokens side by side (the tables and scan_max
+ * as for pegainfer_decay_attention; everything stays fp32).  n_chunks or n_long 0: the scan takes every entry.
+ * workspace: pegainfer_ssd_scan_workspace(...) floats. */
+typedef struct {
+  const float* xbc;
+  int64_t xbc_stride;
+  const void* proj;
+  int64_t proj_stride, dt_off;
+  const void *A_log, *dt_bias, *D;
+  float* state;
+  int64_t slot_stride;
+  float* o;
+  int32_t heads, groups, n_state, vdim;
+  const int32_t* entry_row0;
+  const int32_t* entry_slot;
+  int32_t n_entries;
+  int32_t scan_max;
+  const int32_t* chunk_row0;
+  const int32_t* chunk_rows;
+  int32_t n_chunks;
+  const int32_t* long_chunk0;
+  const int32_t* long_slot;
+  int32_t n_long;
+  float* workspace;
+  int32_t dtype;
+} pegainfer_ssd_scan_desc;
+int64_t pegainfer_ssd_scan_workspace(int32_t n_chunks, int32_t heads, int32_t n_state, int32_t vdim);
+pegainfer_status_t pegainfer_ssd_scan_form(const pegainfer_ssd_scan_desc* d, pegainfer_stream_t stream);
 /* Gated linear attention: the same state with a decay per (head, key channel) and token that acts on the rows of S.
  * Per row of `proj` (dtype): q at q_off, k at k_off (heads x dim), v at v_off (heads x vdim);  z: fp32 [rows][heads * dim] at z_stride,
  * z_bias [heads * dim] of dtype or NULL:

@@ -85,6 +85,9 @@ constexpr int kPageSize = 16;   // tokens per cache page, as in the other runtim
 constexpr int kAttRows = 16;    // (token, query head) rows of one attention workgroup
 constexpr int kSplitGroups = 512;   // most (tile, kv head, key split) workgroups of an attention launch that cuts its keys
 constexpr int kMaxSplits = 16;
+// longest entry whose state-space scan runs token by token: 32 heads of 128 x 64, scan / chunks 27 / 41 us at 128 tokens, 48 / 44 at 256,
+// 91 / 50 at 512; eight entries of 128 tokens 56 / 65 us
+constexpr int kScanMax = 224;
 
 enum { kAttention = 1, kParallel = 2 };
 // softmax attention: the "attention" mixer and the left half of "parallel"
@@ -178,6 +181,8 @@ struct Model {
   float* tap = nullptr;
   size_t tap_cap = 0;
   int tap_rows = 0;
+  float* chunk_ws = nullptr;   // states between the chunks of long entries
+  size_t chunk_cap = 0;
   float* att_part = nullptr;   // softmax states of the key splits of an attention launch
   int mx_proj = 0, mx_mix = 0, mx_inner = 0, mx_conv = 0, mx_q = 0, mx_ff = 0, mx_vdim = 0;
 
@@ -710,6 +715,20 @@ struct Model {
     cap_rows = n;
     return 0;
   }
+  int ensure_chunks(int n) {
+    size_t need = 0;
+    if (n > 0)
+      for (auto& l : layers)
+        if (l.sm.heads > 0) need = std::max(need, (size_t)pegainfer_ssd_scan_workspace(n, l.sm.heads, l.sm.state, l.sm.vdim));
+    if (need <= chunk_cap) return 0;
+    KK_HIP(hipStreamSynchronize(stream));
+    if (chunk_ws) (void)hipFree(chunk_ws);
+    chunk_ws = nullptr;
+    chunk_cap = 0;
+    KK_HIP(hipMalloc(reinterpret_cast<void**>(&chunk_ws), need * 4));
+    chunk_cap = need;
+    return 0;
+  }
   int ensure_want(size_t n) {
     if (n <= cap_want) return 0;
     KK_HIP(hipStreamSynchronize(stream));
@@ -807,6 +826,12 @@ struct Model {
       tile_cnt[k] = ptiles::count(lens, n, ts.per, tile_rows[k]);
       words += 4 * tile_cnt[k];
     }
+    // long entries of the state-space scan in chunks (never part of a captured step)
+    const ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, mx_inner > 0 && !plain_kernels ? kScanMax : INT32_MAX);
+    const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
+    size_t chunk_off[4];
+    for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
+    if (ensure_chunks((int)chunks.row0.size())) return -1;
     const size_t o_pages = words;
     words += total_pages;
     if (words > cap_meta) {
@@ -841,6 +866,7 @@ struct Model {
       mh[o_ind + n] = (int32_t)pg;
       for (int i = 0; i < W; ++i) mh[o_want + i] = want[i];
       for (size_t k = 0; k < tile_sets.size(); ++k) ptiles::cut(lens, n, tile_sets[k].per, tile_rows[k], tile_cnt[k], mh + tile_off[k]);
+      for (int k = 0; k < 4; ++k) std::copy(chunk_cols[k]->begin(), chunk_cols[k]->end(), mh + chunk_off[k]);
     }
     KK_HIP(hipEventRecord(ev0, stream));
     KK_HIP(hipMemcpyAsync(meta_dev, meta_host, words * 4, hipMemcpyHostToDevice, stream));
@@ -945,9 +971,16 @@ struct Model {
         // right: [z | x | B | C | dt] at o_in; x | B | C through the convolution, the scan, y * silu(z) normed in groups
         const int inner = s.inner();
         if (conv(at(proj, (size_t)(c.o_in + inner)), w.sconv, nullptr, w.sconv_b, r.st_sconv, s.conv_ch(), s.taps, 2)) return -1;
-        KK_K(pegainfer_ssd_scan(conv32, s.conv_ch(), proj, c.proj_rows, c.o_in + 2 * inner + 2 * s.groups * s.state, w.A_log, w.dt_bias,
-                                w.Dskip, state + r.st_mem, slot_stride, o32, s.heads, s.groups, s.state, s.vdim, d_row0, d_slot, n, dtype,
-                                S()));
+        pegainfer_ssd_scan_desc sd{};
+        sd.xbc = conv32; sd.xbc_stride = s.conv_ch(); sd.proj = proj; sd.proj_stride = c.proj_rows;
+        sd.dt_off = c.o_in + 2 * inner + 2 * s.groups * s.state;
+        sd.A_log = w.A_log; sd.dt_bias = w.dt_bias; sd.D = w.Dskip; sd.state = state + r.st_mem; sd.slot_stride = slot_stride; sd.o = o32;
+        sd.heads = s.heads; sd.groups = s.groups; sd.n_state = s.state; sd.vdim = s.vdim;
+        sd.entry_row0 = d_row0; sd.entry_slot = d_slot; sd.n_entries = n; sd.scan_max = kScanMax;
+        sd.chunk_row0 = md + chunk_off[0]; sd.chunk_rows = md + chunk_off[1]; sd.n_chunks = (int)chunks.row0.size();
+        sd.long_chunk0 = md + chunk_off[2]; sd.long_slot = md + chunk_off[3]; sd.n_long = (int)chunks.slot.size();
+        sd.workspace = chunk_ws; sd.dtype = dtype;
+        KK_K(pegainfer_ssd_scan_form(&sd, S()));
         KK_K(pegainfer_head_gate_rms(o32, w.snorm, 1, at(proj, (size_t)c.o_in), c.proj_rows, 0, 1, 1.0f, eps, mixr, inner, s.norm_groups,
                                      inner / s.norm_groups, Ti, dtype, S()));
         if (linear(w.ro, mixr, y2, D, Ti, inner)) return -1;
@@ -1049,6 +1082,7 @@ struct Model {
     free_all(&step_owned);
     free_all(&want_owned);
     if (tap) (void)hipFree(tap);
+    if (chunk_ws) (void)hipFree(chunk_ws);
     if (meta_dev) (void)hipFree(meta_dev);
     if (meta_host) (void)hipHostFree(meta_host);
     if (ev0) (void)hipEventDestroy(ev0);

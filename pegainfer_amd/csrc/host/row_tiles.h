@@ -1,10 +1,12 @@
+// Tables of a step's launches that follow from its entries' row counts.
 // Row tiles of the paged attention launches (pegainfer_paged_attention_opt): a tile is a run of token rows of one entry times a run of the
-// query heads of one key/value head.
+// query heads of one key/value head.  Chunks of long entries, for recurrences with a chunk form.
 #pragma once
 
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 namespace ptiles {
 
@@ -40,6 +42,24 @@ inline void cut(const int32_t* lens, int n, int per, int rows, size_t tiles, int
       for (int q0 = 0; q0 < per; q0 += rows, ++at) {
         row0[at] = r0 + t0; ntok[at] = std::min(tpt, lens[i] - t0); qh0[at] = q0; nqh[at] = std::min(rows, per - q0);
       }
+}
+
+// the chunks of the entries of more than scan_max rows (pegainfer_decay_attention's tables)
+struct Chunks {
+  std::vector<int32_t> row0, rows, first{0}, slot;     // per chunk; per long entry: its first chunk (one more at the end), its state slot
+};
+inline Chunks chunks(const int32_t* ids, const int32_t* lens, int n, int width, int scan_max) {
+  Chunks c;
+  for (int i = 0, r0 = 0; i < n; r0 += lens[i++]) {
+    if (lens[i] <= scan_max) continue;
+    for (int k = 0; k < lens[i]; k += width) {
+      c.row0.push_back(r0 + k);
+      c.rows.push_back(std::min(width, lens[i] - k));
+    }
+    c.first.push_back((int32_t)c.row0.size());
+    c.slot.push_back(ids[i]);
+  }
+  return c;
 }
 
 }  // namespace ptiles

@@ -703,20 +703,10 @@ class StepModel {
     return put_columns(mb, c);
   }
   void put_chunks(std::vector<int32_t>* mb, const int32_t* ids, const int32_t* lens, int n, ChunkTable* t, size_t* off) const {
-    std::vector<int32_t> row0, rows, first{0}, slot;
-    int r0 = 0;
-    for (int i = 0; i < n; r0 += lens[i++]) {
-      if (lens[i] <= scan_max) continue;
-      for (int k = 0; k < lens[i]; k += PEGAINFER_DECAY_CHUNK) {
-        row0.push_back(r0 + k);
-        rows.push_back(std::min<int>(PEGAINFER_DECAY_CHUNK, lens[i] - k));
-      }
-      first.push_back((int32_t)row0.size());
-      slot.push_back(ids[i]);
-    }
-    t->n_chunks = (int)row0.size();
-    t->n_long = (int)slot.size();
-    const std::vector<int32_t>* v[4] = {&row0, &rows, &first, &slot};
+    const ptiles::Chunks c = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, scan_max);
+    t->n_chunks = (int)c.row0.size();
+    t->n_long = (int)c.slot.size();
+    const std::vector<int32_t>* v[4] = {&c.row0, &c.rows, &c.first, &c.slot};
     for (int k = 0; k < 4; ++k) {
       off[k] = mb->size();
       mb->insert(mb->end(), v[k]->begin(), v[k]->end());

@@ -488,13 +488,16 @@ def paged_attention_masked(q, cache, page_stride, k_off, v_off, page_size, rg, p
     return out
 
 
-def ssd_scan(xbc_f32, proj, dt_off, A_log, dt_bias, D, state, heads, groups, n_state, vdim, rg):
+def ssd_scan(xbc_f32, proj, dt_off, A_log, dt_bias, D, state, heads, groups, n_state, vdim, rg, scan_max=0):
     """selective state-space scan; xbc fp32 [rows, heads * vdim + 2 * groups * n_state]; proj rows (storage type) hold the raw step
-    sizes at dt_off; state fp32 [slots, heads * n_state * vdim] is read and moved on; -> y fp32 [rows, heads * vdim]"""
+    sizes at dt_off; state fp32 [slots, heads * n_state * vdim] is read and moved on; scan_max > 0: entries of more rows take the chunk
+    form; -> y fp32 [rows, heads * vdim]"""
     y = torch.empty((xbc_f32.shape[0], heads * vdim), dtype=torch.float32, device=proj.device)
-    _chk(ffi.lib().pegainfer_ssd_scan(_p(xbc_f32), xbc_f32.stride(0), _p(proj), proj.stride(0), dt_off, _p(A_log), _p(dt_bias), _p(D),
-                                      _p(state), state.stride(0), _p(y), heads, groups, n_state, vdim, _p(rg.entry_row0), _p(rg.entry_slot),
-                                      rg.n, _dt(proj), _stream()), "ssd_scan")
+    d = SsdScanDesc(xbc=_p(xbc_f32), xbc_stride=xbc_f32.stride(0), proj=_p(proj), proj_stride=proj.stride(0), dt_off=dt_off, A_log=_p(A_log),
+                    dt_bias=_p(dt_bias), D=_p(D), state=_p(state), slot_stride=state.stride(0), o=_p(y), heads=heads, groups=groups,
+                    n_state=n_state, vdim=vdim, entry_row0=_p(rg.entry_row0), entry_slot=_p(rg.entry_slot), n_entries=rg.n, dtype=_dt(proj))
+    keep = _chunk_tables(d, rg, scan_max, ffi.lib().pegainfer_ssd_scan_workspace, heads, n_state, vdim)  # noqa: F841 (alive until enqueued)
+    _chk(ffi.lib().pegainfer_ssd_scan_form(ctypes.addressof(d), _stream()), "ssd_scan")
     return y
 
 
@@ -514,6 +517,10 @@ LatentPrepDesc = _struct("LatentPrepDesc", [("p", "dkv"), ("l", "dkv_stride"), (
 StreamMixDesc = _struct("StreamMixDesc", [("p", "x_in embed token_ids"), ("f", "embed_scale"), ("p", "row_index y"), ("l", "y_row_stride"),
                                           ("p", "mix out_w"), ("f", "mult"), ("p", "x_out sum_out read_w gain n_out"), ("f", "eps"),
                                           ("i", "norm_kind streams d rows dtype")])
+SsdScanDesc = _struct("SsdScanDesc", [("p", "xbc"), ("l", "xbc_stride"), ("p", "proj"), ("l", "proj_stride dt_off"), ("p", "A_log dt_bias D state"),
+                                      ("l", "slot_stride"), ("p", "o"), ("i", "heads groups n_state vdim"), ("p", "entry_row0 entry_slot"),
+                                      ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"), ("i", "n_chunks"), ("p", "long_chunk0 long_slot"),
+                                      ("i", "n_long"), ("p", "workspace"), ("i", "dtype")])
 DecayAttentionDesc = _struct("DecayAttentionDesc", [("p", "proj"), ("l", "proj_stride q_off k_off v_off"), ("i", "silu"), ("p", "decay_pow"),
                                                     ("i", "pow_n"), ("p", "state"), ("l", "slot_stride"), ("p", "o"), ("i", "heads dim vdim"),
                                                     ("p", "entry_row0 entry_slot"), ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"),

@@ -415,6 +415,45 @@ def test_an_old_write_is_kept_by_a_slow_head_and_forgotten_by_a_fast_one():
         assert abs(float(y[2, P]) - 50.0) < 1e-4 and float(y[1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,groups,N,P", [(4, 2, 128, 64), (2, 1, 16, 8), (3, 3, 20, 33), (2, 2, 256, 130), (1, 1, 5, 64)])
+def test_state_space_chunks_against_the_scan_in_64_bits(dtype, heads, groups, N, P):
+    """portions around the 64 tokens of a chunk beside one that stays with the scan, state left from an earlier portion, odd sizes and rows that are
+    not aligned; heads that keep, fade and forget at once.  The scan in 64 bits is the reference: the outputs are sums of up to 320 products of
+    about one, each a few 1e-6 off at most by the running product of the decays."""
+    Bk = B()
+    g = torch.Generator().manual_seed(N + P)
+    lens, slots = [64, 3, 65, 320, 127], [1, 4, 0, 3, 5]
+    inner = heads * P
+    ch, T = inner + 2 * groups * N, sum(lens)
+    xbc = torch.randn(T, ch, generator=g)
+    xbc[:, inner:] *= N ** -0.25
+    proj = C.bf16_round(torch.randn(T, heads + 3, generator=g))
+    A_log = C.bf16_round(torch.tensor([[-9.0, -1.0, 3.0, 6.0][i % 4] for i in range(heads)]))
+    dt_bias, D = C.bf16_round(torch.randn(heads, generator=g)), C.bf16_round(torch.randn(heads, generator=g))
+    state = torch.randn(6, heads * N * P, generator=g).cuda()
+    S = state.cpu().double().view(6, heads, N, P)
+    rg = Bk.Ragged(lens, slots=slots)
+    args = (dev(proj, dtype), 3, dev(A_log, dtype), dev(dt_bias, dtype), dev(D, dtype))
+    y = Bk.ssd_scan(xbc.cuda(), *args, state, heads, groups, N, P, rg, scan_max=32).cpu().double()
+    at = 0
+    for n, s in zip(lens, slots):
+        for h in range(heads):
+            b0 = inner + (h // (heads // groups)) * N
+            x, b, c = (xbc[at:at + n, k:k + w].double() for k, w in ((h * P, P), (b0, N), (b0 + groups * N, N)))
+            dt = torch.nn.functional.softplus(proj[at:at + n, 3 + h].double() + dt_bias[h].double())
+            a = torch.exp(-torch.exp(A_log[h].double()) * dt)
+            St, ref = S[s, h].clone(), torch.empty(n, P, dtype=torch.float64)
+            for t in range(n):
+                St = a[t] * St + dt[t] * torch.outer(b[t], x[t])
+                ref[t] = St.T @ c[t] + D[h].double() * x[t]
+            tol = 2e-5 * max(1.0, float(ref.abs().max()))
+            assert float((y[at:at + n, h * P:(h + 1) * P] - ref).abs().max()) < tol, (n, h)
+            assert float((state[s].cpu().double().view(heads, N, P)[h] - St).abs().max()) < 2e-5 * max(1.0, float(St.abs().max())), (n, h)
+        at += n
+    assert torch.equal(state[2].cpu().double().view(heads, N, P), S[2])          # a slot of nobody
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
