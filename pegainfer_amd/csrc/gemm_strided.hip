@@ -100,42 +100,62 @@ __global__ __launch_bounds__(256) void gemm_strided_kernel(pegainfer_gemm_desc d
 
 
 // ------------------------------------------------------------------ matrix-core form (bf16 weights, k contiguous)
-// The same addressing (groups, gathered rows, tile table), K in slices of 64 staged as bf16 through registers (the next slice
-// is in flight while this one is multiplied), four waves in a 2 x 2 arrangement of v_mfma_f32_16x16x32_bf16 blocks.  fp32 x (the attention output in front of the value
-// up-projection) is rounded to bf16 while it is staged.  Needs 16-byte chunks: K % 8 == 0, strides % 8 == 0, aligned bases.
-constexpr int MK = 64, MS = MK + 8;
-
-__device__ __forceinline__ u32x4 stage8(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
-__device__ __forceinline__ u32x4 stage8(const float* p) {
-  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-  return u32x4{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
-}
-
-// Output tile TR rows x 128 outputs (TR = 64 or 128): with 64 x 64 tiles the kernel moved 32 flop per byte staged and sat on
-// the L2 -> CU bandwidth (7.5 TB/s of staging traffic at 1024 tokens x 4 experts); 128 x 128 halves the bytes per flop.
+// The same addressing (groups, gathered rows, tile table), output tiles of TR rows (64 or 128) x 128 outputs, four waves in a 2 x 2
+// arrangement of v_mfma_f32_16x16x32_bf16 blocks, K in slices of MK (64 or 32).  Both operands travel by LDS-DMA into two slots, one slice ahead: a
+// lane's source address carries the gather and the swizzle (swizzled()), so fragment reads meet no bank twice.  A wave's loads of a slice are
+// waited for by count, the next slice's stay in flight under the products.
+// fp32 x (the attention output in front of the value up-projection) is rounded to bf16 as it is read into fragments.  Rows and outputs past the
+// tile's end load a valid row and are dropped at the store; the last slice's values past K are made zero in both operands.
+// Needs 16-byte chunks: K % 8 == 0, strides % 8 == 0, aligned bases.
+// Bound by what a compute unit takes in: 32 KB per slice and workgroup against 128 MFMAs, two workgroups per compute unit in turn.
+// Work items go to the XCDs in eight contiguous runs (an XCD's L2 is where workgroups share an operand): with a tile table the outputs of a
+// tile run fastest, so the neighbouring tiles of one expert read its weights together; without one the larger operand is read once.
+// Before (slices staged through registers, fp32 chunks converted as they were fetched, so every load was waited for at once):
+// 9600 pairs of 32 experts of 2048 x 2048 204 -> 134 us (600 TFLOP/s), of 2048 x 1024 into fp32 131 -> 75; 1024 fp32 rows x 2048 x 4096
+// 127 -> 50; 2400 rows, 16 groups of 512 x 128 48 -> 21, fp32 rows of 128 x 512 34 -> 21.
 constexpr int MM = 128;
 
-template <typename TX, typename TY, typename TG, int TR>
-__global__ __launch_bounds__(256) void gemm_strided_mfma_kernel(pegainfer_gemm_desc d) {
-  __shared__ __align__(16) uint16_t xs[TR * MS];
-  __shared__ __align__(16) uint16_t ws[MM * MS];
+// position of 16-byte chunk c of a row in LDS, CH chunks to a row: the rows a fragment read meets lie on different banks
+template <int CH>
+__device__ __forceinline__ int swizzled(int c, int row) { return c ^ (CH == 4 ? (row >> 1) & 3 : row & (CH - 1)); }
+
+template <typename TX, int TR, int MK>
+struct StridedMfmaShape {
+  static constexpr int kXE = 16 / (int)sizeof(TX);                         // values of a chunk of x
+  static constexpr int kXCh = MK / kXE, kWCh = MK / 8;                     // chunks of a row's slice
+  static constexpr int kX = TR * kXCh * 16, kW = MM * kWCh * 16, kSlot = kX + kW;   // bytes of a slot
+  static constexpr int kXLoads = kX / 4096, kWLoads = kW / 4096;           // DMA instructions per wave and slice
+};
+
+template <typename TX, typename TY, typename TG, int TR, int MK>
+__global__ __launch_bounds__(256) void gemm_strided_mfma_kernel(pegainfer_gemm_desc d, int row_tiles, int rows_first) {
+  typedef StridedMfmaShape<TX, TR, MK> Sh;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t mfma_lds[];
   __shared__ int xrow[TR], yrow[TR];
-  int g, row0, nrows;
+  const int mt = (d.m + MM - 1) / MM;
+  int rt, m0, g;
+  {
+    const int tiles = d.tile_group ? *d.n_tiles : row_tiles, n = tiles * mt * (d.tile_group ? 1 : d.groups);
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3, q = n >> 3, rest = n & 7;
+    if (pos >= q + (xcd < rest ? 1 : 0)) return;
+    const int item = xcd * q + min(xcd, rest) + pos;
+    g = item / (tiles * mt);
+    const int i = item - g * (tiles * mt);
+    rt = rows_first ? i % tiles : i / mt;
+    m0 = (rows_first ? i / tiles : i % mt) * MM;
+  }
+  int row0 = rt * TR, nrows;
   if (d.tile_group) {
-    if ((int)blockIdx.x >= *d.n_tiles) return;
-    g = d.tile_group[blockIdx.x];
-    row0 = d.tile_row0[blockIdx.x];
-    nrows = min(TR, d.tile_rows[blockIdx.x]);
+    g = d.tile_group[rt];
+    row0 = d.tile_row0[rt];
+    nrows = min(TR, d.tile_rows[rt]);
   } else {
-    g = blockIdx.z;
-    row0 = blockIdx.x * TR;
     nrows = min(TR, d.rows - row0);
   }
-  const int m0 = blockIdx.y * MM;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
   if (tid < TR) {
-    const int p = row0 + tid;
-    xrow[tid] = tid < nrows ? (d.x_row_index ? d.x_row_index[p] : p) : -1;
+    const int p = row0 + min(tid, nrows - 1);
+    xrow[tid] = d.x_row_index ? d.x_row_index[p] : p;
     yrow[tid] = tid < nrows ? (d.y_row_index ? d.y_row_index[p] : p) : -1;
   }
   __syncthreads();
@@ -148,53 +168,84 @@ __global__ __launch_bounds__(256) void gemm_strided_mfma_kernel(pegainfer_gemm_d
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < RJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  constexpr int XC = TR * (MK / 8) / 256, WC = MM * (MK / 8) / 256;   // chunks per thread and K slice
-  // this thread's rows are the same in every K slice: resolve them once
-  const TX* xsrc[XC];
-  const uint16_t* wsrc[WC];
+  const TX* xsrc[Sh::kXLoads];
+  const uint16_t* wsrc[Sh::kWLoads];
+  int xk[Sh::kXLoads], wk[Sh::kWLoads];             // first value of this lane's chunk in a slice
 #pragma unroll
-  for (int i = 0; i < XC; ++i) {
-    const int c = tid + i * 256, src = xrow[c >> 3];
-    xsrc[i] = src >= 0 ? X + (int64_t)src * d.x_row_stride + (c & 7) * 8 : nullptr;
+  for (int i = 0; i < Sh::kXLoads; ++i) {
+    const int unit = (wave * Sh::kXLoads + i) * 64 + lane, row = unit / Sh::kXCh;
+    xk[i] = swizzled<Sh::kXCh>(unit % Sh::kXCh, row) * Sh::kXE;
+    xsrc[i] = X + (int64_t)xrow[row] * d.x_row_stride;
   }
 #pragma unroll
-  for (int i = 0; i < WC; ++i) {
-    const int c = tid + i * 256, m = m0 + (c >> 3);
-    wsrc[i] = m < d.m ? W + (int64_t)m * d.w_m_stride + (c & 7) * 8 : nullptr;
+  for (int i = 0; i < Sh::kWLoads; ++i) {
+    const int unit = (wave * Sh::kWLoads + i) * 64 + lane, row = unit / Sh::kWCh;
+    wk[i] = swizzled<Sh::kWCh>(unit % Sh::kWCh, row) * 8;
+    wsrc[i] = W + (int64_t)min(m0 + row, d.m - 1) * d.w_m_stride;
   }
-  u32x4 px[XC], pw[WC];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < XC; ++i) px[i] = (xsrc[i] && k0 + ((tid + i * 256) & 7) * 8 < d.k) ? stage8(xsrc[i] + k0) : zero;
-#pragma unroll
-    for (int i = 0; i < WC; ++i) pw[i] = (wsrc[i] && k0 + ((tid + i * 256) & 7) * 8 < d.k) ? stage8(wsrc[i] + k0) : zero;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr_t)mfma_lds;
+  auto dma = [&](const void* src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :: "v"(src), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
   };
-  fetch(0);
-  for (int k0 = 0; k0 < d.k; k0 += MK) {
-    __syncthreads();
+  auto issue = [&](int k0, int slot) {              // chunks past K load the row's last one: zeros in the products
+    const uint32_t base = ring + slot * Sh::kSlot;
 #pragma unroll
-    for (int i = 0; i < XC; ++i) { const int c = tid + i * 256; *reinterpret_cast<u32x4*>(xs + (c >> 3) * MS + (c & 7) * 8) = px[i]; }
+    for (int i = 0; i < Sh::kXLoads; ++i)
+      dma(xsrc[i] + min(k0 + xk[i], d.k - Sh::kXE), base + (wave * Sh::kXLoads + i) * 1024);
 #pragma unroll
-    for (int i = 0; i < WC; ++i) { const int c = tid + i * 256; *reinterpret_cast<u32x4*>(ws + (c >> 3) * MS + (c & 7) * 8) = pw[i]; }
-    __syncthreads();
-    if (k0 + MK < d.k) fetch(k0 + MK);            // the next slice's loads fly while this one is multiplied
+    for (int i = 0; i < Sh::kWLoads; ++i) dma(wsrc[i] + min(k0 + wk[i], d.k - 8), base + Sh::kX + (wave * Sh::kWLoads + i) * 1024);
+  };
+  auto multiply = [&](int k0, int slot, auto tail) {
+    const uint8_t *xs = mfma_lds + slot * Sh::kSlot, *ws = xs + Sh::kX;
 #pragma unroll
-    for (int ks = 0; ks < MK; ks += 32) {
+    for (int ks = 0; ks < MK / 32; ++ks) {
+      const int c = ks * 4 + gq;                    // this lane's eight values of k
+      const bool past = tail.value && k0 + c * 8 >= d.k;
       bf16x8_t a[4], b[RJ];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        a[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(ws + (wm + i * 16 + l15) * MS + ks + gq * 8));
+      for (int i = 0; i < 4; ++i) {
+        u32x4 v = *reinterpret_cast<const u32x4*>(ws + ((wm + i * 16 + l15) * Sh::kWCh + swizzled<Sh::kWCh>(c, l15)) * 16);
+        if (past) v = u32x4{0u, 0u, 0u, 0u};
+        a[i] = __builtin_bit_cast(bf16x8_t, v);
+      }
 #pragma unroll
-      for (int j = 0; j < RJ; ++j)
-        b[j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(xs + (wr + j * 16 + l15) * MS + ks + gq * 8));
+      for (int j = 0; j < RJ; ++j) {
+        const uint8_t* row = xs + (wr + j * 16 + l15) * Sh::kXCh * 16;
+        u32x4 v;
+        if constexpr (sizeof(TX) == 2) v = *reinterpret_cast<const u32x4*>(row + swizzled<Sh::kXCh>(c, l15) * 16);
+        else {
+          const f32x4 lo = *reinterpret_cast<const f32x4*>(row + swizzled<Sh::kXCh>(2 * c, l15) * 16),
+                      hi = *reinterpret_cast<const f32x4*>(row + swizzled<Sh::kXCh>(2 * c + 1, l15) * 16);
+          v = u32x4{pack_bf2(lo.x, lo.y), pack_bf2(lo.z, lo.w), pack_bf2(hi.x, hi.y), pack_bf2(hi.z, hi.w)};
+        }
+        if (past) v = u32x4{0u, 0u, 0u, 0u};
+        b[j] = __builtin_bit_cast(bf16x8_t, v);
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < RJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     }
+  };
+  issue(0, 0);
+  int slot = 0;
+  for (int k0 = 0; k0 < d.k; k0 += MK, slot ^= 1) {
+    if (k0 + MK < d.k) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");       // the slice before is multiplied: its slot is free
+      issue(k0 + MK, slot ^ 1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Sh::kXLoads + Sh::kWLoads) : "memory");   // this wave's part of slice k0 has landed
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_barrier" ::: "memory");          // everyone's part
+    if (k0 + MK <= d.k) multiply(k0, slot, std::false_type{});
+    else multiply(k0, slot, std::true_type{});
   }
   TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
+  constexpr int kYBytes = 4 * (int)sizeof(TY);       // four neighbouring outputs of a row
+  const bool vec = d.y_row_stride % 4 == 0 && d.y_group_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(d.y) & (kYBytes - 1)) == 0;
 #pragma unroll
   for (int j = 0; j < RJ; ++j) {
     const int r = wr + j * 16 + l15;
@@ -204,27 +255,53 @@ __global__ __launch_bounds__(256) void gemm_strided_mfma_kernel(pegainfer_gemm_d
     if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
       scale = sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)xrow[r] * d.gate_row_stride + g));
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + wm + i * 16 + gq * 4;
+      f32x4 v = acc[i][j];
+      if (d.epilogue == PEGAINFER_EPI_RELU_SQ) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + wm + i * 16 + gq * 4 + e;
-        if (m >= d.m) continue;
-        float v = acc[i][j][e];
-        if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
-        else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
-        else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE) v *= scale;
-        st(Y + (int64_t)dst * d.y_row_stride + m, v);
+        for (int e = 0; e < 4; ++e) { v[e] = fmaxf(v[e], 0.f); v[e] *= v[e]; }
+      } else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = gelu_erf_f(v[e]);
+      } else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE) {
+        v *= scale;
       }
+      TY* out = Y + (int64_t)dst * d.y_row_stride + m;
+      if (vec && m + 4 <= d.m) {
+        if constexpr (sizeof(TY) == 4) *reinterpret_cast<f32x4*>(out) = v;
+        else *reinterpret_cast<u32x2*>(out) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (m + e < d.m) st(out + e, v[e]);
+      }
+    }
   }
 }
 
+template <typename TX, typename TY, typename TG, int TR>
+static void mfma_tiles_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
+  // fp32 rows of 128: slices of 32, so that more than one workgroup fits a compute unit's LDS (4096 x 4096 x 4096: 296 -> 279 us)
+  constexpr int MK = sizeof(TX) == 4 && TR == 128 ? 32 : 64;
+  auto kern = &gemm_strided_mfma_kernel<TX, TY, TG, TR, MK>;
+  constexpr size_t lds = 2 * StridedMfmaShape<TX, TR, MK>::kSlot;
+  static const bool once = (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
+  (void)once;
+  const int tiles = d.tile_group ? d.max_tiles : ceil_div(d.rows, TR), mt = ceil_div(d.m, MM);
+  const long items = (long)tiles * mt * (d.tile_group ? 1 : d.groups);
+  const bool rows_first = !d.tile_group && (long)d.rows * sizeof(TX) < (long)d.m * 2;     // the weights are the larger operand: read once
+  kern<<<dim3((unsigned)(8 * ceil_div(items, 8))), 256, lds, s>>>(d, tiles, rows_first ? 1 : 0);
+}
 template <typename TX, typename TY, typename TG>
 static void mfma_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
-  const bool big = d.tile_group ? d.tile_rows_cap >= 128 : d.rows > 64;
-  const int TR = big ? 128 : 64;
-  dim3 grid(d.tile_group ? d.max_tiles : ceil_div(d.rows, TR), ceil_div(d.m, MM), d.tile_group ? 1 : d.groups);
-  if (big) gemm_strided_mfma_kernel<TX, TY, TG, 128><<<grid, 256, 0, s>>>(d);
-  else gemm_strided_mfma_kernel<TX, TY, TG, 64><<<grid, 256, 0, s>>>(d);
+  // Tiles of 128 rows where they give two workgroups per compute unit, four for fp32 rows (128- / 64-row tiles): bf16 rows, 256 workgroups
+  // (2048 x 2048 x 2048) 33 / 28 us, 320 (600 rows, 16 groups of 512 x 128) 10.9 / 9.4, 512 (4096 x 2048 x 2048) 45 / 53; fp32 rows, 304 (2400
+  // x 2048 x 4096) 128 / 100 us, 1024 (4096 x 4096 x 4096) 279 / 302, (8192 rows, 16 groups of 128 x 512) 69 / 67.
+  const long wide = (long)ceil_div(d.rows, 128) * ceil_div(d.m, MM) * d.groups;
+  const bool big = d.tile_group ? d.tile_rows_cap >= 128 : wide >= (sizeof(TX) == 4 ? 4L : 2L) * device_cus();
+  if (big) mfma_tiles_launch<TX, TY, TG, 128>(d, s);
+  else mfma_tiles_launch<TX, TY, TG, 64>(d, s);
 }
 
 // ------------------------------------------------------------------ few-rows form (decode), fp32 weights or one fp32 row

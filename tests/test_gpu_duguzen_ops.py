@@ -356,6 +356,61 @@ def test_matrix_core_form_sees_a_far_key_and_masks_an_unseen_one():
             assert float(o[0][:, 3].abs().max()) < 1.0
 
 
+@pytest.mark.parametrize("xd,yd", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "bfloat16"), ("float32", "float32")])
+@pytest.mark.parametrize("T,M,K,G", [(17, 128, 8, 1), (65, 130, 56, 2), (128, 127, 64, 3), (129, 300, 72, 1), (200, 1, 200, 2), (513, 514, 136, 40)])
+def test_tiles_on_the_matrix_cores_at_their_edges(T, M, K, G, xd, yd):
+    """slices that end inside K (what lies behind K in the wider rows is no number), rows and outputs past a tile's end, several groups, odd output
+    rows, gathered and scattered rows with a gate: against the product of the operands as the matrix cores see them (fp32 rows rounded to
+    bf16).  Sums of K products of about one in fp32: 1e-6 K; a bf16 result adds half a unit in the last place, 2^-8 of the value."""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(T + M)
+    xs, ws = G * (K + 8) + 8, K + 16
+    x = torch.full((T + 3, xs), float("nan"))
+    w = torch.full((G, M, ws), float("nan"))
+    for i in range(G):
+        x[:, i * (K + 8):i * (K + 8) + K] = torch.randn(T + 3, K, generator=g)
+    w[:, :, :K] = C.bf16_round(torch.randn(G, M, K, generator=g))
+    if xd == "bfloat16":
+        x = C.bf16_round(x)
+    src, dst = torch.randperm(T + 3, generator=g)[:T].int(), torch.randperm(T, generator=g).int()
+    gate = torch.randn(T + 3, G, generator=g)
+    x_d, w_d, src_d, dst_d, gate_d = dev(x, DT[xd]), dev(w, torch.bfloat16), src.cuda(), dst.cuda(), gate.cuda()
+    ref = torch.einsum("tgk,gmk->tgm", C.bf16_round(x[src.long()]).double()[:, :G * (K + 8)].reshape(T, G, K + 8)[..., :K], w[..., :K].double())
+    for epi in (B.EPI_NONE, B.EPI_RELU_SQ, B.EPI_SIGMOID_GATE):
+        r = ref if epi == B.EPI_NONE else torch.relu(ref) ** 2 if epi == B.EPI_RELU_SQ else ref * torch.sigmoid(gate[src.long()].double())[..., None]
+        for pad in (0, 1):
+            y = torch.full((T, G * M + pad), -7.0, device="cuda", dtype=DT[yd])
+            B.gemm_strided(B.GemmDesc(x=x_d.data_ptr(), w=w_d.data_ptr(), y=y.data_ptr(), x_dtype=B._dt(x_d), w_dtype=0, y_dtype=B._dt(y), m=M, k=K,
+                                      rows=T, groups=G, x_row_stride=xs, x_group_stride=K + 8, w_m_stride=ws, w_k_stride=1, w_group_stride=M * ws,
+                                      y_row_stride=G * M + pad, y_group_stride=M, x_row_index=src_d.data_ptr(), y_row_index=dst_d.data_ptr(),
+                                      epilogue=epi, gate=gate_d.data_ptr(), gate_dtype=1, gate_row_stride=G))
+            got = y.cpu().double()
+            assert pad == 0 or float((got[:, -1] + 7.0).abs().max()) == 0.0
+            got = got[dst.long()][:, :G * M].reshape(T, G, M)
+            tol = 1e-6 * K * (1 + r.abs()) ** (1 if epi != B.EPI_RELU_SQ else 0.5) * (4 if epi == B.EPI_RELU_SQ else 1)
+            assert bool(((got - r).abs() <= tol + (r.abs() / 256 if yd == "bfloat16" else 0)).all()), (epi, pad, float((got - r).abs().max()))
+
+
+@pytest.mark.parametrize("rows_per_tile", [64, 128])
+def test_tiles_of_an_expert_table_reach_every_pair(rows_per_tile):
+    """live tiles dealt over eight runs: one tile, seven, eight, nine and many, more places in the table than tiles"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(rows_per_tile)
+    for E, rows, top in ((1, 20, 1), (7, 40, 2), (8, 64, 3), (9, 41, 4), (40, 300, 5)):
+        K, M = 72, 200
+        expert = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(rows)]).int()
+        pos_pair, pos_row, tg, t0, tr, nt, max_tiles = B.route_sort(expert.cuda(), E, rows_per_tile=rows_per_tile)
+        x, w = C.bf16_round(torch.randn(rows, K, generator=g)), C.bf16_round(torch.randn(E, M, K, generator=g))
+        xd, wd = dev(x, torch.bfloat16), dev(w, torch.bfloat16)
+        y = torch.full((rows * top, M), float("nan"), device="cuda")
+        B.gemm_strided(B.GemmDesc(x=xd.data_ptr(), w=wd.data_ptr(), y=y.data_ptr(), x_dtype=0, w_dtype=0, y_dtype=1, m=M, k=K, x_row_stride=K,
+                                  w_m_stride=K, w_k_stride=1, w_group_stride=M * K, y_row_stride=M, tile_group=tg.data_ptr(),
+                                  tile_row0=t0.data_ptr(), tile_rows=tr.data_ptr(), n_tiles=nt.data_ptr(), max_tiles=max_tiles,
+                                  x_row_index=pos_row.data_ptr(), y_row_index=pos_pair.data_ptr(), tile_rows_cap=rows_per_tile))
+        ref = torch.einsum("pk,pmk->pm", x.double().repeat_interleave(top, 0), w.double()[expert.reshape(-1).long()])
+        assert float((y.cpu().double() - ref).abs().max()) < 1e-6 * K * (1 + float(ref.abs().max()))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_strided_gemm_forms_agree(dtype):
     """the few-rows form (<= 8 rows), the matrix-core tile form (bf16 weights) and the fp32-FMA tile form compute the same
