@@ -54,8 +54,8 @@ pegainfer_status_t pegainfer_silu_mul_rows(const void* gate_up, void* out, int32
  * Kernels behind one entry: an fp32-FMA tile kernel (any sizes and strides, both storage types), a matrix-core tile
  * kernel each for bf16 weights (contiguous k in 16-byte chunks; an fp32 x is rounded to bf16 as it is staged) and for fp32 weights (fp32
  * products and sums), and two few-rows
- * forms that stream the weights once (decode): bf16 weights on the matrix cores (<= 16 rows per tile; an fp32 x enters in three exact
- * parts), fp32 weights by FMA (<= 8 rows).  In each the k order of an output is fixed, so a row's
+ * forms that stream the weights once (decode, <= 16 rows per tile): bf16 weights on the matrix cores (an fp32 x enters in three exact
+ * parts), fp32 weights by FMA (<= 4 rows) or on the fp32 matrix cores.  In each the k order of an output is fixed, so a row's
  * result does not depend on what else is in the launch; which kernel runs depends on the launch's shape. */
 enum { PEGAINFER_EPI_NONE = 0, PEGAINFER_EPI_RELU_SQ = 1, PEGAINFER_EPI_SIGMOID_GATE = 2, PEGAINFER_EPI_GELU_ERF = 3 };
 typedef struct {

@@ -305,11 +305,11 @@ static void mfma_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ few-rows form (decode), fp32 weights or one fp32 row
-// At most R rows per tile (a decode step's tokens, or the pairs one expert received): the weights are streamed once with
+// At most R = 1, 2 or 4 rows per tile (a decode step's tokens, or the pairs one expert received): the weights are streamed once with
 // 16-byte loads, the rows wait in LDS as fp32 (2048 k values at a time), a wave owns one output at a time (lanes over k, butterfly sum), 32 outputs per
 // workgroup - or 8 (OUT) when 32 would leave most of the chip without a workgroup (a matrix of a few thousand outputs).  fp32
 // arithmetic for both storage types; the k order of an output is fixed by K alone, whatever OUT is.
-constexpr int kRowsFormChunk = 2048;   // k values of the rows that wait in LDS at a time (a multiple of the 512 a wave strides by)
+constexpr int kRowsFormChunk = 2048;   // k values of the rows that wait in LDS at a time (a multiple of the 512 a wave strides by): 32 KB at most
 
 template <typename TX, typename TW, typename TY, typename TG, int R, int OUT = 32>
 __global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_desc d) {
@@ -338,8 +338,8 @@ __global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_d
   const int K = d.k, xs = min(K, kRowsFormChunk);
   TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
   // a wave owns a quarter of the workgroup's outputs and walks them four at a time: four independent weight streams in flight.
-  // The rows pass through LDS a chunk of k at a time (a long row times eight rows would leave room for one workgroup per compute
-  // unit); every output's sums stay in registers across the chunks, so its k order is what it would be in one piece.
+  // The rows pass through LDS a chunk of k at a time (four long rows would leave room for one workgroup per compute unit); every
+  // output's sums stay in registers across the chunks, so its k order is what it would be in one piece.
   constexpr int OW = OUT / 4, MB = OW >= 4 ? 4 : OW, NG = OW / MB;
   const int m_base = blockIdx.y * OUT + wave * OW;
   float acc[NG][MB][R];
@@ -413,20 +413,19 @@ __global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_d
   }
 }
 
+// 32 outputs per workgroup unless that leaves most compute units without one
+static bool rows_form_fine(const pegainfer_gemm_desc& d, int R) {
+  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
+  return (long)row_tiles * groups * ceil_div(d.m, 32) < device_cus();
+}
 template <typename TX, typename TW, typename TY, typename TG, int R>
 static void rows_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   auto kern = &gemm_strided_rows_kernel<TX, TW, TY, TG, R, 32>;
   auto kern8 = &gemm_strided_rows_kernel<TX, TW, TY, TG, R, 8>;
-  // 150 KB of rows at most (checked by the caller) next to the kernel's few static words
-  static const bool once = (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024),
-                            hipFuncSetAttribute(reinterpret_cast<const void*>(kern8), hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024),
-                            true);
-  (void)once;
   // the tiles that a table's bound allows for and that are empty come last: an even grid width would send the others' workgroups, in
   // their round robin over the XCDs, to some of the eight only
   const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  // 32 outputs per workgroup unless that leaves most compute units without one
-  const bool fine = (long)row_tiles * groups * ceil_div(d.m, 32) < device_cus();
+  const bool fine = rows_form_fine(d, R);
   dim3 grid(row_tiles, ceil_div(d.m, fine ? 8 : 32), groups);
   const size_t lds = (size_t)R * std::min(d.k, kRowsFormChunk) * sizeof(float);
   if (fine) kern8<<<grid, 256, lds, s>>>(d);
@@ -619,6 +618,115 @@ static void rows_mfma_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   else gemm_rows_mfma_kernel<TX, TY, TG, 1><<<dim3(row_tiles, blocks, groups), 256, 0, s>>>(d, wk);
 }
 
+// ------------------------------------------------------------------ few-rows form on the matrix cores (fp32 weights, decode)
+// At most 16 rows per tile, on v_mfma_f32_16x16x4_f32.  A wave takes OB blocks of 16 outputs, wk waves of the workgroup's eight share a
+// block's K (wave j the 32-wide pieces j, j + wk, ...; wk follows from K alone), their sums meet in LDS in wave order: an output's k
+// order is fixed by K.  Lane (l15, g) fetches the eight values from 8 g of a piece of output l15 and of row l15, whole lines of weights;
+// product e of a piece takes value e of every lane, both operands numbered alike.  Four pieces of both operands are in flight per wave,
+// nothing is staged and no barrier stands before the sums.
+// Against FMA with eight rows in LDS: 32 768 x 1024 weights and 8 rows 54.9 -> 35.8 us, 1024 x 3072 19.2 -> 14.4; 16 rows (two passes over the
+// weights there) 46.6 -> 16.3.
+template <typename TY, typename TG, int OB>
+__global__ __launch_bounds__(512) void gemm_rows_f32_kernel(pegainfer_gemm_desc d, int wk) {
+  constexpr int NW = 8, CH = 2;                               // pieces per register set
+  __shared__ f32x4 red[NW][OB][64];
+  int g, row0, nrows;
+  if (d.tile_group) {
+    if ((int)blockIdx.x >= *d.n_tiles) return;
+    g = d.tile_group[blockIdx.x];
+    row0 = d.tile_row0[blockIdx.x];
+    nrows = min(kRowsMax, d.tile_rows[blockIdx.x]);
+  } else {
+    g = blockIdx.z;
+    row0 = blockIdx.x * kRowsMax;
+    nrows = min(kRowsMax, d.rows - row0);
+  }
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
+  const int per_wg = NW / wk * OB * 16;                       // outputs of a workgroup
+  const int blk = wave / wk, ks = wave - blk * wk;
+  const int m0 = blockIdx.y * per_wg + blk * OB * 16;
+  const int tok = row0 + min(l15, nrows - 1);                 // absent rows repeat the last one; they are never stored
+  const float* xp = static_cast<const float*>(d.x) + (int64_t)g * d.x_group_stride +
+                    (int64_t)(d.x_row_index ? d.x_row_index[tok] : tok) * d.x_row_stride;
+  const float* wp[OB];
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+    wp[o] = static_cast<const float*>(d.w) + (int64_t)g * d.w_group_stride + (int64_t)min(m0 + o * 16 + l15, d.m - 1) * d.w_m_stride;
+  const int K = d.k, np = (K + 31) >> 5, mine = ks < np ? (np - ks + wk - 1) / wk : 0;   // pieces of k; those of this wave
+  f32x4 acc[OB][2];
+#pragma unroll
+  for (int o = 0; o < OB; ++o) acc[o][0] = acc[o][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Set { f32x4 x[CH][2], w[CH][OB][2]; } A, B;
+  auto issue = [&](int i0, Set& s) {                          // past the wave's pieces or K: a valid chunk, not multiplied
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int k = (ks + min(i0 + c, mine - 1) * wk) * 32 + gq * 8, kc = k < K ? k : 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        s.x[c][h] = *reinterpret_cast<const f32x4*>(xp + kc + 4 * h);
+#pragma unroll
+        for (int o = 0; o < OB; ++o) s.w[c][o][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(wp[o] + kc + 4 * h));
+      }
+    }
+  };
+  auto compute = [&](int i0, const Set& s) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (i0 + c >= mine) continue;
+      const bool past = (ks + (i0 + c) * wk) * 32 + gq * 8 >= K;           // the last piece of a K that is no multiple of 32
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float xv = past ? 0.f : s.x[c][h][e];
+#pragma unroll
+          for (int o = 0; o < OB; ++o)
+            acc[o][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(past ? 0.f : s.w[c][o][h][e], xv, acc[o][e & 1], 0, 0, 0);
+        }
+    }
+  };
+  if (mine > 0) {
+    issue(0, A);
+    issue(CH, B);
+    for (int i0 = 0; i0 < mine; i0 += 2 * CH) {
+      compute(i0, A);
+      if (i0 + 2 * CH < mine) issue(i0 + 2 * CH, A);
+      if (i0 + CH >= mine) break;
+      compute(i0 + CH, B);
+      if (i0 + 3 * CH < mine) issue(i0 + 3 * CH, B);
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < OB; ++o) red[wave][o][lane] = acc[o][0] + acc[o][1];   // outputs 4 (lane >> 4) .. of the block, row lane & 15
+  __syncthreads();
+  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
+  const float* part = reinterpret_cast<const float*>(red);
+  for (int e = tid; e < per_wg * nrows; e += 512) {           // consecutive threads: consecutive outputs of one row
+    const int out = e % per_wg, r = e / per_wg;
+    const int m = blockIdx.y * per_wg + out;
+    if (m >= d.m) continue;
+    const int b = out / (OB * 16), o = (out >> 4) % OB, j = out & 15;
+    const int at = (o * 64 + (j >> 2) * 16 + r) * 4 + (j & 3);
+    float v = part[b * wk * OB * 256 + at];
+    for (int w = 1; w < wk; ++w) v += part[(b * wk + w) * OB * 256 + at];
+    const int p = row0 + r;
+    if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+    else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
+    else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
+      v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)(d.x_row_index ? d.x_row_index[p] : p) * d.gate_row_stride + g));
+    st(Y + (int64_t)(d.y_row_index ? d.y_row_index[p] : p) * d.y_row_stride + m, v);
+  }
+}
+template <typename TY, typename TG>
+static void rows_f32_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
+  const int np = ceil_div(d.k, 32), wk = np >= 16 ? 8 : np >= 8 ? 4 : np >= 4 ? 2 : 1;
+  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, kRowsMax), groups = d.tile_group ? 1 : d.groups;   // | 1: as above
+  const int blocks = ceil_div(d.m, 16 * (8 / wk));
+  const bool two = (long)row_tiles * groups * blocks >= 4L * device_cus();
+  if (two) gemm_rows_f32_kernel<TY, TG, 2><<<dim3(row_tiles, ceil_div(blocks, 2), groups), 512, 0, s>>>(d, wk);
+  else gemm_rows_f32_kernel<TY, TG, 1><<<dim3(row_tiles, blocks, groups), 512, 0, s>>>(d, wk);
+}
+
 // ------------------------------------------------------------------ fp32 tiles on the fp32 matrix cores (fp32 operands, k contiguous)
 // v_mfma_f32_16x16x4_f32 multiplies and adds in fp32 - the products of the FMA form, summed four k at a time - at the vector units' own peak,
 // without their operand traffic: a lane's 16-byte LDS read feeds four instructions.  TR rows x 64 outputs per workgroup, wave w the
@@ -752,13 +860,28 @@ static bool gemm_strided_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
         return true;
       }
     }
-    constexpr bool kWide = std::is_same<TW, float>::value;    // bf16 weights reach the FMA form with one row only
-    const int R = tr <= 1 ? 1 : tr <= 4 ? 4 : tr <= 8 ? 8 : 0;
-    if (R && (size_t)R * d.k * sizeof(float) <= 150 * 1024) {
-      if (R == 1) { if (gate32) rows_form_launch<TX, TW, TY, float, 1>(d, s); else rows_form_launch<TX, TW, TY, uint16_t, 1>(d, s); return true; }
-      if constexpr (kWide) {
-        if (gate32) { if (R == 4) rows_form_launch<TX, TW, TY, float, 4>(d, s); else rows_form_launch<TX, TW, TY, float, 8>(d, s); }
-        else { if (R == 4) rows_form_launch<TX, TW, TY, uint16_t, 4>(d, s); else rows_form_launch<TX, TW, TY, uint16_t, 8>(d, s); }
+    if constexpr (std::is_same<TW, float>::value) {
+      if (tr <= kRowsMax) {
+        // Few rows by FMA, which needs no more than the rows' own products: 1024 x 1024 weights and 1 / 2 / 4 rows 4.1 / 4.4 / 6.1 us against
+        // 6.3 / 6.4 / 6.6 on the matrix cores, 8 rows 9.0 / 7.1, 16 rows 17.1 / 7.9; 6144 x 1024 and 8 rows 16.5 / 10.8, 32 768 x 1024 54.9 / 35.8.
+        // Beyond two chunks of k the rows' way through LDS costs more than that: 4096 x 12 288 and 3 rows 178 / 46 us.
+        const int R = tr <= 1 ? 1 : d.k > 2 * kRowsFormChunk ? 0 : tr <= 2 ? 2 : tr <= 4 ? 4 : 0;
+        auto run = [&](auto gate) {
+          using TG = std::remove_pointer_t<decltype(gate)>;
+          if (R == 1) rows_form_launch<TX, TW, TY, TG, 1>(d, s);
+          // two rows of their own where workgroups are small (5.7 -> 4.4 us at 1024 x 1024); 65 536 x 2048 took 117 us so, 105 with four
+          else if (R == 2 && rows_form_fine(d, 2)) rows_form_launch<TX, TW, TY, TG, 2>(d, s);
+          else if (R) rows_form_launch<TX, TW, TY, TG, 4>(d, s);
+          else rows_f32_launch<TY, TG>(d, s);
+        };
+        if (gate32) run((float*)nullptr);
+        else run((uint16_t*)nullptr);
+        return true;
+      }
+    } else if constexpr (std::is_same<TX, float>::value) {
+      if (tr <= 1) {
+        if (gate32) rows_form_launch<TX, TW, TY, float, 1>(d, s);
+        else rows_form_launch<TX, TW, TY, uint16_t, 1>(d, s);
         return true;
       }
     }

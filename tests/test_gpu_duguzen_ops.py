@@ -356,6 +356,36 @@ def test_matrix_core_form_sees_a_far_key_and_masks_an_unseen_one():
             assert float(o[0][:, 3].abs().max()) < 1.0
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 16])
+@pytest.mark.parametrize("M,K", [(1, 8), (15, 40), (129, 520), (40, 2056), (33, 4104), (8200, 72)])
+def test_few_rows_of_fp32_weights(T, M, K):
+    """FMA with one, two and four rows and the fp32 matrix cores, a K that ends inside a piece, a chunk and beyond two of them (what lies behind it in
+    the wider rows is no number), gathered and scattered rows, also from an expert table: sums of K products of about one in fp32"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(T * 1000 + M + K)
+    x, w = torch.full((T + 2, K + 8), float("nan")), torch.full((3, M, K + 8), float("nan"))
+    x[:, :K], w[..., :K] = torch.randn(T + 2, K, generator=g), torch.randn(3, M, K, generator=g)
+    xd, wd = x.cuda(), w.cuda()
+    base = dict(x=xd.data_ptr(), w=wd.data_ptr(), x_dtype=1, w_dtype=1, y_dtype=1, m=M, k=K, x_row_stride=K + 8, w_m_stride=K + 8, w_k_stride=1,
+                w_group_stride=M * (K + 8), epilogue=B.EPI_RELU_SQ)
+    src, dst = torch.randperm(T + 2, generator=g)[:T].int(), torch.randperm(T, generator=g).int()
+    src_d, dst_d = src.cuda(), dst.cuda()
+    y = torch.full((T, 3 * M), -7.0, device="cuda")
+    B.gemm_strided(B.GemmDesc(y=y.data_ptr(), rows=T, groups=3, y_row_stride=3 * M, y_group_stride=M, x_row_index=src_d.data_ptr(),
+                              y_row_index=dst_d.data_ptr(), **base))
+    ref = torch.relu(torch.einsum("tk,gmk->tgm", x[src.long(), :K].double(), w[..., :K].double())) ** 2
+    tol = 1e-6 * K * (1 + ref.sqrt().max())
+    assert float((y.cpu().double()[dst.long()].reshape(T, 3, M) - ref).abs().max()) < tol
+    expert = torch.randint(0, 3, (T, 1), generator=g, dtype=torch.int32)
+    pos_pair, pos_row, tg, t0, tr, nt, max_tiles = B.route_sort(expert.cuda(), 3)
+    y = torch.full((T, M), float("nan"), device="cuda")
+    B.gemm_strided(B.GemmDesc(y=y.data_ptr(), y_row_stride=M, tile_group=tg.data_ptr(), tile_row0=t0.data_ptr(), tile_rows=tr.data_ptr(),
+                              n_tiles=nt.data_ptr(), max_tiles=max_tiles, max_tile_rows=T, x_row_index=pos_row.data_ptr(), y_row_index=pos_pair.data_ptr(),
+                              **base))
+    ref = torch.relu(torch.einsum("tk,tmk->tm", x[:T, :K].double(), w[expert[:, 0].long(), :, :K].double())) ** 2
+    assert float((y.cpu().double() - ref).abs().max()) < tol
+
+
 @pytest.mark.parametrize("xd,yd", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "bfloat16"), ("float32", "float32")])
 @pytest.mark.parametrize("T,M,K,G", [(17, 128, 8, 1), (65, 130, 56, 2), (128, 127, 64, 3), (129, 300, 72, 1), (200, 1, 200, 2), (513, 514, 136, 40)])
 def test_tiles_on_the_matrix_cores_at_their_edges(T, M, K, G, xd, yd):
