@@ -14,6 +14,8 @@
 //   matrix_memory_kernel   m' = max(f + m, i);  S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise;  o = S^T q / (max(|n.q|, e^-m') + 1e-6)
 // A row's result depends only on the rows before it in its own request: the token order is fixed, and cutting a prompt into
 // steps only moves where the state passes through HBM (exactly, it is fp32 either way).
+#include <algorithm>
+
 #include "common.h"
 #include "typed.h"
 #include "recurrent_core.h"
@@ -25,7 +27,8 @@ __device__ __forceinline__ float softplus_f(float x) { return x > 20.0f ? x : lo
 __device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
 
 // Per row, before the recurrence: q and k heads made unit vectors in place (x / sqrt(sum(x^2) + 1e-6), q also * dim^-1/2),
-// gates[row] = [g: heads | beta: heads].  One workgroup per row, a wave per head.
+// gates[row] = [g: heads | beta: heads].  A wave per head; a row's heads and gates are dealt over gridDim.y workgroups (few rows: as many
+// as its heads fill - one workgroup took 10.0 us for a row of 32 heads of 128, eight take 4.2 us; from 256 rows on one).
 template <typename A>
 __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                          int64_t proj_stride, int64_t b_off, int64_t a_off,
@@ -34,7 +37,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ qkv
   const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   float* qk = qkv + (int64_t)row * qkv_stride;
   const float qs = 1.0f / sqrtf((float)dim);
-  for (int hh = wave; hh < 2 * G; hh += 4) {
+  for (int hh = blockIdx.y * 4 + wave; hh < 2 * G; hh += 4 * gridDim.y) {
     float* x = qk + (int64_t)hh * dim;
     float ss = 0.f;
     for (int d = lane; d < dim; d += 64) ss = fmaf(x[d], x[d], ss);
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ qkv
     for (int d = lane; d < dim; d += 64) x[d] *= sc;
   }
   const A* pr = proj + (int64_t)row * proj_stride;
-  for (int h = threadIdx.x; h < H; h += 256) {
+  for (int h = blockIdx.y * 256 + threadIdx.x; h < H; h += 256 * gridDim.y) {
     gates[(int64_t)row * 2 * H + h] = expf(-expf(ld(A_log + h)) * softplus_f(ld(pr + a_off + h) + ld(dt_bias + h)));
     gates[(int64_t)row * 2 * H + H + h] = sigmoid_f(ld(pr + b_off + h));
   }
@@ -59,7 +62,7 @@ __global__ __launch_bounds__(256) void delta_prep_channel_kernel(float* __restri
   const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   float* qk = qkv + (int64_t)row * qkv_stride;
   const float qs = 1.0f / sqrtf((float)dim);
-  for (int hh = wave; hh < 2 * G; hh += 4) {
+  for (int hh = blockIdx.y * 4 + wave; hh < 2 * G; hh += 4 * gridDim.y) {
     float* x = qk + (int64_t)hh * dim;
     float ss = 0.f;
     for (int d = lane; d < dim; d += 64) ss = fmaf(x[d], x[d], ss);
@@ -68,9 +71,9 @@ __global__ __launch_bounds__(256) void delta_prep_channel_kernel(float* __restri
   }
   const A* pr = proj + (int64_t)row * proj_stride;
   float* gr = gates + (int64_t)row * ((int64_t)H * dim + H);
-  for (int i = threadIdx.x; i < H * dim; i += 256)
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < H * dim; i += 256 * gridDim.y)
     gr[i] = expf(-expf(ld(A_log + i / dim)) * softplus_f(a[(int64_t)row * a_stride + i] + ld(dt_bias + i)));
-  for (int h = threadIdx.x; h < H; h += 256) gr[(int64_t)H * dim + h] = sigmoid_f(ld(pr + b_off + h));
+  for (int h = blockIdx.y * 256 + threadIdx.x; h < H; h += 256 * gridDim.y) gr[(int64_t)H * dim + h] = sigmoid_f(ld(pr + b_off + h));
 }
 
 // CH: the decay is one number per (head, key channel) - it scales the ROWS of S - and the gates row is laid out as
@@ -274,6 +277,9 @@ using namespace pk;
 
 #define PK_BAD ((pegainfer_status_t)hipErrorInvalidValue)
 
+// workgroups per row of the launches before the recurrence
+static int prep_parts(int rows, int heads) { return rows >= 256 ? 1 : std::max(1, std::min(ceil_div(heads, 4), 1024 / rows)); }
+
 pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
                                         int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
                                         int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
@@ -284,7 +290,7 @@ pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const vo
     return PK_BAD;
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        delta_prep_kernel<A><<<n_rows, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off,
+        delta_prep_kernel<A><<<dim3(n_rows, prep_parts(n_rows, 2 * kv_heads)), 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off,
                                                                     a_off, static_cast<const A*>(A_log),
                                                                     static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim);
       }))
@@ -310,7 +316,7 @@ pegainfer_status_t pegainfer_delta_rule_channel(float* qkv, int64_t qkv_stride, 
     return PK_BAD;
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        delta_prep_channel_kernel<A><<<n_rows, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride,
+        delta_prep_channel_kernel<A><<<dim3(n_rows, prep_parts(n_rows, 2 * kv_heads)), 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride,
                                                                             b_off, a, a_stride, static_cast<const A*>(A_log),
                                                                             static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim);
       }))
