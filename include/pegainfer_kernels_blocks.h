@@ -528,6 +528,32 @@ typedef struct {
 } pegainfer_ssd_scan_desc;
 int64_t pegainfer_ssd_scan_workspace(int32_t n_chunks, int32_t heads, int32_t n_state, int32_t vdim);
 pegainfer_status_t pegainfer_ssd_scan_form(const pegainfer_ssd_scan_desc* d, pegainfer_stream_t stream);
+/* The matrix memory with the entries of the tables in chunks (as pegainfer_ssd_scan_form).
+ * workspace: pegainfer_gated_matrix_memory_workspace(...) floats. */
+typedef struct {
+  const void* proj;
+  int64_t proj_stride, q_off, k_off, v_off, i_off, f_off;
+  const void *i_bias, *f_bias;
+  float cap;
+  float* state;
+  int64_t slot_stride;
+  float* o;
+  int32_t heads, dim, vdim;
+  const int32_t* entry_row0;
+  const int32_t* entry_slot;
+  int32_t n_entries;
+  int32_t scan_max;
+  const int32_t* chunk_row0;
+  const int32_t* chunk_rows;
+  int32_t n_chunks;
+  const int32_t* long_chunk0;
+  const int32_t* long_slot;
+  int32_t n_long;
+  float* workspace;
+  int32_t dtype;
+} pegainfer_gated_matrix_memory_desc;
+int64_t pegainfer_gated_matrix_memory_workspace(int32_t n_chunks, int32_t heads, int32_t dim, int32_t vdim);
+pegainfer_status_t pegainfer_gated_matrix_memory_form(const pegainfer_gated_matrix_memory_desc* d, pegainfer_stream_t stream);
 /* Gated linear attention: the same state with a decay per (head, key channel) and token that acts on the rows of S.
  * Per row of `proj` (dtype): q at q_off, k at k_off (heads x dim), v at v_off (heads x vdim);  z: fp32 [rows][heads * dim] at z_stride,
  * z_bias [heads * dim] of dtype or NULL:

@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "row_tiles.h"
 #include "seq_state.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
@@ -76,6 +77,9 @@ static inline float host_bf2f(uint16_t h) {
 
 constexpr int kPageSize = 16;        // tokens per cache page, as in the other runtimes
 constexpr float kGluAlpha = 1.702f;  // the clamp-GLU's sigmoid slope, fixed by the design
+// longest entry whose matrix memory runs token by token: 8 heads of 128 x 256, scan / chunks 42 / 48 us at 96 tokens, 54 / 50 at 128,
+// 222 / 65 at 512; eight entries of 64 tokens 57 / 62, of 128 96 / 71
+constexpr int kScanMax = 112;
 constexpr int kAttRows = 16;         // (token, query head) rows of one attention workgroup
 
 enum { kDelta = 1, kParallel = 2 };
@@ -153,6 +157,8 @@ struct Model {
   uint8_t* top1_state = nullptr;
   uint8_t *meta_host = nullptr, *meta_dev = nullptr;
   uint8_t* sample_scratch = nullptr;
+  float* chunk_ws = nullptr;   // states between the chunks of long entries
+  size_t chunk_cap = 0;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -669,6 +675,25 @@ struct Model {
     cap_rows = n;
     return 0;
   }
+  bool has_memory() const {
+    for (auto& l : layers)
+      if (l.mm.heads > 0) return true;
+    return false;
+  }
+  int ensure_chunks(int n) {
+    size_t need = 0;
+    if (n > 0)
+      for (auto& l : layers)
+        if (l.mm.heads > 0) need = std::max(need, (size_t)pegainfer_gated_matrix_memory_workspace(n, l.mm.heads, l.mm.dim, l.mm.vdim));
+    if (need <= chunk_cap) return 0;
+    FZ_HIP(hipStreamSynchronize(stream));
+    if (chunk_ws) (void)hipFree(chunk_ws);
+    chunk_ws = nullptr;
+    chunk_cap = 0;
+    FZ_HIP(hipMalloc(reinterpret_cast<void**>(&chunk_ws), need * 4));
+    chunk_cap = need;
+    return 0;
+  }
   int ensure_want(size_t n) {
     if (n <= cap_want) return 0;
     FZ_HIP(hipStreamSynchronize(stream));
@@ -789,6 +814,12 @@ struct Model {
       tile_cnt[k] = cnt;
       words += 4 * cnt;
     }
+    // long entries of the matrix memory in chunks (never part of a captured step)
+    const ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
+    const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
+    size_t chunk_off[4];
+    for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
+    if (ensure_chunks((int)chunks.row0.size())) return -1;
     const size_t o_pages = words;
     words += total_pages;
     if (words > cap_meta) {
@@ -826,6 +857,7 @@ struct Model {
       mh[o_ind + n] = (int32_t)pg;
       mh[o_rows] = (int32_t)T;
       for (int i = 0; i < W; ++i) mh[o_want + i] = want[i];
+      for (int k = 0; k < 4; ++k) std::copy(chunk_cols[k]->begin(), chunk_cols[k]->end(), mh + chunk_off[k]);
       for (size_t k = 0; k < tile_sets.size(); ++k) {
         const int per = tile_sets[k].per;
         int32_t *t_row0 = mh + tile_off[k], *t_ntok = t_row0 + tile_cnt[k], *t_qh0 = t_ntok + tile_cnt[k], *t_nqh = t_qh0 + tile_cnt[k];
@@ -963,8 +995,16 @@ struct Model {
                                          a.kv, a.dim, a.vdim, a.scale, c.left_scale, tb, tb + tile_cnt[ts], tb + 2 * tile_cnt[ts],
                                          tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, c.mix_cols, dtype, S()));
         }
-        FZ_K(pegainfer_gated_matrix_memory(proj, Mp, c.o_rq, c.o_rk, c.o_rv, c.o_ri, c.o_rf, w.i_bias, w.f_bias, r.cap,
-                                           state + c.st_mem, slot_stride, o32, r.heads, r.dim, r.vdim, d_row0, d_slot, n, dtype, S()));
+        pegainfer_gated_matrix_memory_desc mm{};
+        mm.proj = proj; mm.proj_stride = Mp;
+        mm.q_off = c.o_rq; mm.k_off = c.o_rk; mm.v_off = c.o_rv; mm.i_off = c.o_ri; mm.f_off = c.o_rf;
+        mm.i_bias = w.i_bias; mm.f_bias = w.f_bias; mm.cap = r.cap; mm.state = state + c.st_mem; mm.slot_stride = slot_stride; mm.o = o32;
+        mm.heads = r.heads; mm.dim = r.dim; mm.vdim = r.vdim;
+        mm.entry_row0 = d_row0; mm.entry_slot = d_slot; mm.n_entries = n; mm.scan_max = kScanMax;
+        mm.chunk_row0 = md + chunk_off[0]; mm.chunk_rows = md + chunk_off[1]; mm.n_chunks = (int)chunks.row0.size();
+        mm.long_chunk0 = md + chunk_off[2]; mm.long_slot = md + chunk_off[3]; mm.n_long = (int)chunks.slot.size();
+        mm.workspace = chunk_ws; mm.dtype = dtype;
+        FZ_K(pegainfer_gated_matrix_memory_form(&mm, S()));
         FZ_K(pegainfer_head_rms_gate(o32, w.rnorm, 1, at(proj, (size_t)c.o_rg), Mp, 1, c.right_scale, eps,
                                      at(mix, (size_t)a.heads * a.vdim), c.mix_cols, r.heads, r.vdim, Ti, dtype, S()));
       }
@@ -1129,6 +1169,7 @@ struct Model {
     free_all(&owned);
     free_all(&step_owned);
     free_all(&want_owned);
+    if (chunk_ws) (void)hipFree(chunk_ws);
     if (tap) (void)hipFree(tap);
     if (meta_dev) (void)hipFree(meta_dev);
     if (meta_host) (void)hipHostFree(meta_host);

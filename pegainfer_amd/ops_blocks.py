@@ -261,14 +261,16 @@ def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_hea
     return o
 
 
-def gated_matrix_memory(proj, offs, i_bias, f_bias, cap, state, heads, dim, vdim, rg):
+def gated_matrix_memory(proj, offs, i_bias, f_bias, cap, state, heads, dim, vdim, rg, scan_max=0):
     """proj [rows, *] with q / k / v / i / f at the column offsets `offs`; state fp32 [slots, heads (dim vdim + dim + 1)] laid
-    out [S of all heads | n of all heads | m of all heads]; returns o fp32 [rows, heads * vdim]"""
+    out [S of all heads | n of all heads | m of all heads]; scan_max > 0: entries of more rows take the chunk form; returns o fp32
+    [rows, heads * vdim]"""
     o = torch.empty((proj.shape[0], heads * vdim), dtype=torch.float32, device=proj.device)
-    _chk(ffi.lib().pegainfer_gated_matrix_memory(_p(proj), proj.stride(0), offs[0], offs[1], offs[2], offs[3], offs[4], _p(i_bias),
-                                                 _p(f_bias), float(cap), _p(state), state.stride(0), _p(o), heads, dim, vdim,
-                                                 _p(rg.entry_row0), _p(rg.entry_slot), rg.n, _dt(proj), _stream()),
-         "gated_matrix_memory")
+    d = MatrixMemoryDesc(proj=_p(proj), proj_stride=proj.stride(0), q_off=offs[0], k_off=offs[1], v_off=offs[2], i_off=offs[3], f_off=offs[4],
+                         i_bias=_p(i_bias), f_bias=_p(f_bias), cap=float(cap), state=_p(state), slot_stride=state.stride(0), o=_p(o), heads=heads,
+                         dim=dim, vdim=vdim, entry_row0=_p(rg.entry_row0), entry_slot=_p(rg.entry_slot), n_entries=rg.n, dtype=_dt(proj))
+    keep = _chunk_tables(d, rg, scan_max, ffi.lib().pegainfer_gated_matrix_memory_workspace, heads, dim, vdim)  # noqa: F841 (alive until enqueued)
+    _chk(ffi.lib().pegainfer_gated_matrix_memory_form(ctypes.addressof(d), _stream()), "gated_matrix_memory")
     return o
 
 
@@ -517,6 +519,10 @@ LatentPrepDesc = _struct("LatentPrepDesc", [("p", "dkv"), ("l", "dkv_stride"), (
 StreamMixDesc = _struct("StreamMixDesc", [("p", "x_in embed token_ids"), ("f", "embed_scale"), ("p", "row_index y"), ("l", "y_row_stride"),
                                           ("p", "mix out_w"), ("f", "mult"), ("p", "x_out sum_out read_w gain n_out"), ("f", "eps"),
                                           ("i", "norm_kind streams d rows dtype")])
+MatrixMemoryDesc = _struct("MatrixMemoryDesc", [("p", "proj"), ("l", "proj_stride q_off k_off v_off i_off f_off"), ("p", "i_bias f_bias"), ("f", "cap"),
+                                                ("p", "state"), ("l", "slot_stride"), ("p", "o"), ("i", "heads dim vdim"),
+                                                ("p", "entry_row0 entry_slot"), ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"),
+                                                ("i", "n_chunks"), ("p", "long_chunk0 long_slot"), ("i", "n_long"), ("p", "workspace"), ("i", "dtype")])
 SsdScanDesc = _struct("SsdScanDesc", [("p", "xbc"), ("l", "xbc_stride"), ("p", "proj"), ("l", "proj_stride dt_off"), ("p", "A_log dt_bias D state"),
                                       ("l", "slot_stride"), ("p", "o"), ("i", "heads groups n_state vdim"), ("p", "entry_row0 entry_slot"),
                                       ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"), ("i", "n_chunks"), ("p", "long_chunk0 long_slot"),

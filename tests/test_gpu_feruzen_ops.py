@@ -323,3 +323,48 @@ def test_matrix_memory_keeps_a_far_strong_write_and_resets_with_its_slot():
     mem.zero_()
     again = Bk.gated_matrix_memory(proj[:3].cuda().contiguous(), offs, zero, zero, 15.0, mem, 1, d, dv, Bk.Ragged([3]))
     assert float((again.cpu() - torch.cat(outs)[:3].cpu()).abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 256), (3, 16, 8), (1, 20, 33), (2, 256, 130)])
+def test_matrix_memory_chunks_against_the_scan_in_64_bits(dtype, heads, dim, vdim):
+    """portions around the 64 tokens of a chunk beside one that stays with the scan, a state, its norm and its maximum left from before, odd sizes;
+    gates that open and close by turns, so the maximum jumps.  The scan in 64 bits from the stored operands is the reference; outputs are
+    quotients, so their error is that of a weighted mean of values of about one."""
+    from pegainfer_amd import ops_blocks as Bk
+    g = torch.Generator().manual_seed(dim + vdim)
+    lens, slots, cap = [64, 3, 65, 320, 127], [1, 4, 0, 3, 5], 15.0
+    T, cols = sum(lens), heads * (2 * dim + vdim + 2)
+    proj = C.bf16_round(torch.randn(T, cols + 1, generator=g))
+    offs = [1, 1 + heads * dim, 1 + 2 * heads * dim, 1 + heads * (2 * dim + vdim), 1 + heads * (2 * dim + vdim + 1)]
+    proj[:, offs[3]:] *= 4
+    ib, fb = C.bf16_round(torch.randn(heads, generator=g)), C.bf16_round(torch.randn(heads, generator=g) + 2)
+    per = heads * (dim * vdim + dim + 1)
+    state = torch.randn(6, per, generator=g).cuda()
+    before = state.cpu().double()
+    td = DT[dtype]
+    y = Bk.gated_matrix_memory(proj.cuda().to(td), offs, ib.cuda().to(td), fb.cuda().to(td), cap, state, heads, dim, vdim, Bk.Ragged(lens, slots=slots), scan_max=32)
+    y, after, at = y.cpu().double(), state.cpu().double(), 0
+    P = proj.double()
+    for n, s in zip(lens, slots):
+        for h in range(heads):
+            S = before[s, h * dim * vdim:(h + 1) * dim * vdim].view(dim, vdim).clone()
+            N = before[s, heads * dim * vdim + h * dim:][:dim].clone()
+            m = before[s, heads * dim * (vdim + 1) + h].clone()
+            for t in range(n):
+                row = P[at + t]
+                q, k, v = row[offs[0] + h * dim:][:dim] * dim ** -0.5, row[offs[1] + h * dim:][:dim], row[offs[2] + h * vdim:][:vdim]
+                i = cap * torch.tanh((row[offs[3] + h] + ib[h].double()) / cap)
+                f = torch.nn.functional.logsigmoid(cap * torch.tanh((row[offs[4] + h] + fb[h].double()) / cap))
+                mn = torch.maximum(f + m, i)
+                a, b = torch.exp(f + m - mn), torch.exp(i - mn)
+                S, N, m = a * S + b * torch.outer(k, v), a * N + b * k, mn
+                den = torch.maximum((N @ q).abs(), torch.exp(-m)) + 1e-6
+                ref = (S.T @ q) / den
+                scale = float(((S.abs().T @ q.abs()) / den).max())
+                assert float((y[at + t, h * vdim:(h + 1) * vdim] - ref).abs().max()) < 2e-5 * max(1.0, scale), (n, h, t)
+            assert float((after[s, h * dim * vdim:(h + 1) * dim * vdim].view(dim, vdim) - S).abs().max()) < 2e-5 * max(1.0, float(S.abs().max()))
+            assert float((after[s, heads * dim * vdim + h * dim:][:dim] - N).abs().max()) < 2e-5 * max(1.0, float(N.abs().max()))
+            assert abs(float(after[s, heads * dim * (vdim + 1) + h] - m)) < 2e-5 * max(1.0, abs(float(m)))
+        at += n
+    assert torch.equal(after[2], before[2])
