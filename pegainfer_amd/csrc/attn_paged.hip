@@ -320,28 +320,35 @@ __global__ __launch_bounds__(256) void paged_attention_kernel(
         const A* vp = cache + pg + v_cache_off + ((int64_t)(p % page_size) * G + g) * vdim;
         float* dk = s_k + j * kd;
         float* dv = s_v + j * vdim;
-        if (vec_k) {
-          for (int d = sub * 8; d < kw; d += 32) {
-            float t[8];
-            Vec8<A>::load(kp + d, t);
+        if (vec_k && vec_v) {
+          // 128 values of the key and of the value requested before the first is stored (one chunk at a time: 19.4 -> 17.0 us for two decoded
+          // fp32 tokens of 8 heads of 128, 77 -> 70 us for their prompts of 470)
+          for (int d0 = sub * 8; d0 < max(kw, vdim); d0 += 128) {
+            float tk[4][8], tv[4][8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) dk[d + u] = t[u];
-          }
-        } else {
-          for (int d = sub; d < kw; d += 4) dk[d] = ld(kp + d);
-        }
-        if (vec_v) {
-          for (int d = sub * 8; d < vdim; d += 32) {
-            float t[8];
-            Vec8<A>::load(vp + d, t);
+            for (int c = 0; c < 4; ++c) {
+              if (d0 + 32 * c < kw) Vec8<A>::load(kp + d0 + 32 * c, tk[c]);
+              if (d0 + 32 * c < vdim) Vec8<A>::load(vp + d0 + 32 * c, tv[c]);
+            }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) dv[d + u] = t[u];
-            if (tail && d >= kw) {
+            for (int c = 0; c < 4; ++c) {
+              const int d = d0 + 32 * c;
+              if (d < kw) {
 #pragma unroll
-              for (int u = 0; u < 8; ++u) dk[d + u] = t[u];
+                for (int u = 0; u < 8; ++u) dk[d + u] = tk[c][u];
+              }
+              if (d < vdim) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) dv[d + u] = tv[c][u];
+                if (tail && d >= kw) {
+#pragma unroll
+                  for (int u = 0; u < 8; ++u) dk[d + u] = tv[c][u];
+                }
+              }
             }
           }
         } else {
+          for (int d = sub; d < kw; d += 4) dk[d] = ld(kp + d);
           for (int d = sub; d < vdim; d += 4) {
             const float t = ld(vp + d);
             dv[d] = t;
