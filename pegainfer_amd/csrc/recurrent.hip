@@ -13,7 +13,8 @@
 //   delta_rule_kernel      S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
 //   matrix_memory_kernel   m' = max(f + m, i);  S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise;  o = S^T q / (max(|n.q|, e^-m') + 1e-6)
 // A row's result depends only on the rows before it in its own request: the token order is fixed, and cutting a prompt into
-// steps only moves where the state passes through HBM (exactly, it is fp32 either way).
+// steps only moves where the state passes through HBM (exactly, it is fp32 either way).  The matrix memory also has a form in chunks
+// for long portions (below); which portions take it moves results by rounding only.
 #include <algorithm>
 
 #include "common.h"
