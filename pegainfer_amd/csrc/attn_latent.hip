@@ -455,6 +455,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
 // stay in registers (a wave's own quarter of the entry), so LDS holds the key tile and the tile's scores alone.
 // The fp32 instance works on v_mfma_f32_16x16x4_f32: lane (l15, g) fetches four neighbouring values at 4 g of a 16-wide block with one
 // 16-byte read, and product e of the block takes value e of every lane - both operands numbered alike; its weights stay fp32.
+// A key that a row does not see has weight zero in the products, as in the form above: an entry that is infinite or no number reaches
+// the rows of its request that share its key tile.
 // Bound by the latency of one pass through scores, softmax and values (three barriers per tile of 32 keys), not by memory.
 // With the merge, 16 heads of 512 + 64 and 4 requests of 500 to 900 keys in splits of 32: 17.1 (the form above) -> 15.9 us, 32 requests
 // 53.6 -> 35.0 us.  In fp32, where a workgroup took one head and a thread one key: 8 heads of 256 + 64, two requests of up to 300 keys

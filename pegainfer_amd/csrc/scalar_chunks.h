@@ -7,7 +7,8 @@
 // Decays enter as products of the decays themselves, never as quotients or differences of logarithms: every factor is at most one, nothing
 // cancels however fast a head forgets, and the roundings of a product are those of a scan's state.
 // Products run on v_mfma_f32_16x16x4_f32 (chunk_core.h).  Scores are computed transposed (keys as rows), which leaves lane l with the scores of
-// query l % 16 against keys 4 (l / 16) + r: the A operand of the product with the values.
+// query l % 16 against keys 4 (l / 16) + r: the A operand of the product with the values.  A later key's score is a zero there, so a value
+// that is infinite or no number reaches the tokens before it in its block of 16 (never another entry, whose chunks are its own).
 // An In describes the recurrence: rows() / row_stride() of type Row with q_at, k_at, v_at of a head, q_factor; steps(chunk, head, row0, n, lane,
 // &b, &a): lane i of a wave gets token i's factor and decay (0 and 1 past the chunk's end); H, dim, vdim; kNorm, floor_of, skip: see the outputs.
 #pragma once
