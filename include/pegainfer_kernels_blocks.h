@@ -78,7 +78,7 @@ typedef struct {
   const void* gate;
   int32_t gate_dtype;
   int64_t gate_row_stride;
-  int32_t max_tile_rows;     /* grouped form: an upper bound of tile_rows the caller knows (0 = tile_rows_cap) */
+  int32_t max_tile_rows;     /* grouped form: an upper bound of tile_rows the caller knows (0 = tile_rows_cap); rows of a tile past it may be left out */
   int32_t tile_rows_cap;     /* grouped form: the rows_per_tile the table was cut with (0 = 64) */
   int32_t plain;             /* != 0: always the fp32-FMA tile kernel (exact products of the stored values) */
 } pegainfer_gemm_desc;
@@ -176,7 +176,7 @@ pegainfer_status_t pegainfer_route_sigmoid_grouped(const void* h, const void* w_
                                                    int32_t n_groups, int32_t keep_groups, int32_t top, int32_t rows,
                                                    int32_t dtype, pegainfer_stream_t stream);
 /* Sort the rows * top (row, choice) pairs by expert into a position list and cut it into row tiles of <= rows_per_tile
- * (64 or 128) positions:
+ * (64 or 128; 1 .. 16 for a step of few rows, whose tables are cut at its row count) positions:
  *   pos_pair[p] = pair index (row * top + choice) at position p;  pos_row[p] = its row
  *   tile_group / tile_row0 / tile_rows [max_tiles], *n_tiles;  max_tiles >= ceil(pairs / rows_per_tile) + experts
  * One workgroup, counters in LDS (experts <= 8192).  The order inside an expert is arbitrary; results do not depend on it. */

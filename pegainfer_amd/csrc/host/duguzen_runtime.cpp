@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "row_tiles.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -761,7 +762,7 @@ struct Model {
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     DZ_K(pegainfer_route_sigmoid_grouped(h, w.router, w.corr, route_e, route_w, D, f.experts, f.groups, f.keep, f.top, T, dtype, S()));
     // 128-row tiles for the matrix-core form (bf16, prompt-sized steps), 64-row tiles otherwise
-    const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && f.ff % 8 == 0 ? 128 : 64;
+    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0);
     DZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
     pegainfer_gemm_desc d{};
     d.x = h; d.w = w.gate_up_e; d.y = gu;
@@ -770,10 +771,9 @@ struct Model {
     d.x_row_stride = D; d.w_m_stride = D; d.w_k_stride = 1; d.w_group_stride = (int64_t)2 * f.ff * D;
     d.y_row_stride = 2 * f.ff;
     d.tile_group = t_group; d.tile_row0 = t_row0; d.tile_rows = t_rows; d.n_tiles = n_tiles;
-    d.max_tiles = std::min(P, (P + per_tile - 1) / per_tile + f.experts);   // every tile holds a pair
+    d.max_tiles = ptiles::expert_tiles(T, f.top, f.experts, per_tile);
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
-    d.max_tile_rows = std::min(T, 64);   // a row chooses distinct experts: an expert never gets more pairs than there are rows
     d.plain = plain_kernels;
     DZ_K(pegainfer_gemm_strided(&d, S()));
     DZ_K(pegainfer_silu_mul_rows(gu, act, f.ff, P, dtype, S()));
@@ -785,7 +785,6 @@ struct Model {
     e.y_row_stride = D;
     e.tile_group = t_group; e.tile_row0 = t_row0; e.tile_rows = t_rows; e.n_tiles = n_tiles; e.max_tiles = d.max_tiles;
     e.y_row_index = pos_pair;
-    e.max_tile_rows = d.max_tile_rows;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
     DZ_K(pegainfer_gemm_strided(&e, S()));

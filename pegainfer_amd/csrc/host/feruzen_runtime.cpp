@@ -1079,7 +1079,7 @@ struct Model {
     const MlpCfg& f = c.mlp;
     const int ff = f.glu.ff, P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
-    const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && ff % 8 == 0 ? 128 : 64;
+    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0);
     if (T > 8 || f.experts > 1024) {   // many rows (or more experts than the selection kernel's four rows hold in LDS): one
                                        // workgroup per row does logits and selection
       FZ_K(pegainfer_route_topk(xb, w.router, nullptr, route_e, route_w, D, f.experts, 1, 1, f.top, T, PEGAINFER_SCORE_SOFTMAX, dtype, S()));
@@ -1108,10 +1108,9 @@ struct Model {
     d.x_row_stride = D; d.w_m_stride = D; d.w_k_stride = 1; d.w_group_stride = (int64_t)2 * ff * D;
     d.y_row_stride = 2 * ff;
     d.tile_group = t_group; d.tile_row0 = t_row0; d.tile_rows = t_rows; d.n_tiles = n_tiles;
-    d.max_tiles = std::min(P, (P + per_tile - 1) / per_tile + f.experts);   // every tile holds a pair
+    d.max_tiles = ptiles::expert_tiles(T, f.top, f.experts, per_tile);
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
-    d.max_tile_rows = std::min(T, 64);   // a row chooses distinct experts: an expert never gets more pairs than there are rows
     d.plain = plain_kernels;
     FZ_K(pegainfer_gemm_strided(&d, S()));
     FZ_K(pegainfer_clamp_glu_rows(gu_e, act_e, ff, P, f.glu.limit, kGluAlpha, dtype, S()));
@@ -1123,7 +1122,6 @@ struct Model {
     e.y_row_stride = D;
     e.tile_group = t_group; e.tile_row0 = t_row0; e.tile_rows = t_rows; e.n_tiles = n_tiles; e.max_tiles = d.max_tiles;
     e.y_row_index = pos_pair;
-    e.max_tile_rows = d.max_tile_rows;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
     FZ_K(pegainfer_gemm_strided(&e, S()));

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "row_tiles.h"
 #include "seq_state.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
@@ -1061,7 +1062,7 @@ struct Model {
     const int ff = f.ff, P = T * f.top, E1 = f.experts + 1;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     if (linear_strided(w.router, hb, dtype, D, route_logits, PEGAINFER_DTYPE_F32, E1, T, D)) return -1;
-    const int per_tile = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8 && D % 8 == 0 && ff % 8 == 0 ? 128 : 64;
+    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0);
     pegainfer_route_plan_desc r{};      // selection and sort: one launch for few rows
     r.logits = route_logits; r.logits_stride = E1; r.out_expert = route_e; r.out_weight = route_w;
     r.experts = f.experts; r.n_groups = f.groups; r.keep_groups = f.keep; r.top = f.top; r.rows = T;
@@ -1077,10 +1078,9 @@ struct Model {
     d.x_row_stride = D; d.w_m_stride = D; d.w_k_stride = 1; d.w_group_stride = (int64_t)2 * ff * D;
     d.y_row_stride = 2 * ff;
     d.tile_group = t_group; d.tile_row0 = t_row0; d.tile_rows = t_rows; d.n_tiles = n_tiles;
-    d.max_tiles = std::min(P, (P + per_tile - 1) / per_tile + f.experts);   // every tile holds a pair
+    d.max_tiles = ptiles::expert_tiles(T, f.top, f.experts, per_tile);
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
-    d.max_tile_rows = std::min(T, 64);   // a row chooses distinct experts: an expert never gets more pairs than there are rows
     d.plain = plain_kernels;
     RX_K(pegainfer_gemm_strided(&d, S()));
     RX_K(pegainfer_silu_mul_rows(gu_e, act_e, ff, P, dtype, S()));
@@ -1092,7 +1092,6 @@ struct Model {
     e.y_row_stride = D;
     e.tile_group = t_group; e.tile_row0 = t_row0; e.tile_rows = t_rows; e.n_tiles = n_tiles; e.max_tiles = d.max_tiles;
     e.y_row_index = pos_pair;
-    e.max_tile_rows = d.max_tile_rows;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
     RX_K(pegainfer_gemm_strided(&e, S()));

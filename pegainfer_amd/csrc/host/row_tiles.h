@@ -44,6 +44,17 @@ inline void cut(const int32_t* lens, int n, int per, int rows, size_t tiles, int
       }
 }
 
+// Rows of a tile of the experts' table of a step of T rows.  Up to kFewRows rows the table is cut at T: the GEMMs of few rows take no
+// more than that from a tile, and an expert can have more pairs than there are rows (a row that no expert is eligible for puts all its
+// choices on one).  wide: the GEMMs walk tiles of 128 rows.
+constexpr int kFewRows = 16;
+inline int expert_tile_rows(int T, bool wide) { return T <= kFewRows ? T : wide ? 128 : 64; }
+// most tiles of a step of T rows with `top` choices each: every tile holds a pair
+inline int expert_tiles(int T, int top, int experts, int per_tile) {
+  const int P = T * top;
+  return std::min(P, (P + per_tile - 1) / per_tile + experts);
+}
+
 // the chunks of the entries of more than scan_max rows (pegainfer_decay_attention's tables)
 struct Chunks {
   std::vector<int32_t> row0, rows, first{0}, slot;     // per chunk; per long entry: its first chunk (one more at the end), its state slot

@@ -393,10 +393,9 @@ class Model : public StepModel {
   // h -> the stream, and h of the next layer
   int feed_forward(const StepCtx& s, const LayerCfg& c, const LayerW& w, const void* next) {
     const MoeCfg& f = c.moe;
-    const int T = s.T, P = T * f.top, all = f.experts + f.identity;
-    const bool tuned = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 8;      // many rows in bf16
+    const int T = s.T, all = f.experts + f.identity;
     if (linear_strided(w.router, h, dtype, D, logits_r, PEGAINFER_DTYPE_F32, all + 1, T, D)) return -1;
-    const int per_tile = tuned && D % 8 == 0 && f.ff % 8 == 0 ? 128 : 64;
+    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0);
     pegainfer_route_plan_desc r{};
     r.logits = logits_r; r.logits_stride = all + 1; r.correction = w.correction; r.out_expert = route_e; r.out_weight = route_w;
     r.experts = all; r.n_groups = 1; r.keep_groups = 1; r.top = f.top; r.rows = T; r.score_kind = PEGAINFER_SCORE_SOFTMAX; r.renorm = 1;
@@ -404,11 +403,10 @@ class Model : public StepModel {
     r.sort_experts = f.experts;
     r.pos_pair = pos_pair; r.pos_row = pos_row;
     r.tile_group = tiles; r.tile_row0 = tiles + max_tiles; r.tile_rows = tiles + 2 * max_tiles; r.n_tiles = tiles + 3 * max_tiles;
-    r.max_tiles = std::min(P, (P + per_tile - 1) / per_tile + f.experts); r.rows_per_tile = per_tile; r.dtype = dtype;
+    r.max_tiles = ptiles::expert_tiles(T, f.top, f.experts, per_tile); r.rows_per_tile = per_tile; r.dtype = dtype;
     PSTEP_K(pegainfer_route_plan(&r, S()));
     pegainfer_gemm_desc g{};
     g.tile_group = r.tile_group; g.tile_row0 = r.tile_row0; g.tile_rows = r.tile_rows; g.n_tiles = r.n_tiles; g.max_tiles = r.max_tiles;
-    g.max_tile_rows = std::min(T, 64);   // a row chooses distinct experts: an expert never gets more pairs than there are rows
     g.tile_rows_cap = per_tile;
     g.w_k_stride = 1;
     g.plain = plain_kernels;

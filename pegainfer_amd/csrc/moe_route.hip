@@ -8,7 +8,8 @@
 //                   `top` wave-wide arg-max steps); ties go to the lower index.
 //   sort_kernel     (row, choice) pairs bucketed by expert with LDS counters, an exclusive scan, and the table of <= 64-row
 //                   tiles the grouped GEMM walks.  The order of pairs inside an expert comes from atomics; every pair owns
-//                   its output row, so results do not depend on it.  Tiles hold <= 64 or <= 128 rows, as the GEMM form that walks them wants.
+//                   its output row, so results do not depend on it.  Tiles hold <= 64 or <= 128 rows, as the GEMM form that walks them wants, or no
+//                   more than a step of few rows has: an expert gets more pairs than that when a row without eligible experts fills its choices.
 //   combine_kernel  out[row] = sum over the row's choices, in choice order, of weight * expert output (fp32 sum), plus a row
 //                   every token gets (a shared expert), optionally times the sigmoid of a per-row gate logit.
 // Options of the selection: a group's score = its two largest choices (default) or its largest; the chosen weights as they
@@ -319,6 +320,9 @@ __global__ __launch_bounds__(256) void route_combine_kernel(const float* __restr
 extern "C" {
 using namespace pk;
 
+// 64 or 128, or for few rows whatever no tile of the table may pass
+static bool tile_rows_ok(int n) { return n == 64 || n == 128 || (n >= 1 && n <= 16); }
+
 pegainfer_status_t pegainfer_route_topk(const void* h, const void* w_router, const void* correction, int32_t* out_expert,
                                         float* out_weight, int32_t d, int32_t experts, int32_t n_groups, int32_t keep_groups,
                                         int32_t top, int32_t rows, int32_t score_kind, int32_t dtype, pegainfer_stream_t stream) {
@@ -355,7 +359,7 @@ pegainfer_status_t pegainfer_route_plan(const pegainfer_route_plan_desc* q, pega
     return bad;
   const int64_t pairs = (int64_t)q->rows * top;
   const bool sorted = q->sort_experts > 0;
-  if (sorted && ((q->rows_per_tile != 64 && q->rows_per_tile != 128) || q->sort_experts > 7000 || pairs > 0x7FFFFFFF || !q->pos_pair ||
+  if (sorted && (!tile_rows_ok(q->rows_per_tile) || q->sort_experts > 7000 || pairs > 0x7FFFFFFF || !q->pos_pair ||
                  !q->pos_row || !q->tile_group || !q->tile_row0 || !q->tile_rows || !q->n_tiles ||
                  q->max_tiles < std::min<int64_t>(pairs, (pairs + q->rows_per_tile - 1) / q->rows_per_tile + q->sort_experts)))
     return bad;
@@ -412,7 +416,7 @@ pegainfer_status_t pegainfer_route_sort(const int32_t* expert, int32_t n_pairs, 
                                         int32_t* tile_rows, int32_t* n_tiles, int32_t max_tiles, int32_t rows_per_tile,
                                         pegainfer_stream_t stream) {
   if (n_pairs <= 0) return 0;
-  if ((rows_per_tile != 64 && rows_per_tile != 128) || experts <= 0 || experts > 7000 ||
+  if (!tile_rows_ok(rows_per_tile) || experts <= 0 || experts > 7000 ||
       max_tiles < (n_pairs + rows_per_tile - 1) / rows_per_tile + experts)
     return (pegainfer_status_t)hipErrorInvalidValue;
   const SortOut o{pos_pair, pos_row, tile_group, tile_row0, tile_rows, n_tiles, max_tiles, rows_per_tile};
