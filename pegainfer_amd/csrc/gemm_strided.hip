@@ -152,6 +152,7 @@ __global__ __launch_bounds__(256) void gemm_strided_mfma_kernel(pegainfer_gemm_d
   } else {
     nrows = min(TR, d.rows - row0);
   }
+  if (nrows <= 0) return;                            // a table may hold empty tiles; absent rows repeat the last one below
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
   if (tid < TR) {
     const int p = row0 + min(tid, nrows - 1);
@@ -505,6 +506,7 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
     row0 = blockIdx.x * kRowsMax;
     nrows = min(kRowsMax, d.rows - row0);
   }
+  if (nrows <= 0) return;                                     // an empty tile of a table has no last row to repeat
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
   const int per_wg = 4 / wk * OB * 16;                        // outputs of a workgroup
   const int blk = wave / wk, ks = wave - blk * wk;
@@ -641,6 +643,7 @@ __global__ __launch_bounds__(512) void gemm_rows_f32_kernel(pegainfer_gemm_desc 
     row0 = blockIdx.x * kRowsMax;
     nrows = min(kRowsMax, d.rows - row0);
   }
+  if (nrows <= 0) return;                                     // an empty tile of a table has no last row to repeat
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
   const int per_wg = NW / wk * OB * 16;                       // outputs of a workgroup
   const int blk = wave / wk, ks = wave - blk * wk;

@@ -441,6 +441,26 @@ def test_tiles_of_an_expert_table_reach_every_pair(rows_per_tile):
         assert float((y.cpu().double() - ref).abs().max()) < 1e-6 * K * (1 + float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("known", [1, 4, 16, 0])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_empty_tiles_of_a_table_are_passed_over(dtype, known):
+    """a tile without rows, before the first position, between others and at the end: nothing is read or written for it"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(known)
+    T, M, K = min(known or 40, 5), 70, 72
+    x, w = C.bf16_round(torch.randn(T, K, generator=g)), C.bf16_round(torch.randn(3, M, K, generator=g))
+    xd, wd = dev(x, DT[dtype]), dev(w, DT[dtype])
+    tg, t0, tr, nt = (torch.tensor(v, dtype=torch.int32).cuda() for v in ([2, 0, 1, 1], [0, 0, T, T], [0, T, 0, 0], [4]))
+    rows = torch.arange(T, dtype=torch.int32).flip(0).contiguous()
+    rd = rows.cuda()
+    y = torch.full((T, M), -7.0, device="cuda")
+    B.gemm_strided(B.GemmDesc(x=xd.data_ptr(), w=wd.data_ptr(), y=y.data_ptr(), x_dtype=B._dt(xd), w_dtype=B._dt(wd), y_dtype=1, m=M, k=K, x_row_stride=K,
+                              w_m_stride=K, w_k_stride=1, w_group_stride=M * K, y_row_stride=M, tile_group=tg.data_ptr(), tile_row0=t0.data_ptr(),
+                              tile_rows=tr.data_ptr(), n_tiles=nt.data_ptr(), max_tiles=4, max_tile_rows=known, x_row_index=rd.data_ptr()))
+    ref = x.double()[rows.long()] @ w[0].double().T
+    assert float((y.cpu().double() - ref).abs().max()) < 1e-6 * K * (1 + float(ref.abs().max()))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_strided_gemm_forms_agree(dtype):
     """the few-rows form (<= 8 rows), the matrix-core tile form (bf16 weights) and the fp32-FMA tile form compute the same
