@@ -454,9 +454,11 @@ __device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, bf16x8_t 
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const float x = v[2 * i + e];
-      hi[e] = __builtin_bit_cast(uint32_t, x) & 0xFFFF0000u;
-      // an infinity has no remainder (x - x would be NaN)
-      const float r1 = (hi[e] & 0x7FFFFFFFu) == 0x7F800000u ? 0.f : x - __builtin_bit_cast(float, hi[e]);
+      const uint32_t bits = __builtin_bit_cast(uint32_t, x);
+      hi[e] = bits & 0xFFFF0000u;
+      // an infinity has no remainder (x - x would be NaN); what is no number leaves one that is none, also where its cut-off part alone tells
+      // it from an infinity
+      const float r1 = (bits & 0x7FFFFFFFu) == 0x7F800000u ? 0.f : x - __builtin_bit_cast(float, hi[e]);
       mid[e] = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
       lo[e] = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, mid[e]));
     }

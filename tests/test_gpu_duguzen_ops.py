@@ -551,6 +551,16 @@ def test_few_rows_keep_infinities():
     assert torch.isinf(got[0]).all() and torch.isnan(got[1]).all() and torch.isfinite(got[2]).all()
 
 
+@pytest.mark.parametrize("bits", [0x7F800001, 0xFF80FFFF, 0x7F810000, 0xFFFFFFFF])
+def test_few_rows_keep_what_is_no_number(bits):
+    """whatever the payload, also one that lies in the bits a bf16 does not have"""
+    from pegainfer_amd import ops_blocks as B
+    x, w = torch.ones(3, 72), torch.ones(17, 72)
+    x.view(torch.int32)[1, 70] = np.uint32(bits).astype(np.int32).item()
+    got = B.linear(x.cuda(), w.bfloat16().cuda(), out_dtype=torch.float32).cpu()
+    assert torch.isnan(got[1]).all() and torch.equal(got[0], got[2]) and float(got[0, 0]) == 72.0
+
+
 def test_grouped_gemm_over_128_row_tiles():
     from pegainfer_amd import ops_blocks as B
     g = torch.Generator().manual_seed(11)
