@@ -601,6 +601,16 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
     float v = part[b * wk * OB * 256 + at];
     for (int w = 1; w < wk; ++w) v += part[(b * wk + w) * OB * 256 + at];
     const int p = row0 + r;
+    if constexpr (NP > 1) {
+      // a cut-off part of zero times an infinite weight is no number where the value's own product is an infinity: summed again from whole
+      // values, up to the first that settles it
+      if (v != v) {
+        const TX* xr = X + (int64_t)(d.x_row_index ? d.x_row_index[p] : p) * d.x_row_stride;
+        const uint16_t* wr = W + (int64_t)m * d.w_m_stride;
+        v = 0.f;
+        for (int k = 0; k < K && v == v; ++k) v = fmaf(ld(xr + k), ld(wr + k), v);
+      }
+    }
     if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
     else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
     else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)

@@ -561,6 +561,20 @@ def test_few_rows_keep_what_is_no_number(bits):
     assert torch.isnan(got[1]).all() and torch.equal(got[0], got[2]) and float(got[0, 0]) == 72.0
 
 
+@pytest.mark.parametrize("M", [19, 40003])
+def test_few_rows_against_infinite_weights(M):
+    """finite values times an infinite weight are infinities of their sign, whether a bf16 holds the value or not; zeros and infinities of both signs
+    give no number"""
+    from pegainfer_amd import ops_blocks as B
+    x, w = torch.full((6, 136), 0.7), torch.full((M, 136), 0.5)
+    x[0, 5], x[1, 5], x[2, 5], x[3, 5], x[4, 5] = 1.5, -0.3, 0.0, float("inf"), float("-inf")
+    w[1, 5], w[2, 5] = float("inf"), float("-inf")
+    w[M - 1, 5], w[M - 1, 130] = float("inf"), float("-inf")
+    got = B.linear(x.cuda(), w.bfloat16().cuda(), out_dtype=torch.float32).cpu().double()
+    ref = torch.tensor([[sum((x[r].double() * w[m].double()).tolist()) for m in (0, 1, 2, M - 1)] for r in range(6)], dtype=torch.float64)
+    torch.testing.assert_close(got[:, [0, 1, 2, M - 1]], ref, rtol=1e-5, atol=1e-4, equal_nan=True)
+
+
 def test_grouped_gemm_over_128_row_tiles():
     from pegainfer_amd import ops_blocks as B
     g = torch.Generator().manual_seed(11)
