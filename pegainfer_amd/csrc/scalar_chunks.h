@@ -79,7 +79,10 @@ __global__ __launch_bounds__(256) void scalar_chunk_sum_kernel(In in, ScalarWs w
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) U[(int64_t)(d0 + 4 * lg + r) * vp + 16 * b + l15] = acc[b][r];
+      for (int r = 0; r < 4; ++r) {
+        const int d = d0 + 4 * lg + r;
+        U[(int64_t)d * vp + 16 * b + l15] = d < in.dim ? acc[b][r] : 0.f;    // zeros of padding times an infinity would be no numbers
+      }
   }
 }
 

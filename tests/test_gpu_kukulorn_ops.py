@@ -454,6 +454,21 @@ def test_state_space_chunks_against_the_scan_in_64_bits(dtype, heads, groups, N,
     assert torch.equal(state[2].cpu().double().view(heads, N, P), S[2])          # a slot of nobody
 
 
+@pytest.mark.parametrize("N", [20, 5])
+def test_state_space_chunks_keep_their_padding_zero(N):
+    """state sizes that are no multiple of 16: an infinite value late in a chunk reaches no token of the blocks of 16 before its own"""
+    Bk = B()
+    g = torch.Generator().manual_seed(N)
+    heads, P, T = 2, 33, 128
+    inner = heads * P
+    xbc, proj = torch.randn(T, inner + 2 * N, generator=g), torch.randn(T, heads, generator=g).cuda()
+    xbc[60, 7] = float("inf")
+    args = (proj, 0, torch.tensor([-1.0, 0.5]).cuda(), torch.randn(heads, generator=g).cuda(), torch.randn(heads, generator=g).cuda())
+    y = Bk.ssd_scan(xbc.cuda(), *args, torch.ones(1, heads * N * P).cuda(), heads, 1, N, P, Bk.Ragged([T]), scan_max=32).cpu()
+    assert torch.isfinite(y[:48]).all() and not torch.isfinite(y[60:, 7]).any()
+    assert torch.isfinite(y[:, [i for i in range(inner) if i != 7]]).all()
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
