@@ -7,8 +7,9 @@
 // Decays enter as products of the decays themselves, never as quotients or differences of logarithms: every factor is at most one, nothing
 // cancels however fast a head forgets, and the roundings of a product are those of a scan's state.
 // Products run on v_mfma_f32_16x16x4_f32 (chunk_core.h).  Scores are computed transposed (keys as rows), which leaves lane l with the scores of
-// query l % 16 against keys 4 (l / 16) + r: the A operand of the product with the values.  A later key's score is a zero there, so a value
-// that is infinite or no number reaches the tokens before it in its block of 16 (never another entry, whose chunks are its own).
+// query l % 16 against keys 4 (l / 16) + r: the A operand of the product with the values.  A later key's score is a zero there, so where a
+// block of 16 tokens holds a value that is infinite or no number its own queries take the keys one by one (the product would bring it to the tokens
+// before it): what is spoilt is what a token scan spoils.
 // An In describes the recurrence: rows() / row_stride() of type Row with q_at, k_at, v_at of a head, q_factor; steps(chunk, head, row0, n, lane,
 // &b, &a): lane i of a wave gets token i's factor and decay (0 and 1 past the chunk's end); H, dim, vdim; kNorm, floor_of, skip: see the outputs.
 #pragma once
@@ -228,14 +229,38 @@ __global__ __launch_bounds__(256) void scalar_chunk_out_kernel(In in, ScalarWs w
     }
     s[0] = (s[0] + s[1]) + (s[2] + s[3]);
     const f32x4 w = *reinterpret_cast<const f32x4*>(&s_p[i0 + l15][jb * 16 + 4 * lg]);
+    float p[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int j = jb * 16 + 4 * lg + r;
-      const float p = j <= i0 + l15 ? s[0][r] * w[r] : 0.f;
-      if constexpr (In::kNorm) nq += p;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, s_v[j * sv + 16 * b + l15], acc[b], 0, 0, 0);
+      p[r] = jb * 16 + 4 * lg + r <= i0 + l15 ? s[0][r] * w[r] : 0.f;
+      if constexpr (In::kNorm) nq += p[r];
     }
+    const float* vr = s_v + (jb * 16 + 4 * lg) * sv + l15;
+    if (jb == wave) {
+      bool spoilt = false;                           // a value that is infinite or no number: not for the queries before it
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) spoilt |= !(fabsf(vr[r * sv + 16 * b]) <= __FLT_MAX__);
+      if (__any(spoilt)) {
+        for (int k = 0; k < 16; ++k)                 // one key after the other, each query row of this lane on its own
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int src = (k >> 2) * 16 + 4 * lg + r;                     // the lane that holds p of query 4 lg + r and key k
+            const float a = __shfl(p[0], src, kWave), c = __shfl(p[1], src, kWave), d = __shfl(p[2], src, kWave), e = __shfl(p[3], src, kWave);
+            const float pk = (k & 2) ? ((k & 1) ? e : d) : ((k & 1) ? c : a);
+            if (k <= 4 * lg + r) {
+#pragma unroll
+              for (int b = 0; b < 4; ++b) acc[b][r] = fmaf(pk, s_v[(jb * 16 + k) * sv + 16 * b + l15], acc[b][r]);
+            }
+          }
+        continue;                                    // the last block of keys
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], vr[r * sv + 16 * b], acc[b], 0, 0, 0);
   }
   float den = 1.0f;                                  // of query i0 + l15
   if constexpr (In::kNorm) {

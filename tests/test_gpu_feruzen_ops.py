@@ -368,3 +368,28 @@ def test_matrix_memory_chunks_against_the_scan_in_64_bits(dtype, heads, dim, vdi
             assert abs(float(after[s, heads * dim * (vdim + 1) + h] - m)) < 2e-5 * max(1.0, abs(float(m)))
         at += n
     assert torch.equal(after[2], before[2])
+
+
+@pytest.mark.parametrize("what", ["value", "key", "query", "gate"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("dim,vdim", [(128, 64), (20, 33)])
+def test_matrix_memory_chunks_let_nothing_reach_earlier_tokens(dim, vdim, bad, what):
+    """as for the state-space scan: exactly what the token scan spoils is spoilt"""
+    from pegainfer_amd import ops_blocks as Bk
+    g = torch.Generator().manual_seed(dim)
+    heads, T, cap = 2, 150, 15.0
+    cols = heads * (2 * dim + vdim + 2)
+    offs = [0, heads * dim, 2 * heads * dim, heads * (2 * dim + vdim), heads * (2 * dim + vdim + 1)]
+    for at in (16, 45, 63, 64, 121):
+        proj = torch.randn(T, cols, generator=g)
+        proj[at, {"value": offs[2] + vdim // 2, "key": offs[1] + dim - 1, "query": offs[0] + 2, "gate": offs[4] + 1}[what]] = bad
+        ib, fb = torch.randn(heads, generator=g).cuda(), (torch.randn(heads, generator=g) + 2).cuda()
+        runs = []
+        for scan_max in (0, 32):
+            state = torch.zeros(1, heads * (dim * vdim + dim + 1)).cuda()
+            y = Bk.gated_matrix_memory(proj.cuda(), offs, ib, fb, cap, state, heads, dim, vdim, Bk.Ragged([T]), scan_max=scan_max)
+            runs += [y.cpu(), state.cpu()]
+        for a, b in ((runs[0], runs[2]), (runs[1], runs[3])):
+            ok = torch.isfinite(a)
+            assert torch.equal(ok, torch.isfinite(b)), (at, int((ok != torch.isfinite(b)).sum()))
+            assert float((a[ok] - b[ok]).abs().max()) < 1e-4 * max(1.0, float(a[ok].abs().max()))

@@ -469,6 +469,35 @@ def test_state_space_chunks_keep_their_padding_zero(N):
     assert torch.isfinite(y[:, [i for i in range(inner) if i != 7]]).all()
 
 
+@pytest.mark.parametrize("what", ["value", "key", "query", "step"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("N,P", [(128, 64), (20, 33), (5, 64)])
+def test_state_space_chunks_let_nothing_reach_earlier_tokens(N, P, bad, what):
+    """a value, key, query or step that is infinite or no number, at the start, inside and at the end of a block of 16 and of a chunk: exactly the
+    outputs and states that the scan spoils are spoilt, the others stay within the rounding of sums of about a hundred products"""
+    Bk = B()
+    g = torch.Generator().manual_seed(N)
+    heads, T = 2, 150
+    inner, ch = heads * P, heads * P + 2 * N
+    for at in (16, 45, 63, 64, 121):
+        xbc, proj = torch.randn(T, ch, generator=g), torch.randn(T, heads, generator=g)
+        xbc[:, inner:] *= N ** -0.25
+        if what == "step":
+            proj[at, 1] = bad
+        else:
+            xbc[at, {"value": P + P // 2, "key": inner + N - 1, "query": inner + N + 2}[what]] = bad
+        args = (proj.cuda(), 0, torch.tensor([-1.0, 0.5]).cuda(), torch.randn(heads, generator=g).cuda(), torch.randn(heads, generator=g).cuda())
+        runs = []
+        for scan_max in (0, 32):
+            state = torch.ones(1, heads * N * P).cuda()
+            y = Bk.ssd_scan(xbc.cuda(), *args, state, heads, 1, N, P, Bk.Ragged([T]), scan_max=scan_max)
+            runs += [y.cpu(), state.cpu()]
+        for a, b in ((runs[0], runs[2]), (runs[1], runs[3])):
+            ok = torch.isfinite(a)
+            assert torch.equal(ok, torch.isfinite(b)), (at, int((ok != torch.isfinite(b)).sum()))
+            assert float((a[ok] - b[ok]).abs().max()) < 1e-4 * max(1.0, float(a[ok].abs().max()))
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
