@@ -455,8 +455,9 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
 // stay in registers (a wave's own quarter of the entry), so LDS holds the key tile and the tile's scores alone.
 // The fp32 instance works on v_mfma_f32_16x16x4_f32: lane (l15, g) fetches four neighbouring values at 4 g of a 16-wide block with one
 // 16-byte read, and product e of the block takes value e of every lane - both operands numbered alike; its weights stay fp32.
-// A key that a row does not see has weight zero in the products, as in the form above: an entry that is infinite or no number reaches
-// the rows of its request that share its key tile.
+// A key that a row does not see has weight zero in the products.  In bf16, as in the form above, an entry that is infinite or no number so reaches
+// the rows of its request that share its key tile; in fp32 a tile with such an entry (all its scores are none) is summed key by key for the
+// rows that see it, and the rows before it keep what the plain form gives them.
 // Bound by the latency of one pass through scores, softmax and values (three barriers per tile of 32 keys), not by memory.
 // With the merge, 16 heads of 512 + 64 and 4 requests of 500 to 900 keys in splits of 32: 17.1 (the form above) -> 15.9 us, 32 requests
 // 53.6 -> 35.0 us.  In fp32, where a workgroup took one head and a thread one key: 8 heads of 256 + 64, two requests of up to 300 keys
@@ -486,6 +487,7 @@ __global__ __launch_bounds__(256) void latent_attn_few_kernel(const float* __res
   float* S = reinterpret_cast<float*>(Ck + kTileKeys * cs);                    // [4][kRows][kSStride] parts of the scores
   A* P = reinterpret_cast<A*>(S + 4 * kRows * kSStride);                       // [kRows][kSStride] weights
   float* s_row = reinterpret_cast<float*>(P + kRows * kSStride);               // [kRows] rescale of the tile, at the end 1 / sum
+  __shared__ int s_spoilt[4];                              // per wave of the softmax: a score of the tile is no finite number
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
   const int tile = blockIdx.x, sub = blockIdx.z, split = blockIdx.y;
   const int cnt = min(kRows, tile_rows[tile] - sub * kRows);
@@ -594,6 +596,12 @@ __global__ __launch_bounds__(256) void latent_attn_few_kernel(const float* __res
       f32x4 v = *reinterpret_cast<const f32x4*>(S + my_row * kSStride + my_key);
 #pragma unroll
       for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(S + (w * kRows + my_row) * kSStride + my_key);
+      if constexpr (F32) {
+        bool spoilt = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) spoilt |= !(fabsf(v[e]) <= __FLT_MAX__);
+        if (const bool any = __any(spoilt); lane == 0) s_spoilt[wave] = any;
+      }
       float mx = -INFINITY;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -629,21 +637,42 @@ __global__ __launch_bounds__(256) void latent_attn_few_kernel(const float* __res
       }
     }
     if constexpr (F32) {
+      bool spoilt = false;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        f32x4 p[RB];
+      for (int w = 0; w < 2 * RB; ++w) spoilt |= s_spoilt[w] != 0;
+      if (spoilt) {                                        // uniform: each row takes the keys that it sees, one by one
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) p[rb] = *reinterpret_cast<const f32x4*>(P + (rb * 16 + l15) * kSStride + 16 * kb + 4 * g);
+        for (int rb = 0; rb < RB; ++rb) {
+          const int row = rb * 16 + l15, seen = row < cnt ? min(positions[(row0 + row) / H] + 1, j_hi) - j0 : 0;
+          for (int k = 0; k < min(seen, kTileKeys); ++k) {
+            const float w = P[row * kSStride + k];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+            for (int d = 0; d < ND; ++d) {
+              const int dd = (wave + 4 * d) * 16;
+              if (dd >= r) break;
+              const f32x4 c = *reinterpret_cast<const f32x4*>(Ck + k * cs + dd + 4 * g);
 #pragma unroll
-          for (int d = 0; d < ND; ++d) {
-            const int dd = (wave + 4 * d) * 16;
-            if (dd >= r) break;
-            const float c = Ck[(16 * kb + 4 * g + e) * cs + dd + l15];
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) o[rb][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(c, p[rb][e], o[rb][d], 0, 0, 0);
+              for (int e = 0; e < 4; ++e) o[rb][d][e] = fmaf(w, c[e], o[rb][d][e]);
+            }
           }
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          f32x4 p[RB];
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) p[rb] = *reinterpret_cast<const f32x4*>(P + (rb * 16 + l15) * kSStride + 16 * kb + 4 * g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+              const int dd = (wave + 4 * d) * 16;
+              if (dd >= r) break;
+              const float c = Ck[(16 * kb + 4 * g + e) * cs + dd + l15];
+#pragma unroll
+              for (int rb = 0; rb < RB; ++rb) o[rb][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(c, p[rb][e], o[rb][d], 0, 0, 0);
+            }
+        }
       }
     } else {
       bf16x8_t p[RB];

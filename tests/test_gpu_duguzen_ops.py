@@ -327,6 +327,34 @@ def test_latent_attention_few_rows_form(shape, dtype, split_keys):
         assert (o[i].cpu().double() - ref).abs().max() < tol, (i, pos[i], float((o[i].cpu().double() - ref).abs().max()))
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("H,r,dr", [(8, 256, 64), (3, 16, 8), (40, 512, 64)])
+def test_fp32_latent_attention_keeps_later_entries_from_earlier_rows(H, r, dr, bad):
+    """an entry that is infinite or no number, in the latent or in the rotated part, at the start, in the middle and at the end of a key tile: the rows
+    before it are what they are without it, the rows from it on are no numbers"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(r)
+    E, ps, T = r + dr, 16, 75
+    ent, qc = torch.randn(T, E, generator=g) * 0.5, torch.randn(T, H, E, generator=g) / E ** 0.5
+    npages = (T + ps - 1) // ps
+    pos, req = torch.arange(T, dtype=torch.int32).cuda(), torch.zeros(T, dtype=torch.int32).cuda()
+    indptr, ids = torch.tensor([0, npages], dtype=torch.int32).cuda(), torch.arange(npages, dtype=torch.int32).cuda()
+
+    def run(e, **kw):
+        pool = torch.zeros(npages * ps, E)
+        pool[:T] = e
+        return B.latent_attention(qc.cuda(), pool.cuda(), ps * E, 0, ps, pos, req, indptr, ids, r, dr, 1.0, T, tiles=B.row_tiles([T], H), **kw).cpu()
+
+    for at, col in ((31, 3), (32, r - 1), (50, 0), (74, r + dr - 1)):
+        e = ent.clone()
+        e[at, col] = bad
+        for kw in ({}, {"split_keys": 32}):
+            sound, got = run(ent, **kw), run(e, **kw)
+            assert float((got[:at] - sound[:at]).abs().max()) < 1e-5, (at, col)     # sums of 32 products in another order
+            if col < r:
+                assert not torch.isfinite(got[at:, :, col]).any()
+
+
 def ffi_ok(B, r, dr, page_stride):
     from pegainfer_amd import ffi
     return ffi.lib().pegainfer_latent_attention_tiled_ok(r, dr, page_stride, 0, 0) == 1
