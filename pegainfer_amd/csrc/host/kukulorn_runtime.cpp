@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -159,7 +160,8 @@ struct Model {
   std::vector<KvState> requests;
   pq::StateLayout state_layout;
   float* state = nullptr;
-  struct TileSet { int per, wide_kv; };   // query heads per kv head; fewest kv heads of its layers (0: some layer takes no wide tiles)
+  // query heads per kv head; fewest kv heads of its layers (0: some layer takes no wide tiles); the most keys that a row of them walks
+  struct TileSet { int per, wide_kv, span; };
   std::vector<TileSet> tile_sets;         // one per distinct query-heads-per-kv-head value of the attention layers
   // step buffers
   size_t cap_rows = 0, cap_want = 0, cap_meta = 0;
@@ -248,8 +250,9 @@ struct Model {
     const int wide = dtype == PEGAINFER_DTYPE_BF16 && pegainfer_paged_attention_rows_ok(a->dim, a->vdim, 0, 0, 0, kPageSize) ? a->kv : 0;
     size_t k = 0;
     while (k < tile_sets.size() && tile_sets[k].per != per) ++k;
-    if (k == tile_sets.size()) tile_sets.push_back({per, wide});
-    else tile_sets[k].wide_kv = std::min(tile_sets[k].wide_kv, wide);
+    if (k == tile_sets.size()) tile_sets.push_back({per, wide, 0});
+    tile_sets[k].wide_kv = std::min(tile_sets[k].wide_kv, wide);
+    tile_sets[k].span = std::max(tile_sets[k].span, a->window > 0 ? (int)std::min<int64_t>((int64_t)a->window + a->keep_first, INT_MAX) : INT_MAX);
     return (int)k;
   }
   int parse_config(const std::string& text) {
@@ -812,7 +815,11 @@ struct Model {
     //   tokens | positions | row_entry | entry_row0 | entry_slot | page_indptr | want | attention tile sets | page_ids
     // One set of attention tiles (row_tiles.h) per distinct heads-per-kv-head value of the model's attention layers.
     bool single = true;   // every entry brings one token: decoding
-    for (int i = 0; i < n && single; ++i) single = lens[i] == 1;
+    int most_keys = 0;
+    for (int i = 0; i < n; ++i) {
+      single = single && lens[i] == 1;
+      most_keys = std::max(most_keys, requests[ids[i]].seq_len + lens[i]);
+    }
     const size_t o_tok = 0, o_pos = o_tok + T, o_ent = o_pos + T, o_row0 = o_ent + T, o_slot = o_row0 + (size_t)n + 1,
                  o_ind = o_slot + (size_t)n, o_want = o_ind + (size_t)n + 1;
     size_t words = o_want + (size_t)std::max(1, W);   // the page lists come last: everything before them sits at offsets that
@@ -821,7 +828,7 @@ struct Model {
     std::vector<int> tile_rows(tile_sets.size());
     for (size_t k = 0; k < tile_sets.size(); ++k) {
       const TileSet& ts = tile_sets[k];
-      tile_rows[k] = plain_kernels ? ptiles::kGroupRows : ptiles::wide_rows(lens, n, (int)T, ts.per, ts.wide_kv);
+      tile_rows[k] = plain_kernels ? ptiles::kGroupRows : ptiles::wide_rows(lens, n, (int)T, ts.per, ts.wide_kv, std::min(single ? INT_MAX : most_keys, ts.span));
       tile_off[k] = words;
       tile_cnt[k] = ptiles::count(lens, n, ts.per, tile_rows[k]);
       words += 4 * tile_cnt[k];
@@ -915,7 +922,7 @@ struct Model {
       o.softcap = a.softcap; o.window = a.window; o.keep_first = a.keep_first; o.dist_bias = w.dist_bias; o.n_dist = w.n_dist;
       o.gate = gate; o.gate_stride = proj_stride; o.gate_kind = gate_kind;
       o.tile_rows = tile_rows[ts];
-      o.n_split = wgs >= 128 || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
+      o.n_split = wgs >= ptiles::kUnsplitGroups || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
       o.workspace = att_part;
       o.plain = plain_kernels ? 1 : 0;
       KK_K(pegainfer_paged_attention_opt(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,

@@ -11,10 +11,14 @@
 namespace ptiles {
 
 constexpr int kGroupRows = 16;      // (token, query head) rows of one workgroup of the general attention kernels
-// A step whose 64- (32-) row tiles give so many workgroups takes those; below, 16-row tiles whose keys are dealt to several workgroups have more
-// of them.  16 heads over 4 key/value heads of 128, 16 / 32 / 64 rows: 1024 tokens 82 / 38 / 28 us, 128 tokens (32 workgroups of 64 rows)
-// 14.5 / 10.4 / 10.2 us, behind 2048 cached tokens 128 / 55 / 45 us.
-constexpr int kWideGroups = 32;
+// Wide tiles (64 or 32 rows) walk their keys in one workgroup; launches of fewer than kUnsplitGroups workgroups of 16-row tiles deal theirs
+// to several, up to 512 in all.  Where the 16-row form is not split either, wide tiles win at any length: 16 heads over 4 key/value heads of
+// 128, 128 tokens (128 workgroups of 16 rows, 32 of 64) alone 13.9 / 9.9 us, behind 4096 cached tokens 239 / 81, behind 16 384 904 / 293;
+// 32 decoding requests of 64 heads over 4 behind 2048 tokens 126 / 44.  Where it is, they win up to about 670 keys (64 tokens) to 800 (96
+// tokens): 64 tokens alone 18.8 / 8.4 us, behind 1024 cached tokens 25 / 30, behind 4096 53 / 96, behind 16 384 141 / 360; 8 decoding
+// requests of 64 heads over 4 behind 8192 tokens 57 / 143.  There a step takes them while no row walks more than kWideKeys keys and they give
+// kWideGroups workgroups.
+constexpr int kUnsplitGroups = 128, kWideGroups = 32, kWideKeys = 640;
 
 inline size_t count(const int32_t* lens, int n, int per, int rows) {
   const int tpt = std::max(1, rows / per), cuts = (per + rows - 1) / rows;
@@ -22,9 +26,10 @@ inline size_t count(const int32_t* lens, int n, int per, int rows) {
   for (int i = 0; i < n; ++i) c += (size_t)((lens[i] + tpt - 1) / tpt) * cuts;
   return c;
 }
-// rows of a tile for a step of prompts: the widest tiles that still fill the chip (kv: key/value heads of the launch; <= 0: the launch
-// takes no wide tiles) and are at least half full
-inline int wide_rows(const int32_t* lens, int n, int T, int per, int kv) {
+// Rows of a tile, at least half full when wide.  kv: key/value heads of the launch (<= 0: it takes no wide tiles); keys: the most a row
+// walks (INT_MAX where the choice must follow from the step's shape alone, as in a step that is captured).
+inline int wide_rows(const int32_t* lens, int n, int T, int per, int kv, int keys) {
+  if (keys > kWideKeys && (long)count(lens, n, per, kGroupRows) * kv < kUnsplitGroups) return kGroupRows;
   for (int rows : {64, 32}) {
     const long tiles = (long)count(lens, n, per, rows);
     if (tiles * kv >= kWideGroups && (long)T * per * 2 >= tiles * rows) return rows;

@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -298,11 +299,13 @@ class StepModel {
     StepCtx c;
     c.T = (int)T; c.n = n; c.W = W;
     c.single = true;
+    int most_keys = 0;
     {
       size_t t = 0, pg = 0;
       for (int i = 0; i < n; ++i) {
         const KvState& st = requests[ids[i]];
         c.single = c.single && lens[i] == 1;
+        most_keys = std::max(most_keys, st.seq_len + lens[i]);
         mb[o_row0 + i] = (int32_t)t;
         mb[o_slot + i] = ids[i];
         mb[o_ind + i] = (int32_t)pg;
@@ -321,7 +324,8 @@ class StepModel {
     std::vector<std::pair<size_t, int>> group_at, flat_at;    // (offset, tiles)
     std::vector<int> group_rows;
     for (auto& gt : group_sets) {
-      const int rows = plain_kernels ? kGroupRows : ptiles::wide_rows(lens, n, (int)T, gt.per, gt.wide_kv);
+      const int keys = std::min(c.single ? INT_MAX : most_keys, gt.span);
+      const int rows = plain_kernels ? kGroupRows : ptiles::wide_rows(lens, n, (int)T, gt.per, gt.wide_kv, keys);
       group_rows.push_back(rows);
       group_at.push_back(put_group_tiles(&mb, lens, n, gt.per, rows));
     }
@@ -429,8 +433,11 @@ class StepModel {
   std::vector<void*> step_owned, want_owned, owned;
   float* logits32 = nullptr;         // [wanted, V]: run_step leaves them here
   // distinct parameters of the tile tables a model's launches read.  wide_kv: key/value heads of a layer whose prompts may take wider
-  // group tiles (0: never)
-  struct GroupSet { int per, wide_kv; bool operator==(const GroupSet& o) const { return per == o.per && wide_kv == o.wide_kv; } };
+  // group tiles (0: never); span: the most keys that a row of the layer walks
+  struct GroupSet {
+    int per, wide_kv, span;
+    bool operator==(const GroupSet& o) const { return per == o.per && wide_kv == o.wide_kv && span == o.span; }
+  };
   std::vector<GroupSet> group_sets;
   std::vector<int> flat_heads;
   int scan_max = 0;                  // > 0: entries with more rows go into the chunk table
@@ -461,7 +468,9 @@ class StepModel {
     v->push_back(x);
     return (int)v->size() - 1;
   }
-  int group_tiles(int heads_per_kv, int wide_kv = 0) { return index_of(&group_sets, GroupSet{heads_per_kv, wide_kv}); }
+  int group_tiles(int heads_per_kv, int wide_kv = 0, int span = INT_MAX) {
+    return index_of(&group_sets, GroupSet{heads_per_kv, wide_kv, span});
+  }
   int flat_tiles(int heads) { return index_of(&flat_heads, heads); }
 
   template <typename T>

@@ -1,6 +1,7 @@
 """CPU-only tests of the pure-host pieces of libpegainfer_qwen3.so against the oracle / the
 reference's own unit tests (pegainfer-core/src/page_pool.rs:124-199, kv_pool.rs:290-310,
 batch_decode_buffers.rs)."""
+import ctypes
 import os
 
 import numpy as np
@@ -170,3 +171,29 @@ def test_native_safetensors_reader_matches_python(tmp_path):
     for nme in (names[0], names[-1]):
         rc, shp, dt, bs, nt = probe(str(d), nme)
         assert (rc, shp, dt, nt) == (0, ref[nme][1], ref[nme][0], len(ref)) and bs == checksum(ref[nme][2])
+
+
+@pytest.fixture(scope="module")
+def tables(tmp_path_factory):
+    """csrc/host/row_tiles.h behind C entries"""
+    import subprocess
+    d = tmp_path_factory.mktemp("tables")
+    (d / "t.cpp").write_text('#include "row_tiles.h"\nextern "C" int wide_rows(const int32_t* lens, int n, int T, int per, int kv, int keys) '
+                             '{ return ptiles::wide_rows(lens, n, T, per, kv, keys); }\n')
+    host = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc", "host")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-I", host, "-o", str(d / "t.so"), str(d / "t.cpp")], check=True)
+    return ctypes.CDLL(str(d / "t.so"))
+
+
+@pytest.mark.parametrize("lens,heads,kv,keys,rows", [
+    ([1024], 16, 4, 1024, 64), ([128], 16, 4, 128, 64), ([128], 16, 4, 16512, 64),      # 128 workgroups of 16 rows and more: their keys were not dealt
+    ([64], 16, 4, 64, 32), ([64], 16, 4, 640, 32), ([64], 16, 4, 641, 16), ([64], 16, 4, 4160, 16), ([127], 16, 4, 640, 64), ([124], 16, 4, 641, 16),
+    ([32], 16, 4, 32, 16),                                                               # too few workgroups of wide tiles
+    ([64, 1, 1, 1], 16, 4, 4097, 16),                                                    # one long context among short ones
+    ([1] * 8, 64, 4, None, 16), ([1] * 31, 64, 4, None, 16), ([1] * 32, 64, 4, None, 32), ([1] * 64, 128, 4, None, 64), ([1] * 64, 16, 4, None, 16),
+    ([1024], 16, 0, 1024, 16)])
+def test_wide_attention_tiles_leave_no_key_split_behind(tables, lens, heads, kv, keys, rows):
+    """short of 128 workgroups the 16-row tiles deal a long context's keys to up to 512, so wide tiles are for short ones; decoding steps
+    (keys None: the choice may not depend on the contexts) take them only where nothing was dealt"""
+    a = np.array(lens, np.int32)
+    assert tables.wide_rows(ctypes.c_void_p(a.ctypes.data), len(lens), int(a.sum()), heads // max(kv, 1), kv, 2 ** 31 - 1 if keys is None else keys) == rows
