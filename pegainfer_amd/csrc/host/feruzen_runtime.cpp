@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "optional_scratch.h"
 #include "row_tiles.h"
 #include "seq_state.h"
 #include "safetensors_loader.h"
@@ -157,8 +158,7 @@ struct Model {
   uint8_t* top1_state = nullptr;
   uint8_t *meta_host = nullptr, *meta_dev = nullptr;
   uint8_t* sample_scratch = nullptr;
-  float* chunk_ws = nullptr;   // states between the chunks of long entries
-  size_t chunk_cap = 0;
+  pq::OptionalScratch chunk_ws;   // states between the chunks of long entries
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -680,19 +680,22 @@ struct Model {
       if (l.mm.heads > 0) return true;
     return false;
   }
-  int ensure_chunks(int n) {
+  // room for the states between the chunks of a step; false: there is none
+  bool ensure_chunks(int n) {
     size_t need = 0;
     if (n > 0)
       for (auto& l : layers)
         if (l.mm.heads > 0) need = std::max(need, (size_t)pegainfer_gated_matrix_memory_workspace(n, l.mm.heads, l.mm.dim, l.mm.vdim));
-    if (need <= chunk_cap) return 0;
-    FZ_HIP(hipStreamSynchronize(stream));
-    if (chunk_ws) (void)hipFree(chunk_ws);
-    chunk_ws = nullptr;
-    chunk_cap = 0;
-    FZ_HIP(hipMalloc(reinterpret_cast<void**>(&chunk_ws), need * 4));
-    chunk_cap = need;
-    return 0;
+    return chunk_ws.grow(need, [](size_t bytes) {
+      void* p = nullptr;
+      if (hipMalloc(&p, bytes) == hipSuccess) return p;
+      (void)hipGetLastError();
+      return (void*)nullptr;
+    }, [&](float* p) { free_scratch(p); });
+  }
+  void free_scratch(float* p) {
+    if (stream) (void)hipStreamSynchronize(stream);
+    (void)hipFree(p);
   }
   int ensure_want(size_t n) {
     if (n <= cap_want) return 0;
@@ -815,11 +818,11 @@ struct Model {
       words += 4 * cnt;
     }
     // long entries of the matrix memory in chunks (never part of a captured step)
-    const ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
+    ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
+    if (!ensure_chunks((int)chunks.row0.size())) chunks = ptiles::Chunks();   // no memory: the scan, which needs none, takes every entry
     const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
     size_t chunk_off[4];
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
-    if (ensure_chunks((int)chunks.row0.size())) return -1;
     const size_t o_pages = words;
     words += total_pages;
     if (words > cap_meta) {
@@ -1003,7 +1006,7 @@ struct Model {
         mm.entry_row0 = d_row0; mm.entry_slot = d_slot; mm.n_entries = n; mm.scan_max = kScanMax;
         mm.chunk_row0 = md + chunk_off[0]; mm.chunk_rows = md + chunk_off[1]; mm.n_chunks = (int)chunks.row0.size();
         mm.long_chunk0 = md + chunk_off[2]; mm.long_slot = md + chunk_off[3]; mm.n_long = (int)chunks.slot.size();
-        mm.workspace = chunk_ws; mm.dtype = dtype;
+        mm.workspace = chunk_ws.p; mm.dtype = dtype;
         FZ_K(pegainfer_gated_matrix_memory_form(&mm, S()));
         FZ_K(pegainfer_head_rms_gate(o32, w.rnorm, 1, at(proj, (size_t)c.o_rg), Mp, 1, c.right_scale, eps,
                                      at(mix, (size_t)a.heads * a.vdim), c.mix_cols, r.heads, r.vdim, Ti, dtype, S()));
@@ -1167,7 +1170,7 @@ struct Model {
     free_all(&owned);
     free_all(&step_owned);
     free_all(&want_owned);
-    if (chunk_ws) (void)hipFree(chunk_ws);
+    chunk_ws.drop([&](float* p) { free_scratch(p); });
     if (tap) (void)hipFree(tap);
     if (meta_dev) (void)hipFree(meta_dev);
     if (meta_host) (void)hipHostFree(meta_host);

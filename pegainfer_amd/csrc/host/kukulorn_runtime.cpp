@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "kv_pool.h"
+#include "optional_scratch.h"
 #include "row_tiles.h"
 #include "seq_state.h"
 #include "safetensors_loader.h"
@@ -183,8 +184,7 @@ struct Model {
   float* tap = nullptr;
   size_t tap_cap = 0;
   int tap_rows = 0;
-  float* chunk_ws = nullptr;   // states between the chunks of long entries
-  size_t chunk_cap = 0;
+  pq::OptionalScratch chunk_ws;   // states between the chunks of long entries
   float* att_part = nullptr;   // softmax states of the key splits of an attention launch
   int mx_proj = 0, mx_mix = 0, mx_inner = 0, mx_conv = 0, mx_q = 0, mx_ff = 0, mx_vdim = 0;
 
@@ -718,19 +718,22 @@ struct Model {
     cap_rows = n;
     return 0;
   }
-  int ensure_chunks(int n) {
+  // room for the states between the chunks of a step; false: there is none
+  bool ensure_chunks(int n) {
     size_t need = 0;
     if (n > 0)
       for (auto& l : layers)
         if (l.sm.heads > 0) need = std::max(need, (size_t)pegainfer_ssd_scan_workspace(n, l.sm.heads, l.sm.state, l.sm.vdim));
-    if (need <= chunk_cap) return 0;
-    KK_HIP(hipStreamSynchronize(stream));
-    if (chunk_ws) (void)hipFree(chunk_ws);
-    chunk_ws = nullptr;
-    chunk_cap = 0;
-    KK_HIP(hipMalloc(reinterpret_cast<void**>(&chunk_ws), need * 4));
-    chunk_cap = need;
-    return 0;
+    return chunk_ws.grow(need, [](size_t bytes) {
+      void* p = nullptr;
+      if (hipMalloc(&p, bytes) == hipSuccess) return p;
+      (void)hipGetLastError();
+      return (void*)nullptr;
+    }, [&](float* p) { free_scratch(p); });
+  }
+  void free_scratch(float* p) {
+    if (stream) (void)hipStreamSynchronize(stream);
+    (void)hipFree(p);
   }
   int ensure_want(size_t n) {
     if (n <= cap_want) return 0;
@@ -834,11 +837,11 @@ struct Model {
       words += 4 * tile_cnt[k];
     }
     // long entries of the state-space scan in chunks (never part of a captured step)
-    const ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, mx_inner > 0 && !plain_kernels ? kScanMax : INT32_MAX);
+    ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, mx_inner > 0 && !plain_kernels ? kScanMax : INT32_MAX);
+    if (!ensure_chunks((int)chunks.row0.size())) chunks = ptiles::Chunks();   // no memory: the scan, which needs none, takes every entry
     const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
     size_t chunk_off[4];
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
-    if (ensure_chunks((int)chunks.row0.size())) return -1;
     const size_t o_pages = words;
     words += total_pages;
     if (words > cap_meta) {
@@ -986,7 +989,7 @@ struct Model {
         sd.entry_row0 = d_row0; sd.entry_slot = d_slot; sd.n_entries = n; sd.scan_max = kScanMax;
         sd.chunk_row0 = md + chunk_off[0]; sd.chunk_rows = md + chunk_off[1]; sd.n_chunks = (int)chunks.row0.size();
         sd.long_chunk0 = md + chunk_off[2]; sd.long_slot = md + chunk_off[3]; sd.n_long = (int)chunks.slot.size();
-        sd.workspace = chunk_ws; sd.dtype = dtype;
+        sd.workspace = chunk_ws.p; sd.dtype = dtype;
         KK_K(pegainfer_ssd_scan_form(&sd, S()));
         KK_K(pegainfer_head_gate_rms(o32, w.snorm, 1, at(proj, (size_t)c.o_in), c.proj_rows, 0, 1, 1.0f, eps, mixr, inner, s.norm_groups,
                                      inner / s.norm_groups, Ti, dtype, S()));
@@ -1089,7 +1092,7 @@ struct Model {
     free_all(&step_owned);
     free_all(&want_owned);
     if (tap) (void)hipFree(tap);
-    if (chunk_ws) (void)hipFree(chunk_ws);
+    chunk_ws.drop([&](float* p) { free_scratch(p); });
     if (meta_dev) (void)hipFree(meta_dev);
     if (meta_host) (void)hipHostFree(meta_host);
     if (ev0) (void)hipEventDestroy(ev0);

@@ -2,7 +2,7 @@
 // long portions of ragged batches in chunks of <= 64 tokens that run side by side.
 //   scalar_chunk_sum_kernel    U_c = sum_i w_i b_i k_i v_i^T with w_i the product of the decays behind token i, and the product of all
 //                              the chunk's decays
-//   scalar_chunk_state_kernel  walks the chunks of an entry, S <- total_c S + U_c, and leaves the state BEFORE each in U_c's place
+//   scalar_chunk_state_kernel  walks the chunks of an entry that the run holds, S <- total_c S + U_c, and leaves the state BEFORE each in U_c's place
 //   scalar_chunk_out_kernel    y_i = (a_1 .. a_i) S^T q_i + sum_{j <= i} (a_(j+1) .. a_i) b_j (q_i . k_j) v_j
 // Decays enter as products of the decays themselves, never as quotients or differences of logarithms: every factor is at most one, nothing
 // cancels however fast a head forgets, and the roundings of a product are those of a scan's state.
@@ -21,7 +21,7 @@
 namespace pk {
 
 // [chunk][head][dim][columns] contributions, then states before the chunks; with a norm [chunk][head][dim] of the keys alone; totals
-struct ScalarWs { float *state, *norm, *total; };
+struct ScalarWs { float *state, *norm, *total; int first; };      // of the chunks from `first` on
 constexpr int kScalarCols = 64;     // value columns of a workgroup
 __host__ __device__ constexpr int scalar_cols(int vdim) { return (vdim + kScalarCols - 1) / kScalarCols * kScalarCols; }
 
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void scalar_chunk_sum_kernel(In in, ScalarWs w
                                                             const int32_t* __restrict__ chunk_row0, const int32_t* __restrict__ chunk_rows) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   __shared__ float s_w[kDecayChunk];
-  const int c = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * kScalarCols, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int slot = blockIdx.x, c = ws.first + slot, h = blockIdx.y, col0 = blockIdx.z * kScalarCols, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l15 = lane & 15, lg = lane >> 4, row0 = chunk_row0[c], n = chunk_rows[c];
   const int dp = pad16(in.dim), vp = scalar_cols(in.vdim), sk = stride_rows4(in.dim), sv = stride_rows4(kScalarCols);
   float *s_k = sm, *s_v = sm + kDecayChunk * sk;
@@ -51,19 +51,19 @@ __global__ __launch_bounds__(256) void scalar_chunk_sum_kernel(In in, ScalarWs w
     in.steps(c, h, row0, n, lane, &dt, &a);
     const float w = product_behind(a, lane);
     s_w[lane] = w * dt;
-    if (lane == 0 && blockIdx.z == 0) ws.total[(int64_t)c * in.H + h] = w * a;
+    if (lane == 0 && blockIdx.z == 0) ws.total[(int64_t)slot * in.H + h] = w * a;
   }
   __syncthreads();
   auto same = [](float x) { return x; };
   stage_rows<4>(in.rows(), in.row_stride(), in.k_at(h), row0, n, in.dim, dp, s_k, sk, s_w, tid, same);
   stage_rows<4>(in.rows(), in.row_stride(), in.v_at(h) + col0, row0, n, min(kScalarCols, in.vdim - col0), kScalarCols, s_v, sv, nullptr, tid, same);
   __syncthreads();
-  float* U = ws.state + ((int64_t)c * in.H + h) * dp * vp + col0;
+  float* U = ws.state + ((int64_t)slot * in.H + h) * dp * vp + col0;
   if (In::kNorm && blockIdx.z == 0)                  // the keys alone: the state of a value that is one
     for (int d = tid; d < dp; d += 256) {
       float t = 0.f;
       for (int i = 0; i < n; ++i) t += s_k[i * sk + d];
-      ws.norm[((int64_t)c * in.H + h) * dp + d] = t;
+      ws.norm[((int64_t)slot * in.H + h) * dp + d] = t;
     }
   const int steps = (n + 3) >> 2;
   for (int d0 = wave * 16; d0 < dp; d0 += 64) {
@@ -91,17 +91,19 @@ __global__ __launch_bounds__(256) void scalar_chunk_sum_kernel(In in, ScalarWs w
 // NORM: dim more per head, the keys' own state behind the heads' matrices.
 template <bool NORM>
 __global__ __launch_bounds__(256) void scalar_chunk_state_kernel(ScalarWs ws, float* __restrict__ state, int64_t slot_stride, int H, int dim, int vdim,
-                                                              const int32_t* __restrict__ long_chunk0, const int32_t* __restrict__ long_slot) {
+                                                              const int32_t* __restrict__ long_chunk0, const int32_t* __restrict__ long_slot,
+                                                              int n) {
   const int e = blockIdx.z, h = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
   const int j = i - dim * vdim;                            // >= 0: an element of the keys' state
   if (j >= (NORM ? dim : 0)) return;
+  const int c_begin = max(long_chunk0[e] - ws.first, 0), c_end = min(long_chunk0[e + 1] - ws.first, n);     // places of the entry's chunks in this run
+  if (c_begin >= c_end) return;
   const int dp = pad16(dim), vp = scalar_cols(vdim);
   float* sp = state + (int64_t)long_slot[e] * slot_stride + (j < 0 ? (int64_t)h * dim * vdim + i : (int64_t)H * dim * vdim + (int64_t)h * dim + j);
   const int64_t cs = (int64_t)H * dp * (j < 0 ? vp : 1);
   float* u = j < 0 ? ws.state + (int64_t)h * dp * vp + (int64_t)(i / vdim) * vp + i % vdim : ws.norm + (int64_t)h * dp + j;
-  const int c_end = long_chunk0[e + 1];
   float S = *sp;
-  for (int c0 = long_chunk0[e]; c0 < c_end; c0 += 8) {      // eight chunks' loads in flight before the first store
+  for (int c0 = c_begin; c0 < c_end; c0 += 8) {      // eight chunks' loads in flight before the first store
     float t[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) t[k] = c0 + k < c_end ? u[(c0 + k) * cs] : 0.f;
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(256) void scalar_chunk_out_kernel(In in, ScalarWs w
   extern __shared__ __attribute__((aligned(16))) float sm[];
   constexpr int sp = kDecayChunk + 4, sv = kScalarCols + 4;
   __shared__ __attribute__((aligned(16))) float s_p[kDecayChunk][sp];   // [query][key] decay between them, times the key's step size
-  const int c = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * kScalarCols, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int slot = blockIdx.x, c = ws.first + slot, h = blockIdx.y, col0 = blockIdx.z * kScalarCols, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l15 = lane & 15, lg = lane >> 4, row0 = chunk_row0[c], n = chunk_rows[c], i0 = wave * 16;
   const int dim = in.dim, dp = pad16(dim), vp = scalar_cols(in.vdim), sk = stride_rows16(dim), vd = min(kScalarCols, in.vdim - col0);
   float *s_k = sm, *s_v = s_k + kDecayChunk * sk;
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(256) void scalar_chunk_out_kernel(In in, ScalarWs w
 #pragma unroll
   for (int b = 0; b < 4; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   {   // what the tokens before the chunk left; rows dim .. dp - 1 and columns past vdim of the state before a chunk are zeros
-    const float* S = ws.state + ((int64_t)c * in.H + h) * dp * vp + col0 + (int64_t)(4 * lg) * vp + l15;
+    const float* S = ws.state + ((int64_t)slot * in.H + h) * dp * vp + col0 + (int64_t)(4 * lg) * vp + l15;
     float cur[4][4], nxt[4][4];
     auto fetch = [&](int k0, float (*t)[4]) {
 #pragma unroll
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(256) void scalar_chunk_out_kernel(In in, ScalarWs w
   }
   float nq = 0.f;                                    // this lane's part of n . q
   if constexpr (In::kNorm) {
-    const float* N = ws.norm + ((int64_t)c * in.H + h) * dp + 4 * lg;
+    const float* N = ws.norm + ((int64_t)slot * in.H + h) * dp + 4 * lg;
 #pragma unroll
     for (int kb = 0; kb < QB; ++kb) {
       if (16 * kb >= dp) break;
@@ -285,32 +287,42 @@ __global__ __launch_bounds__(256) void scalar_chunk_out_kernel(In in, ScalarWs w
   }
 }
 
-// What the three launches of n_chunks chunks need, and they themselves.
+// What the three launches of n_chunks chunks need, and they themselves.  A long step's chunks are walked in runs, one behind the other, whose
+// states take 256 MB at most (or one chunk's): 256 chunks, 16 384 tokens, at 32 heads of 128 states x 64 values.
+constexpr int64_t kScalarRunFloats = (int64_t)1 << 26;
+inline int64_t scalar_chunk_each(int heads, int dim, int vdim, bool norm) {
+  return (int64_t)heads * ((int64_t)pad16(dim) * (scalar_cols(vdim) + (norm ? 1 : 0)) + 1);
+}
+inline int scalar_chunk_run(int n_chunks, int heads, int dim, int vdim, bool norm) {
+  const int64_t fit = kScalarRunFloats / scalar_chunk_each(heads, dim, vdim, norm);
+  return (int)(fit >= n_chunks ? n_chunks : fit > 0 ? fit : 1);
+}
 inline int64_t scalar_chunk_floats(int n_chunks, int heads, int dim, int vdim, bool norm) {
-  return (int64_t)n_chunks * heads * ((int64_t)pad16(dim) * (scalar_cols(vdim) + (norm ? 1 : 0)) + 1);
+  return n_chunks <= 0 ? 0 : scalar_chunk_run(n_chunks, heads, dim, vdim, norm) * scalar_chunk_each(heads, dim, vdim, norm);
 }
 template <typename In>
 inline void scalar_chunk_launch(const In& in, float* workspace, float* state, int64_t slot_stride, float* o, const int32_t* chunk_row0,
                                 const int32_t* chunk_rows, int n_chunks, const int32_t* long_chunk0, const int32_t* long_slot, int n_long,
                                 hipStream_t st) {
-  const int H = in.H, dim = in.dim, vdim = in.vdim, dp = pad16(dim);
-  const int64_t slots = (int64_t)n_chunks * H;
+  const int H = in.H, dim = in.dim, vdim = in.vdim, dp = pad16(dim), run = scalar_chunk_run(n_chunks, H, dim, vdim, In::kNorm);
+  const int64_t slots = (int64_t)run * H;
   ScalarWs ws;
   ws.state = workspace;
   ws.norm = workspace + slots * dp * scalar_cols(vdim);
   ws.total = ws.norm + (In::kNorm ? slots * dp : 0);
-  const dim3 grid(n_chunks, H, ceil_div(vdim, kScalarCols));
   auto sums = &scalar_chunk_sum_kernel<In>;
-  sums<<<grid, 256, with_lds(sums, (size_t)kDecayChunk * (stride_rows4(dim) + stride_rows4(kScalarCols)) * sizeof(float)), st>>>(in, ws, chunk_row0,
-                                                                                                                             chunk_rows);
-  scalar_chunk_state_kernel<In::kNorm><<<dim3(ceil_div((long)dim * (vdim + (In::kNorm ? 1 : 0)), 256), H, n_long), 256, 0, st>>>(
-      ws, state, slot_stride, H, dim, vdim, long_chunk0, long_slot);
-  auto out = [&](auto kern) {
-    kern<<<grid, 256, with_lds(kern, (size_t)kDecayChunk * (stride_rows16(dim) + kScalarCols + 4) * sizeof(float)), st>>>(in, ws, o, chunk_row0,
-                                                                                                                    chunk_rows);
-  };
-  if (dim <= 128) out(&scalar_chunk_out_kernel<In, 8>);
-  else out(&scalar_chunk_out_kernel<In, 16>);
+  const size_t sum_lds = with_lds(sums, (size_t)kDecayChunk * (stride_rows4(dim) + stride_rows4(kScalarCols)) * sizeof(float));
+  auto out = dim <= 128 ? &scalar_chunk_out_kernel<In, 8> : &scalar_chunk_out_kernel<In, 16>;
+  const size_t out_lds = with_lds(out, (size_t)kDecayChunk * (stride_rows16(dim) + kScalarCols + 4) * sizeof(float));
+  for (int c0 = 0; c0 < n_chunks; c0 += run) {
+    const int n = n_chunks - c0 < run ? n_chunks - c0 : run;
+    const dim3 grid(n, H, ceil_div(vdim, kScalarCols));
+    ws.first = c0;
+    sums<<<grid, 256, sum_lds, st>>>(in, ws, chunk_row0, chunk_rows);
+    scalar_chunk_state_kernel<In::kNorm><<<dim3(ceil_div((long)dim * (vdim + (In::kNorm ? 1 : 0)), 256), H, n_long), 256, 0, st>>>(
+        ws, state, slot_stride, H, dim, vdim, long_chunk0, long_slot, n);
+    out<<<grid, 256, out_lds, st>>>(in, ws, o, chunk_row0, chunk_rows);
+  }
 }
 
 }  // namespace pk

@@ -393,3 +393,23 @@ def test_matrix_memory_chunks_let_nothing_reach_earlier_tokens(dim, vdim, bad, w
             ok = torch.isfinite(a)
             assert torch.equal(ok, torch.isfinite(b)), (at, int((ok != torch.isfinite(b)).sum()))
             assert float((a[ok] - b[ok]).abs().max()) < 1e-4 * max(1.0, float(a[ok].abs().max()))
+
+
+def test_matrix_memory_chunks_in_runs_of_bounded_scratch():
+    """as for the state-space scan, with the keys' own state and the gates of all chunks"""
+    from pegainfer_amd import ops_blocks as Bk
+    g = torch.Generator().manual_seed(3)
+    heads, dim, vdim, lens, slots, cap = 16, 256, 512, [1900, 100, 2300, 20], [2, 0, 3, 1], 15.0
+    cols = heads * (2 * dim + vdim + 2)
+    offs = [0, heads * dim, 2 * heads * dim, heads * (2 * dim + vdim), heads * (2 * dim + vdim + 1)]
+    proj = torch.randn(sum(lens), cols, generator=g).cuda()
+    ib, fb = torch.randn(heads, generator=g).cuda(), (torch.randn(heads, generator=g) + 2).cuda()
+    runs = []
+    for scan_max in (0, 64):
+        state = torch.zeros(4, heads * (dim * vdim + dim + 1)).cuda()
+        runs.append((Bk.gated_matrix_memory(proj, offs, ib, fb, cap, state, heads, dim, vdim, Bk.Ragged(lens, slots=slots), scan_max=scan_max), state))
+    # outputs are quotients by a sum that can be small: those of a typical size agree to rounding, all of them to a few units of it
+    (a, sa), (b, sb) = runs
+    assert float((sa - sb).abs().max()) < 2e-5 * float(sa.abs().max())
+    err = (a - b).abs() / (1 + a.abs())
+    assert float(err.mean()) < 1e-5 and float(err.max()) < 2e-2

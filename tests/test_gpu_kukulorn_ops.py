@@ -498,6 +498,24 @@ def test_state_space_chunks_let_nothing_reach_earlier_tokens(N, P, bad, what):
             assert float((a[ok] - b[ok]).abs().max()) < 1e-4 * max(1.0, float(a[ok].abs().max()))
 
 
+def test_state_space_chunks_in_runs_of_bounded_scratch():
+    """sizes whose scratch holds 31 chunks: runs that end inside an entry, at its last chunk and beyond, against the scan"""
+    Bk = B()
+    g = torch.Generator().manual_seed(3)
+    heads, N, P, lens, slots = 16, 256, 512, [1900, 100, 2300, 20], [2, 0, 3, 1]
+    T, inner = sum(lens), heads * P
+    assert 2 ** 26 // Bk.ffi.lib().pegainfer_ssd_scan_workspace(1, heads, N, P) == 31
+    xbc = torch.randn(T, inner + 2 * N, generator=g).cuda()
+    xbc[:, inner:] *= N ** -0.25
+    args = (torch.randn(T, heads, generator=g).cuda(), 0, torch.linspace(-4, 2, heads).cuda(), torch.randn(heads, generator=g).cuda(), torch.randn(heads, generator=g).cuda())
+    runs = []
+    for scan_max in (0, 64):
+        state = torch.ones(4, heads * N * P).cuda()
+        runs.append((Bk.ssd_scan(xbc, *args, state, heads, 1, N, P, Bk.Ragged(lens, slots=slots), scan_max=scan_max), state))
+    for a, b in zip(*runs):
+        assert float((a - b).abs().max()) < 2e-5 * float(a.abs().max())
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}

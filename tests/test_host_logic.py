@@ -197,3 +197,45 @@ def test_wide_attention_tiles_leave_no_key_split_behind(tables, lens, heads, kv,
     (keys None: the choice may not depend on the contexts) take them only where nothing was dealt"""
     a = np.array(lens, np.int32)
     assert tables.wide_rows(ctypes.c_void_p(a.ctypes.data), len(lens), int(a.sum()), heads // max(kv, 1), kv, 2 ** 31 - 1 if keys is None else keys) == rows
+
+
+def test_optional_scratch_is_given_up_when_there_is_no_memory(tmp_path):
+    """csrc/host/optional_scratch.h with an allocator that refuses more than 1000 bytes: a refusal leaves nothing behind, smaller needs are met
+    afterwards, everything is released once"""
+    import subprocess
+    (tmp_path / "t.cpp").write_text(r"""
+#include <cstdlib>
+#include <set>
+#include "optional_scratch.h"
+int main() {
+  std::set<void*> live;
+  pq::OptionalScratch s;
+  auto alloc = [&](size_t n) -> void* { if (n > 1000) return nullptr; void* p = std::malloc(n); live.insert(p); return p; };
+  auto release = [&](float* p) { if (!live.erase(p)) std::exit(9); std::free(p); };
+  if (!s.grow(0, alloc, release) || s.p) return 1;
+  if (!s.grow(100, alloc, release) || !s.p || s.cap != 100) return 2;
+  float* first = s.p;
+  if (!s.grow(60, alloc, release) || s.p != first || s.cap != 100) return 3;
+  if (s.grow(251, alloc, release) || s.p || s.cap || !live.empty()) return 4;
+  if (!s.grow(0, alloc, release) || s.p) return 5;
+  if (!s.grow(250, alloc, release) || !s.p || s.cap != 250 || live.size() != 1) return 6;
+  s.drop(release);
+  s.drop(release);
+  return s.p || s.cap || !live.empty() ? 7 : 0;
+}
+""")
+    host = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc", "host")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", host, "-o", str(tmp_path / "t"), str(tmp_path / "t.cpp")], check=True)
+    assert subprocess.run([str(tmp_path / "t")]).returncode == 0
+
+
+def test_scratch_of_the_chunk_forms_is_bounded(built_libs):
+    """256 MB of states (or one chunk's) however long the step, and the gates' 768 bytes per chunk and head beside them"""
+    L = ffi.lib()
+    for heads, dim, vdim in ((32, 128, 64), (1, 5, 33), (64, 256, 1024)):
+        per = L.pegainfer_ssd_scan_workspace(1, heads, dim, vdim)
+        assert L.pegainfer_ssd_scan_workspace(2, heads, dim, vdim) == 2 * per and L.pegainfer_ssd_scan_workspace(0, heads, dim, vdim) == 0
+        for n in (16, 1000, 30000):
+            assert L.pegainfer_ssd_scan_workspace(n, heads, dim, vdim) == min(n, max(1, 2 ** 26 // per)) * per
+            mem = L.pegainfer_gated_matrix_memory_workspace(n, heads, dim, vdim) - n * heads * 192
+            assert 0 < mem <= max(2 ** 26, L.pegainfer_gated_matrix_memory_workspace(1, heads, dim, vdim))
