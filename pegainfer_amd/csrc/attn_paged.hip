@@ -348,11 +348,34 @@ __global__ __launch_bounds__(256) void paged_attention_kernel(
             }
           }
         } else {
-          for (int d = sub; d < kw; d += 4) dk[d] = ld(kp + d);
-          for (int d = sub; d < vdim; d += 4) {
-            const float t = ld(vp + d);
-            dv[d] = t;
-            if (tail && d >= kw) dk[d] = t;
+          // one side off: the other keeps its 16-byte loads (two fp32 prompts of 470, 8 heads, keys of 128 and values of 100: 127 us, 142 with
+          // single values on both sides)
+          if (vec_k) {
+            for (int d = sub * 8; d < kw; d += 32) {
+              float t[8];
+              Vec8<A>::load(kp + d, t);
+#pragma unroll
+              for (int u = 0; u < 8; ++u) dk[d + u] = t[u];
+            }
+          } else {
+            for (int d = sub; d < kw; d += 4) dk[d] = ld(kp + d);
+          }
+          if (vec_v) {
+            for (int d = sub * 8; d < vdim; d += 32) {
+              float t[8];
+              Vec8<A>::load(vp + d, t);
+#pragma unroll
+              for (int u = 0; u < 8; ++u) {
+                dv[d + u] = t[u];
+                if (tail && d >= kw) dk[d + u] = t[u];
+              }
+            }
+          } else {
+            for (int d = sub; d < vdim; d += 4) {
+              const float t = ld(vp + d);
+              dv[d] = t;
+              if (tail && d >= kw) dk[d] = t;
+            }
           }
         }
       }

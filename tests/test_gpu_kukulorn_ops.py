@@ -516,6 +516,43 @@ def test_state_space_chunks_in_runs_of_bounded_scratch():
         assert float((a - b).abs().max()) < 2e-5 * float(a.abs().max())
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim,vdim,off", [(128, 100, 0), (100, 128, 0), (24, 20, 0), (20, 24, 0), (24, 24, 4), (136, 130, 0), (40, 8, 0), (7, 64, 0)])
+def test_general_attention_with_one_side_off_sixteen_bytes(dim, vdim, off, dtype):
+    """a key or value size that is no multiple of eight, or values that start off 16 bytes, beside a side that is loaded in chunks: against the softmax
+    in 64 bits; 1e-5 covers sums of 136 products and 90 weights in fp32, a bf16 output adds 2^-8 of it"""
+    from pegainfer_amd import ops_blocks as B
+    import ctypes
+    g = torch.Generator().manual_seed(dim + vdim)
+    H, G, page, lens, past = 4, 2, 16, [3, 70, 1], [0, 20, 65]
+    T = sum(lens)
+    need = [-(-(a + b) // page) for a, b in zip(lens, past)]
+    v_off = -(-page * G * dim // 8) * 8 + off
+    stride = -(-(v_off + page * G * vdim) // 8) * 8
+    cache = torch.randn(sum(need) * stride, generator=g).to(DT[dtype])
+    q = torch.randn(T, H, dim, generator=g)
+    pos = [b + i for a, b in zip(lens, past) for i in range(a)]
+    ent = [e for e, a in enumerate(lens) for _ in range(a)]
+    first = np.cumsum([0] + need)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32).cuda()  # noqa: E731
+    cd, qd, posd, entd, ind, ids = cache.cuda(), q.cuda(), i32(pos), i32(ent), i32(first.tolist()), i32(list(range(sum(need))))
+    t = B.attention_tiles(lens, H // G, "cuda", 16)
+    out = torch.full((T, H * vdim), float("nan"), dtype=DT[dtype], device="cuda")
+    a = B.AttnOptions(n_split=1, plain=1)
+    B._chk(B.ffi.lib().pegainfer_paged_attention_opt(
+        qd.data_ptr(), cd.data_ptr(), stride, 0, v_off, page, posd.data_ptr(), entd.data_ptr(), ind.data_ptr(), ids.data_ptr(), H, G, dim, vdim,
+        dim ** -0.5, 1.0, *(c.data_ptr() for c in t), t[0].numel(), out.data_ptr(), out.stride(0), ctypes.addressof(a), B._dt(cd), B._stream()), "attention")
+    pages = cache.double().view(-1, stride)
+    for r in range(T):
+        mine = pages[first[ent[r]]:first[ent[r] + 1]]
+        k = mine[:, :page * G * dim].reshape(-1, G, dim)[:pos[r] + 1]
+        v = mine[:, v_off:v_off + page * G * vdim].reshape(-1, G, vdim)[:pos[r] + 1]
+        for h in range(H):
+            ref = torch.softmax(k[:, h // 2] @ q[r, h].double() * dim ** -0.5, 0) @ v[:, h // 2]
+            got = out[r, h * vdim:(h + 1) * vdim].cpu().double()
+            assert ((got - ref).abs() <= 1e-5 + (ref.abs() / 256 if dtype == "bfloat16" else 0)).all(), (r, h)
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
