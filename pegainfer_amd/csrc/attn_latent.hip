@@ -734,24 +734,33 @@ struct LatentCall {
   const int32_t *positions, *token_req, *page_indptr, *page_ids, *tile_row0, *tile_rows;
   int n_tiles, H, r, dr; float scale; float* ws; int n_tokens, sp; LatentCut cut; hipStream_t s;
 
+  // every instance may take what a compute unit has, asked for once
+  template <typename K>
+  static bool all_lds(K kern) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) == hipSuccess;
+  }
   template <typename A, typename K>
   void run(K kern, int subs, size_t lds) const {
-    if (lds > 48 * 1024)
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     kern<<<dim3(n_tiles, sp, subs), 256, lds, s>>>(qc, o_lat, static_cast<const A*>(cache), page_stride, layer_off, page_size, positions, token_req,
                                            page_indptr, page_ids, tile_row0, tile_rows, H, r, dr, scale, ws, n_tokens, sp, cut);
   }
   template <int ND>
   void wide() const {
+    auto kern = &latent_attn_mfma_kernel<ND>;
+    static const bool once = all_lds(kern);
+    (void)once;
     const int Epad = (r + dr + 31) & ~31;
-    run<uint16_t>(&latent_attn_mfma_kernel<ND>, 1, (size_t)(kTileRows + kTileKeys) * (Epad + 8) * 2);
+    run<uint16_t>(kern, 1, (size_t)(kTileRows + kTileKeys) * (Epad + 8) * 2);
   }
   template <typename A, int ND, int RB>
   void few_rows() const {
+    auto kern = &latent_attn_few_kernel<A, ND, RB>;
+    static const bool once = all_lds(kern);
+    (void)once;
     constexpr int kRows = 16 * RB, KB = std::is_same<A, float>::value ? 16 : 32;
     const size_t cs = (r + dr + KB - 1) / KB * KB + 16 / sizeof(A);
     // the parts of a tile past its rows come last: between the others they would take those from some of the XCDs' turns
-    run<A>(&latent_attn_few_kernel<A, ND, RB>, kTileRows / kRows,
+    run<A>(kern, kTileRows / kRows,
            (kTileKeys * cs + kRows * (kTileKeys + 4)) * sizeof(A) + (4 * kRows * (kTileKeys + 4) + kRows) * sizeof(float));
   }
   bool narrow() const { return (int64_t)n_tokens * H <= 16 * (int64_t)n_tiles; }
