@@ -791,6 +791,7 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   const float inv_cap = form.softcap > 0.f ? 1.0f / form.softcap : 0.f;
   // uniform: no key after `last` concerns the wave; keys of [all_lo, all_hi] are seen by all of its rows, without a look at each
   const int last = rg * 16 < nrows ? positions[row0 + min(rg * 16 + 15, nrows - 1) / nqh] : -1;
+  const int first_lo = last >= 0 ? attn_row_lo(form, positions[row0 + rg * 16 / nqh]) : 0;      // the lowest key of any of its rows
   const int all_lo = last >= 0 ? attn_row_lo(form, last) : 0, all_hi = rg * 16 + 15 < nrows ? positions[row0 + rg * 16 / nqh] : -1;
   bf16x8_t qf[P / 32];
   {
@@ -869,9 +870,10 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   // byte addresses inside a tile: swz(row + 16) = swz(row) for both row widths, so the second half of the keys lies 16 rows on
   const uint32_t ka = (uint32_t)(krow * P * 2 + ((lg ^ swz(krow)) << 4));
   const uint32_t va = (uint32_t)(vrow * P * 2 + ((((l15 & 3) >> 1) ^ swz(vrow)) << 4) + (l15 & 1) * 8);
-  auto multiply = [&](int k0, int stage) {
-    const int kb = k0 + 32 * kh;
-    if (kb > last || kb >= kmax) return;             // uniform over the wave
+  // masked: some row of the wave does not see some of these keys.  Values of keys that none of them sees go in as zeros: an infinity or no number
+  // times a weight of zero would reach rows that the form of 16-row tiles keeps it from.  Two bodies, chosen at the top: masking inside one
+  // cost 13 % (the branch, or 32 instructions a tile, stands between the weights and the second products); 77 us behind 3072 tokens so, 79 unmasked.
+  auto multiply_keys = [&](int kb, int stage, auto masked) {
     const unsigned char* kt = smraw + stage * 2 * Sh::kTile;
     f32x4 sc[2] = {};
 #pragma unroll
@@ -912,7 +914,8 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) sc[t][r] *= kLog2e;
     }
-    if (kb < all_lo || kb + 31 > all_hi) {           // uniform: some row of the wave does not see some of these keys
+    uint32_t see[4];
+    if constexpr (decltype(masked)::value) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -920,6 +923,12 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
           const int kp = kb + 16 * t + 4 * lg + r;
           if (!(kp <= rpos && (kp >= rlo || kp < form.keep_first))) sc[t][r] = -INFINITY;
         }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int kp = kb + 16 * (i >> 1) + 4 * lg + 2 * (i & 1);
+        auto seen = [&](int j) { return j <= last && (j >= first_lo || j < form.keep_first); };
+        see[i] = (seen(kp) ? 0xFFFFu : 0u) | (seen(kp + 1) ? 0xFFFF0000u : 0u);
+      }
     }
     float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])), fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
     if (__any(!(tmax <= mrun + kJump))) {            // uniform; the first keys of a row always, a NaN too
@@ -950,10 +959,17 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
       const uint32_t at = vt + (va ^ (uint32_t)(cb << 5));
-      const u32x2 v0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)at));
-      const u32x2 v1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)(at + 16 * P * 2)));
+      u32x2 v0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)at));
+      u32x2 v1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)(at + 16 * P * 2)));
+      if constexpr (decltype(masked)::value) { v0.x &= see[0]; v0.y &= see[1]; v1.x &= see[2]; v1.y &= see[3]; }
       o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, u32x4{v0.x, v0.y, v1.x, v1.y}), pf, o[cb], 0, 0, 0);
     }
+  };
+  auto multiply = [&](int k0, int stage) {           // uniform over the wave
+    const int kb = k0 + 32 * kh;
+    if (kb > last || kb >= kmax) return;
+    if (kb < all_lo || kb + 31 > all_hi) multiply_keys(kb, stage, std::true_type{});
+    else multiply_keys(kb, stage, std::false_type{});
   };
   int k[S + 1];                                      // k[i]: the tile i ahead
   k[0] = kfirst;

@@ -553,6 +553,49 @@ def test_general_attention_with_one_side_off_sixteen_bytes(dim, vdim, off, dtype
             assert ((got - ref).abs() <= 1e-5 + (ref.abs() / 256 if dtype == "bfloat16" else 0)).all(), (r, h)
 
 
+@pytest.mark.parametrize("tile_rows", [32, 64])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("H,G,dim,window", [(4, 4, 64, 0), (8, 2, 128, 0), (8, 2, 256, 0), (4, 4, 128, 20)])
+def test_wide_tiles_bring_no_value_further_than_sixteen_rows(H, G, dim, window, bad, tile_rows):
+    """a value that is infinite or no number reaches, beside the rows that see it, at most those that share sixteen rows with one of them (as in the
+    form of 16-row tiles), not the rest of a wide tile: the others are bit for bit what they are without it"""
+    from pegainfer_amd import ops_blocks as B
+    import ctypes
+    g = torch.Generator().manual_seed(dim)
+    page, T, per = 16, 100, H // G
+    need = -(-T // page)
+    stride = page * G * 2 * dim
+    v_off = page * G * dim
+    sound = torch.randn(need * stride, generator=g).bfloat16()
+    qd = torch.randn(T, H, dim, generator=g).cuda()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32).cuda()  # noqa: E731
+    pos, ent, ind, ids = i32(list(range(T))), i32([0] * T), i32([0, need]), i32(list(range(need)))
+    t = B.attention_tiles([T], per, "cuda", tile_rows)
+
+    def run(cache):
+        cd, out = cache.cuda(), torch.empty(T, H * dim, dtype=torch.bfloat16, device="cuda")
+        a = B.AttnOptions(n_split=1, tile_rows=tile_rows, window=window)
+        B._chk(B.ffi.lib().pegainfer_paged_attention_opt(
+            qd.data_ptr(), cd.data_ptr(), stride, 0, v_off, page, pos.data_ptr(), ent.data_ptr(), ind.data_ptr(), ids.data_ptr(), H, G, dim, dim,
+            dim ** -0.5, 1.0, *(c.data_ptr() for c in t), t[0].numel(), out.data_ptr(), out.stride(0), ctypes.addressof(a), 0, B._stream()), "attention")
+        return out.cpu()
+
+    ref = run(sound)
+    for at in (0, 15, 31, 40, 63, 64, 99):
+        cache = sound.clone()
+        cache.view(need, stride)[at // page, v_off + (at % page) * G * dim + 3] = bad          # head 0 of that token
+        got = run(cache)
+        group, per_tile = 16 // per, tile_rows // per            # tokens of sixteen rows, of a tile
+        sees = [at <= r and (not window or r - at < window) for r in range(T)]
+        first = lambda r: r // per_tile * per_tile + r % per_tile // group * group  # noqa: E731
+        near = {first(r) for r in range(T) if sees[r]}
+        for r in range(T):
+            if sees[r]:
+                assert not torch.isfinite(got[r, 3]), (at, r)
+            elif first(r) not in near:
+                assert torch.equal(got[r], ref[r]), (at, r)
+
+
 FORMS = {"plain": {}, "cap far above the scores": {"softcap": 60.0}, "binding cap": {"softcap": 1.5}, "window and kept first": {"window": 37, "keep_first": 3},
          "table bias": {"bias": 90, "window": 150}, "slope and cap": {"slope": True, "softcap": 4.0}, "blocks and sink": {"block": 48, "sink": True},
          "gate per value, head norm": {"gate": 1, "norm": True}, "gate per head, bias": {"gate": 2, "bias": 20}}
