@@ -761,7 +761,7 @@ struct Model {
     const int P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     DZ_K(pegainfer_route_sigmoid_grouped(h, w.router, w.corr, route_e, route_w, D, f.experts, f.groups, f.keep, f.top, T, dtype, S()));
-    // 128-row tiles for the matrix-core form (bf16, prompt-sized steps), 64-row tiles otherwise
+    // few rows: tiles of the step's rows; otherwise 128-row tiles for the matrix-core form of bf16 weights, 64-row tiles
     const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0);
     DZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
     pegainfer_gemm_desc d{};
