@@ -381,6 +381,12 @@ pegainfer_status_t pegainfer_act_rows(const void* in, int64_t in_row_stride, voi
                                       int32_t act, int32_t dtype, pegainfer_stream_t stream);
 pegainfer_status_t pegainfer_glu_rows(const void* gate, const void* up, int64_t in_row_stride, void* out, int64_t out_row_stride,
                                       int32_t I, int32_t rows, int32_t act, int32_t dtype, pegainfer_stream_t stream);
+/* The end of a step's logits [rows][vocab], one launch: v = src (src_dtype) times scale, then cap * tanh(v / cap) where cap > 0; out32 = v,
+ * out16 = v rounded to bf16; with out_tokens the greedy token of every row of out16 (ties -> lowest index; state_scratch as in
+ * pegainfer_batched_top1).  src may be out32 (fp32) or, with scale 1 and no cap, out16 (bf16). */
+pegainfer_status_t pegainfer_logits_finish(const void* src, int32_t src_dtype, float* out32, Half* out16, float scale, float cap,
+                                           int32_t vocab_size, int32_t rows, uint8_t* state_scratch, int32_t* out_tokens,
+                                           pegainfer_stream_t stream);
 /* out[i] = cap * tanh(in[i] / cap) over n fp32 values (in place allowed) */
 pegainfer_status_t pegainfer_softcap_rows(const float* in, float* out, int64_t n, float cap, pegainfer_stream_t stream);
 

@@ -125,7 +125,7 @@ struct Model {
   int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
   float *xw = nullptr, *logits32 = nullptr;
-  void *hw = nullptr, *logits = nullptr;
+  void* hw = nullptr;
   Half* logits16 = nullptr;      // bf16 image of the wanted rows' logits for the samplers
   int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
@@ -516,7 +516,7 @@ struct Model {
     size_t c = 16;
     while (c < n) c *= 2;
     auto* wo = &want_owned;
-    if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc_a(&logits, c * V, wo) || dalloc(&logits32, c * V, wo) ||
+    if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
         dalloc(&logits16, c * V, wo) || dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
       return -1;
     cap_want = c;
@@ -736,15 +736,9 @@ struct Model {
     if (W > 0) {
       DZ_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
       DZ_K(pegainfer_dyt_norm(xw, final_norm.alpha, final_norm.w, final_norm.b, hw, D, W, dtype, S()));
-      if (linear(head, hw, logits, V, W, D)) return -1;
-      if (dtype == PEGAINFER_DTYPE_BF16) {
-        DZ_K(deepseek_bf16_to_f32_cuda(static_cast<const Half*>(logits), logits32, W * V, S()));
-        DZ_HIP(hipMemcpyAsync(logits16, logits, (size_t)W * V * 2, hipMemcpyDeviceToDevice, stream));
-      } else {
-        DZ_HIP(hipMemcpyAsync(logits32, logits, (size_t)W * V * 4, hipMemcpyDeviceToDevice, stream));
-        DZ_K(deepseek_f32_to_bf16_cuda(logits32, logits16, W * V, S()));
-      }
-      if (out_tokens) DZ_K(pegainfer_batched_top1(logits16, V, W, V, top1_state, tokens_d, S()));
+      void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
+      if (linear(head, hw, lg, V, W, D)) return -1;
+      DZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr, S()));
     }
     last_rows = W;
     DZ_HIP(hipEventRecord(ev1, stream));

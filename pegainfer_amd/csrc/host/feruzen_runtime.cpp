@@ -152,7 +152,7 @@ struct Model {
   int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
   float *xw = nullptr, *logits32 = nullptr;
-  void *hw = nullptr, *logits = nullptr;
+  void* hw = nullptr;
   Half* logits16 = nullptr;
   int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
@@ -706,7 +706,7 @@ struct Model {
     size_t c = 16;
     while (c < n) c *= 2;
     auto* wo = &want_owned;
-    if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc_a(&logits, c * V, wo) || dalloc(&logits32, c * V, wo) ||
+    if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
         dalloc(&logits16, c * V, wo) || dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
       return -1;
     cap_want = c;
@@ -1034,15 +1034,9 @@ struct Model {
       FZ_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
       FZ_K(pegainfer_group_rms_add(nullptr, xw, PEGAINFER_DTYPE_F32, final_norm, groups, eps, nullptr, hw, D, W, dtype, nullptr, 0,
                                    nullptr, 0, nullptr, nullptr, S()));
-      if (linear(embed, hw, logits, V, W, D)) return -1;
-      if (dtype == PEGAINFER_DTYPE_BF16) {
-        FZ_K(deepseek_bf16_to_f32_cuda(static_cast<const Half*>(logits), logits32, W * V, S()));
-        FZ_HIP(hipMemcpyAsync(logits16, logits, (size_t)W * V * 2, hipMemcpyDeviceToDevice, stream));
-      } else {
-        FZ_HIP(hipMemcpyAsync(logits32, logits, (size_t)W * V * 4, hipMemcpyDeviceToDevice, stream));
-        FZ_K(deepseek_f32_to_bf16_cuda(logits32, logits16, W * V, S()));
-      }
-      if (out_tokens) FZ_K(pegainfer_batched_top1(logits16, V, W, V, top1_state, tokens_d, S()));
+      void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
+      if (linear(embed, hw, lg, V, W, D)) return -1;
+      FZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr, S()));
     }
     return 0;
     };

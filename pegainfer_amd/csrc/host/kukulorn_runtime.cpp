@@ -1015,9 +1015,8 @@ struct Model {
       KK_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
       KK_K(pegainfer_terms_rms_add(xw, nullptr, 0, nullptr, final_norm, eps, hw, PEGAINFER_DTYPE_F32, D, W, dtype, S()));
       if (linear_strided(embed, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
-      if (logit_cap > 0.f) KK_K(pegainfer_softcap_rows(logits32, logits32, (int64_t)W * V, logit_cap, S()));
-      KK_K(deepseek_f32_to_bf16_cuda(logits32, logits16, W * V, S()));
-      if (out_tokens) KK_K(pegainfer_batched_top1(logits16, V, W, V, top1_state, tokens_d, S()));
+      KK_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, logit_cap, V, W, top1_state,
+                                   out_tokens ? tokens_d : nullptr, S()));
     }
     return 0;
     };

@@ -1018,9 +1018,8 @@ struct Model {
       RX_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
       RX_K(pegainfer_scalar_rms_add(xw, nullptr, dtype, nullptr, 0.f, nullptr, nullptr, nullptr, final_norm, eps, hw, D, W, dtype, S()));
       if (linear_strided(head, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
-      if (logit_scale != 1.0f) RX_K(pegainfer_scale_rows(logits32, V, logits32, V, V, W, logit_scale, PEGAINFER_DTYPE_F32, S()));
-      RX_K(deepseek_f32_to_bf16_cuda(logits32, logits16, W * V, S()));
-      if (out_tokens) RX_K(pegainfer_batched_top1(logits16, V, W, V, top1_state, tokens_d, S()));
+      RX_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, logit_scale, 0.f, V, W, top1_state,
+                                   out_tokens ? tokens_d : nullptr, S()));
     }
     return 0;
     };

@@ -352,10 +352,9 @@ class StepModel {
     if (before_step(c)) return -1;
     auto launches = [&]() -> int {
       if (run_step(c)) return -1;
-      if (W > 0) {
-        PSTEP_K(deepseek_f32_to_bf16_cuda(logits32, logits16, W * V, S()));
-        if (out_tokens) PSTEP_K(pegainfer_batched_top1(logits16, V, W, V, top1_state, tokens_d, S()));
-      }
+      if (W > 0)
+        PSTEP_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr,
+                                        S()));
       return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and

@@ -434,6 +434,17 @@ def glu_rows(gate, up, act="relu"):
     return out
 
 
+def logits_finish(src, state, scale=1.0, cap=0.0, tokens=True):
+    """-> (fp32 logits, their bf16 image, greedy tokens or None) of what an output projection left [rows, V]; what needs no change stays in place"""
+    rows, V = src.shape
+    f32 = src if src.dtype == torch.float32 else torch.empty((rows, V), dtype=torch.float32, device=src.device)
+    b16 = src if src.dtype == torch.bfloat16 and scale == 1.0 and cap <= 0 else torch.empty((rows, V), dtype=torch.bfloat16, device=src.device)
+    out = torch.empty(rows, dtype=torch.int32, device=src.device) if tokens else None
+    _chk(ffi.lib().pegainfer_logits_finish(_p(src), _dt(src), _p(f32), _p(b16), float(scale), float(cap), V, rows, _p(state), _p(out) if tokens else None,
+                                           _stream()), "logits_finish")
+    return f32, b16, out
+
+
 def softcap_rows(x_f32, cap):
     out = torch.empty_like(x_f32)
     _chk(ffi.lib().pegainfer_softcap_rows(_p(x_f32), _p(out), x_f32.numel(), float(cap), _stream()), "softcap_rows")

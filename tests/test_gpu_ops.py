@@ -621,6 +621,30 @@ def test_batched_top1_every_row_lowest_index_ties_and_self_resetting_state(P, ro
     assert int(state.sum().item()) == 0
 
 
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 1001), (5, 2048), (8, 65536), (33, 4104), (70000, 8)])
+@pytest.mark.parametrize("dtype,scale,cap", [("float32", 1.0, 0.0), ("float32", 0.37, 0.0), ("float32", 1.0, 15.0), ("bfloat16", 1.0, 0.0)])
+def test_logits_finish_gives_logits_their_bf16_image_and_the_greedy_tokens(P, rows, n, dtype, scale, cap):
+    """== the separate steps (factor, cap, rounding to nearest even, lowest index of the largest): exact but for the cap's tanh, twice in a row"""
+    import torch
+    from pegainfer_amd import ops_blocks as B
+    x = (torch.randn(rows, n, generator=torch.Generator().manual_seed(rows + n)) * 8).to(getattr(torch, dtype))
+    x[:, n // 3] = x[:, n // 2] = x.max()
+    state = torch.zeros(16 * rows, dtype=torch.uint8, device="cuda")
+    for _ in range(2):
+        f32, b16, tok = B.logits_finish(x.cuda(), state, scale, cap)
+        want = x.float() * scale
+        if cap:
+            want = cap * torch.tanh(want.double() / cap)
+        close = f32.cpu().double() - want.double()
+        assert float(close.abs().max()) <= (2e-6 * cap if cap else 0.0)
+        assert torch.equal(b16.cpu(), f32.cpu().bfloat16())
+        best = b16.cpu().float()
+        assert torch.equal(tok.cpu().long(), torch.from_numpy(np.argmax(best.numpy(), axis=1)))
+    assert int(state.sum().item()) == 0
+    if rows < 100:
+        assert B.logits_finish(x.cuda(), state, scale, cap, tokens=False)[2] is None and int(state.sum().item()) == 0
+
+
 @pytest.mark.parametrize("n", [5, 1000, 151936])
 def test_argmax_and_top1_lowest_index_ties(P, n):
     import torch
