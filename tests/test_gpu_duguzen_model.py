@@ -175,6 +175,34 @@ def test_long_decoding_across_the_key_split():
     eng.close()
 
 
+@pytest.mark.parametrize("dtype,name", [("bfloat16", "a"), ("float32", "b"), ("bfloat16", "odd")])
+def test_replayed_decode_steps_give_what_eager_ones_give(dtype, name):
+    """Decode steps are replayed from graphs, one per batch and context length rounded up to 256 tokens; the per-layer tap turns that off.  The
+    same bits either way: contexts of unequal length that cross the rounding, other steps between the replays, buffers that grow."""
+    cfg = CONFIGS[name]()
+    w = C.random_weights(cfg, 31)
+    engs = [C.engine_for(cfg, w, dtype, max_tokens=1200, max_requests=4) for _ in range(2)]
+    engs[1].debug_hidden_enable(True)
+    out = []
+    for eng in engs:
+        r, got = [eng.new_request() for _ in range(3)], []
+        toks = C.tokens_for(cfg, 400, 7)
+        for i, n in enumerate((250, 17, 240)):
+            got.append(eng.step([(r[i], toks[:n])]))
+        for t in range(20):
+            use = r if t % 5 else r[:1]                     # two batch sizes in turn
+            lg, tk = eng.step([(q, [toks[300 + t]]) for q in use], tokens=True)
+            got += [lg, tk]
+            if t == 12:
+                late = eng.new_request()
+                got.append(eng.step([(late, toks[:200])], want=list(range(60))))      # more rows and more wanted rows than before
+                eng.drop_request(late)
+        out.append(got)
+        eng.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_checkpoint_folder_through_the_registry_and_trace_replay(tmp_path):
     from safetensors.torch import save_file
     from pegainfer_amd import registry
