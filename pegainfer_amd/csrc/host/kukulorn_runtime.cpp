@@ -86,7 +86,6 @@ static inline float host_bf2f(uint16_t h) {
 constexpr int kPageSize = 16;   // tokens per cache page, as in the other runtimes
 constexpr int kAttRows = 16;    // (token, query head) rows of one attention workgroup
 constexpr int kSplitGroups = 512;   // most (tile, kv head, key split) workgroups of an attention launch that cuts its keys
-constexpr int kMaxSplits = 16;
 // longest entry whose state-space scan runs token by token: 32 heads of 128 x 64, scan / chunks 27 / 41 us at 128 tokens, 48 / 44 at 256,
 // 91 / 50 at 512; eight entries of 128 tokens 56 / 65 us
 constexpr int kScanMax = 224;
@@ -925,7 +924,7 @@ struct Model {
       o.softcap = a.softcap; o.window = a.window; o.keep_first = a.keep_first; o.dist_bias = w.dist_bias; o.n_dist = w.n_dist;
       o.gate = gate; o.gate_stride = proj_stride; o.gate_kind = gate_kind;
       o.tile_rows = tile_rows[ts];
-      o.n_split = wgs >= ptiles::kUnsplitGroups || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
+      o.n_split = wgs >= ptiles::kUnsplitGroups || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
       o.workspace = att_part;
       o.plain = plain_kernels ? 1 : 0;
       KK_K(pegainfer_paged_attention_opt(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,

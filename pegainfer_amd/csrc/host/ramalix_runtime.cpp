@@ -84,7 +84,6 @@ static inline float host_bf2f(uint16_t h) {
 constexpr int kPageSize = 16;   // tokens per cache page, as in the other runtimes
 constexpr int kAttRows = 16;    // (token, query head) rows of one attention workgroup
 constexpr int kSplitGroups = 512;   // most (tile, kv head, key split) workgroups of an attention launch that cuts its keys
-constexpr int kMaxSplits = 16;
 
 enum { kDiffAttn = 1, kBlockAttn = 2, kChannelDelta = 3 };
 struct AttnCfg {
@@ -992,7 +991,7 @@ struct Model {
         // a step of few rows (decoding, short portions) cannot fill the chip with one workgroup per (row tile, kv head): its
         // keys are dealt to several workgroups.  The count depends on the step's shape only, never on the contexts' lengths.
         const int wgs = (int)tile_cnt[ts] * a.kv;
-        const int nsplit = wgs >= 128 ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
+        const int nsplit = wgs >= 128 ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
         RX_K(pegainfer_paged_attention_ex(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,
                                           a.kv, a.dim, a.vdim, a.scale, two ? 1.0f - a.diff : 1.0f, tb, tb + tile_cnt[ts],
                                           tb + 2 * tile_cnt[ts], tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, c.mix_cols, a.maps,

@@ -19,6 +19,9 @@ constexpr int kGroupRows = 16;      // (token, query head) rows of one workgroup
 // requests of 64 heads over 4 behind 8192 tokens 57 / 143.  There a step takes them while no row walks more than kWideKeys keys and they give
 // kWideGroups workgroups.
 constexpr int kUnsplitGroups = 128, kWideGroups = 32, kWideKeys = 640;
+// Most workgroups that share a row tile's keys.  One past the row's last key tile ends at once, so a short context pays for its own only: one
+// request of 16 heads over 4 behind 4000 tokens 26 -> 10 us with 64 instead of 16 (four tiles of 64 keys each, a quarter of the chip).
+constexpr int kMaxSplits = 64;
 
 inline size_t count(const int32_t* lens, int n, int per, int rows) {
   const int tpt = std::max(1, rows / per), cuts = (per + rows - 1) / rows;

@@ -23,7 +23,6 @@ namespace psx {
 using namespace pstep;
 
 constexpr int kSplitGroups = 512;   // most (tile, kv head, key split) workgroups of an attention launch that cuts its keys
-constexpr int kMaxSplits = 16;
 constexpr int kFusedRows = 8;       // steps of at most so many rows make the decay inputs inside the scan
 constexpr int kScanMax = 32;        // longest entry whose recurrence runs token by token
 constexpr int kSyntheticRank = 32;  // of the decays' two-step projection when no tensor tells it
@@ -352,7 +351,7 @@ class Model : public StepModel {
     o.sink = w.sink;
     o.gate = at(proj, (size_t)a.o_g); o.gate_stride = c.proj_rows; o.gate_kind = PEGAINFER_GATE_PER_HEAD;
     o.tile_rows = t.rows;
-    o.n_split = wgs >= ptiles::kUnsplitGroups || t.rows > kGroupRows ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
+    o.n_split = wgs >= ptiles::kUnsplitGroups || t.rows > kGroupRows ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
     o.workspace = part;
     o.plain = plain_kernels ? 1 : 0;
     o.shared_tail = a.tail();

@@ -24,7 +24,6 @@ namespace pzf {
 using namespace pstep;
 
 constexpr int kSplitGroups = 512;   // most (tile, kv head, key split) workgroups of an attention launch that cuts its keys
-constexpr int kMaxSplits = 16;
 constexpr int kFewTiles = 128;      // launches of the latent attention of fewer tiles deal their keys to several
 constexpr int kMaxDeals = 64;
 constexpr int kScanMax = 32;        // longest entry whose recurrence runs token by token
@@ -384,7 +383,7 @@ class Model : public StepModel {
     o.window = c.window;
     o.dist_slope = w.slopes;
     o.tile_rows = t.rows;
-    o.n_split = wgs >= ptiles::kUnsplitGroups || t.rows > kGroupRows ? 1 : std::max(1, std::min(kMaxSplits, kSplitGroups / wgs));
+    o.n_split = wgs >= ptiles::kUnsplitGroups || t.rows > kGroupRows ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
     o.workspace = part;
     o.plain = plain_kernels ? 1 : 0;
     PSTEP_K(pegainfer_paged_attention_opt(qf, cache, page_stride, c.k_off, c.v_off, kPageSize, s.pos, s.entry, s.page_indptr, s.pages, c.heads,

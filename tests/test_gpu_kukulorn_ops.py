@@ -269,6 +269,30 @@ def crafted_attention(dtype, n, plan, window=0, keep_first=0, softcap=0.0, tab=N
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("form", [{}, dict(window=40), dict(window=70, keep_first=10), dict(block=100)])
+@pytest.mark.parametrize("shape", [(8, 2, 64, 64, 3), (6, 6, 20, 36, 1), (4, 1, 256, 256, 4), (8, 2, 72, 20, 2)])      # heads, kv heads, sizes, rows
+def test_splits_without_a_key_leave_nothing_and_are_not_read(dtype, form, shape):
+    """up to 64 workgroups share a row's keys: those past its last key tile (or past its window) end at once, whatever the workspace holds.  The
+    sums differ from the unsplit launch's by their order alone (fp32), and by the rounding of weights against another maximum (bf16)."""
+    Bk = B()
+    H, G, d, dv, rows = shape
+    gen = torch.Generator().manual_seed(d + rows)
+    ps = 16 * G * (d + dv)
+    cache = dev(torch.randn(70 * ps, generator=gen), dtype)
+    ids, indptr = torch.randperm(70, generator=gen).int().cuda(), torch.tensor([0, 70], dtype=torch.int32).cuda()
+    for start in (0, 61, 64, 500, 1100):
+        rg = Bk.Ragged([rows], starts=[start])
+        q = torch.randn(rows, H, d, generator=gen).cuda()
+        call = lambda **kw: Bk.paged_attention_masked(q, cache, ps, 0, 16 * G * d, 16, rg, indptr, ids, G, dv, d ** -0.5, **form, **kw)  # noqa: E731
+        whole = call()
+        for n_split in (2, 16, 64):
+            want = Bk.ffi.lib().pegainfer_paged_attention_workspace(Bk.attention_tiles(rg.lens, H // G, q.device)[0].numel(), G, dv, 1, n_split)
+            poison = torch.full((want,), float("nan"), device="cuda")       # the block that the launch's workspace is taken from
+            del poison
+            close(call(n_split=n_split), whole.double().cpu(), dtype, tol32=2e-6, tol16=1e-2)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("plan", [[300], [290] + [1] * 10, [64, 64, 2, 62, 2, 96, 10]])
 def test_one_far_key_among_hundreds_takes_the_weight(dtype, plan):
     """key 3 scores 30 against 1 for every other key: every later row reads (nearly) position 3, in a prompt's portion and in
