@@ -381,6 +381,11 @@ pegainfer_status_t pegainfer_act_rows(const void* in, int64_t in_row_stride, voi
                                       int32_t act, int32_t dtype, pegainfer_stream_t stream);
 pegainfer_status_t pegainfer_glu_rows(const void* gate, const void* up, int64_t in_row_stride, void* out, int64_t out_row_stride,
                                       int32_t I, int32_t rows, int32_t act, int32_t dtype, pegainfer_stream_t stream);
+/* dst (device) <- the first *pinned_count 32-bit words of pinned_src, both read when the launch runs (a captured one: at every replay).  Source and
+ * count lie in pinned, coherent host memory; source and destination hold a multiple of four words, PEGAINFER_FETCH_WORDS at least, and start
+ * on 16 bytes. */
+#define PEGAINFER_FETCH_WORDS 4096
+pegainfer_status_t pegainfer_fetch_words(void* dst, const void* pinned_src, const int32_t* pinned_count, pegainfer_stream_t stream);
 /* The end of a step's logits [rows][vocab], one launch: v = src (src_dtype) times scale, then cap * tanh(v / cap) where cap > 0; out32 = v,
  * out16 = v rounded to bf16; with out_tokens the greedy token of every row of out16 (ties -> lowest index; state_scratch as in
  * pegainfer_batched_top1).  src may be out32 (fp32) or, with scale 1 and no cap, out16 (bf16). */

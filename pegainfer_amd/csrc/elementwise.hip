@@ -3,6 +3,7 @@
 // one rounding at the store exactly where the reference rounds.
 //   add, silu_mul (two rounding variants), embedding (3 variants), bf16<->f32 casts.
 #include "common.h"
+#include "pegainfer_kernels_blocks.h"
 
 namespace pk {
 
@@ -132,7 +133,26 @@ __global__ void zero_words_kernel(uint32_t* __restrict__ p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
 }
 
+// `*count` words of pinned host memory into device memory, the first launch of a captured step.  The first 16 KB are requested beside the count,
+// not behind it: one round trip to the host where two would be.
+// 4 KB in 3.4 us, with no copy command for the replay to wait behind.
+__global__ __launch_bounds__(1024) void fetch_words_kernel(const u32x4* __restrict__ src, const int32_t* __restrict__ count, u32x4* __restrict__ dst) {
+  const int i = threadIdx.x;
+  const u32x4 first = src[i];
+  const int n = (*count + 3) >> 2;
+  if (i < n) dst[i] = first;
+#pragma unroll 4
+  for (int k = i + 1024; k < n; k += 1024) dst[k] = src[k];
+}
+static_assert(PEGAINFER_FETCH_WORDS == 4096, "fetch_words_kernel requests 1024 chunks of four words whatever the count is");
+
 extern "C" {
+
+pegainfer_status_t pegainfer_fetch_words(void* dst, const void* pinned_src, const int32_t* pinned_count, pegainfer_stream_t stream) {
+  if (!dst || !pinned_src || !pinned_count || !host_aligned16(dst) || !host_aligned16(pinned_src)) return (pegainfer_status_t)hipErrorInvalidValue;
+  fetch_words_kernel<<<1, 1024, 0, as_stream(stream)>>>(static_cast<const u32x4*>(pinned_src), pinned_count, static_cast<u32x4*>(dst));
+  return last_error();
+}
 
 pegainfer_status_t pegainfer_zero_words(void* ptr, int32_t n_words, pegainfer_stream_t stream) {
   if (n_words > 0)

@@ -29,6 +29,7 @@
 
 #include "kv_pool.h"
 #include "row_tiles.h"
+#include "step_io.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -117,7 +118,7 @@ struct Model {
   PagePool pool{0};
   std::vector<KvState> requests;
   // step buffers (grow-only, sized by token rows / wanted rows)
-  size_t cap_rows = 0, cap_want = 0, cap_meta = 0;
+  size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
   float *x = nullptr, *qc = nullptr, *olat = nullptr, *ypairs = nullptr, *route_w = nullptr, *attn_ws = nullptr;
   size_t attn_ws_cap = 0;
@@ -139,9 +140,8 @@ struct Model {
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
     graphs.clear();
   }
-  int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
-  uint8_t *meta_host = nullptr, *meta_dev = nullptr;
+  pst::StepIo io;
   // sampling scratch
   uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
@@ -531,8 +531,9 @@ struct Model {
     while (c < n) c *= 2;
     auto* wo = &want_owned;
     if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
-        dalloc(&logits16, c * V, wo) || dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
+        dalloc(&logits16, c * V, wo) || dalloc(&top1_state, c * 16, wo))
       return -1;
+    DZ_HIP(io.grow_tokens(c));
     cap_want = c;
     return 0;
   }
@@ -630,20 +631,12 @@ struct Model {
     }
     const size_t o_pages = words;
     words += total_pages;
-    if (words > cap_meta) {
+    if (words > io.words()) {
       DZ_HIP(hipStreamSynchronize(stream));
-      if (meta_host) (void)hipHostFree(meta_host);
-      if (meta_dev) (void)hipFree(meta_dev);
-      meta_host = meta_dev = nullptr;
-      cap_meta = 0;
-      size_t c = 4096;
-      while (c < words) c *= 2;
-      DZ_HIP(hipHostMalloc(reinterpret_cast<void**>(&meta_host), c * 4, hipHostMallocDefault));
-      DZ_HIP(hipMalloc(reinterpret_cast<void**>(&meta_dev), c * 4));
-      cap_meta = c;
       drop_graphs();
+      DZ_HIP(io.grow(words));
     }
-    int32_t* mh = reinterpret_cast<int32_t*>(meta_host);
+    int32_t* mh = io.host();
     {
       size_t t = 0, pg = 0;
       for (int i = 0; i < n; ++i) {
@@ -672,8 +665,8 @@ struct Model {
       }
     }
     DZ_HIP(hipEventRecord(ev0, stream));
-    DZ_HIP(hipMemcpyAsync(meta_dev, meta_host, words * 4, hipMemcpyHostToDevice, stream));
-    const int32_t* md = reinterpret_cast<const int32_t*>(meta_dev);
+    DZ_HIP(io.send(words, captured, stream));
+    const int32_t* md = io.dev();
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
     const int32_t *d_pos = md + o_pos, *d_req = md + o_req, *d_ind = md + o_ind, *d_want = md + o_want, *d_pages = md + o_pages;
     const int Ti = (int)T;
@@ -766,7 +759,7 @@ struct Model {
       DZ_K(pegainfer_dyt_norm(xw, final_norm.alpha, final_norm.w, final_norm.b, hw, D, W, dtype, S()));
       void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
       if (linear(head, hw, lg, V, W, D)) return -1;
-      DZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr, S()));
+      DZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr, S()));
     }
     return 0;
     };
@@ -781,7 +774,7 @@ struct Model {
         if (graphs.size() >= kMaxGraphs) drop_graphs();      // no replay is in flight: every step ends with a synchronisation
         hipGraph_t g = nullptr;
         DZ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = run_layers();
+        const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
         const hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
@@ -796,8 +789,8 @@ struct Model {
     last_rows = W;
     DZ_HIP(hipEventRecord(ev1, stream));
     if (W > 0 && out_logits) DZ_HIP(hipMemcpyAsync(out_logits, logits32, (size_t)W * V * 4, hipMemcpyDeviceToHost, stream));
-    if (W > 0 && out_tokens) DZ_HIP(hipMemcpyAsync(out_tokens, tokens_d, (size_t)W * 4, hipMemcpyDeviceToHost, stream));
     DZ_HIP(hipStreamSynchronize(stream));
+    if (W > 0 && out_tokens) std::memcpy(out_tokens, io.tokens(), (size_t)W * 4);
     (void)hipEventElapsedTime(&last_step_ms, ev0, ev1);
     for (int i = 0; i < n; ++i) requests[ids[i]].seq_len += lens[i];
     return 0;
@@ -878,8 +871,7 @@ struct Model {
     free_all(&want_owned);
     if (attn_ws) (void)hipFree(attn_ws);
     if (tap) (void)hipFree(tap);
-    if (meta_dev) (void)hipFree(meta_dev);
-    if (meta_host) (void)hipHostFree(meta_host);
+    io.drop();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);

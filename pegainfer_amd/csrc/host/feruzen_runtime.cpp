@@ -32,6 +32,7 @@
 #include "optional_scratch.h"
 #include "row_tiles.h"
 #include "seq_state.h"
+#include "step_io.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -139,7 +140,7 @@ struct Model {
   struct TileSet { int per = 1, fast_hd = 0, heads = 0, kv = 0; };
   std::vector<TileSet> tile_sets;   // distinct (query heads per kv head, attention form) of the attention layers
   // step buffers
-  size_t cap_rows = 0, cap_want = 0, cap_meta = 0;
+  size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
   float *gates32 = nullptr;
   int mx_dheads = 0;
@@ -154,9 +155,8 @@ struct Model {
   float *xw = nullptr, *logits32 = nullptr;
   void* hw = nullptr;
   Half* logits16 = nullptr;
-  int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
-  uint8_t *meta_host = nullptr, *meta_dev = nullptr;
+  pst::StepIo io;
   uint8_t* sample_scratch = nullptr;
   pq::OptionalScratch chunk_ws;   // states between the chunks of long entries
   Half* top1_value = nullptr;
@@ -707,8 +707,9 @@ struct Model {
     while (c < n) c *= 2;
     auto* wo = &want_owned;
     if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
-        dalloc(&logits16, c * V, wo) || dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
+        dalloc(&logits16, c * V, wo) || dalloc(&top1_state, c * 16, wo))
       return -1;
+    FZ_HIP(io.grow_tokens(c));
     cap_want = c;
     return 0;
   }
@@ -825,20 +826,12 @@ struct Model {
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
     const size_t o_pages = words;
     words += total_pages;
-    if (words > cap_meta) {
+    if (words > io.words()) {
       FZ_HIP(hipStreamSynchronize(stream));
-      if (meta_host) (void)hipHostFree(meta_host);
-      if (meta_dev) (void)hipFree(meta_dev);
-      meta_host = meta_dev = nullptr;
-      cap_meta = 0;
-      size_t c = 4096;
-      while (c < words) c *= 2;
-      FZ_HIP(hipHostMalloc(reinterpret_cast<void**>(&meta_host), c * 4, hipHostMallocDefault));
-      FZ_HIP(hipMalloc(reinterpret_cast<void**>(&meta_dev), c * 4));
-      cap_meta = c;
       drop_graphs();
+      FZ_HIP(io.grow(words));
     }
-    int32_t* mh = reinterpret_cast<int32_t*>(meta_host);
+    int32_t* mh = io.host();
     {
       size_t t = 0, pg = 0;
       for (int i = 0; i < n; ++i) {
@@ -901,8 +894,9 @@ struct Model {
       }
     }
     FZ_HIP(hipEventRecord(ev0, stream));
-    FZ_HIP(hipMemcpyAsync(meta_dev, meta_host, words * 4, hipMemcpyHostToDevice, stream));
-    const int32_t* md = reinterpret_cast<const int32_t*>(meta_dev);
+    const bool captured = single && graphs_on && !tap_on;
+    FZ_HIP(io.send(words, captured, stream));
+    const int32_t* md = io.dev();
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
     const int32_t *d_pos = md + o_pos, *d_ent = md + o_ent, *d_row0 = md + o_row0, *d_slot = md + o_slot, *d_ind = md + o_ind,
                   *d_want = md + o_want, *d_pages = md + o_pages, *d_lpl = md + o_lpl, *d_kvlen = md + o_kvlen;
@@ -1036,13 +1030,13 @@ struct Model {
                                    nullptr, 0, nullptr, nullptr, S()));
       void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
       if (linear(embed, hw, lg, V, W, D)) return -1;
-      FZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr, S()));
+      FZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr, S()));
     }
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
-    if (single && graphs_on && !tap_on) {
+    if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, split_mask};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
@@ -1050,7 +1044,7 @@ struct Model {
       if (!exec) {
         hipGraph_t g = nullptr;
         FZ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = run_layers();
+        const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
         const hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
@@ -1065,8 +1059,8 @@ struct Model {
     last_rows = W;
     FZ_HIP(hipEventRecord(ev1, stream));
     if (W > 0 && out_logits) FZ_HIP(hipMemcpyAsync(out_logits, logits32, (size_t)W * V * 4, hipMemcpyDeviceToHost, stream));
-    if (W > 0 && out_tokens) FZ_HIP(hipMemcpyAsync(out_tokens, tokens_d, (size_t)W * 4, hipMemcpyDeviceToHost, stream));
     FZ_HIP(hipStreamSynchronize(stream));
+    if (W > 0 && out_tokens) std::memcpy(out_tokens, io.tokens(), (size_t)W * 4);
     (void)hipEventElapsedTime(&last_step_ms, ev0, ev1);
     for (int i = 0; i < n; ++i) requests[ids[i]].seq_len += lens[i];
     return 0;
@@ -1166,8 +1160,7 @@ struct Model {
     free_all(&want_owned);
     chunk_ws.drop([&](float* p) { free_scratch(p); });
     if (tap) (void)hipFree(tap);
-    if (meta_dev) (void)hipFree(meta_dev);
-    if (meta_host) (void)hipHostFree(meta_host);
+    io.drop();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);

@@ -39,6 +39,7 @@
 #include "optional_scratch.h"
 #include "row_tiles.h"
 #include "seq_state.h"
+#include "step_io.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -164,15 +165,14 @@ struct Model {
   struct TileSet { int per, wide_kv, span; };
   std::vector<TileSet> tile_sets;         // one per distinct query-heads-per-kv-head value of the attention layers
   // step buffers
-  size_t cap_rows = 0, cap_want = 0, cap_meta = 0;
+  size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
   float *x = nullptr, *emb = nullptr, *xcat = nullptr, *conv32 = nullptr, *q32 = nullptr, *o32 = nullptr;
   void *hb = nullptr, *proj = nullptr, *mix = nullptr, *mixr = nullptr, *y1 = nullptr, *y2 = nullptr, *y3 = nullptr, *act = nullptr;
   float *xw = nullptr, *hw = nullptr, *logits32 = nullptr;
   Half* logits16 = nullptr;
-  int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
-  uint8_t *meta_host = nullptr, *meta_dev = nullptr;
+  pst::StepIo io;
   uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
@@ -744,8 +744,9 @@ struct Model {
     while (c < n) c *= 2;
     auto* wo = &want_owned;
     if (dalloc(&xw, c * D, wo) || dalloc(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) ||
-        dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
+        dalloc(&top1_state, c * 16, wo))
       return -1;
+    KK_HIP(io.grow_tokens(c));
     cap_want = c;
     return 0;
   }
@@ -843,20 +844,12 @@ struct Model {
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
     const size_t o_pages = words;
     words += total_pages;
-    if (words > cap_meta) {
+    if (words > io.words()) {
       KK_HIP(hipStreamSynchronize(stream));
-      if (meta_host) (void)hipHostFree(meta_host);
-      if (meta_dev) (void)hipFree(meta_dev);
-      meta_host = meta_dev = nullptr;
-      cap_meta = 0;
-      size_t c = 4096;
-      while (c < words) c *= 2;
-      KK_HIP(hipHostMalloc(reinterpret_cast<void**>(&meta_host), c * 4, hipHostMallocDefault));
-      KK_HIP(hipMalloc(reinterpret_cast<void**>(&meta_dev), c * 4));
-      cap_meta = c;
       drop_graphs();
+      KK_HIP(io.grow(words));
     }
-    int32_t* mh = reinterpret_cast<int32_t*>(meta_host);
+    int32_t* mh = io.host();
     {
       size_t t = 0, pg = 0;
       for (int i = 0; i < n; ++i) {
@@ -878,8 +871,9 @@ struct Model {
       for (int k = 0; k < 4; ++k) std::copy(chunk_cols[k]->begin(), chunk_cols[k]->end(), mh + chunk_off[k]);
     }
     KK_HIP(hipEventRecord(ev0, stream));
-    KK_HIP(hipMemcpyAsync(meta_dev, meta_host, words * 4, hipMemcpyHostToDevice, stream));
-    const int32_t* md = reinterpret_cast<const int32_t*>(meta_dev);
+    const bool captured = single && graphs_on && !tap_on;
+    KK_HIP(io.send(words, captured, stream));
+    const int32_t* md = io.dev();
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
     const int32_t *d_pos = md + o_pos, *d_ent = md + o_ent, *d_row0 = md + o_row0, *d_slot = md + o_slot, *d_ind = md + o_ind,
                   *d_want = md + o_want, *d_pages = md + o_pages;
@@ -1015,13 +1009,13 @@ struct Model {
       KK_K(pegainfer_terms_rms_add(xw, nullptr, 0, nullptr, final_norm, eps, hw, PEGAINFER_DTYPE_F32, D, W, dtype, S()));
       if (linear_strided(embed, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
       KK_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, logit_cap, V, W, top1_state,
-                                   out_tokens ? tokens_d : nullptr, S()));
+                                   out_tokens ? io.tokens() : nullptr, S()));
     }
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
-    if (single && graphs_on && !tap_on) {
+    if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
@@ -1029,7 +1023,7 @@ struct Model {
       if (!exec) {
         hipGraph_t g = nullptr;
         KK_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = run_layers();
+        const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
         const hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
@@ -1044,8 +1038,8 @@ struct Model {
     last_rows = W;
     KK_HIP(hipEventRecord(ev1, stream));
     if (W > 0 && out_logits) KK_HIP(hipMemcpyAsync(out_logits, logits32, (size_t)W * V * 4, hipMemcpyDeviceToHost, stream));
-    if (W > 0 && out_tokens) KK_HIP(hipMemcpyAsync(out_tokens, tokens_d, (size_t)W * 4, hipMemcpyDeviceToHost, stream));
     KK_HIP(hipStreamSynchronize(stream));
+    if (W > 0 && out_tokens) std::memcpy(out_tokens, io.tokens(), (size_t)W * 4);
     (void)hipEventElapsedTime(&last_step_ms, ev0, ev1);
     for (int i = 0; i < n; ++i) requests[ids[i]].seq_len += lens[i];
     return 0;
@@ -1091,8 +1085,7 @@ struct Model {
     free_all(&want_owned);
     if (tap) (void)hipFree(tap);
     chunk_ws.drop([&](float* p) { free_scratch(p); });
-    if (meta_dev) (void)hipFree(meta_dev);
-    if (meta_host) (void)hipHostFree(meta_host);
+    io.drop();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);

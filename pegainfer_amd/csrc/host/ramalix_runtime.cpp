@@ -37,6 +37,7 @@
 #include "kv_pool.h"
 #include "row_tiles.h"
 #include "seq_state.h"
+#include "step_io.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -147,7 +148,7 @@ struct Model {
   float* state = nullptr;
   std::vector<int> tile_sets;   // distinct query-heads-per-kv-head values of the attention layers
   // step buffers
-  size_t cap_rows = 0, cap_want = 0, cap_meta = 0;
+  size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
   float *x = nullptr, *emb = nullptr, *n32 = nullptr, *qkv32 = nullptr, *q32 = nullptr, *o32 = nullptr, *a32 = nullptr,
         *gates32 = nullptr, *ypairs = nullptr, *route_w = nullptr, *route_logits = nullptr;
@@ -157,9 +158,8 @@ struct Model {
   int max_tiles = 0;
   float *xw = nullptr, *hw = nullptr, *logits32 = nullptr;
   Half* logits16 = nullptr;
-  int32_t* tokens_d = nullptr;
   uint8_t* top1_state = nullptr;
-  uint8_t *meta_host = nullptr, *meta_dev = nullptr;
+  pst::StepIo io;
   uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
@@ -747,8 +747,9 @@ struct Model {
     while (c < n) c *= 2;
     auto* wo = &want_owned;
     if (dalloc(&xw, c * D, wo) || dalloc(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) ||
-        dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo))
+        dalloc(&top1_state, c * 16, wo))
       return -1;
+    RX_HIP(io.grow_tokens(c));
     cap_want = c;
     return 0;
   }
@@ -850,20 +851,12 @@ struct Model {
     }
     const size_t o_pages = words;
     words += total_pages;
-    if (words > cap_meta) {
+    if (words > io.words()) {
       RX_HIP(hipStreamSynchronize(stream));
-      if (meta_host) (void)hipHostFree(meta_host);
-      if (meta_dev) (void)hipFree(meta_dev);
-      meta_host = meta_dev = nullptr;
-      cap_meta = 0;
-      size_t c = 4096;
-      while (c < words) c *= 2;
-      RX_HIP(hipHostMalloc(reinterpret_cast<void**>(&meta_host), c * 4, hipHostMallocDefault));
-      RX_HIP(hipMalloc(reinterpret_cast<void**>(&meta_dev), c * 4));
-      cap_meta = c;
       drop_graphs();
+      RX_HIP(io.grow(words));
     }
-    int32_t* mh = reinterpret_cast<int32_t*>(meta_host);
+    int32_t* mh = io.host();
     {
       size_t t = 0, pg = 0;
       for (int i = 0; i < n; ++i) {
@@ -902,8 +895,9 @@ struct Model {
       }
     }
     RX_HIP(hipEventRecord(ev0, stream));
-    RX_HIP(hipMemcpyAsync(meta_dev, meta_host, words * 4, hipMemcpyHostToDevice, stream));
-    const int32_t* md = reinterpret_cast<const int32_t*>(meta_dev);
+    const bool captured = single && graphs_on && !tap_on;
+    RX_HIP(io.send(words, captured, stream));
+    const int32_t* md = io.dev();
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
     const int32_t *d_pos = md + o_pos, *d_ent = md + o_ent, *d_row0 = md + o_row0, *d_slot = md + o_slot, *d_ind = md + o_ind,
                   *d_want = md + o_want, *d_pages = md + o_pages;
@@ -1018,13 +1012,13 @@ struct Model {
       RX_K(pegainfer_scalar_rms_add(xw, nullptr, dtype, nullptr, 0.f, nullptr, nullptr, nullptr, final_norm, eps, hw, D, W, dtype, S()));
       if (linear_strided(head, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
       RX_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, logit_scale, 0.f, V, W, top1_state,
-                                   out_tokens ? tokens_d : nullptr, S()));
+                                   out_tokens ? io.tokens() : nullptr, S()));
     }
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
-    if (single && graphs_on && !tap_on) {
+    if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
@@ -1032,7 +1026,7 @@ struct Model {
       if (!exec) {
         hipGraph_t g = nullptr;
         RX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = run_layers();
+        const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
         const hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
@@ -1047,8 +1041,8 @@ struct Model {
     last_rows = W;
     RX_HIP(hipEventRecord(ev1, stream));
     if (W > 0 && out_logits) RX_HIP(hipMemcpyAsync(out_logits, logits32, (size_t)W * V * 4, hipMemcpyDeviceToHost, stream));
-    if (W > 0 && out_tokens) RX_HIP(hipMemcpyAsync(out_tokens, tokens_d, (size_t)W * 4, hipMemcpyDeviceToHost, stream));
     RX_HIP(hipStreamSynchronize(stream));
+    if (W > 0 && out_tokens) std::memcpy(out_tokens, io.tokens(), (size_t)W * 4);
     (void)hipEventElapsedTime(&last_step_ms, ev0, ev1);
     for (int i = 0; i < n; ++i) requests[ids[i]].seq_len += lens[i];
     return 0;
@@ -1137,8 +1131,7 @@ struct Model {
     free_all(&step_owned);
     free_all(&want_owned);
     if (tap) (void)hipFree(tap);
-    if (meta_dev) (void)hipFree(meta_dev);
-    if (meta_host) (void)hipHostFree(meta_host);
+    io.drop();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);

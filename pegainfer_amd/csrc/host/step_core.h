@@ -28,6 +28,7 @@
 #include "kv_pool.h"
 #include "row_tiles.h"
 #include "seq_state.h"
+#include "step_io.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_blocks.h"
@@ -128,8 +129,7 @@ class StepModel {
     free_all(&step_owned);
     free_all(&want_owned);
     if (tap) (void)hipFree(tap);
-    if (meta_dev) (void)hipFree(meta_dev);
-    if (meta_host) (void)hipHostFree(meta_host);
+    io.drop();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -335,10 +335,11 @@ class StepModel {
     const size_t o_pages = mb.size();
     for (int i = 0; i < n; ++i) mb.insert(mb.end(), requests[ids[i]].pages.begin(), requests[ids[i]].pages.end());
     if (ensure_meta(mb.size())) return -1;
-    std::memcpy(meta_host, mb.data(), mb.size() * 4);
+    std::memcpy(io.host(), mb.data(), mb.size() * 4);
+    const bool captured = c.single && graphs_on && !tap_on;
     PSTEP_HIP(hipEventRecord(ev0, stream));
-    PSTEP_HIP(hipMemcpyAsync(meta_dev, meta_host, mb.size() * 4, hipMemcpyHostToDevice, stream));
-    const int32_t* md = reinterpret_cast<const int32_t*>(meta_dev);
+    PSTEP_HIP(io.send(mb.size(), captured, stream));
+    const int32_t* md = io.dev();
     c.tokens = reinterpret_cast<const uint32_t*>(md + o_tok);
     c.prev = md + o_prev; c.pos = md + o_pos; c.entry = md + o_ent; c.row0 = md + o_row0; c.slot = md + o_slot; c.page_indptr = md + o_ind;
     c.want = md + o_want; c.pages = md + o_pages;
@@ -353,13 +354,13 @@ class StepModel {
     auto launches = [&]() -> int {
       if (run_step(c)) return -1;
       if (W > 0)
-        PSTEP_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? tokens_d : nullptr,
+        PSTEP_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr,
                                         S()));
       return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
-    if (c.single && graphs_on && !tap_on) {
+    if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
@@ -367,7 +368,7 @@ class StepModel {
       if (!exec) {
         hipGraph_t g = nullptr;
         PSTEP_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = launches();
+        const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : launches();
         const hipError_t e = hipStreamEndCapture(stream, &g);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
@@ -382,8 +383,8 @@ class StepModel {
     last_rows = W;
     PSTEP_HIP(hipEventRecord(ev1, stream));
     if (W > 0 && out_logits) PSTEP_HIP(hipMemcpyAsync(out_logits, logits32, (size_t)W * V * 4, hipMemcpyDeviceToHost, stream));
-    if (W > 0 && out_tokens) PSTEP_HIP(hipMemcpyAsync(out_tokens, tokens_d, (size_t)W * 4, hipMemcpyDeviceToHost, stream));
     PSTEP_HIP(hipStreamSynchronize(stream));
+    if (W > 0 && out_tokens) std::memcpy(out_tokens, io.tokens(), (size_t)W * 4);
     (void)hipEventElapsedTime(&last_step_ms, ev0, ev1);
     for (int i = 0, t = 0; i < n; ++i) {
       t += lens[i];
@@ -614,11 +615,11 @@ class StepModel {
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;   // captured decode steps, one per shape
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool blas = false;
-  size_t cap_rows = 0, cap_want = 0, cap_meta = 0, tap_cap = 0;
+  size_t cap_rows = 0, cap_want = 0, tap_cap = 0;
   std::vector<int32_t> meta;
-  uint8_t *meta_host = nullptr, *meta_dev = nullptr;
+  pst::StepIo io;
   Half *logits16 = nullptr, *top1_value = nullptr;
-  int32_t *tokens_d = nullptr, *sample_out_d = nullptr;
+  int32_t* sample_out_d = nullptr;
   uint8_t *top1_state = nullptr, *row_states = nullptr, *valid_scratch = nullptr;
   float* tap = nullptr;
   uint8_t* sample_scratch = nullptr;
@@ -654,25 +655,18 @@ class StepModel {
     size_t c = 16;
     while (c < n) c *= 2;
     auto* wo = &want_owned;
-    if (dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) || dalloc(&tokens_d, c, wo) || dalloc(&top1_state, c * 16, wo) ||
+    if (dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) || dalloc(&top1_state, c * 16, wo) ||
         grow_want(c))
       return -1;
+    PSTEP_HIP(io.grow_tokens(c));
     cap_want = c;
     return 0;
   }
   int ensure_meta(size_t words) {
-    if (words <= cap_meta) return 0;
+    if (words <= io.words()) return 0;
     PSTEP_HIP(hipStreamSynchronize(stream));
     drop_graphs();
-    if (meta_host) (void)hipHostFree(meta_host);
-    if (meta_dev) (void)hipFree(meta_dev);
-    meta_host = meta_dev = nullptr;
-    cap_meta = 0;
-    size_t c = 4096;
-    while (c < words) c *= 2;
-    PSTEP_HIP(hipHostMalloc(reinterpret_cast<void**>(&meta_host), c * 4, hipHostMallocDefault));
-    PSTEP_HIP(hipMalloc(reinterpret_cast<void**>(&meta_dev), c * 4));
-    cap_meta = c;
+    PSTEP_HIP(io.grow(words));
     return 0;
   }
   int ensure_tap(size_t T) {

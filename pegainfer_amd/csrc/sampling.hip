@@ -120,7 +120,8 @@ __device__ __forceinline__ void top1_meet(unsigned long long* st, unsigned long 
   if (top1_publish(st, best) != gridDim.x - 1) return;
   const unsigned long long win = __hip_atomic_exchange(&st[0], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(&st[1], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  *out = (int)(0xFFFFFFFFu - (uint32_t)(win & 0xFFFFFFFFu));
+  // the token may go to pinned host memory
+  __hip_atomic_store(out, (int)(0xFFFFFFFFu - (uint32_t)(win & 0xFFFFFFFFu)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // Batched greedy: grid (workgroups of a row, rows); row r uses state words [2r, 2r+1] (self-resetting).
 __global__ __launch_bounds__(256) void batched_top1_kernel(const Half* __restrict__ logits, long row_stride,

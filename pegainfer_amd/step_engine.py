@@ -106,7 +106,7 @@ class StepEngine:
         else:
             w = np.ascontiguousarray(want, dtype=np.int32)
             n_want, wp, rows = int(w.size), (w.ctypes.data if w.size else None), int(w.size)
-        lg = np.zeros((rows, self.vocab), dtype=np.float32) if logits and rows else None
+        lg = np.empty((rows, self.vocab), dtype=np.float32) if logits and rows else None
         tk = np.zeros(rows, dtype=np.int32) if tokens and rows else None
         self._chk(self._fn('step')(self.h, len(entries), ids.ctypes.data, lens.ctypes.data, toks.ctypes.data,
                                                   n_want, wp, lg.ctypes.data if lg is not None else None,
