@@ -83,6 +83,23 @@ typedef struct {
   int32_t plain;             /* != 0: always the fp32-FMA tile kernel (exact products of the stored values) */
 } pegainfer_gemm_desc;
 pegainfer_status_t pegainfer_gemm_strided(const pegainfer_gemm_desc* d, pegainfer_stream_t stream);
+/* The grouped form for the experts of few rows (tile_rows_cap or max_tile_rows <= 16, bf16 x and w in 16-byte chunks; anything else is refused), with
+ *   glu     y[p, m] = act(gate row m) (up row m) of a group that holds 2 m weight rows, gates first: SILU g sigmoid(g) u, CLAMP
+ *           g sigmoid(alpha g) (u + 1) with g = min(g, limit), u = clamp(u, -limit, limit); sums and activation in fp32
+ *   shared  an expert that all shared_rows rows take, in shared_groups slices of m outputs (or k inputs): slice j's weight rows start at
+ *           shared_w + j * shared_group_stride and lie shared_m_stride apart, an up row shared_up behind its gate row.  Its positions are
+ *           shared_pos0 + j * shared_rows + row: y rows by position, x row = row where x_row_index is given, else by position. */
+enum { PEGAINFER_GLU_NONE = 0, PEGAINFER_GLU_SILU = 1, PEGAINFER_GLU_CLAMP = 2 };
+typedef struct {
+  pegainfer_gemm_desc g;
+  int32_t glu;
+  float limit, alpha;
+  const void* shared_w;      /* NULL: none */
+  int32_t shared_groups, shared_rows, shared_pos0;
+  float shared_limit;
+  int64_t shared_m_stride, shared_group_stride, shared_up;
+} pegainfer_expert_rows_desc;
+pegainfer_status_t pegainfer_expert_rows(const pegainfer_expert_rows_desc* q, pegainfer_stream_t stream);
 
 /* ---- attention over a paged latent cache ----
  * Cache: page-first; one layer's entry of one token = [c: rank values | kr: rot values], at
@@ -290,6 +307,11 @@ pegainfer_status_t pegainfer_route_combine_gated(const float* y_pairs, const flo
                                                  const float* add_gate, int64_t add_gate_stride, void* out, int32_t d,
                                                  int32_t top, int32_t rows, int32_t dtype, pegainfer_stream_t stream);
 
+/* pegainfer_route_combine_gated whose added row is the sum of n_add fp32 rows, add_pairs[(j * rows + row) * d ..], j < n_add */
+pegainfer_status_t pegainfer_route_combine_pairs(const float* y_pairs, const float* weight, const float* add_pairs, int32_t n_add,
+                                                 const float* add_gate, int64_t add_gate_stride, void* out, int32_t d, int32_t top,
+                                                 int32_t rows, int32_t dtype, pegainfer_stream_t stream);
+
 /* pegainfer_route_combine_gated in which a pair whose expert[row * top + c] is same_from or more takes the row of `same` ([rows, d] of
  * dtype at same_stride; NULL = no such pairs) instead of its y_pairs row: identity experts */
 pegainfer_status_t pegainfer_route_combine_same(const float* y_pairs, const float* weight, const int32_t* expert, int32_t same_from,
@@ -373,6 +395,8 @@ typedef struct {
   int32_t d, rows, dtype;
 } pegainfer_join_rms_desc;
 pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfer_stream_t stream);
+/* with y_pairs: `add` is the sum of n_add fp32 rows, add_pairs[(j * rows + row) * d ..], j < n_add (q->add NULL) */
+pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream);
 /* out[row, i] = act(gate[row, i]) * up[row, i], i < I; gate and up are column ranges of rows with stride in_row_stride (elements of
  * dtype).  act 0 = silu, 1 = relu, 2 = gelu (tanh form), 3 = gelu (exact form) */
 enum { PEGAINFER_ACT_SILU = 0, PEGAINFER_ACT_RELU = 1, PEGAINFER_ACT_GELU_TANH = 2, PEGAINFER_ACT_GELU_ERF = 3 };

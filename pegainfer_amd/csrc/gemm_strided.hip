@@ -492,13 +492,36 @@ struct RowPiece<float> {
 
 constexpr int kRowsMax = 16;   // token rows of a tile of the matrix-core few-rows form
 
-template <typename TX, typename TY, typename TG, int OB>
-__global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc d, int wk) {
+// What the experts of few rows do beyond the grouped product (EX; pegainfer_expert_rows): a gated activation of two weight rows per output, and
+// the slices of an expert that every row takes as further groups, behind the table's `slots` workgroup columns.
+// In a decode step each launch costs some 4 us whatever it does: 8 rows, 16 experts of 2 x 512 x 1024 and a shared one of twice their size took
+// 9.6 + 4.5 (activation) + 7.0 us and 5.0 + 4.2 for the shared one, here 9.6 + 6.4; 32 experts of 1024 x 2048 and a shared one of 2048
+// 16.2 + 14.5 and 14.0 in three launches, here 16.9 + 15.4; one row, 4 of 32 experts of 2 x 1024 x 2560 13.2 + 4.6 + 8.4 and 15.4, here 14.4 + 9.0.
+struct ExpertForm {
+  int glu, slots, rows, pos0;
+  float limit, alpha, shared_limit;
+  const uint16_t* w;
+  int64_t m_stride, group_stride, up;      // the shared expert's: of a weight row, of a slice, from a gate row to its up row
+};
+__device__ __forceinline__ float glu_f(const ExpertForm& ex, bool shared, float g, float u) {
+  if (ex.glu == PEGAINFER_GLU_SILU) return g * sigmoid_f(g) * u;
+  const float limit = shared ? ex.shared_limit : ex.limit;
+  g = fminf(g, limit);
+  return g * sigmoid_f(ex.alpha * g) * (fminf(fmaxf(u, -limit), limit) + 1.0f);
+}
+
+template <typename TX, typename TY, typename TG, int OB, bool EX = false>
+__global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc d, int wk, ExpertForm ex) {
   constexpr int CH = OB == 1 && sizeof(TX) == 2 ? 4 : 2;      // 64-wide pieces per register set
   constexpr int NP = RowPiece<TX>::kParts;
   __shared__ f32x4 red[4][OB][64];
   int g, row0, nrows;
-  if (d.tile_group) {
+  const bool shared = EX && (int)blockIdx.x >= ex.slots;
+  if (shared) {
+    g = blockIdx.x - ex.slots;
+    row0 = ex.pos0 + g * ex.rows;
+    nrows = ex.rows;
+  } else if (d.tile_group) {
     if ((int)blockIdx.x >= *d.n_tiles) return;
     g = d.tile_group[blockIdx.x];
     row0 = d.tile_row0[blockIdx.x];
@@ -510,20 +533,25 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
   }
   if (nrows <= 0) return;                                     // an empty tile of a table has no last row to repeat
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
-  const int per_wg = 4 / wk * OB * 16;                        // outputs of a workgroup
+  const bool glu = EX && OB == 2 && ex.glu;                   // block 0 holds gate rows, block 1 their up rows
+  const int per_blk = glu ? 16 : OB * 16, per_wg = 4 / wk * per_blk;      // outputs of a wave's share, of a workgroup
   const int blk = wave / wk, ks = wave - blk * wk;
-  const int m0 = blockIdx.y * per_wg + blk * OB * 16;
-  const TX* X = static_cast<const TX*>(d.x) + (int64_t)g * d.x_group_stride;
-  const uint16_t* W = static_cast<const uint16_t*>(d.w) + (int64_t)g * d.w_group_stride;
+  const int m0 = blockIdx.y * per_wg + blk * per_blk;
+  // rows of position p: a shared slice's positions are the step's rows in order
+  auto x_row = [&](int p) { return d.x_row_index ? (shared ? p - row0 : d.x_row_index[p]) : p; };
+  auto y_row = [&](int p) { return d.y_row_index && !shared ? d.y_row_index[p] : p; };
+  const TX* X = static_cast<const TX*>(d.x) + (shared ? 0 : (int64_t)g * d.x_group_stride);
+  const uint16_t* W = shared ? ex.w + g * ex.group_stride : static_cast<const uint16_t*>(d.w) + (int64_t)g * d.w_group_stride;
+  const int64_t wm = shared ? ex.m_stride : d.w_m_stride, up = shared ? ex.up : (int64_t)d.m * d.w_m_stride;
   const int tok = row0 + min(l15, nrows - 1);                 // absent rows repeat the last one; they are never stored
-  const TX* xp = X + (int64_t)(d.x_row_index ? d.x_row_index[tok] : tok) * d.x_row_stride + gq * 16;
+  const TX* xp = X + (int64_t)x_row(tok) * d.x_row_stride + gq * 16;
   const int pchunk = 2 * gq + (lane & 1);
   const uint16_t* wp[OB][2];
 #pragma unroll
   for (int o = 0; o < OB; ++o)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      wp[o][h] = W + (int64_t)min(m0 + o * 16 + h * 8 + ((lane >> 1) & 7), d.m - 1) * d.w_m_stride + pchunk * 8;
+      wp[o][h] = W + (int64_t)min(m0 + (glu ? 0 : o * 16) + h * 8 + ((lane >> 1) & 7), d.m - 1) * wm + (glu && o ? up : 0) + pchunk * 8;
   const int K = d.k, np = (K + 63) >> 6, mine = ks < np ? (np - ks + wk - 1) / wk : 0;   // pieces of k; those of this wave
   f32x4 acc[OB][2][2];
 #pragma unroll
@@ -590,13 +618,13 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
     red[wave][o][lane] = f32x4{acc[o][0][0][0] + acc[o][0][1][1], acc[o][0][0][2] + acc[o][0][1][3],
                                acc[o][1][0][0] + acc[o][1][1][1], acc[o][1][0][2] + acc[o][1][1][3]};
   __syncthreads();
-  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
+  TY* Y = static_cast<TY*>(d.y) + (shared ? 0 : (int64_t)g * d.y_group_stride);
   const float* part = reinterpret_cast<const float*>(red);
   for (int e = tid; e < per_wg * 16; e += 256) {              // consecutive threads: consecutive outputs of one row
     const int out = e % per_wg, r = e / per_wg;
     const int m = blockIdx.y * per_wg + out;
     if (r >= nrows || m >= d.m) continue;
-    const int b = out / (OB * 16), o = (out >> 4) % OB, j = out & 15;
+    const int b = out / per_blk, o = glu ? 0 : (out >> 4) % OB, j = out & 15;
     const int at = (o * 64 + ((j & 7) >> 1) * 16 + r) * 4 + (j >> 3) * 2 + (j & 1);
     float v = part[b * wk * OB * 256 + at];
     for (int w = 1; w < wk; ++w) v += part[(b * wk + w) * OB * 256 + at];
@@ -605,17 +633,21 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
       // a cut-off part of zero times an infinite weight is no number where the value's own product is an infinity: summed again from whole
       // values, up to the first that settles it
       if (v != v) {
-        const TX* xr = X + (int64_t)(d.x_row_index ? d.x_row_index[p] : p) * d.x_row_stride;
+        const TX* xr = X + (int64_t)x_row(p) * d.x_row_stride;
         const uint16_t* wr = W + (int64_t)m * d.w_m_stride;
         v = 0.f;
         for (int k = 0; k < K && v == v; ++k) v = fmaf(ld(xr + k), ld(wr + k), v);
       }
     }
-    if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+    if (glu) {
+      float u = part[b * wk * OB * 256 + at + 256];
+      for (int w = 1; w < wk; ++w) u += part[(b * wk + w) * OB * 256 + at + 256];
+      v = glu_f(ex, shared, v, u);
+    } else if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
     else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
     else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
-      v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)(d.x_row_index ? d.x_row_index[p] : p) * d.gate_row_stride + g));
-    st(Y + (int64_t)(d.y_row_index ? d.y_row_index[p] : p) * d.y_row_stride + m, v);
+      v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)x_row(p) * d.gate_row_stride + g));
+    st(Y + (int64_t)y_row(p) * d.y_row_stride + m, v);
   }
 }
 
@@ -628,8 +660,18 @@ static void rows_mfma_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   const int blocks = ceil_div(d.m, 16 * (4 / wk));
   // two blocks of outputs per wave (each x piece used twice) where that still gives every compute unit two workgroups
   const bool two = (long)row_tiles * groups * blocks >= 4L * device_cus();
-  if (two) gemm_rows_mfma_kernel<TX, TY, TG, 2><<<dim3(row_tiles, ceil_div(blocks, 2), groups), 256, 0, s>>>(d, wk);
-  else gemm_rows_mfma_kernel<TX, TY, TG, 1><<<dim3(row_tiles, blocks, groups), 256, 0, s>>>(d, wk);
+  if (two) gemm_rows_mfma_kernel<TX, TY, TG, 2><<<dim3(row_tiles, ceil_div(blocks, 2), groups), 256, 0, s>>>(d, wk, ExpertForm{});
+  else gemm_rows_mfma_kernel<TX, TY, TG, 1><<<dim3(row_tiles, blocks, groups), 256, 0, s>>>(d, wk, ExpertForm{});
+}
+template <typename TY>
+static void expert_rows_launch(const pegainfer_gemm_desc& d, ExpertForm ex, int slices, hipStream_t s) {
+  const int np = ceil_div(d.k, 64), wk = np >= 8 ? 4 : np >= 4 ? 2 : 1;
+  const int columns = (d.max_tiles + slices) | 1;      // odd, as above; the shared slices last
+  ex.slots = columns - slices;
+  const int blocks = ceil_div(d.m, 16 * (4 / wk));
+  if (ex.glu) gemm_rows_mfma_kernel<uint16_t, TY, uint16_t, 2, true><<<dim3(columns, blocks), 256, 0, s>>>(d, wk, ex);
+  else if ((long)columns * blocks >= 4L * device_cus()) gemm_rows_mfma_kernel<uint16_t, TY, uint16_t, 2, true><<<dim3(columns, ceil_div(blocks, 2)), 256, 0, s>>>(d, wk, ex);
+  else gemm_rows_mfma_kernel<uint16_t, TY, uint16_t, 1, true><<<dim3(columns, blocks), 256, 0, s>>>(d, wk, ex);
 }
 
 // ------------------------------------------------------------------ few-rows form on the matrix cores (fp32 weights, decode)
@@ -935,5 +977,26 @@ extern "C" pegainfer_status_t pegainfer_gemm_strided(const pegainfer_gemm_desc* 
     default: break;
   }
   if (!ok) return (pegainfer_status_t)hipErrorInvalidValue;
+  return (pegainfer_status_t)hipGetLastError();
+}
+
+extern "C" pegainfer_status_t pegainfer_expert_rows(const pegainfer_expert_rows_desc* q, pegainfer_stream_t stream) {
+  using namespace pk;
+  constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
+  if (!q) return bad;
+  const pegainfer_gemm_desc& d = q->g;
+  const int slices = q->shared_w ? q->shared_groups : 0;
+  if (d.m <= 0 || d.k <= 0 || d.max_tiles <= 0) return 0;
+  const int rows = d.max_tile_rows > 0 ? d.max_tile_rows : d.tile_rows_cap;
+  if (!d.tile_group || !d.tile_row0 || !d.tile_rows || !d.n_tiles || d.plain || d.x_dtype != kDtBf16 || d.w_dtype != kDtBf16 ||
+      (d.y_dtype != kDtBf16 && d.y_dtype != kDtF32) || rows < 1 || rows > kRowsMax || !chunks_ok(d) || d.epilogue == PEGAINFER_EPI_SIGMOID_GATE ||
+      q->glu < PEGAINFER_GLU_NONE || q->glu > PEGAINFER_GLU_CLAMP || (q->glu && d.epilogue) || slices < 0 ||
+      (slices && (q->shared_rows < 1 || q->shared_rows > kRowsMax || q->shared_pos0 < 0 || (q->shared_m_stride & 7) || (q->shared_group_stride & 7) ||
+                  (q->shared_up & 7) || (reinterpret_cast<uintptr_t>(q->shared_w) & 15u))))
+    return bad;
+  const ExpertForm ex{q->glu, 0, q->shared_rows, q->shared_pos0, q->limit, q->alpha, q->shared_limit, static_cast<const uint16_t*>(q->shared_w),
+                      q->shared_m_stride, q->shared_group_stride, q->shared_up};
+  if (d.y_dtype == kDtF32) expert_rows_launch<float>(d, ex, slices, as_stream(stream));
+  else expert_rows_launch<uint16_t>(d, ex, slices, as_stream(stream));
   return (pegainfer_status_t)hipGetLastError();
 }

@@ -802,7 +802,8 @@ struct Model {
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     DZ_K(pegainfer_route_sigmoid_grouped(h, w.router, w.corr, route_e, route_w, D, f.experts, f.groups, f.keep, f.top, T, dtype, S()));
     // few rows: tiles of the step's rows; otherwise 128-row tiles for the matrix-core form of bf16 weights, 64-row tiles
-    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0);
+    const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0;
+    const int per_tile = ptiles::expert_tile_rows(T, wide);
     DZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
     pegainfer_gemm_desc d{};
     d.x = h; d.w = w.gate_up_e; d.y = gu;
@@ -815,8 +816,16 @@ struct Model {
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
     d.plain = plain_kernels;
-    DZ_K(pegainfer_gemm_strided(&d, S()));
-    DZ_K(pegainfer_silu_mul_rows(gu, act, f.ff, P, dtype, S()));
+    if (wide && T <= ptiles::kFewRows) {
+      pegainfer_expert_rows_desc x{};      // the activation in the product's launch
+      x.g = d;
+      x.g.y = act; x.g.m = f.ff; x.g.y_row_stride = f.ff;
+      x.glu = PEGAINFER_GLU_SILU;
+      DZ_K(pegainfer_expert_rows(&x, S()));
+    } else {
+      DZ_K(pegainfer_gemm_strided(&d, S()));
+      DZ_K(pegainfer_silu_mul_rows(gu, act, f.ff, P, dtype, S()));
+    }
     pegainfer_gemm_desc e{};
     e.x = act; e.w = w.down_e; e.y = ypairs;
     e.x_dtype = e.w_dtype = dtype; e.y_dtype = PEGAINFER_DTYPE_F32;

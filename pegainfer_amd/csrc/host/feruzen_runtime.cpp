@@ -168,7 +168,7 @@ struct Model {
   float* tap = nullptr;
   size_t tap_cap = 0;
   int tap_rows = 0;
-  int mx_proj = 0, mx_mix = 0, mx_conv = 0, mx_q = 0, mx_o = 0, mx_ff = 0, mx_top = 0, mx_gu_e = 0, mx_experts = 0;
+  int mx_proj = 0, mx_mix = 0, mx_conv = 0, mx_q = 0, mx_o = 0, mx_ff = 0, mx_top = 0, mx_gu_e = 0, mx_experts = 0, mx_slices = 0, mx_sff = 0;
 
   struct GraphKey {
     int n, want; bool tokens, plain; int split;
@@ -344,7 +344,11 @@ struct Model {
         mx_top = std::max(mx_top, c.mlp.top);
         mx_gu_e = std::max(mx_gu_e, c.mlp.top * 2 * c.mlp.glu.ff);
         mx_experts = std::max(mx_experts, c.mlp.experts);
-        if (c.mlp.has_shared) mx_ff = std::max(mx_ff, c.mlp.shared.ff);
+        if (c.mlp.has_shared) {
+          mx_ff = std::max(mx_ff, c.mlp.shared.ff);
+          mx_sff = std::max(mx_sff, c.mlp.shared.ff);
+          mx_slices = std::max(mx_slices, ptiles::shared_slices(1, true, c.mlp.shared.ff, c.mlp.glu.ff));
+        }
       }
     }
     return 0;
@@ -668,9 +672,9 @@ struct Model {
         dalloc_a(&ys, n * D, so) || dalloc_a(&q16, n * (size_t)std::max(1, mx_q), so) ||
         dalloc_a(&attn16, n * (size_t)std::max(1, mx_q), so))
       return -1;
-    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)std::max(1, mx_experts), so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
+    if (mx_top > 0 && (dalloc(&ypairs, (P + ptiles::kFewRows * (size_t)mx_slices) * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)std::max(1, mx_experts), so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
                        dalloc(&pos_row, P, so) || dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu_e, n * mx_gu_e, so) ||
-                       dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2), so)))
+                       dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2) + ptiles::kFewRows * (size_t)mx_sff, so)))
       return -1;
     cap_rows = n;
     return 0;
@@ -1070,7 +1074,8 @@ struct Model {
     const MlpCfg& f = c.mlp;
     const int ff = f.glu.ff, P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
-    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0);
+    const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0;
+    const int per_tile = ptiles::expert_tile_rows(T, wide), slices = f.has_shared ? ptiles::shared_slices(T, wide, f.shared.ff, ff) : 0;
     if (T > 8 || f.experts > 1024) {   // many rows (or more experts than the selection kernel's four rows hold in LDS): one
                                        // workgroup per row does logits and selection
       FZ_K(pegainfer_route_topk(xb, w.router, nullptr, route_e, route_w, D, f.experts, 1, 1, f.top, T, PEGAINFER_SCORE_SOFTMAX, dtype, S()));
@@ -1103,8 +1108,6 @@ struct Model {
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
     d.plain = plain_kernels;
-    FZ_K(pegainfer_gemm_strided(&d, S()));
-    FZ_K(pegainfer_clamp_glu_rows(gu_e, act_e, ff, P, f.glu.limit, kGluAlpha, dtype, S()));
     pegainfer_gemm_desc e{};
     e.x = act_e; e.w = w.down_e; e.y = ypairs;
     e.x_dtype = e.w_dtype = dtype; e.y_dtype = PEGAINFER_DTYPE_F32;
@@ -1115,7 +1118,28 @@ struct Model {
     e.y_row_index = pos_pair;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
-    FZ_K(pegainfer_gemm_strided(&e, S()));
+    if (wide && T <= ptiles::kFewRows) {
+      // activation and the shared expert's slices in the routed experts' two launches; the slices' rows lie behind the pairs
+      pegainfer_expert_rows_desc x{};
+      x.g = d;
+      x.g.y = act_e; x.g.m = ff; x.g.y_row_stride = ff;
+      x.glu = PEGAINFER_GLU_CLAMP; x.limit = f.glu.limit; x.alpha = kGluAlpha; x.shared_limit = f.shared.limit;
+      x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
+      x.shared_w = slices ? w.gate_up : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)ff * D; x.shared_up = (int64_t)f.shared.ff * D;
+      FZ_K(pegainfer_expert_rows(&x, S()));
+      x.g = e;
+      x.glu = PEGAINFER_GLU_NONE;
+      x.shared_w = slices ? w.down : nullptr; x.shared_m_stride = f.shared.ff; x.shared_group_stride = ff;
+      FZ_K(pegainfer_expert_rows(&x, S()));
+    } else {
+      FZ_K(pegainfer_gemm_strided(&d, S()));
+      FZ_K(pegainfer_clamp_glu_rows(gu_e, act_e, ff, P, f.glu.limit, kGluAlpha, dtype, S()));
+      FZ_K(pegainfer_gemm_strided(&e, S()));
+    }
+    if (slices) {
+      FZ_K(pegainfer_route_combine_pairs(ypairs, route_w, ypairs + (size_t)P * D, slices, nullptr, 0, y, D, f.top, T, dtype, S()));
+      return 0;
+    }
     if (f.has_shared && glu(w.gate_up, w.down, f.shared, xb, ys, T)) return -1;
     FZ_K(pegainfer_route_combine_add(ypairs, route_w, f.has_shared ? ys : nullptr, y, D, f.top, T, dtype, S()));
     return 0;

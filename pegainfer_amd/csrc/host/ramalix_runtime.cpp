@@ -172,7 +172,7 @@ struct Model {
   int tap_rows = 0;
   float* att_part = nullptr;   // softmax states of the key splits of an attention launch
   int mx_vdim = 0;
-  int mx_proj = 0, mx_mix = 0, mx_conv = 0, mx_q = 0, mx_o = 0, mx_gates = 0, mx_a = 0, mx_ff = 0, mx_top = 0, mx_gu_e = 0, mx_experts = 0;
+  int mx_proj = 0, mx_mix = 0, mx_conv = 0, mx_q = 0, mx_o = 0, mx_gates = 0, mx_a = 0, mx_ff = 0, mx_top = 0, mx_gu_e = 0, mx_experts = 0, mx_slices = 0, mx_sff = 0;
 
   struct GraphKey {
     int n, want; bool tokens, plain;
@@ -372,7 +372,11 @@ struct Model {
         mx_top = std::max(mx_top, c.mlp.top);
         mx_gu_e = std::max(mx_gu_e, c.mlp.top * 2 * c.mlp.ff);
         mx_experts = std::max(mx_experts, c.mlp.experts);
-        if (c.mlp.has_shared) mx_ff = std::max(mx_ff, c.mlp.shared_ff);
+        if (c.mlp.has_shared) {
+          mx_ff = std::max(mx_ff, c.mlp.shared_ff);
+          mx_sff = std::max(mx_sff, c.mlp.shared_ff);
+          mx_slices = std::max(mx_slices, ptiles::shared_slices(1, true, c.mlp.shared_ff, c.mlp.ff));
+        }
       }
     }
     planned = true;
@@ -729,10 +733,10 @@ struct Model {
         dalloc_a(&act, n * (size_t)std::max(1, mx_ff), so) || dalloc_a(&ys, n * D, so) ||
         dalloc(&att_part, (size_t)kSplitGroups * kAttRows * 2 * (size_t)(mx_vdim + 2), so))
       return -1;
-    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)(mx_experts + 1), so) ||
+    if (mx_top > 0 && (dalloc(&ypairs, (P + ptiles::kFewRows * (size_t)mx_slices) * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)(mx_experts + 1), so) ||
                        dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) || dalloc(&pos_row, P, so) ||
                        dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu_e, n * (size_t)mx_gu_e, so) ||
-                       dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2), so)))
+                       dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2) + ptiles::kFewRows * (size_t)mx_sff, so)))
       return -1;
     cap_rows = n;
     return 0;
@@ -1054,7 +1058,8 @@ struct Model {
     const int ff = f.ff, P = T * f.top, E1 = f.experts + 1;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     if (linear_strided(w.router, hb, dtype, D, route_logits, PEGAINFER_DTYPE_F32, E1, T, D)) return -1;
-    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0);
+    const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0;
+    const int per_tile = ptiles::expert_tile_rows(T, wide), slices = f.has_shared ? ptiles::shared_slices(T, wide, f.shared_ff, ff) : 0;
     pegainfer_route_plan_desc r{};      // selection and sort: one launch for few rows
     r.logits = route_logits; r.logits_stride = E1; r.out_expert = route_e; r.out_weight = route_w;
     r.experts = f.experts; r.n_groups = f.groups; r.keep_groups = f.keep; r.top = f.top; r.rows = T;
@@ -1074,8 +1079,6 @@ struct Model {
     d.tile_rows_cap = per_tile;
     d.x_row_index = pos_row;
     d.plain = plain_kernels;
-    RX_K(pegainfer_gemm_strided(&d, S()));
-    RX_K(pegainfer_silu_mul_rows(gu_e, act_e, ff, P, dtype, S()));
     pegainfer_gemm_desc e{};
     e.x = act_e; e.w = w.down_e; e.y = ypairs;
     e.x_dtype = e.w_dtype = dtype; e.y_dtype = PEGAINFER_DTYPE_F32;
@@ -1086,7 +1089,28 @@ struct Model {
     e.y_row_index = pos_pair;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
-    RX_K(pegainfer_gemm_strided(&e, S()));
+    if (wide && T <= ptiles::kFewRows) {
+      // activation and the shared expert's slices in the routed experts' two launches; the slices' rows lie behind the pairs
+      pegainfer_expert_rows_desc x{};
+      x.g = d;
+      x.g.y = act_e; x.g.m = ff; x.g.y_row_stride = ff;
+      x.glu = PEGAINFER_GLU_SILU;
+      x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
+      x.shared_w = slices ? w.gate_up : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)ff * D; x.shared_up = (int64_t)f.shared_ff * D;
+      RX_K(pegainfer_expert_rows(&x, S()));
+      x.g = e;
+      x.glu = PEGAINFER_GLU_NONE;
+      x.shared_w = slices ? w.down : nullptr; x.shared_m_stride = f.shared_ff; x.shared_group_stride = ff;
+      RX_K(pegainfer_expert_rows(&x, S()));
+    } else {
+      RX_K(pegainfer_gemm_strided(&d, S()));
+      RX_K(pegainfer_silu_mul_rows(gu_e, act_e, ff, P, dtype, S()));
+      RX_K(pegainfer_gemm_strided(&e, S()));
+    }
+    if (slices) {
+      RX_K(pegainfer_route_combine_pairs(ypairs, route_w, ypairs + (size_t)P * D, slices, route_logits + f.experts, E1, y, D, f.top, T, dtype, S()));
+      return 0;
+    }
     if (f.has_shared && swiglu(w.gate_up, w.down, f.shared_ff, hb, ys, T)) return -1;
     RX_K(pegainfer_route_combine_gated(ypairs, route_w, f.has_shared ? ys : nullptr, f.has_shared ? route_logits + f.experts : nullptr, E1, y,
                                        D, f.top, T, dtype, S()));

@@ -63,6 +63,11 @@ inline int expert_tiles(int T, int top, int experts, int per_tile) {
   return std::min(P, (P + per_tile - 1) / per_tile + experts);
 }
 
+// Slices in which an expert that every row takes joins the routed ones' launches of few rows (0: it has launches of its own)
+inline int shared_slices(int T, bool wide, int shared_ff, int ff) {
+  return wide && T <= kFewRows && shared_ff > 0 && shared_ff % ff == 0 ? shared_ff / ff : 0;
+}
+
 // the chunks of the entries of more than scan_max rows (pegainfer_decay_attention's tables)
 struct Chunks {
   std::vector<int32_t> row0, rows, first{0}, slot;     // per chunk; per long entry: its first chunk (one more at the end), its state slot

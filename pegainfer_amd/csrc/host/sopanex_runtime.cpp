@@ -170,7 +170,7 @@ class Model : public StepModel {
       m.o_a = pad8(m.o_g + m.heads * m.vdim);
       c.proj_rows = m.o_a + pad8(m.rank);
     }
-    mx_proj = mx_mix = mx_q = mx_o = mx_z = mx_route = mx_top = mx_pair_ff = mx_shared = mx_experts = 0;
+    mx_proj = mx_mix = mx_q = mx_o = mx_z = mx_route = mx_top = mx_pair_ff = mx_shared = mx_slices = mx_experts = 0;
     part_floats = 0;
     for (auto& c : layers) {
       mx_proj = std::max(mx_proj, c.proj_rows);
@@ -182,6 +182,7 @@ class Model : public StepModel {
       mx_top = std::max(mx_top, c.moe.top);
       mx_pair_ff = std::max(mx_pair_ff, c.moe.top * c.moe.ff);
       mx_shared = std::max(mx_shared, c.moe.shared_ff);
+      if (c.moe.ff > 0) mx_slices = std::max(mx_slices, ptiles::shared_slices(1, true, c.moe.shared_ff, c.moe.ff));
       mx_experts = std::max(mx_experts, c.moe.experts);
       part_floats = std::max(part_floats, (size_t)kSplitGroups * kGroupRows * (size_t)(c.left.dim + 2));
     }
@@ -292,7 +293,8 @@ class Model : public StepModel {
            dalloc_a(&y, n * D, so) || dalloc(&part, part_floats, so) || dalloc(&logits_r, n * (size_t)mx_route, so) ||
            dalloc(&route_e, n * (size_t)mx_top, so) || dalloc(&route_w, n * (size_t)mx_top, so) || dalloc(&pos_pair, n * (size_t)mx_top, so) ||
            dalloc(&pos_row, n * (size_t)mx_top, so) || dalloc(&tiles, 3 * (size_t)max_tiles + 1, so) ||
-           dalloc_a(&act_e, n * (size_t)mx_pair_ff, so) || dalloc(&y_pairs, n * (size_t)mx_top * D, so) ||
+           dalloc_a(&act_e, n * (size_t)mx_pair_ff + ptiles::kFewRows * (size_t)mx_shared, so) ||
+           dalloc(&y_pairs, (n * (size_t)mx_top + ptiles::kFewRows * (size_t)mx_slices) * D, so) ||
            dalloc_a(&act_s, n * (size_t)mx_shared, so) || dalloc_a(&y_s, n * (size_t)(mx_shared ? D : 0), so) ? -1 : 0;
   }
   int grow_want(size_t n) override { return dalloc_a(&hw, n * D, &want_owned); }
@@ -393,7 +395,8 @@ class Model : public StepModel {
     const MoeCfg& f = c.moe;
     const int T = s.T, all = f.experts + f.identity;
     if (linear_strided(w.router, h, dtype, D, logits_r, PEGAINFER_DTYPE_F32, all + 1, T, D)) return -1;
-    const int per_tile = ptiles::expert_tile_rows(T, dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0);
+    const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0;
+    const int per_tile = ptiles::expert_tile_rows(T, wide), slices = ptiles::shared_slices(T, wide, f.shared_ff, f.ff);
     pegainfer_route_plan_desc r{};
     r.logits = logits_r; r.logits_stride = all + 1; r.correction = w.correction; r.out_expert = route_e; r.out_weight = route_w;
     r.experts = all; r.n_groups = 1; r.keep_groups = 1; r.top = f.top; r.rows = T; r.score_kind = PEGAINFER_SCORE_SOFTMAX; r.renorm = 1;
@@ -414,14 +417,26 @@ class Model : public StepModel {
     u.m = f.ff; u.k = D; u.x_row_stride = D; u.w_m_stride = D; u.w_group_stride = (int64_t)f.ff * D; u.y_row_stride = f.ff;
     u.x_row_index = pos_row;
     u.epilogue = PEGAINFER_EPI_GELU_ERF;
-    PSTEP_K(pegainfer_gemm_strided(&u, S()));
     pegainfer_gemm_desc d = g;           // W_down, rows by (token, choice)
     d.x = act_e; d.w = w.down_e; d.y = y_pairs;
     d.x_dtype = d.w_dtype = dtype; d.y_dtype = PEGAINFER_DTYPE_F32;
     d.m = D; d.k = f.ff; d.x_row_stride = f.ff; d.w_m_stride = f.ff; d.w_group_stride = (int64_t)D * f.ff; d.y_row_stride = D;
     d.y_row_index = pos_pair;
-    PSTEP_K(pegainfer_gemm_strided(&d, S()));
-    if (f.shared_ff) {
+    const int P = T * f.top;
+    if (wide && T <= ptiles::kFewRows) {   // the shared expert's slices beside the routed experts, its rows behind the pairs
+      pegainfer_expert_rows_desc x{};
+      x.g = u;
+      x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
+      x.shared_w = slices ? w.up_s : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)f.ff * D;
+      PSTEP_K(pegainfer_expert_rows(&x, S()));
+      x.g = d;
+      x.shared_w = slices ? w.down_s : nullptr; x.shared_m_stride = f.shared_ff; x.shared_group_stride = f.ff;
+      PSTEP_K(pegainfer_expert_rows(&x, S()));
+    } else {
+      PSTEP_K(pegainfer_gemm_strided(&u, S()));
+      PSTEP_K(pegainfer_gemm_strided(&d, S()));
+    }
+    if (f.shared_ff && !slices) {
       if (dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && T > 1) {   // a tuned route and the activation; one row: both in one launch
         if (linear(w.up_s, h, act_s, f.shared_ff, T, D)) return -1;
         PSTEP_K(pegainfer_act_rows(act_s, f.shared_ff, act_s, f.shared_ff, f.shared_ff, T, PEGAINFER_ACT_GELU_ERF, dtype, S()));
@@ -433,8 +448,8 @@ class Model : public StepModel {
     pegainfer_join_rms_desc j = join_desc(s, w.norm2b, next);
     j.y_pairs = y_pairs; j.weight = route_w; j.expert = route_e; j.top = f.top; j.same_from = f.experts;
     if (f.identity) { j.same = h; j.same_stride = D; }
-    if (f.shared_ff) { j.add = y_s; j.add_gate = logits_r + all; j.add_gate_stride = all + 1; }
-    PSTEP_K(pegainfer_join_rms(&j, S()));
+    if (f.shared_ff) { j.add = slices ? nullptr : y_s; j.add_gate = logits_r + all; j.add_gate_stride = all + 1; }
+    PSTEP_K(pegainfer_join_rms_pairs(&j, y_pairs + (size_t)P * D, slices, S()));
     return 0;
   }
   int run_step(const StepCtx& s) override {
@@ -469,7 +484,7 @@ class Model : public StepModel {
   std::vector<LayerCfg> layers;
   std::vector<LayerW> weights;
   void *embed = nullptr, *bigram = nullptr, *head = nullptr, *final_norm = nullptr;
-  int mx_proj = 0, mx_mix = 0, mx_q = 0, mx_o = 0, mx_z = 0, mx_route = 0, mx_top = 0, mx_pair_ff = 0, mx_shared = 0, mx_experts = 0, max_tiles = 0;
+  int mx_proj = 0, mx_mix = 0, mx_q = 0, mx_o = 0, mx_z = 0, mx_route = 0, mx_top = 0, mx_pair_ff = 0, mx_shared = 0, mx_slices = 0, mx_experts = 0, max_tiles = 0;
   size_t part_floats = 0, chunk_cap = 0;
   float *x = nullptr, *q32 = nullptr, *o32 = nullptr, *z32 = nullptr, *part = nullptr, *logits_r = nullptr, *route_w = nullptr, *y_pairs = nullptr,
         *chunk_ws = nullptr;

@@ -301,11 +301,14 @@ __global__ __launch_bounds__(256) void route_combine_kernel(const float* __restr
                                                             const A* __restrict__ add, A* __restrict__ out, int d, int top,
                                                             const float* __restrict__ add_gate, int64_t add_gate_stride,
                                                             const int32_t* __restrict__ expert, int same_from,
-                                                            const A* __restrict__ same, int64_t same_stride) {
+                                                            const A* __restrict__ same, int64_t same_stride,
+                                                            const float* __restrict__ add_pairs, int n_add) {
   const int row = blockIdx.x;
-  const float gate = add && add_gate ? sigmoid_f(add_gate[(size_t)row * add_gate_stride]) : 1.0f;
+  const float gate = (add || n_add) && add_gate ? sigmoid_f(add_gate[(size_t)row * add_gate_stride]) : 1.0f;
   for (int i = blockIdx.y * 256 + threadIdx.x; i < d; i += gridDim.y * 256) {
-    float a = add ? ld(add + (size_t)row * d + i) * gate : 0.f;
+    float a = add ? ld(add + (size_t)row * d + i) : 0.f;
+    for (int j = 0; j < n_add; ++j) a += add_pairs[((size_t)j * gridDim.x + row) * d + i];
+    a *= gate;
     for (int c = 0; c < top; ++c) {
       const bool own = same && expert[(size_t)row * top + c] >= same_from;      // uniform over the workgroup
       const float v = own ? ld(same + (size_t)row * same_stride + i) : y[((size_t)row * top + c) * d + i];
@@ -424,6 +427,24 @@ pegainfer_status_t pegainfer_route_sort(const int32_t* expert, int32_t n_pairs, 
   return (pegainfer_status_t)hipGetLastError();
 }
 
+static pegainfer_status_t combine_launch(const float* y_pairs, const float* weight, const int32_t* expert, int32_t same_from, const void* same,
+                                         int64_t same_stride, const void* add, const float* add_pairs, int32_t n_add, const float* add_gate,
+                                         int64_t add_gate_stride, void* out, int32_t d, int32_t top, int32_t rows, int32_t dtype,
+                                         pegainfer_stream_t stream) {
+  if (rows <= 0) return 0;
+  if (same && !expert) return (pegainfer_status_t)hipErrorInvalidValue;
+  if (!by_dtype(dtype, [&](auto* t) {
+        using A = std::remove_pointer_t<decltype(t)>;
+        // few rows (decoding): the row is cut over several workgroups
+        const dim3 grid(rows, rows >= 256 ? 1 : std::min(16, ceil_div(d, 256)));
+        route_combine_kernel<A><<<grid, 256, 0, as_stream(stream)>>>(y_pairs, weight, static_cast<const A*>(add), static_cast<A*>(out), d,
+                                                                     top, add_gate, add_gate_stride, expert, same_from,
+                                                                     static_cast<const A*>(same), same_stride, add_pairs, n_add);
+      }))
+    return (pegainfer_status_t)hipErrorInvalidValue;
+  return (pegainfer_status_t)hipGetLastError();
+}
+
 pegainfer_status_t pegainfer_route_combine_gated(const float* y_pairs, const float* weight, const void* add,
                                                  const float* add_gate, int64_t add_gate_stride, void* out, int32_t d,
                                                  int32_t top, int32_t rows, int32_t dtype, pegainfer_stream_t stream) {
@@ -434,20 +455,17 @@ pegainfer_status_t pegainfer_route_combine_same(const float* y_pairs, const floa
                                                 const void* same, int64_t same_stride, const void* add, const float* add_gate,
                                                 int64_t add_gate_stride, void* out, int32_t d, int32_t top, int32_t rows, int32_t dtype,
                                                 pegainfer_stream_t stream) {
-  if (rows <= 0) return 0;
-  if (same && !expert) return (pegainfer_status_t)hipErrorInvalidValue;
-  if (!by_dtype(dtype, [&](auto* t) {
-        using A = std::remove_pointer_t<decltype(t)>;
-        // few rows (decoding): the row is cut over several workgroups
-        const dim3 grid(rows, rows >= 256 ? 1 : std::min(16, ceil_div(d, 256)));
-        route_combine_kernel<A><<<grid, 256, 0, as_stream(stream)>>>(y_pairs, weight, static_cast<const A*>(add), static_cast<A*>(out), d,
-                                                                     top, add_gate, add_gate_stride, expert, same_from,
-                                                                     static_cast<const A*>(same), same_stride);
-      }))
-    return (pegainfer_status_t)hipErrorInvalidValue;
-  return (pegainfer_status_t)hipGetLastError();
+  return combine_launch(y_pairs, weight, expert, same_from, same, same_stride, add, nullptr, 0, add_gate, add_gate_stride, out, d, top, rows, dtype,
+                        stream);
 }
 
+pegainfer_status_t pegainfer_route_combine_pairs(const float* y_pairs, const float* weight, const float* add_pairs, int32_t n_add,
+                                                 const float* add_gate, int64_t add_gate_stride, void* out, int32_t d, int32_t top,
+                                                 int32_t rows, int32_t dtype, pegainfer_stream_t stream) {
+  if (n_add < 0 || (n_add > 0 && !add_pairs)) return (pegainfer_status_t)hipErrorInvalidValue;
+  return combine_launch(y_pairs, weight, nullptr, 0, nullptr, 0, nullptr, add_pairs, n_add, add_gate, add_gate_stride, out, d, top, rows, dtype,
+                        stream);
+}
 pegainfer_status_t pegainfer_route_combine_add(const float* y_pairs, const float* weight, const void* add, void* out, int32_t d,
                                                int32_t top, int32_t rows, int32_t dtype, pegainfer_stream_t stream) {
   return pegainfer_route_combine_gated(y_pairs, weight, add, nullptr, 0, out, d, top, rows, dtype, stream);

@@ -545,6 +545,7 @@ struct JoinSource {
   const float *pairs, *weight; const int32_t* expert; int top, same_from;
   const A* same; int64_t same_stride;
   const A* add; const float* add_gate; int64_t add_gate_stride;
+  const float* add_pairs; int n_add;       // in place of `add`: that many fp32 rows per row, a step's rows apart
 };
 template <typename A, int N, int NPT, bool VEC, bool ROUTED>
 __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, JoinSource<A> src, const A* __restrict__ post,
@@ -573,7 +574,17 @@ __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, Join
     }
   }
   if constexpr (ROUTED) {
-    const float g = src.add && src.add_gate ? sigmoid_f(src.add_gate[(int64_t)row * src.add_gate_stride]) : 1.0f;
+    for (int j = 0; j < src.n_add; ++j)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const int i = (threadIdx.x + N * k) * V;
+        if (i >= d) continue;
+        float v[V];
+        load(src.add_pairs + ((int64_t)j * gridDim.x + row) * d + i, v);
+#pragma unroll
+        for (int u = 0; u < V; ++u) y[k][u] += v[u];
+      }
+    const float g = (src.add || src.n_add) && src.add_gate ? sigmoid_f(src.add_gate[(int64_t)row * src.add_gate_stride]) : 1.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
 #pragma unroll
@@ -714,7 +725,11 @@ pegainfer_status_t pegainfer_terms_rms(const pegainfer_terms_rms_desc* q, pegain
 }
 
 pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfer_stream_t stream) {
-  if (!q) return PK_BAD;
+  return pegainfer_join_rms_pairs(q, nullptr, 0, stream);
+}
+
+pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream) {
+  if (!q || n_add < 0 || (n_add > 0 && (!add_pairs || !q->y_pairs || q->add))) return PK_BAD;
   if (q->rows <= 0) return 0;
   const int d = q->d;
   const bool routed = q->y_pairs != nullptr;
@@ -724,8 +739,9 @@ pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfe
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         const JoinSource<A> src{static_cast<const A*>(q->y), q->y_row_stride, q->y_pairs, q->weight, q->expert, q->top, q->same_from,
-                                static_cast<const A*>(q->same), q->same_stride, static_cast<const A*>(q->add), q->add_gate, q->add_gate_stride};
-        const bool vec = d % 4 == 0 && q->y_row_stride % 4 == 0 && q->same_stride % 4 == 0 && host_aligned16(q->x) && host_aligned16(q->y) &&
+                                static_cast<const A*>(q->same), q->same_stride, static_cast<const A*>(q->add), q->add_gate, q->add_gate_stride,
+                                add_pairs, n_add};
+        const bool vec = d % 4 == 0 && host_aligned16(add_pairs) && q->y_row_stride % 4 == 0 && q->same_stride % 4 == 0 && host_aligned16(q->x) && host_aligned16(q->y) &&
                          host_aligned16(q->y_pairs) && host_aligned16(q->same) && host_aligned16(q->add) && host_aligned16(q->post) &&
                          host_aligned16(q->gain) && host_aligned16(q->n_out);
         auto launch = [&](auto kern, int threads) {

@@ -81,6 +81,16 @@ def gemm_strided(desc):
     _chk(ffi.lib().pegainfer_gemm_strided(ctypes.addressof(desc), _stream()), "gemm_strided")
 
 
+class ExpertRowsDesc(ctypes.Structure):
+    _fields_ = [("g", GemmDesc), ("glu", ctypes.c_int32), ("limit", ctypes.c_float), ("alpha", ctypes.c_float), ("shared_w", ctypes.c_void_p),
+                ("shared_groups", ctypes.c_int32), ("shared_rows", ctypes.c_int32), ("shared_pos0", ctypes.c_int32), ("shared_limit", ctypes.c_float),
+                ("shared_m_stride", ctypes.c_int64), ("shared_group_stride", ctypes.c_int64), ("shared_up", ctypes.c_int64)]
+
+
+def expert_rows(desc):
+    _chk(ffi.lib().pegainfer_expert_rows(ctypes.addressof(desc), _stream()), "expert_rows")
+
+
 def linear(x, w, out_dtype=None, epilogue=EPI_NONE, plain=False):
     """y[T, M] = x[T, K] w[M, K]^T through pegainfer_gemm_strided (any sizes, bf16 or fp32 operands, fp32 accumulation; x may be
     a column range of a wider matrix); plain = the fp32-FMA tile kernel whatever the shape"""
@@ -400,6 +410,16 @@ def route_combine_gated(y_pairs, weight, add, add_gate_f32, out_dtype):
     return out
 
 
+def route_combine_pairs(y_pairs, weight, add_pairs, add_gate_f32, out_dtype):
+    """the added row is the sum of the fp32 rows add_pairs[:, row] ([n_add, rows, d])"""
+    rows, top = weight.shape
+    out = torch.empty((rows, y_pairs.shape[1]), dtype=out_dtype, device=y_pairs.device)
+    _chk(ffi.lib().pegainfer_route_combine_pairs(_p(y_pairs), _p(weight), _p(add_pairs), add_pairs.shape[0], _p(add_gate_f32),
+                                                 0 if add_gate_f32 is None else add_gate_f32.stride(0), _p(out), out.shape[1], top, rows, _dt(out),
+                                                 _stream()), "route_combine_pairs")
+    return out
+
+
 # ---- several sublayers behind one norm, attention with shaped scores and gates, state-space scan ----
 class SumTerm(ctypes.Structure):
     _fields_ = [("y", ctypes.c_void_p), ("y_row_stride", ctypes.c_int64), ("bias", ctypes.c_void_p), ("norm_w", ctypes.c_void_p),
@@ -694,16 +714,16 @@ JoinRmsDesc = _struct("JoinRmsDesc", [("p", "x y"), ("l", "y_row_stride"), ("p",
 
 
 def join_rms(x_f32, post, gain=None, eps=1e-5, gain_offset=0.0, y=None, y_pairs=None, weight=None, expert=None, same_from=0, same=None, add=None,
-             add_gate_f32=None):
+             add_gate_f32=None, add_pairs=None):
     """x (in place) += rms_norm(y) * (gain_offset + post); -> rms_norm(x) * (gain_offset + gain) or None.  y: rows of the weights' type, or the
-    weighted sum of routed experts from y_pairs fp32 [rows * top, d]"""
+    weighted sum of routed experts from y_pairs fp32 [rows * top, d]; add_pairs fp32 [n_add, rows, d]: their sum in place of `add`"""
     rows, d = x_f32.shape
     n = torch.empty((rows, d), dtype=post.dtype, device=post.device) if gain is not None else None
     q = JoinRmsDesc(x=_p(x_f32), y=_p(y), y_row_stride=0 if y is None else y.stride(0), y_pairs=_p(y_pairs), weight=_p(weight), expert=_p(expert),
                     top=0 if weight is None else weight.shape[1], same_from=same_from, same=_p(same), same_stride=0 if same is None else same.stride(0),
                     add=_p(add), add_gate=_p(add_gate_f32), add_gate_stride=0 if add_gate_f32 is None else add_gate_f32.stride(0), post=_p(post),
                     gain=_p(gain), eps=float(eps), gain_offset=float(gain_offset), n_out=_p(n), d=d, rows=rows, dtype=_dt(post))
-    _chk(ffi.lib().pegainfer_join_rms(ctypes.addressof(q), _stream()), "join_rms")
+    _chk(ffi.lib().pegainfer_join_rms_pairs(ctypes.addressof(q), _p(add_pairs), 0 if add_pairs is None else add_pairs.shape[0], _stream()), "join_rms")
     return n
 
 

@@ -414,6 +414,61 @@ def test_few_rows_of_fp32_weights(T, M, K):
     assert float((y.cpu().double() - ref).abs().max()) < tol
 
 
+@pytest.mark.parametrize("T,ff,D,slices", [(1, 8, 8, 2), (1, 512, 1024, 0), (5, 40, 72, 3), (8, 136, 520, 1), (16, 264, 64, 2), (16, 16, 2056, 0)])
+@pytest.mark.parametrize("glu", [0, 1, 2])
+def test_experts_of_few_rows_with_activation_and_shared_slices(T, ff, D, slices, glu):
+    """gate and up rows in one wave, an expert that all rows take in slices behind the table's columns: both products of the feed-forward against
+    double precision; the first product's rows enter the second as they were stored.  Sums of D or ff products of about one in fp32."""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(T * 100 + ff + slices)
+    E, top, sff, two = 6, 3, slices * ff, 2 if glu else 1
+    bf = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    x, up, down, s_up, s_down = bf(T, D), bf(E, two * ff, D), bf(E, D, ff), bf(max(1, two * sff), D), bf(D, max(1, sff))
+    expert = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int()
+    dev_ = [t.cuda() for t in (x, up, down, s_up, s_down)]
+    xd, upd, downd, sud, sdd = dev_
+    pos_pair, pos_row, tg, t0, tr, nt, max_tiles = B.route_sort(expert.cuda(), E)
+    P, n = T * top, T * top + slices * T
+    act, y = torch.full((n, ff), float("nan"), device="cuda").bfloat16(), torch.full((n, D), float("nan"), device="cuda")
+    table = dict(tile_group=tg.data_ptr(), tile_row0=t0.data_ptr(), tile_rows=tr.data_ptr(), n_tiles=nt.data_ptr(), max_tiles=max_tiles, max_tile_rows=T)
+    shared = dict(shared_groups=slices, shared_rows=T, shared_pos0=P)
+    limit, s_limit, alpha = 9.0, 5.0, 1.702
+    g1 = B.GemmDesc(x=xd.data_ptr(), w=upd.data_ptr(), y=act.data_ptr(), x_dtype=0, w_dtype=0, y_dtype=0, m=ff, k=D, x_row_stride=D, w_m_stride=D,
+                    w_k_stride=1, w_group_stride=two * ff * D, y_row_stride=ff, x_row_index=pos_row.data_ptr(), epilogue=0 if glu else B.EPI_RELU_SQ, **table)
+    B.expert_rows(B.ExpertRowsDesc(g=g1, glu=glu, limit=limit, alpha=alpha, shared_limit=s_limit, shared_w=sud.data_ptr() if slices else None,
+                                   shared_m_stride=D, shared_group_stride=ff * D, shared_up=sff * D, **shared))
+    g2 = B.GemmDesc(x=act.data_ptr(), w=downd.data_ptr(), y=y.data_ptr(), x_dtype=0, w_dtype=0, y_dtype=1, m=D, k=ff, x_row_stride=ff, w_m_stride=ff,
+                    w_k_stride=1, w_group_stride=D * ff, y_row_stride=D, y_row_index=pos_pair.data_ptr(), **table)
+    B.expert_rows(B.ExpertRowsDesc(g=g2, shared_w=sdd.data_ptr() if slices else None, shared_m_stride=sff, shared_group_stride=ff, **shared))
+
+    def f(z, lim):
+        if not glu:
+            return torch.relu(z) ** 2
+        a, u = z.chunk(2, -1)
+        if glu == 1:
+            return a * torch.sigmoid(a) * u
+        a, u = a.clamp(max=lim), u.clamp(-lim, lim)
+        return a * torch.sigmoid(alpha * a) * (u + 1)
+    at = pos_pair.cpu().long()                       # sorted position -> pair
+    want = torch.stack([f(x[p // top].double() @ up[expert.view(-1)[p]].double().T, limit) for p in at.tolist()])
+    if slices:
+        s = f(x.double() @ s_up.double().T, s_limit)
+        want = torch.cat([want] + [s[:, j * ff:(j + 1) * ff] for j in range(slices)])
+    a = act.cpu().double()
+    assert float(((a - want).abs() / (want.abs() * 2.0 ** -8 + 1e-6 * D * (1 + want.abs().max().sqrt()))).max()) <= 1.0
+    rows = torch.full((n, D), float("nan"), dtype=torch.float64)
+    for q, p in enumerate(at.tolist()):
+        rows[p] = a[q] @ down[expert.view(-1)[p]].double().T
+    for j in range(slices):
+        rows[P + j * T:P + (j + 1) * T] = a[P + j * T:P + (j + 1) * T] @ s_down[:, j * ff:(j + 1) * ff].double().T
+    assert float((y.cpu().double() - rows).abs().max()) <= 1e-6 * ff * float(a.abs().max().clamp(min=1))
+    if slices:
+        w, gate = torch.rand(T, top, generator=g), torch.randn(T, generator=g)
+        got = B.route_combine_pairs(y[:P], w.cuda(), y[P:].view(slices, T, D), gate.cuda(), torch.float32)
+        ref = torch.einsum("tc,tcd->td", w.double(), rows[:P].view(T, top, D)) + torch.sigmoid(gate.double())[:, None] * rows[P:].view(slices, T, D).sum(0)
+        assert float((got.cpu().double() - ref).abs().max()) <= 2e-6 * ff * float(a.abs().max().clamp(min=1))
+
+
 @pytest.mark.parametrize("xd,yd", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "bfloat16"), ("float32", "float32")])
 @pytest.mark.parametrize("T,M,K,G", [(17, 128, 8, 1), (65, 130, 56, 2), (128, 127, 64, 3), (129, 300, 72, 1), (200, 1, 200, 2), (513, 514, 136, 40)])
 def test_tiles_on_the_matrix_cores_at_their_edges(T, M, K, G, xd, yd):

@@ -86,6 +86,12 @@ def test_one_launch_joins_norms_and_sums_routed_experts(dtype, rows, d):
         close(xs, ref, "float32", tol32=3e-6)
         if extra:
             assert n is None
+            parts = torch.randn(2, rows, d, generator=g)          # the added row in fp32 parts
+            xs = x.cuda()
+            B().join_rms(xs, dev(post, dtype), None, eps=1e-5, gain_offset=1.0, y_pairs=yp.cuda(), weight=wt.cuda(), expert=e.cuda(), same_from=E,
+                         same=dev(h, dtype), add_gate_f32=gate.cuda()[:, 2], add_pairs=parts.cuda())
+            t = routed + parts.double().sum(0) * torch.sigmoid(gate[:, 2:3].double())
+            close(xs, x.double() + R.zrms(t, post.double(), 1e-5), "float32", tol32=3e-6)
         else:
             close(n, R.zrms(ref, gain.double(), 1e-5), dtype, tol16=1e-2)
 
