@@ -397,6 +397,51 @@ typedef struct {
 pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfer_stream_t stream);
 /* with y_pairs: `add` is the sum of n_add fp32 rows, add_pairs[(j * rows + row) * d ..], j < n_add (q->add NULL) */
 pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream);
+/* A decode step's row between two matrix products, one launch (every entry brings one row: row e is entry e's).
+ *   v   = y + bias rows of dtype, or with y_pairs the weighted sum of routed experts (pegainfer_route_combine_gated / _pairs)
+ *   groups == 0:  r = x_in[row_index] + mult * v + add_rows + add_vec  -> x_out;   n = r / sqrt(mean(r^2) + eps) * gain[0]  -> n_out (fp32)
+ *   groups  > 0:  r = x_in + v / sqrt(mean over its group of v^2 + eps) * gain -> x_out, xb_out (dtype);
+ *                 n = sum_j coef[j] * stack[j * stack_stride ..] + coef[n_mix - 1] * r, j < n_mix - 1      -> mix_out (fp32)
+ *   conv        = n + sum over four taps of conv_w[c][tap] * (conv_state tail, n)                              -> conv_out, the tail moved on
+ *                 (pegainfer_time_conv_step: mode 1, four taps)
+ * Outputs and parts whose pointer is NULL are left out (groups == 0 without a gain: the sum alone).  Sizes: pegainfer_row_step_ok (state_off: of the
+ * tail inside a slot); every row on 16 bytes (bf16 vectors on 8). */
+typedef struct {
+  const float* x_in;
+  const int32_t* row_index;
+  float* x_out;
+  const void* y;
+  const void* bias;
+  float mult;
+  const float* y_pairs;
+  const float* weight;
+  int32_t top;
+  const void* add;
+  const float* add_pairs;
+  int32_t n_add;
+  const float* add_gate;
+  int64_t add_gate_stride;
+  const float* add_rows;
+  const void* add_vec;
+  const void* gain;
+  int32_t groups;
+  float eps;
+  float* n_out;
+  void* xb_out;
+  const float* stack;
+  int64_t stack_stride;
+  const void* coef;
+  int32_t n_mix;
+  float* mix_out;
+  const void* conv_w;
+  float* conv_state;
+  int64_t conv_slot_stride;
+  const int32_t* conv_slot;
+  void* conv_out;
+  int32_t d, rows, dtype;
+} pegainfer_row_step_desc;
+int32_t pegainfer_row_step_ok(int32_t d, int32_t groups, int32_t taps, int64_t state_off, int64_t slot_stride);
+pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream);
 /* out[row, i] = act(gate[row, i]) * up[row, i], i < I; gate and up are column ranges of rows with stride in_row_stride (elements of
  * dtype).  act 0 = silu, 1 = relu, 2 = gelu (tanh form), 3 = gelu (exact form) */
 enum { PEGAINFER_ACT_SILU = 0, PEGAINFER_ACT_RELU = 1, PEGAINFER_ACT_GELU_TANH = 2, PEGAINFER_ACT_GELU_ERF = 3 };

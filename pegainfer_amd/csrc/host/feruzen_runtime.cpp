@@ -921,15 +921,26 @@ struct Model {
     // ---- the layers (everything below reads the step's shape from its arguments and the step's contents from the metadata
     //      block, so a launch sequence recorded for one decode step serves every later step of the same shape)
     auto run_layers = [&]() -> int {
+    bool row_steps = single && !plain_kernels && pegainfer_row_step_ok(D, groups, canon_taps, 0, slot_stride);
+    for (const LayerCfg& c : layers) row_steps = row_steps && c.st_canon % 4 == 0;
     FZ_K(pegainfer_embed_f32(embed, d_tok, xs, D, Ti, dtype, S()));
-    FZ_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
+    if (!row_steps) FZ_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
+    // decode steps: a sublayer's output, normed, joins the stream
+    auto join_desc = [&](const float* from, const void* gain) {
+      pegainfer_row_step_desc q{};
+      q.x_in = from; q.y = y; q.gain = gain; q.groups = groups; q.eps = eps; q.d = D; q.rows = Ti; q.dtype = dtype;
+      return q;
+    };
     for (size_t li = 0; li < layers.size(); ++li) {
       const LayerCfg& c = layers[li];
       const LayerW& w = weights[li];
       const int Mp = c.proj_rows;
+      const float* x_in = row_steps && li == 0 ? xs : x;      // the stream at this layer's start
       // input convolution: hb = x + conv(x), then the tail moves on
-      if (single) {
-        FZ_K(pegainfer_time_conv_step(x, PEGAINFER_DTYPE_F32, D, w.canon, dtype, state + c.st_canon, slot_stride, hb, dtype, D, D,
+      if (row_steps && li > 0) {
+        // the launch that closed the layer before has left hb
+      } else if (single) {
+        FZ_K(pegainfer_time_conv_step(x_in, PEGAINFER_DTYPE_F32, D, w.canon, dtype, state + c.st_canon, slot_stride, hb, dtype, D, D,
                                       canon_taps, 1, d_slot, n, S()));
       } else {
         FZ_K(pegainfer_time_conv(x, PEGAINFER_DTYPE_F32, D, w.canon, dtype, state + c.st_canon, slot_stride, hb, dtype, D, D,
@@ -1012,11 +1023,34 @@ struct Model {
       if (linear(w.o, mix, y, D, Ti, c.mix_cols)) return -1;
       float* x_next = xs + (li + 1) * xs_stride;
       const int n_mix = (int)li + 2;
-      if (c.mlp.kind) {
+      if (row_steps) {
+        pegainfer_row_step_desc q = join_desc(x_in, w.norm1);
+        if (c.mlp.kind) {
+          q.x_out = x; q.xb_out = xb;
+          FZ_K(pegainfer_row_step(&q, S()));
+          q = join_desc(x, w.norm2);
+          if (c.mlp.kind == 1) {
+            if (glu(w.gate_up, w.down, c.mlp.glu, xb, y, Ti)) return -1;
+          } else {
+            if (routed_ff(c, w, Ti, true)) return -1;
+            q.y = nullptr;
+            q.y_pairs = ypairs; q.weight = route_w; q.top = c.mlp.top;
+            if (c.mlp.has_shared && expert_slices) { q.add_pairs = ypairs + (size_t)Ti * c.mlp.top * D; q.n_add = expert_slices; }
+            else if (c.mlp.has_shared) q.add = ys;
+          }
+        }
+        // the closing launch also convolves for the next layer
+        q.x_out = x_next; q.stack = xs; q.stack_stride = xs_stride; q.coef = w.dwa; q.n_mix = n_mix; q.mix_out = x;
+        if (li + 1 < layers.size()) {
+          q.conv_w = weights[li + 1].canon; q.conv_state = state + layers[li + 1].st_canon; q.conv_slot_stride = slot_stride; q.conv_slot = d_slot;
+          q.conv_out = hb;
+        }
+        FZ_K(pegainfer_row_step(&q, S()));
+      } else if (c.mlp.kind) {
         FZ_K(pegainfer_group_rms_add(x, y, dtype, w.norm1, groups, eps, x, xb, D, Ti, dtype, nullptr, 0, nullptr, 0, nullptr, nullptr, S()));
         if (c.mlp.kind == 1) {
           if (glu(w.gate_up, w.down, c.mlp.glu, xb, y, Ti)) return -1;
-        } else if (routed_ff(c, w, Ti)) {
+        } else if (routed_ff(c, w, Ti, false)) {
           return -1;
         }
         FZ_K(pegainfer_group_rms_add(x, y, dtype, w.norm2, groups, eps, x_next, nullptr, D, Ti, dtype, xs, xs_stride, w.dwa, n_mix, x,
@@ -1070,7 +1104,9 @@ struct Model {
     return 0;
   }
 
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T) {
+  int expert_slices = 0;   // of the last layer's shared expert: its rows lie behind the pairs
+  // sum_later: the pairs are left to the launch that joins them to the stream
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
     const MlpCfg& f = c.mlp;
     const int ff = f.glu.ff, P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
@@ -1136,11 +1172,14 @@ struct Model {
       FZ_K(pegainfer_clamp_glu_rows(gu_e, act_e, ff, P, f.glu.limit, kGluAlpha, dtype, S()));
       FZ_K(pegainfer_gemm_strided(&e, S()));
     }
+    expert_slices = slices;
+    if (slices && sum_later) return 0;
     if (slices) {
       FZ_K(pegainfer_route_combine_pairs(ypairs, route_w, ypairs + (size_t)P * D, slices, nullptr, 0, y, D, f.top, T, dtype, S()));
       return 0;
     }
     if (f.has_shared && glu(w.gate_up, w.down, f.shared, xb, ys, T)) return -1;
+    if (sum_later) return 0;
     FZ_K(pegainfer_route_combine_add(ypairs, route_w, f.has_shared ? ys : nullptr, y, D, f.top, T, dtype, S()));
     return 0;
   }

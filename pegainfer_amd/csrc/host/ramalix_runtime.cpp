@@ -921,17 +921,37 @@ struct Model {
     }
     // ---- the layer runs (everything below reads the step's shape from its arguments and the step's contents from the
     //      metadata block, so a launch sequence recorded for one decode step serves every later step of the same shape)
+    bool row_steps = single && !plain_kernels && pegainfer_row_step_ok(D, 0, canon_taps, 0, slot_stride);
+    for (const Run& r : runs) row_steps = row_steps && r.st_canon1 % 4 == 0 && r.st_canon2 % 4 == 0;
     // x <- x + mlt (yv + bias) + add_rows + add_vec; with a gain also the norm of the sublayer that follows and its input
     // convolution (hb = n + conv(n), the tail moved on)
+    // routed (decode steps): the layer whose experts' rows are still to be summed, in place of yv
     auto open_sublayer = [&](const void* yv, const void* bias, float mlt, const float* add_rows, const void* add_vec, bool write_x,
-                             const void* gain, const void* conv_w, int64_t st_off) -> int {
+                             const void* gain, const void* conv_w, int64_t st_off, const MlpCfg* routed = nullptr) -> int {
+      if (row_steps) {
+        pegainfer_row_step_desc q{};
+        q.x_in = x; q.x_out = write_x || !gain ? x : nullptr; q.y = yv; q.bias = yv ? bias : nullptr; q.mult = mlt;
+        if (routed) {
+          q.y = nullptr;
+          q.y_pairs = ypairs; q.weight = route_w; q.top = routed->top;
+          if (routed->has_shared) {
+            if (expert_slices) { q.add_pairs = ypairs + (size_t)Ti * routed->top * D; q.n_add = expert_slices; }
+            else q.add = ys;
+            q.add_gate = route_logits + routed->experts; q.add_gate_stride = routed->experts + 1;
+          }
+        }
+        q.add_rows = add_rows; q.add_vec = add_vec; q.gain = gain; q.eps = eps;
+        if (gain) { q.conv_w = conv_w; q.conv_state = state + st_off; q.conv_slot_stride = slot_stride; q.conv_slot = d_slot; q.conv_out = hb; }
+        q.d = D; q.rows = Ti; q.dtype = dtype;
+        RX_K(pegainfer_row_step(&q, S()));
+        return 0;
+      }
       if (!gain) {
         RX_K(pegainfer_scalar_rms_add(x, yv, dtype, bias, mlt, add_rows, add_vec, x, nullptr, eps, nullptr, D, Ti, dtype, S()));
         return 0;
       }
       RX_K(pegainfer_scalar_rms_add(x, yv, dtype, bias, mlt, add_rows, add_vec, write_x ? x : nullptr, gain, eps, n32, D, Ti, dtype, S()));
-      if (single) {   // output and the moved-on tail in one launch (folding it into the norm's launch was measured: one workgroup
-                      // per row then walks every channel's tail, 15 us against 5.6 + 4.3)
+      if (single) {   // output and the moved-on tail in one launch
         RX_K(pegainfer_time_conv_step(n32, PEGAINFER_DTYPE_F32, D, conv_w, dtype, state + st_off, slot_stride, hb, dtype, D, D,
                                       canon_taps, 1, d_slot, n, S()));
         return 0;
@@ -942,7 +962,8 @@ struct Model {
       return 0;
     };
     auto run_layers = [&]() -> int {
-    RX_K(pegainfer_embed_f32(embed, d_tok, emb, D, Ti, dtype, S()));
+    if (std::any_of(runs.begin(), runs.end(), [](const Run& r) { return r.pass > 0; }))      // a later pass reads them again
+      RX_K(pegainfer_embed_f32(embed, d_tok, emb, D, Ti, dtype, S()));
     RX_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
     for (size_t ri = 0; ri < runs.size(); ++ri) {
       const Run& r = runs[ri];
@@ -1003,8 +1024,8 @@ struct Model {
       const int64_t next_st = next_plain ? runs[ri + 1].st_canon1 : 0;
       if (c.mlp.kind) {
         if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, w.norm2, w.canon2, r.st_canon2)) return -1;
-        if (routed_ff(c, w, Ti)) return -1;
-        if (open_sublayer(y, nullptr, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st)) return -1;
+        if (routed_ff(c, w, Ti, row_steps)) return -1;
+        if (open_sublayer(y, nullptr, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st, &c.mlp)) return -1;
       } else if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st)) {
         return -1;
       }
@@ -1012,8 +1033,14 @@ struct Model {
     }
     // ---- wanted rows: final norm, logits over the output table in fp32, the constant factor
     if (W > 0) {
-      RX_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
-      RX_K(pegainfer_scalar_rms_add(xw, nullptr, dtype, nullptr, 0.f, nullptr, nullptr, nullptr, final_norm, eps, hw, D, W, dtype, S()));
+      if (!plain_kernels && pegainfer_row_step_ok(D, 0, 4, 0, 0)) {      // the wanted rows, normed
+        pegainfer_row_step_desc q{};
+        q.x_in = x; q.row_index = d_want; q.gain = final_norm; q.eps = eps; q.n_out = hw; q.d = D; q.rows = W; q.dtype = dtype;
+        RX_K(pegainfer_row_step(&q, S()));
+      } else {
+        RX_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
+        RX_K(pegainfer_scalar_rms_add(xw, nullptr, dtype, nullptr, 0.f, nullptr, nullptr, nullptr, final_norm, eps, hw, D, W, dtype, S()));
+      }
       if (linear_strided(head, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
       RX_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, logit_scale, 0.f, V, W, top1_state,
                                    out_tokens ? io.tokens() : nullptr, S()));
@@ -1052,8 +1079,10 @@ struct Model {
     return 0;
   }
 
-  // hb -> y: router logits and the shared expert's gate logit by one GEMM into fp32, selection, experts, weighted sum
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T) {
+  int expert_slices = 0;   // of the last layer's shared expert: its rows lie behind the pairs
+  // hb -> y: router logits and the shared expert's gate logit by one GEMM into fp32, selection, experts, weighted sum (sum_later: the pairs
+  // are left to the launch that joins them to the stream)
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
     const MlpCfg& f = c.mlp;
     const int ff = f.ff, P = T * f.top, E1 = f.experts + 1;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
@@ -1107,11 +1136,14 @@ struct Model {
       RX_K(pegainfer_silu_mul_rows(gu_e, act_e, ff, P, dtype, S()));
       RX_K(pegainfer_gemm_strided(&e, S()));
     }
+    expert_slices = slices;
+    if (slices && sum_later) return 0;
     if (slices) {
       RX_K(pegainfer_route_combine_pairs(ypairs, route_w, ypairs + (size_t)P * D, slices, route_logits + f.experts, E1, y, D, f.top, T, dtype, S()));
       return 0;
     }
     if (f.has_shared && swiglu(w.gate_up, w.down, f.shared_ff, hb, ys, T)) return -1;
+    if (sum_later) return 0;
     RX_K(pegainfer_route_combine_gated(ypairs, route_w, f.has_shared ? ys : nullptr, f.has_shared ? route_logits + f.experts : nullptr, E1, y,
                                        D, f.top, T, dtype, S()));
     return 0;

@@ -727,6 +727,20 @@ def join_rms(x_f32, post, gain=None, eps=1e-5, gain_offset=0.0, y=None, y_pairs=
     return n
 
 
+RowStepDesc = _struct("RowStepDesc", [("p", "x_in row_index x_out y bias"), ("f", "mult"), ("p", "y_pairs weight"), ("i", "top"), ("p", "add add_pairs"),
+                                      ("i", "n_add"), ("p", "add_gate"), ("l", "add_gate_stride"), ("p", "add_rows add_vec gain"), ("i", "groups"),
+                                      ("f", "eps"), ("p", "n_out xb_out stack"), ("l", "stack_stride"), ("p", "coef"), ("i", "n_mix"),
+                                      ("p", "mix_out conv_w conv_state"), ("l", "conv_slot_stride"), ("p", "conv_slot conv_out"),
+                                      ("i", "d rows dtype")])
+
+
+def row_step(dtype, rows, d, **parts):
+    """tensors by their field (their pointer is taken), numbers as they are"""
+    q = RowStepDesc(d=d, rows=rows, dtype={torch.bfloat16: 0, torch.float32: 1}[dtype],
+                    **{k: _p(v) if torch.is_tensor(v) else v for k, v in parts.items()})
+    _chk(ffi.lib().pegainfer_row_step(ctypes.addressof(q), _stream()), "row_step")
+
+
 def act_rows(x, act):
     """x: a [rows, I] view of rows with one stride"""
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)

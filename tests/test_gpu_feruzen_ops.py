@@ -413,3 +413,66 @@ def test_matrix_memory_chunks_in_runs_of_bounded_scratch():
     assert float((sa - sb).abs().max()) < 2e-5 * float(sa.abs().max())
     err = (a - b).abs() / (1 + a.abs())
     assert float(err.mean()) < 1e-5 and float(err.max()) < 2e-2
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("d,groups", [(4, 1), (1024, 4), (1028, 1), (2560, 5), (4096, 64), (4100, 5), (8192, 2)])
+def test_row_step_joins_norms_mixes_and_convolves(dtype, d, groups):
+    """both norms, a stored output or the routed sum with its added rows (stored or in parts), streams mixed, four taps with their tails moved on in
+    scattered slots: against double precision; fp32 sums of d values, a bf16 result rounded once"""
+    import importlib
+    B = importlib.import_module("pegainfer_amd.ops_blocks")
+    g = torch.Generator().manual_seed(d + groups)
+    rows, top, n_add, n_mix, eps, dt = 3, 2, 2, 4, 1e-5, getattr(torch, dtype)
+    f32 = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    st = lambda *s: torch.randn(*s, generator=g).to(dt)  # noqa: E731
+    x, y, bias, vec, extra, gain, one = f32(rows, d), st(rows, d), st(d), st(d), f32(rows, d), st(d), st(1)
+    pairs, wt, gate, add, parts = f32(rows * top, d), torch.rand(rows, top, generator=g), f32(rows, 3), st(rows, d), f32(n_add, rows, d)
+    stack, coef, cw = f32(n_mix - 1, rows, d), st(n_mix), st(d, 4)
+    slots, stride = torch.tensor([2, 0, 3], dtype=torch.int32), 3 * d + 8
+    state = f32(4, stride)
+    routed = (wt.double()[:, :, None] * pairs.double().view(rows, top, d)).sum(1)
+    sig = torch.sigmoid(gate[:, 1:2].double())
+
+    def close_(got, ref, stored):
+        tol = 4e-6 * ref.abs().max() + (ref.abs() * 2.0 ** -8 if stored and dtype == "bfloat16" else 0)
+        assert bool(((got.cpu().double() - ref).abs() <= tol).all())
+
+    def conv(n, out, sd):
+        tail = state[slots.long(), 4:4 + 3 * d].view(rows, 3, d).double()
+        close_(out, n + (torch.cat([tail, n[:, None]], 1) * cw.double().T[None]).sum(1), True)
+        want = state.clone().double()
+        want[slots.long(), 4:4 + 3 * d] = torch.cat([tail[:, 1:], n[:, None]], 1).reshape(rows, -1)
+        close_(sd, want, False)
+    for kind in ("stored", "routed", "parts"):
+        src = dict(y=y.cuda(), bias=bias.cuda()) if kind == "stored" else dict(y_pairs=pairs.cuda(), weight=wt.cuda(), top=top)
+        v = y.double() + bias.double() if kind == "stored" else routed
+        if kind != "stored":
+            gd = gate.cuda()
+            src.update(add_gate=gd[:, 1], add_gate_stride=3)
+            src.update(dict(add=add.cuda()) if kind == "routed" else dict(add_pairs=parts.cuda(), n_add=n_add))
+            v = v + sig * (add.double() if kind == "routed" else parts.double().sum(0))
+        for grouped in (False, True):
+            sd, xo, out = state.cuda(), x.cuda(), torch.zeros(rows, d, dtype=dt, device="cuda")
+            cv = dict(conv_w=cw.cuda(), conv_state=sd[0, 4:], conv_slot_stride=stride, conv_slot=slots.cuda(), conv_out=out)
+            if grouped:
+                xb, mix = torch.zeros(rows, d, dtype=dt, device="cuda"), torch.zeros(rows, d, device="cuda")
+                sk, cf, gn = stack.cuda(), coef.cuda(), gain.cuda()
+                B.row_step(dt, rows, d, x_in=xo, x_out=xo, gain=gn, groups=groups, eps=eps, xb_out=xb, stack=sk, stack_stride=rows * d, coef=cf, n_mix=n_mix,
+                           mix_out=mix, **src, **cv)
+                vn = v.view(rows, groups, -1)
+                r = x.double() + (vn / torch.sqrt((vn * vn).mean(-1, keepdim=True) + eps)).view(rows, d) * gain.double()
+                n = (coef.double()[:-1, None, None] * stack.double()).sum(0) + coef.double()[-1] * r
+                close_(xb, r, True)
+                close_(mix, n, False)
+            else:
+                no, ex, vc, on = torch.zeros(rows, d, device="cuda"), extra.cuda(), vec.cuda(), one.cuda()
+                B.row_step(dt, rows, d, x_in=xo, x_out=xo, mult=0.3, add_rows=ex, add_vec=vc, gain=on, eps=eps, n_out=no, **src, **cv)
+                r = x.double() + 0.3 * v + extra.double() + vec.double()
+                n = r / torch.sqrt((r * r).mean(-1, keepdim=True) + eps) * one.double()
+                close_(no, n, False)
+            close_(xo, r, False)
+            conv(n, out, sd)
+    pick, no, xd, on = torch.tensor([2, 2, 0, 1, 2], dtype=torch.int32).cuda(), torch.zeros(5, d, device="cuda"), x.cuda(), one.cuda()
+    B.row_step(dt, 5, d, x_in=xd, row_index=pick, gain=on, eps=eps, n_out=no)
+    close_(no, (x.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + eps) * one.double())[pick.cpu().long()], False)
