@@ -414,6 +414,110 @@ __global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_d
   }
 }
 
+// The same sums for fp32 weights with a wave's weights on their way before anything else: the whole first chunk of k (and the next chunk piece by
+// piece as this one is used), one output per wave where that leaves every compute unit a workgroup at most.  The rows pass through LDS as above, so
+// an output's k order is the same.  Bound by one memory latency behind the launch: 1024 x 1024 and 1 / 2 / 4 rows 4.4 / 4.7 / 6.4 -> 3.3 / 4.1 / 5.3 us,
+// 1024 x 3072 7.7 / 8.6 / 12.2 -> 5.6 / 7.3 / 10.1; one row of any size: 6144 x 1024 7.8 -> 7.0, 65 536 x 2048 108 -> 91.  With more outputs than
+// that, two and four rows lose: the rows' way into LDS is paid per workgroup (6144 x 1024, 2 rows: 8.0 us above, 10.5 here).
+template <typename TX, typename TY, typename TG, int R, int OUT>
+__global__ __launch_bounds__(256) void gemm_rows_fma_kernel(pegainfer_gemm_desc d) {
+  extern __shared__ __attribute__((aligned(16))) float xr[];    // [R][min(K, chunk)]
+  __shared__ int xrow[R], yrow[R];
+  constexpr int MB = OUT / 4, PF = kRowsFormChunk / 512;
+  int g, row0, nrows;
+  if (d.tile_group) {
+    if ((int)blockIdx.x >= *d.n_tiles) return;
+    g = d.tile_group[blockIdx.x];
+    row0 = d.tile_row0[blockIdx.x];
+    nrows = min(R, d.tile_rows[blockIdx.x]);
+  } else {
+    g = blockIdx.z;
+    row0 = blockIdx.x * R;
+    nrows = min(R, d.rows - row0);
+  }
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, K = d.k, xs = min(K, kRowsFormChunk);
+  const int m0 = blockIdx.y * OUT + wave * MB;
+  const float* W = static_cast<const float*>(d.w) + (int64_t)g * d.w_group_stride;
+  f32x4 w[PF][MB][2];
+  auto request = [&](int p, int k0) {                         // piece p of the chunk that starts at k0
+    const int k = k0 + p * 512 + lane * 8;
+    if (k < K) {
+#pragma unroll
+      for (int q = 0; q < MB; ++q) {
+        const float* src = W + (int64_t)min(m0 + q, d.m - 1) * d.w_m_stride + k;      // a clamped row is loaded and dropped at the store
+        w[p][q][0] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src));
+        w[p][q][1] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + 4));
+      }
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < PF; ++p) request(p, 0);
+  if (tid < R) {
+    const int p = row0 + tid;
+    xrow[tid] = tid < nrows ? (d.x_row_index ? d.x_row_index[p] : p) : -1;
+    yrow[tid] = tid < nrows ? (d.y_row_index ? d.y_row_index[p] : p) : -1;
+  }
+  __syncthreads();
+  const TX* X = static_cast<const TX*>(d.x) + (int64_t)g * d.x_group_stride;
+  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
+  float acc[MB][R];
+#pragma unroll
+  for (int q = 0; q < MB; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[q][r] = 0.f;
+  for (int kc0 = 0; kc0 < K; kc0 += kRowsFormChunk) {
+    const int kl = min(kRowsFormChunk, K - kc0);      // a multiple of 8, as K is
+    if (kc0 > 0) __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      for (int k = tid * 8; k < kl; k += 2048) {
+        float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (xrow[r] >= 0) Vec8<TX>::load(X + (int64_t)xrow[r] * d.x_row_stride + kc0 + k, t);
+        *reinterpret_cast<f32x4*>(xr + r * xs + k) = f32x4{t[0], t[1], t[2], t[3]};
+        *reinterpret_cast<f32x4*>(xr + r * xs + k + 4) = f32x4{t[4], t[5], t[6], t[7]};
+      }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PF; ++p) {
+      const int k = p * 512 + lane * 8;
+      if (k < kl) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const f32x4 xa = *reinterpret_cast<const f32x4*>(xr + r * xs + k), xb = *reinterpret_cast<const f32x4*>(xr + r * xs + k + 4);
+#pragma unroll
+          for (int q = 0; q < MB; ++q) {
+            float a = acc[q][r];
+            a = fmaf(w[p][q][0].x, xa.x, a); a = fmaf(w[p][q][0].y, xa.y, a); a = fmaf(w[p][q][0].z, xa.z, a); a = fmaf(w[p][q][0].w, xa.w, a);
+            a = fmaf(w[p][q][1].x, xb.x, a); a = fmaf(w[p][q][1].y, xb.y, a); a = fmaf(w[p][q][1].z, xb.z, a); a = fmaf(w[p][q][1].w, xb.w, a);
+            acc[q][r] = a;
+          }
+        }
+      }
+      request(p, kc0 + kRowsFormChunk);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < MB; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[q][r] = wave_sum(acc[q][r]);
+  if (lane != 0) return;
+#pragma unroll
+  for (int q = 0; q < MB; ++q) {
+    const int m = m0 + q;
+    if (m >= d.m) break;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (yrow[r] < 0) continue;
+      float v = acc[q][r];
+      if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+      else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
+      else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
+        v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)xrow[r] * d.gate_row_stride + g));
+      st(Y + (int64_t)yrow[r] * d.y_row_stride + m, v);
+    }
+  }
+}
+
 // 32 outputs per workgroup unless that leaves most compute units without one
 static bool rows_form_fine(const pegainfer_gemm_desc& d, int R) {
   const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
@@ -431,6 +535,18 @@ static void rows_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   const size_t lds = (size_t)R * std::min(d.k, kRowsFormChunk) * sizeof(float);
   if (fine) kern8<<<grid, 256, lds, s>>>(d);
   else kern<<<grid, 256, lds, s>>>(d);
+}
+
+// two and four rows: no more than a workgroup of four outputs per compute unit (1024 outputs on 256)
+static bool rows_fma_takes(const pegainfer_gemm_desc& d, int R) {
+  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
+  return (long)row_tiles * groups * ceil_div(d.m, 4) <= device_cus();
+}
+template <typename TX, typename TY, typename TG, int R>
+static void rows_fma_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
+  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
+  const size_t lds = (size_t)R * std::min(d.k, kRowsFormChunk) * sizeof(float);
+  gemm_rows_fma_kernel<TX, TY, TG, R, 4><<<dim3(row_tiles, ceil_div(d.m, 4), groups), 256, lds, s>>>(d);
 }
 
 // ------------------------------------------------------------------ few-rows form on the matrix cores (bf16 weights, decode)
@@ -925,7 +1041,10 @@ static bool gemm_strided_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
         const int R = tr <= 1 ? 1 : d.k > 2 * kRowsFormChunk ? 0 : tr <= 2 ? 2 : tr <= 4 ? 4 : 0;
         auto run = [&](auto gate) {
           using TG = std::remove_pointer_t<decltype(gate)>;
-          if (R == 1) rows_form_launch<TX, TW, TY, TG, 1>(d, s);
+          if (R == 1 && d.m <= 4 * 65535) rows_fma_launch<TX, TY, TG, 1>(d, s);      // as many columns of workgroups as a grid takes
+          else if (R == 1) rows_form_launch<TX, TW, TY, TG, 1>(d, s);
+          else if (R == 2 && rows_fma_takes(d, 2)) rows_fma_launch<TX, TY, TG, 2>(d, s);
+          else if (R == 4 && rows_fma_takes(d, 4)) rows_fma_launch<TX, TY, TG, 4>(d, s);
           // two rows of their own where workgroups are small (5.7 -> 4.4 us at 1024 x 1024); 65 536 x 2048 took 117 us so, 105 with four
           else if (R == 2 && rows_form_fine(d, 2)) rows_form_launch<TX, TW, TY, TG, 2>(d, s);
           else if (R) rows_form_launch<TX, TW, TY, TG, 4>(d, s);
