@@ -273,7 +273,11 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(float* __restric
 constexpr int kTileRows = 64, kTileKeys = 32;
 constexpr int kLatPrefetch = 10;     // 16-byte chunks per thread and key tile: 32 keys x (E / 8) <= 2560 chunks, E <= 640
 
-template <int ND>
+// FULL: the rank is 16 ND, so no step over the latent dims asks whether it is there and the reads of several are on their way together: with
+// the longer unroll of the scores 16 heads of 512 + 64, prompts of 300 - 900 tokens 225 -> 208 us, one of 1800 436 -> 387, 100 tokens behind 2000
+// 317 -> 280.  A maximum that follows with a lag (no rescaling of most tiles) would take 194 us, but rounds the largest weight, which is
+// exactly one here: 1.5 times the error on peaked rows.
+template <int ND, bool FULL>
 __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
                                                                const uint16_t* __restrict__ cache, int64_t page_stride,
                                                                int64_t layer_off, int page_size,
@@ -362,7 +366,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
     const uint16_t* kp0 = Ck + l15 * cs + g * 8;
     const uint16_t* kp1 = Ck + (16 + l15) * cs + g * 8;
     int kb = 0;
-#pragma unroll 2
+#pragma unroll 3
     for (; kb + 64 <= Epad; kb += 64) {
       const bf16x8_t qa = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(qp + kb));
       const bf16x8_t qb = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(qp + kb + 32));
@@ -417,7 +421,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
     }
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
-      if (d * 16 >= r) break;
+      if (!FULL && d * 16 >= r) break;
       const v4s_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + d * 16));
       const v4s_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + d * 16 + 16 * cs));
       const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
@@ -746,7 +750,12 @@ struct LatentCall {
   }
   template <int ND>
   void wide() const {
-    auto kern = &latent_attn_mfma_kernel<ND>;
+    if (r == ND * 16) wide_form<ND, true>();
+    else wide_form<ND, false>();
+  }
+  template <int ND, bool FULL>
+  void wide_form() const {
+    auto kern = &latent_attn_mfma_kernel<ND, FULL>;
     static const bool once = all_lds(kern);
     (void)once;
     const int Epad = (r + dr + 31) & ~31;
