@@ -35,6 +35,28 @@ pegainfer_status_t pegainfer_dyt_add_norm(float* x, const void* y, const void* p
                                           const void* post_b, const void* next_alpha, const void* next_w,
                                           const void* next_b, void* out, int32_t d, int32_t rows, int32_t dtype,
                                           pegainfer_stream_t stream);
+/* These in one launch around each row, every part optional: x starts as embed[token_ids[row]] (embed given) or is read in place or, without being
+ * written, through row_index;  x += dyt(v; post) with v = y rows of dtype or the weighted sum of routed experts (pegainfer_route_combine);
+ * out = dyt(x; next).  d % 4 == 0; fp32 rows on 16 bytes, bf16 ones on 8. */
+typedef struct {
+  float* x;
+  const void* embed;
+  const uint32_t* token_ids;
+  const int32_t* row_index;
+  const void* y;
+  const float* y_pairs;
+  const float* weight;
+  int32_t top;
+  const void* post_alpha;
+  const void* post_w;
+  const void* post_b;
+  const void* next_alpha;
+  const void* next_w;
+  const void* next_b;
+  void* out;
+  int32_t d, rows, dtype;
+} pegainfer_dyt_step_desc;
+pegainfer_status_t pegainfer_dyt_step(const pegainfer_dyt_step_desc* q, pegainfer_stream_t stream);
 /* rows of an fp32 matrix gathered by index: out[i, :] = x[rows_index[i], :] (the positions whose logits are wanted) */
 pegainfer_status_t pegainfer_gather_rows_f32(const float* x, const int32_t* rows_index, float* out, int32_t d,
                                              int32_t n_rows, pegainfer_stream_t stream);

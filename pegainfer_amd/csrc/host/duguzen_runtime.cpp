@@ -120,7 +120,7 @@ struct Model {
   // step buffers (grow-only, sized by token rows / wanted rows)
   size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
-  float *x = nullptr, *qc = nullptr, *olat = nullptr, *ypairs = nullptr, *route_w = nullptr, *attn_ws = nullptr;
+  float *x = nullptr, *qc = nullptr, *olat = nullptr, *ypairs = nullptr, *route_w = nullptr, *route_logits = nullptr, *attn_ws = nullptr;
   size_t attn_ws_cap = 0;
   void *h = nullptr, *proj = nullptr, *attn = nullptr, *y = nullptr, *ffb = nullptr, *gu = nullptr, *act = nullptr;
   int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
@@ -514,7 +514,7 @@ struct Model {
         dalloc_a(&proj, n * mx_proj, so) || dalloc_a(&attn, n * mx_attn, so) || dalloc_a(&y, n * D, so) ||
         dalloc_a(&ffb, n * std::max(1, mx_ff), so))
       return -1;
-    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
+    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, ptiles::kFewRows * (size_t)mx_experts, so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
                        dalloc(&pos_row, P, so) || dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu, n * mx_gu, so) ||
                        dalloc_a(&act, n * (size_t)(mx_gu / 2), so)))
       return -1;
@@ -539,7 +539,8 @@ struct Model {
   }
   // Y[T, M] = X[T, K] W[M, K]^T in the model's storage type
   int linear(const void* W, const void* X, void* Y, int M, int T, int K, int epilogue = PEGAINFER_EPI_NONE) {
-    if (dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels) {
+    // few rows with an activation: the strided GEMM's few-rows form leaves it in its epilogue
+    if (dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && !(epilogue && T <= ptiles::kFewRows)) {
       gemm_cuda(static_cast<const Half*>(W), static_cast<const Half*>(X), static_cast<Half*>(Y), M, T, K, S());
       if (epilogue == PEGAINFER_EPI_RELU_SQ) DZ_K(pegainfer_relu_sq(Y, Y, (int64_t)M * T, dtype, S()));
       return 0;
@@ -685,9 +686,34 @@ struct Model {
     // ---- the layers (everything below reads the step's shape from its arguments and the step's contents from the metadata block, so a
     //      launch sequence recorded for one decode step serves every later step of the same shape)
     auto run_layers = [&]() -> int {
-    DZ_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
-    {
+    const bool steps = !plain_kernels && D % 4 == 0;
+    auto set_next = [](pegainfer_dyt_step_desc* q, const Norm* n) {
+      if (n) { q->next_alpha = n->alpha; q->next_w = n->w; q->next_b = n->b; }
+    };
+    // the stream takes a sublayer's output (routed: the experts' rows still to be summed) through its post-norm; the next pre-norm leaves h
+    auto join = [&](const Norm& post, const Norm* next, const MlpCfg* routed = nullptr) -> int {
+      if (!steps) {
+        DZ_K(pegainfer_dyt_add_norm(x, y, post.alpha, post.w, post.b, next ? next->alpha : nullptr, next ? next->w : nullptr, next ? next->b : nullptr,
+                                    h, D, Ti, dtype, S()));
+        return 0;
+      }
+      pegainfer_dyt_step_desc q{};
+      q.x = x; q.d = D; q.rows = Ti; q.dtype = dtype; q.out = h;
+      if (routed) { q.y_pairs = ypairs; q.weight = route_w; q.top = routed->top; }
+      else q.y = y;
+      q.post_alpha = post.alpha; q.post_w = post.w; q.post_b = post.b;
+      set_next(&q, next);
+      DZ_K(pegainfer_dyt_step(&q, S()));
+      return 0;
+    };
+    if (steps) {
+      pegainfer_dyt_step_desc q{};
+      q.x = x; q.embed = embed; q.token_ids = d_tok; q.d = D; q.rows = Ti; q.dtype = dtype; q.out = h;
+      set_next(&q, &weights[layers[0].owner].n1);
+      DZ_K(pegainfer_dyt_step(&q, S()));
+    } else {
       const LayerW& w0 = weights[layers[0].owner];
+      DZ_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
       DZ_K(pegainfer_dyt_norm(x, w0.n1.alpha, w0.n1.w, w0.n1.b, h, D, Ti, dtype, S()));
     }
     for (size_t li = 0; li < layers.size(); ++li) {
@@ -739,24 +765,29 @@ struct Model {
       }
       if (linear(w.o, attn, y, D, Ti, m.heads * m.vdim)) return -1;
       if (c.mlp.kind) {
-        DZ_K(pegainfer_dyt_add_norm(x, y, w.n1b.alpha, w.n1b.w, w.n1b.b, w.n2.alpha, w.n2.w, w.n2.b, h, D, Ti, dtype, S()));
+        if (join(w.n1b, &w.n2)) return -1;
         if (c.mlp.kind == 1) {
           if (linear(w.up, h, ffb, c.mlp.ff, Ti, D, PEGAINFER_EPI_RELU_SQ) || linear(w.down, ffb, y, D, Ti, c.mlp.ff)) return -1;
-        } else if (routed_ff(c, w, Ti)) {
+        } else if (routed_ff(c, w, Ti, steps)) {
           return -1;
         }
-        DZ_K(pegainfer_dyt_add_norm(x, y, w.n2b.alpha, w.n2b.w, w.n2b.b, next_pre ? next_pre->alpha : nullptr,
-                                    next_pre ? next_pre->w : nullptr, next_pre ? next_pre->b : nullptr, h, D, Ti, dtype, S()));
-      } else {
-        DZ_K(pegainfer_dyt_add_norm(x, y, w.n1b.alpha, w.n1b.w, w.n1b.b, next_pre ? next_pre->alpha : nullptr,
-                                    next_pre ? next_pre->w : nullptr, next_pre ? next_pre->b : nullptr, h, D, Ti, dtype, S()));
+        if (join(w.n2b, next_pre, c.mlp.kind == 2 ? &c.mlp : nullptr)) return -1;
+      } else if (join(w.n1b, next_pre)) {
+        return -1;
       }
       if (tap_on) DZ_HIP(hipMemcpyAsync(tap + li * T * D, x, T * D * 4, hipMemcpyDeviceToDevice, stream));
     }
     // ---- wanted rows: final norm + head
     if (W > 0) {
-      DZ_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
-      DZ_K(pegainfer_dyt_norm(xw, final_norm.alpha, final_norm.w, final_norm.b, hw, D, W, dtype, S()));
+      if (steps) {
+        pegainfer_dyt_step_desc q{};
+        q.x = x; q.row_index = d_want; q.d = D; q.rows = W; q.dtype = dtype; q.out = hw;
+        set_next(&q, &final_norm);
+        DZ_K(pegainfer_dyt_step(&q, S()));
+      } else {
+        DZ_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
+        DZ_K(pegainfer_dyt_norm(xw, final_norm.alpha, final_norm.w, final_norm.b, hw, D, W, dtype, S()));
+      }
       void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
       if (linear(head, hw, lg, V, W, D)) return -1;
       DZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr, S()));
@@ -796,15 +827,36 @@ struct Model {
     return 0;
   }
 
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T) {
+  // sum_later: the pairs are left to the launch that joins them to the stream
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
     const MlpCfg& f = c.mlp;
     const int P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
-    DZ_K(pegainfer_route_sigmoid_grouped(h, w.router, w.corr, route_e, route_w, D, f.experts, f.groups, f.keep, f.top, T, dtype, S()));
     // few rows: tiles of the step's rows; otherwise 128-row tiles for the matrix-core form of bf16 weights, 64-row tiles
     const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0;
     const int per_tile = ptiles::expert_tile_rows(T, wide);
-    DZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
+    if (T <= ptiles::kFewRows && f.experts <= 1024) {
+      // few rows (decoding): the few-rows GEMM streams the router with the whole chip into fp32 logits, then selection and sort in one launch
+      // (4 rows of 2048, 32 experts: 10.0 + 4.2 -> 5.0 + 6.3 us)
+      pegainfer_gemm_desc r{};
+      r.x = h; r.w = w.router; r.y = route_logits;
+      r.x_dtype = r.w_dtype = dtype; r.y_dtype = PEGAINFER_DTYPE_F32;
+      r.m = f.experts; r.k = D; r.rows = T; r.groups = 1;
+      r.x_row_stride = D; r.w_m_stride = D; r.w_k_stride = 1; r.y_row_stride = f.experts;
+      r.plain = plain_kernels;
+      DZ_K(pegainfer_gemm_strided(&r, S()));
+      pegainfer_route_plan_desc q{};
+      q.logits = route_logits; q.logits_stride = f.experts; q.correction = w.corr; q.out_expert = route_e; q.out_weight = route_w;
+      q.experts = f.experts; q.n_groups = f.groups; q.keep_groups = f.keep; q.top = f.top; q.rows = T;
+      q.score_kind = PEGAINFER_SCORE_SIGMOID; q.group_kind = PEGAINFER_GROUP_TOP2_SUM; q.factor = 1.0f;
+      q.sort_experts = f.experts; q.pos_pair = pos_pair; q.pos_row = pos_row;
+      q.tile_group = t_group; q.tile_row0 = t_row0; q.tile_rows = t_rows; q.n_tiles = n_tiles;
+      q.max_tiles = max_tiles; q.rows_per_tile = per_tile; q.dtype = dtype;
+      DZ_K(pegainfer_route_plan(&q, S()));
+    } else {
+      DZ_K(pegainfer_route_sigmoid_grouped(h, w.router, w.corr, route_e, route_w, D, f.experts, f.groups, f.keep, f.top, T, dtype, S()));
+      DZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
+    }
     pegainfer_gemm_desc d{};
     d.x = h; d.w = w.gate_up_e; d.y = gu;
     d.x_dtype = d.w_dtype = d.y_dtype = dtype;
@@ -837,6 +889,7 @@ struct Model {
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
     DZ_K(pegainfer_gemm_strided(&e, S()));
+    if (sum_later) return 0;
     DZ_K(pegainfer_route_combine(ypairs, route_w, y, D, f.top, T, dtype, S()));
     return 0;
   }

@@ -727,6 +727,17 @@ def join_rms(x_f32, post, gain=None, eps=1e-5, gain_offset=0.0, y=None, y_pairs=
     return n
 
 
+DytStepDesc = _struct("DytStepDesc", [("p", "x embed token_ids row_index y y_pairs weight"), ("i", "top"),
+                                      ("p", "post_alpha post_w post_b next_alpha next_w next_b out"), ("i", "d rows dtype")])
+
+
+def dyt_step(dtype, rows, d, **parts):
+    """tensors by their field (their pointer is taken), numbers as they are"""
+    q = DytStepDesc(d=d, rows=rows, dtype={torch.bfloat16: 0, torch.float32: 1}[dtype],
+                    **{k: _p(v) if torch.is_tensor(v) else v for k, v in parts.items()})
+    _chk(ffi.lib().pegainfer_dyt_step(ctypes.addressof(q), _stream()), "dyt_step")
+
+
 RowStepDesc = _struct("RowStepDesc", [("p", "x_in row_index x_out y bias"), ("f", "mult"), ("p", "y_pairs weight"), ("i", "top"), ("p", "add add_pairs"),
                                       ("i", "n_add"), ("p", "add_gate"), ("l", "add_gate_stride"), ("p", "add_rows add_vec gain"), ("i", "groups"),
                                       ("f", "eps"), ("p", "n_out xb_out stack"), ("l", "stack_stride"), ("p", "coef"), ("i", "n_mix"),

@@ -414,6 +414,47 @@ def test_few_rows_of_fp32_weights(T, M, K):
     assert float((y.cpu().double() - ref).abs().max()) < tol
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows,d", [(1, 4), (3, 1020), (5, 1024), (300, 1028), (2, 4100)])
+def test_dyt_step_starts_joins_and_picks_rows(dtype, rows, d):
+    """an embedding row and its norm, a stored or routed output through the post-norm and the next norm, picked rows normed; against double
+    precision: a few fp32 operations per value (tanh within 2e-6), a bf16 result rounded once"""
+    from pegainfer_amd import ops_blocks as B
+    g, dt = torch.Generator().manual_seed(rows + d), DT[dtype]
+    st = lambda *s: torch.randn(*s, generator=g).to(dt)  # noqa: E731
+    emb, ids = st(7, d), torch.randint(0, 7, (rows,), generator=g, dtype=torch.int32)
+    pa, pw, pb, na, nw, nb, y = st(1), st(d), st(d), st(1), st(d), st(d), st(rows, d)
+    pairs, wt = torch.randn(rows * 3, d, generator=g), torch.rand(rows, 3, generator=g)
+    D64 = lambda t: t.double()  # noqa: E731
+    norm = lambda t, a, w, b: torch.tanh(D64(a) * t) * D64(w) + D64(b)  # noqa: E731
+
+    def close_(got, ref, stored):
+        tol = 4e-6 * (1 + ref.abs()) + (ref.abs() * 2.0 ** -8 if stored and dtype == "bfloat16" else 0)
+        assert bool(((got.cpu().double() - ref).abs() <= tol).all())
+    k = {n: t.cuda() for n, t in dict(post_alpha=pa, post_w=pw, post_b=pb, next_alpha=na, next_w=nw, next_b=nb).items()}
+    nxt = {n: k[n] for n in ("next_alpha", "next_w", "next_b")}
+    x, out = torch.full((rows, d), float("nan"), device="cuda"), torch.zeros(rows, d, dtype=dt, device="cuda")
+    ed, idd = emb.cuda(), ids.cuda()
+    B.dyt_step(dt, rows, d, x=x, embed=ed, token_ids=idd, out=out, **nxt)
+    ref = D64(emb)[ids.long()]
+    close_(x, ref, False)
+    close_(out, norm(ref, na, nw, nb), True)
+    routed = (D64(wt)[:, :, None] * D64(pairs).view(rows, 3, d)).sum(1)
+    for src, v in ((dict(y=y.cuda()), D64(y)), (dict(y_pairs=pairs.cuda(), weight=wt.cuda(), top=3), routed)):
+        before = x.cpu().double()
+        B.dyt_step(dt, rows, d, x=x, out=out, **src, **k)
+        ref = before + norm(v, pa, pw, pb)
+        # a routed sum is rounded as a stored one is: half a unit of it, through the post-norm's slope alpha * w
+        slack = (v.abs() * 2.0 ** -8 * D64(pa).abs() * D64(pw).abs() if "y_pairs" in src and dtype == "bfloat16" else 0)
+        assert bool(((x.cpu().double() - ref).abs() <= 4e-6 * (1 + ref.abs()) + slack).all())
+        close_(out, norm(x.cpu().double(), na, nw, nb), True)
+    before, pick = x.clone(), torch.randint(0, rows, (4,), generator=g, dtype=torch.int32).cuda()
+    o4 = torch.zeros(4, d, dtype=dt, device="cuda")
+    B.dyt_step(dt, 4, d, x=x, row_index=pick, out=o4, **nxt)
+    close_(o4, norm(before.cpu().double()[pick.cpu().long()], na, nw, nb), True)
+    assert torch.equal(x, before)
+
+
 @pytest.mark.parametrize("T,ff,D,slices", [(1, 8, 8, 2), (1, 512, 1024, 0), (5, 40, 72, 3), (8, 136, 520, 1), (16, 264, 64, 2), (16, 16, 2056, 0)])
 @pytest.mark.parametrize("glu", [0, 1, 2])
 def test_experts_of_few_rows_with_activation_and_shared_slices(T, ff, D, slices, glu):
