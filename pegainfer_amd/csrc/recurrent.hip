@@ -171,6 +171,77 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(const float* __restrict
   }
 }
 
+// a token's log input and forget gate
+template <typename A>
+struct MemoryGates {
+  const A* proj; int64_t proj_stride, i_off, f_off;
+  float ib, fb, cap;
+  int h;
+  __device__ __forceinline__ float in(int64_t row) const { return cap * tanhf((ld(proj + row * proj_stride + i_off + h) + ib) / cap); }
+  __device__ __forceinline__ float forget(int64_t row) const { return logsigmoid_f(cap * tanhf((ld(proj + row * proj_stride + f_off + h) + fb) / cap)); }
+};
+
+// A round's tc tokens, their gates in s_i / s_f: the running maxima s_m[1 ..] from s_m[0], then every token's factors (rows past tc leave S and
+// n as they are).  Ends behind a barrier; s_m[0] is the round's last maximum.
+__device__ __forceinline__ void memory_round(int tid, int tc, const float* s_i, const float* s_f, float* s_m, float* s_a, float* s_b, float* s_em) {
+  if (tid == 0) {                 // the running maximum is a chain of one add and one max per token: one lane walks it
+    float mm = s_m[0];
+    for (int tt = 0; tt < tc; ++tt) {
+      mm = fmaxf(s_f[tt] + mm, s_i[tt]);
+      s_m[tt + 1] = mm;
+    }
+  }
+  __syncthreads();
+  if (tid < kRecTokens) {         // ... and the exponentials it feeds are computed side by side
+    const bool live = tid < tc;   // rows past the entry's end: a = 1, b = 0 - a step that leaves S and n as they are
+    const float mp = live ? s_m[tid] : 0.f, mn = live ? s_m[tid + 1] : 0.f;
+    s_a[tid] = live ? expf(s_f[tid] + mp - mn) : 1.f;
+    s_b[tid] = live ? expf(s_i[tid] - mn) : 0.f;
+    s_em[tid] = live ? expf(-mn) : 1.f;
+  }
+  __syncthreads();
+  if (tid == 0) s_m[0] = s_m[tc];
+}
+
+// n and the running maximum of an (entry, head) are read by every workgroup of the scan below that owns columns of it, so none of these may
+// write them: where there are several, this launch behind the scan moves both on, by the same steps (a thread per value of n).
+template <typename A>
+__global__ __launch_bounds__(256) void memory_carry_kernel(const A* __restrict__ proj, int64_t proj_stride, int64_t k_off, int64_t i_off,
+                                                           int64_t f_off, const A* __restrict__ i_bias, const A* __restrict__ f_bias, float cap,
+                                                           float* __restrict__ state, int64_t slot_stride, int H, int dim, int vdim,
+                                                           const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot,
+                                                           int scan_max) {
+  __shared__ float s_i[kRecTokens], s_f[kRecTokens], s_m[kRecTokens + 1], s_a[kRecTokens], s_b[kRecTokens], s_em[kRecTokens];
+  const int e = blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
+  const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
+  if (scan_max > 0 && len > scan_max) return;      // the chunk form has this entry
+  float* base = state + (int64_t)entry_slot[e] * slot_stride + (int64_t)H * dim * vdim;
+  float *n_g = base + (int64_t)h * dim, *m_g = base + (int64_t)H * dim + h;
+  const MemoryGates<A> gate{proj, proj_stride, i_off, f_off, ld(i_bias + h), ld(f_bias + h), cap, h};
+  const int d = min(tid, dim - 1);
+  float n = n_g[d];
+  if (tid == 0) s_m[0] = *m_g;
+  for (int t0 = 0; t0 < len; t0 += kRecTokens) {
+    const int tc = min(kRecTokens, len - t0);
+    float kk[kRecTokens];
+#pragma unroll
+    for (int t = 0; t < kRecTokens; ++t) kk[t] = ld(proj + (int64_t)(row0 + t0 + min(t, tc - 1)) * proj_stride + k_off + (int64_t)h * dim + d);
+    __syncthreads();
+    if (tid < tc) {
+      s_i[tid] = gate.in(row0 + t0 + tid);
+      s_f[tid] = gate.forget(row0 + t0 + tid);
+    }
+    __syncthreads();
+    memory_round(tid, tc, s_i, s_f, s_m, s_a, s_b, s_em);
+#pragma unroll
+    for (int t = 0; t < kRecTokens; ++t)
+      if (t < tc) n = fmaf(s_b[t], kk[t], s_a[t] * n);
+  }
+  __syncthreads();
+  if (tid < dim) n_g[tid] = n;
+  if (tid == 0) *m_g = s_m[0];
+}
+
 template <int NS, typename A>
 __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict__ proj, int64_t proj_stride, int64_t q_off,
                                                             int64_t k_off, int64_t v_off, int64_t i_off, int64_t f_off,
@@ -200,7 +271,8 @@ __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict_
     n[i] = d < dim ? n_g[d] : 0.f;
   }
   if (tid == 0) s_m[0] = *m_g;     // s_m[0] = the maximum before the round, s_m[t + 1] = after its token t
-  const float ib = ld(i_bias + h), fb = ld(f_bias + h), qs = 1.0f / sqrtf((float)dim);
+  const MemoryGates<A> gate{proj, proj_stride, i_off, f_off, ld(i_bias + h), ld(f_bias + h), cap, h};
+  const float qs = 1.0f / sqrtf((float)dim);
   RoundFetch<NS> nxt;
   auto fetch = [&](int t0) {
     const A* base = proj + (int64_t)(row0 + t0) * proj_stride;
@@ -215,29 +287,12 @@ __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict_
     __syncthreads();
     nxt.land(tid, s_q, s_k, s_v);
     if (tid < tc) {
-      const A* pr = proj + (int64_t)(row0 + t0 + tid) * proj_stride;
-      s_i[tid] = cap * tanhf((ld(pr + i_off + h) + ib) / cap);
-      s_f[tid] = logsigmoid_f(cap * tanhf((ld(pr + f_off + h) + fb) / cap));
+      s_i[tid] = gate.in(row0 + t0 + tid);
+      s_f[tid] = gate.forget(row0 + t0 + tid);
     }
     __syncthreads();
     if (t0 + kRecTokens < len) fetch(t0 + kRecTokens);
-    if (tid == 0) {                 // the running maximum is a chain of one add and one max per token: one lane walks it
-      float mm = s_m[0];
-      for (int tt = 0; tt < tc; ++tt) {
-        mm = fmaxf(s_f[tt] + mm, s_i[tt]);
-        s_m[tt + 1] = mm;
-      }
-    }
-    __syncthreads();
-    if (tid < kRecTokens) {         // ... and the exponentials it feeds are computed side by side
-      const bool live = tid < tc;   // rows past the entry's end: a = 1, b = 0 - a step that leaves S and n as they are
-      const float mp = live ? s_m[tid] : 0.f, mn = live ? s_m[tid + 1] : 0.f;
-      s_a[tid] = live ? expf(s_f[tid] + mp - mn) : 1.f;
-      s_b[tid] = live ? expf(s_i[tid] - mn) : 0.f;
-      s_em[tid] = live ? expf(-mn) : 1.f;
-    }
-    __syncthreads();
-    if (tid == 0) s_m[0] = s_m[tc];
+    memory_round(tid, tc, s_i, s_f, s_m, s_a, s_b, s_em);
     float okeep = 0.f;
     // no token waits for the sums of the one before it here (only S and n carry over): four tokens per trip, their sums and
     // quotients in flight together
@@ -268,9 +323,9 @@ __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict_
   for (int i = 0; i < NS; ++i) {
     const int d = r * NS + i;
     if (d < dim && col < vdim) S_g[(int64_t)d * vdim + col] = S[i];
-    if (blockIdx.x == 0 && tid < kRecSlices && d < dim) n_g[d] = n[i];
+    if (gridDim.x == 1 && tid < kRecSlices && d < dim) n_g[d] = n[i];
   }
-  if (blockIdx.x == 0 && tid == 0) *m_g = s_m[0];
+  if (gridDim.x == 1 && tid == 0) *m_g = s_m[0];   // (several workgroups read both: memory_carry_kernel writes them afterwards)
 }
 
 // ---- the matrix memory over long portions (scalar_chunks.h): with the running maxima known, the decays exp(f + m - m') and the factors
@@ -426,6 +481,10 @@ pegainfer_status_t pegainfer_gated_matrix_memory_form(const pegainfer_gated_matr
             proj, q->proj_stride, q->q_off, q->k_off, q->v_off, q->i_off, q->f_off, i_bias, f_bias, q->cap, q->state, q->slot_stride, q->o, H, dim,
             vdim, q->entry_row0, q->entry_slot, chunks ? q->scan_max : 0);
       });
+    if (ok && vdim > kRecCols && q->n_entries > (chunks ? q->n_long : 0))
+      memory_carry_kernel<A><<<dim3(H, q->n_entries), 256, 0, st>>>(proj, q->proj_stride, q->k_off, q->i_off, q->f_off, i_bias, f_bias, q->cap,
+                                                                    q->state, q->slot_stride, H, dim, vdim, q->entry_row0, q->entry_slot,
+                                                                    chunks ? q->scan_max : 0);
     if (!ok || !chunks) return;
     float* gates = q->workspace + scalar_chunk_floats(q->n_chunks, H, dim, vdim, true);
     memory_gates_kernel<A><<<dim3(q->n_long, H), 64, 0, st>>>(proj, q->proj_stride, q->i_off, q->f_off, i_bias, f_bias, q->cap, q->state,

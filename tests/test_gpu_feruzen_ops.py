@@ -295,6 +295,38 @@ def test_attention_finds_one_far_key_among_hundreds_and_stops_at_the_causal_edge
         assert float((out[3] - v[:4].mean(0)).abs().max()) < 1e-4     # the first tokens: equal scores, the mean of what is visible
 
 
+@pytest.mark.parametrize("vdim,steps", [(1040, [1, 1, 2]), (16, [1, 3])])
+def test_matrix_memory_workgroups_of_a_head_read_the_same_norm_and_maximum(vdim, steps):
+    """a head of 1040 values is dealt over 65 workgroups, and 64 x 8 such heads are more than the chip holds at once: workgroups that begin
+    late must not see the vector n and the running maximum that the step leaves"""
+    E, H, d = 64, 8, 16
+    g = torch.Generator().manual_seed(vdim)
+    width = H * (2 * d + vdim + 2)
+    offs = [0, H * d, 2 * H * d, 2 * H * d + H * vdim, 2 * H * d + H * vdim + H]
+    ib, fb = torch.zeros(H), torch.zeros(H)
+    mem = torch.zeros(E, H * (d * vdim + d + 1), device="cuda")
+    S, n, m = torch.zeros(E, H, d, vdim, dtype=torch.float64), torch.zeros(E, H, d, dtype=torch.float64), torch.zeros(E, H, dtype=torch.float64)
+    for k in steps:
+        x = torch.randn(E * k, width, generator=g)
+        got = B().gated_matrix_memory(x.cuda(), offs, ib.cuda(), fb.cuda(), 15.0, mem, H, d, vdim, B().Ragged([k] * E))
+        xd, ref = x.double().view(E, k, width), []
+        for t in range(k):
+            q, kk = xd[:, t, :H * d].view(E, H, d) * d ** -0.5, xd[:, t, H * d:2 * H * d].view(E, H, d)
+            v = xd[:, t, offs[2]:offs[3]].view(E, H, vdim)
+            i = 15 * torch.tanh(xd[:, t, offs[3]:offs[4]] / 15)
+            f = Fn.logsigmoid(15 * torch.tanh(xd[:, t, offs[4]:] / 15))
+            new = torch.maximum(f + m, i)
+            a, b, m = torch.exp(f + m - new), torch.exp(i - new), new
+            S = a[..., None, None] * S + b[..., None, None] * kk[..., None] * v[..., None, :]
+            n = a[..., None] * n + b[..., None] * kk
+            den = torch.maximum((n * q).sum(-1).abs(), torch.exp(-m)) + 1e-6
+            ref.append((S * q[..., None]).sum(-2) / den[..., None])
+        ref = torch.stack(ref, 1).reshape(E * k, H * vdim)
+        close(got, ref, "float32", tol32=2e-5)
+        close(mem[:, H * d * vdim:H * d * (vdim + 1)], n.reshape(E, -1), "float32", tol32=2e-6)
+        close(mem[:, H * d * (vdim + 1):], m, "float32", tol32=2e-6)
+
+
 def test_matrix_memory_keeps_a_far_strong_write_and_resets_with_its_slot():
     """token 4 is written with a large input gate, the forget gates stay open: 500 weak writes later its value still
     dominates the read-out; the same slot, zeroed and used by a second request, must not see any of it"""
