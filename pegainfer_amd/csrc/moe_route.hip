@@ -296,7 +296,9 @@ constexpr int kPlanRows = kSortThreads / 64;
 
 // expert / same: pairs that chose an expert number of same_from or more take the row of `same` (the feed-forward's own input) instead
 // of a y_pairs row
-template <typename A>
+// V columns per thread; up to four pairs' values are on their way at once (fp32 pairs of 1024 rows of 2560, three experts: 23.2 -> 9.8 us,
+// 3421 rows of 1024 22.4 -> 12.3 us against a column and a pair at a time; bound by the pairs' bytes)
+template <typename A, int V>
 __global__ __launch_bounds__(256) void route_combine_kernel(const float* __restrict__ y, const float* __restrict__ w,
                                                             const A* __restrict__ add, A* __restrict__ out, int d, int top,
                                                             const float* __restrict__ add_gate, int64_t add_gate_stride,
@@ -305,16 +307,37 @@ __global__ __launch_bounds__(256) void route_combine_kernel(const float* __restr
                                                             const float* __restrict__ add_pairs, int n_add) {
   const int row = blockIdx.x;
   const float gate = (add || n_add) && add_gate ? sigmoid_f(add_gate[(size_t)row * add_gate_stride]) : 1.0f;
-  for (int i = blockIdx.y * 256 + threadIdx.x; i < d; i += gridDim.y * 256) {
-    float a = add ? ld(add + (size_t)row * d + i) : 0.f;
-    for (int j = 0; j < n_add; ++j) a += add_pairs[((size_t)j * gridDim.x + row) * d + i];
-    a *= gate;
-    for (int c = 0; c < top; ++c) {
-      const bool own = same && expert[(size_t)row * top + c] >= same_from;      // uniform over the workgroup
-      const float v = own ? ld(same + (size_t)row * same_stride + i) : y[((size_t)row * top + c) * d + i];
-      a = fmaf(w[(size_t)row * top + c], v, a);
+  auto load = [&](const auto* p, float* t) {
+    if constexpr (V == 4) ld4(p, t); else t[0] = ld(p);
+  };
+  for (int i = (blockIdx.y * 256 + threadIdx.x) * V; i < d; i += gridDim.y * 256 * V) {
+    float a[V] = {};
+    if (add) load(add + (size_t)row * d + i, a);
+    for (int j = 0; j < n_add; ++j) {
+      float t[V];
+      load(add_pairs + ((size_t)j * gridDim.x + row) * d + i, t);
+#pragma unroll
+      for (int u = 0; u < V; ++u) a[u] += t[u];
     }
-    st(out + (size_t)row * d + i, a);
+#pragma unroll
+    for (int u = 0; u < V; ++u) a[u] *= gate;
+    for (int c0 = 0; c0 < top; c0 += 4) {
+      float v[4][V], wt[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int c = c0 + k;
+        if (c >= top) continue;
+        const bool own = same && expert[(size_t)row * top + c] >= same_from;      // uniform over the workgroup
+        if (own) load(same + (size_t)row * same_stride + i, v[k]); else load(y + ((size_t)row * top + c) * d + i, v[k]);
+        wt[k] = w[(size_t)row * top + c];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (c0 + k < top)
+#pragma unroll
+          for (int u = 0; u < V; ++u) a[u] = fmaf(wt[k], v[k][u], a[u]);
+    }
+    if constexpr (V == 4) st4(out + (size_t)row * d + i, a); else st(out + (size_t)row * d + i, a[0]);
   }
 }
 
@@ -435,11 +458,17 @@ static pegainfer_status_t combine_launch(const float* y_pairs, const float* weig
   if (same && !expert) return (pegainfer_status_t)hipErrorInvalidValue;
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        // few rows (decoding): the row is cut over several workgroups
-        const dim3 grid(rows, rows >= 256 ? 1 : std::min(16, ceil_div(d, 256)));
-        route_combine_kernel<A><<<grid, 256, 0, as_stream(stream)>>>(y_pairs, weight, static_cast<const A*>(add), static_cast<A*>(out), d,
-                                                                     top, add_gate, add_gate_stride, expert, same_from,
-                                                                     static_cast<const A*>(same), same_stride, add_pairs, n_add);
+        auto go = [&](auto kern, int per_row) {
+          kern<<<dim3(rows, per_row), 256, 0, as_stream(stream)>>>(y_pairs, weight, static_cast<const A*>(add), static_cast<A*>(out), d, top,
+                                                                   add_gate, add_gate_stride, expert, same_from,
+                                                                   static_cast<const A*>(same), same_stride, add_pairs, n_add);
+        };
+        // many rows: four columns per thread where rows and pointers allow it; few rows (decoding) are cut over as many threads as there
+        // are columns
+        const bool vec = d % 4 == 0 && (!same || same_stride % 4 == 0) && host_aligned16(y_pairs) && host_aligned16(add) &&
+                         host_aligned16(same) && host_aligned16(add_pairs) && host_aligned16(out);
+        if (vec && rows >= 256) go(route_combine_kernel<A, 4>, std::min(16, ceil_div(d, 1024)));
+        else go(route_combine_kernel<A, 1>, rows >= 256 ? 1 : std::min(16, ceil_div(d, 256)));
       }))
     return (pegainfer_status_t)hipErrorInvalidValue;
   return (pegainfer_status_t)hipGetLastError();

@@ -5,7 +5,6 @@
 //                           oldest first, so it never reads what it has already written)
 //   group_rms_add_kernel    RMS norm in equal consecutive groups of a sublayer's OUTPUT, the residual sum, and a weighted
 //                           sum over the streams of earlier layers (depth-weighted averaging) in one pass over the row
-//   clamp_glu_rows_kernel   g = min(gate, L), u = clamp(up, -L, L):  g sigmoid(alpha g) (u + 1)
 //   head_rms_gate_kernel    per-head RMS norm of a read-out * weight * silu / sigmoid gate * constant
 //   scalar_rms_add_kernel   residual sum with a constant factor (+ bias, + extra rows, + one extra vector), then an RMS norm
 //                           whose gain is a single number
@@ -16,7 +15,8 @@
 //                           addressed by the previous and the current token)
 //   join_rms_kernel         one normed output joins the stream in place and the next norm follows, with everything a row needs in
 //                           registers from the start; the output may be the weighted sum of routed experts, made on the way
-//   glu_rows_kernel         act(gate) * up from two column ranges of a wider row (silu, relu, tanh-gelu or erf-gelu)
+//   glu_rows_kernel         act(gate) * up from two column ranges of a wider row (silu, relu, tanh-gelu or erf-gelu); or, from one row,
+//                           g = min(gate, L), u = clamp(up, -L, L):  g sigmoid(alpha g) (u + 1)
 //   act_rows_kernel         the same activations alone
 //   softcap_rows_kernel     cap * tanh(x / cap) on fp32 rows
 #include <algorithm>
@@ -58,7 +58,11 @@ __global__ __launch_bounds__(256) void time_conv_kernel(const I* __restrict__ in
 // step; while it stays inside an entry each row costs ONE load (the window slides), the taps' weights stay in registers.
 // Window and weights are right-aligned (slot KMAX - 1 = the current row) and summed oldest first, the order of the plain
 // kernel; slots beyond the taps hold weight 0 and input 0.
-constexpr int kConvRows = 32;
+// A walk is as long as the rows that a thread can have on their way at once: all its rows (and their entry numbers) are requested before the
+// first is used.  Walks of 32 rows that asked for one row at a time waited for memory once per row: 1024 rows of 2560 channels 16.1 -> 8.0 us,
+// of 8192 channels 20.9 -> 19.8 us (two channels per thread: 9.5 and 18.6).
+constexpr int kConvRows = 8;
+constexpr int kConvWindowFrom = 128;   // rows from which walks fill the chip better than a thread per (row, channel)
 template <typename I, typename W, typename O, int KMAX>
 __global__ __launch_bounds__(256) void time_conv_window_kernel(const I* __restrict__ in, int64_t in_stride,
                                                                const W* __restrict__ w, const float* __restrict__ state,
@@ -70,6 +74,15 @@ __global__ __launch_bounds__(256) void time_conv_window_kernel(const I* __restri
                                                                const W* __restrict__ in_bias, const W* __restrict__ out_bias) {
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= C) return;
+  const int row_begin = blockIdx.x * kConvRows, rows = min(n_rows - row_begin, kConvRows);
+  float x[kConvRows];
+  int entry[kConvRows];
+#pragma unroll
+  for (int k = 0; k < kConvRows; ++k) {
+    const int row = row_begin + min(k, rows - 1);
+    x[k] = ld(in + (int64_t)row * in_stride + c);
+    entry[k] = row_entry[row];
+  }
   const float ib = in_bias ? ld(in_bias + c) : 0.f, ob = out_bias ? ld(out_bias + c) : 0.f;
   float wr[KMAX], win[KMAX];
 #pragma unroll
@@ -78,10 +91,11 @@ __global__ __launch_bounds__(256) void time_conv_window_kernel(const I* __restri
     wr[j] = t < K ? ld(w + (int64_t)c * K + (K - 1 - t)) : 0.f;
     win[j] = 0.f;
   }
-  const int row_begin = blockIdx.x * kConvRows, row_end = min(n_rows, row_begin + kConvRows);
   int cur_e = -1;
-  for (int row = row_begin; row < row_end; ++row) {
-    const int e = row_entry[row];
+#pragma unroll
+  for (int k = 0; k < kConvRows; ++k) {
+    if (k >= rows) break;
+    const int row = row_begin + k, e = entry[k];
     if (e != cur_e) {             // first row of this walk inside the entry: fill the window's past from rows or the tail
       cur_e = e;
       const int r0 = entry_row0[e], local = row - r0;
@@ -95,7 +109,7 @@ __global__ __launch_bounds__(256) void time_conv_window_kernel(const I* __restri
     }
 #pragma unroll
     for (int j = 0; j < KMAX - 1; ++j) win[j] = win[j + 1];
-    const float cur = ld(in + (int64_t)row * in_stride + c) + ib;
+    const float cur = x[k] + ib;
     win[KMAX - 1] = cur;
     float acc = 0.f;
 #pragma unroll
@@ -223,17 +237,6 @@ __global__ __launch_bounds__(256) void group_rms_add_kernel(const float* x_in, c
   }
 }
 
-template <typename A>
-__global__ __launch_bounds__(256) void clamp_glu_rows_kernel(const A* __restrict__ gu, A* __restrict__ out, int I, float limit,
-                                                             float alpha) {
-  const int row = blockIdx.x;
-  const int i = blockIdx.y * 256 + threadIdx.x;
-  if (i >= I) return;
-  const float g = fminf(ld(gu + (int64_t)row * 2 * I + i), limit);
-  const float u = fminf(fmaxf(ld(gu + (int64_t)row * 2 * I + I + i), -limit), limit);
-  st(out + (int64_t)row * I + i, g * sigmoid_f(alpha * g) * (u + 1.0f));
-}
-
 // The norm-and-gate below for heads wider than a wave should walk alone (one norm over a whole row, say): a workgroup per (row, head).
 // VEC: rows, strides and pointers allow four values per load.
 constexpr int kWideKeep = 4;
@@ -305,33 +308,53 @@ __global__ __launch_bounds__(256) void wide_rms_gate_kernel(const float* __restr
   }
 }
 
-// one wave per (row, head)
-template <typename A>
+// One wave per (row, head), vdim <= 512; a lane's values, gates and weights are all requested before the first is used, V at a time.  Bound by
+// memory with many heads, by the launch with few: 8192 x 4 heads of 128 16.5 -> 12.6 us, one row of four groups of 512 9.7 -> 4.6 us (read
+// value by value and a second time for the output before).
+template <typename A, int V>
 __global__ __launch_bounds__(256) void head_rms_gate_kernel(const float* __restrict__ o, const A* __restrict__ w, int w_per_head,
                                                             const A* __restrict__ gate, int64_t gate_stride, int gate_kind,
                                                             float factor, float eps, A* __restrict__ out, int64_t out_stride,
                                                             int heads, int vdim, int rows, int gate_first) {
+  constexpr int K = 8 / V;
   const int64_t rh = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (rh >= (int64_t)rows * heads) return;
   const int row = (int)(rh / heads), h = (int)(rh % heads);
   const float* p = o + ((int64_t)row * heads + h) * vdim;
   const A* gr = gate + (int64_t)row * gate_stride + (int64_t)h * vdim;
-  auto act = [&](int i) {
-    const float z = ld(gr + i);
-    return gate_kind == 0 ? silu_f(z) : sigmoid_f(z);
+  const A* wr = w + (w_per_head ? (int64_t)h * vdim : 0);
+  A* dst = out + (int64_t)row * out_stride + (int64_t)h * vdim;
+  auto load = [&](const auto* q, float* t) {
+    if constexpr (V == 4) ld4(q, t); else if constexpr (V == 2) ld2(q, t); else t[0] = ld(q);
   };
-  float ss = 0.f;
-  for (int i = lane; i < vdim; i += 64) {
-    const float v = gate_first ? p[i] * act(i) : p[i];   // gate_first: the gated values are what is normed
-    ss = fmaf(v, v, ss);
+  float v[K][V], z[K][V], wv[K][V];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = (lane + 64 * k) * V;
+    if (i < vdim) { load(p + i, v[k]); load(gr + i, z[k]); load(wr + i, wv[k]); }
   }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if ((lane + 64 * k) * V < vdim)
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        z[k][u] = gate_kind == 0 ? silu_f(z[k][u]) : sigmoid_f(z[k][u]);
+        if (gate_first) v[k][u] *= z[k][u];   // gate_first: the gated values are what is normed
+        ss = fmaf(v[k][u], v[k][u], ss);
+      }
   ss = wave_sum(ss);
   const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
-  for (int i = lane; i < vdim; i += 64) {
-    const float wv = ld(w + (w_per_head ? h * vdim : 0) + i);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = (lane + 64 * k) * V;
+    if (i >= vdim) continue;
+    float r[V];
     // (each order keeps its own sequence of roundings: norm, weight, gate, factor - or gate, norm, weight, factor)
-    st(out + (int64_t)row * out_stride + h * vdim + i, gate_first ? p[i] * act(i) * inv * wv * factor : p[i] * inv * wv * act(i) * factor);
+#pragma unroll
+    for (int u = 0; u < V; ++u) r[u] = gate_first ? v[k][u] * inv * wv[k][u] * factor : v[k][u] * inv * wv[k][u] * z[k][u] * factor;
+    if constexpr (V == 4) st4(dst + i, r); else if constexpr (V == 2) st2(dst + i, r); else st(dst + i, r[0]);
   }
 }
 
@@ -636,15 +659,53 @@ __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, Join
   }
 }
 
-// out[row, i] = act(gate[row, i]) * up[row, i]; gate and up are column ranges of rows with one stride
-template <typename A>
+// Gated linear units: out[row, i] = F(gate[row, i], up[row, i]); gate and up are column ranges of rows with one stride.  The rows' values are
+// numbered through, V to a thread, so that no lane idles at a row's end.  Bound by memory with many values (eight to a thread: pairs of a
+// 2404-row feed-forward 22.1 -> 13.1 us, 1024 rows of 9216 17.3 -> 14.1 us, of 6144 11.6 -> 8.2 us against a value per thread), by the launch
+// with few.
+enum : int { kGluAct = 0, kGluSilu = 1, kGluClamp = 2 };
+struct GluForm { int act; float limit, alpha; };
+template <int F>
+__device__ __forceinline__ float glu_f(const GluForm& q, float g, float u) {
+  if constexpr (F == kGluAct) return act_f(q.act, g) * u;
+  if constexpr (F == kGluSilu) return g * sigmoid_f(g) * u;
+  g = fminf(g, q.limit);
+  u = fminf(fmaxf(u, -q.limit), q.limit);
+  return g * sigmoid_f(q.alpha * g) * (u + 1.0f);
+}
+template <typename A, int F, int V>
 __global__ __launch_bounds__(256) void glu_rows_kernel(const A* __restrict__ gate, const A* __restrict__ up, int64_t in_stride,
-                                                       A* __restrict__ out, int64_t out_stride, int I, int act) {
-  const int row = blockIdx.x;
-  const int i = blockIdx.y * 256 + threadIdx.x;
-  if (i >= I) return;
-  const float g = ld(gate + (int64_t)row * in_stride + i), u = ld(up + (int64_t)row * in_stride + i);
-  st(out + (int64_t)row * out_stride + i, act_f(act, g) * u);
+                                                       A* __restrict__ out, int64_t out_stride, uint32_t per_row, uint32_t n, GluForm q) {
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= n) return;
+  const uint32_t row = t / per_row, i = (t - row * per_row) * V;
+  const A *gr = gate + (int64_t)row * in_stride + i, *ur = up + (int64_t)row * in_stride + i;
+  A* o = out + (int64_t)row * out_stride + i;
+  if constexpr (V == 8) {
+    float g[8], u[8];
+    Vec8<A>::load(gr, g);
+    Vec8<A>::load(ur, u);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] = glu_f<F>(q, g[k], u[k]);
+    Vec8<A>::store(o, g);
+  } else {
+    st(o, glu_f<F>(q, ld(gr), ld(ur)));
+  }
+}
+// Eight values per thread where rows, strides and pointers allow 16-byte accesses and that still leaves a wave for each SIMD.
+template <typename A, int F>
+void launch_glu(const A* gate, const A* up, int64_t in_stride, A* out, int64_t out_stride, int I, int rows, const GluForm& q, hipStream_t stream) {
+  const bool wide = (int64_t)rows * I >= 8 * 64 * 1024 && I % 8 == 0 && in_stride % 8 == 0 && out_stride % 8 == 0 && host_aligned16(gate) &&
+                    host_aligned16(up) && host_aligned16(out);
+  const int per_row = wide ? I / 8 : I;
+  const int slab = std::max(1, (1 << 30) / per_row);   // rows whose values one launch can number
+  for (int r = 0; r < rows; r += slab) {
+    const uint32_t n = (uint32_t)std::min(slab, rows - r) * (uint32_t)per_row;
+    const A *g = gate + (int64_t)r * in_stride, *u = up + (int64_t)r * in_stride;
+    A* o = out + (int64_t)r * out_stride;
+    if (wide) glu_rows_kernel<A, F, 8><<<ceil_div(n, 256), 256, 0, stream>>>(g, u, in_stride, o, out_stride, per_row, n, q);
+    else glu_rows_kernel<A, F, 1><<<ceil_div(n, 256), 256, 0, stream>>>(g, u, in_stride, o, out_stride, per_row, n, q);
+  }
 }
 
 // out[row, i] = act(in[row, i]) (in place allowed); V values per thread
@@ -794,11 +855,22 @@ pegainfer_status_t pegainfer_glu_rows(const void* gate, const void* up, int64_t 
                                       int32_t I, int32_t rows, int32_t act, int32_t dtype, pegainfer_stream_t stream) {
   if (rows <= 0 || I <= 0) return 0;
   if (act < 0 || act > PEGAINFER_ACT_GELU_ERF) return PK_BAD;
-  const dim3 grid(rows, ceil_div(I, 256));
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        glu_rows_kernel<A><<<grid, 256, 0, as_stream(stream)>>>(static_cast<const A*>(gate), static_cast<const A*>(up), in_row_stride,
-                                                                static_cast<A*>(out), out_row_stride, I, act);
+        launch_glu<A, kGluAct>(static_cast<const A*>(gate), static_cast<const A*>(up), in_row_stride, static_cast<A*>(out), out_row_stride, I,
+                               rows, GluForm{act, 0.f, 0.f}, as_stream(stream));
+      }))
+    return PK_BAD;
+  return (pegainfer_status_t)hipGetLastError();
+}
+
+pegainfer_status_t pegainfer_silu_mul_rows(const void* gate_up, void* out, int32_t I, int32_t rows, int32_t dtype,
+                                           pegainfer_stream_t stream) {
+  if (rows <= 0 || I <= 0) return 0;
+  if (!by_dtype(dtype, [&](auto* t) {
+        using A = std::remove_pointer_t<decltype(t)>;
+        const A* g = static_cast<const A*>(gate_up);
+        launch_glu<A, kGluSilu>(g, g + I, 2 * (int64_t)I, static_cast<A*>(out), I, I, rows, GluForm{}, as_stream(stream));
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();
@@ -835,17 +907,14 @@ pegainfer_status_t pegainfer_time_conv_biased(const void* in, int32_t in_dtype, 
            using W = std::remove_pointer_t<decltype(tw)>;
            ok = by_dtype(out_dtype, [&](auto* to) {
                   using O = std::remove_pointer_t<decltype(to)>;
-                  const dim3 wgrid(ceil_div(n_rows, kConvRows), ceil_div(channels, 256));
-                  if (n_rows >= 4 * kConvRows && taps <= 4)
-                    time_conv_window_kernel<I, W, O, 4><<<wgrid, 256, 0, as_stream(stream)>>>(
+                  auto window = [&](auto kern) {
+                    kern<<<dim3(ceil_div(n_rows, kConvRows), ceil_div(channels, 256)), 256, 0, as_stream(stream)>>>(
                         static_cast<const I*>(in), in_row_stride, static_cast<const W*>(w), state, slot_stride,
                         static_cast<O*>(out), out_row_stride, channels, taps, mode, n_rows, row_entry, entry_row0, entry_slot,
                         static_cast<const W*>(in_bias), static_cast<const W*>(out_bias));
-                  else if (n_rows >= 4 * kConvRows && taps <= 8)
-                    time_conv_window_kernel<I, W, O, 8><<<wgrid, 256, 0, as_stream(stream)>>>(
-                        static_cast<const I*>(in), in_row_stride, static_cast<const W*>(w), state, slot_stride,
-                        static_cast<O*>(out), out_row_stride, channels, taps, mode, n_rows, row_entry, entry_row0, entry_slot,
-                        static_cast<const W*>(in_bias), static_cast<const W*>(out_bias));
+                  };
+                  if (n_rows >= kConvWindowFrom && taps <= 4) window(time_conv_window_kernel<I, W, O, 4>);
+                  else if (n_rows >= kConvWindowFrom && taps <= 8) window(time_conv_window_kernel<I, W, O, 8>);
                   else
                     time_conv_kernel<I, W, O><<<grid, 256, 0, as_stream(stream)>>>(
                         static_cast<const I*>(in), in_row_stride, static_cast<const W*>(w), state, slot_stride,
@@ -947,11 +1016,10 @@ pegainfer_status_t pegainfer_group_rms_add(const float* x_in, const void* y, int
 pegainfer_status_t pegainfer_clamp_glu_rows(const void* gate_up, void* out, int32_t I, int32_t rows, float limit, float alpha,
                                             int32_t dtype, pegainfer_stream_t stream) {
   if (rows <= 0 || I <= 0) return 0;
-  const dim3 grid(rows, ceil_div(I, 256));
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        clamp_glu_rows_kernel<A><<<grid, 256, 0, as_stream(stream)>>>(static_cast<const A*>(gate_up), static_cast<A*>(out), I,
-                                                                      limit, alpha);
+        const A* g = static_cast<const A*>(gate_up);
+        launch_glu<A, kGluClamp>(g, g + I, 2 * (int64_t)I, static_cast<A*>(out), I, I, rows, GluForm{0, limit, alpha}, as_stream(stream));
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();
@@ -986,10 +1054,16 @@ pegainfer_status_t pegainfer_head_gate_rms(const float* o, const void* w, int32_
           else wide(wide_rms_gate_kernel<A, false>);
           return;
         }
-        head_rms_gate_kernel<A><<<blocks, 256, 0, as_stream(stream)>>>(o, static_cast<const A*>(w), w_per_head,
-                                                                       static_cast<const A*>(gate), gate_stride, gate_kind,
-                                                                       factor, eps, static_cast<A*>(out), out_stride, heads,
-                                                                       vdim, rows, gate_first);
+        // as many values per access as rows, strides and pointers allow, without leaving lanes of a narrow head idle
+        const bool aligned = gate_stride % 4 == 0 && out_stride % 4 == 0 && host_aligned16(o) && host_aligned16(w) && host_aligned16(gate) &&
+                             host_aligned16(out);
+        auto narrow = [&](auto kern) {
+          kern<<<blocks, 256, 0, as_stream(stream)>>>(o, static_cast<const A*>(w), w_per_head, static_cast<const A*>(gate), gate_stride,
+                                                      gate_kind, factor, eps, static_cast<A*>(out), out_stride, heads, vdim, rows, gate_first);
+        };
+        if (aligned && vdim % 4 == 0 && vdim > 128) narrow(head_rms_gate_kernel<A, 4>);
+        else if (aligned && vdim % 4 == 0 && vdim > 64) narrow(head_rms_gate_kernel<A, 2>);
+        else narrow(head_rms_gate_kernel<A, 1>);
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();

@@ -32,6 +32,9 @@ struct Vec8<uint16_t> {
     o[0] = bf_lo(v.x); o[1] = bf_hi(v.x); o[2] = bf_lo(v.y); o[3] = bf_hi(v.y);
     o[4] = bf_lo(v.z); o[5] = bf_hi(v.z); o[6] = bf_lo(v.w); o[7] = bf_hi(v.w);
   }
+  static __device__ __forceinline__ void store(uint16_t* p, const float* o) {
+    *reinterpret_cast<u32x4*>(p) = u32x4{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]), pack_bf2(o[4], o[5]), pack_bf2(o[6], o[7])};
+  }
 };
 template <>
 struct Vec8<float> {
@@ -40,7 +43,19 @@ struct Vec8<float> {
     const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
     o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
   }
+  static __device__ __forceinline__ void store(float* p, const float* o) {
+    *reinterpret_cast<f32x4*>(p) = f32x4{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<f32x4*>(p + 4) = f32x4{o[4], o[5], o[6], o[7]};
+  }
 };
+// two consecutive values (8-byte aligned for fp32, 4-byte for bf16)
+__device__ __forceinline__ void ld2(const float* p, float* o) { const f32x2 v = *reinterpret_cast<const f32x2*>(p); o[0] = v.x; o[1] = v.y; }
+__device__ __forceinline__ void ld2(const uint16_t* p, float* o) {
+  const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
+  o[0] = bf_lo(v); o[1] = bf_hi(v);
+}
+__device__ __forceinline__ void st2(float* p, const float* o) { *reinterpret_cast<f32x2*>(p) = f32x2{o[0], o[1]}; }
+__device__ __forceinline__ void st2(uint16_t* p, const float* o) { *reinterpret_cast<uint32_t*>(p) = pack_bf2(o[0], o[1]); }
 // four consecutive values (16-byte aligned for fp32, 8-byte for bf16)
 __device__ __forceinline__ void ld4(const float* p, float* o) { const f32x4 v = *reinterpret_cast<const f32x4*>(p); o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w; }
 __device__ __forceinline__ void ld4(const uint16_t* p, float* o) {

@@ -101,6 +101,73 @@ def test_gate_before_the_norm_in_groups(dtype, shape):
     close(got, R.rms(o.double().view(9, heads, vd), 1e-6).reshape(9, -1) * w.double() * R.silu(z[:, 3:].double()), dtype, tol16=2e-2)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows,I", [(1024, 512), (1023, 520), (13109, 40), (700, 750)])
+def test_many_gated_units_eight_values_to_a_thread(dtype, rows, I):
+    # at, just above and below the 2^19 values from which a thread takes eight; 750 is no multiple of eight.  One stored rounding (2^-9 of
+    # the value) plus a few fp32 ones
+    g = torch.Generator().manual_seed(I)
+    gu = C.bf16_round(torch.randn(rows, 2 * I, generator=g) * 2)
+    d, gate, up = dev(gu, dtype), gu[:, :I].double(), gu[:, I:].double()
+    silu = gate * torch.sigmoid(gate) * up
+    close(B().silu_mul_rows(d), silu, dtype, tol32=2e-6, tol16=4e-3)
+    close(B().glu_rows(d[:, :I], d[:, I:], "silu"), silu, dtype, tol32=2e-6, tol16=4e-3)
+    ga = gate.clamp(max=1.25)
+    close(B().clamp_glu_rows(d, 1.25), ga * torch.sigmoid(1.702 * ga) * (up.clamp(-1.25, 1.25) + 1), dtype, tol32=2e-6, tol16=4e-3)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows,d,top", [(256, 1028, 5), (255, 1028, 4), (300, 1026, 1), (300, 64, 8)])
+def test_routed_sum_four_columns_to_a_thread(dtype, rows, d, top):
+    g = torch.Generator().manual_seed(d + top)
+    y, w = torch.randn(rows * top, d, generator=g), torch.rand(rows, top, generator=g)
+    add, lg = C.bf16_round(torch.randn(rows, d, generator=g)), torch.randn(rows, generator=g)
+    got = B().route_combine_gated(y.cuda(), w.cuda(), dev(add, dtype), lg.cuda(), DT[dtype])
+    ref = torch.sigmoid(lg.double())[:, None] * add.double() + (w.double()[:, :, None] * y.double().view(rows, top, d)).sum(1)
+    close(got, ref, dtype, tol32=2e-6, tol16=4e-3)                      # one stored rounding, top + 2 fp32 ones
+    got = B().route_combine_pairs(y.cuda(), w.cuda(), torch.stack([y[:rows], y[-rows:]]).cuda(), None, DT[dtype])
+    close(got, y[:rows].double() + y[-rows:].double() + (w.double()[:, :, None] * y.double().view(rows, top, d)).sum(1), dtype, tol32=2e-6, tol16=4e-3)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,vd", [(3, 64), (2, 68), (3, 96), (5, 128), (2, 132), (4, 512), (2, 508), (3, 37)])
+def test_norm_and_gate_of_heads_several_values_to_a_lane(dtype, heads, vd):
+    g = torch.Generator().manual_seed(vd)
+    n = heads * vd
+    o, z, w = torch.randn(7, n, generator=g), C.bf16_round(torch.randn(7, n, generator=g)), C.bf16_round(1 + 0.2 * torch.randn(n, generator=g))
+    zd, normed = dev(z, dtype), R.rms(o.double().view(7, heads, vd), 1e-6).reshape(7, -1)
+    close(B().head_gate_rms(o.cuda(), dev(w, dtype), zd, "silu", 1e-6, heads, vd, gate_first=False), normed * w.double() * R.silu(z.double()),
+          dtype, tol32=4e-6, tol16=4e-3)                                # one stored rounding, fp32 before it
+    gated = (o.double() * R.silu(z.double())).view(7, heads, vd)
+    close(B().head_gate_rms(o.cuda(), dev(w, dtype), zd, "silu", 1e-6, heads, vd, gate_first=True),
+          R.rms(gated, 1e-6).reshape(7, -1) * w.double(), dtype, tol32=4e-6, tol16=4e-3)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("channels,taps", [(301, 4), (514, 3), (513, 8), (1026, 5)])
+def test_convolution_of_long_portions_in_walks_of_eight_rows(dtype, channels, taps):
+    g = torch.Generator().manual_seed(channels)
+    w, lens = C.bf16_round(torch.randn(channels, taps, generator=g)), (130, 5, 1, 77)      # entries end inside a walk of eight rows
+    x = C.bf16_round(torch.randn(sum(lens), channels, generator=g))
+    state = torch.randn(4, taps - 1, channels, generator=g)
+    out = B().time_conv(dev(x, dtype), dev(w, dtype), state.cuda(), B().Ragged(list(lens), slots=[2, 0, 3, 1]), silu=True, out_dtype=torch.float32)
+    at = 0
+    for n, slot in zip(lens, (2, 0, 3, 1)):
+        past = torch.cat([state[slot].double(), x[at:at + n].double()])
+        ref = sum(past[j:j + n] * w[:, j].double() for j in range(taps))
+        close(out[at:at + n], R.silu(ref), "float32", tol32=2e-6)
+        at += n
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n", [7, 1 << 19, (1 << 19) + 5])
+def test_squared_relu(dtype, n):
+    x = C.bf16_round(torch.randn(n, generator=torch.Generator().manual_seed(n)))
+    ref = torch.relu(x.double()) ** 2
+    got = B().relu_sq(dev(x, dtype)).double().cpu()
+    assert float(((got - ref).abs() - 2.0 ** -8 * ref).max()) <= 0       # at most one stored rounding
+
+
 # ------------------------------------------------------------------ time convolution with biases
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps", [1, 2, 4, 7])
