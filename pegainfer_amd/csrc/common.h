@@ -108,6 +108,7 @@ __device__ __forceinline__ float block_sum(float v, float* smem /* >= WAVES floa
 __device__ __forceinline__ bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
+inline bool host_aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 inline bool host_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline hipStream_t as_stream(pegainfer_stream_t s) { return reinterpret_cast<hipStream_t>(s); }

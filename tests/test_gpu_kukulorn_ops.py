@@ -295,6 +295,53 @@ def test_convolved_rotated_capped_attention_whole_and_in_portions(dtype, layer):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,H,G,d,dv,rot,kind", [(3, 5, 2, 66, 34, 66, "all_weight"), (520, 3, 1, 6, 10, 2, "head_weight"), (513, 6, 5, 128, 256, 64, "all_weight"),
+                                                 (2, 9, 9, 256, 130, 256, "head_unit_after"), (2, 4, 1, 64, 3, 0, "head_weight")])
+def test_heads_are_prepared_alike_one_or_two_values_to_a_lane(dtype, n, H, G, d, dv, rot, kind):
+    """the same rows from an even column on (two values to a lane, unless a size is odd) and from an odd one, against float64"""
+    Bk = B()
+    g = torch.Generator().manual_seed(n + d)
+    cols = (H + G) * d + G * dv
+    x = C.bf16_round(torch.randn(n, cols, generator=g))
+    bias = C.bf16_round(torch.randn(cols, generator=g))
+    qn, kn = (H * d, G * d) if kind == "all_weight" else (d, d)
+    qw, kw = C.bf16_round(1 + 0.2 * torch.randn(qn, generator=g)), C.bf16_round(1 + 0.2 * torch.randn(kn, generator=g))
+    inv = torch.rand(max(rot // 2, 1), generator=g) / 4
+    ang = torch.arange(n, dtype=torch.float64)[:, None, None] * inv.double()
+    ref = (x + bias).double() if dtype == "float32" else (x.double() + bias.double())
+    heads = []
+    for t, w, k in ((ref[:, :H * d].view(n, H, d), qw, H), (ref[:, H * d:(H + G) * d].view(n, G, d), kw, G)):
+        if kind == "all_weight":
+            t = R.rms(t.reshape(n, -1), 1e-6).view(n, k, d) * w.double().view(k, d)
+        elif kind == "head_weight":
+            t = R.rms(t, 1e-6) * w.double()
+        if rot:
+            a, b = t[..., :rot // 2], t[..., rot // 2:rot]
+            cs, sn = torch.cos(ang), torch.sin(ang)
+            t = torch.cat([a * cs - b * sn, b * cs + a * sn, t[..., rot:]], -1)
+        heads.append(R.rms(t, 1e-6) if kind == "head_unit_after" else t)
+    rg = Bk.Ragged([n])
+    for shift in (0, 1):
+        pc = Paged(list(range((n + 15) // 16))[::-1], G, d, dv, dtype)
+        pc.page_stride -= 1 - shift                   # the helper's pages are an odd number of values apart
+        proj = torch.zeros(n, cols + 4, dtype=DT[dtype], device="cuda")
+        proj[:, shift:shift + cols] = dev(x, dtype)
+        b = dev(bias, dtype)
+        q = Bk.qk_prep_paged_form(proj, [shift, shift + H * d, shift + (H + G) * d], H, G, d, dv, rg, pc.indptr, pc.pids, pc.cache, pc.page_stride,
+                                  pc.k_off, pc.v_off, 16, q_norm=None if kind == "head_unit_after" else dev(qw, dtype),
+                                  k_norm=None if kind == "head_unit_after" else dev(kw, dtype), norm_kind=kind, eps=1e-6, q_bias=b[:H * d],
+                                  k_bias=b[H * d:(H + G) * d].clone(), v_bias=b[(H + G) * d:].clone(), inv_freq=inv.cuda(), rot_dims=rot, halves=True)
+        close(q, heads[0], "float32", tol32=3e-5)     # fp32 angles up to 130 are off by 2^-24 of that: 8e-6 of a value
+        flat = pc.cache.view(-1).double().cpu()
+        page = pc.pids.cpu().long()
+        rows = [(int(page[i // 16]) * pc.page_stride, i % 16) for i in range(n)]
+        keys = torch.stack([flat[o + pc.k_off + sl * G * d:o + pc.k_off + (sl + 1) * G * d] for o, sl in rows])
+        vals = torch.stack([flat[o + pc.v_off + sl * G * dv:o + pc.v_off + (sl + 1) * G * dv] for o, sl in rows])
+        close(keys, heads[1].reshape(n, -1), dtype, tol32=3e-5, tol16=4e-3)
+        close(vals, ref[:, (H + G) * d:], dtype, tol32=1e-6, tol16=4e-3)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("layer", [("a", 0), ("a", 3), ("wide", 1), ("odd", 1), ("odd", 2), ("b", 1)])
 def test_windowed_biased_attention_whole_and_in_portions(dtype, layer):
     cfg = C.CONFIGS[layer[0]]()
