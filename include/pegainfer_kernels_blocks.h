@@ -26,6 +26,9 @@ enum { PEGAINFER_ROT_PAIRS = 0, PEGAINFER_ROT_HALVES = 1 };
 /* out[t, :] = embed[token_ids[t], :] widened to fp32 */
 pegainfer_status_t pegainfer_embed_f32(const void* embed, const uint32_t* token_ids, float* out, int32_t width,
                                        int32_t n_tokens, int32_t dtype, pegainfer_stream_t stream);
+/* the same rows into out (may be NULL) and into both halves of pair [n_tokens][2 * width] */
+pegainfer_status_t pegainfer_embed_f32_pair(const void* embed, const uint32_t* token_ids, float* out, float* pair, int32_t width,
+                                            int32_t n_tokens, int32_t dtype, pegainfer_stream_t stream);
 /* Dynamic Tanh: out = tanh(alpha * x) * w + b.  x fp32 [rows, d]; alpha a one-element tensor, w / b [d]; out [rows, d] */
 pegainfer_status_t pegainfer_dyt_norm(const float* x, const void* alpha, const void* w, const void* b, void* out,
                                       int32_t d, int32_t rows, int32_t dtype, pegainfer_stream_t stream);
@@ -472,6 +475,20 @@ pegainfer_status_t pegainfer_act_rows(const void* in, int64_t in_row_stride, voi
                                       int32_t act, int32_t dtype, pegainfer_stream_t stream);
 pegainfer_status_t pegainfer_glu_rows(const void* gate, const void* up, int64_t in_row_stride, void* out, int64_t out_row_stride,
                                       int32_t I, int32_t rows, int32_t act, int32_t dtype, pegainfer_stream_t stream);
+/* A decode step's time convolution (as pegainfer_time_conv_step_biased, in and w of one storage type, fp32 out) and, from the same
+ * projected rows, glu_out[e, i] = act(gate[e, i]) * up[e, i], in one launch */
+typedef struct {
+  const void* in; int64_t in_row_stride;      /* also the stride of gate and up */
+  const void *w, *in_bias, *out_bias;
+  float* state; int64_t slot_stride;
+  float* out; int64_t out_row_stride;
+  int32_t channels, taps, mode;
+  const int32_t* entry_slot;
+  const void *gate, *up;
+  void* glu_out; int64_t glu_row_stride;
+  int32_t I, act, n_entries, dtype;
+} pegainfer_conv_glu_step_desc;
+pegainfer_status_t pegainfer_conv_glu_step(const pegainfer_conv_glu_step_desc* q, pegainfer_stream_t stream);
 /* dst (device) <- the first *pinned_count 32-bit words of pinned_src, both read when the launch runs (a captured one: at every replay).  Source and
  * count lie in pinned, coherent host memory; source and destination hold a multiple of four words, PEGAINFER_FETCH_WORDS at least, and start
  * on 16 bytes. */

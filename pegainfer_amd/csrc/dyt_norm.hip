@@ -22,6 +22,18 @@ __global__ __launch_bounds__(256) void embed_f32_kernel(const A* __restrict__ em
   for (int i = threadIdx.x; i < width; i += 256) dst[i] = ld(src + i);
 }
 
+// (beside the stream itself, both halves of the rows that a projection of [stream | embedding] reads: one launch for three)
+template <typename A>
+__global__ __launch_bounds__(256) void embed_f32_pair_kernel(const A* __restrict__ embed, const uint32_t* __restrict__ ids,
+                                                             float* __restrict__ out, float* __restrict__ pair, int width) {
+  const int i = blockIdx.y * 256 + threadIdx.x;
+  if (i >= width) return;
+  const float v = ld(embed + (size_t)ids[blockIdx.x] * width + i);
+  if (out) out[(size_t)blockIdx.x * width + i] = v;
+  pair[(size_t)blockIdx.x * 2 * width + i] = v;
+  pair[(size_t)blockIdx.x * 2 * width + width + i] = v;
+}
+
 template <typename A>
 __global__ __launch_bounds__(256) void dyt_norm_kernel(const float* __restrict__ x, const A* __restrict__ alpha,
                                                        const A* __restrict__ w, const A* __restrict__ b,
@@ -143,6 +155,19 @@ pegainfer_status_t pegainfer_embed_f32(const void* embed, const uint32_t* token_
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         embed_f32_kernel<A><<<n_tokens, 256, 0, as_stream(stream)>>>(static_cast<const A*>(embed), token_ids, out, width);
+      }))
+    return (pegainfer_status_t)hipErrorInvalidValue;
+  return (pegainfer_status_t)hipGetLastError();
+}
+
+pegainfer_status_t pegainfer_embed_f32_pair(const void* embed, const uint32_t* token_ids, float* out, float* pair, int32_t width,
+                                            int32_t n_tokens, int32_t dtype, pegainfer_stream_t stream) {
+  if (n_tokens <= 0) return 0;
+  if (width <= 0 || !pair || ceil_div(width, 256) > 65535) return (pegainfer_status_t)hipErrorInvalidValue;
+  if (!by_dtype(dtype, [&](auto* t) {
+        using A = std::remove_pointer_t<decltype(t)>;
+        embed_f32_pair_kernel<A><<<dim3(n_tokens, ceil_div(width, 256)), 256, 0, as_stream(stream)>>>(static_cast<const A*>(embed), token_ids, out,
+                                                                                                     pair, width);
       }))
     return (pegainfer_status_t)hipErrorInvalidValue;
   return (pegainfer_status_t)hipGetLastError();

@@ -169,7 +169,7 @@ struct Model {
   std::vector<void*> step_owned, want_owned;
   float *x = nullptr, *emb = nullptr, *xcat = nullptr, *conv32 = nullptr, *q32 = nullptr, *o32 = nullptr;
   void *hb = nullptr, *proj = nullptr, *mix = nullptr, *mixr = nullptr, *y1 = nullptr, *y2 = nullptr, *y3 = nullptr, *act = nullptr;
-  float *xw = nullptr, *hw = nullptr, *logits32 = nullptr;
+  float *hw = nullptr, *logits32 = nullptr;
   Half* logits16 = nullptr;
   uint8_t* top1_state = nullptr;
   pst::StepIo io;
@@ -743,7 +743,7 @@ struct Model {
     size_t c = 16;
     while (c < n) c *= 2;
     auto* wo = &want_owned;
-    if (dalloc(&xw, c * D, wo) || dalloc(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) ||
+    if (dalloc(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) || dalloc(&logits16, c * V, wo) ||
         dalloc(&top1_state, c * 16, wo))
       return -1;
     KK_HIP(io.grow_tokens(c));
@@ -894,9 +894,19 @@ struct Model {
     // ---- the layer runs (everything below reads the step's shape from its arguments and the step's contents from the
     //      metadata block, so a launch sequence recorded for one decode step serves every later step of the same shape)
     // time convolution of some columns of `proj` into fp32, with the request's tail moved on
-    auto conv = [&](const void* in, const void* w, const void* in_bias, const void* out_bias, int64_t st_off, int ch, int taps,
-                    int mode) -> int {
+    // (a decode step: with the layer's gated unit `c` beside it, which reads the same projected rows)
+    auto conv = [&](const LayerCfg& c, const void* in, const void* w, const void* in_bias, const void* out_bias, int64_t st_off, int ch,
+                    int taps, int mode) -> int {
       float* tail = state + st_off;   // taps == 1: never touched
+      if (single && c.ff > 0) {
+        pegainfer_conv_glu_step_desc q{};
+        q.in = in; q.in_row_stride = proj_stride; q.w = w; q.in_bias = in_bias; q.out_bias = out_bias; q.state = tail; q.slot_stride = slot_stride;
+        q.out = conv32; q.out_row_stride = ch; q.channels = ch; q.taps = taps; q.mode = mode; q.entry_slot = d_slot;
+        q.gate = at(proj, (size_t)c.o_ffg); q.up = at(proj, (size_t)c.o_ffu); q.glu_out = act; q.glu_row_stride = c.ff; q.I = c.ff;
+        q.act = PEGAINFER_ACT_RELU; q.n_entries = n; q.dtype = dtype;
+        KK_K(pegainfer_conv_glu_step(&q, S()));
+        return 0;
+      }
       if (single) {
         KK_K(pegainfer_time_conv_step_biased(in, dtype, proj_stride, w, dtype, in_bias, out_bias, tail, slot_stride, conv32,
                                              PEGAINFER_DTYPE_F32, ch, ch, taps, mode, d_slot, n, S()));
@@ -927,8 +937,9 @@ struct Model {
       return 0;
     };
     auto run_layers = [&]() -> int {
-    KK_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
-    if (has_loop) KK_K(pegainfer_scale_rows(x, D, xcat + D, 2 * D, D, Ti, 1.0f, PEGAINFER_DTYPE_F32, S()));
+    const bool opens_pass = runs[0].pass >= 0;       // its input projection writes the stream
+    if (has_loop) KK_K(pegainfer_embed_f32_pair(embed, d_tok, opens_pass ? nullptr : x, xcat, D, Ti, dtype, S()));
+    else KK_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
     for (size_t ri = 0; ri < runs.size(); ++ri) {
       const Run& r = runs[ri];
       const LayerCfg& c = layers[(size_t)r.layer];
@@ -937,7 +948,7 @@ struct Model {
       proj_stride = c.proj_rows;
       if (r.pass >= 0) {
         // a pass over the repeated span begins: the stream is mixed with the embedding rows again
-        KK_K(pegainfer_scale_rows(x, D, xcat, 2 * D, D, Ti, 1.0f, PEGAINFER_DTYPE_F32, S()));
+        if (ri > 0) KK_K(pegainfer_scale_rows(x, D, xcat, 2 * D, D, Ti, 1.0f, PEGAINFER_DTYPE_F32, S()));
         if (linear_strided(loop_in, xcat, PEGAINFER_DTYPE_F32, 2 * D, x, PEGAINFER_DTYPE_F32, D, Ti, 2 * D)) return -1;
       }
       if (r.pass >= 0 || ri == 0)   // otherwise the launch that closed the run before has left hb
@@ -951,7 +962,7 @@ struct Model {
         int64_t qkv_stride = c.proj_rows;
         const void* bias = w.qkv_bias;
         if (a.taps > 0) {   // biases join the inputs of the convolution; what it leaves is fp32
-          if (conv(proj, w.conv, w.qkv_bias, nullptr, r.st_conv, c.qkv_ch, a.taps, 0)) return -1;
+          if (conv(c, proj, w.conv, w.qkv_bias, nullptr, r.st_conv, c.qkv_ch, a.taps, 0)) return -1;
           qkv = conv32; qkv_dtype = PEGAINFER_DTYPE_F32; qkv_stride = c.qkv_ch; bias = nullptr;
         }
         KK_K(pegainfer_qk_prep_paged_form(qkv, qkv_dtype, qkv_stride, c.o_q, c.o_k, c.o_v, a.heads, a.kv, a.dim, a.vdim, nullptr, nullptr,
@@ -973,7 +984,7 @@ struct Model {
         if (linear(w.o, mix, y1, D, Ti, a.heads * a.vdim)) return -1;
         // right: [z | x | B | C | dt] at o_in; x | B | C through the convolution, the scan, y * silu(z) normed in groups
         const int inner = s.inner();
-        if (conv(at(proj, (size_t)(c.o_in + inner)), w.sconv, nullptr, w.sconv_b, r.st_sconv, s.conv_ch(), s.taps, 2)) return -1;
+        if (conv(c, at(proj, (size_t)(c.o_in + inner)), w.sconv, nullptr, w.sconv_b, r.st_sconv, s.conv_ch(), s.taps, 2)) return -1;
         pegainfer_ssd_scan_desc sd{};
         sd.xbc = conv32; sd.xbc_stride = s.conv_ch(); sd.proj = proj; sd.proj_stride = c.proj_rows;
         sd.dt_off = c.o_in + 2 * inner + 2 * s.groups * s.state;
@@ -991,8 +1002,9 @@ struct Model {
         terms[n_terms++] = pegainfer_sum_term{y2, D, nullptr, w.right_out, 0.5f};
       }
       if (c.ff > 0) {
-        KK_K(pegainfer_glu_rows(at(proj, (size_t)c.o_ffg), at(proj, (size_t)c.o_ffu), c.proj_rows, act, c.ff, c.ff, Ti, PEGAINFER_ACT_RELU,
-                                dtype, S()));
+        if (!(single && (c.type != kAttention || a.taps > 0)))      // otherwise the convolution's launch has done it
+          KK_K(pegainfer_glu_rows(at(proj, (size_t)c.o_ffg), at(proj, (size_t)c.o_ffu), c.proj_rows, act, c.ff, c.ff, Ti, PEGAINFER_ACT_RELU,
+                                  dtype, S()));
         if (linear(w.down, act, y3, D, Ti, c.ff)) return -1;
         terms[n_terms++] = pegainfer_sum_term{y3, D, nullptr, nullptr, 1.0f};
       }
@@ -1005,8 +1017,10 @@ struct Model {
     }
     // ---- wanted rows: final norm, logits over the embedding table in fp32, the soft cap
     if (W > 0) {
-      KK_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
-      KK_K(pegainfer_terms_rms_add(xw, nullptr, 0, nullptr, final_norm, eps, hw, PEGAINFER_DTYPE_F32, D, W, dtype, S()));
+      pegainfer_terms_rms_desc fin{};
+      fin.x_in = x; fin.row_index = d_want; fin.gain = final_norm; fin.eps = eps; fin.n_out = hw; fin.n_dtype = PEGAINFER_DTYPE_F32;
+      fin.d = D; fin.rows = W; fin.dtype = dtype;
+      KK_K(pegainfer_terms_rms(&fin, S()));
       if (linear_strided(embed, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
       KK_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, logit_cap, V, W, top1_state,
                                    out_tokens ? io.tokens() : nullptr, S()));

@@ -45,6 +45,15 @@ def embed_f32(embed, token_ids_u32):
     return out
 
 
+def embed_f32_pair(embed, token_ids_u32, stream=True):
+    """-> (the rows fp32 or None, the rows twice side by side)"""
+    n, width = token_ids_u32.numel(), embed.shape[1]
+    out = torch.empty((n, width), dtype=torch.float32, device=embed.device) if stream else None
+    pair = torch.empty((n, 2 * width), dtype=torch.float32, device=embed.device)
+    _chk(ffi.lib().pegainfer_embed_f32_pair(_p(embed), _p(token_ids_u32), _p(out), _p(pair), width, n, _dt(embed), _stream()), "embed_f32_pair")
+    return out, pair
+
+
 def dyt_norm(x_f32, alpha, w, b):
     """out = tanh(alpha x) w + b; x fp32 [rows, d]; alpha / w / b (and the result) in the storage type of w"""
     assert x_f32.dtype == torch.float32 and x_f32.is_contiguous()
@@ -670,6 +679,26 @@ def decay_attention(proj, offs, decay, state, heads, dim, vdim, rg, silu=True, s
 
 
 # ---- norms with offset gains, rows of token pairs, identity experts, values that are keys, gated linear attention ----
+ConvGluStepDesc = _struct("ConvGluStepDesc", [("p", "in_"), ("l", "in_row_stride"), ("p", "w in_bias out_bias state"), ("l", "slot_stride"), ("p", "out"),
+                                              ("l", "out_row_stride"), ("i", "channels taps mode"), ("p", "entry_slot gate up glu_out"),
+                                              ("l", "glu_row_stride"), ("i", "I act n_entries dtype")])
+
+
+def conv_glu_step(x, w, state, rg, gate, up, act="relu", silu=False, in_bias=None, out_bias=None):
+    """one row per entry: the time convolution of x [n, C] (a view of rows; state as in time_conv) and act(gate) * up of views with the same
+    row stride, in one launch -> (fp32 [n, C], [n, I])"""
+    n, C, I = x.shape[0], w.shape[0], gate.shape[1]
+    assert x.stride(0) == gate.stride(0) == up.stride(0)
+    out = torch.empty((n, C), dtype=torch.float32, device=x.device)
+    glu = torch.empty((n, I), dtype=x.dtype, device=x.device)
+    q = ConvGluStepDesc(in_=_p(x), in_row_stride=x.stride(0), w=_p(w), in_bias=_p(in_bias), out_bias=_p(out_bias), state=_p(state),
+                        slot_stride=state.shape[1] * state.shape[2], out=_p(out), out_row_stride=C, channels=C, taps=w.shape[1],
+                        mode=2 if silu else 0, entry_slot=_p(rg.entry_slot), gate=_p(gate), up=_p(up), glu_out=_p(glu), glu_row_stride=I, I=I,
+                        act=ACTS[act], n_entries=n, dtype=_dt(x))
+    _chk(ffi.lib().pegainfer_conv_glu_step(ctypes.addressof(q), _stream()), "conv_glu_step")
+    return out, glu
+
+
 TermsRmsDesc = _struct("TermsRmsDesc", [("p", "x_in row_index embed token_ids"), ("f", "embed_scale"), ("p", "pair_table prev_ids"),
                                         ("l", "mul_prev mul_cur buckets"), ("p", "terms"), ("i", "n_terms"), ("p", "x_out gain"),
                                         ("f", "eps gain_offset"), ("p", "n_out"), ("i", "n_dtype d rows dtype")])

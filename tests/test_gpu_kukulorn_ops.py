@@ -73,6 +73,64 @@ def test_sum_of_normed_and_plain_terms_then_norm(dtype, d):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows,d", [(1, 64), (3, 260), (255, 2048), (256, 2048), (2, 4096), (2, 4100), (3, 1026)])
+def test_terms_of_few_and_many_rows(dtype, rows, d):
+    # below 256 rows of up to 4096 columns in fours a row is one pass of its workgroup; the other shapes take the general form
+    g = torch.Generator().manual_seed(rows + d)
+    x = torch.randn(rows, d, generator=g)
+    y1, y2, y3 = (C.bf16_round(torch.randn(rows, d, generator=g)) for _ in range(3))
+    w1, w3, b1, gain = (C.bf16_round(torch.randn(d, generator=g)) for _ in range(4))
+    terms = [(dev(y1, dtype), dev(b1, dtype), dev(w1, dtype), 0.5), (dev(y2, dtype), None, None, -2.0), (dev(y3, dtype), None, dev(w3, dtype), 1.0)]
+    r, n = B().terms_rms_add(x.cuda(), terms, gain=dev(gain, dtype), eps=1e-5, out_dtype=torch.float32)
+    ref = x.double() + 0.5 * R.rms(y1.double() + b1.double(), 1e-5) * w1.double() - 2 * y2.double() + R.rms(y3.double(), 1e-5) * w3.double()
+    close(r, ref, "float32", tol32=3e-6)
+    close(n, R.rms(ref, 1e-5) * gain.double(), "float32", tol32=3e-6)
+    pick = torch.randint(0, rows, (rows,), generator=g, dtype=torch.int32)
+    dt = DT[dtype]
+    r, n = B().terms_rms(dt, d, x=x.cuda(), row_index=pick.cuda(), gain=dev(gain, dtype), eps=1e-5, gain_offset=1.0)
+    close(n, R.rms(x[pick.long()].double(), 1e-5) * (1 + gain.double()), dtype, tol32=3e-6, tol16=4e-3)
+    emb, pairs = C.bf16_round(torch.randn(11, d, generator=g)), C.bf16_round(torch.randn(8, d, generator=g))
+    ids = torch.randint(0, 11, (rows,), generator=g)
+    prev = torch.randint(-1, 11, (rows,), generator=g)
+    r, n = B().terms_rms(dt, d, embed=dev(emb, dtype), token_ids=ids.to(torch.int32).cuda().view(torch.uint32), embed_scale=1.5,
+                         pair_table=dev(pairs, dtype), prev_ids=prev.to(torch.int32).cuda(), muls=(5, 3), gain=dev(gain, dtype), eps=1e-5)
+    at = torch.where(prev < 0, torch.full_like(prev, 7), (prev * 5 + ids * 3) % 7)
+    ref = emb[ids].double() * 1.5 + pairs[at].double()
+    close(r, ref, "float32", tol32=1e-6)
+    close(n, R.rms(ref, 1e-5) * gain.double(), dtype, tol32=3e-6, tol16=4e-3)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("channels,taps,I", [(300, 4, 257), (256, 1, 40), (70, 8, 300), (33, 10, 7)])
+def test_convolution_step_with_a_gated_unit_beside_it(dtype, channels, taps, I):
+    g = torch.Generator().manual_seed(channels)
+    n = 5
+    rows = C.bf16_round(torch.randn(n, channels + 2 * I + 3, generator=g))
+    w, ib, ob = (C.bf16_round(torch.randn(*s, generator=g)) for s in ((channels, taps), (channels,), (channels,)))
+    state = torch.randn(6, max(taps - 1, 1), channels, generator=g)
+    d, st, rg = dev(rows, dtype), state.cuda(), B().Ragged([1] * n, slots=[4, 0, 5, 2, 1])
+    conv, glu = B().conv_glu_step(d[:, :channels], dev(w, dtype), st, rg, d[:, channels:channels + I], d[:, channels + I:channels + 2 * I], "silu",
+                                  silu=True, in_bias=dev(ib, dtype), out_bias=dev(ob, dtype))
+    close(glu, R.silu(rows[:, channels:channels + I].double()) * rows[:, channels + I:channels + 2 * I].double(), dtype, tol32=2e-6, tol16=4e-3)
+    for e, slot in enumerate((4, 0, 5, 2, 1)):
+        past = torch.cat([state[slot, :taps - 1].double(), (rows[e:e + 1, :channels] + ib).double()])
+        close(conv[e], R.silu((past * w.double().t()).sum(0) + ob.double()), "float32", tol32=2e-6)
+        if taps > 1:
+            close(st[slot], past[1:], "float32", tol32=1e-6)
+    assert torch.equal(st[3].cpu(), state[3])
+
+
+def test_embedding_rows_beside_themselves():
+    emb = torch.randn(9, 300).bfloat16().cuda()
+    ids = torch.tensor([3, 8, 3, 0], dtype=torch.int32).cuda().view(torch.uint32)
+    out, pair = B().embed_f32_pair(emb, ids)
+    ref = emb[torch.tensor([3, 8, 3, 0]).cuda()].float()
+    assert torch.equal(out, ref) and torch.equal(pair, torch.cat([ref, ref], 1))
+    none, pair = B().embed_f32_pair(emb, ids, stream=False)
+    assert none is None and torch.equal(pair, torch.cat([ref, ref], 1))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_glu_activations_and_soft_cap(dtype):
     g = torch.Generator().manual_seed(1)
     gu = C.bf16_round(torch.randn(7, 2 * 37 + 5, generator=g) * 2)
