@@ -712,6 +712,51 @@ int32_t pegainfer_gated_linear_chunked_ok(int32_t dim, int32_t vdim);
 int32_t pegainfer_gated_linear_fused_ok(int32_t rank, int32_t rank_stride, const void* w_up);
 int64_t pegainfer_gated_linear_workspace(int32_t n_chunks, int32_t heads, int32_t dim, int32_t vdim);
 pegainfer_status_t pegainfer_gated_linear(const pegainfer_gated_linear_desc* d, pegainfer_stream_t stream);
+/* One decode step (every entry one row) of a recurrence with a matrix state per head, its read-out normed and gated:
+ *   STEP_GATED          pegainfer_gated_linear:          qkv = projected rows of dtype, decays from z / w_up, z_bias (may be NULL), tau; q_scale
+ *   STEP_DELTA          pegainfer_delta_rule:            qkv fp32 (q and k of kv_heads heads; not changed), decay and beta inputs of proj at
+ *                       a_off / b_off, A_log [heads], z_bias = dt_bias [heads]
+ *   STEP_DELTA_CHANNEL  pegainfer_delta_rule_channel:    the same, decays per key channel from z / w_up, z_bias = dt_bias [heads * dim]
+ *   out[e, h vdim + c] = y[c] / sqrt(mean(y^2) + eps) * norm_w[c] * act(gate[e, h vdim + c]) * factor          (gate_kind 0 silu, 1 sigmoid)
+ * z (fp32 [n][heads * dim]) may be made on the way, w_up [heads * dim][rank_stride] times the low-rank values of proj at low_off (columns
+ * past rank are zero), and so may the gate (w_gate, rounded to dtype as a stored value): pegainfer_recurrent_step_up_ok. */
+#define PEGAINFER_STEP_GATED 0
+#define PEGAINFER_STEP_DELTA 1
+#define PEGAINFER_STEP_DELTA_CHANNEL 2
+typedef struct {
+  int32_t kind;
+  const void* qkv;                            /* 16-byte aligned, qkv_stride and v_off multiples of four */
+  int64_t qkv_stride, q_off, k_off, v_off;
+  float q_scale;
+  const void* proj;
+  int64_t proj_stride;
+  const float* z;
+  int64_t z_stride;
+  const void* w_up;
+  int64_t low_off;
+  int32_t rank, rank_stride;
+  const void* z_bias;
+  float tau;
+  const void* A_log;
+  int64_t a_off, b_off;
+  float* state;                               /* 16-byte aligned, slot_stride a multiple of four */
+  int64_t slot_stride;
+  const int32_t* entry_slot;
+  const void* norm_w;
+  const void* gate;
+  int64_t gate_stride;
+  const void* w_gate;
+  int64_t gate_low_off;
+  int32_t gate_rank, gate_rank_stride, gate_kind;
+  float factor, eps;
+  void* out;
+  int64_t out_stride;
+  int32_t heads, kv_heads, dim, vdim, n_entries, dtype;
+} pegainfer_recurrent_step_desc;
+int32_t pegainfer_recurrent_step_up_ok(const void* w, int32_t rank, int32_t rank_stride, const void* proj, int64_t proj_stride, int64_t low_off);
+/* heads of at most 128 key channels and 128 values in fours, and what is said above; otherwise the separate launches */
+int32_t pegainfer_recurrent_step_ok(const pegainfer_recurrent_step_desc* q);
+pegainfer_status_t pegainfer_recurrent_step(const pegainfer_recurrent_step_desc* q, pegainfer_stream_t stream);
 /* Per-head RMS norm of a memory's read-out, a weight, a gate and a constant factor:
  *   out[row, h, :] = o[row, h, :] / sqrt(mean(o[row, h, :]^2) + eps) * w * act(gate[row, h, :]) * factor
  * w: [vdim] shared by the heads (w_per_head == 0) or [heads * vdim]; gate_kind 0 = silu, 1 = sigmoid; gate rows of dtype

@@ -31,7 +31,7 @@ HOST_LIB = os.path.join(LIBDIR, "libpegainfer_qwen3.so")
 FAMILY_SOURCES = {
     "zofadra": (("attn_latent", "attn_paged", "decay_attn", "elementwise", "gemm_strided", "linear", "norm", "sampling", "seq_blocks", "stream_mix"),
                 ("logprobs", "zofadra_runtime")),
-    "sopanex": (("attn_paged", "elementwise", "gated_linear", "gemm_strided", "linear", "moe_route", "norm", "sampling", "seq_blocks"),
+    "sopanex": (("attn_paged", "elementwise", "gated_linear", "gemm_strided", "linear", "moe_route", "norm", "recurrent_step", "sampling", "seq_blocks"),
                 ("logprobs", "sopanex_runtime")),
 }
 

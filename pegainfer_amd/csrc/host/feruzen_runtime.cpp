@@ -958,10 +958,22 @@ struct Model {
                                    c.conv_ch, c.conv_ch, d.taps, 2, d_ent, d_row0, d_slot, Ti, S()));
           FZ_K(pegainfer_time_conv_commit(proj, dtype, Mp, state + c.st_conv, slot_stride, c.conv_ch, d.taps, d_row0, d_slot, n, S()));
         }
-        FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
-                                  o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
-        FZ_K(pegainfer_head_rms_gate(o32, w.onorm, 0, at(proj, (size_t)c.o_g), Mp, 0, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
-                                     Ti, dtype, S()));
+        pegainfer_recurrent_step_desc q{};
+        q.kind = PEGAINFER_STEP_DELTA;
+        q.qkv = qkv32; q.qkv_stride = c.conv_ch; q.k_off = (int64_t)d.kv * d.dim; q.v_off = (int64_t)2 * d.kv * d.dim;
+        q.proj = proj; q.proj_stride = Mp; q.a_off = c.o_a; q.b_off = c.o_b; q.A_log = w.A_log; q.z_bias = w.dt_bias;
+        q.state = state + c.st_mem; q.slot_stride = slot_stride; q.entry_slot = d_slot;
+        q.norm_w = w.onorm; q.gate = at(proj, (size_t)c.o_g); q.gate_stride = Mp; q.factor = 1.0f; q.eps = eps;
+        q.out = mix; q.out_stride = c.mix_cols;
+        q.heads = d.heads; q.kv_heads = d.kv; q.dim = d.dim; q.vdim = d.vdim; q.n_entries = n; q.dtype = dtype;
+        if (single && !plain_kernels && pegainfer_recurrent_step_ok(&q)) {       // preparation, scan, norm and gate in one launch
+          FZ_K(pegainfer_recurrent_step(&q, S()));
+        } else {
+          FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
+                                    o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
+          FZ_K(pegainfer_head_rms_gate(o32, w.onorm, 0, at(proj, (size_t)c.o_g), Mp, 0, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
+                                       Ti, dtype, S()));
+        }
       } else {
         const AttnCfg& a = c.at;
         const MemCfg& r = c.mm;

@@ -990,14 +990,31 @@ struct Model {
                                    c.conv_ch, c.conv_ch, d.taps, 2, d_ent, d_row0, d_slot, Ti, S()));
           RX_K(pegainfer_time_conv_commit(proj, dtype, Mp, state + r.st_conv, slot_stride, c.conv_ch, d.taps, d_row0, d_slot, n, S()));
         }
+        pegainfer_recurrent_step_desc q{};
+        q.kind = PEGAINFER_STEP_DELTA_CHANNEL;
+        q.qkv = qkv32; q.qkv_stride = c.conv_ch; q.k_off = (int64_t)d.kv * d.dim; q.v_off = (int64_t)2 * d.kv * d.dim;
+        q.proj = proj; q.proj_stride = Mp; q.b_off = c.o_b; q.A_log = w.A_log; q.z_bias = w.dt_bias;
+        q.z = a32; q.z_stride = (int64_t)d.heads * d.dim; q.gate = gate_d; q.gate_stride = (int64_t)d.heads * d.vdim;
+        if (pegainfer_recurrent_step_up_ok(w.a2, d.a_rank, d.a_rank, proj, Mp, c.o_a1)) { q.w_up = w.a2; q.low_off = c.o_a1; q.rank = q.rank_stride = d.a_rank; }
+        if (pegainfer_recurrent_step_up_ok(w.g2, d.g_rank, d.g_rank, proj, Mp, c.o_g1)) {
+          q.w_gate = w.g2; q.gate_low_off = c.o_g1; q.gate_rank = q.gate_rank_stride = d.g_rank;
+        }
+        q.state = state + r.st_mem; q.slot_stride = slot_stride; q.entry_slot = d_slot;
+        q.norm_w = w.onorm; q.gate_kind = 1; q.factor = 1.0f; q.eps = eps; q.out = mix; q.out_stride = c.mix_cols;
+        q.heads = d.heads; q.kv_heads = d.kv; q.dim = d.dim; q.vdim = d.vdim; q.n_entries = n; q.dtype = dtype;
+        const bool step = single && !plain_kernels && pegainfer_recurrent_step_ok(&q);
         // second stage of the two-step projections: decay inputs (kept in fp32) and the output gate
-        if (linear_strided(w.a2, at(proj, (size_t)c.o_a1), dtype, Mp, a32, PEGAINFER_DTYPE_F32, d.heads * d.dim, Ti, d.a_rank) ||
-            linear_strided(w.g2, at(proj, (size_t)c.o_g1), dtype, Mp, gate_d, dtype, d.heads * d.vdim, Ti, d.g_rank))
+        if ((!(step && q.w_up) && linear_strided(w.a2, at(proj, (size_t)c.o_a1), dtype, Mp, a32, PEGAINFER_DTYPE_F32, d.heads * d.dim, Ti, d.a_rank)) ||
+            (!(step && q.w_gate) && linear_strided(w.g2, at(proj, (size_t)c.o_g1), dtype, Mp, gate_d, dtype, d.heads * d.vdim, Ti, d.g_rank)))
           return -1;
-        RX_K(pegainfer_delta_rule_channel(qkv32, c.conv_ch, proj, Mp, c.o_b, a32, (int64_t)d.heads * d.dim, w.A_log, w.dt_bias, gates32,
-                                          state + r.st_mem, slot_stride, o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
-        RX_K(pegainfer_head_rms_gate(o32, w.onorm, 0, gate_d, (int64_t)d.heads * d.vdim, 1, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
-                                     Ti, dtype, S()));
+        if (step) {       // decoding: second stages, preparation, scan, norm and gate in one launch
+          RX_K(pegainfer_recurrent_step(&q, S()));
+        } else {
+          RX_K(pegainfer_delta_rule_channel(qkv32, c.conv_ch, proj, Mp, c.o_b, a32, (int64_t)d.heads * d.dim, w.A_log, w.dt_bias, gates32,
+                                            state + r.st_mem, slot_stride, o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
+          RX_K(pegainfer_head_rms_gate(o32, w.onorm, 0, gate_d, (int64_t)d.heads * d.vdim, 1, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
+                                       Ti, dtype, S()));
+        }
       } else {
         const AttnCfg& a = c.at;
         const size_t ts = (size_t)c.tile_set;

@@ -366,6 +366,22 @@ class Model : public StepModel {
     const MemCfg& m = c.right;
     const int rd = m.heads * m.dim;
     const int rp = pad8(m.rank);
+    // decoding: decays, scan, norm and gate in one launch
+    if (s.single && !plain_kernels) {
+      pegainfer_recurrent_step_desc d{};
+      d.kind = PEGAINFER_STEP_GATED;
+      d.qkv = d.proj = proj; d.qkv_stride = d.proj_stride = c.proj_rows; d.q_off = m.o_q; d.k_off = m.o_k; d.v_off = m.o_v;
+      d.q_scale = (float)(1.0 / std::sqrt((double)m.dim));
+      d.w_up = w.a2; d.low_off = m.o_a; d.rank = m.rank; d.rank_stride = rp; d.z_bias = w.a2_bias; d.tau = m.tau;
+      d.state = state + m.st_off; d.slot_stride = state_layout.floats_per_slot(); d.entry_slot = s.slot;
+      d.norm_w = w.mem_norm; d.gate = at(proj, (size_t)m.o_g); d.gate_stride = c.proj_rows; d.factor = c.right_scale; d.eps = eps;
+      d.out = at(mix, (size_t)c.mix_right); d.out_stride = c.mix_cols;
+      d.heads = d.kv_heads = m.heads; d.dim = m.dim; d.vdim = m.vdim; d.n_entries = s.n; d.dtype = dtype;
+      if (pegainfer_recurrent_step_ok(&d)) {
+        PSTEP_K(pegainfer_recurrent_step(&d, S()));
+        return 0;
+      }
+    }
     // few rows: the scan makes the decay inputs itself (its workgroups read W_a2 once per row)
     const bool fused = s.T <= kFusedRows && s.chunks.n_long == 0 && !plain_kernels && pegainfer_gated_linear_fused_ok(m.rank, rp, w.a2);
     if (!fused && linear_strided(w.a2, at(proj, (size_t)m.o_a), dtype, c.proj_rows, z32, PEGAINFER_DTYPE_F32, rd, s.T, rp)) return -1;

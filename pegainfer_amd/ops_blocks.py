@@ -843,3 +843,33 @@ def gated_linear(proj, offs, z_f32, z_bias, tau, q_scale, state, heads, dim, vdi
     keep = _chunk_tables(d, rg, scan_max, ffi.lib().pegainfer_gated_linear_workspace, heads, dim, vdim)  # noqa: F841 (alive until enqueued)
     _chk(ffi.lib().pegainfer_gated_linear(ctypes.addressof(d), _stream()), "gated_linear")
     return o
+
+
+RecurrentStepDesc = _struct("RecurrentStepDesc", [("i", "kind"), ("p", "qkv"), ("l", "qkv_stride q_off k_off v_off"), ("f", "q_scale"), ("p", "proj"),
+                                                  ("l", "proj_stride"), ("p", "z"), ("l", "z_stride"), ("p", "w_up"), ("l", "low_off"),
+                                                  ("i", "rank rank_stride"), ("p", "z_bias"), ("f", "tau"), ("p", "A_log"), ("l", "a_off b_off"),
+                                                  ("p", "state"), ("l", "slot_stride"), ("p", "entry_slot norm_w gate"), ("l", "gate_stride"),
+                                                  ("p", "w_gate"), ("l", "gate_low_off"), ("i", "gate_rank gate_rank_stride gate_kind"),
+                                                  ("f", "factor eps"), ("p", "out"), ("l", "out_stride"), ("i", "heads kv_heads dim vdim n_entries dtype")])
+STEP_KINDS = {"gated": 0, "delta": 1, "delta_channel": 2}
+
+
+def recurrent_step(kind, qkv, offs, proj, state, slots, norm_w, heads, kv_heads, dim, vdim, q_scale=1.0, z=None, w_up=None, low_off=0, rank=0,
+                   z_bias=None, tau=1.0, A_log=None, a_off=0, b_off=0, gate=None, w_gate=None, gate_low_off=0, gate_rank=0, gate_kind="silu",
+                   factor=1.0, eps=1e-6):
+    """one row per entry; qkv rows (of proj's type for "gated", else fp32) with q, k, v at offs -> the normed and gated read-out [n, heads * vdim]
+    in proj's type, or None where the launch does not take these sizes"""
+    n = proj.shape[0]
+    out = torch.empty((n, heads * vdim), dtype=proj.dtype, device=proj.device)
+    q = RecurrentStepDesc(kind=STEP_KINDS[kind], qkv=_p(qkv), qkv_stride=qkv.stride(0), q_off=offs[0], k_off=offs[1], v_off=offs[2],
+                          q_scale=float(q_scale), proj=_p(proj), proj_stride=proj.stride(0), z=_p(z), z_stride=0 if z is None else z.stride(0),
+                          w_up=_p(w_up), low_off=low_off, rank=rank, rank_stride=0 if w_up is None else w_up.stride(0), z_bias=_p(z_bias),
+                          tau=float(tau), A_log=_p(A_log), a_off=a_off, b_off=b_off, state=_p(state), slot_stride=state.stride(0),
+                          entry_slot=_p(slots), norm_w=_p(norm_w), gate=_p(gate), gate_stride=0 if gate is None else gate.stride(0),
+                          w_gate=_p(w_gate), gate_low_off=gate_low_off, gate_rank=gate_rank, gate_rank_stride=0 if w_gate is None else w_gate.stride(0),
+                          gate_kind=0 if gate_kind == "silu" else 1, factor=float(factor), eps=float(eps), out=_p(out), out_stride=heads * vdim,
+                          heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, n_entries=n, dtype=_dt(proj))
+    if not ffi.lib().pegainfer_recurrent_step_ok(ctypes.addressof(q)):
+        return None
+    _chk(ffi.lib().pegainfer_recurrent_step(ctypes.addressof(q), _stream()), "recurrent_step")
+    return out
