@@ -92,3 +92,42 @@ def test_sizes_that_the_launch_leaves_to_the_others():
         proj, slots = torch.zeros(1, 2 * dim + vdim + 8, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
         assert B.recurrent_step("gated", proj, [0, dim, 2 * dim], proj, torch.zeros(1, dim * vdim, device="cuda"), slots, torch.ones(vdim, device="cuda"),
                                 1, 1, dim, vdim, z=torch.zeros(1, dim, device="cuda"), gate=proj) is None
+
+
+# the scan behind them: rounds of sixteen tokens (edges, remainders, an empty entry), values in fours and one by one, every number of values a lane holds
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("heads,kv,dim,vdim,lens", [(2, 1, 16, 16, [1, 15, 16]), (2, 2, 30, 20, [17, 2]), (2, 1, 64, 33, [0, 33, 1]), (1, 1, 100, 16, [48]),
+                                                    (4, 2, 128, 48, [31, 3, 16]), (2, 2, 99, 30, [32, 5]), (1, 1, 200, 17, [18])])
+@pytest.mark.parametrize("odd", [False, True])
+def test_delta_scan_against_float64(channel, heads, kv, dim, vdim, lens, odd):
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator().manual_seed(dim + vdim)
+    n, width = sum(lens), 2 * kv * dim + heads * vdim
+    qkv = torch.randn(n, width + (4 - width % 4) % 4 + int(odd), generator=g)
+    proj, a = torch.randn(n, 2 * heads, generator=g), torch.randn(n, heads * dim, generator=g)
+    A_log, dt_bias = torch.randn(heads, generator=g) * 0.3, torch.randn(heads * (dim if channel else 1), generator=g)
+    state = torch.randn(len(lens) + 1, heads, dim, vdim, generator=g)
+    slots = torch.randperm(len(lens) + 1, generator=g)[:len(lens)].tolist()
+    unit = lambda t: t / (t.pow(2).sum(-1, keepdim=True) + 1e-6).sqrt()
+    parts = lambda o: qkv[:, o:o + kv * dim].double().view(n, kv, dim).repeat_interleave(heads // kv, 1)
+    q, k = unit(parts(0)) * dim ** -0.5, unit(parts(kv * dim))
+    v, beta = qkv[:, 2 * kv * dim:width].double().view(n, heads, vdim), torch.sigmoid(proj[:, :heads].double())
+    z = a.double() if channel else proj[:, heads:].double()
+    rate = A_log.double().exp().repeat_interleave(dim) if channel else A_log.double().exp()
+    decay = torch.exp(-rate * torch.nn.functional.softplus(z + dt_bias.double())).view(n, heads, -1, 1)
+    want, at, after = torch.zeros(n, heads, vdim, dtype=torch.float64), 0, state.double().clone()
+    for length, slot in zip(lens, slots):
+        S = after[slot]
+        for t in range(at, at + length):
+            S = decay[t] * S
+            S = S + k[t][..., None] * (beta[t][:, None] * (v[t] - (S * k[t][..., None]).sum(1)))[:, None]
+            want[t] = (S * q[t][..., None]).sum(1)
+        after[slot], at = S, at + length
+    rg, mem, x = B.Ragged(lens, slots), state.cuda(), qkv.cuda()
+    if channel:
+        o = B.delta_rule_channel(x, proj.cuda(), 0, a.cuda(), A_log.cuda(), dt_bias.cuda(), mem, heads, kv, dim, vdim, rg)
+    else:
+        o = B.delta_rule(x, proj.cuda(), 0, heads, A_log.cuda(), dt_bias.cuda(), mem, heads, kv, dim, vdim, rg)
+    # at most 48 steps of fp32 sums of at most 200 terms, each a contraction: some 1e-6 of the largest value; five times that is asked for
+    assert float((o.double().cpu().view(n, heads, vdim) - want).abs().max() / want.abs().max()) < 5e-6
+    assert float((mem.double().cpu() - after).abs().max() / after.abs().max()) < 5e-6
