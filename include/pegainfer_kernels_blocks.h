@@ -929,6 +929,18 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
                                                  const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
                                                  int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
                                                  pegainfer_stream_t stream);
+/* the same, and tile_rows = 32 / 64 with two maps as well where pegainfer_paged_attention_maps_rows_ok says so (dim 32 with vdim <= 64, dim 64
+ * with vdim <= 128) */
+pegainfer_status_t pegainfer_paged_attention_maps(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
+                                                  int64_t v_cache_off, int32_t page_size, const int32_t* positions,
+                                                  const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,
+                                                  int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float scale,
+                                                  float factor, const int32_t* tile_row0, const int32_t* tile_ntok,
+                                                  const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
+                                                  int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
+                                                  pegainfer_stream_t stream);
+int32_t pegainfer_paged_attention_maps_rows_ok(int32_t maps, int32_t dim, int32_t vdim, int64_t page_stride, int64_t v_cache_off,
+                                               int32_t page_size);
 /* fp32 values of scratch a launch with n_split > 1 needs (0 for n_split <= 1) */
 int64_t pegainfer_paged_attention_workspace(int32_t n_tiles, int32_t kv_heads, int32_t vdim, int32_t maps, int32_t n_split);
 /* out[row, :cols] = in[row, :cols] * factor; rows of in / out at their own strides (elements of dtype) */

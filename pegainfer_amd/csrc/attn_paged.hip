@@ -878,7 +878,7 @@ static size_t mfma_attention_lds(int maps, int dim, int ncb) {
   return std::max(tiles, fold);
 }
 
-// Prompts: the same attention with 16 RG rows per workgroup (32 or 64), for a bf16 cache, one map, sizes in multiples of 8.
+// Prompts: the same attention with 16 RG rows per workgroup (32 or 64), for a bf16 cache, one map or two, sizes in multiples of 8.
 // Two waves per 16 rows, each on 32 of a tile's 64 keys, two softmax streams per row folded once at the end.  Keys and values travel by
 // LDS-DMA into a ring of S tiles, row-major, requested S - 1 tiles ahead (their page numbers one tile further, in scalar registers: a vector
 // load beside the DMAs could only be waited for together with them): a tile costs one barrier and a counted wait, no LDS writes.  A row's 16-byte chunks are XORed with bits of its number (the DMA
@@ -892,13 +892,15 @@ static size_t mfma_attention_lds(int maps, int dim, int ncb) {
 // third of the LDS cycles repeat for bank conflicts.  1024 rows x 16 heads of 128: 28 us
 // causal (153 TFLOP/s), 86 us behind 3072 cached tokens, 103 us with a cap - against 39, 131 and 160 us with both tiles
 // passing through registers, values transposed on the way, scores shaped one by one and the maximum exchanged in every tile.
+// Two maps (of P / 2 values each, a key's halves): a stream per map, every value fragment read once for both.  Eight prompts of 350 - 700 tokens, 16 heads of
+// 2 x 64 over 128 values: 195 -> 56 us against tiles of 16 rows; the same prompts' block-masked layer of one map 65 -> 29 us.
 template <int P, int RG>
 struct RowsShape {
   static constexpr int N = RG * 128, CH = P / 8, S = P == 256 || RG == 2 ? 2 : 3;   // threads, chunks of a row, tiles in the ring
   static constexpr int kTile = kAttKeys * P * 2;                                  // bytes of a key (or value) tile
   static constexpr int kLoads = 2 * (kTile / 1024) / (2 * RG);                    // DMA instructions per wave and tile
 };
-template <int P, int RG>
+template <int P, int RG, int MAPS>
 __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     const float* __restrict__ q, const uint16_t* __restrict__ cache, int64_t page_stride, int64_t k_cache_off, int64_t v_cache_off,
     int page_size, const int32_t* __restrict__ positions, const int32_t* __restrict__ row_entry,
@@ -923,7 +925,7 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     return k >= form.keep_first && k + kAttKeys <= lo0 ? (lo0 / kAttKeys) * kAttKeys : k;
   };
   const int kfirst = form.keep_first > 0 ? 0 : (lo0 / kAttKeys) * kAttKeys;
-  const int kw = form.k_keep;
+  const int kw = form.k_keep, qd = MAPS * dim;        // two maps: qd = P
   // this wave's rows
   const int lr = rg * 16 + l15;
   const bool mine = lr < nrows;
@@ -937,16 +939,16 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   const int all_lo = last >= 0 ? attn_row_lo(form, last) : 0, all_hi = rg * 16 + 15 < nrows ? positions[row0 + rg * 16 / nqh] : -1;
   bf16x8_t qf[P / 32];
   {
-    const float* qr = q + ((int64_t)(row0 + (mine ? lr / nqh : 0)) * H + rqh) * dim;
+    const float* qr = q + ((int64_t)(row0 + (mine ? lr / nqh : 0)) * H + rqh) * qd;
 #pragma unroll
     for (int st = 0; st < P / 32; ++st) {
       const int c = st * 32 + lg * 8;
       float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (mine && c < dim) Vec8<float>::load(qr + c, t);
+      if (mine && c < qd) Vec8<float>::load(qr + c, t);
       qf[st] = __builtin_bit_cast(bf16x8_t, u32x4{pack_bf2(t[0], t[1]), pack_bf2(t[2], t[3]), pack_bf2(t[4], t[5]), pack_bf2(t[6], t[7])});
     }
   }
-  if (dim < P || vdim < P) {       // chunks past a row's end are never fetched: they stay zero
+  if (qd < P || vdim < P) {       // chunks past a row's end are never fetched: they stay zero
     for (int i = tid; i < S * 2 * Sh::kTile / 16; i += N) reinterpret_cast<u32x4*>(smraw)[i] = u32x4{0u, 0u, 0u, 0u};
   }
   // swizzle of row j: CH 16 - its low four bits; CH 8 - two rows share 256 bytes, the three bits above the lowest
@@ -982,7 +984,7 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   auto fetch = [&](int i, int64_t page, int ok, int ov, int stage) {
     const int c = src_c[i];
     const uint32_t dst = ring + (uint32_t)(stage * 2 * Sh::kTile + (wave_u * kHalf + i) * 1024);
-    if (c < dim) dma((c < kw ? kbase : vbase) + page + ok, dst);
+    if (c < qd) dma((c < kw ? kbase : vbase) + page + ok, dst);
     if (c < vdim) dma(vbase + page + ov, dst + Sh::kTile);
   };
   auto fetch_at = [&](int i, int p, int page, int stage) {     // the general form: a key's own page and place
@@ -1004,10 +1006,15 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
       }
     }
   };
-  float mrun = -INFINITY, lrun = 0.f;                 // log2 units; lrun: this lane's part of the row sum
-  f32x4 o[NCB];
+  float mrun[MAPS], lrun[MAPS];                       // log2 units; lrun: this lane's part of the row sum
+  f32x4 o[MAPS][NCB];
 #pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) o[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < MAPS; ++m) {
+    mrun[m] = -INFINITY;
+    lrun[m] = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) o[m][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const int krow = 32 * kh + l15, vrow = 32 * kh + 4 * lg + (l15 >> 2);
   // byte addresses inside a tile: swz(row + 16) = swz(row) for both row widths, so the second half of the keys lies 16 rows on
   const uint32_t ka = (uint32_t)(krow * P * 2 + ((lg ^ swz(krow)) << 4));
@@ -1017,17 +1024,22 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   // cost 13 % (the branch, or 32 instructions a tile, stands between the weights and the second products); 77 us behind 3072 tokens so, 79 unmasked.
   auto multiply_keys = [&](int kb, int stage, auto masked) {
     const unsigned char* kt = smraw + stage * 2 * Sh::kTile;
-    f32x4 sc[2] = {};
+    f32x4 maps[MAPS][2] = {};
 #pragma unroll
     for (int st = 0; st < P / 32; ++st)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(kt + 16 * t * P * 2 + (ka ^ (uint32_t)(st << 6)))), qf[st], sc[t], 0, 0, 0);
+        maps[st * 32 * MAPS / P][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(kt + 16 * t * P * 2 + (ka ^ (uint32_t)(st << 6)))), qf[st], maps[st * 32 * MAPS / P][t], 0, 0, 0);
     // dot products -> scores times log2(e); each option in a pass of its own: one uniform branch per tile, its loads in flight together
     const int dist = rpos - kb - 4 * lg;             // of this lane's key (t, r): dist - 16 t - r
     const bool options = form.softcap > 0.f || form.dist_bias || form.dist_slope;
     const float f0 = options ? scale : scale * kLog2e;
+    uint32_t see[4];
+    bf16x8_t pf[MAPS];
+#pragma unroll
+    for (int m = 0; m < MAPS; ++m) {
+    f32x4 (&sc)[2] = maps[m];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -1056,7 +1068,6 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) sc[t][r] *= kLog2e;
     }
-    uint32_t see[4];
     if constexpr (decltype(masked)::value) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -1073,17 +1084,17 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
       }
     }
     float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])), fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
-    if (__any(!(tmax <= mrun + kJump))) {            // uniform; the first keys of a row always, a NaN too
+    if (__any(!(tmax <= mrun[m] + kJump))) {            // uniform; the first keys of a row always, a NaN too
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-      const float mnew = fmaxf(mrun, tmax);
-      const float corr = __builtin_amdgcn_exp2f(mrun - (mnew == -INFINITY ? 0.f : mnew));   // a row that has met no key yet: 0, and nothing to scale
-      lrun *= corr;
+      const float mnew = fmaxf(mrun[m], tmax);
+      const float corr = __builtin_amdgcn_exp2f(mrun[m] - (mnew == -INFINITY ? 0.f : mnew));   // a row that has met no key yet: 0, and nothing to scale
+      lrun[m] *= corr;
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) { o[cb].x *= corr; o[cb].y *= corr; o[cb].z *= corr; o[cb].w *= corr; }
-      mrun = mnew;
+      for (int cb = 0; cb < NCB; ++cb) { o[m][cb].x *= corr; o[m][cb].y *= corr; o[m][cb].z *= corr; o[m][cb].w *= corr; }
+      mrun[m] = mnew;
     }
-    const float mref = mrun == -INFINITY ? 0.f : mrun;
+    const float mref = mrun[m] == -INFINITY ? 0.f : mrun[m];
     uint32_t pb[4];
     float psum = 0.f;
 #pragma unroll
@@ -1094,8 +1105,9 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
         pb[2 * t + (r >> 1)] = w;
         psum += bf_lo(w) + bf_hi(w);                 // the sum of the weights as they are multiplied
       }
-    lrun += psum;
-    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, u32x4{pb[0], pb[1], pb[2], pb[3]});
+    lrun[m] += psum;
+    pf[m] = __builtin_bit_cast(bf16x8_t, u32x4{pb[0], pb[1], pb[2], pb[3]});
+    }
     typedef v4s_t __attribute__((address_space(3)))* lds_v4_t;
     const uint32_t vt = ring + (uint32_t)(stage * 2 * Sh::kTile + Sh::kTile);
 #pragma unroll
@@ -1104,7 +1116,9 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
       u32x2 v0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)at));
       u32x2 v1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(uintptr_t)(at + 16 * P * 2)));
       if constexpr (decltype(masked)::value) { v0.x &= see[0]; v0.y &= see[1]; v1.x &= see[2]; v1.y &= see[3]; }
-      o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, u32x4{v0.x, v0.y, v1.x, v1.y}), pf, o[cb], 0, 0, 0);
+#pragma unroll
+      for (int m = 0; m < MAPS; ++m)
+        o[m][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, u32x4{v0.x, v0.y, v1.x, v1.y}), pf[m], o[m][cb], 0, 0, 0);
     }
   };
   auto multiply = [&](int k0, int stage) {           // uniform over the wave
@@ -1140,35 +1154,46 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in the memory that is reused below
   __syncthreads();                                   // the tiles' LDS is free
-  lrun += __shfl_xor(lrun, 16, kWave);
-  lrun += __shfl_xor(lrun, 32, kWave);
-  f32x4* f_o = reinterpret_cast<f32x4*>(smraw);      // [RG][NCB][64]
-  float* f_ml = reinterpret_cast<float*>(f_o + RG * NCB * 64);        // [RG][64][2]
-  if (kh == 1) {
+  f32x4* f_o = reinterpret_cast<f32x4*>(smraw);      // [MAPS][RG][NCB][64]
+  float* f_ml = reinterpret_cast<float*>(f_o + MAPS * RG * NCB * 64);        // [MAPS][RG][64][2]
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) f_o[(rg * NCB + cb) * 64 + lane] = o[cb];
-    f_ml[(rg * 64 + lane) * 2] = mrun;
-    f_ml[(rg * 64 + lane) * 2 + 1] = lrun;
+  for (int m = 0; m < MAPS; ++m) {
+    lrun[m] += __shfl_xor(lrun[m], 16, kWave);
+    lrun[m] += __shfl_xor(lrun[m], 32, kWave);
+    if (kh == 1) {
+#pragma unroll
+      for (int cb = 0; cb < NCB; ++cb) f_o[((m * RG + rg) * NCB + cb) * 64 + lane] = o[m][cb];
+      f_ml[((m * RG + rg) * 64 + lane) * 2] = mrun[m];
+      f_ml[((m * RG + rg) * 64 + lane) * 2 + 1] = lrun[m];
+    }
   }
   __syncthreads();
   if (kh == 1 || rg * 16 >= nrows) return;
-  const float m1 = f_ml[(rg * 64 + lane) * 2], l1 = f_ml[(rg * 64 + lane) * 2 + 1];
-  float mall = fmaxf(mrun, m1), sink = -INFINITY;
-  if (form.sink && mine) {
-    sink = bf2f(static_cast<const uint16_t*>(form.sink)[rqh]) * kLog2e;
-    mall = fmaxf(mall, sink);
+  float i0[MAPS], i1[MAPS];
+#pragma unroll
+  for (int m = 0; m < MAPS; ++m) {
+    const float m1 = f_ml[((m * RG + rg) * 64 + lane) * 2], l1 = f_ml[((m * RG + rg) * 64 + lane) * 2 + 1];
+    float mall = fmaxf(mrun[m], m1), sink = -INFINITY;
+    if (form.sink && mine) {
+      sink = bf2f(static_cast<const uint16_t*>(form.sink)[rqh]) * kLog2e;
+      mall = fmaxf(mall, sink);
+    }
+    const float w0 = mrun[m] == -INFINITY ? 0.f : exp2f(mrun[m] - mall), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - mall);
+    const float l = lrun[m] * w0 + l1 * w1 + (sink == -INFINITY ? 0.f : exp2f(sink - mall));
+    i0[m] = w0 / l;
+    i1[m] = w1 / l;
   }
-  const float w0 = mrun == -INFINITY ? 0.f : exp2f(mrun - mall), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - mall);
-  const float l = lrun * w0 + l1 * w1 + (sink == -INFINITY ? 0.f : exp2f(sink - mall));
-  const float i0 = w0 / l, i1 = w1 / l;
   float ss = 0.f;
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) {
     const f32x4 t = f_o[(rg * NCB + cb) * 64 + lane];
+    f32x4 v = {};
+    if constexpr (MAPS == 2) v = f_o[((RG + rg) * NCB + cb) * 64 + lane];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      o[cb][r] = o[cb][r] * i0 + t[r] * i1;
-      if (16 * cb + 4 * lg + r < vdim) ss = fmaf(o[cb][r], o[cb][r], ss);
+      o[0][cb][r] = o[0][cb][r] * i0[0] + t[r] * i1[0];
+      if constexpr (MAPS == 2) o[0][cb][r] -= form.lambda * (o[1][cb][r] * i0[1] + v[r] * i1[1]);
+      if (16 * cb + 4 * lg + r < vdim) ss = fmaf(o[0][cb][r], o[0][cb][r], ss);
     }
   }
   float post = factor;
@@ -1189,16 +1214,16 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     float v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      v[r] = o[cb][r] * post;
+      v[r] = o[0][cb][r] * post;
       if (form.gate_kind == 1) v[r] *= sigmoid_f(bf2f(gate[(int64_t)rqh * vdim + c + r]));
     }
     st4(dst + c, v);
   }
 }
-template <int P, int RG>
+template <int P, int RG, int MAPS>
 static constexpr size_t rows_attention_lds() {
   typedef RowsShape<P, RG> Sh;
-  return std::max((size_t)Sh::S * 2 * Sh::kTile, (size_t)RG * 64 * (P + 8));
+  return std::max((size_t)Sh::S * 2 * Sh::kTile, (size_t)MAPS * RG * 64 * (P + 8));
 }
 
 // The states that the live splits of a tile have left, brought to their common maximum and summed, then finished like an unsplit row.  A
@@ -1404,14 +1429,18 @@ pegainfer_status_t pegainfer_paged_attention_masked(const float* q, const void* 
                                           n_tiles, out, out_stride, &o, dtype, stream);
 }
 
-pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
-                                                 int64_t v_cache_off, int32_t page_size, const int32_t* positions,
-                                                 const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,
-                                                 int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float scale,
-                                                 float factor, const int32_t* tile_row0, const int32_t* tile_ntok,
-                                                 const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
-                                                 int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
-                                                 pegainfer_stream_t stream) {
+// the kernel for prompts with two maps: a map's share of a key is a whole number of its 32-wide products, known at compile time
+static bool rows_two_maps_ok(int dim, int vdim) { return (dim == 32 && vdim <= 64) || (dim == 64 && vdim <= 128); }
+
+static pegainfer_status_t paged_attention(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
+                                         int64_t v_cache_off, int32_t page_size, const int32_t* positions,
+                                         const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,
+                                         int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float scale,
+                                         float factor, const int32_t* tile_row0, const int32_t* tile_ntok,
+                                         const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
+                                         int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
+                                         pegainfer_stream_t stream,
+                                         bool two_wide) {
   if (n_tiles <= 0) return 0;
   if (!opt) return PK_BAD;
   const int32_t maps = opt->maps > 0 ? opt->maps : 1, block = opt->block, window = opt->window, keep_first = opt->keep_first,
@@ -1447,9 +1476,9 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
   form.k_keep = qd - opt->shared_tail;
   bool ok = true;
   if (opt->tile_rows > kAttRows) {    // tables cut for the prompts' kernel
-    if ((opt->tile_rows != 32 && opt->tile_rows != 64) || maps != 1 || n_split != 1 || plain || dtype != kDtBf16 || out_stride % 4 ||
+    if ((opt->tile_rows != 32 && opt->tile_rows != 64) || (maps != 1 && !(two_wide && rows_two_maps_ok(dim, vdim))) || n_split != 1 || plain || dtype != kDtBf16 || out_stride % 4 ||
         !host_aligned16(out) || !host_aligned16(q) || !host_aligned16(cache) || k_cache_off % 8 ||
-        !pegainfer_paged_attention_rows_ok(dim, vdim, opt->shared_tail, page_stride, v_cache_off, page_size))
+        !pegainfer_paged_attention_rows_ok(qd, vdim, opt->shared_tail, page_stride, v_cache_off, page_size))
       return PK_BAD;
     auto launch = [&](auto kern, size_t lds, int rg) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
@@ -1462,10 +1491,12 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
     };
     auto by_size = [&](auto rg) {
       constexpr int RG = decltype(rg)::value;
-      const int most = std::max(dim, vdim);
-      if (most <= 64) launch(paged_attention_rows_kernel<64, RG>, rows_attention_lds<64, RG>(), RG);
-      else if (most <= 128) launch(paged_attention_rows_kernel<128, RG>, rows_attention_lds<128, RG>(), RG);
-      else launch(paged_attention_rows_kernel<256, RG>, rows_attention_lds<256, RG>(), RG);
+      const int most = std::max(qd, vdim);
+      if (maps == 2 && most <= 64) launch(paged_attention_rows_kernel<64, RG, 2>, rows_attention_lds<64, RG, 2>(), RG);
+      else if (maps == 2) launch(paged_attention_rows_kernel<128, RG, 2>, rows_attention_lds<128, RG, 2>(), RG);
+      else if (most <= 64) launch(paged_attention_rows_kernel<64, RG, 1>, rows_attention_lds<64, RG, 1>(), RG);
+      else if (most <= 128) launch(paged_attention_rows_kernel<128, RG, 1>, rows_attention_lds<128, RG, 1>(), RG);
+      else launch(paged_attention_rows_kernel<256, RG, 1>, rows_attention_lds<256, RG, 1>(), RG);
     };
     if (opt->tile_rows == 64) by_size(std::integral_constant<int, 4>());
     else by_size(std::integral_constant<int, 2>());
@@ -1530,6 +1561,36 @@ pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cac
     }
   });
   return known && ok ? (pegainfer_status_t)hipGetLastError() : PK_BAD;
+}
+
+pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
+                                                 int64_t v_cache_off, int32_t page_size, const int32_t* positions,
+                                                 const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,
+                                                 int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float scale,
+                                                 float factor, const int32_t* tile_row0, const int32_t* tile_ntok,
+                                                 const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
+                                                 int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
+                                                 pegainfer_stream_t stream) {
+  return paged_attention(q, cache, page_stride, k_cache_off, v_cache_off, page_size, positions, row_entry, page_indptr, page_ids, heads, kv_heads, dim, vdim,
+                         scale, factor, tile_row0, tile_ntok, tile_qh0, tile_nqh, n_tiles, out, out_stride, opt, dtype, stream, false);
+}
+
+pegainfer_status_t pegainfer_paged_attention_maps(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
+                                                  int64_t v_cache_off, int32_t page_size, const int32_t* positions,
+                                                  const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,
+                                                  int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float scale,
+                                                  float factor, const int32_t* tile_row0, const int32_t* tile_ntok,
+                                                  const int32_t* tile_qh0, const int32_t* tile_nqh, int32_t n_tiles, void* out,
+                                                  int64_t out_stride, const pegainfer_attn_options* opt, int32_t dtype,
+                                                  pegainfer_stream_t stream) {
+  return paged_attention(q, cache, page_stride, k_cache_off, v_cache_off, page_size, positions, row_entry, page_indptr, page_ids, heads, kv_heads, dim, vdim,
+                         scale, factor, tile_row0, tile_ntok, tile_qh0, tile_nqh, n_tiles, out, out_stride, opt, dtype, stream, true);
+}
+
+int32_t pegainfer_paged_attention_maps_rows_ok(int32_t maps, int32_t dim, int32_t vdim, int64_t page_stride, int64_t v_cache_off,
+                                               int32_t page_size) {
+  return (maps == 1 || (maps == 2 && rows_two_maps_ok(dim, vdim))) &&
+         pegainfer_paged_attention_rows_ok(maps * dim, vdim, 0, page_stride, v_cache_off, page_size);
 }
 
 int32_t pegainfer_paged_attention_rows_ok(int32_t dim, int32_t vdim, int32_t shared_tail, int64_t page_stride, int64_t v_cache_off,

@@ -146,7 +146,8 @@ struct Model {
   std::vector<KvState> requests;
   pq::StateLayout state_layout;
   float* state = nullptr;
-  std::vector<int> tile_sets;   // distinct query-heads-per-kv-head values of the attention layers
+  struct TileSet { int per, wide_kv; };    // wide_kv: fewest key/value heads of a layer that takes it, 0 where one takes no wide tiles
+  std::vector<TileSet> tile_sets;          // one per distinct query-heads-per-kv-head value of the attention layers
   // step buffers
   size_t cap_rows = 0, cap_want = 0;
   std::vector<void*> step_owned, want_owned;
@@ -255,8 +256,10 @@ struct Model {
         c.mix_cols = a.heads * a.vdim;
         const int per = a.heads / a.kv;
         size_t k = 0;
-        while (k < tile_sets.size() && tile_sets[k] != per) ++k;
-        if (k == tile_sets.size()) tile_sets.push_back(per);
+        const int wide = dtype == PEGAINFER_DTYPE_BF16 && pegainfer_paged_attention_maps_rows_ok(a.maps, a.dim, a.vdim, 0, 0, kPageSize) ? a.kv : 0;
+        while (k < tile_sets.size() && tile_sets[k].per != per) ++k;
+        if (k == tile_sets.size()) tile_sets.push_back({per, wide});
+        tile_sets[k].wide_kv = std::min(tile_sets[k].wide_kv, wide);
         c.tile_set = (int)k;
       } else if (ty->str == "channel_delta") {
         c.type = kChannelDelta;
@@ -828,15 +831,16 @@ struct Model {
     const int W = (int)want.size();
     if (ensure_rows(T) || ensure_want((size_t)std::max(1, W))) return -1;
     size_t total_pages = 0;
+    int most_keys = 0;
     for (int i = 0; i < n; ++i) {
       KvState& st = requests[ids[i]];
+      most_keys = std::max(most_keys, st.seq_len + lens[i]);
       if (!st.ensure_capacity(&pool, st.seq_len + lens[i], kPageSize)) return set_error("step: page pool ran dry");
       total_pages += st.pages.size();
     }
     // ---- the packed metadata block:
     //   tokens | positions | row_entry | entry_row0 | entry_slot | page_indptr | want | attention tile sets | page_ids
-    // An attention tile is a run of token rows of one entry times a run of the query heads of one key/value head, at most
-    // 16 rows in all; one set of tiles per distinct heads-per-kv-head value of the model's attention layers.
+    // One set of attention tiles (row_tiles.h) per distinct heads-per-kv-head value of the model's attention layers.
     bool single = true;   // every entry brings one token: decoding
     for (int i = 0; i < n && single; ++i) single = lens[i] == 1;
     const size_t o_tok = 0, o_pos = o_tok + T, o_ent = o_pos + T, o_row0 = o_ent + T, o_slot = o_row0 + (size_t)n + 1,
@@ -844,14 +848,12 @@ struct Model {
     size_t words = o_want + (size_t)std::max(1, W);   // the page lists come last: everything before them sits at offsets that
                                                       // depend on the step's shape only, which a captured graph relies on
     std::vector<size_t> tile_off(tile_sets.size()), tile_cnt(tile_sets.size());
-    for (size_t k = 0; k < tile_sets.size(); ++k) {
-      const int per = tile_sets[k];
-      size_t cnt = 0;
-      for (int i = 0; i < n; ++i)
-        cnt += per <= kAttRows ? ((size_t)lens[i] + (kAttRows / per) - 1) / (kAttRows / per) : (size_t)lens[i] * ((per + kAttRows - 1) / kAttRows);
+    std::vector<int> tile_rows(tile_sets.size());
+    for (size_t k = 0; k < tile_sets.size(); ++k) {   // decoding keeps its 16 rows: what it captures follows from the step's shape alone
+      tile_rows[k] = plain_kernels || single ? ptiles::kGroupRows : ptiles::wide_rows(lens, n, (int)T, tile_sets[k].per, tile_sets[k].wide_kv, most_keys);
       tile_off[k] = words;
-      tile_cnt[k] = cnt;
-      words += 4 * cnt;
+      tile_cnt[k] = ptiles::count(lens, n, tile_sets[k].per, tile_rows[k]);
+      words += 4 * tile_cnt[k];
     }
     const size_t o_pages = words;
     words += total_pages;
@@ -878,25 +880,7 @@ struct Model {
       mh[o_row0 + n] = (int32_t)t;
       mh[o_ind + n] = (int32_t)pg;
       for (int i = 0; i < W; ++i) mh[o_want + i] = want[i];
-      for (size_t k = 0; k < tile_sets.size(); ++k) {
-        const int per = tile_sets[k];
-        int32_t *t_row0 = mh + tile_off[k], *t_ntok = t_row0 + tile_cnt[k], *t_qh0 = t_ntok + tile_cnt[k], *t_nqh = t_qh0 + tile_cnt[k];
-        size_t at_ = 0, r0 = 0;
-        for (int i = 0; i < n; ++i) {
-          if (per <= kAttRows) {
-            const int tpt = kAttRows / per;
-            for (int t0 = 0; t0 < lens[i]; t0 += tpt, ++at_) {
-              t_row0[at_] = (int32_t)r0 + t0; t_ntok[at_] = std::min(tpt, lens[i] - t0); t_qh0[at_] = 0; t_nqh[at_] = per;
-            }
-          } else {
-            for (int t0 = 0; t0 < lens[i]; ++t0)
-              for (int q0 = 0; q0 < per; q0 += kAttRows, ++at_) {
-                t_row0[at_] = (int32_t)r0 + t0; t_ntok[at_] = 1; t_qh0[at_] = q0; t_nqh[at_] = std::min(kAttRows, per - q0);
-              }
-          }
-          r0 += (size_t)lens[i];
-        }
-      }
+      for (size_t k = 0; k < tile_sets.size(); ++k) ptiles::cut(lens, n, tile_sets[k].per, tile_rows[k], tile_cnt[k], mh + tile_off[k]);
     }
     RX_HIP(hipEventRecord(ev0, stream));
     const bool captured = single && graphs_on && !tap_on;
@@ -1027,11 +1011,15 @@ struct Model {
         // a step of few rows (decoding, short portions) cannot fill the chip with one workgroup per (row tile, kv head): its
         // keys are dealt to several workgroups.  The count depends on the step's shape only, never on the contexts' lengths.
         const int wgs = (int)tile_cnt[ts] * a.kv;
-        const int nsplit = wgs >= 128 ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
-        RX_K(pegainfer_paged_attention_ex(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,
-                                          a.kv, a.dim, a.vdim, a.scale, two ? 1.0f - a.diff : 1.0f, tb, tb + tile_cnt[ts],
-                                          tb + 2 * tile_cnt[ts], tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, c.mix_cols, a.maps,
-                                          w.lambda, a.block, w.sink, two ? 1 : 0, eps, nsplit, att_part, plain_kernels ? 1 : 0, dtype, S()));
+        pegainfer_attn_options o{};
+        o.maps = a.maps; o.lambda = w.lambda; o.block = a.block; o.sink = w.sink; o.head_norm = two ? 1 : 0; o.norm_eps = eps;
+        o.n_split = wgs >= ptiles::kUnsplitGroups || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
+        o.workspace = att_part;
+        o.plain = plain_kernels ? 1 : 0;
+        o.tile_rows = tile_rows[ts] > ptiles::kGroupRows ? tile_rows[ts] : 0;
+        RX_K(pegainfer_paged_attention_maps(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,
+                                            a.kv, a.dim, a.vdim, a.scale, two ? 1.0f - a.diff : 1.0f, tb, tb + tile_cnt[ts],
+                                            tb + 2 * tile_cnt[ts], tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, c.mix_cols, &o, dtype, S()));
       }
       if (linear(w.o, mix, y, D, Ti, c.mix_cols)) return -1;
       // what the launch that closes this run norms for: the next run's first sublayer, unless that run opens a pass (its own

@@ -369,3 +369,50 @@ def test_weighted_sum_with_a_gated_shared_row(dtype):
     close(out, ref, dtype, tol32=2e-6, tol16=1e-2)
     out = B().route_combine_gated(y.cuda(), wgt.cuda(), None, None, DT[dtype])
     close(out, (wgt[:, :, None].double() * y.reshape(rows, top, d).double()).sum(1), dtype, tol32=2e-6, tol16=1e-2)
+
+
+TWO_MAP_FORMS = {"plain": {}, "sink and head norm": {"sink": True, "norm": True}, "blocks": {"block": 48, "sink": True}, "window, cap": {"window": 37, "cap": 1.5},
+                 "gate per value, head norm": {"gate": 1, "norm": True}}
+
+
+@pytest.mark.parametrize("tile_rows", [32, 64])
+@pytest.mark.parametrize("dim,vdim,page", [(32, 40, 16), (32, 64, 5), (64, 72, 8), (64, 128, 16)])
+@pytest.mark.parametrize("form", TWO_MAP_FORMS)
+def test_two_maps_on_wide_tiles(form, dim, vdim, page, tile_rows):
+    """The kernel for prompts with two maps against the fp32-FMA kernel on the same bf16 cache: values that fill a row of LDS and values that do not, pages
+    that hold a whole number of a DMA's rows and pages that do not, entries that end around a 64-key tile, a portion behind a prefix.  q and the
+    weights enter the matrix cores in bf16 (2^-9 each, relative): a score of size s moves by 2^-9 s, 2^-7 of a map's largest value covers s up to 4, and
+    the difference of two maps adds theirs; a head norm divides by the mean size of what is left, which lambda = 0.3 keeps at that of a map."""
+    import ctypes
+    import numpy as np
+    from pegainfer_amd import ops_blocks as B
+    o = TWO_MAP_FORMS[form]
+    g = torch.Generator().manual_seed(dim * 7 + vdim + page)
+    H, G = 6, 2
+    lens, past = [1, 63, 64, 65, 130, 7], [0, 0, 0, 3, 0, 140]
+    T = sum(lens)
+    need = [-(-(a + b) // page) for a, b in zip(lens, past)]
+    stride, v_off = (page * G * (2 * dim + vdim) + 7) // 8 * 8, page * G * 2 * dim
+    cache = torch.randn(sum(need) * stride, generator=g).bfloat16().cuda()
+    q = torch.randn(T, H, 2 * dim, generator=g).cuda()
+    pos = torch.cat([torch.arange(b, a + b) for a, b in zip(lens, past)]).int().cuda()
+    ent = torch.cat([torch.full((a,), i) for i, a in enumerate(lens)]).int().cuda()
+    ind, ids = torch.tensor([0] + np.cumsum(need).tolist(), dtype=torch.int32).cuda(), torch.randperm(sum(need), generator=g).int().cuda()
+    sink, gate = torch.randn(H, generator=g).bfloat16().cuda(), torch.randn(T, H * vdim, generator=g).bfloat16().cuda()
+    outs = []
+    for entry, rows, plain in (("maps", 16, 1), ("maps", tile_rows, 0), ("opt", tile_rows, 0)):
+        t = B.attention_tiles(lens, H // G, "cuda", rows)
+        out = torch.full((T, H * vdim), float("nan"), dtype=torch.bfloat16, device="cuda")
+        a = B.AttnOptions(maps=2, lambda_=0.3, softcap=o.get("cap", 0.0), window=o.get("window", 0), block=o.get("block", 0),
+                          sink=sink.data_ptr() if "sink" in o else None, head_norm=int(o.get("norm", False)), norm_eps=1e-6,
+                          gate=gate.data_ptr() if "gate" in o else None, gate_stride=H * vdim, gate_kind=o.get("gate", 0), n_split=1, plain=plain,
+                          tile_rows=rows if rows > 16 else 0)
+        status = getattr(B.ffi.lib(), "pegainfer_paged_attention_" + entry)(
+            q.data_ptr(), cache.data_ptr(), stride, 0, v_off, page, pos.data_ptr(), ent.data_ptr(), ind.data_ptr(), ids.data_ptr(), H, G, dim, vdim,
+            dim ** -0.5, 1.0, *(c.data_ptr() for c in t), t[0].numel(), out.data_ptr(), out.stride(0), ctypes.addressof(a), 0, B._stream())
+        if entry == "opt":
+            assert status != 0                    # one map only
+        else:
+            assert status == 0
+            outs.append(out.float().cpu())
+    assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * 1.3 * outs[0].abs().max()
