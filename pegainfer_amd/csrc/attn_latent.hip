@@ -268,7 +268,8 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(float* __restric
 // dims 4c..4c+3 of key row j, and lane i receives dim i of the four rows - so the latent tile is staged once, row-major, and
 // serves both products.  Every head of a token reads the same entries, so a tile of 64 rows (8 tokens x 8 heads, or one
 // decoded token's heads) shares each staged key tile.  The next key tile's global loads are issued into registers before the
-// current tile's products and written to LDS after them.  Softmax state (max, sum) and the output accumulators are fp32; q and
+// current tile's products and written to LDS after them.  KH = 2: eight waves, the second four on keys 32 .. 63 of tiles of 64, with a
+// softmax state of their own; the two meet in LDS at the end.  Softmax state (max, sum) and the output accumulators are fp32; q and
 // the weights are rounded to bf16 where they enter the matrix cores.  Keys are split over blockIdx.y like the plain form.
 constexpr int kTileRows = 64, kTileKeys = 32;
 constexpr int kLatPrefetch = 10;     // 16-byte chunks per thread and key tile: 32 keys x (E / 8) <= 2560 chunks, E <= 640
@@ -277,8 +278,8 @@ constexpr int kLatPrefetch = 10;     // 16-byte chunks per thread and key tile: 
 // the longer unroll of the scores 16 heads of 512 + 64, prompts of 300 - 900 tokens 225 -> 208 us, one of 1800 436 -> 387, 100 tokens behind 2000
 // 317 -> 280.  A maximum that follows with a lag (no rescaling of most tiles) would take 194 us, but rounds the largest weight, which is
 // exactly one here: 1.5 times the error on peaked rows.
-template <int ND, bool FULL>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
+template <int ND, bool FULL, int KH>
+__global__ __launch_bounds__(256 * KH) void latent_attn_mfma_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
                                                                const uint16_t* __restrict__ cache, int64_t page_stride,
                                                                int64_t layer_off, int page_size,
                                                                const int32_t* __restrict__ positions,
@@ -291,46 +292,45 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
                                                                int max_splits, LatentCut cut) {
   extern __shared__ __align__(16) uint8_t lat_smem[];
   typedef short v4s_t __attribute__((ext_vector_type(4)));
+  constexpr int N = 256 * KH, KEYS = kTileKeys * KH;
   const int E = r + dr, Epad = (E + 31) & ~31;
   const int qs = Epad + 8, cs = Epad + 8;                          // LDS row strides (bf16 elements), 16-byte multiples
   uint16_t* Qs = reinterpret_cast<uint16_t*>(lat_smem);            // [64][qs]
-  uint16_t* Ck = Qs + kTileRows * qs;                              // [32][cs]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  uint16_t* Ck = Qs + kTileRows * qs;                              // [KEYS][cs]
+  const int tid = threadIdx.x, wave = (tid >> 6) & 3, kh = tid >> 8, lane = tid & 63, l15 = lane & 15, g = lane >> 4;
   const int row0 = tile_row0[blockIdx.x], cnt = tile_rows[blockIdx.x], split = blockIdx.y;
   const int t_first = row0 / H, t_last = (row0 + cnt - 1) / H;
   const int pmax = positions[t_last];
   const int j_lo = split * cut.grain;
   if (j_lo > pmax) return;
-  const int j_hi = cut.end_of(split, pmax + 1), j_step = cut.step(kTileKeys, max_splits);
+  const int j_hi = cut.end_of(split, pmax + 1), j_step = cut.step(KEYS, max_splits);
   const int32_t* pages = page_ids + page_indptr[token_req[t_first]];
-  const int nchunk = E >> 3, tile_chunks = kTileKeys * nchunk;
+  const int nchunk = E >> 3, tile_chunks = KEYS * nchunk;
   // this thread's chunks of a key tile: key kk, element offset ch * 8 - fixed for the whole loop, so the integer divisions
   // happen once (a wave64 VALU instruction costs four cycles; an emulated division about forty of them)
   u32x4 pre[kLatPrefetch];
-  int ck_kk[kLatPrefetch], ck_el[kLatPrefetch];
+  int ck[kLatPrefetch];                                              // key << 16 | element
 #pragma unroll
   for (int i = 0; i < kLatPrefetch; ++i) {
-    const int c = tid + i * 256;
-    const int kk = c < tile_chunks ? c / nchunk : -1;
-    ck_kk[i] = kk;
-    ck_el[i] = kk < 0 ? 0 : (c - kk * nchunk) * 8;
+    const int c = tid + i * N;
+    ck[i] = c < tile_chunks ? c / nchunk << 16 | c % nchunk * 8 : -1;
   }
   const int pshift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int i = 0; i < kLatPrefetch; ++i) {
-      if (ck_kk[i] >= 0) {
-        const int j = min(j0 + ck_kk[i], j_hi - 1);
+      if (ck[i] >= 0) {
+        const int j = min(j0 + (ck[i] >> 16), j_hi - 1);
         const int pg = pshift >= 0 ? j >> pshift : j / page_size;
         const int slot = pshift >= 0 ? j & (page_size - 1) : j - pg * page_size;
-        pre[i] = *reinterpret_cast<const u32x4*>(cache + (int64_t)pages[pg] * page_stride + layer_off + (int64_t)slot * E + ck_el[i]);
+        pre[i] = *reinterpret_cast<const u32x4*>(cache + (int64_t)pages[pg] * page_stride + layer_off + (int64_t)slot * E + (ck[i] & 0xFFFF));
       }
     }
   };
   fetch(j_lo);
   {  // q rows -> bf16 in LDS, eight values per step; only the 16-row blocks that hold rows are staged
     const int qchunks = Epad >> 3, rows_staged = min(kTileRows, (cnt + 15) & ~15);
-    for (int c = tid; c < rows_staged * qchunks; c += 256) {
+    for (int c = tid; c < rows_staged * qchunks; c += N) {
       const int row = c / qchunks, k = (c - row * qchunks) * 8;
       u32x4 v = {0u, 0u, 0u, 0u};
       if (row < cnt && k < E) {
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
       *reinterpret_cast<u32x4*>(Qs + row * qs + k) = v;
     }
   }
-  for (int i = tid; i < kTileKeys * (Epad - E); i += 256) Ck[(i / (Epad - E)) * cs + E + i % (Epad - E)] = 0;
+  for (int i = tid; i < KEYS * (Epad - E); i += N) Ck[(i / (Epad - E)) * cs + E + i % (Epad - E)] = 0;
   const int my_row = wave * 16 + l15;
   const int pq = my_row < cnt ? positions[(row0 + my_row) / H] : -1;
   const bool wave_live = wave * 16 < cnt;                            // a wave without rows only helps staging
@@ -350,21 +350,22 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
   for (int d = 0; d < ND; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   // per-lane element offset of the transposed reads inside the key tile: key row 4g + (l15 >> 2), dims 4 (l15 & 3) ..
-  const int tr_off = (4 * g + (l15 >> 2)) * cs + 4 * (l15 & 3);
+  const int tr_off = (kTileKeys * kh + 4 * g + (l15 >> 2)) * cs + 4 * (l15 & 3);
   for (int j0 = j_lo; j0 < j_hi; j0 += j_step) {
     __syncthreads();                                                 // the previous tile's reads are done
 #pragma unroll
     for (int i = 0; i < kLatPrefetch; ++i)
-      if (ck_kk[i] >= 0) *reinterpret_cast<u32x4*>(Ck + ck_kk[i] * cs + ck_el[i]) = pre[i];
+      if (ck[i] >= 0) *reinterpret_cast<u32x4*>(Ck + (ck[i] >> 16) * cs + (ck[i] & 0xFFFF)) = pre[i];
     __syncthreads();
     if (j0 + j_step < j_hi) fetch(j0 + j_step);
-    if (!wave_live) continue;
+    const int jw = j0 + kTileKeys * kh;                              // this wave's keys of the tile
+    if (!wave_live || jw >= j_hi) continue;
     // two independent accumulator pairs over alternating k slices: with one wave per SIMD the LDS read -> MFMA -> MFMA chain
     // of a single pair would run at its latency
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f}, s3 = {0.f, 0.f, 0.f, 0.f};
     const uint16_t* qp = Qs + my_row * qs + g * 8;
-    const uint16_t* kp0 = Ck + l15 * cs + g * 8;
-    const uint16_t* kp1 = Ck + (16 + l15) * cs + g * 8;
+    const uint16_t* kp0 = Ck + (kTileKeys * kh + l15) * cs + g * 8;
+    const uint16_t* kp1 = kp0 + 16 * cs;
     int kb = 0;
 #pragma unroll 3
     for (; kb + 64 <= Epad; kb += 64) {
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int j = j0 + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4);
+      const int j = jw + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4);
       const float v = (i < 4 ? s0[i] : s1[i - 4]) * scale;
       sc[i] = (j <= pq && j < j_hi) ? v : -INFINITY;
       mx = fmaxf(mx, sc[i]);
@@ -428,6 +429,25 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
       const bf16x8_t cv = __builtin_bit_cast(bf16x8_t, u32x4{w0.x, w0.y, w1.x, w1.y});
       o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cv, pv, o[d], 0, 0, 0);
     }
+  }
+  if constexpr (KH == 2) {                                           // the two halves of the keys meet in LDS
+    __syncthreads();
+    f32x4* fold = reinterpret_cast<f32x4*>(lat_smem);                // [4][ND][64], then [4][64][2]
+    float* ml = reinterpret_cast<float*>(fold + 4 * ND * 64) + (wave * 64 + lane) * 2;
+    if (kh == 1) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) fold[(wave * ND + d) * 64 + lane] = o[d];
+      ml[0] = m;
+      ml[1] = l;
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const float m1 = ml[0], m_all = fmaxf(m, m1), m_use = m_all == -INFINITY ? 0.f : m_all;
+    const float w0 = __expf(m - m_use), w1 = __expf(m1 - m_use);
+    l = l * w0 + ml[1] * w1;
+    m = m_all;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = o[d] * w0 + fold[(wave * ND + d) * 64 + lane] * w1;
   }
   if (my_row >= cnt) return;
   const int own_splits = cut.splits_of(pq + 1, max_splits);
@@ -744,22 +764,30 @@ struct LatentCall {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) == hipSuccess;
   }
   template <typename A, typename K>
-  void run(K kern, int subs, size_t lds) const {
-    kern<<<dim3(n_tiles, sp, subs), 256, lds, s>>>(qc, o_lat, static_cast<const A*>(cache), page_stride, layer_off, page_size, positions, token_req,
+  void run(K kern, int subs, size_t lds, int threads = 256) const {
+    kern<<<dim3(n_tiles, sp, subs), threads, lds, s>>>(qc, o_lat, static_cast<const A*>(cache), page_stride, layer_off, page_size, positions, token_req,
                                            page_indptr, page_ids, tile_row0, tile_rows, H, r, dr, scale, ws, n_tokens, sp, cut);
   }
   template <int ND>
   void wide() const {
-    if (r == ND * 16) wide_form<ND, true>();
-    else wide_form<ND, false>();
+    // A second set of waves, on the other half of tiles of 64 keys, where one workgroup's rows and keys fill a compute unit's LDS anyhow and both halves'
+    // keys fit (entries of 417 to 608 values): each SIMD has two chains to work on.  16 heads of 512 + 64, four prompts of up to 900 tokens 214 -> 156 us
+    // (longest tiles first: 179).  Keys dealt in runs of 32 stay with one set.
+    const size_t one = tile_lds(1);
+    if (2 * one > kCuLds && tile_lds(2) <= 159 * 1024 && !(cut.dealt && sp > 1)) {
+      if (r == ND * 16) wide_form<ND, true, 2>();
+      else wide_form<ND, false, 2>();
+    } else if (r == ND * 16) wide_form<ND, true, 1>();
+    else wide_form<ND, false, 1>();
   }
-  template <int ND, bool FULL>
+  static constexpr size_t kCuLds = 160 * 1024;
+  size_t tile_lds(int kh) const { return (size_t)(kTileRows + kh * kTileKeys) * (((r + dr + 31) & ~31) + 8) * 2; }
+  template <int ND, bool FULL, int KH>
   void wide_form() const {
-    auto kern = &latent_attn_mfma_kernel<ND, FULL>;
+    auto kern = &latent_attn_mfma_kernel<ND, FULL, KH>;
     static const bool once = all_lds(kern);
     (void)once;
-    const int Epad = (r + dr + 31) & ~31;
-    run<uint16_t>(kern, 1, (size_t)(kTileRows + kTileKeys) * (Epad + 8) * 2);
+    run<uint16_t>(kern, 1, std::max(tile_lds(KH), KH == 2 ? (size_t)4 * 64 * (ND * 16 + 8) : 0), 256 * KH);
   }
   template <typename A, int ND, int RB>
   void few_rows() const {

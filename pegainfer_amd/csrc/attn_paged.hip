@@ -892,7 +892,7 @@ static size_t mfma_attention_lds(int maps, int dim, int ncb) {
 // third of the LDS cycles repeat for bank conflicts.  1024 rows x 16 heads of 128: 28 us
 // causal (153 TFLOP/s), 86 us behind 3072 cached tokens, 103 us with a cap - against 39, 131 and 160 us with both tiles
 // passing through registers, values transposed on the way, scores shaped one by one and the maximum exchanged in every tile.
-// Two maps (of P / 2 values each, a key's halves): a stream per map, every value fragment read once for both.  Eight prompts of 350 - 700 tokens, 16 heads of
+// Two maps (of P / 2 values each, a key's halves): a stream per map, every value fragment read once for both.  Eight prompts of 350 - 700 tokens, 8 heads of
 // 2 x 64 over 128 values: 195 -> 56 us against tiles of 16 rows; the same prompts' block-masked layer of one map 65 -> 29 us.
 template <int P, int RG>
 struct RowsShape {

@@ -285,6 +285,14 @@ def test_latent_attention_matrix_core_form(shape, split_keys):
     assert float((o - plain).abs().mean()) < 2e-3
 
 
+# entries of 417 to 608 values take a second set of waves: both ends and one beyond each, ranks that fill their blocks and one that does not, tiles of keys
+# that end in either half
+@pytest.mark.parametrize("split_keys", [0, 128, 72])
+@pytest.mark.parametrize("shape", [(16, 384, 32, [40, 5]), (8, 400, 24, [70, 1, 9]), (16, 512, 64, [33, 2, 64]), (4, 512, 96, [100, 33]), (4, 512, 104, [21])])
+def test_latent_attention_two_sets_of_waves(shape, split_keys):
+    test_latent_attention_matrix_core_form(shape, split_keys)
+
+
 @pytest.mark.parametrize("split_keys", [0, 32, -3])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(8, 256, 64, [1, 1, 1]), (16, 512, 64, [1, 1]), (3, 16, 8, [5, 1, 9]), (40, 512, 128, [1]), (5, 272, 24, [3, 13, 1]),
