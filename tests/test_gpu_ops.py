@@ -369,6 +369,23 @@ def test_gemm_split3_mid_batch_matches_oracle_and_full_gemm(P):
         r0 += m
 
 
+@pytest.mark.parametrize("T", [17, 40, 100])
+@pytest.mark.parametrize("k_tiles", [8, 12, 16, 20, 24, 28, 32])          # two to eight K slices of four tiles and more
+def test_slice_sums_of_two_to_eight_slices(P, T, k_tiles):
+    """a row's outputs in one piece and in three == each other bit for bit, and the fp64 product within a bf16 rounding (2^-8) and fp32 sums"""
+    import torch
+    rng = np.random.default_rng(k_tiles)
+    ms, K = (96, 32, 4), 64 * k_tiles
+    W, X = rnd(rng, sum(ms), K, scale=0.05), rnd(rng, T, K)
+    Wd, Xd = to_dev(W), to_dev(X)
+    outs = [torch.empty((T, m), dtype=torch.bfloat16, device=Xd.device) for m in ms]
+    P.gemm_split3_into(Wd, Xd, *outs)
+    full = from_dev(P.gemm(Wd, Xd))
+    assert np.array_equal(bf16_bits(np.concatenate([from_dev(o) for o in outs], 1)), bf16_bits(full))
+    ref = X.astype(np.float64) @ W.astype(np.float64).T
+    assert (np.abs(full - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all()
+
+
 @pytest.mark.parametrize("ms", [(8192, 4096, 32, 32), (512, 512), (64, 8, 4, 12)])
 def test_gemm_split_n_outputs_equals_separate_gemms(P, ms):
     """2- and 4-output stacked GEMM (Qwen3.5 gate|up and qkv|z|b|a) == separate gemm_cuda calls, bit for bit."""
