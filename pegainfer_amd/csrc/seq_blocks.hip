@@ -257,15 +257,15 @@ __global__ __launch_bounds__(256) void group_rms_add_kernel(const float* x_in, c
 }
 
 // The norm-and-gate below for heads wider than a wave should walk alone (one norm over a whole row, say): a workgroup per (row, head).
-// VEC: rows, strides and pointers allow four values per load.
+// VEC: rows, strides and pointers allow four values per load.  first: the grid's first head.
 constexpr int kWideKeep = 4;
 template <typename A, bool VEC>
 __global__ __launch_bounds__(256) void wide_rms_gate_kernel(const float* __restrict__ o, const A* __restrict__ w, int w_per_head,
                                                             const A* __restrict__ gate, int64_t gate_stride, int gate_kind, float factor,
                                                             float eps, A* __restrict__ out, int64_t out_stride, int heads, int vdim,
-                                                            int gate_first) {
+                                                            int gate_first, int first) {
   __shared__ float red[4];
-  const int row = blockIdx.x, h = blockIdx.y;
+  const int row = blockIdx.x, h = first + blockIdx.y;
   const float* p = o + ((int64_t)row * heads + h) * vdim;
   const A* gr = gate + (int64_t)row * gate_stride + (int64_t)h * vdim;
   const A* wr = w + (w_per_head ? (int64_t)h * vdim : 0);
@@ -1182,13 +1182,14 @@ pegainfer_status_t pegainfer_head_gate_rms(const float* o, const void* w, int32_
   const int blocks = ceil_div((long)rows * heads, 4);
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        if (vdim > 512 && heads <= 65535) {
+        if (vdim > 512) {      // (the kernel below holds no more)
           const bool vec = vdim % 4 == 0 && gate_stride % 4 == 0 && out_stride % 4 == 0 && host_aligned16(o) && host_aligned16(w) &&
                            host_aligned16(gate) && host_aligned16(out);
           auto wide = [&](auto kern) {
-            kern<<<dim3(rows, heads), 256, 0, as_stream(stream)>>>(o, static_cast<const A*>(w), w_per_head, static_cast<const A*>(gate),
-                                                                   gate_stride, gate_kind, factor, eps, static_cast<A*>(out), out_stride,
-                                                                   heads, vdim, gate_first);
+            for (int first = 0; first < heads; first += 65535)      // as many heads as a grid has
+              kern<<<dim3(rows, std::min(heads - first, 65535)), 256, 0, as_stream(stream)>>>(
+                  o, static_cast<const A*>(w), w_per_head, static_cast<const A*>(gate), gate_stride, gate_kind, factor, eps, static_cast<A*>(out),
+                  out_stride, heads, vdim, gate_first, first);
           };
           if (vec) wide(wide_rms_gate_kernel<A, true>);
           else wide(wide_rms_gate_kernel<A, false>);

@@ -201,6 +201,21 @@ def test_norm_and_gate_of_heads_several_values_to_a_lane(dtype, heads, vd):
           R.rms(gated, 1e-6).reshape(7, -1) * w.double(), dtype, tol32=4e-6, tol16=4e-3)
 
 
+@pytest.mark.parametrize("vd", [513, 516])
+def test_norm_and_gate_of_wide_heads_beyond_a_grid(vd):
+    # more heads than a launch's grid has, wider than the kernel of one wave per head holds: one value and four to an access
+    heads = 65535 + 3
+    g = torch.Generator(device="cuda").manual_seed(vd)
+    o, z = (torch.randn(2, heads * vd, generator=g, device="cuda") for _ in range(2))
+    w = 1 + 0.2 * torch.randn(vd, generator=g, device="cuda")
+    for first in (True, False):
+        got = B().head_gate_rms(o, w, z, "silu", 1e-6, heads, vd, gate_first=first).view(2, heads, vd)
+        for h in (slice(0, 300), slice(heads - 300, heads)):      # both ends of the heads, in 64 bits
+            a, act = o.view(2, heads, vd)[:, h].double().cpu(), R.silu(z.view(2, heads, vd)[:, h].double().cpu())
+            ref = (R.rms(a * act, 1e-6) if first else R.rms(a, 1e-6) * act) * w.double().cpu()
+            close(got[:, h].cpu(), ref, "float32", tol32=4e-6)    # as for the narrow heads above
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("channels,taps", [(301, 4), (514, 3), (513, 8), (1026, 5)])
 def test_convolution_of_long_portions_in_walks_of_eight_rows(dtype, channels, taps):
