@@ -496,7 +496,7 @@ pegainfer_status_t pegainfer_conv_glu_step(const pegainfer_conv_glu_step_desc* q
 pegainfer_status_t pegainfer_fetch_words(void* dst, const void* pinned_src, const int32_t* pinned_count, pegainfer_stream_t stream);
 /* The end of a step's logits [rows][vocab], one launch: v = src (src_dtype) times scale, then cap * tanh(v / cap) where cap > 0; out32 = v,
  * out16 = v rounded to bf16; with out_tokens the greedy token of every row of out16 (ties -> lowest index; state_scratch as in
- * pegainfer_batched_top1).  src may be out32 (fp32) or, with scale 1 and no cap, out16 (bf16). */
+ * pegainfer_batched_top1).  src may be out32 (fp32) or, with scale 1 and no cap, out16 (bf16); other uses of one buffer are refused. */
 pegainfer_status_t pegainfer_logits_finish(const void* src, int32_t src_dtype, float* out32, Half* out16, float scale, float cap,
                                            int32_t vocab_size, int32_t rows, uint8_t* state_scratch, int32_t* out_tokens,
                                            pegainfer_stream_t stream);

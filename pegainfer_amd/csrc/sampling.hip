@@ -683,6 +683,10 @@ pegainfer_status_t pegainfer_logits_finish(const void* src, int32_t src_dtype, f
   constexpr pegainfer_status_t bad = static_cast<pegainfer_status_t>(hipErrorInvalidValue);
   if (rows <= 0) return 0;
   if (!src || !out32 || !out16 || vocab_size <= 0 || (out_tokens && !state_scratch)) return bad;
+  // in place: where type and values stay what they are, or in fp32
+  if (out32 == static_cast<const void*>(out16) || (src == out32 && src_dtype != kDtF32) ||
+      (src == out16 && (src_dtype != kDtBf16 || scale != 1.0f || cap > 0.f)))
+    return bad;
   const int wgs = std::min(top1_blocks(rows), ceil_div(vocab_size, 8 * 256));
   if (!by_dtype(src_dtype, [&](auto* t) {
         using T = std::remove_pointer_t<decltype(t)>;

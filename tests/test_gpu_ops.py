@@ -662,6 +662,22 @@ def test_logits_finish_gives_logits_their_bf16_image_and_the_greedy_tokens(P, ro
         assert B.logits_finish(x.cuda(), state, scale, cap, tokens=False)[2] is None and int(state.sum().item()) == 0
 
 
+def test_logits_finish_refuses_to_leave_outputs_that_disagree(P):
+    """in place where the type and (bf16) the values stay: anything else is an error and changes nothing"""
+    import torch
+    from pegainfer_amd import ops_blocks as B
+    rows, n = 2, 16
+    f32, b16 = torch.full((rows, n), 3.0, device="cuda"), torch.full((rows, n), 3.0, dtype=torch.bfloat16, device="cuda")
+    call = lambda src, dt, o32, o16, scale=1.0, cap=0.0: B.ffi.lib().pegainfer_logits_finish(  # noqa: E731
+        src.data_ptr(), dt, o32.data_ptr(), o16.data_ptr(), scale, cap, n, rows, None, None, B._stream())
+    F32, BF16 = B._dt(f32), B._dt(b16)
+    for args in ((b16, BF16, f32, b16, 0.5), (b16, BF16, f32, b16, 1.0, 15.0), (b16, F32, f32, b16), (f32, BF16, f32, b16), (f32, F32, f32, f32)):
+        assert call(*args) != 0, args[1:]
+    assert bool((f32 == 3.0).all()) and bool((b16 == 3.0).all())
+    assert call(b16, BF16, f32, b16) == 0 and call(f32, F32, f32, b16, 0.5) == 0
+    assert bool((f32 == 1.5).all()) and bool((b16 == 1.5).all())
+
+
 @pytest.mark.parametrize("n", [5, 1000, 151936])
 def test_argmax_and_top1_lowest_index_ties(P, n):
     import torch
