@@ -429,8 +429,9 @@ pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, co
  *                 n = sum_j coef[j] * stack[j * stack_stride ..] + coef[n_mix - 1] * r, j < n_mix - 1      -> mix_out (fp32)
  *   conv        = n + sum over four taps of conv_w[c][tap] * (conv_state tail, n)                              -> conv_out, the tail moved on
  *                 (pegainfer_time_conv_step: mode 1, four taps)
- * Outputs and parts whose pointer is NULL are left out (groups == 0 without a gain: the sum alone).  Sizes: pegainfer_row_step_ok (state_off: of the
- * tail inside a slot); every row on 16 bytes (bf16 vectors on 8). */
+ * Outputs and parts whose pointer is NULL are left out (groups == 0 without a gain: the sum alone).  Parts that the form does not name, a
+ * bias without y, and x_out in place of x_in with a row_index are refused.  Sizes: pegainfer_row_step_ok (state_off: of the tail inside a
+ * slot); every row on 16 bytes (bf16 vectors on 8). */
 typedef struct {
   const float* x_in;
   const int32_t* row_index;

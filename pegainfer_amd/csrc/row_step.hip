@@ -238,6 +238,10 @@ pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfe
       (grouped && (!q->gain || (!q->y && !routed) || q->n_mix < 0 || (q->n_mix > 0 && !q->coef) || (q->n_mix > 1 && !q->stack) ||
                    (q->conv_w && q->n_mix < 1) || q->stack_stride % 4)))
     return bad;
+  // what the other form alone works on, and rows picked from a matrix that other workgroups write
+  if (grouped ? q->row_index || q->add_rows || q->add_vec || q->n_out : q->stack || q->coef || q->mix_out || q->xb_out) return bad;
+  if (q->bias && !q->y) return bad;
+  if (q->row_index && q->x_out == q->x_in) return bad;
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         auto a = [](const void* p) { return static_cast<const A*>(p); };

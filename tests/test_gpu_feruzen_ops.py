@@ -508,3 +508,25 @@ def test_row_step_joins_norms_mixes_and_convolves(dtype, d, groups):
     pick, no, xd, on = torch.tensor([2, 2, 0, 1, 2], dtype=torch.int32).cuda(), torch.zeros(5, d, device="cuda"), x.cuda(), one.cuda()
     B.row_step(dt, 5, d, x_in=xd, row_index=pick, gain=on, eps=eps, n_out=no)
     close_(no, (x.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + eps) * one.double())[pick.cpu().long()], False)
+
+
+def test_row_step_refuses_what_its_form_leaves_out():
+    """parts of the other form, a bias without an output to add it to, and rows picked from the matrix that is written: an error, and nothing is written"""
+    import importlib
+    B = importlib.import_module("pegainfer_amd.ops_blocks")
+    rows, d, dt = 3, 64, torch.bfloat16
+    ones = lambda *s, t=torch.float32: torch.ones(*s, dtype=t, device="cuda")  # noqa: E731
+    x, other, y, vec, pairs, weight = ones(rows, d), ones(rows, d), ones(rows, d, t=dt), ones(d, t=dt), ones(rows, d), ones(rows, 1)
+    pick = torch.tensor([2, 0, 1], dtype=torch.int32, device="cuda")
+    grouped, scalar = dict(x_in=x, x_out=x, y=y, gain=vec, groups=4, eps=1e-5), dict(x_in=x, x_out=x, y=y, gain=vec, eps=1e-5)
+    routed = dict(x_in=x, x_out=x, y_pairs=pairs, weight=weight, top=1, gain=vec, eps=1e-5)
+    for form, part in ([(grouped, p) for p in (dict(row_index=pick), dict(add_rows=other), dict(add_vec=vec), dict(n_out=other))] +
+                       [(scalar, p) for p in (dict(stack=other), dict(coef=vec), dict(mix_out=other), dict(xb_out=y), dict(row_index=pick))] +
+                       [(routed, dict(bias=vec)), (dict(routed, groups=4), dict(bias=vec)), (dict(scalar, y=None), dict(bias=vec))]):
+        with pytest.raises(RuntimeError):
+            B.row_step(dt, rows, d, **{k: v for k, v in dict(form, **part).items() if v is not None})
+        torch.cuda.synchronize()
+        assert all(bool((t == 1).all()) for t in (x, other, y, vec))
+    for form in (scalar, grouped, routed):
+        B.row_step(dt, rows, d, **dict(form, x_out=other))
+    B.row_step(dt, rows, d, **dict(scalar, row_index=pick, x_out=other))
