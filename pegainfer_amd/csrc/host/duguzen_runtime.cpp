@@ -27,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_capture.h"
 #include "kv_pool.h"
 #include "row_tiles.h"
 #include "step_io.h"
@@ -803,14 +804,11 @@ struct Model {
         if (g.first == key) exec = g.second;
       if (!exec) {
         if (graphs.size() >= kMaxGraphs) drop_graphs();      // no replay is in flight: every step ends with a synchronisation
-        hipGraph_t g = nullptr;
         DZ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
-        const hipError_t e = hipStreamEndCapture(stream, &g);
+        const hipError_t e = pst::end_capture(stream, rc == 0, &exec);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
-        DZ_HIP(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
-        DZ_HIP(hipGraphDestroy(g));
         graphs.emplace_back(key, exec);
       }
       DZ_HIP(hipGraphLaunch(exec, stream));

@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_capture.h"
 #include "kv_pool.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
@@ -809,13 +810,10 @@ struct Model35 {
           P35_HIP(hipGraphExecDestroy(graph_cache.front().second));
           graph_cache.erase(graph_cache.begin());
         }
-        hipGraph_t g = nullptr;
         P35_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = run_decode_kernels(c.n, c.rs, c.split);
-        hipError_t e = hipStreamEndCapture(stream, &g);
+        const hipError_t e = pst::end_capture(stream, rc == 0, &graph);
         if (rc || e != hipSuccess) { if (!rc) set_error("graph capture failed"); return -1; }
-        P35_HIP(hipGraphInstantiate(&graph, g, nullptr, nullptr, 0));
-        P35_HIP(hipGraphDestroy(g));
         graph_ids = c.key;
       }
       P35_HIP(hipGraphLaunch(graph, stream));

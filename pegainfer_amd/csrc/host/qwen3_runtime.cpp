@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_capture.h"
 #include "kv_pool.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
@@ -863,13 +864,10 @@ struct Model {
       const int gv = !c.split ? 0 : (oproj_plan && attn_oproj && c.padded <= pq::oproj_fused_max_batch() && !tp_comm && decode_mode >= 1 ? 2 : 1);
       hipGraphExec_t& exec = graphs[bi][gv];
       if (!exec) {  // capture once (cuda_graph.rs:36-55), thread-local mode
-        hipGraph_t graph = nullptr;
         PQ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = decode_kernels(c.padded, c.split, c.plan_slots);
-        hipError_t e = hipStreamEndCapture(stream, &graph);
+        const hipError_t e = pst::end_capture(stream, rc == 0, &exec);
         if (rc || e != hipSuccess) { set_error("graph capture failed: " + err); return -1; }
-        PQ_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-        PQ_HIP(hipGraphDestroy(graph));
       }
       PQ_HIP(hipGraphLaunch(exec, stream));
       return 0;

@@ -34,6 +34,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_capture.h"
 #include "kv_pool.h"
 #include "row_tiles.h"
 #include "seq_state.h"
@@ -1060,14 +1061,11 @@ struct Model {
       for (auto& g : graphs)
         if (g.first == key) exec = g.second;
       if (!exec) {
-        hipGraph_t g = nullptr;
         RX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
-        const hipError_t e = hipStreamEndCapture(stream, &g);
+        const hipError_t e = pst::end_capture(stream, rc == 0, &exec);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
-        RX_HIP(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
-        RX_HIP(hipGraphDestroy(g));
         graphs.emplace_back(key, exec);
       }
       RX_HIP(hipGraphLaunch(exec, stream));

@@ -25,6 +25,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_capture.h"
 #include "kv_pool.h"
 #include "row_tiles.h"
 #include "seq_state.h"
@@ -366,14 +367,11 @@ class StepModel {
       for (auto& g : graphs)
         if (g.first == key) exec = g.second;
       if (!exec) {
-        hipGraph_t g = nullptr;
         PSTEP_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : launches();
-        const hipError_t e = hipStreamEndCapture(stream, &g);
+        const hipError_t e = pst::end_capture(stream, rc == 0, &exec);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
-        PSTEP_HIP(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
-        PSTEP_HIP(hipGraphDestroy(g));
         graphs.emplace_back(key, exec);
       }
       PSTEP_HIP(hipGraphLaunch(exec, stream));

@@ -229,6 +229,48 @@ int main() {
     assert subprocess.run([str(tmp_path / "t")]).returncode == 0
 
 
+def test_a_capture_that_fails_leaves_no_graph_behind(tmp_path):
+    """csrc/host/graph_capture.h over a runtime of counters: the recording is destroyed once whether a launch was refused, the capture or the instantiation
+    failed or all went well, and only then is there an executable graph"""
+    import subprocess
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(r"""
+#pragma once
+enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999 };
+typedef int* hipStream_t;
+typedef int* hipGraph_t;
+typedef int* hipGraphExec_t;
+inline int graphs = 0, execs = 0, dummy = 0;
+inline bool bad_end = false, bad_make = false;
+inline hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { if (bad_end) return hipErrorUnknown; ++graphs; *g = &dummy; return hipSuccess; }
+inline hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, void*, char*, unsigned long) {
+  *e = &dummy;
+  if (bad_make) return hipErrorUnknown;
+  ++execs;
+  return hipSuccess;
+}
+inline hipError_t hipGraphDestroy(hipGraph_t) { --graphs; return hipSuccess; }
+""")
+    (tmp_path / "t.cpp").write_text(r"""
+#include "graph_capture.h"
+int main() {
+  hipGraphExec_t e = &dummy;
+  if (pst::end_capture(nullptr, false, &e) != hipSuccess || e || graphs || execs) return 1;      // a launch was refused
+  bad_end = true;
+  if (pst::end_capture(nullptr, true, &e) == hipSuccess || e || graphs || execs) return 2;
+  bad_end = false; bad_make = true;
+  if (pst::end_capture(nullptr, true, &e) == hipSuccess || e || graphs || execs) return 3;
+  bad_make = false;
+  return pst::end_capture(nullptr, true, &e) != hipSuccess || !e || graphs || execs != 1 ? 4 : 0;
+}
+""")
+    host = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc", "host")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", str(tmp_path), "-I", host, "-o", str(tmp_path / "t"), str(tmp_path / "t.cpp")], check=True)
+    assert subprocess.run([str(tmp_path / "t")]).returncode == 0
+    sources = [os.path.join(host, f) for f in os.listdir(host) if f.endswith((".cpp", ".h")) and f != "graph_capture.h"]
+    assert not [f for f in sources if "hipStreamEndCapture" in open(f).read()]      # every runtime ends its captures here
+
+
 def test_scratch_of_the_chunk_forms_is_bounded(built_libs):
     """256 MB of states (or one chunk's) however long the step, and the gates' 768 bytes per chunk and head beside them"""
     L = ffi.lib()
