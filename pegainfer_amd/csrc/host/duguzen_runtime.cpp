@@ -27,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "graph_cache.h"
 #include "graph_capture.h"
 #include "kv_pool.h"
 #include "row_tiles.h"
@@ -133,14 +134,14 @@ struct Model {
     int n, want; bool tokens, plain; int keys;
     bool operator==(const GraphKey& o) const { return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && keys == o.keys; }
   };
+  // captured decode steps, one per shape and context length rounded up to 256, 512, ... kGraphMaxKeys tokens.  A capture takes 0.6 - 0.9 ms, about two
+  // steps: with bands of 256 tokens a batch met a new one every 256 steps and a few batch sizes filled the cache; so a batch size has six.
   static constexpr int kGraphKeys = 256, kGraphMaxKeys = 8192;
-  static constexpr size_t kMaxGraphs = 64;
-  std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;   // captured decode steps, one per shape and rounded context length
+  int graph_keys_most = kGraphMaxKeys;
+  pst::GraphCache<GraphKey, hipGraphExec_t> graphs{64};
   bool graphs_on = [] { const char* e = getenv("PEGAINFER_DUGUZEN_GRAPH"); return !(e && e[0] == '0'); }();
-  void drop_graphs() {   // the buffers a graph was recorded over are about to move
-    for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
-    graphs.clear();
-  }
+  static void destroy_graph(hipGraphExec_t g) { (void)hipGraphExecDestroy(g); }
+  void drop_graphs() { graphs.drop(destroy_graph); }   // the buffers a graph was recorded over are about to move
   uint8_t* top1_state = nullptr;
   pst::StepIo io;
   // sampling scratch
@@ -594,20 +595,32 @@ struct Model {
     // decode-like steps (few rows) cut the keys finely so that one request's context spreads over many workgroups;
     // prompt-sized steps have rows enough and only cut very long contexts
     const int split_keys = T * (size_t)mx_heads <= 1024 ? 32 : 4096;
-    // A step of single tokens is captured; its grids hold the splits of a context rounded up to kGraphKeys, the ones past a row's own keys end at
-    // once.  Longer contexts than kGraphMaxKeys run eagerly: their scratch is not rounded up, and their attention hides the launches.
-    const bool captured = single && graphs_on && !tap_on && max_kv <= kGraphMaxKeys;
-    if (captured) max_kv = (max_kv + kGraphKeys - 1) / kGraphKeys * kGraphKeys;
-    const int64_t ws_need = pegainfer_latent_attention_workspace((int)T, mx_heads, mx_rank, max_kv, split_keys);
-    if ((size_t)ws_need > attn_ws_cap) {
-      DZ_HIP(hipStreamSynchronize(stream));
+    auto reserve = [&](int keys) -> hipError_t {      // scratch for contexts of so many tokens
+      const size_t need = (size_t)pegainfer_latent_attention_workspace((int)T, mx_heads, mx_rank, keys, split_keys);
+      if (need <= attn_ws_cap) return hipSuccess;
+      hipError_t e = hipStreamSynchronize(stream);
       drop_graphs();
       if (attn_ws) (void)hipFree(attn_ws);
       attn_ws = nullptr;
       attn_ws_cap = 0;
-      DZ_HIP(hipMalloc(reinterpret_cast<void**>(&attn_ws), (size_t)ws_need * 4));
-      attn_ws_cap = (size_t)ws_need;
+      if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&attn_ws), need * 4);
+      if (e == hipSuccess) attn_ws_cap = need;
+      else attn_ws = nullptr;
+      return e;
+    };
+    // A step of single tokens is captured; its grids hold the splits of the rounded context, the ones past a row's own keys end at once.  Contexts
+    // past graph_keys_most run eagerly and need no more scratch than their own: kGraphMaxKeys (their attention hides the launches), or what
+    // there has been memory for.
+    int rounded = kGraphKeys;
+    while (rounded < max_kv && rounded < kGraphMaxKeys) rounded *= 2;
+    bool captured = single && graphs_on && !tap_on && max_kv <= rounded && rounded <= graph_keys_most;
+    if (captured && reserve(rounded) == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      graph_keys_most = rounded / 2;
+      captured = false;
     }
+    if (captured) max_kv = rounded;
+    DZ_HIP(reserve(max_kv));
     // ---- pages, then the packed metadata block: tokens | positions | token_req | page_indptr | want | row tiles | page_ids
     //      (the page lists come last: everything before them sits at offsets that depend on the step's shape only, which a captured graph relies on)
     size_t total_pages = 0;
@@ -796,20 +809,17 @@ struct Model {
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and replayed; steps with
-    // prompt portions run eagerly.  4 requests of ~900 tokens, 62 launches a step: 10.0 -> 9.8 ms for their prompts and 16 steps.
+    // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step: 9.3 -> 9.05 ms for their prompts and 16 steps.
     if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, max_kv};
-      hipGraphExec_t exec = nullptr;
-      for (auto& g : graphs)
-        if (g.first == key) exec = g.second;
+      hipGraphExec_t exec = graphs.find(key);
       if (!exec) {
-        if (graphs.size() >= kMaxGraphs) drop_graphs();      // no replay is in flight: every step ends with a synchronisation
         DZ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         const int rc = io.fetch(S()) ? set_error("step: the metadata block cannot be fetched") : run_layers();
         const hipError_t e = pst::end_capture(stream, rc == 0, &exec);
         if (rc) return -1;
         if (e != hipSuccess) return set_error("graph capture failed");
-        graphs.emplace_back(key, exec);
+        graphs.add(key, exec, destroy_graph);      // no replay is in flight: every step ends with a synchronisation
       }
       DZ_HIP(hipGraphLaunch(exec, stream));
     } else if (run_layers()) {

@@ -203,6 +203,35 @@ def test_replayed_decode_steps_give_what_eager_ones_give(dtype, name):
         assert np.array_equal(a, b)
 
 
+def test_more_shapes_than_graphs_are_kept_and_contexts_past_the_last_graph():
+    """80 shapes of a decode step (1 - 8 requests, any number of wanted rows, tokens or not) twice in turn, more than the 64 graphs that are kept; then a
+    context that grows from the last one captured (8192 tokens) to one that runs eagerly.  The same bits as steps that are never captured."""
+    cfg = C.config_tiny()
+    w = C.random_weights(cfg, 5)
+    engs = [C.engine_for(cfg, w, "bfloat16", max_tokens=9000, max_requests=8) for _ in range(2)]
+    engs[1].debug_hidden_enable(True)
+    toks = C.tokens_for(cfg, 8220, 9)
+    shapes = [(n, k, t) for n in range(1, 9) for k in range(n + 1) for t in ((False, True) if k else (False,))]
+    assert len(shapes) == 80
+    out = []
+    for eng in engs:
+        r, got = [eng.new_request() for _ in range(8)], []
+        eng.step([(q, toks[i:i + 3 + 5 * i]) for i, q in enumerate(r)], want=[])
+        for step, (n, k, t) in enumerate(shapes + shapes):
+            res = eng.step([(q, [toks[step]]) for q in r[:n]], want=list(range(k)), logits=k > 0, tokens=t)
+            got += [] if not k else list(res) if t else [res]
+        for q in r[1:]:
+            eng.drop_request(q)
+        done = eng.seq_len(r[0])
+        eng.step([(r[0], toks[done:8180])], want=[])
+        for t in range(8180, 8210):
+            got.append(eng.step([(r[0], [toks[t]])]))
+        assert eng.seq_len(r[0]) == 8210
+        out.append(got)
+        eng.close()
+    assert len(out[0]) == len(out[1]) and all(np.array_equal(a, b) for a, b in zip(*out))
+
+
 def test_checkpoint_folder_through_the_registry_and_trace_replay(tmp_path):
     from safetensors.torch import save_file
     from pegainfer_amd import registry

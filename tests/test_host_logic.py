@@ -271,6 +271,35 @@ int main() {
     assert not [f for f in sources if "hipStreamEndCapture" in open(f).read()]      # every runtime ends its captures here
 
 
+def test_the_graph_that_goes_is_the_one_not_asked_for_the_longest(tmp_path):
+    """csrc/host/graph_cache.h: what was asked for stays beyond what was added earlier, one goes per addition, everything is destroyed once"""
+    import subprocess
+    (tmp_path / "t.cpp").write_text(r"""
+#include <set>
+#include "graph_cache.h"
+int main() {
+  int things[16];
+  std::multiset<int*> gone;
+  auto destroy = [&](int* p) { gone.insert(p); };
+  pst::GraphCache<int, int*> c(3);
+  if (c.find(0)) return 1;
+  for (int k = 0; k < 3; ++k) c.add(k, things + k, destroy);
+  if (!gone.empty() || c.find(0) != things || c.find(2) != things + 2) return 2;
+  c.add(3, things + 3, destroy);                              // 1 goes
+  if (gone != std::multiset<int*>{things + 1} || c.find(1) || c.find(0) != things) return 3;
+  c.add(4, things + 4, destroy);                              // 2 goes
+  if (gone != std::multiset<int*>{things + 1, things + 2} || c.find(2) || c.find(3) != things + 3 || c.find(0) != things || c.find(4) != things + 4) return 4;
+  c.drop(destroy);
+  if (gone != std::multiset<int*>{things, things + 1, things + 2, things + 3, things + 4} || c.find(0) || c.find(4)) return 5;
+  c.add(0, things + 5, destroy);
+  return c.find(0) != things + 5 || gone.size() != 5 ? 6 : 0;
+}
+""")
+    host = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc", "host")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", host, "-o", str(tmp_path / "t"), str(tmp_path / "t.cpp")], check=True)
+    assert subprocess.run([str(tmp_path / "t")]).returncode == 0
+
+
 def test_scratch_of_the_chunk_forms_is_bounded(built_libs):
     """256 MB of states (or one chunk's) however long the step, and the gates' 768 bytes per chunk and head beside them"""
     L = ffi.lib()
