@@ -501,7 +501,8 @@ pegainfer_status_t pegainfer_fetch_words(void* dst, const void* pinned_src, cons
 pegainfer_status_t pegainfer_logits_finish(const void* src, int32_t src_dtype, float* out32, Half* out16, float scale, float cap,
                                            int32_t vocab_size, int32_t rows, uint8_t* state_scratch, int32_t* out_tokens,
                                            pegainfer_stream_t stream);
-/* out[i] = cap * tanh(in[i] / cap) over n fp32 values (in place allowed) */
+/* out[i] = cap * tanh(in[i] / cap) over n fp32 values (in place allowed).  For a caller's own logits: an engine's are capped by
+ * pegainfer_logits_finish. */
 pegainfer_status_t pegainfer_softcap_rows(const float* in, float* out, int64_t n, float cap, pegainfer_stream_t stream);
 
 /* ---- several residual streams with learned mixing (hyper-connections) ----
@@ -860,12 +861,12 @@ pegainfer_status_t pegainfer_paged_attention(const float* q, const void* cache, 
  * block > 0: a key j is visible to position i only if j <= i and floor(j / block) == floor(i / block), blocks counted from
  * position 0 of the sequence.  sink: [heads] logits of dtype (or NULL) that join every softmax denominator as exp(sink), without
  * scale, key or value.  head_norm != 0: out / sqrt(mean(out^2) + norm_eps) over the head's vdim values.  `factor` comes last.
- * n_split > 1: every tile's keys are dealt in tiles of 64 to n_split workgroups (split z takes key tiles z, z + n_split, ...:
- * the grid does not depend on the contexts' lengths) whose softmax states a second launch folds in split order - for steps of
- * few rows over long contexts (decoding); `workspace` then holds pegainfer_paged_attention_workspace(...) floats.
+ * n_split > 1 (64 at most): every tile's keys are dealt in tiles of 64 to n_split workgroups (split z takes key tiles z, z + n_split, ...:
+ * the grid does not depend on the contexts' lengths) whose softmax states a second launch folds, every fourth split in a wave and the waves
+ * in order - for steps of few rows over long contexts (decoding); `workspace` then holds pegainfer_paged_attention_workspace(...) floats.
  * Two kernels behind the entry: a bf16 cache runs on the matrix cores (q and the softmax weights rounded to bf16 where they enter
  * them; scores, maxima, sums and outputs fp32) unless plain != 0; an fp32 cache, or plain, runs the fp32-FMA kernel.
- * pegainfer_paged_attention is the plain kernel's plain form. */
+ * pegainfer_paged_attention is the plain kernel's plain form; the engines call pegainfer_paged_attention_opt and _maps. */
 pegainfer_status_t pegainfer_paged_attention_ex(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,
                                                 int64_t v_cache_off, int32_t page_size, const int32_t* positions,
                                                 const int32_t* row_entry, const int32_t* page_indptr, const int32_t* page_ids,

@@ -1041,74 +1041,74 @@ __global__ __launch_bounds__(RG * 128) void paged_attention_rows_kernel(
     bf16x8_t pf[MAPS];
 #pragma unroll
     for (int m = 0; m < MAPS; ++m) {
-    f32x4 (&sc)[2] = maps[m];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sc[t][r] *= f0;
-    if (form.softcap > 0.f) soft_cap8(sc, form.softcap, inv_cap);
-    if (form.dist_bias) {
-      float bias[2][4];
+      f32x4 (&sc)[2] = maps[m];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) bias[t][r] = form.dist_bias[(int64_t)max(0, min(dist - 16 * t - r, form.n_dist - 1)) * H + rqh];
+        for (int r = 0; r < 4; ++r) sc[t][r] *= f0;
+      if (form.softcap > 0.f) soft_cap8(sc, form.softcap, inv_cap);
+      if (form.dist_bias) {
+        float bias[2][4];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[t][r] += bias[t][r];
-    }
-    if (form.dist_slope) {
+          for (int r = 0; r < 4; ++r) bias[t][r] = form.dist_bias[(int64_t)max(0, min(dist - 16 * t - r, form.n_dist - 1)) * H + rqh];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[t][r] = fmaf(-rsl, (float)(dist - 16 * t - r), sc[t][r]);
-    }
-    if (options) {
+          for (int r = 0; r < 4; ++r) sc[t][r] += bias[t][r];
+      }
+      if (form.dist_slope) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[t][r] *= kLog2e;
-    }
-    if constexpr (decltype(masked)::value) {
+          for (int r = 0; r < 4; ++r) sc[t][r] = fmaf(-rsl, (float)(dist - 16 * t - r), sc[t][r]);
+      }
+      if (options) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kp = kb + 16 * t + 4 * lg + r;
-          if (!(kp <= rpos && (kp >= rlo || kp < form.keep_first))) sc[t][r] = -INFINITY;
+          for (int r = 0; r < 4; ++r) sc[t][r] *= kLog2e;
+      }
+      if constexpr (decltype(masked)::value) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kp = kb + 16 * t + 4 * lg + r;
+            if (!(kp <= rpos && (kp >= rlo || kp < form.keep_first))) sc[t][r] = -INFINITY;
+          }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int kp = kb + 16 * (i >> 1) + 4 * lg + 2 * (i & 1);
+          auto seen = [&](int j) { return j <= last && (j >= first_lo || j < form.keep_first); };
+          see[i] = (seen(kp) ? 0xFFFFu : 0u) | (seen(kp + 1) ? 0xFFFF0000u : 0u);
         }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kp = kb + 16 * (i >> 1) + 4 * lg + 2 * (i & 1);
-        auto seen = [&](int j) { return j <= last && (j >= first_lo || j < form.keep_first); };
-        see[i] = (seen(kp) ? 0xFFFFu : 0u) | (seen(kp + 1) ? 0xFFFF0000u : 0u);
       }
-    }
-    float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])), fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
-    if (__any(!(tmax <= mrun[m] + kJump))) {            // uniform; the first keys of a row always, a NaN too
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-      const float mnew = fmaxf(mrun[m], tmax);
-      const float corr = __builtin_amdgcn_exp2f(mrun[m] - (mnew == -INFINITY ? 0.f : mnew));   // a row that has met no key yet: 0, and nothing to scale
-      lrun[m] *= corr;
+      float tmax = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])), fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
+      if (__any(!(tmax <= mrun[m] + kJump))) {            // uniform; the first keys of a row always, a NaN too
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+        const float mnew = fmaxf(mrun[m], tmax);
+        const float corr = __builtin_amdgcn_exp2f(mrun[m] - (mnew == -INFINITY ? 0.f : mnew));   // a row that has met no key yet: 0, and nothing to scale
+        lrun[m] *= corr;
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) { o[m][cb].x *= corr; o[m][cb].y *= corr; o[m][cb].z *= corr; o[m][cb].w *= corr; }
-      mrun[m] = mnew;
-    }
-    const float mref = mrun[m] == -INFINITY ? 0.f : mrun[m];
-    uint32_t pb[4];
-    float psum = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const uint32_t w = pack_bf2(__builtin_amdgcn_exp2f(sc[t][r] - mref), __builtin_amdgcn_exp2f(sc[t][r + 1] - mref));
-        pb[2 * t + (r >> 1)] = w;
-        psum += bf_lo(w) + bf_hi(w);                 // the sum of the weights as they are multiplied
+        for (int cb = 0; cb < NCB; ++cb) { o[m][cb].x *= corr; o[m][cb].y *= corr; o[m][cb].z *= corr; o[m][cb].w *= corr; }
+        mrun[m] = mnew;
       }
-    lrun[m] += psum;
-    pf[m] = __builtin_bit_cast(bf16x8_t, u32x4{pb[0], pb[1], pb[2], pb[3]});
+      const float mref = mrun[m] == -INFINITY ? 0.f : mrun[m];
+      uint32_t pb[4];
+      float psum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          const uint32_t w = pack_bf2(__builtin_amdgcn_exp2f(sc[t][r] - mref), __builtin_amdgcn_exp2f(sc[t][r + 1] - mref));
+          pb[2 * t + (r >> 1)] = w;
+          psum += bf_lo(w) + bf_hi(w);                 // the sum of the weights as they are multiplied
+        }
+      lrun[m] += psum;
+      pf[m] = __builtin_bit_cast(bf16x8_t, u32x4{pb[0], pb[1], pb[2], pb[3]});
     }
     typedef v4s_t __attribute__((address_space(3)))* lds_v4_t;
     const uint32_t vt = ring + (uint32_t)(stage * 2 * Sh::kTile + Sh::kTile);

@@ -241,7 +241,7 @@ pegainfer_status_t pegainfer_relu_sq(const void* x, void* out, int64_t n, int32_
   if (n <= 0) return 0;
   if (!by_dtype(dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-if (n >= 8 * 64 * 1024 && host_aligned16(x) && host_aligned16(out))   // (a wave for each SIMD)
+        if (n >= 8 * 64 * 1024 && host_aligned16(x) && host_aligned16(out))   // (a wave for each SIMD)
           relu_sq_kernel<A, 8><<<grid_for((n + 7) / 8), 256, 0, as_stream(stream)>>>(static_cast<const A*>(x), static_cast<A*>(out), n);
         else
           relu_sq_kernel<A, 1><<<grid_for(n), 256, 0, as_stream(stream)>>>(static_cast<const A*>(x), static_cast<A*>(out), n);
