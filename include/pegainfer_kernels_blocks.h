@@ -38,6 +38,20 @@ pegainfer_status_t pegainfer_dyt_add_norm(float* x, const void* y, const void* p
                                           const void* post_b, const void* next_alpha, const void* next_w,
                                           const void* next_b, void* out, int32_t d, int32_t rows, int32_t dtype,
                                           pegainfer_stream_t stream);
+/* The router of a feed-forward behind a row that a launch leaves (pegainfer_dyt_step_routed, pegainfer_row_step_routed, pegainfer_join_rms_routed): logits =
+ * w row (the row as it is stored; w [experts, d], and one row more where gate_logit is given: its logit goes to gate_logit[row * gate_stride]), then the
+ * selection of pegainfer_route_plan into out_expert / out_weight [rows, top].  For bf16 rows; the sizes it takes are router_tail_ok's. */
+typedef struct {
+  const void* w;
+  const void* correction;
+  int32_t* out_expert;
+  float* out_weight;
+  float* gate_logit;
+  int64_t gate_stride;
+  int32_t experts, n_groups, keep_groups, top, score_kind, group_kind, renorm;
+  float factor;
+} pegainfer_router_tail_desc;
+int32_t pegainfer_router_tail_ok(int32_t experts, int32_t has_gate, int32_t d, int32_t dtype);
 /* These in one launch around each row, every part optional: x starts as embed[token_ids[row]] (embed given) or is read in place or, without being
  * written, through row_index;  x += dyt(v; post) with v = y rows of dtype or the weighted sum of routed experts (pegainfer_route_combine);
  * out = dyt(x; next).  d % 4 == 0; fp32 rows on 16 bytes, bf16 ones on 8. */
@@ -60,6 +74,7 @@ typedef struct {
   int32_t d, rows, dtype;
 } pegainfer_dyt_step_desc;
 pegainfer_status_t pegainfer_dyt_step(const pegainfer_dyt_step_desc* q, pegainfer_stream_t stream);
+pegainfer_status_t pegainfer_dyt_step_routed(const pegainfer_dyt_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream);
 /* rows of an fp32 matrix gathered by index: out[i, :] = x[rows_index[i], :] (the positions whose logits are wanted) */
 pegainfer_status_t pegainfer_gather_rows_f32(const float* x, const int32_t* rows_index, float* out, int32_t d,
                                              int32_t n_rows, pegainfer_stream_t stream);
@@ -125,6 +140,19 @@ typedef struct {
   int64_t shared_m_stride, shared_group_stride, shared_up;
 } pegainfer_expert_rows_desc;
 pegainfer_status_t pegainfer_expert_rows(const pegainfer_expert_rows_desc* q, pegainfer_stream_t stream);
+/* The same straight from the choices expert [rows, top] of rows <= 16 rows, without a table (g's table and row indices NULL): the rows of group e are
+ * the pairs (row * top + choice) that name e, numbers from `experts` on name none.  y rows by pair; x row = the pair's row, or with
+ * x_by_pair the pair.  A shared expert's positions count from shared_pos0 as above (x row = row, or with x_by_pair the position).
+ * tiles (NULL: none; PEGAINFER_CHOSEN_WORDS words): a launch without x_by_pair leaves there which pairs its workgroups found, one with x_by_pair behind it
+ * and the same choices reads them.  expert_rows_chosen_ok says which sizes are taken. */
+#define PEGAINFER_CHOSEN_WORDS 1536
+typedef struct {
+  const int32_t* expert;
+  int32_t rows, top, experts, x_by_pair;
+  int32_t* tiles;
+} pegainfer_chosen_desc;
+int32_t pegainfer_expert_rows_chosen_ok(int32_t rows, int32_t top, int32_t experts);
+pegainfer_status_t pegainfer_expert_rows_chosen(const pegainfer_expert_rows_desc* q, const pegainfer_chosen_desc* chosen, pegainfer_stream_t stream);
 
 /* ---- attention over a paged latent cache ----
  * Cache: page-first; one layer's entry of one token = [c: rank values | kr: rot values], at
@@ -422,6 +450,8 @@ typedef struct {
 pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfer_stream_t stream);
 /* with y_pairs: `add` is the sum of n_add fp32 rows, add_pairs[(j * rows + row) * d ..], j < n_add (q->add NULL) */
 pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream);
+/* with the router behind n_out's row; not with y_pairs */
+pegainfer_status_t pegainfer_join_rms_routed(const pegainfer_join_rms_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream);
 /* A decode step's row between two matrix products, one launch (every entry brings one row: row e is entry e's).
  *   v   = y + bias rows of dtype, or with y_pairs the weighted sum of routed experts (pegainfer_route_combine_gated / _pairs)
  *   groups == 0:  r = x_in[row_index] + mult * v + add_rows + add_vec  -> x_out;   n = r / sqrt(mean(r^2) + eps) * gain[0]  -> n_out (fp32)
@@ -468,6 +498,8 @@ typedef struct {
 } pegainfer_row_step_desc;
 int32_t pegainfer_row_step_ok(int32_t d, int32_t groups, int32_t taps, int64_t state_off, int64_t slot_stride);
 pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream);
+/* with the router behind conv_out's row (groups == 0) or xb_out's row (groups > 0); not with y_pairs */
+pegainfer_status_t pegainfer_row_step_routed(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream);
 /* out[row, i] = act(gate[row, i]) * up[row, i], i < I; gate and up are column ranges of rows with stride in_row_stride (elements of
  * dtype).  act 0 = silu, 1 = relu, 2 = gelu (tanh form), 3 = gelu (exact form) */
 enum { PEGAINFER_ACT_SILU = 0, PEGAINFER_ACT_RELU = 1, PEGAINFER_ACT_GELU_TANH = 2, PEGAINFER_ACT_GELU_ERF = 3 };

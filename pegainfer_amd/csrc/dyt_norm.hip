@@ -8,9 +8,7 @@
 //   dyt_step           all of these around one row: the stream read in place, through a row index or as an embedding row; a stored output or the
 //                      routed experts' weighted sum joins it; the next pre-norm
 // Memory-bound: 4 B read + 2-4 B written per element.
-#include "common.h"
-#include "typed.h"
-#include "pegainfer_kernels_blocks.h"
+#include "route_core.h"
 
 namespace pk {
 
@@ -72,45 +70,54 @@ struct DytStep {
   A* out;
   int d;
 };
-template <typename A>
-__global__ __launch_bounds__(256) void dyt_step_kernel(DytStep<A> p) {
-  const int row = blockIdx.x, i = (blockIdx.y * 256 + threadIdx.x) * 4;
-  if (i >= p.d) return;
+// T: the router of the feed-forward behind the row, which then lies in one workgroup
+template <typename A, int N = 256, typename T = NoTail>
+__global__ __launch_bounds__(N) void dyt_step_kernel(DytStep<A> p, RouterTail router) {
+  __shared__ typename T::Shared sh;
+  if (T::helps(router, p.d)) return;
+  T tail;
+  const int row = blockIdx.x, i = (blockIdx.y * N + threadIdx.x) * 4;
   const int64_t at = (int64_t)row * p.d + i;
-  float v[4], pw[4], pb[4], nw[4], nb[4];
-  if (p.embed) ld4(p.embed + (int64_t)p.ids[row] * p.d + i, v);
-  else ld4(p.x + (p.row_index ? (int64_t)p.row_index[row] * p.d + i : at), v);
-  const bool joins = p.y || p.pairs;
-  if (joins) { ld4(p.pw + i, pw); ld4(p.pb + i, pb); }
-  if (p.nw) { ld4(p.nw + i, nw); ld4(p.nb + i, nb); }
-  if (joins) {
-    float y[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.y) {
-      ld4(p.y + at, y);
-    } else {
-#pragma unroll 4
-      for (int c = 0; c < p.top; ++c) {
-        const float w = p.weight[(int64_t)row * p.top + c];
-        float t[4];
-        ld4(p.pairs + ((int64_t)row * p.top + c) * p.d + i, t);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) y[u] = fmaf(w, t[u], y[u]);
-      }
-      if constexpr (sizeof(A) == 2) {      // as a stored sum: a router behind it sees the same rows whichever launch made the sum
-#pragma unroll
-        for (int u = 0; u < 4; ++u) y[u] = bf16_round_f(y[u]);
-      }
-    }
-    const float a = ld(p.pa);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] += tanhf(a * y[u]) * pw[u] + pb[u];
+  const bool on = i < p.d, joins = p.y || p.pairs;
+  float v[4], pw[4], pb[4], nw[4], nb[4], y[4] = {0.f, 0.f, 0.f, 0.f};
+  if (on) {
+    if (p.embed) ld4(p.embed + (int64_t)p.ids[row] * p.d + i, v);
+    else ld4(p.x + (p.row_index ? (int64_t)p.row_index[row] * p.d + i : at), v);
+    if (joins) { ld4(p.pw + i, pw); ld4(p.pb + i, pb); }
+    if (p.nw) { ld4(p.nw + i, nw); ld4(p.nb + i, nb); }
+    if (p.y) ld4(p.y + at, y);
   }
-  if (!p.row_index && (joins || p.embed)) st4(p.x + at, v);
-  if (!p.nw) return;
-  const float a = ld(p.na);
+  tail.request(router, p.d);
+  if (on) {
+    if (joins) {
+      if (!p.y) {
+#pragma unroll 4
+        for (int c = 0; c < p.top; ++c) {
+          const float w = p.weight[(int64_t)row * p.top + c];
+          float t[4];
+          ld4(p.pairs + ((int64_t)row * p.top + c) * p.d + i, t);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) v[u] = tanhf(a * v[u]) * nw[u] + nb[u];
-  st4(p.out + at, v);
+          for (int u = 0; u < 4; ++u) y[u] = fmaf(w, t[u], y[u]);
+        }
+        if constexpr (sizeof(A) == 2) {      // as a stored sum: a router behind it sees the same rows whichever launch made the sum
+#pragma unroll
+          for (int u = 0; u < 4; ++u) y[u] = bf16_round_f(y[u]);
+        }
+      }
+      const float a = ld(p.pa);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] += tanhf(a * y[u]) * pw[u] + pb[u];
+    }
+    if (!p.row_index && (joins || p.embed)) st4(p.x + at, v);
+    if (p.nw) {
+      const float a = ld(p.na);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = tanhf(a * v[u]) * nw[u] + nb[u];
+      st4(p.out + at, v);
+      tail.put(sh, i, v);
+    }
+  }
+  tail.finish(router, sh, p.d, row);
 }
 
 __global__ __launch_bounds__(256) void gather_rows_f32_kernel(const float* __restrict__ x, const int32_t* __restrict__ idx,
@@ -206,7 +213,7 @@ pegainfer_status_t pegainfer_dyt_add_norm(float* x, const void* y, const void* p
   return (pegainfer_status_t)hipGetLastError();
 }
 
-pegainfer_status_t pegainfer_dyt_step(const pegainfer_dyt_step_desc* q, pegainfer_stream_t stream) {
+static pegainfer_status_t dyt_step_launch(const pegainfer_dyt_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (!q) return bad;
   if (q->rows <= 0) return 0;
@@ -219,15 +226,36 @@ pegainfer_status_t pegainfer_dyt_step(const pegainfer_dyt_step_desc* q, pegainfe
   for (const void* v : stored)
     if (reinterpret_cast<uintptr_t>(v) & (q->dtype == kDtF32 ? 15u : 7u)) return bad;
   if (!host_aligned16(q->x) || !host_aligned16(q->y_pairs)) return bad;
+  RouterTail tail{};
+  if (router && (!q->next_w || q->y_pairs || !router_tail(router, q->rows, q->d, q->dtype, &tail))) return bad;
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         auto c = [](const void* p) { return static_cast<const A*>(p); };
         const DytStep<A> p{q->x, c(q->embed), q->token_ids, q->row_index, c(q->y), q->y_pairs, q->weight, q->top, c(q->post_alpha), c(q->post_w),
                            c(q->post_b), c(q->next_alpha), c(q->next_w), c(q->next_b), static_cast<A*>(q->out), q->d};
-        dyt_step_kernel<A><<<dim3(q->rows, ceil_div(q->d, 1024)), 256, 0, as_stream(stream)>>>(p);
+        if constexpr (sizeof(A) == 2) {
+          if (router) {
+            auto behind = [&](auto n) {
+              constexpr int N = decltype(n)::value;
+              const int blocks = tail_blocks(tail, q->d);
+              if (tail.E + tail.extra <= 32) dyt_step_kernel<A, N, RouteTail<N, 2>><<<blocks, N, 0, as_stream(stream)>>>(p, tail);
+              else dyt_step_kernel<A, N, RouteTail<N, 3>><<<blocks, N, 0, as_stream(stream)>>>(p, tail);
+            };
+            if (q->d <= 1024) behind(std::integral_constant<int, 256>());
+            else if (q->d <= 2048) behind(std::integral_constant<int, 512>());
+            else behind(std::integral_constant<int, 1024>());
+            return;
+          }
+        }
+        dyt_step_kernel<A><<<dim3(q->rows, ceil_div(q->d, 1024)), 256, 0, as_stream(stream)>>>(p, tail);
       }))
     return bad;
   return (pegainfer_status_t)hipGetLastError();
+}
+
+pegainfer_status_t pegainfer_dyt_step(const pegainfer_dyt_step_desc* q, pegainfer_stream_t stream) { return dyt_step_launch(q, nullptr, stream); }
+pegainfer_status_t pegainfer_dyt_step_routed(const pegainfer_dyt_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
+  return router ? dyt_step_launch(q, router, stream) : (pegainfer_status_t)hipErrorInvalidValue;
 }
 
 pegainfer_status_t pegainfer_gather_rows_f32(const float* x, const int32_t* rows_index, float* out, int32_t d,

@@ -618,7 +618,59 @@ struct ExpertForm {
   float limit, alpha, shared_limit;
   const uint16_t* w;
   int64_t m_stride, group_stride, up;      // the shared expert's: of a weight row, of a slice, from a gate row to its up row
+  // no table: the choices of the step's rows, one behind the other
+  const int32_t* chosen;
+  int32_t* tiles;                          // what the first product found for the second: per tile expert, pairs, their numbers
+  int pairs, top, experts, by_pair;
 };
+// The tile'th run of at most 16 pairs of one expert, experts ascending and an expert's pairs as they lie, found by one wave from the choices (up to 256 of up
+// to 64 experts): a load and some ballots where a launch would sort them into a table first (4.3 - 6.2 us).  By every wave for itself it
+// takes 1.4 us longer: their instructions share the SIMDs.  A lane stands for an expert: its mask of 64 pairs is the conjunction of the
+// number's bits over the lanes that hold them.  Returns the number of pairs, 0: no such tile.
+constexpr int kChosenMost = 4, kTileWords = kRowsMax + 2;      // times 64 pairs
+__device__ __forceinline__ int chosen_tile(const ExpertForm& ex, int tile, int lane, int* list, int* group) {
+  auto expert_of = [&](int c) { return c + lane < ex.pairs ? ex.chosen[c + lane] : -1; };
+  int e = 0, count = 0;
+#pragma unroll 1
+  for (int c = 0; c < ex.pairs; c += 64) {
+    e = expert_of(c);
+    unsigned long long m = __ballot((unsigned)e < (unsigned)ex.experts);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const unsigned long long one = __ballot((e >> b) & 1);
+      m &= (lane >> b) & 1 ? one : ~one;
+    }
+    count += __popcll(m);
+  }
+  const int tiles = (count + kRowsMax - 1) / kRowsMax;
+  int before;                              // tiles of the experts ahead
+  if (__ballot(tiles > 1)) {
+    before = tiles;
+#pragma unroll 1
+    for (int x = 1; x < 64; x <<= 1) {
+      const int o = __shfl_up(before, x, kWave);
+      if (lane >= x) before += o;
+    }
+    before -= tiles;
+  } else {
+    before = __popcll(__ballot(tiles > 0) & ((1ull << lane) - 1));
+  }
+  const unsigned long long mine = __ballot(tile >= before && tile < before + tiles);
+  if (!mine) return 0;
+  const int g = __ffsll(mine) - 1;
+  const int skip = (tile - __builtin_amdgcn_readlane(before, g)) * kRowsMax, left = __builtin_amdgcn_readlane(count, g) - skip;
+  *group = g;
+  int rank = -skip;
+#pragma unroll 1
+  for (int c = 0; c < ex.pairs; c += 64) {
+    if (ex.pairs > 64) e = expert_of(c);
+    const unsigned long long m = __ballot(e == g);
+    const int at = rank + __popcll(m & ((1ull << lane) - 1));
+    if (e == g && at >= 0 && at < kRowsMax) list[at] = c + lane;
+    rank += __popcll(m);
+  }
+  return min(left, kRowsMax);
+}
 __device__ __forceinline__ float glu_f(const ExpertForm& ex, bool shared, float g, float u) {
   if (ex.glu == PEGAINFER_GLU_SILU) return g * sigmoid_f(g) * u;
   const float limit = shared ? ex.shared_limit : ex.limit;
@@ -631,12 +683,43 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
   constexpr int CH = OB == 1 && sizeof(TX) == 2 ? 4 : 2;      // 64-wide pieces per register set
   constexpr int NP = RowPiece<TX>::kParts;
   __shared__ f32x4 red[4][OB][64];
-  int g, row0, nrows;
-  const bool shared = EX && (int)blockIdx.x >= ex.slots;
+  __shared__ int list[EX ? kRowsMax : 1], found[2];          // of a tile without a table: its pairs; its expert, their number
+  int g, row0, nrows, my_pair = 0;
+  const bool shared = EX && (int)blockIdx.x >= ex.slots, chosen = EX && !shared && ex.chosen;
   if (shared) {
     g = blockIdx.x - ex.slots;
     row0 = ex.pos0 + g * ex.rows;
     nrows = ex.rows;
+  } else if (chosen) {
+    if ((int)blockIdx.x >= d.max_tiles) return;               // (an odd number of columns may hold one more)
+    row0 = 0;
+    int32_t* t = ex.tiles ? ex.tiles + blockIdx.x * kTileWords : nullptr;
+    if (t && ex.by_pair) {                                    // found by the product before, asked for all at once
+      g = t[0];
+      nrows = t[1];
+      my_pair = t[2 + (threadIdx.x & 15)];
+      if (threadIdx.x < kRowsMax) list[threadIdx.x] = my_pair;
+      const int first = __builtin_amdgcn_readfirstlane(my_pair);      // of all lanes, before any is left out
+      if ((int)(threadIdx.x & 15) >= nrows) my_pair = first;
+    } else {
+      if (threadIdx.x < 64) {
+        int e = 0;
+        const int c = chosen_tile(ex, blockIdx.x, threadIdx.x, list, &e);
+        if (threadIdx.x == 0) { found[0] = e; found[1] = c; }
+        __builtin_amdgcn_wave_barrier();                      // the list is read by other lanes of this wave
+        if (t && blockIdx.y == 0 && threadIdx.x < kTileWords) {
+          if (threadIdx.x == 0) t[0] = e;
+          if (threadIdx.x == 1) t[1] = c;
+          if (threadIdx.x >= 2 && (int)threadIdx.x < 2 + c) t[threadIdx.x] = list[threadIdx.x - 2];
+        }
+      }
+      __syncthreads();
+      g = found[0];
+      nrows = found[1];
+      if (nrows > 0) my_pair = list[min((int)threadIdx.x & 15, nrows - 1)];
+    }
+    g = __builtin_amdgcn_readfirstlane(g);
+    nrows = __builtin_amdgcn_readfirstlane(nrows);
   } else if (d.tile_group) {
     if ((int)blockIdx.x >= *d.n_tiles) return;
     g = d.tile_group[blockIdx.x];
@@ -648,14 +731,17 @@ __global__ __launch_bounds__(256) void gemm_rows_mfma_kernel(pegainfer_gemm_desc
     nrows = min(kRowsMax, d.rows - row0);
   }
   if (nrows <= 0) return;                                     // an empty tile of a table has no last row to repeat
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l15 = lane & 15, gq = lane >> 4;
   const bool glu = EX && OB == 2 && ex.glu;                   // block 0 holds gate rows, block 1 their up rows
   const int per_blk = glu ? 16 : OB * 16, per_wg = 4 / wk * per_blk;      // outputs of a wave's share, of a workgroup
   const int blk = wave / wk, ks = wave - blk * wk;
   const int m0 = blockIdx.y * per_wg + blk * per_blk;
   // rows of position p: a shared slice's positions are the step's rows in order
-  auto x_row = [&](int p) { return d.x_row_index ? (shared ? p - row0 : d.x_row_index[p]) : p; };
-  auto y_row = [&](int p) { return d.y_row_index && !shared ? d.y_row_index[p] : p; };
+  auto x_row = [&](int p) {
+    if (EX && ex.chosen) return shared ? (ex.by_pair ? p : p - row0) : ex.by_pair ? my_pair : my_pair / ex.top;      // a lane's own row
+    return d.x_row_index ? (shared ? p - row0 : d.x_row_index[p]) : p;
+  };
+  auto y_row = [&](int p) { return chosen ? list[p] : d.y_row_index && !shared ? d.y_row_index[p] : p; };
   const TX* X = static_cast<const TX*>(d.x) + (shared ? 0 : (int64_t)g * d.x_group_stride);
   const uint16_t* W = shared ? ex.w + g * ex.group_stride : static_cast<const uint16_t*>(d.w) + (int64_t)g * d.w_group_stride;
   const int64_t wm = shared ? ex.m_stride : d.w_m_stride, up = shared ? ex.up : (int64_t)d.m * d.w_m_stride;
@@ -1099,23 +1185,43 @@ extern "C" pegainfer_status_t pegainfer_gemm_strided(const pegainfer_gemm_desc* 
   return (pegainfer_status_t)hipGetLastError();
 }
 
-extern "C" pegainfer_status_t pegainfer_expert_rows(const pegainfer_expert_rows_desc* q, pegainfer_stream_t stream) {
+static pegainfer_status_t expert_rows_impl(const pegainfer_expert_rows_desc* q, const pegainfer_chosen_desc* c, pegainfer_stream_t stream) {
   using namespace pk;
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (!q) return bad;
-  const pegainfer_gemm_desc& d = q->g;
+  pegainfer_gemm_desc d = q->g;
+  if (c) {
+    if (d.tile_group || d.x_row_index || d.y_row_index || !c->expert || !pegainfer_expert_rows_chosen_ok(c->rows, c->top, c->experts)) return bad;
+    // no more tiles than pairs, and no more than one per expert and 16 pairs
+    const int pairs = c->rows * c->top;
+    d.max_tiles = std::min(pairs, c->experts + pairs / kRowsMax);
+    d.tile_rows_cap = kRowsMax;
+    d.max_tile_rows = 0;
+  }
   const int slices = q->shared_w ? q->shared_groups : 0;
   if (d.m <= 0 || d.k <= 0 || d.max_tiles <= 0) return 0;
   const int rows = d.max_tile_rows > 0 ? d.max_tile_rows : d.tile_rows_cap;
-  if (!d.tile_group || !d.tile_row0 || !d.tile_rows || !d.n_tiles || d.plain || d.x_dtype != kDtBf16 || d.w_dtype != kDtBf16 ||
+  if ((!c && (!d.tile_group || !d.tile_row0 || !d.tile_rows || !d.n_tiles)) || d.plain || d.x_dtype != kDtBf16 || d.w_dtype != kDtBf16 ||
       (d.y_dtype != kDtBf16 && d.y_dtype != kDtF32) || rows < 1 || rows > kRowsMax || !chunks_ok(d) || d.epilogue == PEGAINFER_EPI_SIGMOID_GATE ||
       q->glu < PEGAINFER_GLU_NONE || q->glu > PEGAINFER_GLU_CLAMP || (q->glu && d.epilogue) || slices < 0 ||
       (slices && (q->shared_rows < 1 || q->shared_rows > kRowsMax || q->shared_pos0 < 0 || (q->shared_m_stride & 7) || (q->shared_group_stride & 7) ||
                   (q->shared_up & 7) || (reinterpret_cast<uintptr_t>(q->shared_w) & 15u))))
     return bad;
   const ExpertForm ex{q->glu, 0, q->shared_rows, q->shared_pos0, q->limit, q->alpha, q->shared_limit, static_cast<const uint16_t*>(q->shared_w),
-                      q->shared_m_stride, q->shared_group_stride, q->shared_up};
+                      q->shared_m_stride, q->shared_group_stride, q->shared_up, c ? c->expert : nullptr, c ? c->tiles : nullptr, c ? c->rows * c->top : 0, c ? c->top : 1,
+                      c ? c->experts : 0, c ? c->x_by_pair : 0};
   if (d.y_dtype == kDtF32) expert_rows_launch<float>(d, ex, slices, as_stream(stream));
   else expert_rows_launch<uint16_t>(d, ex, slices, as_stream(stream));
   return (pegainfer_status_t)hipGetLastError();
+}
+
+extern "C" pegainfer_status_t pegainfer_expert_rows(const pegainfer_expert_rows_desc* q, pegainfer_stream_t stream) {
+  return expert_rows_impl(q, nullptr, stream);
+}
+
+extern "C" int32_t pegainfer_expert_rows_chosen_ok(int32_t rows, int32_t top, int32_t experts) {
+  return rows > 0 && rows <= pk::kRowsMax && top > 0 && (int64_t)rows * top <= 64 * pk::kChosenMost && experts > 0 && experts <= 64;
+}
+extern "C" pegainfer_status_t pegainfer_expert_rows_chosen(const pegainfer_expert_rows_desc* q, const pegainfer_chosen_desc* chosen, pegainfer_stream_t stream) {
+  return chosen ? expert_rows_impl(q, chosen, stream) : (pegainfer_status_t)hipErrorInvalidValue;
 }

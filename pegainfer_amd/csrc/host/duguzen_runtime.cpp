@@ -125,7 +125,7 @@ struct Model {
   float *x = nullptr, *qc = nullptr, *olat = nullptr, *ypairs = nullptr, *route_w = nullptr, *route_logits = nullptr, *attn_ws = nullptr;
   size_t attn_ws_cap = 0;
   void *h = nullptr, *proj = nullptr, *attn = nullptr, *y = nullptr, *ffb = nullptr, *gu = nullptr, *act = nullptr;
-  int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
+  int32_t *route_e = nullptr, *pos_pair = nullptr, *chosen_tiles = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
   float *xw = nullptr, *logits32 = nullptr;
   void* hw = nullptr;
@@ -516,7 +516,7 @@ struct Model {
         dalloc_a(&proj, n * mx_proj, so) || dalloc_a(&attn, n * mx_attn, so) || dalloc_a(&y, n * D, so) ||
         dalloc_a(&ffb, n * std::max(1, mx_ff), so))
       return -1;
-    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, ptiles::kFewRows * (size_t)mx_experts, so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
+    if (mx_top > 0 && (dalloc(&ypairs, P * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, ptiles::kFewRows * (size_t)mx_experts, so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) || dalloc(&chosen_tiles, PEGAINFER_CHOSEN_WORDS, so) ||
                        dalloc(&pos_row, P, so) || dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu, n * mx_gu, so) ||
                        dalloc_a(&act, n * (size_t)(mx_gu / 2), so)))
       return -1;
@@ -705,7 +705,7 @@ struct Model {
       if (n) { q->next_alpha = n->alpha; q->next_w = n->w; q->next_b = n->b; }
     };
     // the stream takes a sublayer's output (routed: the experts' rows still to be summed) through its post-norm; the next pre-norm leaves h
-    auto join = [&](const Norm& post, const Norm* next, const MlpCfg* routed = nullptr) -> int {
+    auto join = [&](const Norm& post, const Norm* next, const MlpCfg* routed = nullptr, const pegainfer_router_tail_desc* router = nullptr) -> int {
       if (!steps) {
         DZ_K(pegainfer_dyt_add_norm(x, y, post.alpha, post.w, post.b, next ? next->alpha : nullptr, next ? next->w : nullptr, next ? next->b : nullptr,
                                     h, D, Ti, dtype, S()));
@@ -717,7 +717,8 @@ struct Model {
       else q.y = y;
       q.post_alpha = post.alpha; q.post_w = post.w; q.post_b = post.b;
       set_next(&q, next);
-      DZ_K(pegainfer_dyt_step(&q, S()));
+      if (router) DZ_K(pegainfer_dyt_step_routed(&q, router, S()));
+      else DZ_K(pegainfer_dyt_step(&q, S()));
       return 0;
     };
     if (steps) {
@@ -779,10 +780,17 @@ struct Model {
       }
       if (linear(w.o, attn, y, D, Ti, m.heads * m.vdim)) return -1;
       if (c.mlp.kind) {
-        if (join(w.n1b, &w.n2)) return -1;
+        // few rows: the launch that leaves a row's feed-forward input also routes it, and the experts' launches find their rows by the choices
+        const MlpCfg& f = c.mlp;
+        const bool chosen = f.kind == 2 && steps && Ti <= ptiles::kFewRows && D % 8 == 0 && f.ff % 8 == 0 &&
+                            pegainfer_router_tail_ok(f.experts, 0, D, dtype) && pegainfer_expert_rows_chosen_ok(Ti, f.top, f.experts);
+        pegainfer_router_tail_desc rt{};
+        rt.w = w.router; rt.correction = w.corr; rt.out_expert = route_e; rt.out_weight = route_w; rt.experts = f.experts; rt.n_groups = f.groups;
+        rt.keep_groups = f.keep; rt.top = f.top; rt.score_kind = PEGAINFER_SCORE_SIGMOID; rt.group_kind = PEGAINFER_GROUP_TOP2_SUM; rt.factor = 1.0f;
+        if (join(w.n1b, &w.n2, nullptr, chosen ? &rt : nullptr)) return -1;
         if (c.mlp.kind == 1) {
           if (linear(w.up, h, ffb, c.mlp.ff, Ti, D, PEGAINFER_EPI_RELU_SQ) || linear(w.down, ffb, y, D, Ti, c.mlp.ff)) return -1;
-        } else if (routed_ff(c, w, Ti, steps)) {
+        } else if (routed_ff(c, w, Ti, steps, chosen)) {
           return -1;
         }
         if (join(w.n2b, next_pre, c.mlp.kind == 2 ? &c.mlp : nullptr)) return -1;
@@ -835,15 +843,28 @@ struct Model {
     return 0;
   }
 
+  // one product of the experts of few rows: by the table, or by the choices
+  int experts(pegainfer_expert_rows_desc* x, bool chosen, const MlpCfg& f, int T, int by_pair) {
+    if (!chosen) {
+      DZ_K(pegainfer_expert_rows(x, S()));
+      return 0;
+    }
+    x->g.tile_group = x->g.x_row_index = x->g.y_row_index = nullptr;
+    const pegainfer_chosen_desc c{route_e, T, f.top, f.experts, by_pair, chosen_tiles};
+    DZ_K(pegainfer_expert_rows_chosen(x, &c, S()));
+    return 0;
+  }
   // sum_later: the pairs are left to the launch that joins them to the stream
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
+  // chosen: the rows are routed already, see there
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later, bool chosen) {
     const MlpCfg& f = c.mlp;
     const int P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     // few rows: tiles of the step's rows; otherwise 128-row tiles for the matrix-core form of bf16 weights, 64-row tiles
     const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0;
     const int per_tile = ptiles::expert_tile_rows(T, wide);
-    if (T <= ptiles::kFewRows && f.experts <= 1024) {
+    if (chosen) {
+    } else if (T <= ptiles::kFewRows && f.experts <= 1024) {
       // few rows (decoding): the few-rows GEMM streams the router with the whole chip into fp32 logits, then selection and sort in one launch
       // (4 rows of 2048, 32 experts: 10.0 + 4.2 -> 5.0 + 6.3 us)
       pegainfer_gemm_desc r{};
@@ -881,7 +902,7 @@ struct Model {
       x.g = d;
       x.g.y = act; x.g.m = f.ff; x.g.y_row_stride = f.ff;
       x.glu = PEGAINFER_GLU_SILU;
-      DZ_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, chosen, f, T, 0)) return -1;
     } else {
       DZ_K(pegainfer_gemm_strided(&d, S()));
       DZ_K(pegainfer_silu_mul_rows(gu, act, f.ff, P, dtype, S()));
@@ -896,7 +917,13 @@ struct Model {
     e.y_row_index = pos_pair;
     e.tile_rows_cap = per_tile;
     e.plain = plain_kernels;
-    DZ_K(pegainfer_gemm_strided(&e, S()));
+    if (chosen) {
+      pegainfer_expert_rows_desc x{};
+      x.g = e;
+      if (experts(&x, chosen, f, T, 1)) return -1;
+    } else {
+      DZ_K(pegainfer_gemm_strided(&e, S()));
+    }
     if (sum_later) return 0;
     DZ_K(pegainfer_route_combine(ypairs, route_w, y, D, f.top, T, dtype, S()));
     return 0;

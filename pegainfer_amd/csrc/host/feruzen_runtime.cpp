@@ -151,7 +151,7 @@ struct Model {
   void *q16 = nullptr, *attn16 = nullptr;   // stored-type queries and contiguous output of the matrix-core attention
   void *hb = nullptr, *xb = nullptr, *proj = nullptr, *mix = nullptr, *y = nullptr, *gu = nullptr, *act = nullptr, *ys = nullptr,
        *gu_e = nullptr, *act_e = nullptr;
-  int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
+  int32_t *route_e = nullptr, *pos_pair = nullptr, *chosen_tiles = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
   float *xw = nullptr, *logits32 = nullptr;
   void* hw = nullptr;
@@ -673,7 +673,7 @@ struct Model {
         dalloc_a(&ys, n * D, so) || dalloc_a(&q16, n * (size_t)std::max(1, mx_q), so) ||
         dalloc_a(&attn16, n * (size_t)std::max(1, mx_q), so))
       return -1;
-    if (mx_top > 0 && (dalloc(&ypairs, (P + ptiles::kFewRows * (size_t)mx_slices) * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)std::max(1, mx_experts), so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) ||
+    if (mx_top > 0 && (dalloc(&ypairs, (P + ptiles::kFewRows * (size_t)mx_slices) * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)std::max(1, mx_experts), so) || dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) || dalloc(&chosen_tiles, PEGAINFER_CHOSEN_WORDS, so) ||
                        dalloc(&pos_row, P, so) || dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu_e, n * mx_gu_e, so) ||
                        dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2) + ptiles::kFewRows * (size_t)mx_sff, so)))
       return -1;
@@ -1040,12 +1040,20 @@ struct Model {
         pegainfer_row_step_desc q = join_desc(x_in, w.norm1);
         if (c.mlp.kind) {
           q.x_out = x; q.xb_out = xb;
-          FZ_K(pegainfer_row_step(&q, S()));
+          // few rows: the launch that leaves a row's feed-forward input also routes it, and the experts' launches find their rows by the choices
+          const MlpCfg& f = c.mlp;
+          const bool chosen = f.kind == 2 && Ti <= ptiles::kFewRows && D % 8 == 0 && f.glu.ff % 8 == 0 && pegainfer_router_tail_ok(f.experts, 0, D, dtype) &&
+                              pegainfer_expert_rows_chosen_ok(Ti, f.top, f.experts);
+          pegainfer_router_tail_desc rt{};
+          rt.w = w.router; rt.out_expert = route_e; rt.out_weight = route_w; rt.experts = f.experts; rt.n_groups = rt.keep_groups = 1; rt.top = f.top;
+          rt.score_kind = PEGAINFER_SCORE_SOFTMAX; rt.factor = 1.0f;
+          if (chosen) FZ_K(pegainfer_row_step_routed(&q, &rt, S()));
+          else FZ_K(pegainfer_row_step(&q, S()));
           q = join_desc(x, w.norm2);
           if (c.mlp.kind == 1) {
             if (glu(w.gate_up, w.down, c.mlp.glu, xb, y, Ti)) return -1;
           } else {
-            if (routed_ff(c, w, Ti, true)) return -1;
+            if (routed_ff(c, w, Ti, true, chosen)) return -1;
             q.y = nullptr;
             q.y_pairs = ypairs; q.weight = route_w; q.top = c.mlp.top;
             if (c.mlp.has_shared && expert_slices) { q.add_pairs = ypairs + (size_t)Ti * c.mlp.top * D; q.n_add = expert_slices; }
@@ -1063,7 +1071,7 @@ struct Model {
         FZ_K(pegainfer_group_rms_add(x, y, dtype, w.norm1, groups, eps, x, xb, D, Ti, dtype, nullptr, 0, nullptr, 0, nullptr, nullptr, S()));
         if (c.mlp.kind == 1) {
           if (glu(w.gate_up, w.down, c.mlp.glu, xb, y, Ti)) return -1;
-        } else if (routed_ff(c, w, Ti, false)) {
+        } else if (routed_ff(c, w, Ti, false, false)) {
           return -1;
         }
         FZ_K(pegainfer_group_rms_add(x, y, dtype, w.norm2, groups, eps, x_next, nullptr, D, Ti, dtype, xs, xs_stride, w.dwa, n_mix, x,
@@ -1115,14 +1123,27 @@ struct Model {
   }
 
   int expert_slices = 0;   // of the last layer's shared expert: its rows lie behind the pairs
+  // one product of the experts of few rows: by the table, or by the choices
+  int experts(pegainfer_expert_rows_desc* x, bool chosen, const MlpCfg& f, int T, int by_pair) {
+    if (!chosen) {
+      FZ_K(pegainfer_expert_rows(x, S()));
+      return 0;
+    }
+    x->g.tile_group = x->g.x_row_index = x->g.y_row_index = nullptr;
+    const pegainfer_chosen_desc c{route_e, T, f.top, f.experts, by_pair, chosen_tiles};
+    FZ_K(pegainfer_expert_rows_chosen(x, &c, S()));
+    return 0;
+  }
   // sum_later: the pairs are left to the launch that joins them to the stream
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
+  // chosen: the rows are routed already, see there
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later, bool chosen) {
     const MlpCfg& f = c.mlp;
     const int ff = f.glu.ff, P = T * f.top;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
     const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0;
     const int per_tile = ptiles::expert_tile_rows(T, wide), slices = f.has_shared ? ptiles::shared_slices(T, wide, f.shared.ff, ff) : 0;
-    if (T > 8 || f.experts > 1024) {   // many rows (or more experts than the selection kernel's four rows hold in LDS): one
+    if (chosen) {
+    } else if (T > 8 || f.experts > 1024) {   // many rows (or more experts than the selection kernel's four rows hold in LDS): one
                                        // workgroup per row does logits and selection
       FZ_K(pegainfer_route_topk(xb, w.router, nullptr, route_e, route_w, D, f.experts, 1, 1, f.top, T, PEGAINFER_SCORE_SOFTMAX, dtype, S()));
       FZ_K(pegainfer_route_sort(route_e, P, f.top, f.experts, pos_pair, pos_row, t_group, t_row0, t_rows, n_tiles, max_tiles, per_tile, S()));
@@ -1172,11 +1193,11 @@ struct Model {
       x.glu = PEGAINFER_GLU_CLAMP; x.limit = f.glu.limit; x.alpha = kGluAlpha; x.shared_limit = f.shared.limit;
       x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
       x.shared_w = slices ? w.gate_up : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)ff * D; x.shared_up = (int64_t)f.shared.ff * D;
-      FZ_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, chosen, f, T, 0)) return -1;
       x.g = e;
       x.glu = PEGAINFER_GLU_NONE;
       x.shared_w = slices ? w.down : nullptr; x.shared_m_stride = f.shared.ff; x.shared_group_stride = ff;
-      FZ_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, chosen, f, T, 1)) return -1;
     } else {
       FZ_K(pegainfer_gemm_strided(&d, S()));
       FZ_K(pegainfer_clamp_glu_rows(gu_e, act_e, ff, P, f.glu.limit, kGluAlpha, dtype, S()));

@@ -156,7 +156,7 @@ struct Model {
         *gates32 = nullptr, *ypairs = nullptr, *route_w = nullptr, *route_logits = nullptr;
   void *hb = nullptr, *proj = nullptr, *mix = nullptr, *y = nullptr, *gate_d = nullptr, *gu = nullptr, *act = nullptr, *ys = nullptr,
        *gu_e = nullptr, *act_e = nullptr;
-  int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
+  int32_t *route_e = nullptr, *pos_pair = nullptr, *chosen_tiles = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
   float *xw = nullptr, *hw = nullptr, *logits32 = nullptr;
   Half* logits16 = nullptr;
@@ -738,7 +738,7 @@ struct Model {
         dalloc(&att_part, (size_t)kSplitGroups * kAttRows * 2 * (size_t)(mx_vdim + 2), so))
       return -1;
     if (mx_top > 0 && (dalloc(&ypairs, (P + ptiles::kFewRows * (size_t)mx_slices) * D, so) || dalloc(&route_w, P, so) || dalloc(&route_logits, n * (size_t)(mx_experts + 1), so) ||
-                       dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) || dalloc(&pos_row, P, so) ||
+                       dalloc(&route_e, P, so) || dalloc(&pos_pair, P, so) || dalloc(&chosen_tiles, PEGAINFER_CHOSEN_WORDS, so) || dalloc(&pos_row, P, so) ||
                        dalloc(&tiles, (size_t)3 * max_tiles + 1, so) || dalloc_a(&gu_e, n * (size_t)mx_gu_e, so) ||
                        dalloc_a(&act_e, n * (size_t)(mx_gu_e / 2) + ptiles::kFewRows * (size_t)mx_sff, so)))
       return -1;
@@ -912,7 +912,8 @@ struct Model {
     // convolution (hb = n + conv(n), the tail moved on)
     // routed (decode steps): the layer whose experts' rows are still to be summed, in place of yv
     auto open_sublayer = [&](const void* yv, const void* bias, float mlt, const float* add_rows, const void* add_vec, bool write_x,
-                             const void* gain, const void* conv_w, int64_t st_off, const MlpCfg* routed = nullptr) -> int {
+                             const void* gain, const void* conv_w, int64_t st_off, const MlpCfg* routed = nullptr,
+                             const pegainfer_router_tail_desc* router = nullptr) -> int {
       if (row_steps) {
         pegainfer_row_step_desc q{};
         q.x_in = x; q.x_out = write_x || !gain ? x : nullptr; q.y = yv; q.bias = yv ? bias : nullptr; q.mult = mlt;
@@ -928,7 +929,8 @@ struct Model {
         q.add_rows = add_rows; q.add_vec = add_vec; q.gain = gain; q.eps = eps;
         if (gain) { q.conv_w = conv_w; q.conv_state = state + st_off; q.conv_slot_stride = slot_stride; q.conv_slot = d_slot; q.conv_out = hb; }
         q.d = D; q.rows = Ti; q.dtype = dtype;
-        RX_K(pegainfer_row_step(&q, S()));
+        if (router) RX_K(pegainfer_row_step_routed(&q, router, S()));
+        else RX_K(pegainfer_row_step(&q, S()));
         return 0;
       }
       if (!gain) {
@@ -1029,8 +1031,16 @@ struct Model {
       const LayerW* nw = next_plain ? &weights[(size_t)runs[ri + 1].layer] : nullptr;
       const int64_t next_st = next_plain ? runs[ri + 1].st_canon1 : 0;
       if (c.mlp.kind) {
-        if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, w.norm2, w.canon2, r.st_canon2)) return -1;
-        if (routed_ff(c, w, Ti, row_steps)) return -1;
+        // few rows: the launch that leaves a row's feed-forward input also routes it, and the experts' launches find their rows by the choices
+        const MlpCfg& f = c.mlp;
+        const bool chosen = row_steps && Ti <= ptiles::kFewRows && D % 8 == 0 && f.ff % 8 == 0 && pegainfer_router_tail_ok(f.experts, 1, D, dtype) &&
+                            pegainfer_expert_rows_chosen_ok(Ti, f.top, f.experts);
+        pegainfer_router_tail_desc rt{};
+        rt.w = w.router; rt.out_expert = route_e; rt.out_weight = route_w; rt.experts = f.experts; rt.n_groups = f.groups; rt.keep_groups = f.keep;
+        rt.top = f.top; rt.score_kind = PEGAINFER_SCORE_SOFTMAX; rt.group_kind = PEGAINFER_GROUP_MAX; rt.renorm = 1; rt.factor = 1.0f;
+        if (f.has_shared) { rt.gate_logit = route_logits + f.experts; rt.gate_stride = f.experts + 1; }
+        if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, w.norm2, w.canon2, r.st_canon2, nullptr, chosen ? &rt : nullptr)) return -1;
+        if (routed_ff(c, w, Ti, row_steps, chosen)) return -1;
         if (open_sublayer(y, nullptr, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st, &c.mlp)) return -1;
       } else if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st)) {
         return -1;
@@ -1083,13 +1093,25 @@ struct Model {
   }
 
   int expert_slices = 0;   // of the last layer's shared expert: its rows lie behind the pairs
+  // one product of the experts of few rows: by the table, or by the choices
+  int experts(pegainfer_expert_rows_desc* x, bool chosen, const MlpCfg& f, int T, int by_pair) {
+    if (!chosen) {
+      RX_K(pegainfer_expert_rows(x, S()));
+      return 0;
+    }
+    x->g.tile_group = x->g.x_row_index = x->g.y_row_index = nullptr;
+    const pegainfer_chosen_desc c{route_e, T, f.top, f.experts, by_pair, chosen_tiles};
+    RX_K(pegainfer_expert_rows_chosen(x, &c, S()));
+    return 0;
+  }
   // hb -> y: router logits and the shared expert's gate logit by one GEMM into fp32, selection, experts, weighted sum (sum_later: the pairs
   // are left to the launch that joins them to the stream)
-  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later) {
+  // chosen: the rows are routed already, see there
+  int routed_ff(const LayerCfg& c, const LayerW& w, int T, bool sum_later, bool chosen) {
     const MlpCfg& f = c.mlp;
     const int ff = f.ff, P = T * f.top, E1 = f.experts + 1;
     int32_t *t_group = tiles, *t_row0 = tiles + max_tiles, *t_rows = tiles + 2 * max_tiles, *n_tiles = tiles + 3 * max_tiles;
-    if (linear_strided(w.router, hb, dtype, D, route_logits, PEGAINFER_DTYPE_F32, E1, T, D)) return -1;
+    if (!chosen && linear_strided(w.router, hb, dtype, D, route_logits, PEGAINFER_DTYPE_F32, E1, T, D)) return -1;
     const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && ff % 8 == 0;
     const int per_tile = ptiles::expert_tile_rows(T, wide), slices = f.has_shared ? ptiles::shared_slices(T, wide, f.shared_ff, ff) : 0;
     pegainfer_route_plan_desc r{};      // selection and sort: one launch for few rows
@@ -1099,7 +1121,7 @@ struct Model {
     r.sort_experts = f.experts; r.pos_pair = pos_pair; r.pos_row = pos_row;
     r.tile_group = t_group; r.tile_row0 = t_row0; r.tile_rows = t_rows; r.n_tiles = n_tiles;
     r.max_tiles = max_tiles; r.rows_per_tile = per_tile; r.dtype = dtype;
-    RX_K(pegainfer_route_plan(&r, S()));
+    if (!chosen) RX_K(pegainfer_route_plan(&r, S()));
     pegainfer_gemm_desc d{};
     d.x = hb; d.w = w.gate_up_e; d.y = gu_e;
     d.x_dtype = d.w_dtype = d.y_dtype = dtype;
@@ -1129,11 +1151,11 @@ struct Model {
       x.glu = PEGAINFER_GLU_SILU;
       x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
       x.shared_w = slices ? w.gate_up : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)ff * D; x.shared_up = (int64_t)f.shared_ff * D;
-      RX_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, chosen, f, T, 0)) return -1;
       x.g = e;
       x.glu = PEGAINFER_GLU_NONE;
       x.shared_w = slices ? w.down : nullptr; x.shared_m_stride = f.shared_ff; x.shared_group_stride = ff;
-      RX_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, chosen, f, T, 1)) return -1;
     } else {
       RX_K(pegainfer_gemm_strided(&d, S()));
       RX_K(pegainfer_silu_mul_rows(gu_e, act_e, ff, P, dtype, S()));

@@ -291,7 +291,7 @@ class Model : public StepModel {
     return dalloc(&x, n * D, so) || dalloc_a(&h, n * D, so) || dalloc_a(&proj, n * (size_t)mx_proj, so) || dalloc(&q32, n * (size_t)mx_q, so) ||
            dalloc(&o32, n * (size_t)mx_o, so) || dalloc(&z32, n * (size_t)mx_z, so) || dalloc_a(&mix, n * (size_t)mx_mix, so) ||
            dalloc_a(&y, n * D, so) || dalloc(&part, part_floats, so) || dalloc(&logits_r, n * (size_t)mx_route, so) ||
-           dalloc(&route_e, n * (size_t)mx_top, so) || dalloc(&route_w, n * (size_t)mx_top, so) || dalloc(&pos_pair, n * (size_t)mx_top, so) ||
+           dalloc(&route_e, n * (size_t)mx_top, so) || dalloc(&route_w, n * (size_t)mx_top, so) || dalloc(&pos_pair, n * (size_t)mx_top, so) || dalloc(&chosen_tiles, PEGAINFER_CHOSEN_WORDS, so) ||
            dalloc(&pos_row, n * (size_t)mx_top, so) || dalloc(&tiles, 3 * (size_t)max_tiles + 1, so) ||
            dalloc_a(&act_e, n * (size_t)mx_pair_ff + ptiles::kFewRows * (size_t)mx_shared, so) ||
            dalloc(&y_pairs, (n * (size_t)mx_top + ptiles::kFewRows * (size_t)mx_slices) * D, so) ||
@@ -331,11 +331,26 @@ class Model : public StepModel {
     d.eps = eps; d.gain_offset = kGainOffset; d.d = D; d.rows = s.T; d.dtype = dtype;
     return d;
   }
-  int join(const StepCtx& s, const void* post, const void* next) {
+  int join(const StepCtx& s, const void* post, const void* next, const pegainfer_router_tail_desc* router = nullptr) {
     pegainfer_join_rms_desc d = join_desc(s, post, next);
     d.y = y; d.y_row_stride = D;
-    PSTEP_K(pegainfer_join_rms(&d, S()));
+    if (router) PSTEP_K(pegainfer_join_rms_routed(&d, router, S()));
+    else PSTEP_K(pegainfer_join_rms(&d, S()));
     return 0;
+  }
+  // few rows: the launch that leaves a row's feed-forward input also routes it, and the experts' launches find their rows by the choices
+  bool routed_rows(const StepCtx& s, const MoeCfg& f) const {
+    const int all = f.experts + f.identity;
+    return !plain_kernels && s.T <= ptiles::kFewRows && D % 8 == 0 && f.ff % 8 == 0 && pegainfer_router_tail_ok(all, 1, D, dtype) &&
+           pegainfer_expert_rows_chosen_ok(s.T, f.top, f.experts);
+  }
+  pegainfer_router_tail_desc router_of(const MoeCfg& f, const LayerW& w) const {
+    const int all = f.experts + f.identity;
+    pegainfer_router_tail_desc r{};
+    r.w = w.router; r.correction = w.correction; r.out_expert = route_e; r.out_weight = route_w;
+    if (f.shared_ff) { r.gate_logit = logits_r + all; r.gate_stride = all + 1; }
+    r.experts = all; r.n_groups = 1; r.keep_groups = 1; r.top = f.top; r.score_kind = PEGAINFER_SCORE_SOFTMAX; r.renorm = 1; r.factor = f.scale;
+    return r;
   }
   int attention(const StepCtx& s, const LayerCfg& c, const LayerW& w) {
     const AttnCfg& a = c.left;
@@ -406,11 +421,23 @@ class Model : public StepModel {
                                     at(mix, (size_t)c.mix_right), c.mix_cols, m.heads, m.vdim, s.T, dtype, S()));
     return 0;
   }
+  // one product of the experts of few rows: by the table, or by the choices
+  int experts(pegainfer_expert_rows_desc* x, bool routed, const MoeCfg& f, int T, int by_pair) {
+    if (!routed) {
+      PSTEP_K(pegainfer_expert_rows(x, S()));
+      return 0;
+    }
+    x->g.tile_group = x->g.x_row_index = x->g.y_row_index = nullptr;
+    const pegainfer_chosen_desc c{route_e, T, f.top, f.experts, by_pair, chosen_tiles};
+    PSTEP_K(pegainfer_expert_rows_chosen(x, &c, S()));
+    return 0;
+  }
   // h -> the stream, and h of the next layer
   int feed_forward(const StepCtx& s, const LayerCfg& c, const LayerW& w, const void* next) {
     const MoeCfg& f = c.moe;
     const int T = s.T, all = f.experts + f.identity;
-    if (linear_strided(w.router, h, dtype, D, logits_r, PEGAINFER_DTYPE_F32, all + 1, T, D)) return -1;
+    const bool routed = routed_rows(s, f);
+    if (!routed && linear_strided(w.router, h, dtype, D, logits_r, PEGAINFER_DTYPE_F32, all + 1, T, D)) return -1;
     const bool wide = dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && D % 8 == 0 && f.ff % 8 == 0;
     const int per_tile = ptiles::expert_tile_rows(T, wide), slices = ptiles::shared_slices(T, wide, f.shared_ff, f.ff);
     pegainfer_route_plan_desc r{};
@@ -421,7 +448,7 @@ class Model : public StepModel {
     r.pos_pair = pos_pair; r.pos_row = pos_row;
     r.tile_group = tiles; r.tile_row0 = tiles + max_tiles; r.tile_rows = tiles + 2 * max_tiles; r.n_tiles = tiles + 3 * max_tiles;
     r.max_tiles = ptiles::expert_tiles(T, f.top, f.experts, per_tile); r.rows_per_tile = per_tile; r.dtype = dtype;
-    PSTEP_K(pegainfer_route_plan(&r, S()));
+    if (!routed) PSTEP_K(pegainfer_route_plan(&r, S()));
     pegainfer_gemm_desc g{};
     g.tile_group = r.tile_group; g.tile_row0 = r.tile_row0; g.tile_rows = r.tile_rows; g.n_tiles = r.n_tiles; g.max_tiles = r.max_tiles;
     g.tile_rows_cap = per_tile;
@@ -444,10 +471,10 @@ class Model : public StepModel {
       x.g = u;
       x.shared_groups = slices; x.shared_rows = T; x.shared_pos0 = P;
       x.shared_w = slices ? w.up_s : nullptr; x.shared_m_stride = D; x.shared_group_stride = (int64_t)f.ff * D;
-      PSTEP_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, routed, f, T, 0)) return -1;
       x.g = d;
       x.shared_w = slices ? w.down_s : nullptr; x.shared_m_stride = f.shared_ff; x.shared_group_stride = f.ff;
-      PSTEP_K(pegainfer_expert_rows(&x, S()));
+      if (experts(&x, routed, f, T, 1)) return -1;
     } else {
       PSTEP_K(pegainfer_gemm_strided(&u, S()));
       PSTEP_K(pegainfer_gemm_strided(&d, S()));
@@ -481,7 +508,9 @@ class Model : public StepModel {
       const LayerW& w = weights[i];
       const void* next = i + 1 < layers.size() ? weights[i + 1].norm1 : nullptr;
       if (linear(w.proj, h, proj, c.proj_rows, s.T, D) || attention(s, c, w) || memory(s, c, w) || linear(w.o, mix, y, D, s.T, c.mix_cols)) return -1;
-      if (join(s, w.norm1b, c.moe.ff ? w.norm2 : next)) return -1;
+      const bool routed = c.moe.ff && routed_rows(s, c.moe);
+      const pegainfer_router_tail_desc router = router_of(c.moe, w);
+      if (join(s, w.norm1b, c.moe.ff ? w.norm2 : next, routed ? &router : nullptr)) return -1;
       if (c.moe.ff && feed_forward(s, c, w, next)) return -1;
       if (tap_on) PSTEP_HIP(hipMemcpyAsync(tap_at((int)i), x, (size_t)s.T * D * 4, hipMemcpyDeviceToDevice, stream));
     }
@@ -505,7 +534,7 @@ class Model : public StepModel {
   float *x = nullptr, *q32 = nullptr, *o32 = nullptr, *z32 = nullptr, *part = nullptr, *logits_r = nullptr, *route_w = nullptr, *y_pairs = nullptr,
         *chunk_ws = nullptr;
   void *h = nullptr, *proj = nullptr, *mix = nullptr, *y = nullptr, *act_e = nullptr, *act_s = nullptr, *y_s = nullptr, *hw = nullptr;
-  int32_t *route_e = nullptr, *pos_pair = nullptr, *pos_row = nullptr, *tiles = nullptr;
+  int32_t *route_e = nullptr, *pos_pair = nullptr, *chosen_tiles = nullptr, *pos_row = nullptr, *tiles = nullptr;
 };
 
 }  // namespace psx

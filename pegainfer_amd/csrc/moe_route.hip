@@ -18,118 +18,9 @@
 //   route_plan_kernel  selection and sort in one launch for steps of up to 16 rows
 #include <algorithm>
 
-#include "common.h"
-#include "typed.h"
-#include "pegainfer_kernels_blocks.h"
+#include "route_core.h"
 
 namespace pk {
-
-// Selection on one wave from per-expert values in LDS (s: sigmoid scores, or logits when score is softmax; ch: s + correction):
-// softmax over ALL experts if asked, group scores, kept groups, then `top` wave-wide arg-max steps.  LDS accesses of one wave
-// complete in order, so no barrier is needed between its steps.
-template <typename A>
-__device__ __forceinline__ void route_select_wave(float* s, float* ch, float* gs, const A* __restrict__ corr,
-                                                  int32_t* __restrict__ out_e, float* __restrict__ out_w, int row, int lane, int E,
-                                                  int G, int keep, int top, int score, int group_kind = 0, int renorm = 0,
-                                                  float factor = 1.0f, int* pairs = nullptr) {
-  if (score == PEGAINFER_SCORE_SOFTMAX) {            // s = exp(z - max) / sum over ALL experts, then the choice scores
-    float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, s[e]);
-    mx = wave_max(mx);
-    float sum = 0.f;
-    for (int e = lane; e < E; e += 64) sum += expf(s[e] - mx);
-    sum = wave_sum(sum);
-    for (int e = lane; e < E; e += 64) {
-      const float sc = expf(s[e] - mx) / sum;
-      s[e] = sc;
-      ch[e] = corr ? sc + ld(corr + e) : sc;
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  if (G > 1) {
-    const int per = E / G;
-    for (int g = lane; g < G; g += 64) {             // a lane scores a group: its two largest choices
-      float b0 = -INFINITY, b1 = -INFINITY;
-      for (int i = 0; i < per; ++i) {
-        const float v = ch[g * per + i];
-        if (v > b0) { b1 = b0; b0 = v; } else if (v > b1) b1 = v;
-      }
-      gs[g] = per >= 2 && group_kind == PEGAINFER_GROUP_TOP2_SUM ? b0 + b1 : b0;
-    }
-    __builtin_amdgcn_wave_barrier();
-    for (int g = lane; g < G; g += 64) {             // kept = fewer than `keep` groups rank ahead (ties: the lower index)
-      const float mine = gs[g];
-      int ahead = 0;
-      for (int o = 0; o < G; ++o) {
-        const float v = gs[o];
-        ahead += (v > mine || (v == mine && o < g)) ? 1 : 0;
-      }
-      if (ahead >= keep)
-        for (int i = 0; i < per; ++i) ch[g * per + i] = -INFINITY;
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  // The chosen experts with their weights, in choice order, go to out_e / out_w and, for whoever continues in this workgroup, to pairs.
-  if (E <= 64) {
-    // a lane per expert: its place is the number of eligible experts ahead of it (ties: the lower index)
-    const float v = lane < E ? ch[lane] : -INFINITY, w = lane < E ? s[lane] : 0.f;
-    // false for no number, which is never chosen (the compiler's ballot of `v > -INFINITY` counts it: an ordered "not equal" made unordered)
-    const bool eligible = v >= -__FLT_MAX__;
-    int ahead = 0;
-    for (int o = 0; o < E; ++o) {
-      const float ov = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), o));
-      ahead += (ov > v || (ov == v && o < lane)) ? 1 : 0;
-    }
-    const int found = __popcll(__ballot(eligible));
-    float scale = 1.0f;
-    if (renorm || factor != 1.0f) {                  // the chosen weights divided by their sum (in choice order), times the factor
-      if (eligible) ch[ahead] = w;                   // every lane holds its own value by now
-      __builtin_amdgcn_wave_barrier();
-      float sum = 0.f;
-      for (int k = 0; k < min(top, found); ++k) sum += ch[k];
-      scale = factor * (renorm ? 1.0f / (sum + 1e-20f) : 1.0f);
-    }
-    if (eligible && ahead < top) {
-      out_e[(size_t)row * top + ahead] = lane;
-      out_w[(size_t)row * top + ahead] = w * scale;
-      if (pairs) pairs[row * top + ahead] = lane;
-    }
-    if (lane >= found && lane < top) {               // fewer eligible experts than choices
-      out_e[(size_t)row * top + lane] = 0;
-      out_w[(size_t)row * top + lane] = 0.f;
-      if (pairs) pairs[row * top + lane] = 0;
-    }
-    return;
-  }
-  for (int k = 0; k < top; ++k) {
-    float bv = -INFINITY;
-    int be = 0x7FFFFFFF;
-    for (int e = lane; e < E; e += 64) {             // ascending e per lane: the first maximum is the lowest index
-      const float v = ch[e];
-      if (v > bv) { bv = v; be = e; }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(bv, off, kWave);
-      const int oe = __shfl_xor(be, off, kWave);
-      if (ov > bv || (ov == bv && oe < be)) { bv = ov; be = oe; }
-    }
-    const bool found = bv != -INFINITY;
-    if (lane == 0) {
-      out_e[(size_t)row * top + k] = found ? be : 0;
-      out_w[(size_t)row * top + k] = found ? s[be] : 0.f;
-      if (pairs) pairs[row * top + k] = found ? be : 0;
-      if (found) ch[be] = -INFINITY;
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  if ((renorm || factor != 1.0f) && lane == 0) {
-    float sum = 0.f;
-    for (int k = 0; k < top; ++k) sum += out_w[(size_t)row * top + k];
-    const float inv = factor * (renorm ? 1.0f / (sum + 1e-20f) : 1.0f);
-    for (int k = 0; k < top; ++k) out_w[(size_t)row * top + k] *= inv;
-  }
-}
 
 // Few rows: sixteen waves of two experts each, four loads of the width ahead; many rows fill the chip with four waves of four experts.
 // 4 rows of 2048, 32 experts: 20.0 us with four waves -> 9.8 us.  The order of a logit's sum is the lanes' alone.
@@ -345,6 +236,10 @@ __global__ __launch_bounds__(256) void route_combine_kernel(const float* __restr
 
 extern "C" {
 using namespace pk;
+
+int32_t pegainfer_router_tail_ok(int32_t experts, int32_t has_gate, int32_t d, int32_t dtype) {
+  return router_tail_sizes(experts, has_gate, d, dtype);
+}
 
 // 64 or 128, or for few rows whatever no tile of the table may pass
 static bool tile_rows_ok(int n) { return n == 64 || n == 128 || (n >= 1 && n <= 16); }

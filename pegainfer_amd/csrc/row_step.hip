@@ -11,9 +11,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
-#include "typed.h"
-#include "pegainfer_kernels_blocks.h"
+#include "route_core.h"
 
 namespace pk {
 
@@ -57,7 +55,9 @@ struct StepConv {
       for (int q = 0; q < kStepTaps; ++q) ld4(p.conv_w + (int64_t)i * kStepTaps + 4 * q, w[k] + 4 * q);
     });
   }
-  __device__ __forceinline__ void finish(const RowStep<A>& p, int row, const float (&cur)[NV][4]) const {
+  // seen(i, o): the four values of a chunk as they are left
+  template <typename F>
+  __device__ __forceinline__ void finish(const RowStep<A>& p, int row, const float (&cur)[NV][4], F&& seen) const {
     each_chunk<N, NV>(p.d, [&](int k, int i) {
       float o[4];
 #pragma unroll
@@ -71,6 +71,7 @@ struct StepConv {
       for (int j = 1; j < kStepTaps - 1; ++j) st4(tail + (int64_t)(j - 1) * p.d + i, t[j][k]);
       st4(tail + (int64_t)(kStepTaps - 2) * p.d + i, cur[k]);
       st4(p.conv_out + (int64_t)row * p.d + i, o);
+      seen(i, o);
     });
   }
 };
@@ -121,9 +122,12 @@ __device__ __forceinline__ void step_output(const RowStep<A>& p, int row, float 
   }
 }
 
-template <typename A, int N, int NV, bool ROUTED>
-__global__ __launch_bounds__(N) void row_scalar_step_kernel(RowStep<A> p) {
+template <typename A, int N, int NV, bool ROUTED, typename T = NoTail>
+__global__ __launch_bounds__(N) void row_scalar_step_kernel(RowStep<A> p, RouterTail router) {
   __shared__ float red[N / 64];
+  __shared__ typename T::Shared sh;
+  if (T::helps(router, p.d)) return;
+  T tail;
   const int row = blockIdx.x;
   const int64_t src = (int64_t)(p.row_index ? p.row_index[row] : row) * p.d, base = (int64_t)row * p.d;
   StepConv<A, N, NV> conv;
@@ -135,6 +139,7 @@ __global__ __launch_bounds__(N) void row_scalar_step_kernel(RowStep<A> p) {
   each_chunk<N, NV>(p.d, [&](int k, int i) { ld4(p.x_in + src + i, r[k]); });
   if (p.conv_w) conv.request(p, row);
   step_output<A, N, NV, ROUTED>(p, row, y);
+  tail.request(router, p.d);
   float ss = 0.f;
   each_chunk<N, NV>(p.d, [&](int k, int i) {
     float a[4] = {}, v[4] = {};
@@ -156,11 +161,15 @@ __global__ __launch_bounds__(N) void row_scalar_step_kernel(RowStep<A> p) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) r[k][u] *= sc;
   if (p.n_out) each_chunk<N, NV>(p.d, [&](int k, int i) { st4(p.n_out + base + i, r[k]); });
-  if (p.conv_w) conv.finish(p, row, r);
+  if (p.conv_w) conv.finish(p, row, r, [&](int i, const float* o) { tail.put(sh, i, o); });
+  tail.finish(router, sh, p.d, row);
 }
 
-template <typename A, int N, int NV, bool ROUTED>
-__global__ __launch_bounds__(N) void row_group_step_kernel(RowStep<A> p) {
+template <typename A, int N, int NV, bool ROUTED, typename T = NoTail>
+__global__ __launch_bounds__(N) void row_group_step_kernel(RowStep<A> p, RouterTail router) {
+  __shared__ typename T::Shared sh;
+  if (T::helps(router, p.d)) return;
+  T tail;
   __shared__ float part[N * NV], inv[kStepGroups];
   const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, gs = p.d / p.groups;
   const int64_t base = (int64_t)row * p.d;
@@ -176,6 +185,7 @@ __global__ __launch_bounds__(N) void row_group_step_kernel(RowStep<A> p) {
   });
   if (p.conv_w) conv.request(p, row);
   step_output<A, N, NV, ROUTED>(p, row, y);
+  tail.request(router, p.d);
   each_chunk<N, NV>(p.d, [&](int k, int i) { part[i >> 2] = fmaf(y[k][0], y[k][0], fmaf(y[k][1], y[k][1], fmaf(y[k][2], y[k][2], y[k][3] * y[k][3]))); });
 #pragma unroll 4
   for (int j = 0; j < p.n_mix - 1; ++j) {
@@ -205,9 +215,11 @@ __global__ __launch_bounds__(N) void row_group_step_kernel(RowStep<A> p) {
     }
     if (p.x_out) st4(p.x_out + base + i, r[k]);
     if (p.xb_out) st4(p.xb_out + base + i, r[k]);
+    tail.put(sh, i, r[k]);
     if (p.n_mix > 0 && p.mix_out) st4(p.mix_out + base + i, m[k]);
   });
-  if (p.conv_w) conv.finish(p, row, m);
+  if (p.conv_w) conv.finish(p, row, m, [](int, const float*) {});
+  tail.finish(router, sh, p.d, row);
 }
 
 }  // namespace pk
@@ -220,7 +232,7 @@ int32_t pegainfer_row_step_ok(int32_t d, int32_t groups, int32_t taps, int64_t s
          taps == kStepTaps && state_off % 4 == 0 && slot_stride % 4 == 0;
 }
 
-pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream) {
+static pegainfer_status_t row_step_launch(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (!q) return bad;
   if (q->rows <= 0) return 0;
@@ -242,6 +254,8 @@ pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfe
   if (grouped ? q->row_index || q->add_rows || q->add_vec || q->n_out : q->stack || q->coef || q->mix_out || q->xb_out) return bad;
   if (q->bias && !q->y) return bad;
   if (q->row_index && q->x_out == q->x_in) return bad;
+  RouterTail tail{};
+  if (router && (routed || (grouped ? !q->xb_out : !q->conv_w) || !router_tail(router, q->rows, q->d, q->dtype, &tail))) return bad;
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         auto a = [](const void* p) { return static_cast<const A*>(p); };
@@ -251,7 +265,17 @@ pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfe
                            q->conv_slot_stride, q->conv_slot, static_cast<A*>(q->conv_out), q->d, q->rows};
         auto shape = [&](auto n, auto nv) {
           constexpr int N = decltype(n)::value, NV = decltype(nv)::value;
-          auto launch = [&](auto kern) { kern<<<q->rows, N, 0, as_stream(stream)>>>(p); };
+          auto launch = [&](auto kern) { kern<<<router ? tail_blocks(tail, q->d) : q->rows, N, 0, as_stream(stream)>>>(p, tail); };
+          if constexpr (sizeof(A) == 2 && NV == 1) {
+            if (router) {
+              auto behind = [&](auto* t) {
+                using T = std::remove_pointer_t<decltype(t)>;
+                grouped ? launch(row_group_step_kernel<A, N, NV, false, T>) : launch(row_scalar_step_kernel<A, N, NV, false, T>);
+              };
+              tail.E + tail.extra <= 32 ? behind(static_cast<RouteTail<N, 2>*>(nullptr)) : behind(static_cast<RouteTail<N, 3>*>(nullptr));
+              return;
+            }
+          }
           if (grouped) routed ? launch(row_group_step_kernel<A, N, NV, true>) : launch(row_group_step_kernel<A, N, NV, false>);
           else routed ? launch(row_scalar_step_kernel<A, N, NV, true>) : launch(row_scalar_step_kernel<A, N, NV, false>);
         };
@@ -263,6 +287,10 @@ pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfe
       }))
     return bad;
   return (pegainfer_status_t)hipGetLastError();
+}
+pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream) { return row_step_launch(q, nullptr, stream); }
+pegainfer_status_t pegainfer_row_step_routed(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
+  return router ? row_step_launch(q, router, stream) : (pegainfer_status_t)hipErrorInvalidValue;
 }
 
 }  // extern "C"

@@ -21,9 +21,7 @@
 //   softcap_rows_kernel     cap * tanh(x / cap) on fp32 rows
 #include <algorithm>
 
-#include "common.h"
-#include "typed.h"
-#include "pegainfer_kernels_blocks.h"
+#include "route_core.h"
 
 namespace pk {
 
@@ -589,10 +587,13 @@ struct JoinSource {
   const A* add; const float* add_gate; int64_t add_gate_stride;
   const float* add_pairs; int n_add;       // in place of `add`: that many fp32 rows per row, a step's rows apart
 };
-template <typename A, int N, int NPT, bool VEC, bool ROUTED>
+template <typename A, int N, int NPT, bool VEC, bool ROUTED, typename T = NoTail>
 __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, JoinSource<A> src, const A* __restrict__ post,
-                                                     const A* __restrict__ gain, float eps, float gain_offset, A* n_out, int d) {
+                                                     const A* __restrict__ gain, float eps, float gain_offset, A* n_out, int d, RouterTail router) {
   __shared__ float red[N / 64];
+  __shared__ typename T::Shared sh;
+  if (T::helps(router, d)) return;
+  T tail;
   constexpr int V = VEC ? 4 : 1, NV = NPT / V;
   const int row = blockIdx.x;
   float* xr = x + (int64_t)row * d;
@@ -615,6 +616,7 @@ __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, Join
       load(src.add + (int64_t)row * d + i, y[k]);
     }
   }
+  tail.request(router, d);
   if constexpr (ROUTED) {
     for (int j = 0; j < src.n_add; ++j)
 #pragma unroll
@@ -675,7 +677,9 @@ __global__ __launch_bounds__(N) void join_rms_kernel(float* __restrict__ x, Join
 #pragma unroll
     for (int u = 0; u < V; ++u) o[u] = xv[k][u] * sc * (gain_offset + gw[k][u]);
     if constexpr (VEC) st4(n_out + (int64_t)row * d + i, o); else st(n_out + (int64_t)row * d + i, o[0]);
+    tail.put(sh, i, o);
   }
+  tail.finish(router, sh, d, row);
 }
 
 // Gated linear units: out[row, i] = F(gate[row, i], up[row, i]); gate and up are column ranges of rows with one stride.  The rows' values are
@@ -909,7 +913,8 @@ pegainfer_status_t pegainfer_join_rms(const pegainfer_join_rms_desc* q, pegainfe
   return pegainfer_join_rms_pairs(q, nullptr, 0, stream);
 }
 
-pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream) {
+static pegainfer_status_t join_rms_launch(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, const pegainfer_router_tail_desc* router,
+                                          pegainfer_stream_t stream) {
   if (!q || n_add < 0 || (n_add > 0 && (!add_pairs || !q->y_pairs || q->add))) return PK_BAD;
   if (q->rows <= 0) return 0;
   const int d = q->d;
@@ -917,6 +922,9 @@ pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, co
   if (d <= 0 || d > 32768 || !q->x || !q->post || (!routed && !q->y) || (q->gain && !q->n_out) ||
       (routed && (!q->weight || q->top <= 0 || (q->same && !q->expert))))
     return PK_BAD;
+  RouterTail tail{};
+  if (router && (routed || !q->gain || !router_tail(router, q->rows, d, q->dtype, &tail))) return PK_BAD;
+  bool done = true;
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         const JoinSource<A> src{static_cast<const A*>(q->y), q->y_row_stride, q->y_pairs, q->weight, q->expert, q->top, q->same_from,
@@ -926,9 +934,23 @@ pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, co
                          host_aligned16(q->y_pairs) && host_aligned16(q->same) && host_aligned16(q->add) && host_aligned16(q->post) &&
                          host_aligned16(q->gain) && host_aligned16(q->n_out);
         auto launch = [&](auto kern, int threads) {
-          kern<<<q->rows, threads, 0, as_stream(stream)>>>(q->x, src, static_cast<const A*>(q->post), static_cast<const A*>(q->gain), q->eps,
-                                                          q->gain_offset, static_cast<A*>(q->n_out), d);
+          kern<<<router ? tail_blocks(tail, d) : q->rows, threads, 0, as_stream(stream)>>>(q->x, src, static_cast<const A*>(q->post), static_cast<const A*>(q->gain), q->eps,
+                                                          q->gain_offset, static_cast<A*>(q->n_out), d, tail);
         };
+        if constexpr (sizeof(A) == 2) {
+          if (router) {
+            if (!vec) { done = false; return; }
+            auto behind = [&](auto n) {
+              constexpr int N = decltype(n)::value;
+              if (tail.E + tail.extra <= 32) launch(join_rms_kernel<A, N, 4, true, false, RouteTail<N, 2>>, N);
+              else launch(join_rms_kernel<A, N, 4, true, false, RouteTail<N, 3>>, N);
+            };
+            if (d <= 1024) behind(std::integral_constant<int, 256>());
+            else if (d <= 2048) behind(std::integral_constant<int, 512>());
+            else behind(std::integral_constant<int, 1024>());
+            return;
+          }
+        }
         auto shape = [&](auto n, auto npt) {
           constexpr int N = decltype(n)::value, NPT = decltype(npt)::value;
           if (routed) {
@@ -948,9 +970,15 @@ pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, co
         else if (d <= 4096) shape(narrow, std::integral_constant<int, 16>());
         else if (d <= 8192) shape(wide, std::integral_constant<int, 8>());
         else shape(wide, std::integral_constant<int, 32>());
-      }))
+      }) || !done)
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();
+}
+pegainfer_status_t pegainfer_join_rms_pairs(const pegainfer_join_rms_desc* q, const float* add_pairs, int32_t n_add, pegainfer_stream_t stream) {
+  return join_rms_launch(q, add_pairs, n_add, nullptr, stream);
+}
+pegainfer_status_t pegainfer_join_rms_routed(const pegainfer_join_rms_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
+  return router ? join_rms_launch(q, nullptr, 0, router, stream) : PK_BAD;
 }
 
 pegainfer_status_t pegainfer_act_rows(const void* in, int64_t in_row_stride, void* out, int64_t out_row_stride, int32_t I, int32_t rows,

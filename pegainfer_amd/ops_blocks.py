@@ -90,14 +90,27 @@ def gemm_strided(desc):
     _chk(ffi.lib().pegainfer_gemm_strided(ctypes.addressof(desc), _stream()), "gemm_strided")
 
 
+CHOSEN_WORDS = 1536
+
+
+class ChosenDesc(ctypes.Structure):
+    _fields_ = [("expert", ctypes.c_void_p), ("rows", ctypes.c_int32), ("top", ctypes.c_int32), ("experts", ctypes.c_int32), ("x_by_pair", ctypes.c_int32),
+                ("tiles", ctypes.c_void_p)]
+
+
 class ExpertRowsDesc(ctypes.Structure):
     _fields_ = [("g", GemmDesc), ("glu", ctypes.c_int32), ("limit", ctypes.c_float), ("alpha", ctypes.c_float), ("shared_w", ctypes.c_void_p),
                 ("shared_groups", ctypes.c_int32), ("shared_rows", ctypes.c_int32), ("shared_pos0", ctypes.c_int32), ("shared_limit", ctypes.c_float),
                 ("shared_m_stride", ctypes.c_int64), ("shared_group_stride", ctypes.c_int64), ("shared_up", ctypes.c_int64)]
 
 
-def expert_rows(desc):
-    _chk(ffi.lib().pegainfer_expert_rows(ctypes.addressof(desc), _stream()), "expert_rows")
+def expert_rows(desc, choices=None, experts=0, by_pair=False, tiles=None):
+    """choices int32 [rows, top]: the rows of a group are found from them, without a table; tiles int32 [CHOSEN_WORDS]: by the first product for both"""
+    if choices is None:
+        _chk(ffi.lib().pegainfer_expert_rows(ctypes.addressof(desc), _stream()), "expert_rows")
+        return
+    c = ChosenDesc(expert=_p(choices), rows=choices.shape[0], top=choices.shape[1], experts=experts, x_by_pair=int(by_pair), tiles=_p(tiles))
+    _chk(ffi.lib().pegainfer_expert_rows_chosen(ctypes.addressof(desc), ctypes.addressof(c), _stream()), "expert_rows_chosen")
 
 
 def linear(x, w, out_dtype=None, epilogue=EPI_NONE, plain=False):
@@ -743,7 +756,7 @@ JoinRmsDesc = _struct("JoinRmsDesc", [("p", "x y"), ("l", "y_row_stride"), ("p",
 
 
 def join_rms(x_f32, post, gain=None, eps=1e-5, gain_offset=0.0, y=None, y_pairs=None, weight=None, expert=None, same_from=0, same=None, add=None,
-             add_gate_f32=None, add_pairs=None):
+             add_gate_f32=None, add_pairs=None, router=None):
     """x (in place) += rms_norm(y) * (gain_offset + post); -> rms_norm(x) * (gain_offset + gain) or None.  y: rows of the weights' type, or the
     weighted sum of routed experts from y_pairs fp32 [rows * top, d]; add_pairs fp32 [n_add, rows, d]: their sum in place of `add`"""
     rows, d = x_f32.shape
@@ -752,18 +765,28 @@ def join_rms(x_f32, post, gain=None, eps=1e-5, gain_offset=0.0, y=None, y_pairs=
                     top=0 if weight is None else weight.shape[1], same_from=same_from, same=_p(same), same_stride=0 if same is None else same.stride(0),
                     add=_p(add), add_gate=_p(add_gate_f32), add_gate_stride=0 if add_gate_f32 is None else add_gate_f32.stride(0), post=_p(post),
                     gain=_p(gain), eps=float(eps), gain_offset=float(gain_offset), n_out=_p(n), d=d, rows=rows, dtype=_dt(post))
+    if router is not None:
+        _chk(ffi.lib().pegainfer_join_rms_routed(ctypes.addressof(q), ctypes.addressof(router), _stream()), "join_rms_routed")
+        return n
     _chk(ffi.lib().pegainfer_join_rms_pairs(ctypes.addressof(q), _p(add_pairs), 0 if add_pairs is None else add_pairs.shape[0], _stream()), "join_rms")
     return n
+
+
+RouterTailDesc = _struct("RouterTailDesc", [("p", "w correction out_expert out_weight gate_logit"), ("l", "gate_stride"),
+                                            ("i", "experts n_groups keep_groups top score_kind group_kind renorm"), ("f", "factor")])
 
 
 DytStepDesc = _struct("DytStepDesc", [("p", "x embed token_ids row_index y y_pairs weight"), ("i", "top"),
                                       ("p", "post_alpha post_w post_b next_alpha next_w next_b out"), ("i", "d rows dtype")])
 
 
-def dyt_step(dtype, rows, d, **parts):
-    """tensors by their field (their pointer is taken), numbers as they are"""
+def dyt_step(dtype, rows, d, router=None, **parts):
+    """tensors by their field (their pointer is taken), numbers as they are; router: a RouterTailDesc behind the row"""
     q = DytStepDesc(d=d, rows=rows, dtype={torch.bfloat16: 0, torch.float32: 1}[dtype],
                     **{k: _p(v) if torch.is_tensor(v) else v for k, v in parts.items()})
+    if router is not None:
+        _chk(ffi.lib().pegainfer_dyt_step_routed(ctypes.addressof(q), ctypes.addressof(router), _stream()), "dyt_step_routed")
+        return
     _chk(ffi.lib().pegainfer_dyt_step(ctypes.addressof(q), _stream()), "dyt_step")
 
 
@@ -774,10 +797,13 @@ RowStepDesc = _struct("RowStepDesc", [("p", "x_in row_index x_out y bias"), ("f"
                                       ("i", "d rows dtype")])
 
 
-def row_step(dtype, rows, d, **parts):
-    """tensors by their field (their pointer is taken), numbers as they are"""
+def row_step(dtype, rows, d, router=None, **parts):
+    """tensors by their field (their pointer is taken), numbers as they are; router: a RouterTailDesc behind the row"""
     q = RowStepDesc(d=d, rows=rows, dtype={torch.bfloat16: 0, torch.float32: 1}[dtype],
                     **{k: _p(v) if torch.is_tensor(v) else v for k, v in parts.items()})
+    if router is not None:
+        _chk(ffi.lib().pegainfer_row_step_routed(ctypes.addressof(q), ctypes.addressof(router), _stream()), "row_step_routed")
+        return
     _chk(ffi.lib().pegainfer_row_step(ctypes.addressof(q), _stream()), "row_step")
 
 
