@@ -1,6 +1,7 @@
 """Python driver shared by the host runtimes that serve a model through ONE batched step function (libpegainfer_qwen3.so:
 include/pegainfer_duguzen.h, include/pegainfer_feruzen.h): prompts, portions of prompts and single decoded tokens of
 several requests run as one batch.  No CPU fallback."""
+import array
 import json
 import os
 
@@ -9,6 +10,17 @@ import numpy as np
 from . import ffi
 
 DTYPES = {"bfloat16": 0, "bf16": 0, "float32": 1, "f32": 1}
+
+
+def _words(code, dtype, values):
+    """a list of numbers as the C entry points read it, and its address.  A step of single tokens is a few hundred microseconds long and the device
+    waits for its lists: three of them take 4 us here, 8.5 us as numpy arrays (which take what is no integer)."""
+    try:
+        a = array.array(code, values)
+        return a, a.buffer_info()[0]
+    except (TypeError, OverflowError):
+        a = np.ascontiguousarray(values, dtype=dtype)
+        return a, a.ctypes.data
 
 
 class StepEngine:
@@ -36,6 +48,7 @@ class StepEngine:
         self.width = self._fn('width')(self.h)
         self.layer_runs = self._fn('num_layer_runs')(self.h)
         self.page_size = self._fn('page_size')(self.h)
+        self._step = self._fn('step')
 
     @classmethod
     def from_pretrained(cls, model_dir, max_tokens=4096, max_requests=8, dtype="bfloat16", device=0):
@@ -98,9 +111,9 @@ class StepEngine:
     def step(self, entries, want=None, logits=True, tokens=False):
         """entries: [(request id, [token ids])]; want: rows of the concatenated tokens whose logits are computed (None = the
         last row of every entry).  Returns float32 logits [wanted, vocab] (and / or the greedy tokens of those rows)."""
-        ids = np.ascontiguousarray([e[0] for e in entries], dtype=np.int32)
-        lens = np.ascontiguousarray([len(e[1]) for e in entries], dtype=np.int32)
-        toks = np.ascontiguousarray([t for e in entries for t in e[1]], dtype=np.uint32)
+        ids, ids_p = _words('i', np.int32, [e[0] for e in entries])
+        lens, lens_p = _words('i', np.int32, [len(e[1]) for e in entries])
+        toks, toks_p = _words('I', np.uint32, [t for e in entries for t in e[1]])
         if want is None:
             n_want, wp, rows = -1, None, len(entries)
         else:
@@ -108,9 +121,8 @@ class StepEngine:
             n_want, wp, rows = int(w.size), (w.ctypes.data if w.size else None), int(w.size)
         lg = np.empty((rows, self.vocab), dtype=np.float32) if logits and rows else None
         tk = np.zeros(rows, dtype=np.int32) if tokens and rows else None
-        self._chk(self._fn('step')(self.h, len(entries), ids.ctypes.data, lens.ctypes.data, toks.ctypes.data,
-                                                  n_want, wp, lg.ctypes.data if lg is not None else None,
-                                                  tk.ctypes.data if tk is not None else None), "step")
+        self._chk(self._step(self.h, len(entries), ids_p, lens_p, toks_p, n_want, wp, lg.ctypes.data if lg is not None else None,
+                             tk.ctypes.data if tk is not None else None), "step")
         if logits and tokens:
             return lg, tk
         return tk if tokens else lg
