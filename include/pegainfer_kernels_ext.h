@@ -150,6 +150,9 @@ void pegainfer_debug_attn_trace(uint64_t* buf);
  * 4 tickets, 5 lazy tickets; -1 = the dot2 GEMV at 1-2 columns or the tiled skinny kernel), out[2] = partial buffers * 100
  * + rows per row block. */
 pegainfer_status_t pegainfer_debug_gemm_route(int32_t M, int32_t T, int32_t K, int32_t silu_I, int32_t* out);
+/* what a plain GEMM of kind 256 hands to smaller tiles: out[0] = tiles of 256 rows before the cut (0: nothing is handed on), out[1] = 64 (128-row x
+ * 64-token tiles) or 96 (96 x 256 tiles) behind it */
+pegainfer_status_t pegainfer_debug_gemm_tail(int32_t M, int32_t T, int32_t K, int32_t* out);
 
 /* Debug / test hook: 1 = prefill GEMMs whose 256 x 256 tiling leaves >= 8 % of a CU round idle take the persistent stream-K
  * launch (kind 258 of pegainfer_debug_gemm_route), 0 = never, -1 = the environment decides (PEGAINFER_STREAMK=1; default off:

@@ -305,9 +305,10 @@ inline bool gemm_t_major(int M, int T, const SplitOut& so) {   // PEGAINFER_GEMM
   static const bool on = [] { const char* e = getenv("PEGAINFER_GEMM_T_MAJOR"); return !(e && e[0] == '0'); }();
   return on && so.silu_I == 0 && T > M;
 }
-inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, SplitOut so, hipStream_t s) {
+// m_head > 0: that many tiles of rows, what follows is another launch's (plain form)
+inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, SplitOut so, hipStream_t s, int m_head = 0) {
   const bool silu = so.silu_I > 0;
-  const int m_tiles = silu ? ceil_div(silu_cols_end(so) - so.silu_c0, 128) : ceil_div(M, G256_BM), t_tiles = ceil_div(T, G256_BT);
+  const int m_tiles = silu ? ceil_div(silu_cols_end(so) - so.silu_c0, 128) : m_head ? m_head : ceil_div(M, G256_BM), t_tiles = ceil_div(T, G256_BT);
   so.w_nt = t_tiles == 1 && weights_nt_on();
   so.t_major = gemm_t_major(M, T, so);
   {  // PEGAINFER_GEMM_CHUNK=0: the plain order (A/B); N: chunks of N tiles
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(512 + NF * 64) void mfma_gemm128x256_kernel(const H
   }
   const int mt = so.t_major ? tile % m_tiles : tile / t_tiles, tt = so.t_major ? tile / m_tiles : tile - mt * t_tiles;   // see mfma_gemm256_kernel
   constexpr int BMT = 32 * MT;            // W rows per tile
-  const int m0 = mt * BMT, t0 = tt * G256_BT;
+  const int m0 = so.m_first + mt * BMT, t0 = tt * G256_BT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wr = wave >> 2, wc = wave & 3;
   const int l15 = lane & 15, g = lane >> 4;
@@ -997,7 +998,7 @@ inline void gemm128x256_launch_nf(const Half* W, const Half* X, Half* Y, int M, 
 inline void gemm96x256_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, SplitOut so, hipStream_t s) {
   const int t_tiles = ceil_div(T, G256_BT);
   so.w_nt = t_tiles == 1 && weights_nt_on();
-  gemm128x256_launch_nf<false, 4, 3>(W, X, Y, M, T, K, so, nullptr, 1, 0, ceil_div(M, 96), t_tiles, s);
+  gemm128x256_launch_nf<false, 4, 3>(W, X, Y, M, T, K, so, nullptr, 1, 0, ceil_div(M - so.m_first, 96), t_tiles, s);
 }
 // SwiGLU form on 64-row tiles (MT = 2: 16 gate rows + their 16 up rows per wave row): the thin tail behind the 256 x 256 round
 inline void gemm64x256_silu_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, SplitOut so, hipStream_t s) {
@@ -1018,7 +1019,7 @@ inline void gemm128x256_launch(const Half* W, const Half* X, Half* Y, int M, int
     else gemm128x256_launch_nf<true, 0>(W, X, Y, M, T, K, so, nullptr, 1, 0, m_tiles, t_tiles, s);
     return;
   }
-  const int m_tiles = ceil_div(M, G128_BM);
+  const int m_tiles = ceil_div(M - so.m_first, G128_BM);
   if (feed) gemm128x256_launch_nf<false, 4>(W, X, Y, M, T, K, so, part, ksplit, nk_slice, m_tiles, t_tiles, s);
   else gemm128x256_launch_nf<false, 0>(W, X, Y, M, T, K, so, part, ksplit, nk_slice, m_tiles, t_tiles, s);
 }

@@ -162,7 +162,8 @@ __global__ __launch_bounds__(256) void mfma_gemm_kernel(const Half* __restrict__
 // with different tile shapes share one SwiGLU GEMM (the thin last round of the 256 x 256 tiling, glds_gemm_launch)
 // w_nt (set by the launchers, never by callers): the W tiles are requested with the non-temporal policy - each W byte is
 // read by ONE workgroup once (a single token tile), so it should not displace the x rows every workgroup re-reads from L2.
-struct SplitOut { Half* Y1; Half* Y2; Half* Y3; int M0; int M1; int M2; int silu_I; int silu_round; int silu_c0; int silu_c1; int w_nt; int xcd_slices; int t_major; int chunk; };
+struct SplitOut { Half* Y1; Half* Y2; Half* Y3; int M0; int M1; int M2; int silu_I; int silu_round; int silu_c0; int silu_c1; int w_nt; int xcd_slices; int t_major; int chunk; int m_first; };
+// m_first: rows of W before it are another launch's (plain un-split forms)
 // t_major (set by the gemm256.h launchers for plain GEMMs with T > M): row tile fastest inside an XCD's run of tiles
 // xcd_slices (set by the K-split launchers of gemm256.h): deal the (slice, tile) work items to the XCDs in slice-major runs.  NOT for
 // the 128-row kernel below: at 256 tokens (6-8 slices: 0.8-1.6 KB of every W row per XCD) it measured 1.1 % slower (r6_splitk_xcd_ab2.txt)
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(256) void mfma_gemm_glds_kernel(const Half* __restr
     tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
   }
   const int mt = tile / t_tiles, tt = tile - mt * t_tiles;
-  const int m0 = mt * BM, t0 = tt * TT;
+  const int m0 = so.m_first + mt * BM, t0 = tt * TT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = (wave >> 1) * 64, wt = (wave & 1) * (TT / 2);
   const int l15 = lane & 15, g = lane >> 4;
@@ -567,7 +568,7 @@ static void glds_gemm_launch_t(const Half* W, const Half* X, Half* Y, int M, int
     return true;
   }();
   (void)once;
-  const int m_tiles = so.silu_I > 0 ? ceil_div(silu_cols_end(so) - so.silu_c0, 64) : ceil_div(M, BM), t_tiles = ceil_div(T, TT);
+  const int m_tiles = so.silu_I > 0 ? ceil_div(silu_cols_end(so) - so.silu_c0, 64) : ceil_div(M - so.m_first, BM), t_tiles = ceil_div(T, TT);
   so.w_nt = t_tiles == 1 && weights_nt_on();
   mfma_gemm_glds_kernel<TT, ST><<<m_tiles * t_tiles, 256, kLds, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
 }
@@ -713,7 +714,22 @@ static void glds_splitk_launch(const Half* W, const Half* X, Half* Y, int M, int
   if (reduce) splitk_reduce(g_splitk_ws, Y, M, T, pl.ksplit, so, s);
 }
 
-// Which tiled kernel a prefill-shaped GEMM (T > 64, not K-split) takes - by shape only.  kind: 12 / 13 / 22 / 23 = the
+// The rows behind the full rounds of 256 x 256 tiles of a plain GEMM, when they would fill a small part of a further round: 64 = 128-row x 64-token
+// tiles, 96 = 96 x 256 tiles, 0 = they stay a round of their own.  The kernels keep the same per-element K order: the cut changes no bit.
+// A round of a few dozen tiles costs as much as a full one; measured with cold weights, whole / 64 / 96 (us): 17 408 x 2048 and 900
+// tokens (272 tiles) 100 / 79 / 84, 18 432 x 2560 and 1024 (288) 132 / 103 / 107, 6144 x 2560 and 3072 (288) 122 / 104 / 109, 8192 x 2048 and
+// 2100 (288) 100 / 83 / 84; 19 472 x 2048 and 1024 (308) 111 / 103 / 98, 8192 x 2048 and 2404 (320) 102 / 101 / 89.  The small tiles win while
+// a quarter more than one workgroup per compute unit takes them, the 96-row ones (one workgroup per compute unit) while one round does.
+static int plain_tail_kernel(int M, int T, int K, int m_head) {
+  const int rows = M - m_head * G256_BM;
+  if (rows <= 0) return 0;
+  if (4L * ceil_div(rows, BM) * ceil_div(T, 64) <= 5L * device_cus()) return 64;
+  const bool feeder = gemm128x256_on() && gemm128x256_feed_on() && gemm128x256_ok(M, T, K);
+  return feeder && (long)ceil_div(rows, 96) * ceil_div(T, G256_BT) <= device_cus() ? 96 : 0;
+}
+
+// Which tiled kernel a prefill-shaped GEMM (T > 64, not K-split) takes - by shape only.  kind: 259 = 256 with the rows behind its full rounds on a kernel
+// of smaller tiles (plain_tail_kernel; m_head = tiles of rows of the head), 12 / 13 / 22 / 23 = the
 // 128-row LDS-DMA kernel with 128- / 64-token tiles and that ring depth, 256 = the 256 x 256 8-phase kernel, 257 = its
 // SwiGLU form with the thin last round handed to the 128-row kernel (m_head = activation-column tiles of the head), 1280 /
 // 1281 = the 128 x 256 kernel, plain / SwiGLU.  One function for the launcher and for pegainfer_debug_gemm_route (the
@@ -756,6 +772,7 @@ static TiledRoute tiled_route(int M, int T, int K, const SplitOut& so, bool assu
       const int m_head = (int)((tiles256 / kCus) * kCus / tt256);   // whole activation-column tiles in full rounds
       if (tail_on && so.silu_I > 0 && so.silu_c1 == 0 && rem > 0 && rem * 2 <= kCus && m_head > 0 && m_head < mt256)
         return {257, m_head};
+      if (tail_on && so.silu_I == 0 && rem > 0 && m_head > 0 && m_head < mt256 && plain_tail_kernel(M, T, K, m_head)) return {259, m_head};
       return {256, 0};
     }
   }
@@ -816,6 +833,14 @@ static void glds_gemm_launch(const Half* W, const Half* X, Half* Y, int M, int T
       return;
     }
     if (r.kind == 258) { gemm256_streamk_launch(W, X, Y, M, T, K, so, g_splitk_ws, g_streamk_flags, device_cus(), s); return; }
+    if (r.kind == 259) {
+      gemm256_launch(W, X, Y, M, T, K, so, s, r.m_head);
+      SplitOut tail = so;
+      tail.m_first = r.m_head * G256_BM;
+      if (plain_tail_kernel(M, T, K, r.m_head) == 64) glds_gemm_launch_t<64, 3>(W, X, Y, M, T, K, tail, s);
+      else gemm96x256_launch(W, X, Y, M, T, K, tail, s);
+      return;
+    }
     if (r.kind == 256) { gemm256_launch(W, X, Y, M, T, K, so, s); return; }
     if (r.kind == 1283) { gemm96x256_launch(W, X, Y, M, T, K, so, s); return; }
     if (r.kind == 1280 || r.kind == 1281) { gemm128x256_launch(W, X, Y, M, T, K, so, nullptr, 1, 0, s); return; }
@@ -1150,7 +1175,17 @@ pegainfer_status_t pegainfer_debug_gemm_route(int32_t M, int32_t T, int32_t K, i
   }
   SplitOut so{nullptr, nullptr, nullptr, 0, 0, 0, silu_I > 0 ? silu_I : 0, 0, 0, 0};
   const TiledRoute r = tiled_route(silu_I > 0 ? 2 * silu_I : M, T, K, so, true);
-  out[0] = r.kind; out[2] = r.m_head;
+  out[0] = r.kind == 259 ? 256 : r.kind; out[2] = r.kind == 259 ? 0 : r.m_head;      // the hand-off behind it: pegainfer_debug_gemm_tail
+  return 0;
+}
+
+pegainfer_status_t pegainfer_debug_gemm_tail(int32_t M, int32_t T, int32_t K, int32_t* out) {
+  using namespace pk;
+  if (!out || M <= 0 || T <= 64 || K <= 0) return (pegainfer_status_t)hipErrorInvalidValue;
+  const bool whole = splitk_plan(M, T, K, true).nk_slice == 0;
+  const TiledRoute r = whole ? tiled_route(M, T, K, SplitOut{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0}, true) : TiledRoute{0, 0};
+  out[0] = r.kind == 259 ? r.m_head : 0;
+  out[1] = r.kind == 259 ? plain_tail_kernel(M, T, K, r.m_head) : 0;
   return 0;
 }
 

@@ -135,3 +135,23 @@ def test_flush_form_override_hook(route):
     finally:
         lib.pegainfer_debug_skinny_flush(-1)
     assert route(0, 16, 2560, I)[1] == 5
+
+
+def test_rows_behind_the_full_rounds_of_large_tiles():
+    """a plain GEMM whose last round of 256 x 256 tiles would be thin hands those rows to smaller tiles (256 compute units)"""
+    from pegainfer_amd import ffi
+    lib = ffi.lib()
+    out = (ctypes.c_int32 * 2)()
+
+    def tail(M, T, K):
+        assert lib.pegainfer_debug_gemm_tail(M, T, K, out) == 0
+        return tuple(out)
+    assert tail(16384, 1024, 2048) == (0, 0)           # one full round
+    assert tail(17408, 1024, 2048) == (64, 64)         # 272 tiles
+    assert tail(18432, 1024, 2560) == (64, 64)         # 288
+    assert tail(19472, 1024, 2048) == (64, 96)         # 308
+    assert tail(8192, 2404, 2048) == (25, 96)          # 320, ten tiles of tokens
+    assert tail(6144, 3072, 2560) == (21, 64)
+    assert tail(6144, 4096, 2560) == (0, 0)            # 384: half a round more
+    assert tail(6144, 10000, 2560) == (0, 0)
+    assert tail(2560, 1024, 9728) == (0, 0)            # K split over workgroups
