@@ -619,6 +619,12 @@ static SplitKPlan splitk_plan(int M, int T, int K, bool assume_ws = false) {
   if (!enabled || (!g_splitk_ws && !assume_ws) || T <= 16) return {0, 0, 0};
   const int m_tiles = ceil_div(M, BM), nk_all = K / BK;
   if (T > 64) {
+    // A short K is over before its slices' sums would be: whole tiles of 128 rows x 64 tokens take 3.5 us + 7.3 us per 1024 of K while every one has a
+    // compute unit (with more, a round of them), the split forms 9 - 13 us at 160 tokens, 13 - 20 at 300 and 19 - 26 from 1000 on, a third of it the
+    // sum.  Split / whole, cold weights (us): 1024 x 512 and 160 tokens 8.7 / 7.6; 1024 x 1024 and 1024 18.6 / 11.0, and 3000 25.5 / 15.0; 2048 x 2048
+    // and 600 22.5 / 18.4, and 1024 24.2 / 19.2, and 2404 26.3 / 26.6; but 2048 x 1024 and 160 tokens (48 tiles) 9.9 / 11.0, 2048 x 2560 and 300
+    // 20.3 / 23.0, 2560 x 2560 and 1024 28.0 / 32.7.
+    if (K <= 512 || (K <= 2048 && (long)m_tiles * ceil_div(T, 64) >= 80)) return {0, 0, 0};
     // long-K matrices at ~1.3-3 k tokens (down_proj: 50-128 tiles of 256 x 256): the 8-phase kernel over 2-5 K
     // slices, one workgroup per CU (tt == 256 marks this plan; PEGAINFER_SPLITK256=0 switches it off).  Same-box A/B of
     // TTFT: 2048 tokens 23.05 -> 21.4 ms; 1024 tokens (40 tiles, 6 slices: 63 MB of partials each way) 12.60 vs 12.56,
