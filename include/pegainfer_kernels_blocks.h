@@ -123,6 +123,15 @@ typedef struct {
   int32_t plain;             /* != 0: always the fp32-FMA tile kernel (exact products of the stored values) */
 } pegainfer_gemm_desc;
 pegainfer_status_t pegainfer_gemm_strided(const pegainfer_gemm_desc* d, pegainfer_stream_t stream);
+/* y[row, m] = act(gate row m . x) * (up row m . x) for up to four fp32 rows and fp32 weights in 16-byte chunks (no tile table, no epilogue): g.m pairs, the
+ * gate rows as g.w says, a pair's up row `up` elements behind its gate row.  Sums as in pegainfer_gemm_strided; act as in pegainfer_glu_rows. */
+typedef struct {
+  pegainfer_gemm_desc g;
+  int32_t act;
+  int64_t up;
+} pegainfer_glu_gemm_desc;
+int32_t pegainfer_glu_gemm_ok(const pegainfer_glu_gemm_desc* q);
+pegainfer_status_t pegainfer_glu_gemm(const pegainfer_glu_gemm_desc* q, pegainfer_stream_t stream);
 /* The grouped form for the experts of few rows (tile_rows_cap or max_tile_rows <= 16, bf16 x and w in 16-byte chunks; anything else is refused), with
  *   glu     y[p, m] = act(gate row m) (up row m) of a group that holds 2 m weight rows, gates first: SILU g sigmoid(g) u, CLAMP
  *           g sigmoid(alpha g) (u + 1) with g = min(g, limit), u = clamp(u, -limit, limit); sums and activation in fp32

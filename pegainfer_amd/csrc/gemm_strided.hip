@@ -305,17 +305,42 @@ static void mfma_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
   else mfma_tiles_launch<TX, TY, TG, 64>(d, s);
 }
 
-// ------------------------------------------------------------------ few-rows form (decode), fp32 weights or one fp32 row
-// At most R = 1, 2 or 4 rows per tile (a decode step's tokens, or the pairs one expert received): the weights are streamed once with
-// 16-byte loads, the rows wait in LDS as fp32 (2048 k values at a time), a wave owns one output at a time (lanes over k, butterfly sum), 32 outputs per
-// workgroup - or 8 (OUT) when 32 would leave most of the chip without a workgroup (a matrix of a few thousand outputs).  fp32
-// arithmetic for both storage types; the k order of an output is fixed by K alone, whatever OUT is.
-constexpr int kRowsFormChunk = 2048;   // k values of the rows that wait in LDS at a time (a multiple of the 512 a wave strides by): 32 KB at most
-
-template <typename TX, typename TW, typename TY, typename TG, int R, int OUT = 32>
-__global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_desc d) {
-  extern __shared__ __attribute__((aligned(16))) float xr[];    // [R][min(K, chunk)]
-  __shared__ int xrow[R], yrow[R];
+// ------------------------------------------------------------------ up to four fp32 rows against fp32 weights (decode)
+// No LDS and no barrier: a wave takes MB outputs (GLU: MB pairs of a gate row and its up row), lanes over k four values at a time, and fetches the rows
+// it multiplies with beside the weights, pieces of 512 k two ahead of the products.  An output's k order is fixed by K alone.
+// Bound by one memory latency behind the launch with few outputs and by the stream of weights with many.  With the rows in LDS first (a barrier
+// before any product, 32-byte strides between lanes), 1 / 2 / 4 rows: 1024 x 1024 3.3 / 4.1 / 5.3 -> 3.1 / 3.4 / 3.9 us, 1024 x 3072
+// 5.7 / 7.4 / 10.2 -> 4.9 / 6.1 / 7.0, 3072 x 1024 4.8 / 6.3 / 8.3 -> 4.5 / 4.9 / 6.3, 6144 x 1024 7.0 / 8.3 / 10.4 -> 7.3 / 8.0 / 9.7,
+// 32 768 x 1024 25.9 / 32.2 / 34.2 -> 25.3 / 25.8 / 28.2 (5.2 TB/s); on the fp32 matrix cores 2048 x 8192 takes 26.9 with two rows, 16.3 here.
+// Four outputs a wave where that leaves every SIMD a wave, then two, then one.
+// a lane's eight values of a piece of 512, in one or two loads that are whole lines over the wave
+template <typename TW>
+struct DirectPiece;
+template <>
+struct DirectPiece<float> {
+  f32x4 v[2];
+  static __device__ __forceinline__ int k_of(int p, int lane, int h) { return p * 512 + h * 256 + lane * 4; }
+  static __device__ __forceinline__ int last(int K, int) { return K - 4; }
+  __device__ __forceinline__ void load(const float* w, const int (&k)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) v[h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w + k[h]));
+  }
+  __device__ __forceinline__ f32x4 half(int h) const { return v[h]; }
+};
+template <>
+struct DirectPiece<uint16_t> {
+  u32x4 v;
+  static __device__ __forceinline__ int k_of(int p, int lane, int h) { return p * 512 + lane * 8 + h * 4; }
+  static __device__ __forceinline__ int last(int K, int h) { return K - 8 + 4 * h; }
+  __device__ __forceinline__ void load(const uint16_t* w, const int (&k)[2]) { v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w + k[0])); }
+  __device__ __forceinline__ f32x4 half(int h) const {
+    return h ? f32x4{bf_lo(v.z), bf_hi(v.z), bf_lo(v.w), bf_hi(v.w)} : f32x4{bf_lo(v.x), bf_hi(v.x), bf_lo(v.y), bf_hi(v.y)};
+  }
+};
+template <typename TW, typename TY, typename TG, int R, int MB, bool GLU>
+__global__ __launch_bounds__(256) void gemm_rows_direct_kernel(pegainfer_gemm_desc d, int act, int64_t up) {
+  constexpr int NW = GLU ? 2 : 1, CH = (MB == 4 ? 1 : 2) * (sizeof(TW) == 2 ? 2 : 1);      // pieces per register set
+  typedef DirectPiece<TW> Piece;
   int g, row0, nrows;
   if (d.tile_group) {
     if ((int)blockIdx.x >= *d.n_tiles) return;
@@ -327,226 +352,113 @@ __global__ __launch_bounds__(256) void gemm_strided_rows_kernel(pegainfer_gemm_d
     row0 = blockIdx.x * R;
     nrows = min(R, d.rows - row0);
   }
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (tid < R) {
-    const int p = row0 + tid;
-    xrow[tid] = tid < nrows ? (d.x_row_index ? d.x_row_index[p] : p) : -1;
-    yrow[tid] = tid < nrows ? (d.y_row_index ? d.y_row_index[p] : p) : -1;
-  }
-  __syncthreads();
-  const TX* X = static_cast<const TX*>(d.x) + (int64_t)g * d.x_group_stride;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, K = d.k;
+  const int m0 = (blockIdx.y * 4 + wave) * MB;
+  if (m0 >= d.m || nrows <= 0) return;
+  auto x_row = [&](int r) {                                   // absent rows repeat the last one; they are never stored
+    const int p = row0 + min(r, nrows - 1);
+    return d.x_row_index ? d.x_row_index[p] : p;
+  };
+  const float* X = static_cast<const float*>(d.x) + (int64_t)g * d.x_group_stride;
   const TW* W = static_cast<const TW*>(d.w) + (int64_t)g * d.w_group_stride;
-  const int K = d.k, xs = min(K, kRowsFormChunk);
-  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
-  // a wave owns a quarter of the workgroup's outputs and walks them four at a time: four independent weight streams in flight.
-  // The rows pass through LDS a chunk of k at a time (four long rows would leave room for one workgroup per compute unit); every
-  // output's sums stay in registers across the chunks, so its k order is what it would be in one piece.
-  constexpr int OW = OUT / 4, MB = OW >= 4 ? 4 : OW, NG = OW / MB;
-  const int m_base = blockIdx.y * OUT + wave * OW;
-  float acc[NG][MB][R];
+  const float* xp[R];
+  const TW* wp[MB];
 #pragma unroll
-  for (int n = 0; n < NG; ++n)
+  for (int r = 0; r < R; ++r) xp[r] = X + (int64_t)x_row(r) * d.x_row_stride;
 #pragma unroll
-    for (int q = 0; q < MB; ++q)
+  for (int q = 0; q < MB; ++q) wp[q] = W + (int64_t)min(m0 + q, d.m - 1) * d.w_m_stride;      // a clamped row is loaded and dropped at the store
+  struct Set { Piece w[CH][MB][NW]; f32x4 x[CH][R][2]; } A, B;
+  auto issue = [&](int p0, Set& s) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) acc[n][q][r] = 0.f;
-  for (int kc0 = 0; kc0 < K; kc0 += kRowsFormChunk) {
-    const int kl = min(kRowsFormChunk, K - kc0);      // a multiple of 8, as K is
-    if (kc0 > 0) __syncthreads();
-    for (int i = tid * 8; i < R * kl; i += 2048) {
-      const int r = i / kl, k = i - r * kl;
-      float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (xrow[r] >= 0) Vec8<TX>::load(X + (int64_t)xrow[r] * d.x_row_stride + kc0 + k, t);
-      *reinterpret_cast<f32x4*>(xr + r * xs + k) = f32x4{t[0], t[1], t[2], t[3]};
-      *reinterpret_cast<f32x4*>(xr + r * xs + k + 4) = f32x4{t[4], t[5], t[6], t[7]};
-    }
-    __syncthreads();
+    for (int c = 0; c < CH; ++c) {
+      int k[2];                                               // a lane past the end repeats the last values, unused
 #pragma unroll
-    for (int n = 0; n < NG; ++n) {
-      const int mw = m_base + n * MB;
-      if (mw >= d.m) continue;
-      for (int k = lane * 8; k < kl; k += 512) {      // (unrolling this loop by four was measured: 52 -> 66 us for a 65 536 x 2048 matrix)
-        float wv[MB][8];
+      for (int h = 0; h < 2; ++h) k[h] = min(Piece::k_of(p0 + c, lane, h), Piece::last(K, h));
 #pragma unroll
-        for (int q = 0; q < MB; ++q) {
-          const int m = min(mw + q, d.m - 1);          // a clamped row is loaded and dropped at the store
-          Vec8<TW>::load(W + (int64_t)m * d.w_m_stride + kc0 + k, wv[q]);
-        }
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const f32x4 xa = *reinterpret_cast<const f32x4*>(xr + r * xs + k), xb = *reinterpret_cast<const f32x4*>(xr + r * xs + k + 4);
+        for (int h = 0; h < 2; ++h) s.x[c][r][h] = *reinterpret_cast<const f32x4*>(xp[r] + k[h]);
 #pragma unroll
-          for (int q = 0; q < MB; ++q) {
-            float a = acc[n][q][r];
-            a = fmaf(wv[q][0], xa.x, a); a = fmaf(wv[q][1], xa.y, a); a = fmaf(wv[q][2], xa.z, a); a = fmaf(wv[q][3], xa.w, a);
-            a = fmaf(wv[q][4], xb.x, a); a = fmaf(wv[q][5], xb.y, a); a = fmaf(wv[q][6], xb.z, a); a = fmaf(wv[q][7], xb.w, a);
-            acc[n][q][r] = a;
-          }
-        }
-      }
-    }
-  }
+      for (int q = 0; q < MB; ++q)
 #pragma unroll
-  for (int n = 0; n < NG; ++n) {
-    const int mw = m_base + n * MB;
-    if (mw >= d.m) continue;
-#pragma unroll
-    for (int q = 0; q < MB; ++q)
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[n][q][r] = wave_sum(acc[n][q][r]);
-    if (lane == 0) {
-#pragma unroll
-      for (int q = 0; q < MB; ++q) {
-        const int m = mw + q;
-        if (m >= d.m) break;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if (yrow[r] < 0) continue;
-          float v = acc[n][q][r];
-          if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
-          else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
-          else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
-            v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)xrow[r] * d.gate_row_stride + g));
-          st(Y + (int64_t)yrow[r] * d.y_row_stride + m, v);
-        }
-      }
-    }
-  }
-}
-
-// The same sums for fp32 weights with a wave's weights on their way before anything else: the whole first chunk of k (and the next chunk piece by
-// piece as this one is used), one output per wave where that leaves every compute unit a workgroup at most.  The rows pass through LDS as above, so
-// an output's k order is the same.  Bound by one memory latency behind the launch: 1024 x 1024 and 1 / 2 / 4 rows 4.4 / 4.7 / 6.4 -> 3.3 / 4.1 / 5.3 us,
-// 1024 x 3072 7.7 / 8.6 / 12.2 -> 5.6 / 7.3 / 10.1; one row of any size: 6144 x 1024 7.8 -> 7.0, 65 536 x 2048 108 -> 91.  With more outputs than
-// that, two and four rows lose: the rows' way into LDS is paid per workgroup (6144 x 1024, 2 rows: 8.0 us above, 10.5 here).
-template <typename TX, typename TY, typename TG, int R, int OUT>
-__global__ __launch_bounds__(256) void gemm_rows_fma_kernel(pegainfer_gemm_desc d) {
-  extern __shared__ __attribute__((aligned(16))) float xr[];    // [R][min(K, chunk)]
-  __shared__ int xrow[R], yrow[R];
-  constexpr int MB = OUT / 4, PF = kRowsFormChunk / 512;
-  int g, row0, nrows;
-  if (d.tile_group) {
-    if ((int)blockIdx.x >= *d.n_tiles) return;
-    g = d.tile_group[blockIdx.x];
-    row0 = d.tile_row0[blockIdx.x];
-    nrows = min(R, d.tile_rows[blockIdx.x]);
-  } else {
-    g = blockIdx.z;
-    row0 = blockIdx.x * R;
-    nrows = min(R, d.rows - row0);
-  }
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, K = d.k, xs = min(K, kRowsFormChunk);
-  const int m0 = blockIdx.y * OUT + wave * MB;
-  const float* W = static_cast<const float*>(d.w) + (int64_t)g * d.w_group_stride;
-  f32x4 w[PF][MB][2];
-  auto request = [&](int p, int k0) {                         // piece p of the chunk that starts at k0
-    const int k = k0 + p * 512 + lane * 8;
-    if (k < K) {
-#pragma unroll
-      for (int q = 0; q < MB; ++q) {
-        const float* src = W + (int64_t)min(m0 + q, d.m - 1) * d.w_m_stride + k;      // a clamped row is loaded and dropped at the store
-        w[p][q][0] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src));
-        w[p][q][1] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + 4));
-      }
+        for (int n = 0; n < NW; ++n) s.w[c][q][n].load(wp[q] + (n ? up : 0), k);
     }
   };
-#pragma unroll
-  for (int p = 0; p < PF; ++p) request(p, 0);
-  if (tid < R) {
-    const int p = row0 + tid;
-    xrow[tid] = tid < nrows ? (d.x_row_index ? d.x_row_index[p] : p) : -1;
-    yrow[tid] = tid < nrows ? (d.y_row_index ? d.y_row_index[p] : p) : -1;
-  }
-  __syncthreads();
-  const TX* X = static_cast<const TX*>(d.x) + (int64_t)g * d.x_group_stride;
-  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
-  float acc[MB][R];
+  float acc[MB][NW][R];
 #pragma unroll
   for (int q = 0; q < MB; ++q)
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[q][r] = 0.f;
-  for (int kc0 = 0; kc0 < K; kc0 += kRowsFormChunk) {
-    const int kl = min(kRowsFormChunk, K - kc0);      // a multiple of 8, as K is
-    if (kc0 > 0) __syncthreads();
+    for (int n = 0; n < NW; ++n)
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      for (int k = tid * 8; k < kl; k += 2048) {
-        float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (xrow[r] >= 0) Vec8<TX>::load(X + (int64_t)xrow[r] * d.x_row_stride + kc0 + k, t);
-        *reinterpret_cast<f32x4*>(xr + r * xs + k) = f32x4{t[0], t[1], t[2], t[3]};
-        *reinterpret_cast<f32x4*>(xr + r * xs + k + 4) = f32x4{t[4], t[5], t[6], t[7]};
+      for (int r = 0; r < R; ++r) acc[q][n][r] = 0.f;
+  auto compute = [&](int p0, const Set& s) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (Piece::k_of(p0 + c, lane, h) >= K) continue;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int q = 0; q < MB; ++q)
+#pragma unroll
+            for (int n = 0; n < NW; ++n) {
+              const f32x4 w = s.w[c][q][n].half(h), x = s.x[c][r][h];
+              float a = acc[q][n][r];
+              a = fmaf(w.x, x.x, a); a = fmaf(w.y, x.y, a); a = fmaf(w.z, x.z, a); a = fmaf(w.w, x.w, a);
+              acc[q][n][r] = a;
+            }
       }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int k = p * 512 + lane * 8;
-      if (k < kl) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const f32x4 xa = *reinterpret_cast<const f32x4*>(xr + r * xs + k), xb = *reinterpret_cast<const f32x4*>(xr + r * xs + k + 4);
-#pragma unroll
-          for (int q = 0; q < MB; ++q) {
-            float a = acc[q][r];
-            a = fmaf(w[p][q][0].x, xa.x, a); a = fmaf(w[p][q][0].y, xa.y, a); a = fmaf(w[p][q][0].z, xa.z, a); a = fmaf(w[p][q][0].w, xa.w, a);
-            a = fmaf(w[p][q][1].x, xb.x, a); a = fmaf(w[p][q][1].y, xb.y, a); a = fmaf(w[p][q][1].z, xb.z, a); a = fmaf(w[p][q][1].w, xb.w, a);
-            acc[q][r] = a;
-          }
-        }
-      }
-      request(p, kc0 + kRowsFormChunk);
-    }
+  };
+  const int np = (K + 511) >> 9;
+  issue(0, A);
+  if (np > CH) issue(CH, B);
+  for (int p = 0; p < np; p += 2 * CH) {
+    compute(p, A);
+    if (p + 2 * CH < np) issue(p + 2 * CH, A);
+    if (p + CH >= np) break;
+    compute(p + CH, B);
+    if (p + 3 * CH < np) issue(p + 3 * CH, B);
   }
 #pragma unroll
   for (int q = 0; q < MB; ++q)
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[q][r] = wave_sum(acc[q][r]);
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[q][n][r] = wave_sum(acc[q][n][r]);
   if (lane != 0) return;
+  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
 #pragma unroll
-  for (int q = 0; q < MB; ++q) {
-    const int m = m0 + q;
-    if (m >= d.m) break;
+  for (int r = 0; r < R; ++r) {
+    if (r >= nrows) break;
+    const int yr = d.y_row_index ? d.y_row_index[row0 + r] : row0 + r;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (yrow[r] < 0) continue;
-      float v = acc[q][r];
-      if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+    for (int q = 0; q < MB; ++q) {
+      const int m = m0 + q;
+      if (m >= d.m) break;
+      float v = acc[q][0][r];
+      if constexpr (GLU) v = act_f(act, v) * acc[q][1][r];
+      else if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
       else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
       else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
-        v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)xrow[r] * d.gate_row_stride + g));
-      st(Y + (int64_t)yrow[r] * d.y_row_stride + m, v);
+        v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)x_row(r) * d.gate_row_stride + g));
+      st(Y + (int64_t)yr * d.y_row_stride + m, v);
     }
   }
 }
-
-// 32 outputs per workgroup unless that leaves most compute units without one
-static bool rows_form_fine(const pegainfer_gemm_desc& d, int R) {
+template <typename TW, typename TY, typename TG, int R, bool GLU>
+static void rows_direct_launch(const pegainfer_gemm_desc& d, int act, int64_t up, hipStream_t s) {
   const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  return (long)row_tiles * groups * ceil_div(d.m, 32) < device_cus();
-}
-template <typename TX, typename TW, typename TY, typename TG, int R>
-static void rows_form_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
-  auto kern = &gemm_strided_rows_kernel<TX, TW, TY, TG, R, 32>;
-  auto kern8 = &gemm_strided_rows_kernel<TX, TW, TY, TG, R, 8>;
-  // the tiles that a table's bound allows for and that are empty come last: an even grid width would send the others' workgroups, in
-  // their round robin over the XCDs, to some of the eight only
-  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  const bool fine = rows_form_fine(d, R);
-  dim3 grid(row_tiles, ceil_div(d.m, fine ? 8 : 32), groups);
-  const size_t lds = (size_t)R * std::min(d.k, kRowsFormChunk) * sizeof(float);
-  if (fine) kern8<<<grid, 256, lds, s>>>(d);
-  else kern<<<grid, 256, lds, s>>>(d);
-}
-
-// two and four rows: no more than a workgroup of four outputs per compute unit (1024 outputs on 256)
-static bool rows_fma_takes(const pegainfer_gemm_desc& d, int R) {
-  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  return (long)row_tiles * groups * ceil_div(d.m, 4) <= device_cus();
-}
-template <typename TX, typename TY, typename TG, int R>
-static void rows_fma_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
-  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  const size_t lds = (size_t)R * std::min(d.k, kRowsFormChunk) * sizeof(float);
-  gemm_rows_fma_kernel<TX, TY, TG, R, 4><<<dim3(row_tiles, ceil_div(d.m, 4), groups), 256, lds, s>>>(d);
+  const long outputs = (long)row_tiles * groups * d.m, waves = 4L * device_cus();
+  auto go = [&](auto mb) {
+    constexpr int MB = decltype(mb)::value;
+    gemm_rows_direct_kernel<TW, TY, TG, R, MB, GLU><<<dim3(row_tiles, ceil_div(d.m, 4 * MB), groups), 256, 0, s>>>(d, act, up);
+  };
+  if constexpr (!GLU) {
+    if (outputs >= 4 * waves) { go(std::integral_constant<int, 4>()); return; }
+  }
+  if (outputs >= 2 * waves) go(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 1>());
 }
 
 // ------------------------------------------------------------------ few-rows form on the matrix cores (bf16 weights, decode)
@@ -1121,19 +1033,13 @@ static bool gemm_strided_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
     }
     if constexpr (std::is_same<TW, float>::value) {
       if (tr <= kRowsMax) {
-        // Few rows by FMA, which needs no more than the rows' own products: 1024 x 1024 weights and 1 / 2 / 4 rows 4.1 / 4.4 / 6.1 us against
-        // 6.3 / 6.4 / 6.6 on the matrix cores, 8 rows 9.0 / 7.1, 16 rows 17.1 / 7.9; 6144 x 1024 and 8 rows 16.5 / 10.8, 32 768 x 1024 54.9 / 35.8.
-        // Beyond two chunks of k the rows' way through LDS costs more than that: 4096 x 12 288 and 3 rows 178 / 46 us.
-        const int R = tr <= 1 ? 1 : d.k > 2 * kRowsFormChunk ? 0 : tr <= 2 ? 2 : tr <= 4 ? 4 : 0;
+        // Few rows by FMA, which needs no more than the rows' own products, while a grid's columns hold the outputs.
+        const int R = d.m > 16 * 65535 ? 0 : tr <= 1 ? 1 : tr <= 2 ? 2 : tr <= 4 ? 4 : 0;
         auto run = [&](auto gate) {
           using TG = std::remove_pointer_t<decltype(gate)>;
-          if (R == 1 && d.m <= 4 * 65535) rows_fma_launch<TX, TY, TG, 1>(d, s);      // as many columns of workgroups as a grid takes
-          else if (R == 1) rows_form_launch<TX, TW, TY, TG, 1>(d, s);
-          else if (R == 2 && rows_fma_takes(d, 2)) rows_fma_launch<TX, TY, TG, 2>(d, s);
-          else if (R == 4 && rows_fma_takes(d, 4)) rows_fma_launch<TX, TY, TG, 4>(d, s);
-          // two rows of their own where workgroups are small (5.7 -> 4.4 us at 1024 x 1024); 65 536 x 2048 took 117 us so, 105 with four
-          else if (R == 2 && rows_form_fine(d, 2)) rows_form_launch<TX, TW, TY, TG, 2>(d, s);
-          else if (R) rows_form_launch<TX, TW, TY, TG, 4>(d, s);
+          if (R == 1) rows_direct_launch<TW, TY, TG, 1, false>(d, 0, 0, s);
+          else if (R == 2) rows_direct_launch<TW, TY, TG, 2, false>(d, 0, 0, s);
+          else if (R == 4) rows_direct_launch<TW, TY, TG, 4, false>(d, 0, 0, s);
           else rows_f32_launch<TY, TG>(d, s);
         };
         if (gate32) run((float*)nullptr);
@@ -1141,9 +1047,9 @@ static bool gemm_strided_launch(const pegainfer_gemm_desc& d, hipStream_t s) {
         return true;
       }
     } else if constexpr (std::is_same<TX, float>::value) {
-      if (tr <= 1) {
-        if (gate32) rows_form_launch<TX, TW, TY, float, 1>(d, s);
-        else rows_form_launch<TX, TW, TY, uint16_t, 1>(d, s);
+      if (tr <= 1 && d.m <= 16 * 65535) {
+        if (gate32) rows_direct_launch<TW, TY, float, 1, false>(d, 0, 0, s);
+        else rows_direct_launch<TW, TY, uint16_t, 1, false>(d, 0, 0, s);
         return true;
       }
     }
@@ -1224,4 +1130,23 @@ extern "C" int32_t pegainfer_expert_rows_chosen_ok(int32_t rows, int32_t top, in
 }
 extern "C" pegainfer_status_t pegainfer_expert_rows_chosen(const pegainfer_expert_rows_desc* q, const pegainfer_chosen_desc* chosen, pegainfer_stream_t stream) {
   return chosen ? expert_rows_impl(q, chosen, stream) : (pegainfer_status_t)hipErrorInvalidValue;
+}
+
+extern "C" int32_t pegainfer_glu_gemm_ok(const pegainfer_glu_gemm_desc* q) {
+  using namespace pk;
+  if (!q) return 0;
+  const pegainfer_gemm_desc& d = q->g;
+  return d.x_dtype == kDtF32 && d.w_dtype == kDtF32 && d.y_dtype == kDtF32 && !d.plain && !d.tile_group && !d.epilogue && d.m > 0 && d.m <= 4 * 65535 &&
+         d.k > 0 && d.rows > 0 && d.rows <= 4 && d.groups > 0 && d.groups <= 65535 && chunks_ok(d) && (q->up & 7) == 0 && q->act >= 0 &&
+         q->act <= PEGAINFER_ACT_GELU_ERF;
+}
+extern "C" pegainfer_status_t pegainfer_glu_gemm(const pegainfer_glu_gemm_desc* q, pegainfer_stream_t stream) {
+  using namespace pk;
+  if (!pegainfer_glu_gemm_ok(q)) return (pegainfer_status_t)hipErrorInvalidValue;
+  const int rows = q->g.rows;
+  hipStream_t s = as_stream(stream);
+  if (rows == 1) rows_direct_launch<float, float, float, 1, true>(q->g, q->act, q->up, s);
+  else if (rows == 2) rows_direct_launch<float, float, float, 2, true>(q->g, q->act, q->up, s);
+  else rows_direct_launch<float, float, float, 4, true>(q->g, q->act, q->up, s);
+  return (pegainfer_status_t)hipGetLastError();
 }

@@ -427,8 +427,17 @@ class Model : public StepModel {
       if (linear(w.o, mix, y, D, s.T, c.heads * c.vdim)) return -1;
       if (c.ff) {
         if (join(s, w.hc[0], &w.hc[1], w.norm[1], nullptr)) return -1;
-        if (linear(w.gu, h, gu, c.gu_rows, s.T, D)) return -1;
-        PSTEP_K(pegainfer_glu_rows(gu, at(gu, (size_t)c.o_up), c.gu_rows, act, c.ff, c.ff, s.T, PEGAINFER_ACT_GELU_TANH, dtype, S()));
+        pegainfer_glu_gemm_desc q{};      // few fp32 rows: both projections and the gated unit in one launch
+        q.g.x = h; q.g.w = w.gu; q.g.y = act; q.g.x_dtype = q.g.w_dtype = q.g.y_dtype = dtype;
+        q.g.m = c.ff; q.g.k = D; q.g.rows = s.T; q.g.groups = 1; q.g.x_row_stride = D; q.g.w_m_stride = D; q.g.w_k_stride = 1; q.g.y_row_stride = c.ff;
+        q.g.plain = plain_kernels;
+        q.act = PEGAINFER_ACT_GELU_TANH; q.up = (int64_t)c.o_up * D;
+        if (pegainfer_glu_gemm_ok(&q)) {
+          PSTEP_K(pegainfer_glu_gemm(&q, S()));
+        } else {
+          if (linear(w.gu, h, gu, c.gu_rows, s.T, D)) return -1;
+          PSTEP_K(pegainfer_glu_rows(gu, at(gu, (size_t)c.o_up), c.gu_rows, act, c.ff, c.ff, s.T, PEGAINFER_ACT_GELU_TANH, dtype, S()));
+        }
         if (linear(w.down, act, y, D, s.T, c.ff)) return -1;
       }
       if (join(s, w.hc[c.ff ? 1 : 0], nx ? &nx->hc[0] : nullptr, nx ? nx->norm[0] : nullptr, tap)) return -1;

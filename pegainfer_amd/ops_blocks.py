@@ -90,6 +90,14 @@ def gemm_strided(desc):
     _chk(ffi.lib().pegainfer_gemm_strided(ctypes.addressof(desc), _stream()), "gemm_strided")
 
 
+class GluGemmDesc(ctypes.Structure):
+    _fields_ = [("g", GemmDesc), ("act", ctypes.c_int32), ("up", ctypes.c_int64)]
+
+
+def glu_gemm(desc):
+    _chk(ffi.lib().pegainfer_glu_gemm(ctypes.addressof(desc), _stream()), "glu_gemm")
+
+
 CHOSEN_WORDS = 1536
 
 
