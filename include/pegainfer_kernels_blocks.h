@@ -961,7 +961,12 @@ typedef struct {
   int32_t shared_tail;       /* > 0: the last shared_tail values of a key are its value's (see pegainfer_qk_prep); one map, vdim == dim */
   int32_t tile_rows;         /* 32 or 64: the tiles hold ntok * nqh <= tile_rows rows and run on the kernel for prompts (bf16 cache, one map,
                                 unsplit, pegainfer_paged_attention_rows_ok); otherwise <= 16 */
+  /* not NULL: a decode step of a recurrence (kind GATED) that reads nothing the attention writes and writes nothing it reads, done in the
+   * attention's launch.  pegainfer_paged_attention_beside_ok says which forms take one (bf16, one map, the matrix-core form with tiles of up to
+   * 16 rows); pegainfer_paged_attention_opt refuses the others, pegainfer_paged_attention_gated all. */
+  const pegainfer_recurrent_step_desc* beside;
 } pegainfer_attn_options;
+int32_t pegainfer_paged_attention_beside_ok(const pegainfer_attn_options* opt, int32_t dtype);
 int32_t pegainfer_paged_attention_rows_ok(int32_t dim, int32_t vdim, int32_t shared_tail, int64_t page_stride, int64_t v_cache_off,
                                           int32_t page_size);
 pegainfer_status_t pegainfer_paged_attention_opt(const float* q, const void* cache, int64_t page_stride, int64_t k_cache_off,

@@ -352,7 +352,8 @@ class Model : public StepModel {
     r.experts = all; r.n_groups = 1; r.keep_groups = 1; r.top = f.top; r.score_kind = PEGAINFER_SCORE_SOFTMAX; r.renorm = 1; r.factor = f.scale;
     return r;
   }
-  int attention(const StepCtx& s, const LayerCfg& c, const LayerW& w) {
+  // `step`: the memory's step of the same layer, taken into the attention's launch where that can be (`taken` says so)
+  int attention(const StepCtx& s, const LayerCfg& c, const LayerW& w, const pegainfer_recurrent_step_desc* step, bool& taken) {
     const AttnCfg& a = c.left;
     pegainfer_qk_prep_desc p{};
     p.proj = proj; p.proj_dtype = dtype; p.proj_stride = c.proj_rows; p.q_off = a.o_q; p.k_off = a.o_k; p.v_off = a.o_k;
@@ -372,31 +373,44 @@ class Model : public StepModel {
     o.workspace = part;
     o.plain = plain_kernels ? 1 : 0;
     o.shared_tail = a.tail();
+    o.beside = step;
+    taken = step && pegainfer_paged_attention_beside_ok(&o, dtype);
+    if (!taken) o.beside = nullptr;
     PSTEP_K(pegainfer_paged_attention_opt(q32, cache, page_stride, c.k_off, c.v_off, kPageSize, s.pos, s.entry, s.page_indptr, s.pages, a.heads,
                                           a.kv, a.dim, a.dim, a.scale, c.left_scale, t.col(0), t.col(1), t.col(2), t.col(3), t.count, mix,
                                           c.mix_cols, &o, dtype, S()));
+    return 0;
+  }
+  // decoding: decays, scan, norm and gate in one launch
+  bool memory_step(const StepCtx& s, const LayerCfg& c, const LayerW& w, pegainfer_recurrent_step_desc& d) {
+    if (!s.single || plain_kernels) return false;
+    const MemCfg& m = c.right;
+    d = pegainfer_recurrent_step_desc{};
+    d.kind = PEGAINFER_STEP_GATED;
+    d.qkv = d.proj = proj; d.qkv_stride = d.proj_stride = c.proj_rows; d.q_off = m.o_q; d.k_off = m.o_k; d.v_off = m.o_v;
+    d.q_scale = (float)(1.0 / std::sqrt((double)m.dim));
+    d.w_up = w.a2; d.low_off = m.o_a; d.rank = m.rank; d.rank_stride = pad8(m.rank); d.z_bias = w.a2_bias; d.tau = m.tau;
+    d.state = state + m.st_off; d.slot_stride = state_layout.floats_per_slot(); d.entry_slot = s.slot;
+    d.norm_w = w.mem_norm; d.gate = at(proj, (size_t)m.o_g); d.gate_stride = c.proj_rows; d.factor = c.right_scale; d.eps = eps;
+    d.out = at(mix, (size_t)c.mix_right); d.out_stride = c.mix_cols;
+    d.heads = d.kv_heads = m.heads; d.dim = m.dim; d.vdim = m.vdim; d.n_entries = s.n; d.dtype = dtype;
+    return pegainfer_recurrent_step_ok(&d);
+  }
+  // both halves of a layer's mixer; neither reads what the other writes
+  int mixer(const StepCtx& s, const LayerCfg& c, const LayerW& w) {
+    pegainfer_recurrent_step_desc d{};
+    const bool step = memory_step(s, c, w, d);
+    bool taken = false;
+    if (attention(s, c, w, step ? &d : nullptr, taken)) return -1;
+    if (taken) return 0;
+    if (!step) return memory(s, c, w);
+    PSTEP_K(pegainfer_recurrent_step(&d, S()));
     return 0;
   }
   int memory(const StepCtx& s, const LayerCfg& c, const LayerW& w) {
     const MemCfg& m = c.right;
     const int rd = m.heads * m.dim;
     const int rp = pad8(m.rank);
-    // decoding: decays, scan, norm and gate in one launch
-    if (s.single && !plain_kernels) {
-      pegainfer_recurrent_step_desc d{};
-      d.kind = PEGAINFER_STEP_GATED;
-      d.qkv = d.proj = proj; d.qkv_stride = d.proj_stride = c.proj_rows; d.q_off = m.o_q; d.k_off = m.o_k; d.v_off = m.o_v;
-      d.q_scale = (float)(1.0 / std::sqrt((double)m.dim));
-      d.w_up = w.a2; d.low_off = m.o_a; d.rank = m.rank; d.rank_stride = rp; d.z_bias = w.a2_bias; d.tau = m.tau;
-      d.state = state + m.st_off; d.slot_stride = state_layout.floats_per_slot(); d.entry_slot = s.slot;
-      d.norm_w = w.mem_norm; d.gate = at(proj, (size_t)m.o_g); d.gate_stride = c.proj_rows; d.factor = c.right_scale; d.eps = eps;
-      d.out = at(mix, (size_t)c.mix_right); d.out_stride = c.mix_cols;
-      d.heads = d.kv_heads = m.heads; d.dim = m.dim; d.vdim = m.vdim; d.n_entries = s.n; d.dtype = dtype;
-      if (pegainfer_recurrent_step_ok(&d)) {
-        PSTEP_K(pegainfer_recurrent_step(&d, S()));
-        return 0;
-      }
-    }
     // few rows: the scan makes the decay inputs itself (its workgroups read W_a2 once per row)
     const bool fused = s.T <= kFusedRows && s.chunks.n_long == 0 && !plain_kernels && pegainfer_gated_linear_fused_ok(m.rank, rp, w.a2);
     if (!fused && linear_strided(w.a2, at(proj, (size_t)m.o_a), dtype, c.proj_rows, z32, PEGAINFER_DTYPE_F32, rd, s.T, rp)) return -1;
@@ -507,7 +521,7 @@ class Model : public StepModel {
       const LayerCfg& c = layers[i];
       const LayerW& w = weights[i];
       const void* next = i + 1 < layers.size() ? weights[i + 1].norm1 : nullptr;
-      if (linear(w.proj, h, proj, c.proj_rows, s.T, D) || attention(s, c, w) || memory(s, c, w) || linear(w.o, mix, y, D, s.T, c.mix_cols)) return -1;
+      if (linear(w.proj, h, proj, c.proj_rows, s.T, D) || mixer(s, c, w) || linear(w.o, mix, y, D, s.T, c.mix_cols)) return -1;
       const bool routed = c.moe.ff && routed_rows(s, c.moe);
       const pegainfer_router_tail_desc router = router_of(c.moe, w);
       if (join(s, w.norm1b, c.moe.ff ? w.norm2 : next, routed ? &router : nullptr)) return -1;

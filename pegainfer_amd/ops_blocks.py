@@ -572,7 +572,8 @@ def _struct(name, fields):
 
 AttnOptions = _struct("AttnOptions", [("i", "maps"), ("f", "lambda_"), ("i", "block"), ("p", "sink"), ("i", "head_norm"), ("f", "norm_eps softcap"),
                                       ("i", "window keep_first"), ("p", "dist_bias"), ("i", "n_dist"), ("p", "dist_slope gate"),
-                                      ("l", "gate_stride"), ("i", "gate_kind n_split"), ("p", "workspace"), ("i", "plain shared_tail tile_rows")])
+                                      ("l", "gate_stride"), ("i", "gate_kind n_split"), ("p", "workspace"), ("i", "plain shared_tail tile_rows"),
+                                      ("p", "beside")])
 LatentPrepDesc = _struct("LatentPrepDesc", [("p", "dkv"), ("l", "dkv_stride"), ("p", "c_norm_w ql"), ("l", "ql_stride"), ("p", "ql_norm_w ql_out"),
                                             ("i", "q_rank"), ("p", "q"), ("l", "q_stride"), ("p", "qc"), ("f", "eps"), ("p", "inv_freq"),
                                             ("i", "rot_dims rot_layout"), ("p", "positions token_req page_indptr page_ids cache"),
@@ -596,9 +597,11 @@ DecayAttentionDesc = _struct("DecayAttentionDesc", [("p", "proj"), ("l", "proj_s
 
 
 def paged_attention_opt(q, cache, page_stride, k_off, v_off, page_size, rg, page_indptr, page_ids, kv_heads, vdim, scale, window=0,
-                        dist_slope=None, softcap=0.0, n_split=1, plain=False, sink=None, gate=None, factor=1.0, shared_tail=0, tile_rows=16):
+                        dist_slope=None, softcap=0.0, n_split=1, plain=False, sink=None, gate=None, factor=1.0, shared_tail=0, tile_rows=16,
+                        beside=None):
     """q fp32 [rows, heads, dim]; dist_slope fp32 [heads]: slope * distance is taken off the scores; gate: a [rows, heads] view in the
-    cache's type, one output gate logit per head; shared_tail: values of a key that are read from its value"""
+    cache's type, one output gate logit per head; shared_tail: values of a key that are read from its value;
+    beside: a RecurrentStepDesc whose step is done in the same launch (None is returned where the launch does not take one)"""
     T, H, dim = q.shape
     out = torch.empty((T, H * vdim), dtype=cache.dtype, device=q.device)
     t = attention_tiles(rg.lens, H // kv_heads, q.device, tile_rows)
@@ -608,7 +611,9 @@ def paged_attention_opt(q, cache, page_stride, k_off, v_off, page_size, rg, page
                          device=q.device)
     o = AttnOptions(window=int(window), dist_slope=_p(dist_slope), softcap=float(softcap), n_split=int(n_split), workspace=_p(ws),
                     plain=int(bool(plain)), sink=_p(sink), gate=_p(gate), gate_stride=0 if gate is None else gate.stride(0),
-                    gate_kind=0 if gate is None else 2, shared_tail=int(shared_tail), tile_rows=tile_rows if tile_rows > 16 else 0)
+                    gate_kind=0 if gate is None else 2, shared_tail=int(shared_tail), tile_rows=tile_rows if tile_rows > 16 else 0, beside=None if beside is None else ctypes.addressof(beside))
+    if beside is not None and not ffi.lib().pegainfer_paged_attention_beside_ok(ctypes.addressof(o), _dt(cache)):
+        return None
     _chk(ffi.lib().pegainfer_paged_attention_opt(_p(q), _p(cache), page_stride, k_off, v_off, page_size, _p(rg.positions), _p(rg.row_entry),
                                                  _p(page_indptr), _p(page_ids), H, kv_heads, dim, vdim, float(scale), float(factor), _p(t[0]),
                                                  _p(t[1]), _p(t[2]), _p(t[3]), t[0].numel(), _p(out), out.stride(0), ctypes.addressof(o), _dt(cache),
@@ -890,9 +895,10 @@ STEP_KINDS = {"gated": 0, "delta": 1, "delta_channel": 2}
 
 def recurrent_step(kind, qkv, offs, proj, state, slots, norm_w, heads, kv_heads, dim, vdim, q_scale=1.0, z=None, w_up=None, low_off=0, rank=0,
                    z_bias=None, tau=1.0, A_log=None, a_off=0, b_off=0, gate=None, w_gate=None, gate_low_off=0, gate_rank=0, gate_kind="silu",
-                   factor=1.0, eps=1e-6):
+                   factor=1.0, eps=1e-6, launch=True):
     """one row per entry; qkv rows (of proj's type for "gated", else fp32) with q, k, v at offs -> the normed and gated read-out [n, heads * vdim]
-    in proj's type, or None where the launch does not take these sizes"""
+    in proj's type, or None where the launch does not take these sizes; not launch: (the
+    step's description, where it will leave the read-out)"""
     n = proj.shape[0]
     out = torch.empty((n, heads * vdim), dtype=proj.dtype, device=proj.device)
     q = RecurrentStepDesc(kind=STEP_KINDS[kind], qkv=_p(qkv), qkv_stride=qkv.stride(0), q_off=offs[0], k_off=offs[1], v_off=offs[2],
@@ -905,5 +911,7 @@ def recurrent_step(kind, qkv, offs, proj, state, slots, norm_w, heads, kv_heads,
                           heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, n_entries=n, dtype=_dt(proj))
     if not ffi.lib().pegainfer_recurrent_step_ok(ctypes.addressof(q)):
         return None
+    if not launch:
+        return q, out
     _chk(ffi.lib().pegainfer_recurrent_step(ctypes.addressof(q), _stream()), "recurrent_step")
     return out
