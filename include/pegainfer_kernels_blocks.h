@@ -211,6 +211,11 @@ typedef struct {
   int32_t heads, nope, rot, rank, n_tokens, dtype;
 } pegainfer_latent_prep_desc;
 pegainfer_status_t pegainfer_latent_prep_form(const pegainfer_latent_prep_desc* d, pegainfer_stream_t stream);
+/* The prep and, in the same launch, the product that leaves qc[t, h, :rank] (a decode step; _ok says whether these rows and sizes are taken:
+ * up to 16 bf16 or 4 fp32 rows, without a row index, tile table or epilogue).  The two may read the same rows; neither may write what the other
+ * reads or writes. */
+int32_t pegainfer_latent_prep_absorb_ok(const pegainfer_latent_prep_desc* d, const pegainfer_gemm_desc* g);
+pegainfer_status_t pegainfer_latent_prep_absorb(const pegainfer_latent_prep_desc* d, const pegainfer_gemm_desc* g, pegainfer_stream_t stream);
 /* Causal softmax attention of every (token, head) row over its request's cache entries 0 .. position:
  *   score_j = (qc[t, h, :] . entry_j) * scale;  o_lat[t, h, :] = sum_j softmax(score)_j * entry_j[:rank]
  * qc fp32 [T, heads, rank + rot], o_lat fp32 [T, heads, rank]; scores, running maxima / sums and accumulators in fp32.

@@ -21,9 +21,7 @@
 // function of the row's key count alone; with dealt splits it also depends on the step's shape (rounding only).
 #include <type_traits>
 
-#include "common.h"
-#include "typed.h"
-#include "pegainfer_kernels_blocks.h"
+#include "gemm_rows.h"
 
 namespace pk {
 
@@ -63,60 +61,94 @@ struct LatentPrep {
   const A* q; int64_t q_stride; float* qc;                                // rotated parts of the heads' queries -> qc (fp32)
 };
 
+// the sizes and the cache of a prep launch
+struct LatentPlace {
+  float eps;
+  const float* inv_freq;
+  int rot_dims, pairs;
+  const int32_t *positions, *token_req, *page_indptr, *page_ids;
+  int64_t page_stride, layer_off;
+  int page_size, H, dn, dr, r;
+};
+
+// of 256 threads: token row t, workgroup y of ny of the row
 template <typename A>
-__global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrep<A> a, float eps, const float* __restrict__ inv_freq, int rot_dims,
-                                                          int pairs, const int32_t* __restrict__ positions,
-                                                          const int32_t* __restrict__ token_req,
-                                                          const int32_t* __restrict__ page_indptr,
-                                                          const int32_t* __restrict__ page_ids, A* __restrict__ cache,
-                                                          int64_t page_stride, int64_t layer_off, int page_size, int H, int dn,
-                                                          int dr, int r) {
+__device__ __forceinline__ void latent_prep_block(int t, int y, int ny, const LatentPrep<A>& a, const LatentPlace& p, A* __restrict__ cache) {
   __shared__ float red[4];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  const int pos = positions[t];
-  const int E = r + dr;
+  const int tid = threadIdx.x;
+  const int pos = p.positions[t];
+  const int r = p.r, E = r + p.dr;
   const A* dkv = a.dkv ? a.dkv + (int64_t)t * a.dkv_stride : nullptr;
   A* entry = nullptr;
   if (dkv) {
-    const int req = token_req[t];
-    entry = cache + (int64_t)page_ids[page_indptr[req] + pos / page_size] * page_stride + layer_off + (int64_t)(pos % page_size) * E;
+    const int req = p.token_req[t];
+    entry = cache + (int64_t)p.page_ids[p.page_indptr[req] + pos / p.page_size] * p.page_stride + p.layer_off + (int64_t)(pos % p.page_size) * E;
   }
   // with several workgroups per row (few rows) the first norms the key latent, the last the query latent
-  if (dkv && blockIdx.y == 0) {
+  if (dkv && y == 0) {
     float ss = 0.f;
     for (int i = tid; i < r; i += 256) { const float v = ld(dkv + i); ss += v * v; }
     ss = block_sum<4>(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)r + eps);
+    const float inv = 1.0f / sqrtf(ss / (float)r + p.eps);
     for (int i = tid; i < r; i += 256) st(entry + i, ld(dkv + i) * inv * ld(a.c_norm + i));
   }
-  if (a.ql && blockIdx.y + 1 == gridDim.y) {
+  if (a.ql && y + 1 == ny) {
     const A* ql = a.ql + (int64_t)t * a.ql_stride;
     A* out = a.ql_out + (int64_t)t * a.q_rank;
     float ss = 0.f;
     for (int i = tid; i < a.q_rank; i += 256) { const float v = ld(ql + i); ss += v * v; }
     ss = block_sum<4>(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)a.q_rank + eps);
+    const float inv = 1.0f / sqrtf(ss / (float)a.q_rank + p.eps);
     for (int i = tid; i < a.q_rank; i += 256) st(out + i, ld(ql + i) * inv * ld(a.ql_norm + i));
   }
-  const int half = rot_dims >> 1;
+  const int half = p.rot_dims >> 1;
   const float fpos = (float)pos;
-  // vector 0 = the shared key part (-> cache), vectors 1 .. H = the heads' rotated query parts (-> qc, fp32)
-  const int w_end = (a.q ? H + 1 : 1) * dr;
-  for (int w = (dkv ? 0 : dr) + blockIdx.y * 256 + tid; w < w_end; w += 256 * gridDim.y) {
-    const int vec = w / dr, i = w % dr;
-    const A* src = vec == 0 ? dkv + r : a.q + (int64_t)t * a.q_stride + (int64_t)(vec - 1) * (dn + dr) + dn;
+  // vector 0 = the shared key part (-> cache), vectors 1 .. p.H = the heads' rotated query parts (-> qc, fp32)
+  const int w_end = (a.q ? p.H + 1 : 1) * p.dr;
+  for (int w = (dkv ? 0 : p.dr) + y * 256 + tid; w < w_end; w += 256 * ny) {
+    const int vec = w / p.dr, i = w % p.dr;
+    const A* src = vec == 0 ? dkv + r : a.q + (int64_t)t * a.q_stride + (int64_t)(vec - 1) * (p.dn + p.dr) + p.dn;
     float out = ld(src + i);
-    if (i < rot_dims) {
+    if (i < p.rot_dims) {
       float sn, cs;
-      const int f = pairs ? i >> 1 : (i < half ? i : i - half);
-      const bool second = pairs ? (i & 1) : i >= half;
-      const float other = ld(src + (pairs ? i ^ 1 : second ? i - half : i + half));
-      sincosf(fpos * inv_freq[f], &sn, &cs);
+      const int f = p.pairs ? i >> 1 : (i < half ? i : i - half);
+      const bool second = p.pairs ? (i & 1) : i >= half;
+      const float other = ld(src + (p.pairs ? i ^ 1 : second ? i - half : i + half));
+      sincosf(fpos * p.inv_freq[f], &sn, &cs);
       out = second ? out * cs + other * sn : out * cs - other * sn;
     }
     if (vec == 0) st(entry + r + i, out);
-    else a.qc[((int64_t)t * H + (vec - 1)) * E + r + i] = out;
+    else a.qc[((int64_t)t * p.H + (vec - 1)) * E + r + i] = out;
   }
+}
+template <typename A>
+__global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrep<A> a, LatentPlace p, A* __restrict__ cache) {
+  latent_prep_block<A>(blockIdx.x, blockIdx.y, gridDim.y, a, p, cache);
+}
+
+// Few rows (decoding): the prep and the product that carries the heads' queries into the latent space, which touch different values of qc and
+// read the same rows, in one grid - two launches that wait on chains of their own and leave most of the chip idle.  The product's workgroups
+// first.  4 rows, 16 heads, rank 512: 4.5 + 5.0 us one after the other, 5.1 in one; 16 steps of four such layers and their prompts
+// 8.70 -> 8.43 ms.
+template <int OB>
+__global__ __launch_bounds__(256) void latent_prep_absorb_kernel(LatentPrep<uint16_t> a, LatentPlace p, uint16_t* __restrict__ cache, int ny,
+                                                                 pegainfer_gemm_desc d, int wk, int gx, int gy, int n_gemm) {
+  const int b = blockIdx.x;
+  if (b < n_gemm) {
+    gemm_rows_mfma_block<uint16_t, float, uint16_t, OB, false>(d, wk, ExpertForm{}, b % gx, b / gx % gy, b / (gx * gy));
+    return;
+  }
+  latent_prep_block<uint16_t>((b - n_gemm) / ny, (b - n_gemm) % ny, ny, a, p, cache);
+}
+template <int R, int MB>
+__global__ __launch_bounds__(256) void latent_prep_absorb_f32_kernel(LatentPrep<float> a, LatentPlace p, float* __restrict__ cache, int ny,
+                                                                     pegainfer_gemm_desc d, int gy, int n_gemm) {
+  const int b = blockIdx.x;
+  if (b < n_gemm) {
+    gemm_rows_direct_block<float, float, uint16_t, R, MB, false>(d, 0, 0, 0, b % gy, b / gy);
+    return;
+  }
+  latent_prep_block<float>((b - n_gemm) / ny, (b - n_gemm) % ny, ny, a, p, cache);
 }
 
 // What a split of a row leaves for the merge, all fp32: the rows' accumulators ([row][split][rank]; row = t * H + h), and behind
@@ -817,6 +849,28 @@ static inline int latent_max_splits(int max_kv_len, int split_keys) {
   return std::max(1, (max_kv_len + sk - 1) / sk);
 }
 
+static bool latent_prep_ok(const pegainfer_latent_prep_desc* d) {
+  return !(d->rot_dims < 0 || d->rot_dims > d->rot || (d->rot_dims & 1) || d->rank <= 0 || d->page_size <= 0 || d->heads < 0 || d->nope < 0 ||
+           (d->rot_dims > 0 && !d->inv_freq) || (d->rot_layout != PEGAINFER_ROT_PAIRS && d->rot_layout != PEGAINFER_ROT_HALVES) ||
+           (!d->dkv && !d->q && !d->ql) || (d->dkv && (!d->c_norm_w || !d->cache)) || (d->q && !d->qc) ||
+           (d->ql && (!d->ql_norm_w || !d->ql_out || d->q_rank <= 0)));
+}
+template <typename A>
+static LatentPrep<A> latent_prep_parts(const pegainfer_latent_prep_desc* d) {
+  return {static_cast<const A*>(d->dkv), d->dkv_stride, static_cast<const A*>(d->c_norm_w),
+          static_cast<const A*>(d->ql), d->ql_stride, static_cast<const A*>(d->ql_norm_w), static_cast<A*>(d->ql_out), d->q_rank,
+          static_cast<const A*>(d->q), d->q_stride, d->qc};
+}
+static LatentPlace latent_prep_place(const pegainfer_latent_prep_desc* d) {
+  return {d->eps, d->inv_freq, d->rot_dims, d->rot_layout == PEGAINFER_ROT_PAIRS, d->positions, d->token_req, d->page_indptr, d->page_ids,
+          d->page_stride, d->layer_off, d->page_size, d->heads, d->nope, d->rot, d->rank};
+}
+// few rows (decoding): a row's rotated parts spread over several workgroups; many rows fill the chip alone
+static int latent_prep_per_row(const pegainfer_latent_prep_desc* d) {
+  const int vals = (d->q ? d->heads + 1 : 1) * d->rot;
+  return d->n_tokens >= 256 ? 1 : std::max(d->ql && d->dkv ? 2 : 1, std::min(8, (vals + 255) / 256));
+}
+
 }  // namespace pk
 
 extern "C" {
@@ -842,24 +896,52 @@ pegainfer_status_t pegainfer_latent_prep(const void* proj, int64_t proj_row_stri
 pegainfer_status_t pegainfer_latent_prep_form(const pegainfer_latent_prep_desc* d, pegainfer_stream_t stream) {
   if (!d) return (pegainfer_status_t)hipErrorInvalidValue;
   if (d->n_tokens <= 0) return 0;
-  if (d->rot_dims < 0 || d->rot_dims > d->rot || (d->rot_dims & 1) || d->rank <= 0 || d->page_size <= 0 || d->heads < 0 || d->nope < 0 ||
-      (d->rot_dims > 0 && !d->inv_freq) || (d->rot_layout != PEGAINFER_ROT_PAIRS && d->rot_layout != PEGAINFER_ROT_HALVES) ||
-      (!d->dkv && !d->q && !d->ql) || (d->dkv && (!d->c_norm_w || !d->cache)) || (d->q && !d->qc) ||
-      (d->ql && (!d->ql_norm_w || !d->ql_out || d->q_rank <= 0)))
-    return (pegainfer_status_t)hipErrorInvalidValue;
+  if (!latent_prep_ok(d)) return (pegainfer_status_t)hipErrorInvalidValue;
   if (!by_dtype(d->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
-        LatentPrep<A> a{static_cast<const A*>(d->dkv), d->dkv_stride, static_cast<const A*>(d->c_norm_w),
-                        static_cast<const A*>(d->ql), d->ql_stride, static_cast<const A*>(d->ql_norm_w), static_cast<A*>(d->ql_out), d->q_rank,
-                        static_cast<const A*>(d->q), d->q_stride, d->qc};
-        // few rows (decoding): a row's rotated parts spread over several workgroups; many rows fill the chip alone
-        const int vals = (d->q ? d->heads + 1 : 1) * d->rot;
-        const int per_row = d->n_tokens >= 256 ? 1 : std::max(d->ql && d->dkv ? 2 : 1, std::min(8, (vals + 255) / 256));
-        latent_prep_kernel<A><<<dim3(d->n_tokens, per_row), 256, 0, as_stream(stream)>>>(
-            a, d->eps, d->inv_freq, d->rot_dims, d->rot_layout == PEGAINFER_ROT_PAIRS, d->positions, d->token_req, d->page_indptr,
-            d->page_ids, static_cast<A*>(d->cache), d->page_stride, d->layer_off, d->page_size, d->heads, d->nope, d->rot, d->rank);
+        latent_prep_kernel<A><<<dim3(d->n_tokens, latent_prep_per_row(d)), 256, 0, as_stream(stream)>>>(latent_prep_parts<A>(d), latent_prep_place(d),
+                                                                                                       static_cast<A*>(d->cache));
       }))
     return (pegainfer_status_t)hipErrorInvalidValue;
+  return (pegainfer_status_t)hipGetLastError();
+}
+
+int32_t pegainfer_latent_prep_absorb_ok(const pegainfer_latent_prep_desc* d, const pegainfer_gemm_desc* g) {
+  if (!d || !g || d->n_tokens <= 0 || !latent_prep_ok(d) || g->plain || g->tile_group || g->x_row_index || g->y_row_index || g->m <= 0 || g->k <= 0 ||
+      g->groups <= 0 || g->groups > 65535 || g->epilogue != PEGAINFER_EPI_NONE || g->rows != d->n_tokens || g->x_dtype != d->dtype || g->w_dtype != d->dtype ||
+      g->y_dtype != kDtF32 || !chunks_ok(*g))
+    return 0;
+  // the forms that these rows take by themselves, so the same bits; of fp32 up to two outputs per wave (beyond, the product fills the chip by itself)
+  if (d->dtype == kDtBf16) return g->rows <= kRowsMax;
+  return d->dtype == kDtF32 && g->rows <= 4 && rows_direct_outputs(*g, g->rows == 3 ? 4 : g->rows, false) <= 2;
+}
+
+pegainfer_status_t pegainfer_latent_prep_absorb(const pegainfer_latent_prep_desc* d, const pegainfer_gemm_desc* g, pegainfer_stream_t stream) {
+  if (!pegainfer_latent_prep_absorb_ok(d, g)) return (pegainfer_status_t)hipErrorInvalidValue;
+  hipStream_t st = as_stream(stream);
+  const int ny = latent_prep_per_row(d), n_prep = d->n_tokens * ny;
+  const LatentPlace place = latent_prep_place(d);
+  if (d->dtype == kDtBf16) {
+    const RowsMfmaShape f = rows_mfma_shape(*g);
+    const int gx = (int)f.grid.x, gy = (int)f.grid.y, n_gemm = gx * gy * (int)f.grid.z;
+    auto go = [&](auto kern) {
+      kern<<<n_gemm + n_prep, 256, 0, st>>>(latent_prep_parts<uint16_t>(d), place, static_cast<uint16_t*>(d->cache), ny, *g, f.wk, gx, gy, n_gemm);
+    };
+    if (f.ob == 2) go(latent_prep_absorb_kernel<2>);
+    else go(latent_prep_absorb_kernel<1>);
+  } else {
+    const int R = g->rows == 3 ? 4 : g->rows, mb = rows_direct_outputs(*g, R, false);
+    const int gy = ceil_div(g->m, 4 * mb), n_gemm = gy * g->groups;
+    auto go = [&](auto kern) { kern<<<n_gemm + n_prep, 256, 0, st>>>(latent_prep_parts<float>(d), place, static_cast<float*>(d->cache), ny, *g, gy, n_gemm); };
+    auto by_outputs = [&](auto r) {
+      constexpr int RR = decltype(r)::value;
+      if (mb == 2) go(latent_prep_absorb_f32_kernel<RR, 2>);
+      else go(latent_prep_absorb_f32_kernel<RR, 1>);
+    };
+    if (R == 1) by_outputs(std::integral_constant<int, 1>());
+    else if (R == 2) by_outputs(std::integral_constant<int, 2>());
+    else by_outputs(std::integral_constant<int, 4>());
+  }
   return (pegainfer_status_t)hipGetLastError();
 }
 

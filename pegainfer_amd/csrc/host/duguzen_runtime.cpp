@@ -738,17 +738,26 @@ struct Model {
       const int E = c.entry(), Mp = c.proj_rows(), qrow = m.heads * (m.nope + m.rot);
       const Norm* next_pre = li + 1 < layers.size() ? &weights[layers[li + 1].owner].n1 : nullptr;
       if (linear(w.proj, h, proj, Mp, Ti, D)) return -1;
-      DZ_K(pegainfer_latent_prep(proj, Mp, qrow, w.cnorm, eps, w.inv_freq, m.rot_dims, d_pos, d_req, d_ind, d_pages, cache,
-                                 page_stride, c.cache_off, kPageSize, qc, m.heads, m.nope, m.rot, m.rank, Ti, dtype, S()));
-      if (m.nope > 0) {   // absorb: qc[t, h, :rank] = sum_d q[t, h, d] * Wuk[h * nope + d, :]
-        pegainfer_gemm_desc d{};
-        d.x = proj; d.w = w.uk; d.y = qc;
-        d.x_dtype = d.w_dtype = dtype; d.y_dtype = PEGAINFER_DTYPE_F32;
-        d.m = m.rank; d.k = m.nope; d.rows = Ti; d.groups = m.heads;
-        d.x_row_stride = Mp; d.x_group_stride = m.nope + m.rot;
-        d.w_m_stride = m.nope; d.w_k_stride = 1; d.w_group_stride = (int64_t)m.nope * m.rank;
-        d.y_row_stride = (int64_t)m.heads * E; d.y_group_stride = E;
-        d.plain = plain_kernels;
+      pegainfer_latent_prep_desc pr{};
+      pr.dkv = static_cast<const uint8_t*>(proj) + (size_t)qrow * esize(); pr.dkv_stride = Mp; pr.c_norm_w = w.cnorm;
+      pr.q = proj; pr.q_stride = Mp; pr.qc = qc;
+      pr.eps = eps; pr.inv_freq = w.inv_freq; pr.rot_dims = m.rot_dims; pr.rot_layout = PEGAINFER_ROT_HALVES;
+      pr.positions = d_pos; pr.token_req = d_req; pr.page_indptr = d_ind; pr.page_ids = d_pages;
+      pr.cache = cache; pr.page_stride = page_stride; pr.layer_off = c.cache_off; pr.page_size = kPageSize;
+      pr.heads = m.heads; pr.nope = m.nope; pr.rot = m.rot; pr.rank = m.rank; pr.n_tokens = Ti; pr.dtype = dtype;
+      pegainfer_gemm_desc d{};   // absorb: qc[t, h, :rank] = sum_d q[t, h, d] * Wuk[h * nope + d, :]
+      d.x = proj; d.w = w.uk; d.y = qc;
+      d.x_dtype = d.w_dtype = dtype; d.y_dtype = PEGAINFER_DTYPE_F32;
+      d.m = m.rank; d.k = m.nope; d.rows = Ti; d.groups = m.heads;
+      d.x_row_stride = Mp; d.x_group_stride = m.nope + m.rot;
+      d.w_m_stride = m.nope; d.w_k_stride = 1; d.w_group_stride = (int64_t)m.nope * m.rank;
+      d.y_row_stride = (int64_t)m.heads * E; d.y_group_stride = E;
+      d.plain = plain_kernels;
+      const bool together = m.nope > 0 && pegainfer_latent_prep_absorb_ok(&pr, &d);
+      if (!together) DZ_K(pegainfer_latent_prep_form(&pr, S()));
+      if (together) {
+        DZ_K(pegainfer_latent_prep_absorb(&pr, &d, S()));
+      } else if (m.nope > 0) {
         DZ_K(pegainfer_gemm_strided(&d, S()));
       } else if (captured) {
         DZ_K(pegainfer_zero_words(qc, Ti * m.heads * E, S()));
@@ -817,7 +826,7 @@ struct Model {
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and replayed; steps with
-    // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step: 9.3 -> 9.05 ms for their prompts and 16 steps.
+    // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step at the time (45 now): 9.3 -> 9.05 ms for their prompts and 16 steps.
     if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, max_kv};
       hipGraphExec_t exec = graphs.find(key);

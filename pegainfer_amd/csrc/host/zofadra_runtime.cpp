@@ -344,7 +344,6 @@ class Model : public StepModel {
     PSTEP_K(pegainfer_latent_prep_form(&p, S()));
     if (linear(w.uq, ql, qb, H * qrow, s.T, c.q_rank)) return -1;
     p2.q = qb; p2.q_stride = (int64_t)H * qrow; p2.qc = qf;
-    PSTEP_K(pegainfer_latent_prep_form(&p2, S()));
     pegainfer_gemm_desc g{};            // absorb: qc[t, h, :rank] = W_uk_h^T q[t, h, :dim]
     g.x = qb; g.w = w.uk; g.y = qf;
     g.x_dtype = g.w_dtype = dtype; g.y_dtype = PEGAINFER_DTYPE_F32;
@@ -353,7 +352,12 @@ class Model : public StepModel {
     g.w_m_stride = c.dim; g.w_k_stride = 1; g.w_group_stride = (int64_t)c.dim * c.kv_rank;
     g.y_row_stride = (int64_t)H * E; g.y_group_stride = E;
     g.plain = plain_kernels;
-    PSTEP_K(pegainfer_gemm_strided(&g, S()));
+    if (pegainfer_latent_prep_absorb_ok(&p2, &g)) {
+      PSTEP_K(pegainfer_latent_prep_absorb(&p2, &g, S()));
+    } else {
+      PSTEP_K(pegainfer_latent_prep_form(&p2, S()));
+      PSTEP_K(pegainfer_gemm_strided(&g, S()));
+    }
     const TileTable& t = s.flat_tiles[(size_t)c.tiles];
     const bool tiled = !plain_kernels && pegainfer_latent_attention_tiled_ok(c.kv_rank, c.rot_dim, page_stride, c.c_off, dtype);
     const int deals = t.count >= kFewTiles ? 1 : std::max(1, std::min(kMaxDeals, kSplitGroups / t.count));

@@ -622,8 +622,9 @@ def paged_attention_opt(q, cache, page_stride, k_off, v_off, page_size, rg, page
 
 
 def latent_prep_form(rg, page_indptr, page_ids, cache, page_stride, layer_off, page_size, heads, nope, rot, rank, eps, inv_freq, pairs,
-                     dkv=None, c_norm_w=None, ql=None, ql_norm_w=None, q=None, qc=None):
-    """dkv [rows, rank + rot] -> cache; ql [rows, q_rank] -> returned normed; q [rows, heads * (nope + rot)] -> qc[:, :, rank:]"""
+                     dkv=None, c_norm_w=None, ql=None, ql_norm_w=None, q=None, qc=None, absorb=None):
+    """dkv [rows, rank + rot] -> cache; ql [rows, q_rank] -> returned normed; q [rows, heads * (nope + rot)] -> qc[:, :, rank:];
+    absorb: a GemmDesc done in the same launch, False is returned where the launch does not take it"""
     T = rg.positions.numel()
     out = torch.empty((T, ql.shape[1]), dtype=cache.dtype, device=cache.device) if ql is not None else None
     d = LatentPrepDesc(eps=float(eps), inv_freq=_p(inv_freq), rot_dims=rot, rot_layout=0 if pairs else 1, positions=_p(rg.positions),
@@ -636,6 +637,11 @@ def latent_prep_form(rg, page_indptr, page_ids, cache, page_stride, layer_off, p
         d.ql, d.ql_stride, d.ql_norm_w, d.ql_out, d.q_rank = _p(ql), ql.stride(0), _p(ql_norm_w), _p(out), ql.shape[1]
     if q is not None:
         d.q, d.q_stride, d.qc = _p(q), q.stride(0), _p(qc)
+    if absorb is not None:
+        if not ffi.lib().pegainfer_latent_prep_absorb_ok(ctypes.addressof(d), ctypes.addressof(absorb)):
+            return False
+        _chk(ffi.lib().pegainfer_latent_prep_absorb(ctypes.addressof(d), ctypes.addressof(absorb), _stream()), "latent_prep_absorb")
+        return out
     _chk(ffi.lib().pegainfer_latent_prep_form(ctypes.addressof(d), _stream()), "latent_prep_form")
     return out
 
