@@ -1,0 +1,343 @@
+// The gated delta rule of recurrent.hip (one decay per head) for prompts: 16 tokens at a time on fp32 matrix-core products.
+//   S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
+// Token by token the recurrence is a chain of one state update per token, 374 cycles of it a token with one wave per SIMD (53 instructions of its
+// own, waits for the rest).  Over a chunk the updates are known from the state S0 before it: with c_t = g_0 .. g_t and D[t][s] = g_{s+1} .. g_t
+//   U = T' (V - diag(c) K S0),   T' = (I + L)^-1 diag(beta),   L[t][s] = beta_t D[t][s] k_t . k_s  (s < t)
+//   O = diag(c) Q S0 + M U,      M[t][s] = D[t][s] q_t . k_s   (s <= t)
+//   S = c_15 S0 + K^T diag(D[15][.]) U
+// delta_chunk_prep_kernel brings q and k to unit length and makes T', M and the factors for every (chunk, head) side by side; delta_chunk_kernel walks the chunks of an (entry,
+// head, 16 value columns), its four waves dim / 4 rows of S each.  All products are v_mfma_f32_16x16x4_f32 (plain fp32) and every decay is a product of
+// gates at most 1, never a quotient, so strong decays only underflow as they do one by one.
+// 1024 tokens of 32 heads of 128 x 128: 15 + 181 us (prep and token by token), 15 + 74 here; eight entries of 700 tokens, 8 heads 16 + 173 and 19 + 110.
+// Against 64 bits the read-outs are off by 2.1e-7 (2.3e-7 token by token) with slow decays, by 1.2 - 1.8e-7 (1.1 - 1.5e-7) with fast ones; fp32 logits of
+// whole models by the same amount either way (0.9 - 1.8e-6).
+#include <algorithm>
+
+#include "common.h"
+#include "typed.h"
+#include "sigmoid_power.h"
+#include "pegainfer_kernels_blocks.h"
+
+namespace pk {
+
+constexpr int kDc = 16;                        // tokens of a chunk
+constexpr int kDcFloats = 2 * kDc * kDc + 2 * kDc + 32;  // of a (chunk, head): T', M, c, D[15][.], pad
+
+// Chunks are numbered without a table: entry e's first is row0 / 16 + e (the next entry's first lies behind its last), so there are
+// rows / 16 + entries numbers at most and some that stand for none.
+__device__ __forceinline__ int delta_first_chunk(int row0, int e) { return row0 / kDc + e; }
+
+// A wave per (chunk, key head): k . k and q . k of the chunk's tokens, then, sixteen lanes per value head, the triangular matrix and its inverse
+// by forward substitution, a lane per column.
+template <typename A, int NB>
+__global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
+                                                               int64_t proj_stride, int64_t b_off, int64_t a_off, const A* __restrict__ A_log,
+                                                               const A* __restrict__ dt_bias, float* __restrict__ ws, int H, int G,
+                                                               const int32_t* __restrict__ entry_row0, int n_entries) {
+  constexpr int DIM = 64 * NB;
+  __shared__ float s_kk[4][kDc][kDc + 1], s_qk[4][kDc][kDc + 1];
+  __shared__ __attribute__((aligned(16))) float s_l[4][4][kDc][kDc + 4], s_gb[4][4][kDc][2];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = lane & 15, j = lane >> 4;
+  const int chunk = blockIdx.x, g = blockIdx.y * 4 + wave;
+  int lo = 0, hi = n_entries - 1;              // the last entry whose first chunk is not behind this one
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (delta_first_chunk(entry_row0[mid], mid) <= chunk) lo = mid; else hi = mid - 1;
+  }
+  const int row0 = entry_row0[lo], len = entry_row0[lo + 1] - row0, at = (chunk - delta_first_chunk(row0, lo)) * kDc;
+  if (at < 0 || at >= len || g >= G) return;   // (waves share nothing: there is no barrier below)
+  const int tc = min(kDc, len - at);
+  const int64_t row = row0 + at + min(t, tc - 1);
+  const float live = t < tc ? 1.f : 0.f;
+  // lane: token t, dims 16 b + 4 j .. + 3 - both operands of the products below
+  f32x4 k[DIM / 16], q[DIM / 16];
+  float *qp = qkv + row * qkv_stride + (int64_t)g * DIM + 4 * j, *kp = qp + (int64_t)G * DIM;
+  f32x4 ks[2] = {}, qs[2] = {};                // (short sums: a length's error is in all of its values)
+#pragma unroll
+  for (int b = 0; b < DIM / 16; ++b) {
+    k[b] = *reinterpret_cast<const f32x4*>(kp + 16 * b);
+    q[b] = *reinterpret_cast<const f32x4*>(qp + 16 * b);
+  }
+#pragma unroll
+  for (int b = 0; b < DIM / 16; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      k[b][r] = t < tc ? k[b][r] : 0.f;
+      q[b][r] = t < tc ? q[b][r] : 0.f;
+      ks[b & 1][r] = fmaf(k[b][r], k[b][r], ks[b & 1][r]);
+      qs[b & 1][r] = fmaf(q[b][r], q[b][r], qs[b & 1][r]);
+    }
+  ks[0] += ks[1];
+  qs[0] += qs[1];
+  float kss = (ks[0].x + ks[0].y) + (ks[0].z + ks[0].w), qss = (qs[0].x + qs[0].y) + (qs[0].z + qs[0].w);
+  kss += __shfl_xor(kss, 16, kWave); kss += __shfl_xor(kss, 32, kWave);
+  qss += __shfl_xor(qss, 16, kWave); qss += __shfl_xor(qss, 32, kWave);
+  const float ik = 1.0f / sqrtf(kss + 1e-6f), iq = 1.0f / (sqrtf((float)DIM) * sqrtf(qss + 1e-6f));
+  f32x4 kk[8] = {}, qk[8] = {};                // (eight sums each: closer to the sum in 64 bits than one long chain)
+#pragma unroll
+  for (int b = 0; b < DIM / 16; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      k[b][r] *= ik;
+      q[b][r] *= iq;
+      f32x4 &a = kk[4 * (b & 1) + r], &c = qk[4 * (b & 1) + r];
+      a = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][r], k[b][r], a, 0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(q[b][r], k[b][r], c, 0, 0, 0);
+    }
+  if (t < tc) {
+#pragma unroll
+    for (int b = 0; b < DIM / 16; ++b) {
+      *reinterpret_cast<f32x4*>(kp + 16 * b) = k[b];
+      *reinterpret_cast<f32x4*>(qp + 16 * b) = q[b];
+    }
+  }
+#pragma unroll
+  for (int w = 4; w; w >>= 1)
+#pragma unroll
+    for (int i = 0; i < w; ++i) {
+      kk[i] += kk[i + w];
+      qk[i] += qk[i + w];
+    }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {                // lane: rows 4 j + r, column t
+    s_kk[wave][4 * j + r][t] = kk[0][r];
+    s_qk[wave][4 * j + r][t] = qk[0][r];
+  }
+  const int per = H / G;
+  for (int h0 = 0; h0 < per; h0 += 4) {
+    const int h = g * per + min(h0 + j, per - 1);
+    const bool own = h0 + j < per;
+    const A* pr = proj + row * proj_stride;
+    const float gt = live > 0.f ? expf(-expf(ld(A_log + h)) * softplus_f(ld(pr + a_off + h) + ld(dt_bias + h))) : 1.f;
+    const float bt = live * sigmoid_f(ld(pr + b_off + h));
+    s_gb[wave][j][t][0] = gt;
+    s_gb[wave][j][t][1] = bt;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // a wave's own LDS writes, in its own order
+    float* out = ws + ((int64_t)chunk * H + h) * kDcFloats;
+    // lane: column t of head h; p = D[row][t]
+    float p = 0.f;
+#pragma unroll
+    for (int i = 0; i < kDc; ++i) {
+      const float gi = s_gb[wave][j][i][0], bi = s_gb[wave][j][i][1];
+      p = i == t ? 1.f : p * gi;               // 0 above the diagonal
+      s_l[wave][j][i][t] = i > t ? bi * p * s_kk[wave][i][t] : 0.f;
+      if (own) out[kDc * kDc + i * kDc + t] = i >= t ? p * s_qk[wave][i][t] : 0.f;
+      if (t == 0 && own) out[2 * kDc * kDc + i] = s_gb[wave][j][0][0] * p;     // c_i = g_0 D[i][0]
+    }
+    if (own) out[2 * kDc * kDc + kDc + t] = p;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    float T[kDc];
+#pragma unroll
+    for (int i = 0; i < kDc; ++i) {
+      float sum[2] = {};
+#pragma unroll
+      for (int s4 = 0; s4 * 4 < i; ++s4) {
+        const f32x4 l = *reinterpret_cast<const f32x4*>(&s_l[wave][j][i][4 * s4]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (4 * s4 + u < i) sum[u & 1] = fmaf(l[u], T[4 * s4 + u], sum[u & 1]);
+      }
+      T[i] = i == t ? 1.f : i > t ? -(sum[0] + sum[1]) : 0.f;
+      if (own) out[i * kDc + t] = T[i] * bt;
+    }
+  }
+}
+
+// Bound by its chain of products: 4 NB for K S0, as many for Q S0, 4 for U and 4 NB for S, 32 cycles each, and one exchange through LDS per chunk.
+// S lies as the products leave it, which is also how they take it: accumulator r of block b is a wave's row NB (4 (lane / 16) + r) + b of S, so
+// K and Q come as 16-byte loads in that order of k (and K's other operand, a lane per row, NB values at a time), and U's accumulators are
+// the next product's operand in the same way.  Vector memory takes 16 cycles an instruction whatever it carries, so what all four waves need is
+// fetched by a fifth, which also makes the outputs; nothing waits for those.  Operands are asked for two chunks ahead.
+constexpr int kDcThreads = 320;
+template <int NB>
+__global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qkv, int qkv_stride, const float* ws, float* __restrict__ state,
+                                                                 int64_t slot_stride, float* __restrict__ o, int H, int G, int vdim,
+                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot) {
+  constexpr int DIM = 64 * NB;
+  __shared__ f32x4 s_part[2][4][2][64];        // K S0 and Q S0 over a wave's rows of S
+  __shared__ f32x4 s_common[2][4][64];         // by lane: values, T', c, D[15][.]
+  __shared__ float s_end[2];
+  const int e = blockIdx.z, h = blockIdx.y, col = blockIdx.x * 16 + (threadIdx.x & 15);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l15 = lane & 15, j = lane >> 4;
+  const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
+  if (len <= 0) return;
+  const int n = (len + kDc - 1) / kDc, g0 = h / (H / G);
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };     // (not the loads of the chunks ahead)
+  // rows past the entry's end: its last one, which T' leaves out
+  auto row_at = [&](int c, int t) { return (int64_t)(row0 + min(c * kDc + t, len - 1)) * qkv_stride; };
+  auto sum_of_waves = [&](int c, int which) {
+    const auto& part = s_part[c & 1];
+    return (part[0][which][lane] + part[1][which][lane]) + (part[2][which][lane] + part[3][which][lane]);
+  };
+  auto updates = [&](const f32x4& v, const f32x4& T, const f32x4& decay, int c) {
+    f32x4 U = {};
+    const f32x4 R = v - decay * sum_of_waves(c, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) U = __builtin_amdgcn_mfma_f32_16x16x4f32(T[s], R[s], U, 0, 0, 0);
+    return U;
+  };
+  // Chunk c's operands in x; those of c + 1 are on the way while it is worked on, those of c + 2 are asked for.  One loop with one way out: with
+  // more, the compiler's waits at its head have to cover them all.  `whole`: all of the chunk's rows are there.
+  auto walk = [&](auto& x, auto& y, auto& z, auto&& fetch, auto&& work) {
+    fetch(x, 0);
+    fetch(y, 1);
+    int c = 0;
+    for (; (c + 3) * kDc <= len; c += 3) {
+      fetch(z, c + 2);
+      work(x, c, std::true_type());
+      fetch(x, c + 3);
+      work(y, c + 1, std::true_type());
+      fetch(y, c + 4);
+      work(z, c + 2, std::true_type());
+    }
+    if (c + 2 < n) fetch(z, c + 2);
+    if (c < n) work(x, c, std::false_type());
+    if (c + 1 < n) work(y, c + 1, std::false_type());
+    if (c + 2 < n) work(z, c + 2, std::false_type());
+  };
+  if (wave == 4) {
+    const float *w0 = ws + ((int64_t)delta_first_chunk(row0, e) * H + h) * kDcFloats, *v0 = qkv + (int64_t)2 * G * DIM + (int64_t)h * vdim + col;
+    struct Chunk { f32x4 v, T, M, decay, left; float end; } x, y, z;
+    auto fetch = [&](Chunk& x, int c) {
+      // asked for here and in this order: the compiler would gather the loads of three chunks, whose waits are then one (the pointers are not
+      // `__restrict__`, so that these hold)
+      asm volatile("" ::: "memory");
+      c = min(c, n - 1);
+      const float *w = w0 + (int64_t)c * H * kDcFloats, *f = w + 2 * kDc * kDc;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x.v[s] = v0[row_at(c, 4 * j + s)];
+      x.T = *reinterpret_cast<const f32x4*>(w + l15 * kDc + 4 * j);
+      x.M = *reinterpret_cast<const f32x4*>(w + kDc * kDc + l15 * kDc + 4 * j);
+      x.decay = *reinterpret_cast<const f32x4*>(f + 4 * j);
+      x.left = *reinterpret_cast<const f32x4*>(f + kDc + 4 * j);
+      x.end = f[kDc - 1];
+      asm volatile("" ::: "memory");
+    };
+    auto work = [&](const Chunk& x, int c, auto whole) {
+      auto& to = s_common[c & 1];
+      to[0][lane] = x.v;
+      to[1][lane] = x.T;
+      to[2][lane] = x.decay;
+      to[3][lane] = x.left;
+      if (lane == 0) s_end[c & 1] = x.end;
+      barrier();
+      const f32x4 Q = sum_of_waves(c, 1), U = updates(x.v, x.T, x.decay, c);
+      f32x4 O = {};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(x.M[s], U[s], O, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) O[r] = fmaf(x.decay[r], Q[r], O[r]);
+      float* out = o + (int64_t)(row0 + c * kDc) * ((int64_t)H * vdim) + (int64_t)h * vdim + col;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (whole.value || c * kDc + 4 * j + r < len) out[(int64_t)(4 * j + r) * (H * vdim)] = O[r];
+    };
+    walk(x, y, z, fetch, work);
+    return;
+  }
+  const int d0 = wave * 16 * NB;
+  float* S_g = state + (int64_t)entry_slot[e] * slot_stride + (int64_t)h * DIM * vdim + col;
+  f32x4 S[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[b][r] = S_g[(int64_t)(d0 + NB * (4 * j + r) + b) * vdim];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) asm volatile("" : "+v"(S[b]));    // waited for here: the wait must not land in the loop
+  const float *q0 = qkv + (int64_t)g0 * DIM + d0, *k0 = q0 + (int64_t)G * DIM;
+  struct Chunk { float k[4 * NB], q[4 * NB], kt[4][NB]; } x, y, z;
+  auto fetch = [&](Chunk& x, int c) {
+    asm volatile("" ::: "memory");
+    c = min(c, n - 1);
+    const int64_t mine = row_at(c, l15) + 4 * NB * j;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      ld4(k0 + mine + 4 * b, &x.k[4 * b]);
+      ld4(q0 + mine + 4 * b, &x.q[4 * b]);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) __builtin_memcpy(x.kt[s], __builtin_assume_aligned(k0 + row_at(c, 4 * j + s) + NB * l15, NB % 4 == 0 ? 16 : NB % 2 == 0 ? 8 : 4), 4 * NB);
+    asm volatile("" ::: "memory");
+  };
+  auto work = [&](const Chunk& x, int c, auto) {
+    f32x4 P[4] = {}, Q[4] = {};
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        P[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[NB * r + b], S[b][r], P[r], 0, 0, 0);
+        Q[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[NB * r + b], S[b][r], Q[r], 0, 0, 0);
+      }
+    s_part[c & 1][wave][0][lane] = (P[0] + P[1]) + (P[2] + P[3]);
+    s_part[c & 1][wave][1][lane] = (Q[0] + Q[1]) + (Q[2] + Q[3]);
+    barrier();
+    const auto& from = s_common[c & 1];
+    const f32x4 left = from[3][lane];
+    const float end = s_end[c & 1];
+    const f32x4 E = left * updates(from[0][lane], from[1][lane], from[2][lane], c);
+    f32x4 X[NB] = {};                          // (a sum of its own, so that S is rounded once per chunk)
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) X[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kt[s][b], E[s], X[b], 0, 0, 0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[b][r] = fmaf(end, S[b][r], X[b][r]);
+  };
+  walk(x, y, z, fetch, work);
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S_g[(int64_t)(d0 + NB * (4 * j + r) + b) * vdim] = S[b][r];
+}
+
+template <typename F>
+static bool by_rows_of_s(int dim, F&& fn) {
+  if (dim == 64) fn(std::integral_constant<int, 1>());
+  else if (dim == 128) fn(std::integral_constant<int, 2>());
+  else if (dim == 192) fn(std::integral_constant<int, 3>());
+  else if (dim == 256) fn(std::integral_constant<int, 4>());
+  else return false;
+  return true;
+}
+
+}  // namespace pk
+
+extern "C" {
+using namespace pk;
+
+int64_t pegainfer_delta_rule_workspace(int32_t n_rows, int32_t n_entries, int32_t heads) {
+  return ((int64_t)n_rows / kDc + n_entries) * heads * kDcFloats;
+}
+
+int32_t pegainfer_delta_rule_chunked_ok(int32_t dim, int32_t vdim, const float* qkv, int64_t qkv_stride) {
+  return (dim == 64 || dim == 128 || dim == 192 || dim == 256) && vdim > 0 && vdim % 16 == 0 && qkv_stride % 4 == 0 && qkv_stride <= INT32_MAX && host_aligned16(qkv);
+}
+
+pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                                int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
+                                                int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
+                                                int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
+                                                int32_t dtype, pegainfer_stream_t stream) {
+  constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
+  if (n_entries <= 0 || n_rows <= 0) return 0;
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || !workspace || !host_aligned16(workspace) ||
+      !pegainfer_delta_rule_chunked_ok(dim, vdim, qkv, qkv_stride))
+    return bad;
+  hipStream_t st = as_stream(stream);
+  const dim3 prep(n_rows / kDc + n_entries, ceil_div(kv_heads, 4)), grid(vdim / 16, heads, n_entries);
+  const bool known = by_dtype(dtype, [&](auto* ptr) {
+    using A = std::remove_pointer_t<decltype(ptr)>;
+    by_rows_of_s(dim, [&](auto nb) {
+      constexpr int NB = decltype(nb)::value;
+      delta_chunk_prep_kernel<A, NB><<<prep, 256, 0, st>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off,
+                                                           static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace, heads, kv_heads,
+                                                           entry_row0, n_entries);
+      delta_chunk_kernel<NB><<<grid, kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads, vdim, entry_row0, entry_slot);
+    });
+  });
+  return known ? (pegainfer_status_t)hipGetLastError() : bad;
+}
+
+}  // extern "C"

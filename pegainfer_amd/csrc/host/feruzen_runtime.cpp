@@ -83,6 +83,9 @@ constexpr float kGluAlpha = 1.702f;  // the clamp-GLU's sigmoid slope, fixed by 
 // longest entry whose matrix memory runs token by token: 8 heads of 128 x 256, scan / chunks 42 / 48 us at 96 tokens, 54 / 50 at 128,
 // 222 / 65 at 512; eight entries of 64 tokens 57 / 62, of 128 96 / 71
 constexpr int kScanMax = 112;
+// longest entry whose delta rule runs token by token: 32 heads of 128 x 128, one entry of 32 tokens 14.6 / 17.4, of 64 20 / 19, of 128 32 / 27, of 1024 196 / 89 us token
+// by token / 16 at a time
+constexpr int kDeltaScanMax = 64;
 constexpr int kAttRows = 16;         // (token, query head) rows of one attention workgroup
 
 enum { kDelta = 1, kParallel = 2 };
@@ -160,6 +163,7 @@ struct Model {
   pst::StepIo io;
   uint8_t* sample_scratch = nullptr;
   pq::OptionalScratch chunk_ws;   // states between the chunks of long entries
+  pq::OptionalScratch delta_ws;   // the delta rule's triangles
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
   int32_t* sample_out_d = nullptr;
@@ -691,7 +695,17 @@ struct Model {
     if (n > 0)
       for (auto& l : layers)
         if (l.mm.heads > 0) need = std::max(need, (size_t)pegainfer_gated_matrix_memory_workspace(n, l.mm.heads, l.mm.dim, l.mm.vdim));
-    return chunk_ws.grow(need, [](size_t bytes) {
+    return grow_scratch(chunk_ws, need);
+  }
+  // room for the delta rule of a step with prompts 16 tokens at a time; false: token by token
+  bool ensure_delta(int64_t rows, int entries) {
+    size_t need = 0;
+    for (auto& l : layers)
+      if (l.type == kDelta) need = std::max(need, (size_t)pegainfer_delta_rule_workspace((int32_t)rows, entries, l.dl.heads));
+    return need > 0 && grow_scratch(delta_ws, need);
+  }
+  bool grow_scratch(pq::OptionalScratch& ws, size_t need) {
+    return ws.grow(need, [](size_t bytes) {
       void* p = nullptr;
       if (hipMalloc(&p, bytes) == hipSuccess) return p;
       (void)hipGetLastError();
@@ -826,6 +840,7 @@ struct Model {
     // long entries of the matrix memory in chunks (never part of a captured step)
     ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
     if (!ensure_chunks((int)chunks.row0.size())) chunks = ptiles::Chunks();   // no memory: the scan, which needs none, takes every entry
+    const bool delta_chunks = !single && !plain_kernels && *std::max_element(lens, lens + n) > kDeltaScanMax && ensure_delta(T, n);
     const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
     size_t chunk_off[4];
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
@@ -970,8 +985,12 @@ struct Model {
         if (single && !plain_kernels && pegainfer_recurrent_step_ok(&q)) {       // preparation, scan, norm and gate in one launch
           FZ_K(pegainfer_recurrent_step(&q, S()));
         } else {
-          FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
-                                    o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
+          if (delta_chunks && pegainfer_delta_rule_chunked_ok(d.dim, d.vdim, qkv32, c.conv_ch))
+            FZ_K(pegainfer_delta_rule_chunked(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
+                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
+          else
+            FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
+                                      o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
           FZ_K(pegainfer_head_rms_gate(o32, w.onorm, 0, at(proj, (size_t)c.o_g), Mp, 0, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
                                        Ti, dtype, S()));
         }
@@ -1253,6 +1272,7 @@ struct Model {
     free_all(&step_owned);
     free_all(&want_owned);
     chunk_ws.drop([&](float* p) { free_scratch(p); });
+    delta_ws.drop([&](float* p) { free_scratch(p); });
     if (tap) (void)hipFree(tap);
     io.drop();
     if (ev0) (void)hipEventDestroy(ev0);

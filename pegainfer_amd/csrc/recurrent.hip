@@ -10,7 +10,7 @@
 // the state is computed before or beside the chain, once per token: unit vectors and gates of the delta rule by a prep
 // launch over all rows, the matrix memory's running maximum by one lane per round and its three exponentials by sixteen.
 // A round's sixteen outputs of a column leave in one store per lane.
-//   delta_rule_kernel      S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
+//   delta_rule_kernel      S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q      (long entries with one decay per head: delta_chunk.hip)
 //   matrix_memory_kernel   m' = max(f + m, i);  S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise;  o = S^T q / (max(|n.q|, e^-m') + 1e-6)
 // A row's result depends only on the rows before it in its own request: the token order is fixed, and cutting a prompt into
 // steps only moves where the state passes through HBM (exactly, it is fp32 either way).  The matrix memory also has a form in chunks

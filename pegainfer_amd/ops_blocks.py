@@ -288,11 +288,20 @@ def route_combine_add(y_pairs, weight, add, out_dtype):
     return out
 
 
-def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_heads, dim, vdim, rg):
+def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_heads, dim, vdim, rg, chunked=False):
     """qkv fp32 [rows, 2 kv dim + heads vdim] (after convolution and silu), proj [rows, *] with the beta / decay inputs;
     state fp32 [slots, heads, dim, vdim] is updated in place, and so are the q / k parts of qkv (made unit vectors);
-    returns o fp32 [rows, heads * vdim]"""
+    returns o fp32 [rows, heads * vdim]; chunked: 16 tokens at a time, None where that form does not take the sizes"""
     o = torch.empty((qkv_f32.shape[0], heads * vdim), dtype=torch.float32, device=proj.device)
+    if chunked:
+        L, T = ffi.lib(), qkv_f32.shape[0]
+        if not L.pegainfer_delta_rule_chunked_ok(dim, vdim, _p(qkv_f32), qkv_f32.stride(0)):
+            return None
+        ws = torch.empty(L.pegainfer_delta_rule_workspace(T, rg.n, heads), dtype=torch.float32, device=proj.device)
+        _chk(L.pegainfer_delta_rule_chunked(_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log), _p(dt_bias), _p(ws),
+                                            _p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim, T, _p(rg.entry_row0),
+                                            _p(rg.entry_slot), rg.n, _dt(proj), _stream()), "delta_rule_chunked")
+        return o
     gates = torch.empty((qkv_f32.shape[0], 2 * heads), dtype=torch.float32, device=proj.device)
     _chk(ffi.lib().pegainfer_delta_rule(_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log),
                                         _p(dt_bias), _p(gates), _p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim,

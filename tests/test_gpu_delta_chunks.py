@@ -1,0 +1,60 @@
+"""The delta rule 16 tokens at a time against float64, token by token: entries around whole chunks (and empty ones), every number of rows of S a wave
+holds, more value heads per key head than are prepared side by side, decays from none to all at once, a state carried on by the token-by-token form."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+
+
+def reference(qkv, g, beta, S, H, G, d, dv):
+    q, k, v = qkv[:, :G * d].view(-1, G, d), qkv[:, G * d:2 * G * d].view(-1, G, d), qkv[:, 2 * G * d:].view(-1, H, dv)
+    q, k = ((t / (t.pow(2).sum(-1, keepdim=True) + 1e-6).sqrt()).repeat_interleave(H // G, 1) for t in (q, k))
+    out = []
+    for t in range(len(q)):
+        S = S * g[t].view(H, 1, 1)
+        u = beta[t].view(H, 1) * (v[t] - (S * k[t][..., None]).sum(1))
+        S = S + k[t][..., None] * u[:, None]
+        out.append((S * q[t][..., None]).sum(1).reshape(-1) * d ** -0.5)
+    return (torch.stack(out) if out else qkv.new_zeros(0, H * dv)), S
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("gate", [-40.0, -3.0, 3.0, 200.0])        # no decay, slow, fast, all at once
+@pytest.mark.parametrize("H,G,d,dv,lens", [(2, 1, 64, 16, [1, 0, 16]), (6, 6, 128, 48, [17, 15, 2]), (12, 2, 128, 16, [0, 33, 48]), (5, 1, 192, 32, [49, 31]),
+                                           (4, 4, 256, 16, [64, 5, 80, 1])])
+def test_chunks_against_float64(dtype, gate, H, G, d, dv, lens):
+    from pegainfer_amd import ops_blocks as B
+    gen = torch.Generator().manual_seed(H * d + len(lens))
+    n, T, dt = len(lens), sum(lens), DT[dtype]
+    slots = torch.randperm(n + 1, generator=gen)[:n]
+    mem = torch.randn(n + 1, H, d, dv, generator=gen)
+    A_log, bias = (torch.randn(H, generator=gen) * 0.3).to(dt), (torch.randn(H, generator=gen) * 0.3).to(dt)
+    S, st = mem.double(), mem.cuda()
+    for step in range(2):                                          # the second one through the token-by-token form
+        qkv = torch.randn(T, 2 * G * d + H * dv, generator=gen)
+        qkv[1:, G * d:2 * G * d] = 0.6 * qkv[:-1, G * d:2 * G * d] + 0.8 * qkv[1:, G * d:2 * G * d]
+        proj = torch.randn(T, 2 * H + 3, generator=gen).to(dt)
+        proj[:, H:2 * H] += gate
+        p64 = proj.double()
+        g = torch.exp(-A_log.double().exp() * torch.nn.functional.softplus(p64[:, H:2 * H] + bias.double()))
+        rg = B.Ragged(lens, slots=slots.tolist())
+        got = B.delta_rule(qkv.cuda(), proj.cuda(), 0, H, A_log.cuda(), bias.cuda(), st, H, G, d, dv, rg, chunked=step == 0)
+        at = 0
+        for e, (length, slot) in enumerate(zip(lens, slots.tolist())):
+            rows = slice(at, at + length)
+            ref, S[slot] = reference(qkv[rows].double(), g[rows], torch.sigmoid(p64[rows, :H]), S[slot], H, G, d, dv)
+            at += length
+            if length:      # sums of up to 256 fp32 products, 2^-24 each, through a triangle of up to 16 and some chunks: 1e-5 of the largest value
+                assert float((got[rows].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5, (step, e)
+            assert float((st[slot].double().cpu() - S[slot]).abs().max() / S[slot].abs().max()) < 1e-5, (step, e)
+    untouched = [i for i in range(n + 1) if i not in slots.tolist()]
+    assert torch.equal(st[untouched].cpu(), mem[untouched])
+
+
+def test_sizes_that_are_left_to_the_token_form():
+    from pegainfer_amd import ops_blocks as B
+    for d, dv in ((32, 16), (128, 24), (320, 16)):
+        qkv, z = torch.zeros(20, 2 * d + dv, device="cuda"), torch.zeros(1, device="cuda")
+        assert B.delta_rule(qkv, torch.zeros(20, 2, device="cuda"), 0, 1, z, z, torch.zeros(1, 1, d, dv, device="cuda"), 1, 1, d, dv, B.Ragged([20]),
+                            chunked=True) is None
