@@ -15,6 +15,7 @@
 //   latent_attn_kernel        any sizes: one workgroup per (token, head, key split), 256 keys per round, scores by one thread per
 //                             key, online softmax, value accumulation by one thread per latent dimension
 //   latent_attn_mfma_kernel   bf16 cache, tiles of up to 64 (token, head) rows of one request: a wave per 16 rows
+//   latent_attn_tile_kernel   the same tiles where the entry is whole blocks of 32 values of rank 256 or 512: eight waves share 64 rows and 64 keys
 //   latent_attn_few_kernel    tiles of a few rows of a bf16 cache, any tile of an fp32 one: four waves per 16 or 32 rows
 //   latent_attn_merge_kernel  combines the key splits of a row (log-sum-exp weights), fixed split order
 // A row's result depends on its own query, position and cache entries only.  With contiguous splits the split count is a
@@ -503,6 +504,228 @@ __global__ __launch_bounds__(256 * KH) void latent_attn_mfma_kernel(const float*
   }
 }
 
+// ------------------------------------------------------------------ prompts' form (bf16 cache, whole blocks of 32 values)
+// In the form above every wave reads all of a key tile twice from LDS for its sixteen rows, which is what it waits for: 92 KB per 16 rows and 32 keys.
+// Here eight waves share the work on 64 rows and 64 keys so that little is read twice: for the scores a wave takes 16 keys and 32 rows, whose queries
+// stay in its registers; the weights meet in LDS; for the values it takes an eighth of the latent dims for all 64 rows.  Key tiles come by
+// LDS-DMA into two buffers, asked for a whole tile ahead, an instruction per key and part (latent, rotated) with the entry's place in scalar registers; a
+// row's LDS stride of one 16-byte chunk more than its values keeps the reads off each other's banks.  Same products, roundings, masks and running maximum as above, one softmax state per row.
+// 16 heads of 512 + 64, longest tiles first on both sides: prompts of 901, 701, 501 and 301 tokens 152 -> 100 us, one of 1800 226 -> 140, of 700 99 -> 63;
+// 8 heads of 256 + 32 103 -> 65, 168 -> 104, 73 -> 49.  One prompt of 4096 tokens (512 + 64): matrix cores busy 20 % of the time, vector unit 24, LDS 31: the
+// three take turns within a tile, with two waves per SIMD in step; registers (the queries' 144 and the values' 64 of 256) leave no room for more.
+// Three barriers per tile: the tile has landed; the rows' maxima over each wave's keys; the weights and the rows' factors.
+template <int ND, int EB>
+struct LatentTileShape {              // rank 16 ND, entries of 32 EB values
+  static constexpr int kKeys = 64, kR = 16 * ND, kE = 32 * EB, kChunks = kE / 8 + 1, kRow = kChunks * 8, kPStride = kKeys + 8;
+  static constexpr size_t kLds = 2 * kKeys * kRow * 2 + kTileRows * kPStride * 2 + 6 * kTileRows * 4 + 2 * 64 * 16;
+};
+template <int ND, int EB>
+__global__ __launch_bounds__(512) void latent_attn_tile_kernel(const float* __restrict__ qc, float* __restrict__ o_lat,
+                                                               const uint16_t* __restrict__ cache, int64_t page_stride, int64_t layer_off, int page_size,
+                                                               const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req,
+                                                               const int32_t* __restrict__ page_indptr, const int32_t* __restrict__ page_ids,
+                                                               const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_rows, int H, int r,
+                                                               int dr, float scale, float* __restrict__ partial, int n_tokens, int max_splits, LatentCut cut) {
+  typedef short v4s_t __attribute__((ext_vector_type(4)));
+  typedef LatentTileShape<ND, EB> Sh;
+  constexpr int KEYS = Sh::kKeys, E = Sh::kE, S = Sh::kChunks, R = Sh::kR, ROW = Sh::kRow, DB = ND / 8, PS = Sh::kPStride;
+  extern __shared__ __align__(16) uint8_t lat_smem[];
+  uint16_t* Ck = reinterpret_cast<uint16_t*>(lat_smem);              // [2][KEYS][ROW]
+  uint16_t* P = Ck + 2 * KEYS * ROW;                                 // [64][PS] weights
+  float* s_max = reinterpret_cast<float*>(P + kTileRows * PS);       // [4][64] maxima over 16 keys each
+  float* s_corr = s_max + 4 * kTileRows;                             // [64]
+  int* s_pos = reinterpret_cast<int*>(s_corr + kTileRows);           // [64] the rows' positions, -1: no row
+  u32x4* s_q = reinterpret_cast<u32x4*>(s_pos + kTileRows);          // [2][64] the one block of the queries that finds no register
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l15 = lane & 15, g = lane >> 4;
+  const int kb = wave & 3, half = wave >> 2;
+  const int row0 = tile_row0[blockIdx.x], cnt = tile_rows[blockIdx.x], split = blockIdx.y;
+  const int t_first = row0 / H, t_last = (row0 + cnt - 1) / H, pmax = positions[t_last];
+  const int j_lo = split * cut.grain;
+  if (j_lo > pmax) return;
+  const int j_hi = cut.end_of(split, pmax + 1);
+  const int32_t* pages = page_ids + page_indptr[token_req[t_first]];
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  const uint32_t ring = (uint32_t)(uintptr_t)(lds_ptr_t)lat_smem;
+  // a wave fetches eight neighbouring keys, which lie on one page (page_size and the splits' grain are multiples of eight); keys past the end: the last
+  auto page_of = [&](int j0) { return pages[min(j0 + wave * 8, j_hi - 1) / page_size]; };
+  auto request = [&](int j0, int page, int buf) {
+    const int first = min(j0 + wave * 8, j_hi - 1);
+    const uint16_t* base = cache + (int64_t)page * page_stride + layer_off + (int64_t)(first % page_size) * E;
+    const int last = j_hi - 1 - first;
+    const uint32_t off = lane * 16;
+    auto part = [&](int at) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t dst = ring + ((buf * KEYS + wave * 8 + i) * S + at / 8) * 16;
+        const uint64_t src = reinterpret_cast<uint64_t>(base + min(i, last) * E + at);
+        // (readfirstlane is an int: unsigned before it is widened)
+        const uint64_t from = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(src >> 32)) << 32 |
+                              (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)src);
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(from), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+      }
+    };
+    if (R == 512 || lane < R / 8) part(0);
+    if (lane < (E - R) / 8) part(R);
+  };
+  request(j_lo, page_of(j_lo), 0);
+  int page = page_of(j_lo + KEYS);
+  // the rows go through the other buffer, as bf16, to the waves' registers: the scores' second operand
+  if (tid < kTileRows) s_pos[tid] = tid < cnt ? positions[(row0 + tid) / H] : -1;
+  {
+    constexpr int ALL = kTileRows * (E / 8), N = (ALL + 511) / 512;
+    u32x4 v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = min(i * 512 + tid, ALL - 1), row = c / (E / 8);
+      const float* src = qc + (int64_t)(row0 + min(row, cnt - 1)) * E + (c - row * (E / 8)) * 8;
+      const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
+      v[i] = u32x4{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = min(i * 512 + tid, ALL - 1), row = c / (E / 8);
+      *reinterpret_cast<u32x4*>(Ck + (KEYS + row) * ROW + (c - row * (E / 8)) * 8) = v[i];
+    }
+  }
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };      // (not the tile on its way)
+  barrier();
+  bf16x8_t q[2][EB];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int k = 0; k < EB; ++k)
+      q[rb][k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(Ck + (KEYS + half * 32 + rb * 16 + l15) * ROW + 32 * k + 8 * g));
+  if (kb == 0) s_q[half * 64 + lane] = __builtin_bit_cast(u32x4, q[1][EB - 1]);
+  // the lane's number; what follows from it is worked out where it is needed and not kept over the loop, where there is no register for it
+  auto here = [&] {
+    int n = lane;
+    asm volatile("" : "+v"(n));
+    return n;
+  };
+  f32x4 o[4][DB];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int d = 0; d < DB; ++d) o[b][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};            // l: of this lane's keys alone
+  int buf = 0;
+  for (int j0 = j_lo; j0 < j_hi; j0 += KEYS, buf ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (j0 + KEYS < j_hi) request(j0 + KEYS, page, buf ^ 1);
+    page = page_of(j0 + 2 * KEYS);
+    f32x4 s[2] = {};
+    {
+      const int ln = here();
+      const uint16_t* kp = Ck + (buf * KEYS + kb * 16 + (ln & 15)) * ROW + 8 * (ln >> 4);
+      constexpr int AHEAD = 2;                                       // reads on their way
+      u32x4 a[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) a[k] = *reinterpret_cast<const u32x4*>(kp + 32 * k);
+#pragma unroll
+      for (int k = 0; k < EB; ++k) {
+        const bf16x8_t now = __builtin_bit_cast(bf16x8_t, a[k % AHEAD]);
+        s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now, q[0][k], s[0], 0, 0, 0);
+        s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now, k < EB - 1 ? q[1][k] : __builtin_bit_cast(bf16x8_t, s_q[half * 64 + ln]), s[1], 0, 0, 0);
+        if (k + AHEAD < EB) a[k % AHEAD] = *reinterpret_cast<const u32x4*>(kp + 32 * (k + AHEAD));
+        __builtin_amdgcn_sched_barrier(0);                           // (and no more: there is no register for them)
+      }
+    }
+    float sc[2][4];
+    const int ln = here(), l15 = ln & 15, g = ln >> 4;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const int pq = s_pos[half * 32 + rb * 16 + l15];
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = j0 + kb * 16 + 4 * g + i;
+        sc[rb][i] = (j <= pq && j < j_hi) ? s[rb][i] * scale : -INFINITY;
+        mx = fmaxf(mx, sc[rb][i]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      if (g == 0) s_max[kb * kTileRows + half * 32 + rb * 16 + l15] = mx;
+    }
+    barrier();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const int row = half * 32 + rb * 16 + l15;
+      const float m_new = fmaxf(m[rb], fmaxf(fmaxf(s_max[row], s_max[kTileRows + row]), fmaxf(s_max[2 * kTileRows + row], s_max[3 * kTileRows + row])));
+      const float m_use = m_new == -INFINITY ? 0.f : m_new, corr = m_new == -INFINITY ? 1.f : __expf(m[rb] - m_use);
+      float ps[4], sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ps[i] = bf16_round_f(__expf(sc[rb][i] - m_use));             // the sum uses the weights as the matrix core sees them
+        sum += ps[i];
+      }
+      l[rb] = l[rb] * corr + sum;
+      m[rb] = m_new;
+      *reinterpret_cast<u32x2*>(P + row * PS + kb * 16 + 4 * g) = u32x2{pack_bf2(ps[0], ps[1]), pack_bf2(ps[2], ps[3])};
+      if (kb == 0 && g == 0) s_corr[row] = corr;
+    }
+    barrier();
+    {
+      float c[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) c[b] = s_corr[b * 16 + l15];
+      // the running maximum of most rows stops moving after the first tiles: rescale only when some row needs it
+      if (__any(c[0] != 1.0f || c[1] != 1.0f || c[2] != 1.0f || c[3] != 1.0f)) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int d = 0; d < DB; ++d) o[b][d] *= c[b];
+      }
+    }
+    const __attribute__((address_space(3))) uint16_t* ck3 = (const __attribute__((address_space(3))) uint16_t*)(Ck) +
+        (buf * KEYS + 4 * g + (l15 >> 2)) * ROW + 4 * (l15 & 3) + wave * DB * 16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8_t w[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const uint16_t* pp = P + (b * 16 + l15) * PS + 32 * h + 4 * g;
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(pp), hi = *reinterpret_cast<const u32x2*>(pp + 16);
+        w[b] = __builtin_bit_cast(bf16x8_t, u32x4{lo.x, lo.y, hi.x, hi.y});
+      }
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const v4s_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + 32 * h * ROW + d * 16));
+        const v4s_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_t __attribute__((address_space(3)))*)(ck3 + (32 * h + 16) * ROW + d * 16));
+        const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
+        const bf16x8_t cv = __builtin_bit_cast(bf16x8_t, u32x4{w0.x, w0.y, w1.x, w1.y});
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cv, w[b], o[b][d], 0, 0, 0);
+      }
+    }
+  }
+  barrier();
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const int row = half * 32 + rb * 16 + l15;
+    l[rb] += __shfl_xor(l[rb], 16, kWave);
+    l[rb] += __shfl_xor(l[rb], 32, kWave);
+    if (g == 0) s_max[kb * kTileRows + row] = l[rb];
+    if (kb == 0 && g == 0) s_corr[row] = m[rb];
+  }
+  barrier();
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int row = b * 16 + l15;
+    if (row >= cnt) continue;
+    const float sum = (s_max[row] + s_max[kTileRows + row]) + (s_max[2 * kTileRows + row] + s_max[3 * kTileRows + row]);
+    const int own_splits = cut.splits_of(positions[(row0 + row) / H] + 1, max_splits);
+    const int64_t grow = row0 + row;
+    if (own_splits == 1 ? split != 0 : split >= own_splits) continue;
+    const LatentPartial part(partial, (int64_t)n_tokens * H * max_splits, r, grow * max_splits + split);
+    float* dst = own_splits == 1 ? o_lat + grow * r : part.acc;
+    const float inv = own_splits == 1 ? 1.0f / sum : 1.0f;
+    if (own_splits > 1 && wave == 0 && g == 0) { part.max_sum[0] = s_corr[row]; part.max_sum[1] = sum; }
+#pragma unroll
+    for (int d = 0; d < DB; ++d) *reinterpret_cast<f32x4*>(dst + (wave * DB + d) * 16 + 4 * g) = o[b][d] * inv;
+  }
+}
+
 // ------------------------------------------------------------------ few-rows form (decoding, and every tile of an fp32 cache)
 // The form above gives each wave sixteen rows of its own: a decoded token's sixteen heads then keep one wave of four busy, alone on its
 // SIMD, with 2 x 18 dependent products for the scores and 64 transposed reads for the values of every key tile.  Here the four waves share
@@ -792,16 +1015,31 @@ struct LatentCall {
 
   // every instance may take what a compute unit has, asked for once
   template <typename K>
-  static bool all_lds(K kern) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) == hipSuccess;
+  static bool all_lds(K kern, size_t bytes = 159 * 1024) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
   }
   template <typename A, typename K>
   void run(K kern, int subs, size_t lds, int threads = 256) const {
     kern<<<dim3(n_tiles, sp, subs), threads, lds, s>>>(qc, o_lat, static_cast<const A*>(cache), page_stride, layer_off, page_size, positions, token_req,
                                            page_indptr, page_ids, tile_row0, tile_rows, H, r, dr, scale, ws, n_tokens, sp, cut);
   }
+  template <int ND, int EB>
+  void tile_form() const {
+    auto kern = &latent_attn_tile_kernel<ND, EB>;
+    static_assert(LatentTileShape<ND, EB>::kLds <= kCuLds, "a compute unit's LDS");
+    static const bool once = all_lds(kern, LatentTileShape<ND, EB>::kLds);
+    (void)once;
+    run<uint16_t>(kern, 1, LatentTileShape<ND, EB>::kLds, 512);
+  }
   template <int ND>
   void wide() const {
+    // whole blocks of 32 values, eight neighbouring keys on one page: the form that shares LDS reads (both sides measured: at the kernel)
+    if constexpr (ND >= 16) {
+      if (r == ND * 16 && !(cut.dealt && sp > 1) && page_size % 8 == 0 && cut.grain % 8 == 0) {
+        if (dr == 32) return tile_form<ND, ND / 2 + 1>();
+        if (dr == 64) return tile_form<ND, ND / 2 + 2>();
+      }
+    }
     // A second set of waves, on the other half of tiles of 64 keys, where one workgroup's rows and keys fill a compute unit's LDS anyhow and both halves'
     // keys fit (entries of 417 to 608 values): each SIMD has two chains to work on.  16 heads of 512 + 64, four prompts of up to 900 tokens 214 -> 156 us
     // (longest tiles first: 179).  Keys dealt in runs of 32 stay with one set.

@@ -638,8 +638,7 @@ struct Model {
     const size_t o_tok = 0, o_pos = o_tok + T, o_req = o_pos + T, o_ind = o_req + T, o_want = o_ind + (size_t)n + 1;
     size_t words = o_want + (size_t)std::max(1, W);
     for (size_t k = 0; k < head_vals.size(); ++k) {
-      size_t cnt = 0;
-      for (int i = 0; i < n; ++i) cnt += ((size_t)lens[i] * head_vals[k] + 63) / 64;
+      const size_t cnt = ptiles::flat_count(lens, n, head_vals[k], 64);
       tile_off[k] = words;
       tile_cnt[k] = cnt;
       words += 2 * cnt;
@@ -666,18 +665,8 @@ struct Model {
       }
       mh[o_ind + n] = (int32_t)pg;
       for (int i = 0; i < W; ++i) mh[o_want + i] = want[i];
-      for (size_t k = 0; k < head_vals.size(); ++k) {
-        const int Hk = head_vals[k];
-        size_t at = 0, tok0 = 0;
-        for (int i = 0; i < n; ++i) {
-          const int rows = lens[i] * Hk;
-          for (int r0 = 0; r0 < rows; r0 += 64, ++at) {
-            mh[tile_off[k] + at] = (int32_t)(tok0 * Hk) + r0;
-            mh[tile_off[k] + tile_cnt[k] + at] = std::min(64, rows - r0);
-          }
-          tok0 += (size_t)lens[i];
-        }
-      }
+      for (size_t k = 0; k < head_vals.size(); ++k)
+        ptiles::flat_cut(lens, n, head_vals[k], 64, tile_cnt[k], mh + tile_off[k], [&](int i) { return requests[ids[i]].seq_len; });
     }
     DZ_HIP(hipEventRecord(ev0, stream));
     DZ_HIP(io.send(words, captured, stream));

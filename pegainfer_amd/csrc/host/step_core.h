@@ -330,7 +330,7 @@ class StepModel {
       group_rows.push_back(rows);
       group_at.push_back(put_group_tiles(&mb, lens, n, gt.per, rows));
     }
-    for (int heads : flat_heads) flat_at.push_back(put_flat_tiles(&mb, lens, n, heads));
+    for (int heads : flat_heads) flat_at.push_back(put_flat_tiles(&mb, ids, lens, n, heads));
     size_t o_chunks[4] = {0, 0, 0, 0};
     if (scan_max > 0) put_chunks(&mb, ids, lens, n, &c.chunks, o_chunks);
     const size_t o_pages = mb.size();
@@ -681,26 +681,17 @@ class StepModel {
     return 0;
   }
 
-  static std::pair<size_t, int> put_columns(std::vector<int32_t>* mb, const std::vector<std::vector<int32_t>>& cols) {
-    const size_t at = mb->size();
-    for (auto& c : cols) mb->insert(mb->end(), c.begin(), c.end());
-    return {at, (int)cols[0].size()};
-  }
   static std::pair<size_t, int> put_group_tiles(std::vector<int32_t>* mb, const int32_t* lens, int n, int per, int rows) {
     const size_t at = mb->size(), tiles = ptiles::count(lens, n, per, rows);
     mb->resize(at + 4 * tiles);
     ptiles::cut(lens, n, per, rows, tiles, mb->data() + at);
     return {at, (int)tiles};
   }
-  static std::pair<size_t, int> put_flat_tiles(std::vector<int32_t>* mb, const int32_t* lens, int n, int heads) {
-    std::vector<std::vector<int32_t>> c(2);
-    int tok0 = 0;
-    for (int i = 0; i < n; tok0 += lens[i++])
-      for (int r = 0; r < lens[i] * heads; r += kFlatRows) {
-        c[0].push_back(tok0 * heads + r);
-        c[1].push_back(std::min(kFlatRows, lens[i] * heads - r));
-      }
-    return put_columns(mb, c);
+  std::pair<size_t, int> put_flat_tiles(std::vector<int32_t>* mb, const int32_t* ids, const int32_t* lens, int n, int heads) const {
+    const size_t at = mb->size(), tiles = ptiles::flat_count(lens, n, heads, kFlatRows);
+    mb->resize(at + 2 * tiles);
+    ptiles::flat_cut(lens, n, heads, kFlatRows, tiles, mb->data() + at, [&](int i) { return requests[ids[i]].seq_len; });
+    return {at, (int)tiles};
   }
   void put_chunks(std::vector<int32_t>* mb, const int32_t* ids, const int32_t* lens, int n, ChunkTable* t, size_t* off) const {
     const ptiles::Chunks c = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, scan_max);

@@ -179,7 +179,11 @@ def tables(tmp_path_factory):
     import subprocess
     d = tmp_path_factory.mktemp("tables")
     (d / "t.cpp").write_text('#include "row_tiles.h"\nextern "C" int wide_rows(const int32_t* lens, int n, int T, int per, int kv, int keys) '
-                             '{ return ptiles::wide_rows(lens, n, T, per, kv, keys); }\n')
+                             '{ return ptiles::wide_rows(lens, n, T, per, kv, keys); }\n'
+                             'extern "C" int flat(const int32_t* lens, const int32_t* begin, int n, int heads, int most, int32_t* table, int room) {\n'
+                             '  const size_t tiles = ptiles::flat_count(lens, n, heads, most);\n'
+                             '  if ((int)tiles <= room) ptiles::flat_cut(lens, n, heads, most, tiles, table, [&](int i) { return begin[i]; });\n'
+                             '  return (int)tiles; }\n')
     host = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc", "host")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-I", host, "-o", str(d / "t.so"), str(d / "t.cpp")], check=True)
     return ctypes.CDLL(str(d / "t.so"))
@@ -197,6 +201,22 @@ def test_wide_attention_tiles_leave_no_key_split_behind(tables, lens, heads, kv,
     (keys None: the choice may not depend on the contexts) take them only where nothing was dealt"""
     a = np.array(lens, np.int32)
     assert tables.wide_rows(ctypes.c_void_p(a.ctypes.data), len(lens), int(a.sum()), heads // max(kv, 1), kv, 2 ** 31 - 1 if keys is None else keys) == rows
+
+
+@pytest.mark.parametrize("lens,begin,heads", [([3], [0], 8), ([1, 1], [70, 5], 16), ([900, 0, 301, 64], [0, 9, 700, 0], 16), ([1] * 100, list(range(0, 6400, 64)), 3),
+                                              ([33, 1000], [5000, 0], 7)])
+def test_latent_attention_tiles_hold_every_row_once_the_longest_first(tables, lens, begin, heads):
+    a, b, t = np.array(lens, np.int32), np.array(begin, np.int32), np.full(20000, -1, np.int32)
+    n = tables.flat(*(ctypes.c_void_p(x.ctypes.data) for x in (a, b)), len(lens), heads, 64, ctypes.c_void_p(t.ctypes.data), 10000)
+    row0, rows = t[:n], t[n:2 * n]
+    entry, pos = np.repeat(np.arange(len(lens)), a), np.concatenate([np.arange(s, s + k) for s, k in zip(begin, lens)])
+    order = np.argsort(row0, kind="stable")
+    assert n and (rows > 0).all() and (rows <= 64).all() and (t[2 * n:] == -1).all()
+    assert (row0[order] + rows[order] == np.append(row0[order][1:], a.sum() * heads)).all() and row0.min() == 0
+    first, last = row0 // heads, (row0 + rows - 1) // heads
+    assert (entry[first] == entry[last]).all()
+    steps = pos[last] // 64
+    assert (np.diff(steps) <= 0).all() if n >= 64 else (order == np.arange(n)).all()
 
 
 def test_optional_scratch_is_given_up_when_there_is_no_memory(tmp_path):
