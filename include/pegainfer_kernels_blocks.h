@@ -309,6 +309,10 @@ pegainfer_status_t pegainfer_time_conv_step_biased(const void* in, int32_t in_dt
                                                    int64_t slot_stride, void* out, int32_t out_dtype, int64_t out_row_stride,
                                                    int32_t channels, int32_t taps, int32_t mode, const int32_t* entry_slot,
                                                    int32_t n_entries, pegainfer_stream_t stream);
+/* a decode step's convolution of embedding rows: x_out[e] = embed[token_ids[e]] in fp32 and its convolution (embed, w and out of one storage type) */
+pegainfer_status_t pegainfer_embed_conv_step(const void* embed, const uint32_t* token_ids, float* x_out, const void* w, float* state, int64_t slot_stride,
+                                             void* out, int32_t channels, int32_t taps, int32_t mode, const int32_t* entry_slot, int32_t n_entries,
+                                             int32_t dtype, pegainfer_stream_t stream);
 pegainfer_status_t pegainfer_time_conv_commit_biased(const void* in, int32_t in_dtype, int64_t in_row_stride, const void* in_bias,
                                                      int32_t bias_dtype, float* state, int64_t slot_stride, int32_t channels,
                                                      int32_t taps, const int32_t* entry_row0, const int32_t* entry_slot,
@@ -323,6 +327,9 @@ pegainfer_status_t pegainfer_group_rms_add(const float* x_in, const void* y, int
                                            float eps, float* x_out, void* xb_out, int32_t d, int32_t rows, int32_t dtype,
                                            const float* stack, int64_t stack_stride, const void* coef, int32_t n_mix,
                                            float* mix_out, void* mixb_out, pegainfer_stream_t stream);
+/* the norm alone, of fp32 rows x[row_index[i]] */
+pegainfer_status_t pegainfer_group_rms_rows(const float* x, const int32_t* row_index, const void* w, int32_t groups, float eps, void* out, int32_t d,
+                                            int32_t rows, int32_t dtype, pegainfer_stream_t stream);
 
 /* out[row, i] = g * sigmoid(alpha * g) * (u + 1),  g = min(gu[row, i], limit),  u = clamp(gu[row, I + i], -limit, limit) */
 pegainfer_status_t pegainfer_clamp_glu_rows(const void* gate_up, void* out, int32_t I, int32_t rows, float limit, float alpha,
@@ -901,6 +908,30 @@ typedef struct {
   int32_t n_rows, dtype;
 } pegainfer_qk_prep_desc;
 pegainfer_status_t pegainfer_qk_prep(const pegainfer_qk_prep_desc* p, pegainfer_stream_t stream);
+/* A decode step (every entry one row) of a layer with an attention beside the memory, in two launches around the attention's:
+ *   _beside   the memory's scan and the preparation of the attention's rows (_ok says whether: bf16 throughout, pairs of values);
+ *   _finish   what is left of both: n and the running maximum move on, o -> out[e, h vdim + c] = o / sqrt(mean(o^2) + eps) * norm_w[h vdim + c] *
+ *             act(gate) * factor (gate_kind 0 silu, 1 sigmoid), and scaled[e] = scale * rows[e] of scale_cols values (rows NULL: none). */
+typedef struct {
+  const void* norm_w;
+  const void* gate;
+  int64_t gate_stride;
+  int32_t gate_kind;
+  float factor, eps;
+  void* out;
+  int64_t out_stride;
+  const void* rows;
+  int64_t rows_stride;
+  void* scaled;
+  int64_t scaled_stride;
+  int32_t scale_cols;
+  float scale;
+} pegainfer_memory_finish_desc;
+int32_t pegainfer_gated_matrix_memory_beside_ok(const pegainfer_gated_matrix_memory_desc* d, const pegainfer_qk_prep_desc* p);
+pegainfer_status_t pegainfer_gated_matrix_memory_beside(const pegainfer_gated_matrix_memory_desc* d, const pegainfer_qk_prep_desc* p,
+                                                        pegainfer_stream_t stream);
+pegainfer_status_t pegainfer_gated_matrix_memory_finish(const pegainfer_gated_matrix_memory_desc* d, const pegainfer_memory_finish_desc* f,
+                                                        pegainfer_stream_t stream);
 /* Causal softmax attention, scores and weights in fp32:  out[row, h, :] = factor * sum_{j <= position} softmax_j(q . k_j * scale) v_j.
  * The rows are cut by the caller into tiles that stay inside one entry: tile i covers rows tile_row0[i] .. + tile_ntok[i] - 1
  * and, of each key/value group's query heads, tile_qh0[i] .. + tile_nqh[i] - 1, with ntok * nqh <= 16.  dim, vdim <= 256.

@@ -208,7 +208,7 @@ struct OprojArgs {
 };
 constexpr int kOprojMaxRows = 14;  // rows per wave quad (12 until round 5; 14 admits 20 KV chunks = 96 o_proj workgroups for hidden 2560)
 
-template <int GROUP, int NB>   // NB = requests of the step (1, or 2 since round 5)
+template <int GROUP, int NB>   // NB = requests of the step (1 or 2)
 __global__ __launch_bounds__(512) void attn_oproj_kernel(const DecodeAttnArgs a, const OprojArgs g) {
   constexpr int NW = 8;
   const int slot = (int)blockIdx.x % g.slots, kvh = (int)blockIdx.x / g.slots;   // the dim3(slots, kv_heads) order

@@ -156,7 +156,7 @@ struct Model {
        *gu_e = nullptr, *act_e = nullptr;
   int32_t *route_e = nullptr, *pos_pair = nullptr, *chosen_tiles = nullptr, *pos_row = nullptr, *tiles = nullptr;
   int max_tiles = 0;
-  float *xw = nullptr, *logits32 = nullptr;
+  float* logits32 = nullptr;
   void* hw = nullptr;
   Half* logits16 = nullptr;
   uint8_t* top1_state = nullptr;
@@ -725,7 +725,7 @@ struct Model {
     size_t c = 16;
     while (c < n) c *= 2;
     auto* wo = &want_owned;
-    if (dalloc(&xw, c * D, wo) || dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
+    if (dalloc_a(&hw, c * D, wo) || dalloc(&logits32, c * V, wo) ||
         dalloc(&logits16, c * V, wo) || dalloc(&top1_state, c * 16, wo))
       return -1;
     FZ_HIP(io.grow_tokens(c));
@@ -939,7 +939,7 @@ struct Model {
     auto run_layers = [&]() -> int {
     bool row_steps = single && !plain_kernels && pegainfer_row_step_ok(D, groups, canon_taps, 0, slot_stride);
     for (const LayerCfg& c : layers) row_steps = row_steps && c.st_canon % 4 == 0;
-    FZ_K(pegainfer_embed_f32(embed, d_tok, xs, D, Ti, dtype, S()));
+    if (!row_steps) FZ_K(pegainfer_embed_f32(embed, d_tok, xs, D, Ti, dtype, S()));     // otherwise with the first convolution
     if (!row_steps) FZ_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
     // decode steps: a sublayer's output, normed, joins the stream
     auto join_desc = [&](const float* from, const void* gain) {
@@ -955,6 +955,8 @@ struct Model {
       // input convolution: hb = x + conv(x), then the tail moves on
       if (row_steps && li > 0) {
         // the launch that closed the layer before has left hb
+      } else if (row_steps) {
+        FZ_K(pegainfer_embed_conv_step(embed, d_tok, xs, w.canon, state + c.st_canon, slot_stride, hb, D, canon_taps, 1, d_slot, n, dtype, S()));
       } else if (single) {
         FZ_K(pegainfer_time_conv_step(x_in, PEGAINFER_DTYPE_F32, D, w.canon, dtype, state + c.st_canon, slot_stride, hb, dtype, D, D,
                                       canon_taps, 1, d_slot, n, S()));
@@ -1000,9 +1002,26 @@ struct Model {
         const size_t ts = (size_t)c.tile_set;
         const int32_t* tb = md + tile_off[ts];
         const bool fast = tile_cta[ts] != 0, fast_decode = tile_cta[ts] < 0;
-        FZ_K(pegainfer_qk_norm_rope_paged(proj, Mp, c.o_q, c.o_k, c.o_v, a.heads, a.kv, a.dim, a.vdim, w.q_norm, w.k_norm, eps,
-                                          w.inv_freq, a.rot_dims, d_pos, d_ent, d_ind, d_pages, cache, page_stride, c.k_off, c.v_off,
-                                          kPageSize, q32, fast ? q16 : nullptr, Ti, dtype, S()));
+        pegainfer_qk_prep_desc qk{};
+        qk.proj = proj; qk.proj_dtype = qk.dtype = dtype; qk.proj_stride = Mp; qk.q_off = c.o_q; qk.k_off = c.o_k; qk.v_off = c.o_v;
+        qk.heads = a.heads; qk.kv_heads = a.kv; qk.dim = a.dim; qk.vdim = a.vdim; qk.q_norm = w.q_norm; qk.k_norm = w.k_norm;
+        qk.norm_kind = PEGAINFER_QKNORM_HEAD_WEIGHT; qk.eps = eps; qk.inv_freq = w.inv_freq; qk.rot_dims = a.rot_dims;
+        qk.rot_layout = PEGAINFER_ROT_PAIRS; qk.rot_amp = 1.0f; qk.positions = d_pos; qk.row_entry = d_ent; qk.page_indptr = d_ind; qk.page_ids = d_pages;
+        qk.cache = cache; qk.page_stride = page_stride; qk.k_cache_off = c.k_off; qk.v_cache_off = c.v_off; qk.page_size = kPageSize;
+        qk.q_out = q32; qk.q_out_stored = fast ? q16 : nullptr; qk.n_rows = Ti;
+        pegainfer_gated_matrix_memory_desc mm{};
+        mm.proj = proj; mm.proj_stride = Mp;
+        mm.q_off = c.o_rq; mm.k_off = c.o_rk; mm.v_off = c.o_rv; mm.i_off = c.o_ri; mm.f_off = c.o_rf;
+        mm.i_bias = w.i_bias; mm.f_bias = w.f_bias; mm.cap = r.cap; mm.state = state + c.st_mem; mm.slot_stride = slot_stride; mm.o = o32;
+        mm.heads = r.heads; mm.dim = r.dim; mm.vdim = r.vdim;
+        mm.entry_row0 = d_row0; mm.entry_slot = d_slot; mm.n_entries = n; mm.scan_max = kScanMax;
+        mm.chunk_row0 = md + chunk_off[0]; mm.chunk_rows = md + chunk_off[1]; mm.n_chunks = (int)chunks.row0.size();
+        mm.long_chunk0 = md + chunk_off[2]; mm.long_slot = md + chunk_off[3]; mm.n_long = (int)chunks.slot.size();
+        mm.workspace = chunk_ws.p; mm.dtype = dtype;
+        // decoding: the memory's scan beside the attention's preparation, what is left of both behind the attention
+        const bool beside = single && !plain_kernels && pegainfer_gated_matrix_memory_beside_ok(&mm, &qk);
+        if (beside) FZ_K(pegainfer_gated_matrix_memory_beside(&mm, &qk, S()));
+        else FZ_K(pegainfer_qk_prep(&qk, S()));
         if (fast_decode) {
           // decoding: one query row per request; long contexts are cut into chunks that run side by side (partials in bf16)
           const size_t sl = tile_cnt[ts];
@@ -1023,7 +1042,7 @@ struct Model {
                               : paged_attention_decode_cuda(q, out, kv, c.k_off, c.v_off, d_pages, d_ind, d_lpl, d_ent, zeros, d_kvlen, a.heads, a.kv, a.dim,
                                                             kPageSize, n, page_stride, a.scale, S());
           if (rc) return set_error("matrix-core decode attention failed");
-          FZ_K(pegainfer_scale_rows(attn16, (int64_t)a.heads * a.vdim, mix, c.mix_cols, a.heads * a.vdim, Ti, c.left_scale, dtype, S()));
+          if (!beside) FZ_K(pegainfer_scale_rows(attn16, (int64_t)a.heads * a.vdim, mix, c.mix_cols, a.heads * a.vdim, Ti, c.left_scale, dtype, S()));
         } else if (fast) {
           // every entry is a request whose last rows are this step's: the kernel takes a row's position from the request's
           // key count; scores and softmax state in fp32, weights rounded to bf16 where they enter the matrix cores
@@ -1039,18 +1058,17 @@ struct Model {
                                          a.kv, a.dim, a.vdim, a.scale, c.left_scale, tb, tb + tile_cnt[ts], tb + 2 * tile_cnt[ts],
                                          tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, c.mix_cols, dtype, S()));
         }
-        pegainfer_gated_matrix_memory_desc mm{};
-        mm.proj = proj; mm.proj_stride = Mp;
-        mm.q_off = c.o_rq; mm.k_off = c.o_rk; mm.v_off = c.o_rv; mm.i_off = c.o_ri; mm.f_off = c.o_rf;
-        mm.i_bias = w.i_bias; mm.f_bias = w.f_bias; mm.cap = r.cap; mm.state = state + c.st_mem; mm.slot_stride = slot_stride; mm.o = o32;
-        mm.heads = r.heads; mm.dim = r.dim; mm.vdim = r.vdim;
-        mm.entry_row0 = d_row0; mm.entry_slot = d_slot; mm.n_entries = n; mm.scan_max = kScanMax;
-        mm.chunk_row0 = md + chunk_off[0]; mm.chunk_rows = md + chunk_off[1]; mm.n_chunks = (int)chunks.row0.size();
-        mm.long_chunk0 = md + chunk_off[2]; mm.long_slot = md + chunk_off[3]; mm.n_long = (int)chunks.slot.size();
-        mm.workspace = chunk_ws.p; mm.dtype = dtype;
-        FZ_K(pegainfer_gated_matrix_memory_form(&mm, S()));
-        FZ_K(pegainfer_head_rms_gate(o32, w.rnorm, 1, at(proj, (size_t)c.o_rg), Mp, 1, c.right_scale, eps,
-                                     at(mix, (size_t)a.heads * a.vdim), c.mix_cols, r.heads, r.vdim, Ti, dtype, S()));
+        if (beside) {
+          pegainfer_memory_finish_desc fin{};
+          fin.norm_w = w.rnorm; fin.gate = at(proj, (size_t)c.o_rg); fin.gate_stride = Mp; fin.gate_kind = 1; fin.factor = c.right_scale; fin.eps = eps;
+          fin.out = at(mix, (size_t)a.heads * a.vdim); fin.out_stride = c.mix_cols;
+          if (fast_decode) { fin.rows = attn16; fin.rows_stride = fin.scale_cols = a.heads * a.vdim; fin.scaled = mix; fin.scaled_stride = c.mix_cols; fin.scale = c.left_scale; }
+          FZ_K(pegainfer_gated_matrix_memory_finish(&mm, &fin, S()));
+        } else {
+          FZ_K(pegainfer_gated_matrix_memory_form(&mm, S()));
+          FZ_K(pegainfer_head_rms_gate(o32, w.rnorm, 1, at(proj, (size_t)c.o_rg), Mp, 1, c.right_scale, eps,
+                                       at(mix, (size_t)a.heads * a.vdim), c.mix_cols, r.heads, r.vdim, Ti, dtype, S()));
+        }
       }
       if (linear(w.o, mix, y, D, Ti, c.mix_cols)) return -1;
       float* x_next = xs + (li + 1) * xs_stride;
@@ -1103,9 +1121,7 @@ struct Model {
     }
     // ---- wanted rows: final norm + logits over the embedding table
     if (W > 0) {
-      FZ_K(pegainfer_gather_rows_f32(x, d_want, xw, D, W, S()));
-      FZ_K(pegainfer_group_rms_add(nullptr, xw, PEGAINFER_DTYPE_F32, final_norm, groups, eps, nullptr, hw, D, W, dtype, nullptr, 0,
-                                   nullptr, 0, nullptr, nullptr, S()));
+      FZ_K(pegainfer_group_rms_rows(x, d_want, final_norm, groups, eps, hw, D, W, dtype, S()));
       void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
       if (linear(embed, hw, lg, V, W, D)) return -1;
       FZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr, S()));

@@ -19,6 +19,8 @@
 
 #include "common.h"
 #include "typed.h"
+#include "head_rms_core.h"
+#include "qk_prep_core.h"
 #include "recurrent_core.h"
 #include "scalar_chunks.h"
 #include "sigmoid_power.h"
@@ -304,8 +306,9 @@ __global__ __launch_bounds__(256) void memory_carry_kernel(const A* __restrict__
   if (tid == 0) *m_g = s_m[0];
 }
 
+// of 256 threads: columns bx of nbx runs of sixteen, head h, entry e
 template <int NS, typename A>
-__global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict__ proj, int64_t proj_stride, int64_t q_off,
+__device__ __forceinline__ void matrix_memory_block(int bx, int nbx, int h, int e, const A* __restrict__ proj, int64_t proj_stride, int64_t q_off,
                                                             int64_t k_off, int64_t v_off, int64_t i_off, int64_t f_off,
                                                             const A* __restrict__ i_bias, const A* __restrict__ f_bias,
                                                             float cap, float* __restrict__ state, int64_t slot_stride,
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict_
   __shared__ __attribute__((aligned(16))) float s_k[kRecTokens][DP], s_q[kRecTokens][DP];
   __shared__ float s_v[kRecTokens][kRecCols], s_i[kRecTokens], s_f[kRecTokens], s_m[kRecTokens + 1], s_a[kRecTokens],
       s_b[kRecTokens], s_em[kRecTokens];
-  const int e = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * kRecCols;
+  const int col0 = bx * kRecCols;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, cl = wave * 4 + (lane >> 4);
   const int col = col0 + cl;
   const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
@@ -385,9 +388,66 @@ __global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict_
   for (int i = 0; i < NS; ++i) {
     const int d = r * NS + i;
     if (d < dim && col < vdim) S_g[(int64_t)d * vdim + col] = S[i];
-    if (gridDim.x == 1 && tid < kRecSlices && d < dim) n_g[d] = n[i];
+    if (nbx == 1 && tid < kRecSlices && d < dim) n_g[d] = n[i];
   }
-  if (gridDim.x == 1 && tid == 0) *m_g = s_m[0];   // (several workgroups read both: memory_carry_kernel writes them afterwards)
+  if (nbx == 1 && tid == 0) *m_g = s_m[0];   // (several workgroups read both: memory_carry_kernel writes them afterwards)
+}
+template <int NS, typename A>
+__global__ __launch_bounds__(256) void matrix_memory_kernel(const A* __restrict__ proj, int64_t proj_stride, int64_t q_off,
+                                                            int64_t k_off, int64_t v_off, int64_t i_off, int64_t f_off,
+                                                            const A* __restrict__ i_bias, const A* __restrict__ f_bias,
+                                                            float cap, float* __restrict__ state, int64_t slot_stride,
+                                                            float* __restrict__ o, int H, int dim, int vdim,
+                                                            const int32_t* __restrict__ entry_row0,
+                                                            const int32_t* __restrict__ entry_slot, int scan_max) {
+  matrix_memory_block<NS, A>(blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, proj, proj_stride, q_off, k_off, v_off, i_off, f_off, i_bias, f_bias, cap, state,
+                             slot_stride, o, H, dim, vdim, entry_row0, entry_slot, scan_max);
+}
+
+// Decoding, a layer with an attention beside the memory: the scan and the preparation of the attention's rows, which write nothing that the other
+// reads, in one grid (the scan's workgroups first), and behind the attention one launch for all that is left: the memory's n and maximum, the
+// norm and gate of its read-out, the factor on the attention's rows.  One row, 16 heads over 4 of 256 beside 8 heads of 128 x 256:
+// 5.1 + 8.6 and 4.8 + 4.8 + 3.9 us in launches of their own, 9.4 and 4.5 here.
+template <int NS>
+__global__ __launch_bounds__(256) void memory_beside_kernel(pegainfer_gated_matrix_memory_desc m, int nbx, int n_scan, pegainfer_qk_prep_desc p, PrepForm pf,
+                                                            int per_row) {
+  extern __shared__ float sm[];
+  const int b = blockIdx.x;
+  if (b < n_scan) {
+    matrix_memory_block<NS, uint16_t>(b % nbx, nbx, b / nbx % m.heads, b / (nbx * m.heads), static_cast<const uint16_t*>(m.proj), m.proj_stride, m.q_off,
+                                      m.k_off, m.v_off, m.i_off, m.f_off, static_cast<const uint16_t*>(m.i_bias),
+                                      static_cast<const uint16_t*>(m.f_bias), m.cap, m.state, m.slot_stride, m.o, m.heads, m.dim, m.vdim, m.entry_row0,
+                                      m.entry_slot, 0);
+    return;
+  }
+  qk_prep_block<uint16_t, uint16_t, 2>(sm, (b - n_scan) / per_row, (b - n_scan) % per_row, per_row, p, pf);
+}
+
+// grid (heads + workgroups for the rows to scale, entries).  A head's workgroup: the first wave norms, the others move n on.
+template <typename A, int V>
+__global__ __launch_bounds__(256) void memory_finish_kernel(pegainfer_gated_matrix_memory_desc m, pegainfer_memory_finish_desc f) {
+  const int e = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, row = m.entry_row0[e];
+  if (h >= m.heads) {
+    const A* in = static_cast<const A*>(f.rows) + (int64_t)row * f.rows_stride;
+    A* out = static_cast<A*>(f.scaled) + (int64_t)row * f.scaled_stride;
+    for (int i = (h - m.heads) * 256 + tid; i < f.scale_cols; i += (gridDim.x - m.heads) * 256) st(out + i, ld(in + i) * f.scale);
+    return;
+  }
+  if (tid < kWave) {
+    head_rms_gate_wave<A, V>(row, h, m.o, static_cast<const A*>(f.norm_w), 1, static_cast<const A*>(f.gate), f.gate_stride, f.gate_kind, f.factor, f.eps,
+                             static_cast<A*>(f.out), f.out_stride, m.heads, m.vdim, 0);
+    return;
+  }
+  if (m.vdim <= kRecCols) return;                  // one workgroup per head has scanned: it has moved them on itself
+  const A* proj = static_cast<const A*>(m.proj);
+  float* base = m.state + (int64_t)m.entry_slot[e] * m.slot_stride + (int64_t)m.heads * m.dim * m.vdim;
+  float *n_g = base + (int64_t)h * m.dim, *m_g = base + (int64_t)m.heads * m.dim + h;
+  const MemoryGates<A> gate{proj, m.proj_stride, m.i_off, m.f_off, ld(static_cast<const A*>(m.i_bias) + h), ld(static_cast<const A*>(m.f_bias) + h), m.cap, h};
+  const float gi = gate.in(row), gf = gate.forget(row), mp = *m_g, mn = fmaxf(gf + mp, gi), a = expf(gf + mp - mn), b = expf(gi - mn);
+  for (int d = tid - kWave; d < m.dim; d += 256 - kWave)
+    n_g[d] = fmaf(b, ld(proj + (int64_t)row * m.proj_stride + m.k_off + (int64_t)h * m.dim + d), a * n_g[d]);
+  __syncthreads();                                 // the three waves that are left have read the maximum
+  if (tid == kWave) *m_g = mn;
 }
 
 // ---- the matrix memory over long portions (scalar_chunks.h): with the running maxima known, the decays exp(f + m - m') and the factors
@@ -557,6 +617,41 @@ pegainfer_status_t pegainfer_gated_matrix_memory_form(const pegainfer_gated_matr
                         q->n_long, st);
   });
   return known && ok ? (pegainfer_status_t)hipGetLastError() : PK_BAD;
+}
+
+int32_t pegainfer_gated_matrix_memory_beside_ok(const pegainfer_gated_matrix_memory_desc* q, const pegainfer_qk_prep_desc* p) {
+  return q && p && q->n_entries > 0 && q->n_entries <= 65535 && q->heads > 0 && q->dim > 0 && q->dim <= 256 && q->vdim > 0 && q->vdim <= 512 && q->cap > 0.f &&
+         q->n_long == 0 && q->dtype == kDtBf16 && p->dtype == kDtBf16 && p->proj_dtype == kDtBf16 && p->n_rows > 0 && qk_prep_ok(p) && qk_prep_pairs(p) &&
+         (int64_t)ceil_div(q->vdim, kRecCols) * q->heads * q->n_entries < (1 << 22);
+}
+
+pegainfer_status_t pegainfer_gated_matrix_memory_beside(const pegainfer_gated_matrix_memory_desc* q, const pegainfer_qk_prep_desc* p,
+                                                        pegainfer_stream_t stream) {
+  if (!pegainfer_gated_matrix_memory_beside_ok(q, p)) return PK_BAD;
+  const int nbx = ceil_div(q->vdim, kRecCols), n_scan = nbx * q->heads * q->n_entries, per_row = qk_prep_per_row(*p);
+  by_slices(q->dim, [&](auto ns) {
+    memory_beside_kernel<decltype(ns)::value><<<n_scan + p->n_rows * per_row, 256, qk_prep_lds(*p), as_stream(stream)>>>(*q, nbx, n_scan, *p, qk_prep_form(*p),
+                                                                                                                        per_row);
+  });
+  return (pegainfer_status_t)hipGetLastError();
+}
+
+pegainfer_status_t pegainfer_gated_matrix_memory_finish(const pegainfer_gated_matrix_memory_desc* q, const pegainfer_memory_finish_desc* f,
+                                                        pegainfer_stream_t stream) {
+  if (!q || !f || q->n_entries <= 0 || q->n_entries > 65535 || q->heads <= 0 || q->dim <= 0 || q->vdim <= 0 || q->vdim > 512 || !f->norm_w || !f->gate || !f->out ||
+      (f->rows && !f->scaled))
+    return PK_BAD;
+  const int scale = f->rows && f->scale_cols > 0 ? std::min(64, ceil_div(f->scale_cols, 256)) : 0;
+  if (!by_dtype(q->dtype, [&](auto* t) {
+        using A = std::remove_pointer_t<decltype(t)>;
+        auto go = [&](auto kern) { kern<<<dim3(q->heads + scale, q->n_entries), 256, 0, as_stream(stream)>>>(*q, *f); };
+        const int v = head_rms_values(q->o, f->norm_w, f->gate, f->gate_stride, f->out, f->out_stride, q->vdim);
+        if (v == 4) go(memory_finish_kernel<A, 4>);
+        else if (v == 2) go(memory_finish_kernel<A, 2>);
+        else go(memory_finish_kernel<A, 1>);
+      }))
+    return PK_BAD;
+  return (pegainfer_status_t)hipGetLastError();
 }
 
 pegainfer_status_t pegainfer_gated_matrix_memory(const void* proj, int64_t proj_stride, int64_t q_off, int64_t k_off,

@@ -21,6 +21,7 @@
 //   softcap_rows_kernel     cap * tanh(x / cap) on fp32 rows
 #include <algorithm>
 
+#include "head_rms_core.h"
 #include "route_core.h"
 
 namespace pk {
@@ -130,6 +131,9 @@ struct ConvStep {
   int C, K, mode;
   const int32_t* entry_slot;
   const W *in_bias, *out_bias;
+  const uint32_t* tokens = nullptr;   // TABLE: the inputs are these rows of a table, copied to `copy` on the way
+  float* copy = nullptr;
+  template <bool TABLE = false>
   __device__ __forceinline__ void at(int e, int c) const {
     constexpr int kAhead = 7;
     float* tail = state + (int64_t)entry_slot[e] * slot_stride;
@@ -138,7 +142,9 @@ struct ConvStep {
 #pragma unroll
     for (int j = 0; j < kAhead; ++j)
       if (j < K - 1) { past[j] = tail[(int64_t)j * C + c]; wt[j] = ld(wc + j); }
-    const float cur = ld(in + (int64_t)e * in_stride + c) + (in_bias ? ld(in_bias + c) : 0.f), w_cur = ld(wc + K - 1);
+    const float x = ld(in + (int64_t)(TABLE ? tokens[e] : (uint32_t)e) * in_stride + c);
+    const float cur = x + (in_bias ? ld(in_bias + c) : 0.f), w_cur = ld(wc + K - 1);
+    if constexpr (TABLE) copy[(int64_t)e * C + c] = x;
     float acc = 0.f;
 #pragma unroll
     for (int j = 0; j < kAhead; ++j)
@@ -159,10 +165,10 @@ struct ConvStep {
     st(out + (int64_t)e * out_stride + c, acc);
   }
 };
-template <typename I, typename W, typename O>
+template <bool TABLE, typename I, typename W, typename O>
 __global__ __launch_bounds__(256) void time_conv_step_kernel(ConvStep<I, W, O> q) {
   const int c = blockIdx.y * 256 + threadIdx.x;
-  if (c < q.C) q.at(blockIdx.x, c);
+  if (c < q.C) q.template at<TABLE>(blockIdx.x, c);
 }
 
 template <typename I, typename W>
@@ -191,13 +197,13 @@ __global__ __launch_bounds__(256) void group_rms_add_kernel(const float* x_in, c
                                                             const A* __restrict__ w, int groups, float eps, float* x_out,
                                                             A* __restrict__ xb_out, int d, const float* __restrict__ stack,
                                                             int64_t stack_stride, const A* __restrict__ coef, int n_mix,
-                                                            float* mix_out, A* __restrict__ mixb_out) {
+                                                            float* mix_out, A* __restrict__ mixb_out, const int32_t* __restrict__ y_row_index) {
   extern __shared__ float sm[];   // [groups] inverse root mean squares, then [n_mix] coefficients
   float* inv = sm;
   float* cf = sm + groups;
   const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int gs = d / groups;
-  const Y* yr = y + (int64_t)row * d;
+  const Y* yr = y + (int64_t)(y_row_index ? y_row_index[row] : row) * d;
   for (int j = threadIdx.x; j < n_mix; j += 256) cf[j] = ld(coef + j);
   for (int g = wave; g < groups; g += 4) {
     float ss = 0.f;
@@ -325,54 +331,15 @@ __global__ __launch_bounds__(256) void wide_rms_gate_kernel(const float* __restr
   }
 }
 
-// One wave per (row, head), vdim <= 512; a lane's values, gates and weights are all requested before the first is used, V at a time.  Bound by
-// memory with many heads, by the launch with few: 8192 x 4 heads of 128 16.5 -> 12.6 us, one row of four groups of 512 9.7 -> 4.6 us (read
-// value by value and a second time for the output before).
 template <typename A, int V>
 __global__ __launch_bounds__(256) void head_rms_gate_kernel(const float* __restrict__ o, const A* __restrict__ w, int w_per_head,
                                                             const A* __restrict__ gate, int64_t gate_stride, int gate_kind,
                                                             float factor, float eps, A* __restrict__ out, int64_t out_stride,
                                                             int heads, int vdim, int rows, int gate_first) {
-  constexpr int K = 8 / V;
   const int64_t rh = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (rh >= (int64_t)rows * heads) return;
-  const int row = (int)(rh / heads), h = (int)(rh % heads);
-  const float* p = o + ((int64_t)row * heads + h) * vdim;
-  const A* gr = gate + (int64_t)row * gate_stride + (int64_t)h * vdim;
-  const A* wr = w + (w_per_head ? (int64_t)h * vdim : 0);
-  A* dst = out + (int64_t)row * out_stride + (int64_t)h * vdim;
-  auto load = [&](const auto* q, float* t) {
-    if constexpr (V == 4) ld4(q, t); else if constexpr (V == 2) ld2(q, t); else t[0] = ld(q);
-  };
-  float v[K][V], z[K][V], wv[K][V];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = (lane + 64 * k) * V;
-    if (i < vdim) { load(p + i, v[k]); load(gr + i, z[k]); load(wr + i, wv[k]); }
-  }
-  float ss = 0.f;
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if ((lane + 64 * k) * V < vdim)
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        z[k][u] = gate_kind == 0 ? silu_f(z[k][u]) : sigmoid_f(z[k][u]);
-        if (gate_first) v[k][u] *= z[k][u];   // gate_first: the gated values are what is normed
-        ss = fmaf(v[k][u], v[k][u], ss);
-      }
-  ss = wave_sum(ss);
-  const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = (lane + 64 * k) * V;
-    if (i >= vdim) continue;
-    float r[V];
-    // (each order keeps its own sequence of roundings: norm, weight, gate, factor - or gate, norm, weight, factor)
-#pragma unroll
-    for (int u = 0; u < V; ++u) r[u] = gate_first ? v[k][u] * inv * wv[k][u] * factor : v[k][u] * inv * wv[k][u] * z[k][u] * factor;
-    if constexpr (V == 4) st4(dst + i, r); else if constexpr (V == 2) st2(dst + i, r); else st(dst + i, r[0]);
-  }
+  if (rh < (int64_t)rows * heads)
+    head_rms_gate_wave<A, V>((int)(rh / heads), (int)(rh % heads), o, w, w_per_head, gate, gate_stride, gate_kind, factor, eps, out, out_stride, heads, vdim,
+                             gate_first);
 }
 
 // Residual sum with a constant factor, then an RMS norm whose gain is ONE number:
@@ -1117,7 +1084,7 @@ pegainfer_status_t pegainfer_time_conv_step_biased(const void* in, int32_t in_dt
            using W = std::remove_pointer_t<decltype(tw)>;
            ok = by_dtype(out_dtype, [&](auto* to) {
                   using O = std::remove_pointer_t<decltype(to)>;
-                  time_conv_step_kernel<<<grid, 256, 0, as_stream(stream)>>>(ConvStep<I, W, O>{
+                  time_conv_step_kernel<false><<<grid, 256, 0, as_stream(stream)>>>(ConvStep<I, W, O>{
                       static_cast<const I*>(in), in_row_stride, static_cast<const W*>(w), state, slot_stride,
                       static_cast<O*>(out), out_row_stride, channels, taps, mode, entry_slot, static_cast<const W*>(in_bias),
                       static_cast<const W*>(out_bias)});
@@ -1125,6 +1092,21 @@ pegainfer_status_t pegainfer_time_conv_step_biased(const void* in, int32_t in_dt
          }) && ok;
   });
   return known && ok ? (pegainfer_status_t)hipGetLastError() : PK_BAD;
+}
+
+pegainfer_status_t pegainfer_embed_conv_step(const void* embed, const uint32_t* token_ids, float* x_out, const void* w, float* state, int64_t slot_stride,
+                                             void* out, int32_t channels, int32_t taps, int32_t mode, const int32_t* entry_slot, int32_t n_entries,
+                                             int32_t dtype, pegainfer_stream_t stream) {
+  if (n_entries <= 0) return 0;
+  if (channels <= 0 || taps < 1 || !token_ids || !x_out) return PK_BAD;
+  if (!by_dtype(dtype, [&](auto* t) {
+        using A = std::remove_pointer_t<decltype(t)>;
+        time_conv_step_kernel<true><<<dim3(n_entries, ceil_div(channels, 256)), 256, 0, as_stream(stream)>>>(
+            ConvStep<A, A, A>{static_cast<const A*>(embed), channels, static_cast<const A*>(w), state, slot_stride, static_cast<A*>(out), channels, channels,
+                              taps, mode, entry_slot, nullptr, nullptr, token_ids, x_out});
+      }))
+    return PK_BAD;
+  return (pegainfer_status_t)hipGetLastError();
 }
 
 pegainfer_status_t pegainfer_time_conv_commit(const void* in, int32_t in_dtype, int64_t in_row_stride, float* state,
@@ -1153,7 +1135,7 @@ pegainfer_status_t pegainfer_time_conv_commit_biased(const void* in, int32_t in_
   return known && ok ? (pegainfer_status_t)hipGetLastError() : PK_BAD;
 }
 
-pegainfer_status_t pegainfer_group_rms_add(const float* x_in, const void* y, int32_t y_dtype, const void* w, int32_t groups,
+static pegainfer_status_t group_rms_add(const int32_t* y_row_index, const float* x_in, const void* y, int32_t y_dtype, const void* w, int32_t groups,
                                            float eps, float* x_out, void* xb_out, int32_t d, int32_t rows, int32_t dtype,
                                            const float* stack, int64_t stack_stride, const void* coef, int32_t n_mix,
                                            float* mix_out, void* mixb_out, pegainfer_stream_t stream) {
@@ -1171,14 +1153,26 @@ pegainfer_status_t pegainfer_group_rms_add(const float* x_in, const void* y, int
       if (vec)
         group_rms_add_kernel<Y, A, true><<<rows, 256, smem, as_stream(stream)>>>(
             x_in, static_cast<const Y*>(y), static_cast<const A*>(w), groups, eps, x_out, static_cast<A*>(xb_out), d, stack,
-            stack_stride, static_cast<const A*>(coef), n_mix, mix_out, static_cast<A*>(mixb_out));
+            stack_stride, static_cast<const A*>(coef), n_mix, mix_out, static_cast<A*>(mixb_out), y_row_index);
       else
         group_rms_add_kernel<Y, A, false><<<rows, 256, smem, as_stream(stream)>>>(
             x_in, static_cast<const Y*>(y), static_cast<const A*>(w), groups, eps, x_out, static_cast<A*>(xb_out), d, stack,
-            stack_stride, static_cast<const A*>(coef), n_mix, mix_out, static_cast<A*>(mixb_out));
+            stack_stride, static_cast<const A*>(coef), n_mix, mix_out, static_cast<A*>(mixb_out), y_row_index);
     });
   });
   return known && ok ? (pegainfer_status_t)hipGetLastError() : PK_BAD;
+}
+
+pegainfer_status_t pegainfer_group_rms_add(const float* x_in, const void* y, int32_t y_dtype, const void* w, int32_t groups,
+                                           float eps, float* x_out, void* xb_out, int32_t d, int32_t rows, int32_t dtype,
+                                           const float* stack, int64_t stack_stride, const void* coef, int32_t n_mix,
+                                           float* mix_out, void* mixb_out, pegainfer_stream_t stream) {
+  return group_rms_add(nullptr, x_in, y, y_dtype, w, groups, eps, x_out, xb_out, d, rows, dtype, stack, stack_stride, coef, n_mix, mix_out, mixb_out, stream);
+}
+
+pegainfer_status_t pegainfer_group_rms_rows(const float* x, const int32_t* row_index, const void* w, int32_t groups, float eps, void* out, int32_t d,
+                                            int32_t rows, int32_t dtype, pegainfer_stream_t stream) {
+  return group_rms_add(row_index, nullptr, x, kDtF32, w, groups, eps, nullptr, out, d, rows, dtype, nullptr, 0, nullptr, 0, nullptr, nullptr, stream);
 }
 
 pegainfer_status_t pegainfer_clamp_glu_rows(const void* gate_up, void* out, int32_t I, int32_t rows, float limit, float alpha,
@@ -1223,15 +1217,13 @@ pegainfer_status_t pegainfer_head_gate_rms(const float* o, const void* w, int32_
           else wide(wide_rms_gate_kernel<A, false>);
           return;
         }
-        // as many values per access as rows, strides and pointers allow, without leaving lanes of a narrow head idle
-        const bool aligned = gate_stride % 4 == 0 && out_stride % 4 == 0 && host_aligned16(o) && host_aligned16(w) && host_aligned16(gate) &&
-                             host_aligned16(out);
         auto narrow = [&](auto kern) {
           kern<<<blocks, 256, 0, as_stream(stream)>>>(o, static_cast<const A*>(w), w_per_head, static_cast<const A*>(gate), gate_stride,
                                                       gate_kind, factor, eps, static_cast<A*>(out), out_stride, heads, vdim, rows, gate_first);
         };
-        if (aligned && vdim % 4 == 0 && vdim > 128) narrow(head_rms_gate_kernel<A, 4>);
-        else if (aligned && vdim % 4 == 0 && vdim > 64) narrow(head_rms_gate_kernel<A, 2>);
+        const int v = head_rms_values(o, w, gate, gate_stride, out, out_stride, vdim);
+        if (v == 4) narrow(head_rms_gate_kernel<A, 4>);
+        else if (v == 2) narrow(head_rms_gate_kernel<A, 2>);
         else narrow(head_rms_gate_kernel<A, 1>);
       }))
     return PK_BAD;

@@ -594,6 +594,9 @@ MatrixMemoryDesc = _struct("MatrixMemoryDesc", [("p", "proj"), ("l", "proj_strid
                                                 ("p", "state"), ("l", "slot_stride"), ("p", "o"), ("i", "heads dim vdim"),
                                                 ("p", "entry_row0 entry_slot"), ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"),
                                                 ("i", "n_chunks"), ("p", "long_chunk0 long_slot"), ("i", "n_long"), ("p", "workspace"), ("i", "dtype")])
+MemoryFinishDesc = _struct("MemoryFinishDesc", [("p", "norm_w gate"), ("l", "gate_stride"), ("i", "gate_kind"), ("f", "factor eps"), ("p", "out"),
+                                                ("l", "out_stride"), ("p", "rows"), ("l", "rows_stride"), ("p", "scaled"), ("l", "scaled_stride"),
+                                                ("i", "scale_cols"), ("f", "scale")])
 SsdScanDesc = _struct("SsdScanDesc", [("p", "xbc"), ("l", "xbc_stride"), ("p", "proj"), ("l", "proj_stride dt_off"), ("p", "A_log dt_bias D state"),
                                       ("l", "slot_stride"), ("p", "o"), ("i", "heads groups n_state vdim"), ("p", "entry_row0 entry_slot"),
                                       ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"), ("i", "n_chunks"), ("p", "long_chunk0 long_slot"),
