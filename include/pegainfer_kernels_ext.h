@@ -40,6 +40,10 @@ pegainfer_status_t pegainfer_sample(const Half* logits, void* scratch, uint8_t* 
  * take (K % 8, misaligned, ...) so the caller can fall back to the unfused sequence. */
 pegainfer_status_t pegainfer_gemv_fused(const Half* W, const Half* X, Half* Y, int32_t M, int32_t T, int32_t K, const Half* residual, const Half* norm_weight, Half* hidden_out, float eps, int32_t silu_intermediate, pegainfer_stream_t stream);
 
+/* Y[T, I] = clamped gated unit of W X, W = [gate (I rows); up (I rows)]: both rounded to bf16, g = min(gate, limit), u = clamp(up, -limit, limit),
+ * g sigmoid(alpha g) (u + 1).  One or two rows (_ok); the bits of gemm_cuda and pegainfer_clamp_glu_rows. */
+int32_t pegainfer_gemv_clamp_glu_ok(const Half* W, const Half* X, int32_t T, int32_t K);
+pegainfer_status_t pegainfer_gemv_clamp_glu(const Half* W, const Half* X, Half* Y, int32_t I, int32_t T, int32_t K, float limit, float alpha, pegainfer_stream_t stream);
 /* pegainfer_gemv_fused with other rounding points (bits 0 and 2: T <= 4; bit 1 alone: T <= 16): flags bit 0 = the norm weight is (1 + w)
  * (rms_norm_batched_offset_cuda), bit 1 = hidden_out = bf16(X + residual) and the norm runs over that ROUNDED sum
  * (add_cuda then rms_norm_batched_offset_cuda, batch_decode.rs:246-262) instead of FlashInfer's fused add+norm,

@@ -29,7 +29,7 @@ inline int gemv_pick_kt(int NT, int K) {
   return kt < 2048 ? 2048 : kt;
 }
 
-enum { kEpiStore = 0, kEpiSilu = 1 };
+enum { kEpiStore = 0, kEpiSilu = 1, kEpiClamp = 2 };   // kEpiClamp: kEpiSilu's pairs through g = min(gate, L), u = clamp(up, -L, L): g sigmoid(alpha g) (u + 1)
 
 template <int NT>
 __host__ __device__ inline int gemv_xs_bytes(int K, int KT) {
@@ -38,7 +38,7 @@ __host__ __device__ inline int gemv_xs_bytes(int K, int KT) {
 }
 template <int NT, int RPW, int KSPLIT, int EPI>
 inline int gemv_lds_bytes(int K, int KT, bool residual) {
-  constexpr int NW = EPI == kEpiSilu ? 2 : 1;
+  constexpr int NW = EPI != kEpiStore ? 2 : 1;
   // x tile (+ the raw residual rows of the early prologue) + K-split partials + 16 floats: inv_rms per token
   return gemv_xs_bytes<NT>(K, KT) * (residual && NT <= 2 ? 2 : 1) + ((KSPLIT == 1 ? 0 : 4 * NW * RPW * NT) + 16) * 4;
 }
@@ -56,6 +56,7 @@ struct GemvFusedArgs {
   int rpb;                // skinny kernels: W rows per row block (0 = 16); set by the launcher (skinny_pick_rpb)
   int variant;            // skinny resident kernel (launcher: skinny_flush_mode): bit 0 one-barrier flush, bit 2 ticket flush with
                           // the ring size in bits 4..7, bit 1 timing probe
+  float limit, alpha;     // kEpiClamp
 };
 // process-wide debug hook, defined in linear.hip; copied into the launch arguments by gemv_launch_one
 extern unsigned long long* g_gemv_trace;
@@ -80,7 +81,7 @@ constexpr int kGemvNormAllWaves = 32;   // launcher-only bit (PEGAINFER_GEMV_NOR
 template <int NT, int RPW, int KSPLIT, int EPI, int U = 4>
 __global__ __launch_bounds__(256) void gemv_fused_kernel(const GemvFusedArgs a) {
   const int KT = a.KT;
-  constexpr int NW = EPI == kEpiSilu ? 2 : 1;  // weight row sets streamed together
+  constexpr int NW = EPI != kEpiStore ? 2 : 1;  // weight row sets streamed together
   constexpr int ROWS_PER_GROUP = (KSPLIT == 1 ? 4 : 1) * RPW;
   // all LDS is dynamic and sized to the shape (guide G17: one 16-byte aligned carve, no statics): a K = 2560
   // GEMV needs 5 KB, not the 32 KB tile capacity, which is what lets 5+ workgroups share a CU.
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(const GemvFusedArgs a) 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int K = a.K, T = a.T;
   const int pitch = (K < KT ? K : KT) >> 3;  // 16-byte vectors per token row of the x tile
-  const int rows_total = EPI == kEpiSilu ? a.I : a.M;
+  const int rows_total = EPI != kEpiStore ? a.I : a.M;
   const int ngroups = (rows_total + ROWS_PER_GROUP - 1) / ROWS_PER_GROUP;
 
   // Persistent over row groups: the launcher sizes the grid to what is co-resident (gridDim <= ngroups) and a
@@ -361,6 +362,9 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(const GemvFusedArgs a) 
         const float gt = bf16_round_f(v0), up = bf16_round_f(v1);  // the GEMM output is bf16 before SwiGLU
         const float sg = (a.flags & kGemvSiluRound) ? bf16_round_f(silu_f(gt)) : silu_f(gt);
         a.Y[(size_t)t * a.I + row] = f2bf(sg * up);
+      } else if (EPI == kEpiClamp) {
+        const float g = fminf(bf16_round_f(v0), a.limit), u = fminf(fmaxf(bf16_round_f(v1), -a.limit), a.limit);
+        a.Y[(size_t)t * a.I + row] = f2bf(g * (1.0f / (1.0f + expf(-(a.alpha * g)))) * (u + 1.0f));
       } else {
         a.Y[(size_t)t * a.M + row] = f2bf(v0);
       }
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(const GemvFusedArgs a) 
 template <int NT, int RPW, int KSPLIT, int EPI, int U = 4>
 inline void gemv_launch_one(const GemvFusedArgs& a, hipStream_t s) {
   constexpr int ROWS_PER_GROUP = (KSPLIT == 1 ? 4 : 1) * RPW;
-  const int rows = EPI == kEpiSilu ? a.I : a.M;
+  const int rows = EPI != kEpiStore ? a.I : a.M;
   const int ngroups = ceil_div(rows, ROWS_PER_GROUP);
   const int lds = gemv_lds_bytes<NT, RPW, KSPLIT, EPI>(a.K, a.KT, a.residual != nullptr);
   auto kern = &gemv_fused_kernel<NT, RPW, KSPLIT, EPI, U>;
@@ -444,7 +448,7 @@ inline void gemv_launch_one(const GemvFusedArgs& a, hipStream_t s) {
   static const int per_cu_env = [] { const char* e = getenv("PEGAINFER_GEMV_GRID_PER_CU"); return e && *e ? atoi(e) : -1; }();
   static const int cap_min_kb = [] { const char* e = getenv("PEGAINFER_GEMV_CAP_MIN_KB"); return e && *e ? atoi(e) : 40; }();
   const int blocks_per_wave = KSPLIT == 1 ? ceil_div(a.K, 512) : ceil_div(ceil_div(a.K, 512), KSPLIT);
-  constexpr int NW_ = EPI == kEpiSilu ? 2 : 1;
+  constexpr int NW_ = EPI != kEpiStore ? 2 : 1;
   const int inflight_kb = 4 * (blocks_per_wave < U ? blocks_per_wave : U) * NW_ * RPW;
   const int per_cu_cap = per_cu_env >= 0 ? per_cu_env : (NT <= 2 && inflight_kb >= cap_min_kb ? 2 : 0);
   int cap = cached_cap;
@@ -470,7 +474,7 @@ template <int NT, int EPI>
 inline void gemv_launch_nt(const GemvFusedArgs& a, hipStream_t s) {
   // rows per wave: 2 for the plain store (16 KB of loads per wave with U = 4 ... 8 KB), 1 for SwiGLU (two
   // matrices per wave); both stay <= 96 VGPRs for NT <= 2, i.e. 5 workgroups per CU.  RPW never changes results.
-  constexpr int RPW = EPI == kEpiSilu ? 1 : 2;
+  constexpr int RPW = EPI != kEpiStore ? 1 : 2;
   // whole rows in flight (U = 5) for the single-request / pair forms when a wave's share of a row is exactly 5 blocks
   // (PEGAINFER_GEMV_U5=0: the four-then-one form, for A/B runs); wider batches keep U = 4 (register budget)
   static const bool u5 = [] { const char* e = getenv("PEGAINFER_GEMV_U5"); return !(e && *e == '0'); }();
@@ -498,7 +502,7 @@ inline bool gemv_dispatch(const GemvFusedArgs& a_in, hipStream_t s) {
     hi.X = a.X + (size_t)8 * a.K;
     if (a.residual) hi.residual = a.residual + (size_t)8 * a.K;
     if (a.hidden_out) hi.hidden_out = a.hidden_out + (size_t)8 * a.K;
-    hi.Y = a.Y + (size_t)8 * (EPI == kEpiSilu ? a.I : a.M);
+    hi.Y = a.Y + (size_t)8 * (EPI != kEpiStore ? a.I : a.M);
     return gemv_dispatch<EPI>(lo, s) && gemv_dispatch<EPI>(hi, s);
   }
   const int nt = a.T == 1 ? 1 : a.T == 2 ? 2 : a.T <= 4 ? 4 : a.T <= 8 ? 8 : 16;

@@ -749,8 +749,13 @@ struct Model {
   }
   // out = Wdown clamp_glu([Wgate ; Wup] in)
   int glu(const void* gate_up, const void* down, const GluCfg& g, const void* in, void* out, int T) {
-    if (linear(gate_up, in, gu, 2 * g.ff, T, D)) return -1;
-    FZ_K(pegainfer_clamp_glu_rows(gu, act, g.ff, T, g.limit, kGluAlpha, dtype, S()));
+    if (dtype == PEGAINFER_DTYPE_BF16 && !plain_kernels && pegainfer_gemv_clamp_glu_ok(static_cast<const Half*>(gate_up), static_cast<const Half*>(in), T, D)) {
+      FZ_K(pegainfer_gemv_clamp_glu(static_cast<const Half*>(gate_up), static_cast<const Half*>(in), static_cast<Half*>(act), g.ff, T, D, g.limit, kGluAlpha,
+                                    S()));
+    } else {
+      if (linear(gate_up, in, gu, 2 * g.ff, T, D)) return -1;
+      FZ_K(pegainfer_clamp_glu_rows(gu, act, g.ff, T, g.limit, kGluAlpha, dtype, S()));
+    }
     return linear(down, act, out, D, T, g.ff);
   }
 

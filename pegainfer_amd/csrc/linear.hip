@@ -1043,6 +1043,23 @@ pegainfer_status_t pegainfer_gemv_fused(const Half* W, const Half* X, Half* Y, i
   return gemv_fused_impl(W, X, Y, M, T, K, residual, norm_weight, hidden_out, eps, silu_intermediate, 0, stream);
 }
 
+// One or two rows: [gate; up] and the clamped gated unit in the product's own epilogue, with the roundings of the two launches it stands for (a 9216-wide
+// unit behind 2560: 16.0 + 4.6 us, 17.1 here).
+int32_t pegainfer_gemv_clamp_glu_ok(const Half* W, const Half* X, int32_t T, int32_t K) {
+  return T >= 1 && T <= 2 && K > 0 && (K & 7) == 0 && pk::host_aligned16(W) && pk::host_aligned16(X) && !pk::t1_uses_mfma();
+}
+pegainfer_status_t pegainfer_gemv_clamp_glu(const Half* W, const Half* X, Half* Y, int32_t I, int32_t T, int32_t K, float limit, float alpha,
+                                            pegainfer_stream_t stream) {
+  using namespace pk;
+  if (I <= 0 || I > (1 << 29) || !pegainfer_gemv_clamp_glu_ok(W, X, T, K)) return (pegainfer_status_t)hipErrorInvalidValue;
+  GemvFusedArgs a{W, X, Y, 2 * I, T, K, nullptr, nullptr, nullptr, 0.f, I, 0, 0};
+  a.limit = limit;
+  a.alpha = alpha;
+  if (T == 1) { a.KT = gemv_pick_kt(1, K); gemv_launch_nt<1, kEpiClamp>(a, as_stream(stream)); }
+  else { a.KT = gemv_pick_kt(2, K); gemv_launch_nt<2, kEpiClamp>(a, as_stream(stream)); }
+  return (pegainfer_status_t)hipGetLastError();
+}
+
 // Qwen3.5 forms (flags: 1 = (1 + w) norm weight, 2 = residual sum rounded to bf16 before the norm, 4 = silu rounded
 // to bf16 before the multiply); T <= 4 only.
 pegainfer_status_t pegainfer_gemv_fused_ex(const Half* W, const Half* X, Half* Y, int32_t M, int32_t T, int32_t K,
