@@ -908,6 +908,9 @@ typedef struct {
   int32_t n_rows, dtype;
 } pegainfer_qk_prep_desc;
 pegainfer_status_t pegainfer_qk_prep(const pegainfer_qk_prep_desc* p, pegainfer_stream_t stream);
+/* the same and a decode step's convolution and gated unit, which neither reads nor writes what the other writes, in one launch (_ok: bf16, pairs of values) */
+int32_t pegainfer_qk_prep_conv_ok(const pegainfer_qk_prep_desc* p, const pegainfer_conv_glu_step_desc* q);
+pegainfer_status_t pegainfer_qk_prep_conv(const pegainfer_qk_prep_desc* p, const pegainfer_conv_glu_step_desc* q, pegainfer_stream_t stream);
 /* A decode step (every entry one row) of a layer with an attention beside the memory, in two launches around the attention's:
  *   _beside   the memory's scan and the preparation of the attention's rows (_ok says whether: bf16 throughout, pairs of values);
  *   _finish   what is left of both: n and the running maximum move on, o -> out[e, h vdim + c] = o / sqrt(mean(o^2) + eps) * norm_w[h vdim + c] *
@@ -983,6 +986,18 @@ pegainfer_status_t pegainfer_paged_attention_masked(const float* q, const void* 
                                                     int32_t keep_first, const float* dist_bias, int32_t n_dist, const void* gate,
                                                     int64_t gate_stride, int32_t gate_kind, int32_t n_split, float* workspace,
                                                     int32_t plain, int32_t dtype, pegainfer_stream_t stream);
+/* A state-space scan beside an attention (pegainfer_attn_options.scan_beside): `rows` rows of the scan's o, normed in `heads` runs of vdim values and gated as
+ * pegainfer_head_gate_rms does */
+typedef struct {
+  const pegainfer_ssd_scan_desc* scan;
+  const void* norm_w;
+  const void* gate;
+  int64_t gate_stride;
+  void* out;
+  int64_t out_stride;
+  float factor, eps;
+  int32_t w_per_head, gate_kind, gate_first, heads, vdim, rows;
+} pegainfer_scan_beside_desc;
 /* The same with the options in a struct (zeroed = plain causal softmax attention, unsplit; maps 0 counts as 1) and one more:
  * dist_slope: fp32 [heads] (or NULL); dist_slope[h] * (i - j) is taken off the scaled, capped score of query head h - a bias that
  * grows linearly with the distance, without a table and without a limit. */
@@ -1011,7 +1026,11 @@ typedef struct {
    * attention's launch.  pegainfer_paged_attention_beside_ok says which forms take one (bf16, one map, the matrix-core form with tiles of up to
    * 16 rows); pegainfer_paged_attention_opt refuses the others, pegainfer_paged_attention_gated all. */
   const pegainfer_recurrent_step_desc* beside;
+  /* not NULL: a state-space scan of a decode step and the norm and gate of its read-out (as pegainfer_head_gate_rms), done in the attention's launches on
+   * the same terms.  pegainfer_paged_attention_scan_ok: as above, keys split between workgroups, 33 to 128 states, norms of up to 512 values. */
+  const pegainfer_scan_beside_desc* scan_beside;
 } pegainfer_attn_options;
+int32_t pegainfer_paged_attention_scan_ok(const pegainfer_attn_options* opt, int32_t dtype);
 int32_t pegainfer_paged_attention_beside_ok(const pegainfer_attn_options* opt, int32_t dtype);
 int32_t pegainfer_paged_attention_rows_ok(int32_t dim, int32_t vdim, int32_t shared_tail, int64_t page_stride, int64_t v_cache_off,
                                           int32_t page_size);

@@ -21,7 +21,9 @@
 #include "common.h"
 #include "typed.h"
 #include "qk_prep_core.h"
+#include "head_rms_core.h"
 #include "recurrent_step.h"
+#include "ssd_core.h"
 #include "pegainfer_kernels_blocks.h"
 
 namespace pk {
@@ -1093,13 +1095,15 @@ static constexpr size_t rows_attention_lds() {
 // workgroup per row: wave w takes splits w, w + 4, ..., eight splits' values on their way with everything else that the row needs before
 // anything is waited for; the waves' sums meet in LDS in wave order.  Launch- and latency-bound: against a
 // wave per row, splits one batch of loads after another, 8 rows of 8 heads with two maps 8.3 -> 6.8 us; one row over 64 splits 5.6 (over 16 5.8).
+// of 256 threads: row lr of key/value head g of a tile
 template <typename A, int MAPS>
-__global__ __launch_bounds__(256) void paged_attention_merge_kernel(
+__device__ __forceinline__ void paged_attention_merge_block(
+    int tile, int g, int lr,
     const float* __restrict__ part, int nsplit, int H, int G, int vdim, float factor, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_ntok, const int32_t* __restrict__ tile_qh0,
     const int32_t* __restrict__ tile_nqh, A* __restrict__ out, int64_t out_stride, AttnForm form) {
   __shared__ float s_acc[3][MAPS][256];
-  const int tile = blockIdx.x, g = blockIdx.y, lr = blockIdx.z, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int row0 = tile_row0[tile], ntok = tile_ntok[tile], qh0 = tile_qh0[tile], nqh = tile_nqh[tile];
   if (lr >= ntok * nqh) return;
   const int row = row0 + lr / nqh, qh = g * (H / G) + qh0 + lr % nqh;
@@ -1149,6 +1153,52 @@ __global__ __launch_bounds__(256) void paged_attention_merge_kernel(
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[m][c] += s_acc[w][m][lane + 64 * c];
   attn_finish_row<A, MAPS>(mrun, lrun, acc, form, end, vdim, factor, lane, out + (int64_t)row * out_stride + (int64_t)qh * vdim);
+}
+template <typename A, int MAPS>
+__global__ __launch_bounds__(256) void paged_attention_merge_kernel(
+    const float* __restrict__ part, int nsplit, int H, int G, int vdim, float factor, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_ntok, const int32_t* __restrict__ tile_qh0,
+    const int32_t* __restrict__ tile_nqh, A* __restrict__ out, int64_t out_stride, AttnForm form) {
+  paged_attention_merge_block<A, MAPS>(blockIdx.x, blockIdx.y, blockIdx.z, part, nsplit, H, G, vdim, factor, positions, tile_row0, tile_ntok, tile_qh0, tile_nqh, out, out_stride, form);
+}
+
+// Decoding, a layer with a state-space scan beside its attention: the scan's workgroups behind the attention's in one grid, and the norm and gate of its
+// read-out behind the merge's.  One row, 16 heads over 4 of 128 beside 32 heads of 128 x 64: 9.0 + 6.6 and 5.6 + 3.7 us one after the other,
+// 9.6 and 5.6 here.
+template <int NCB, int NS>
+__global__ __launch_bounds__(256) void paged_attention_scan_kernel(
+    const float* __restrict__ q, const uint16_t* __restrict__ cache, int64_t page_stride, int64_t k_cache_off, int64_t v_cache_off,
+    int page_size, const int32_t* __restrict__ positions, const int32_t* __restrict__ row_entry,
+    const int32_t* __restrict__ page_indptr, const int32_t* __restrict__ page_ids, int H, int G, int dim, int vdim, float scale,
+    float factor, const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_ntok,
+    const int32_t* __restrict__ tile_qh0, const int32_t* __restrict__ tile_nqh, uint16_t* __restrict__ out, int64_t out_stride,
+    AttnForm form, int nsplit, float* __restrict__ part, int n_tiles, pegainfer_ssd_scan_desc d, int nbx) {
+  const int n_attention = n_tiles * G * nsplit, b = blockIdx.x;
+  if (b >= n_attention) {
+    const int i = b - n_attention;
+    ssd_scan_block<NS, uint16_t>(i % nbx, i / nbx % d.heads, i / (nbx * d.heads), d.xbc, d.xbc_stride, static_cast<const uint16_t*>(d.proj), d.proj_stride,
+                                 d.dt_off, static_cast<const uint16_t*>(d.A_log), static_cast<const uint16_t*>(d.dt_bias),
+                                 static_cast<const uint16_t*>(d.D), d.state, d.slot_stride, d.o, d.heads, d.groups, d.n_state, d.vdim, d.entry_row0,
+                                 d.entry_slot, 0);
+    return;
+  }
+  paged_attention_mfma_block<1, NCB>(b % n_tiles, b / n_tiles % G, b / (n_tiles * G), q, cache, page_stride, k_cache_off, v_cache_off, page_size, positions, row_entry, page_indptr, page_ids, H, G, dim, vdim, scale, factor, tile_row0, tile_ntok, tile_qh0, tile_nqh, out, out_stride, form, nsplit, part);
+}
+template <int V>
+__global__ __launch_bounds__(256) void paged_attention_merge_norm_kernel(
+    const float* __restrict__ part, int nsplit, int H, int G, int vdim, float factor, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_ntok, const int32_t* __restrict__ tile_qh0,
+    const int32_t* __restrict__ tile_nqh, uint16_t* __restrict__ out, int64_t out_stride, AttnForm form, int n_tiles, pegainfer_scan_beside_desc d, const float* o_scan) {
+  const int n_merge = n_tiles * G * kAttRows, b = blockIdx.x;
+  if (b >= n_merge) {
+    const int rh = (b - n_merge) * 4 + (threadIdx.x >> 6);
+    if (rh < d.rows * d.heads)
+      head_rms_gate_wave<uint16_t, V>(rh / d.heads, rh % d.heads, o_scan, static_cast<const uint16_t*>(d.norm_w), d.w_per_head,
+                                      static_cast<const uint16_t*>(d.gate), d.gate_stride, d.gate_kind, d.factor, d.eps, static_cast<uint16_t*>(d.out),
+                                      d.out_stride, d.heads, d.vdim, d.gate_first);
+    return;
+  }
+  paged_attention_merge_block<uint16_t, 1>(b % n_tiles, b / n_tiles % G, b / (n_tiles * G), part, nsplit, H, G, vdim, factor, positions, tile_row0, tile_ntok, tile_qh0, tile_nqh, out, out_stride, form);
 }
 
 // out[row, :cols] = in[row, :cols] * factor, rows of either side at their own stride
@@ -1275,6 +1325,15 @@ int32_t pegainfer_paged_attention_beside_ok(const pegainfer_attn_options* o, int
          recurrent_step_ok(q) && q->n_entries > 0;
 }
 
+int32_t pegainfer_paged_attention_scan_ok(const pegainfer_attn_options* o, int32_t dtype) {
+  const pegainfer_scan_beside_desc* d = o ? o->scan_beside : nullptr;
+  const pegainfer_ssd_scan_desc* q = d ? d->scan : nullptr;
+  return q && dtype == kDtBf16 && o->maps <= 1 && !o->plain && o->tile_rows <= kAttRows && o->n_split > 1 && q->dtype == dtype && q->n_long == 0 && q->heads > 0 &&
+         q->groups > 0 && q->heads % q->groups == 0 && q->n_state > 32 && q->n_state <= 128 && q->vdim > 0 && q->n_entries > 0 && q->n_entries <= 65535 &&
+         (int64_t)ceil_div(q->vdim, kRecCols) * q->heads * q->n_entries < (1 << 22) && q->o && d->norm_w && d->gate && d->out && d->heads > 0 && d->vdim > 0 &&
+         d->vdim <= 512 && d->rows > 0 && (int64_t)d->rows * d->heads < (1 << 24);
+}
+
 // the kernel for prompts with two maps: a map's share of a key is a whole number of its 32-wide products, known at compile time
 static bool rows_two_maps_ok(int dim, int vdim) { return (dim == 32 && vdim <= 64) || (dim == 64 && vdim <= 128); }
 
@@ -1296,6 +1355,7 @@ static pegainfer_status_t paged_attention(const float* q, const void* cache, int
   if (gate_kind < 0 || gate_kind > 2 || (gate_kind && !opt->gate)) return PK_BAD;
   if (window < 0 || keep_first < 0 || (keep_first > 0 && window <= 0) || opt->softcap < 0.f || (opt->dist_bias && opt->n_dist < 1)) return PK_BAD;
   if (opt->beside && !pegainfer_paged_attention_beside_ok(opt, dtype)) return PK_BAD;
+  if (opt->scan_beside && (opt->beside || !pegainfer_paged_attention_scan_ok(opt, dtype))) return PK_BAD;
   if (n_split < 1) n_split = 1;
   if (n_split > 1 && (!workspace || n_split > 64)) return PK_BAD;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || (maps != 1 && maps != 2) || maps * dim > 256 || vdim <= 0 ||
@@ -1371,6 +1431,31 @@ static pegainfer_status_t paged_attention(const float* q, const void* cache, int
       else if (ncb == 4) both(paged_attention_beside_kernel<4>);
       else if (ncb == 8) both(paged_attention_beside_kernel<8>);
       else both(paged_attention_beside_kernel<16>);
+    } else if (const pegainfer_scan_beside_desc* d = opt->scan_beside) {
+      const pegainfer_ssd_scan_desc& scan = *d->scan;
+      const int nbx = ceil_div(scan.vdim, kRecCols);
+      const dim3 blocks((unsigned)((int64_t)n_tiles * kv_heads * n_split + (int64_t)nbx * scan.heads * scan.n_entries));
+      auto both = [&](auto kern) { launch_as(kern, blocks, 256, (int)n_tiles, scan, nbx); };
+      auto by_states = [&](auto cols) {
+        constexpr int NCB = decltype(cols)::value;
+        if (scan.n_state > 64) both(paged_attention_scan_kernel<NCB, 8>);
+        else both(paged_attention_scan_kernel<NCB, 4>);
+      };
+      if (ncb == 2) by_states(std::integral_constant<int, 2>());
+      else if (ncb == 4) by_states(std::integral_constant<int, 4>());
+      else if (ncb == 8) by_states(std::integral_constant<int, 8>());
+      else by_states(std::integral_constant<int, 16>());
+      if (!ok) return PK_BAD;
+      const unsigned merge = (unsigned)((int64_t)n_tiles * kv_heads * kAttRows + ceil_div((long)d->rows * d->heads, 4));
+      auto finish = [&](auto kern) {
+        kern<<<merge, 256, 0, as_stream(stream)>>>(workspace, n_split, heads, kv_heads, vdim, factor, positions, tile_row0, tile_ntok, tile_qh0, tile_nqh,
+                                                   static_cast<uint16_t*>(out), out_stride, form, (int)n_tiles, *d, scan.o);
+      };
+      const int v = head_rms_values(scan.o, d->norm_w, d->gate, d->gate_stride, d->out, d->out_stride, d->vdim);
+      if (v == 4) finish(paged_attention_merge_norm_kernel<4>);
+      else if (v == 2) finish(paged_attention_merge_norm_kernel<2>);
+      else finish(paged_attention_merge_norm_kernel<1>);
+      return (pegainfer_status_t)hipGetLastError();
     } else {
     auto by_cols = [&](auto maps_c) {
       constexpr int M = decltype(maps_c)::value;

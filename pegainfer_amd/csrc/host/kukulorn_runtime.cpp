@@ -896,15 +896,20 @@ struct Model {
     //      metadata block, so a launch sequence recorded for one decode step serves every later step of the same shape)
     // time convolution of some columns of `proj` into fp32, with the request's tail moved on
     // (a decode step: with the layer's gated unit `c` beside it, which reads the same projected rows)
+    auto conv_glu = [&](const LayerCfg& c, const void* in, const void* w, const void* in_bias, const void* out_bias, float* tail, int ch, int taps,
+                        int mode) {
+      pegainfer_conv_glu_step_desc q{};
+      q.in = in; q.in_row_stride = proj_stride; q.w = w; q.in_bias = in_bias; q.out_bias = out_bias; q.state = tail; q.slot_stride = slot_stride;
+      q.out = conv32; q.out_row_stride = ch; q.channels = ch; q.taps = taps; q.mode = mode; q.entry_slot = d_slot;
+      q.gate = at(proj, (size_t)c.o_ffg); q.up = at(proj, (size_t)c.o_ffu); q.glu_out = act; q.glu_row_stride = c.ff; q.I = c.ff;
+      q.act = PEGAINFER_ACT_RELU; q.n_entries = n; q.dtype = dtype;
+      return q;
+    };
     auto conv = [&](const LayerCfg& c, const void* in, const void* w, const void* in_bias, const void* out_bias, int64_t st_off, int ch,
                     int taps, int mode) -> int {
       float* tail = state + st_off;   // taps == 1: never touched
       if (single && c.ff > 0) {
-        pegainfer_conv_glu_step_desc q{};
-        q.in = in; q.in_row_stride = proj_stride; q.w = w; q.in_bias = in_bias; q.out_bias = out_bias; q.state = tail; q.slot_stride = slot_stride;
-        q.out = conv32; q.out_row_stride = ch; q.channels = ch; q.taps = taps; q.mode = mode; q.entry_slot = d_slot;
-        q.gate = at(proj, (size_t)c.o_ffg); q.up = at(proj, (size_t)c.o_ffu); q.glu_out = act; q.glu_row_stride = c.ff; q.I = c.ff;
-        q.act = PEGAINFER_ACT_RELU; q.n_entries = n; q.dtype = dtype;
+        const pegainfer_conv_glu_step_desc q = conv_glu(c, in, w, in_bias, out_bias, tail, ch, taps, mode);
         KK_K(pegainfer_conv_glu_step(&q, S()));
         return 0;
       }
@@ -918,7 +923,9 @@ struct Model {
       KK_K(pegainfer_time_conv_commit_biased(in, dtype, proj_stride, in_bias, dtype, tail, slot_stride, ch, taps, d_row0, d_slot, n, S()));
       return 0;
     };
-    auto attention = [&](const LayerCfg& c, const LayerW& w, const Run& r, const void* gate, int gate_kind) -> int {
+    // `beside`: a state-space scan taken into the attention's launches where that can be (`taken` says so)
+    auto attention = [&](const LayerCfg& c, const LayerW& w, const Run& r, const void* gate, int gate_kind, const pegainfer_scan_beside_desc* beside = nullptr,
+                         bool* taken = nullptr) -> int {
       const AttnCfg& a = c.at;
       const size_t ts = (size_t)c.tile_set;
       const int32_t* tb = md + tile_off[ts];
@@ -932,6 +939,8 @@ struct Model {
       o.n_split = wgs >= ptiles::kUnsplitGroups || tile_rows[ts] > ptiles::kGroupRows ? 1 : std::max(1, std::min(ptiles::kMaxSplits, kSplitGroups / wgs));
       o.workspace = att_part;
       o.plain = plain_kernels ? 1 : 0;
+      o.scan_beside = beside;
+      if (beside && !(*taken = pegainfer_paged_attention_scan_ok(&o, dtype))) o.scan_beside = nullptr;
       KK_K(pegainfer_paged_attention_opt(q32, cache, page_stride, r.k_off, r.v_off, kPageSize, d_pos, d_ent, d_ind, d_pages, a.heads,
                                          a.kv, a.dim, a.vdim, a.scale, 1.0f, tb, tb + tile_cnt[ts], tb + 2 * tile_cnt[ts],
                                          tb + 3 * tile_cnt[ts], (int)tile_cnt[ts], mix, a.heads * a.vdim, &o, dtype, S()));
@@ -977,15 +986,16 @@ struct Model {
       } else {
         const SsmCfg& s = c.sm;
         // left: attention over a window and the kept first tokens, a bias by distance, a gate per head
-        KK_K(pegainfer_qk_prep_paged_form(proj, dtype, c.proj_rows, c.o_q, c.o_k, c.o_v, a.heads, a.kv, a.dim, a.vdim, w.q_norm, w.k_norm,
-                                          PEGAINFER_QKNORM_ALL_WEIGHT, eps, w.qkv_bias, at(w.qkv_bias, (size_t)c.o_k),
-                                          at(w.qkv_bias, (size_t)c.o_v), 0.f, 0, w.inv_freq, a.rot_dims, PEGAINFER_ROT_HALVES, d_pos, d_ent,
-                                          d_ind, d_pages, cache, page_stride, r.k_off, r.v_off, kPageSize, q32, nullptr, Ti, dtype, S()));
-        if (attention(c, w, r, at(proj, (size_t)c.o_g), PEGAINFER_GATE_PER_HEAD)) return -1;
-        if (linear(w.o, mix, y1, D, Ti, a.heads * a.vdim)) return -1;
+        pegainfer_qk_prep_desc qk{};
+        qk.proj = proj; qk.proj_dtype = qk.dtype = dtype; qk.proj_stride = c.proj_rows; qk.q_off = c.o_q; qk.k_off = c.o_k; qk.v_off = c.o_v;
+        qk.heads = a.heads; qk.kv_heads = a.kv; qk.dim = a.dim; qk.vdim = a.vdim; qk.q_norm = w.q_norm; qk.k_norm = w.k_norm;
+        qk.norm_kind = PEGAINFER_QKNORM_ALL_WEIGHT; qk.eps = eps; qk.q_bias = w.qkv_bias; qk.k_bias = at(w.qkv_bias, (size_t)c.o_k);
+        qk.v_bias = at(w.qkv_bias, (size_t)c.o_v); qk.inv_freq = w.inv_freq; qk.rot_dims = a.rot_dims; qk.rot_layout = PEGAINFER_ROT_HALVES; qk.rot_amp = 1.0f;
+        qk.positions = d_pos; qk.row_entry = d_ent; qk.page_indptr = d_ind; qk.page_ids = d_pages; qk.cache = cache; qk.page_stride = page_stride;
+        qk.k_cache_off = r.k_off; qk.v_cache_off = r.v_off; qk.page_size = kPageSize; qk.q_out = q32; qk.n_rows = Ti;
         // right: [z | x | B | C | dt] at o_in; x | B | C through the convolution, the scan, y * silu(z) normed in groups
         const int inner = s.inner();
-        if (conv(c, at(proj, (size_t)(c.o_in + inner)), w.sconv, nullptr, w.sconv_b, r.st_sconv, s.conv_ch(), s.taps, 2)) return -1;
+        const void* conv_in = at(proj, (size_t)(c.o_in + inner));
         pegainfer_ssd_scan_desc sd{};
         sd.xbc = conv32; sd.xbc_stride = s.conv_ch(); sd.proj = proj; sd.proj_stride = c.proj_rows;
         sd.dt_off = c.o_in + 2 * inner + 2 * s.groups * s.state;
@@ -995,9 +1005,26 @@ struct Model {
         sd.chunk_row0 = md + chunk_off[0]; sd.chunk_rows = md + chunk_off[1]; sd.n_chunks = (int)chunks.row0.size();
         sd.long_chunk0 = md + chunk_off[2]; sd.long_slot = md + chunk_off[3]; sd.n_long = (int)chunks.slot.size();
         sd.workspace = chunk_ws.p; sd.dtype = dtype;
-        KK_K(pegainfer_ssd_scan_form(&sd, S()));
-        KK_K(pegainfer_head_gate_rms(o32, w.snorm, 1, at(proj, (size_t)c.o_in), c.proj_rows, 0, 1, 1.0f, eps, mixr, inner, s.norm_groups,
-                                     inner / s.norm_groups, Ti, dtype, S()));
+        pegainfer_scan_beside_desc beside{};
+        beside.scan = &sd; beside.norm_w = w.snorm; beside.w_per_head = 1; beside.gate = at(proj, (size_t)c.o_in); beside.gate_stride = c.proj_rows;
+        beside.gate_first = 1; beside.factor = 1.0f; beside.eps = eps; beside.out = mixr; beside.out_stride = inner; beside.heads = s.norm_groups;
+        beside.vdim = inner / s.norm_groups; beside.rows = Ti;
+        // decoding: the convolution beside the attention's preparation, then the scan and its norm beside the attention
+        bool conv_done = false, scan_done = false;
+        if (single && c.ff > 0 && !plain_kernels) {
+          const pegainfer_conv_glu_step_desc q = conv_glu(c, conv_in, w.sconv, nullptr, w.sconv_b, state + r.st_sconv, s.conv_ch(), s.taps, 2);
+          conv_done = pegainfer_qk_prep_conv_ok(&qk, &q);
+          if (conv_done) KK_K(pegainfer_qk_prep_conv(&qk, &q, S()));
+        }
+        if (!conv_done) KK_K(pegainfer_qk_prep(&qk, S()));
+        if (attention(c, w, r, at(proj, (size_t)c.o_g), PEGAINFER_GATE_PER_HEAD, conv_done ? &beside : nullptr, &scan_done)) return -1;
+        if (linear(w.o, mix, y1, D, Ti, a.heads * a.vdim)) return -1;
+        if (!conv_done && conv(c, conv_in, w.sconv, nullptr, w.sconv_b, r.st_sconv, s.conv_ch(), s.taps, 2)) return -1;
+        if (!scan_done) {
+          KK_K(pegainfer_ssd_scan_form(&sd, S()));
+          KK_K(pegainfer_head_gate_rms(o32, w.snorm, 1, at(proj, (size_t)c.o_in), c.proj_rows, 0, 1, 1.0f, eps, mixr, inner, s.norm_groups,
+                                       inner / s.norm_groups, Ti, dtype, S()));
+        }
         if (linear(w.ro, mixr, y2, D, Ti, inner)) return -1;
         terms[n_terms++] = pegainfer_sum_term{y1, D, w.o_bias, w.left_out, 0.5f};
         terms[n_terms++] = pegainfer_sum_term{y2, D, nullptr, w.right_out, 0.5f};

@@ -582,7 +582,7 @@ def _struct(name, fields):
 AttnOptions = _struct("AttnOptions", [("i", "maps"), ("f", "lambda_"), ("i", "block"), ("p", "sink"), ("i", "head_norm"), ("f", "norm_eps softcap"),
                                       ("i", "window keep_first"), ("p", "dist_bias"), ("i", "n_dist"), ("p", "dist_slope gate"),
                                       ("l", "gate_stride"), ("i", "gate_kind n_split"), ("p", "workspace"), ("i", "plain shared_tail tile_rows"),
-                                      ("p", "beside")])
+                                      ("p", "beside scan_beside")])
 LatentPrepDesc = _struct("LatentPrepDesc", [("p", "dkv"), ("l", "dkv_stride"), ("p", "c_norm_w ql"), ("l", "ql_stride"), ("p", "ql_norm_w ql_out"),
                                             ("i", "q_rank"), ("p", "q"), ("l", "q_stride"), ("p", "qc"), ("f", "eps"), ("p", "inv_freq"),
                                             ("i", "rot_dims rot_layout"), ("p", "positions token_req page_indptr page_ids cache"),
@@ -597,6 +597,8 @@ MatrixMemoryDesc = _struct("MatrixMemoryDesc", [("p", "proj"), ("l", "proj_strid
 MemoryFinishDesc = _struct("MemoryFinishDesc", [("p", "norm_w gate"), ("l", "gate_stride"), ("i", "gate_kind"), ("f", "factor eps"), ("p", "out"),
                                                 ("l", "out_stride"), ("p", "rows"), ("l", "rows_stride"), ("p", "scaled"), ("l", "scaled_stride"),
                                                 ("i", "scale_cols"), ("f", "scale")])
+ScanBesideDesc = _struct("ScanBesideDesc", [("p", "scan norm_w gate"), ("l", "gate_stride"), ("p", "out"), ("l", "out_stride"), ("f", "factor eps"),
+                                            ("i", "w_per_head gate_kind gate_first heads vdim rows")])
 SsdScanDesc = _struct("SsdScanDesc", [("p", "xbc"), ("l", "xbc_stride"), ("p", "proj"), ("l", "proj_stride dt_off"), ("p", "A_log dt_bias D state"),
                                       ("l", "slot_stride"), ("p", "o"), ("i", "heads groups n_state vdim"), ("p", "entry_row0 entry_slot"),
                                       ("i", "n_entries scan_max"), ("p", "chunk_row0 chunk_rows"), ("i", "n_chunks"), ("p", "long_chunk0 long_slot"),
