@@ -9,8 +9,9 @@
 // head, 16 value columns), its four waves dim / 4 rows of S each.  All products are v_mfma_f32_16x16x4_f32 (plain fp32) and every decay is a product of
 // gates at most 1, never a quotient, so strong decays only underflow as they do one by one.
 // 1024 tokens of 32 heads of 128 x 128: 15 + 181 us (prep and token by token), 15 + 74 here; eight entries of 700 tokens, 8 heads 16 + 173 and 19 + 110.
-// Against 64 bits the read-outs are off by 2.1e-7 (2.3e-7 token by token) with slow decays, by 1.2 - 1.8e-7 (1.1 - 1.5e-7) with fast ones; fp32 logits of
-// whole models by the same amount either way (0.9 - 1.8e-6).
+// Against 64 bits the read-outs are off by 2.0e-7 with slow decays (2.3e-7 token by token), by 0.85 - 1.0e-7 with fast ones (1.1 - 1.2e-7): lengths and the
+// products k . k, q . k are made in 64 bits and rounded once (in fp32 sums the fast ones were off by 1.2 - 1.4e-7).  fp32 logits of whole models are off by the
+// same either way (0.9 - 1.8e-6).
 #include <algorithm>
 
 #include "common.h"
@@ -19,6 +20,8 @@
 #include "pegainfer_kernels_blocks.h"
 
 namespace pk {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDc = 16;                        // tokens of a chunk
 constexpr int kDcFloats = 2 * kDc * kDc + 2 * kDc + 32;  // of a (chunk, head): T', M, c, D[15][.], pad
@@ -52,37 +55,36 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
   // lane: token t, dims 16 b + 4 j .. + 3 - both operands of the products below
   f32x4 k[DIM / 16], q[DIM / 16];
   float *qp = qkv + row * qkv_stride + (int64_t)g * DIM + 4 * j, *kp = qp + (int64_t)G * DIM;
-  f32x4 ks[2] = {}, qs[2] = {};                // (short sums: a length's error is in all of its values)
 #pragma unroll
   for (int b = 0; b < DIM / 16; ++b) {
     k[b] = *reinterpret_cast<const f32x4*>(kp + 16 * b);
     q[b] = *reinterpret_cast<const f32x4*>(qp + 16 * b);
   }
+  // Lengths and products in 64 bits, each rounded once: a read-out of strong decays is little more than q_t . k_t times its token's own update,
+  // where token by token 128 roundings of S average out.
+  double kss = 0, qss = 0;
 #pragma unroll
   for (int b = 0; b < DIM / 16; ++b)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       k[b][r] = t < tc ? k[b][r] : 0.f;
       q[b][r] = t < tc ? q[b][r] : 0.f;
-      ks[b & 1][r] = fmaf(k[b][r], k[b][r], ks[b & 1][r]);
-      qs[b & 1][r] = fmaf(q[b][r], q[b][r], qs[b & 1][r]);
+      kss = fma((double)k[b][r], (double)k[b][r], kss);
+      qss = fma((double)q[b][r], (double)q[b][r], qss);
     }
-  ks[0] += ks[1];
-  qs[0] += qs[1];
-  float kss = (ks[0].x + ks[0].y) + (ks[0].z + ks[0].w), qss = (qs[0].x + qs[0].y) + (qs[0].z + qs[0].w);
   kss += __shfl_xor(kss, 16, kWave); kss += __shfl_xor(kss, 32, kWave);
   qss += __shfl_xor(qss, 16, kWave); qss += __shfl_xor(qss, 32, kWave);
-  const float ik = 1.0f / sqrtf(kss + 1e-6f), iq = 1.0f / (sqrtf((float)DIM) * sqrtf(qss + 1e-6f));
-  f32x4 kk[8] = {}, qk[8] = {};                // (eight sums each: closer to the sum in 64 bits than one long chain)
+  const float ik = (float)(1.0 / sqrt(kss + 1e-6)), iq = (float)(1.0 / sqrt((qss + 1e-6) * DIM));
+  f64x4 kk[2] = {}, qk[2] = {};
 #pragma unroll
   for (int b = 0; b < DIM / 16; ++b)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       k[b][r] *= ik;
       q[b][r] *= iq;
-      f32x4 &a = kk[4 * (b & 1) + r], &c = qk[4 * (b & 1) + r];
-      a = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][r], k[b][r], a, 0, 0, 0);
-      c = __builtin_amdgcn_mfma_f32_16x16x4f32(q[b][r], k[b][r], c, 0, 0, 0);
+      const double kd = k[b][r], qd = q[b][r];
+      kk[r & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(kd, kd, kk[r & 1], 0, 0, 0);
+      qk[r & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(qd, kd, qk[r & 1], 0, 0, 0);
     }
   if (t < tc) {
 #pragma unroll
@@ -92,16 +94,9 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
     }
   }
 #pragma unroll
-  for (int w = 4; w; w >>= 1)
-#pragma unroll
-    for (int i = 0; i < w; ++i) {
-      kk[i] += kk[i + w];
-      qk[i] += qk[i + w];
-    }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {                // lane: rows 4 j + r, column t
-    s_kk[wave][4 * j + r][t] = kk[0][r];
-    s_qk[wave][4 * j + r][t] = qk[0][r];
+  for (int r = 0; r < 4; ++r) {                // lane: rows 4 r + j, column t (64-bit products leave them in that order)
+    s_kk[wave][4 * r + j][t] = (float)(kk[0][r] + kk[1][r]);
+    s_qk[wave][4 * r + j][t] = (float)(qk[0][r] + qk[1][r]);
   }
   const int per = H / G;
   for (int h0 = 0; h0 < per; h0 += 4) {
