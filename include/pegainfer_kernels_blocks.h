@@ -605,7 +605,7 @@ pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const vo
                                         int32_t n_entries, int32_t dtype, pegainfer_stream_t stream);
 /* The same for prompts, 16 tokens at a time on fp32 matrix-core products.  dim 64, 128, 192 or 256, vdim a multiple
  * of 16, qkv on 16 bytes with a stride of a multiple of four (_ok).  workspace: _workspace floats, 16-byte aligned.  The results differ from the
- * token-by-token ones by rounding; a chunk that holds an infinite or undefined value holds them in all its rows. */
+ * token-by-token ones by rounding. */
 int64_t pegainfer_delta_rule_workspace(int32_t n_rows, int32_t n_entries, int32_t heads);
 int32_t pegainfer_delta_rule_chunked_ok(int32_t dim, int32_t vdim, const float* qkv, int64_t qkv_stride);
 pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,

@@ -12,6 +12,8 @@
 // Against 64 bits the read-outs are off by 2.0e-7 with slow decays (2.3e-7 token by token), by 0.85 - 1.0e-7 with fast ones (1.1 - 1.2e-7): lengths and the
 // products k . k, q . k are made in 64 bits and rounded once (in fp32 sums the fast ones were off by 1.2 - 1.4e-7).  fp32 logits of whole models are off by the
 // same either way (0.9 - 1.8e-6).
+// The triangular matrices hold zeros for later tokens, and a zero times what is infinite or no number is no number: such values are kept out of the
+// products of the chunk they appear in and spoil its outputs from their own token on, column by column, as they do token by token.
 #include <algorithm>
 
 #include "common.h"
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
           if (4 * s4 + u < i) sum[u & 1] = fmaf(l[u], T[4 * s4 + u], sum[u & 1]);
       }
       T[i] = i == t ? 1.f : i > t ? -(sum[0] + sum[1]) : 0.f;
-      if (own) out[i * kDc + t] = T[i] * bt;
+      if (own) out[i * kDc + t] = i >= t ? T[i] * bt : 0.f;      // (zeros also where bt is no number)
     }
   }
 }
@@ -164,12 +166,31 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
     const auto& part = s_part[c & 1];
     return (part[0][which][lane] + part[1][which][lane]) + (part[2][which][lane] + part[3][which][lane]);
   };
-  auto updates = [&](const f32x4& v, const f32x4& T, const f32x4& decay, int c) {
-    f32x4 U = {};
-    const f32x4 R = v - decay * sum_of_waves(c, 0);
+  auto times = [&](const f32x4& a, const f32x4& b) {           // of a lower triangle and a chunk's rows
+    f32x4 D = {};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) U = __builtin_amdgcn_mfma_f32_16x16x4f32(T[s], R[s], U, 0, 0, 0);
-    return U;
+    for (int s = 0; s < 4; ++s) D = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], D, 0, 0, 0);
+    return D;
+  };
+  // The same for the outputs: what is not finite enters as zero, and the rows from the first such one of a column on are no numbers.  (For S the
+  // plain product does: its column is no number anyway.)
+  auto finite_times = [&](const f32x4& a, f32x4 b) {
+    int first = kDc;
+    const bool spoilt = __any(!(fabsf(b[0]) + fabsf(b[1]) + (fabsf(b[2]) + fabsf(b[3])) <= __FLT_MAX__));      // (or a sum past the largest number)
+    if (spoilt) {
+#pragma unroll
+      for (int r = 3; r >= 0; --r)
+        if (!(fabsf(b[r]) <= __FLT_MAX__)) { first = 4 * j + r; b[r] = 0.f; }
+      first = min(first, __shfl_xor(first, 16, kWave));
+      first = min(first, __shfl_xor(first, 32, kWave));
+    }
+    f32x4 D = times(a, b);
+    if (spoilt) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * j + r >= first) D[r] = __builtin_nanf("");
+    }
+    return D;
   };
   // Chunk c's operands in x; those of c + 1 are on the way while it is worked on, those of c + 2 are asked for.  One loop with one way out: with
   // more, the compiler's waits at its head have to cover them all.  `whole`: all of the chunk's rows are there.
@@ -216,10 +237,8 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
       to[3][lane] = x.left;
       if (lane == 0) s_end[c & 1] = x.end;
       barrier();
-      const f32x4 Q = sum_of_waves(c, 1), U = updates(x.v, x.T, x.decay, c);
-      f32x4 O = {};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(x.M[s], U[s], O, 0, 0, 0);
+      const f32x4 Q = sum_of_waves(c, 1);
+      f32x4 O = finite_times(x.M, finite_times(x.T, x.v - x.decay * sum_of_waves(c, 0)));
 #pragma unroll
       for (int r = 0; r < 4; ++r) O[r] = fmaf(x.decay[r], Q[r], O[r]);
       float* out = o + (int64_t)(row0 + c * kDc) * ((int64_t)H * vdim) + (int64_t)h * vdim + col;
@@ -269,7 +288,7 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
     const auto& from = s_common[c & 1];
     const f32x4 left = from[3][lane];
     const float end = s_end[c & 1];
-    const f32x4 E = left * updates(from[0][lane], from[1][lane], from[2][lane], c);
+    const f32x4 E = left * times(from[1][lane], from[0][lane] - from[2][lane] * sum_of_waves(c, 0));
     f32x4 X[NB] = {};                          // (a sum of its own, so that S is rounded once per chunk)
 #pragma unroll
     for (int s = 0; s < 4; ++s)

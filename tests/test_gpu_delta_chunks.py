@@ -58,3 +58,30 @@ def test_sizes_that_are_left_to_the_token_form():
         qkv, z = torch.zeros(20, 2 * d + dv, device="cuda"), torch.zeros(1, device="cuda")
         assert B.delta_rule(qkv, torch.zeros(20, 2, device="cuda"), 0, 1, z, z, torch.zeros(1, 1, d, dv, device="cuda"), 1, 1, d, dv, B.Ragged([20]),
                             chunked=True) is None
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("what", ["value", "key", "query", "beta", "decay"])
+@pytest.mark.parametrize("H,G,d,dv", [(2, 1, 64, 32), (3, 3, 192, 16)])
+def test_chunks_let_nothing_reach_earlier_tokens(H, G, d, dv, what, bad):
+    """exactly what the token-by-token form spoils is spoilt: from the token on, in its column or head, the state included; the rest stays within
+    the two forms' rounding of each other (1e-5 each of the largest value)"""
+    from pegainfer_amd import ops_blocks as B
+    gen = torch.Generator().manual_seed(d)
+    T = 47                                                         # two whole chunks and one that repeats its last row
+    A, bias, mem = torch.zeros(H), torch.zeros(H), torch.randn(1, H, d, dv, generator=gen)
+    for at in (0, 9, 15, 16, 38, 46):
+        qkv, proj = torch.randn(T, 2 * G * d + H * dv, generator=gen), torch.randn(T, 2 * H, generator=gen)
+        if what in ("beta", "decay"):
+            proj[at, H - 1 if what == "beta" else 2 * H - 1] = bad
+        else:
+            qkv[at, {"query": 3, "key": 2 * G * d - 1, "value": 2 * G * d + dv + 5}[what]] = bad
+        runs = []
+        for chunked in (False, True):
+            st = mem.cuda()
+            runs.append((B.delta_rule(qkv.cuda(), proj.cuda(), 0, H, A.cuda(), bias.cuda(), st, H, G, d, dv, B.Ragged([T]), chunked=chunked).cpu(), st.cpu()))
+        for a, b in zip(*runs):
+            ok = torch.isfinite(a)
+            assert torch.equal(ok, torch.isfinite(b)), (at, int((ok != torch.isfinite(b)).sum()))
+            if ok.any():
+                assert float((a[ok] - b[ok]).abs().max()) < 2e-5 * float(a[ok].abs().max()), at
