@@ -38,7 +38,7 @@ template <typename A, int NB>
 __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                                int64_t proj_stride, int64_t b_off, int64_t a_off, const A* __restrict__ A_log,
                                                                const A* __restrict__ dt_bias, float* __restrict__ ws, int H, int G,
-                                                               const int32_t* __restrict__ entry_row0, int n_entries) {
+                                                               const int32_t* __restrict__ entry_row0, int n_entries, int scan_max) {
   constexpr int DIM = 64 * NB;
   __shared__ float s_kk[4][kDc][kDc + 1], s_qk[4][kDc][kDc + 1];
   __shared__ __attribute__((aligned(16))) float s_l[4][4][kDc][kDc + 4], s_gb[4][4][kDc][2];
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
     if (delta_first_chunk(entry_row0[mid], mid) <= chunk) lo = mid; else hi = mid - 1;
   }
   const int row0 = entry_row0[lo], len = entry_row0[lo + 1] - row0, at = (chunk - delta_first_chunk(row0, lo)) * kDc;
-  if (at < 0 || at >= len || g >= G) return;   // (waves share nothing: there is no barrier below)
+  if (at < 0 || at >= len || len <= scan_max || g >= G) return;   // (waves share nothing: there is no barrier below)
   const int tc = min(kDc, len - at);
   const int64_t row = row0 + at + min(t, tc - 1);
   const float live = t < tc ? 1.f : 0.f;
@@ -149,7 +149,7 @@ constexpr int kDcThreads = 320;
 template <int NB>
 __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qkv, int qkv_stride, const float* ws, float* __restrict__ state,
                                                                  int64_t slot_stride, float* __restrict__ o, int H, int G, int vdim,
-                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot) {
+                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot, int scan_max) {
   constexpr int DIM = 64 * NB;
   __shared__ f32x4 s_part[2][4][2][64];        // K S0 and Q S0 over a wave's rows of S
   __shared__ f32x4 s_common[2][4][64];         // by lane: values, T', c, D[15][.]
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
   const int e = blockIdx.z, h = blockIdx.y, col = blockIdx.x * 16 + (threadIdx.x & 15);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l15 = lane & 15, j = lane >> 4;
   const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
-  if (len <= 0) return;
+  if (len <= scan_max) return;                 // (0: empty ones)
   const int n = (len + kDc - 1) / kDc, g0 = h / (H / G);
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };     // (not the loads of the chunks ahead)
   // rows past the entry's end: its last one, which T' leaves out
@@ -333,10 +333,10 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
                                                 int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
                                                 int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
                                                 int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
-                                                int32_t dtype, pegainfer_stream_t stream) {
+                                                int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (n_entries <= 0 || n_rows <= 0) return 0;
-  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || !workspace || !host_aligned16(workspace) ||
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || scan_max < 0 || !workspace || !host_aligned16(workspace) ||
       !pegainfer_delta_rule_chunked_ok(dim, vdim, qkv, qkv_stride))
     return bad;
   hipStream_t st = as_stream(stream);
@@ -347,8 +347,9 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
       constexpr int NB = decltype(nb)::value;
       delta_chunk_prep_kernel<A, NB><<<prep, 256, 0, st>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off,
                                                            static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace, heads, kv_heads,
-                                                           entry_row0, n_entries);
-      delta_chunk_kernel<NB><<<grid, kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads, vdim, entry_row0, entry_slot);
+                                                           entry_row0, n_entries, scan_max);
+      delta_chunk_kernel<NB><<<grid, kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads, vdim, entry_row0, entry_slot,
+                                                     scan_max);
     });
   });
   return known ? (pegainfer_status_t)hipGetLastError() : bad;

@@ -845,7 +845,9 @@ struct Model {
     // long entries of the matrix memory in chunks (never part of a captured step)
     ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
     if (!ensure_chunks((int)chunks.row0.size())) chunks = ptiles::Chunks();   // no memory: the scan, which needs none, takes every entry
+    // the delta rule's long entries in chunks, each by its own length
     const bool delta_chunks = !single && !plain_kernels && *std::max_element(lens, lens + n) > kDeltaScanMax && ensure_delta(T, n);
+    const bool delta_short = *std::min_element(lens, lens + n) <= kDeltaScanMax;
     const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
     size_t chunk_off[4];
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
@@ -992,12 +994,16 @@ struct Model {
         if (single && !plain_kernels && pegainfer_recurrent_step_ok(&q)) {       // preparation, scan, norm and gate in one launch
           FZ_K(pegainfer_recurrent_step(&q, S()));
         } else {
-          if (delta_chunks && pegainfer_delta_rule_chunked_ok(d.dim, d.vdim, qkv32, c.conv_ch))
+          if (delta_chunks && pegainfer_delta_rule_chunked_ok(d.dim, d.vdim, qkv32, c.conv_ch)) {
             FZ_K(pegainfer_delta_rule_chunked(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
-                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
-          else
+                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, kDeltaScanMax, dtype, S()));
+            if (delta_short)
+              FZ_K(pegainfer_delta_rule_short(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
+                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, kDeltaScanMax, dtype, S()));
+          } else {
             FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
                                       o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));
+          }
           FZ_K(pegainfer_head_rms_gate(o32, w.onorm, 0, at(proj, (size_t)c.o_g), Mp, 0, 1.0f, eps, mix, c.mix_cols, d.heads, d.vdim,
                                        Ti, dtype, S()));
         }

@@ -13,8 +13,9 @@
 //   delta_rule_kernel      S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q      (long entries with one decay per head: delta_chunk.hip)
 //   matrix_memory_kernel   m' = max(f + m, i);  S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise;  o = S^T q / (max(|n.q|, e^-m') + 1e-6)
 // A row's result depends only on the rows before it in its own request: the token order is fixed, and cutting a prompt into
-// steps only moves where the state passes through HBM (exactly, it is fp32 either way).  The matrix memory also has a form in chunks
-// for long portions (below); which portions take it moves results by rounding only.
+// steps only moves where the state passes through HBM (exactly, it is fp32 either way).  The matrix memory (below) and the delta rule with one
+// decay per head (delta_chunk.hip) also have a form in chunks for long portions; a portion's own length says which it takes, and that moves
+// results by rounding only.
 #include <algorithm>
 
 #include "common.h"
@@ -30,15 +31,31 @@ namespace pk {
 
 __device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
 
+// the entry that holds a row: the last one that begins at or before it
+__device__ __forceinline__ int entry_of_row(const int32_t* __restrict__ entry_row0, int n_entries, int row) {
+  int lo = 0, hi = n_entries - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (entry_row0[mid] <= row) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
 // Per row, before the recurrence: q and k heads made unit vectors in place (x / sqrt(sum(x^2) + 1e-6), q also * dim^-1/2),
 // gates[row] = [g: heads | beta: heads].  A wave per head; a row's heads and gates are dealt over gridDim.y workgroups (few rows: as many
 // as its heads fill - one workgroup took 10.0 us for a row of 32 heads of 128, eight take 4.2 us; from 256 rows on one).
+// scan_max > 0: the rows of entries of up to that many alone.
 template <typename A>
 __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                          int64_t proj_stride, int64_t b_off, int64_t a_off,
                                                          const A* __restrict__ A_log, const A* __restrict__ dt_bias,
-                                                         float* __restrict__ gates, int H, int G, int dim) {
+                                                         float* __restrict__ gates, int H, int G, int dim,
+                                                         const int32_t* __restrict__ entry_row0, int n_entries, int scan_max) {
   const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (scan_max > 0) {
+    const int e = entry_of_row(entry_row0, n_entries, row);
+    if (entry_row0[e + 1] - entry_row0[e] > scan_max) return;      // the chunk form has this entry
+  }
   float* qk = qkv + (int64_t)row * qkv_stride;
   const float qs = 1.0f / sqrtf((float)dim);
   for (int hh = blockIdx.y * 4 + wave; hh < 2 * G; hh += 4 * gridDim.y) {
@@ -92,7 +109,7 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(const float* __restrict
                                                          const float* __restrict__ gates, float* __restrict__ state,
                                                          int64_t slot_stride, float* __restrict__ o, int H, int G, int dim,
                                                          int vdim, const int32_t* __restrict__ entry_row0,
-                                                         const int32_t* __restrict__ entry_slot) {
+                                                         const int32_t* __restrict__ entry_slot, int scan_max) {
   constexpr int DP = kRecSlices * NS;
   constexpr int V = NS >= 4 ? 4 : 1, NV = NS / V;      // values per load, loads of a thread
   __shared__ __attribute__((aligned(16))) float s_k[kRecTokens][DP], s_q[kRecTokens][DP];
@@ -105,6 +122,7 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(const float* __restrict
   const int col = col0 + cl;
   const int g0 = h / (H / G);
   const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
+  if (scan_max > 0 && len > scan_max) return;      // the chunk form has this entry
   float* S_g = state + (int64_t)entry_slot[e] * slot_stride + (int64_t)h * dim * vdim;
   float S[NS];
 #pragma unroll
@@ -530,11 +548,11 @@ using namespace pk;
 // workgroups per row of the launches before the recurrence
 static int prep_parts(int rows, int heads) { return rows >= 256 ? 1 : std::max(1, std::min(ceil_div(heads, 4), 1024 / rows)); }
 
-pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+static pegainfer_status_t delta_rule_launch(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
                                         int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
                                         int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
                                         int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
-                                        int32_t n_entries, int32_t dtype, pegainfer_stream_t stream) {
+                                        int32_t n_entries, int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
   if (n_entries <= 0 || n_rows <= 0) return 0;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > 256 || vdim <= 0 || heads > 65535 || n_entries > 65535)
     return PK_BAD;
@@ -542,17 +560,36 @@ pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const vo
         using A = std::remove_pointer_t<decltype(t)>;
         delta_prep_kernel<A><<<dim3(n_rows, prep_parts(n_rows, 2 * kv_heads)), 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off,
                                                                     a_off, static_cast<const A*>(A_log),
-                                                                    static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim);
+                                                                    static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim, entry_row0, n_entries, scan_max);
       }))
     return PK_BAD;
   const dim3 grid(ceil_div(vdim, kRecCols), heads, n_entries);
   if (!by_slices(dim, [&](auto ns) {
         delta_rule_kernel<decltype(ns)::value, false><<<grid, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, gates, state, slot_stride, o,
                                                                                     heads, kv_heads, dim, vdim, entry_row0,
-                                                                                    entry_slot);
+                                                                                    entry_slot, scan_max);
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();
+}
+
+pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                        int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
+                                        int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
+                                        int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
+                                        int32_t n_entries, int32_t dtype, pegainfer_stream_t stream) {
+  return delta_rule_launch(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, state, slot_stride, o, heads, kv_heads, dim, vdim, n_rows,
+                           entry_row0, entry_slot, n_entries, 0, dtype, stream);
+}
+
+pegainfer_status_t pegainfer_delta_rule_short(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                              int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
+                                              int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
+                                              int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
+                                              int32_t n_entries, int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
+  if (scan_max <= 0) return PK_BAD;
+  return delta_rule_launch(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, state, slot_stride, o, heads, kv_heads, dim, vdim, n_rows,
+                           entry_row0, entry_slot, n_entries, scan_max, dtype, stream);
 }
 
 pegainfer_status_t pegainfer_delta_rule_channel(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride,
@@ -575,7 +612,7 @@ pegainfer_status_t pegainfer_delta_rule_channel(float* qkv, int64_t qkv_stride, 
   if (!by_slices(dim, [&](auto ns) {
         delta_rule_kernel<decltype(ns)::value, true><<<grid, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, gates, state, slot_stride, o,
                                                                                           heads, kv_heads, dim, vdim, entry_row0,
-                                                                                          entry_slot);
+                                                                                          entry_slot, 0);
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();

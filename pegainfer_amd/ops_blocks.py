@@ -288,25 +288,25 @@ def route_combine_add(y_pairs, weight, add, out_dtype):
     return out
 
 
-def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_heads, dim, vdim, rg, chunked=False):
+def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_heads, dim, vdim, rg, chunked=False, scan_max=0):
     """qkv fp32 [rows, 2 kv dim + heads vdim] (after convolution and silu), proj [rows, *] with the beta / decay inputs;
     state fp32 [slots, heads, dim, vdim] is updated in place, and so are the q / k parts of qkv (made unit vectors);
-    returns o fp32 [rows, heads * vdim]; chunked: 16 tokens at a time, None where that form does not take the sizes"""
-    o = torch.empty((qkv_f32.shape[0], heads * vdim), dtype=torch.float32, device=proj.device)
+    returns o fp32 [rows, heads * vdim]; chunked: entries of more than scan_max rows 16 tokens at a time, None where that form does not take the sizes"""
+    L, T = ffi.lib(), qkv_f32.shape[0]
+    o = torch.empty((T, heads * vdim), dtype=torch.float32, device=proj.device)
+    first = (_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log), _p(dt_bias))
+    last = (_p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim, T, _p(rg.entry_row0), _p(rg.entry_slot), rg.n)
     if chunked:
-        L, T = ffi.lib(), qkv_f32.shape[0]
         if not L.pegainfer_delta_rule_chunked_ok(dim, vdim, _p(qkv_f32), qkv_f32.stride(0)):
             return None
         ws = torch.empty(L.pegainfer_delta_rule_workspace(T, rg.n, heads), dtype=torch.float32, device=proj.device)
-        _chk(L.pegainfer_delta_rule_chunked(_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log), _p(dt_bias), _p(ws),
-                                            _p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim, T, _p(rg.entry_row0),
-                                            _p(rg.entry_slot), rg.n, _dt(proj), _stream()), "delta_rule_chunked")
-        return o
-    gates = torch.empty((qkv_f32.shape[0], 2 * heads), dtype=torch.float32, device=proj.device)
-    _chk(ffi.lib().pegainfer_delta_rule(_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log),
-                                        _p(dt_bias), _p(gates), _p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim,
-                                        qkv_f32.shape[0], _p(rg.entry_row0), _p(rg.entry_slot), rg.n, _dt(proj), _stream()),
-         "delta_rule")
+        _chk(L.pegainfer_delta_rule_chunked(*first, _p(ws), *last, scan_max, _dt(proj), _stream()), "delta_rule_chunked")
+    if not chunked or scan_max > 0:
+        gates = torch.empty((T, 2 * heads), dtype=torch.float32, device=proj.device)
+        if chunked:
+            _chk(L.pegainfer_delta_rule_short(*first, _p(gates), *last, scan_max, _dt(proj), _stream()), "delta_rule_short")
+        else:
+            _chk(L.pegainfer_delta_rule(*first, _p(gates), *last, _dt(proj), _stream()), "delta_rule")
     return o
 
 

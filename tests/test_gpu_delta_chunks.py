@@ -85,3 +85,25 @@ def test_chunks_let_nothing_reach_earlier_tokens(H, G, d, dv, what, bad):
             assert torch.equal(ok, torch.isfinite(b)), (at, int((ok != torch.isfinite(b)).sum()))
             if ok.any():
                 assert float((a[ok] - b[ok]).abs().max()) < 2e-5 * float(a[ok].abs().max()), at
+
+
+@pytest.mark.parametrize("lens,scan_max", [([1, 30, 200, 64, 0, 65], 64), ([17, 3, 16], 16), ([5, 6], 64), ([70, 90], 64)])
+def test_an_entry_takes_the_form_of_its_own_length(lens, scan_max):
+    """outputs, states and the rows made unit vectors: the bits that each entry has alone, token by token up to scan_max tokens and in chunks beyond"""
+    from pegainfer_amd import ops_blocks as B
+    H, G, d, dv = 6, 2, 128, 32
+    gen = torch.Generator().manual_seed(len(lens))
+    n, T = len(lens), sum(lens)
+    A, bias = torch.randn(H, generator=gen).cuda(), torch.randn(H, generator=gen).cuda()
+    qkv0, proj, mem = torch.randn(T, 2 * G * d + H * dv, generator=gen).cuda(), torch.randn(T, 2 * H, generator=gen).cuda(), torch.randn(n, H, d, dv, generator=gen).cuda()
+    qkv, st = qkv0.clone(), mem.clone()
+    got = B.delta_rule(qkv, proj, 0, H, A, bias, st, H, G, d, dv, B.Ragged(lens), chunked=True, scan_max=scan_max)
+    at = 0
+    for e, length in enumerate(lens):
+        rows, at = slice(at, at + length), at + length
+        if length == 0:
+            assert torch.equal(st[e], mem[e])
+            continue
+        own, own_st = qkv0[rows].clone(), mem[e:e + 1].clone()
+        alone = B.delta_rule(own, proj[rows].clone(), 0, H, A, bias, own_st, H, G, d, dv, B.Ragged([length]), chunked=length > scan_max)
+        assert torch.equal(got[rows], alone) and torch.equal(st[e], own_st[0]) and torch.equal(qkv[rows], own), e
