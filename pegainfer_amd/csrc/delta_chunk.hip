@@ -31,6 +31,9 @@ constexpr int kDcFloats = 2 * kDc * kDc + 2 * kDc + 32;  // of a (chunk, head): 
 // Chunks are numbered without a table: entry e's first is row0 / 16 + e (the next entry's first lies behind its last), so there are
 // rows / 16 + entries numbers at most and some that stand for none.
 __device__ __forceinline__ int delta_first_chunk(int row0, int e) { return row0 / kDc + e; }
+// A long step's chunks are walked in runs, one behind the other, whose matrices take 256 MB at most (or one chunk's): 3640 chunks at 32 heads.
+constexpr int64_t kDcRunFloats = (int64_t)1 << 26;
+static int64_t delta_chunk_run(int64_t chunks, int heads) { return std::max<int64_t>(1, std::min(chunks, kDcRunFloats / ((int64_t)heads * kDcFloats))); }
 
 // A wave per (chunk, key head): k . k and q . k of the chunk's tokens, then, sixteen lanes per value head, the triangular matrix and its inverse
 // by forward substitution, a lane per column.
@@ -38,12 +41,12 @@ template <typename A, int NB>
 __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                                int64_t proj_stride, int64_t b_off, int64_t a_off, const A* __restrict__ A_log,
                                                                const A* __restrict__ dt_bias, float* __restrict__ ws, int H, int G,
-                                                               const int32_t* __restrict__ entry_row0, int n_entries, int scan_max) {
+                                                               const int32_t* __restrict__ entry_row0, int n_entries, int scan_max, int run0) {
   constexpr int DIM = 64 * NB;
   __shared__ float s_kk[4][kDc][kDc + 1], s_qk[4][kDc][kDc + 1];
   __shared__ __attribute__((aligned(16))) float s_l[4][4][kDc][kDc + 4], s_gb[4][4][kDc][2];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = lane & 15, j = lane >> 4;
-  const int chunk = blockIdx.x, g = blockIdx.y * 4 + wave;
+  const int chunk = run0 + blockIdx.x, g = blockIdx.y * 4 + wave;
   int lo = 0, hi = n_entries - 1;              // the last entry whose first chunk is not behind this one
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
     s_gb[wave][j][t][0] = gt;
     s_gb[wave][j][t][1] = bt;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // a wave's own LDS writes, in its own order
-    float* out = ws + ((int64_t)chunk * H + h) * kDcFloats;
+    float* out = ws + ((int64_t)blockIdx.x * H + h) * kDcFloats;
     // lane: column t of head h; p = D[row][t]
     float p = 0.f;
 #pragma unroll
@@ -149,15 +152,23 @@ constexpr int kDcThreads = 320;
 template <int NB>
 __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qkv, int qkv_stride, const float* ws, float* __restrict__ state,
                                                                  int64_t slot_stride, float* __restrict__ o, int H, int G, int vdim,
-                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot, int scan_max) {
+                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot, int scan_max, int run0, int run) {
   constexpr int DIM = 64 * NB;
   __shared__ f32x4 s_part[2][4][2][64];        // K S0 and Q S0 over a wave's rows of S
   __shared__ f32x4 s_common[2][4][64];         // by lane: values, T', c, D[15][.]
   __shared__ float s_end[2];
   const int e = blockIdx.z, h = blockIdx.y, col = blockIdx.x * 16 + (threadIdx.x & 15);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l15 = lane & 15, j = lane >> 4;
-  const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
+  int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
   if (len <= scan_max) return;                 // (0: empty ones)
+  int place = delta_first_chunk(row0, e) - run0;               // of the entry's first chunk in this run
+  {
+    const int from = max(-place, 0), to = min((len + kDc - 1) / kDc, run - place);
+    if (from >= to) return;
+    row0 += from * kDc;
+    len = min(len, to * kDc) - from * kDc;
+    place += from;
+  }
   const int n = (len + kDc - 1) / kDc, g0 = h / (H / G);
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };     // (not the loads of the chunks ahead)
   // rows past the entry's end: its last one, which T' leaves out
@@ -212,7 +223,7 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
     if (c + 2 < n) work(z, c + 2, std::false_type());
   };
   if (wave == 4) {
-    const float *w0 = ws + ((int64_t)delta_first_chunk(row0, e) * H + h) * kDcFloats, *v0 = qkv + (int64_t)2 * G * DIM + (int64_t)h * vdim + col;
+    const float *w0 = ws + ((int64_t)place * H + h) * kDcFloats, *v0 = qkv + (int64_t)2 * G * DIM + (int64_t)h * vdim + col;
     struct Chunk { f32x4 v, T, M, decay, left; float end; } x, y, z;
     auto fetch = [&](Chunk& x, int c) {
       // asked for here and in this order: the compiler would gather the loads of three chunks, whose waits are then one (the pointers are not
@@ -322,7 +333,7 @@ extern "C" {
 using namespace pk;
 
 int64_t pegainfer_delta_rule_workspace(int32_t n_rows, int32_t n_entries, int32_t heads) {
-  return ((int64_t)n_rows / kDc + n_entries) * heads * kDcFloats;
+  return n_rows <= 0 || n_entries <= 0 || heads <= 0 ? 0 : delta_chunk_run((int64_t)n_rows / kDc + n_entries, heads) * heads * kDcFloats;
 }
 
 int32_t pegainfer_delta_rule_chunked_ok(int32_t dim, int32_t vdim, const float* qkv, int64_t qkv_stride) {
@@ -340,16 +351,19 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
       !pegainfer_delta_rule_chunked_ok(dim, vdim, qkv, qkv_stride))
     return bad;
   hipStream_t st = as_stream(stream);
-  const dim3 prep(n_rows / kDc + n_entries, ceil_div(kv_heads, 4)), grid(vdim / 16, heads, n_entries);
+  const int chunks = n_rows / kDc + n_entries, run = (int)delta_chunk_run(chunks, heads);
   const bool known = by_dtype(dtype, [&](auto* ptr) {
     using A = std::remove_pointer_t<decltype(ptr)>;
     by_rows_of_s(dim, [&](auto nb) {
       constexpr int NB = decltype(nb)::value;
-      delta_chunk_prep_kernel<A, NB><<<prep, 256, 0, st>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off,
-                                                           static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace, heads, kv_heads,
-                                                           entry_row0, n_entries, scan_max);
-      delta_chunk_kernel<NB><<<grid, kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads, vdim, entry_row0, entry_slot,
-                                                     scan_max);
+      for (int c = 0; c < chunks; c += run) {
+        const int n = std::min(run, chunks - c);
+        delta_chunk_prep_kernel<A, NB><<<dim3(n, ceil_div(kv_heads, 4)), 256, 0, st>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off,
+                                                                                       static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace,
+                                                                                       heads, kv_heads, entry_row0, n_entries, scan_max, c);
+        delta_chunk_kernel<NB><<<dim3(vdim / 16, heads, n_entries), kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads,
+                                                                                         vdim, entry_row0, entry_slot, scan_max, c, n);
+      }
     });
   });
   return known ? (pegainfer_status_t)hipGetLastError() : bad;

@@ -697,11 +697,12 @@ struct Model {
         if (l.mm.heads > 0) need = std::max(need, (size_t)pegainfer_gated_matrix_memory_workspace(n, l.mm.heads, l.mm.dim, l.mm.vdim));
     return grow_scratch(chunk_ws, need);
   }
+  bool delta_in_chunks(const LayerCfg& c) const { return pegainfer_delta_rule_chunked_ok(c.dl.dim, c.dl.vdim, qkv32, c.conv_ch); }
   // room for the delta rule of a step with prompts 16 tokens at a time; false: token by token
   bool ensure_delta(int64_t rows, int entries) {
     size_t need = 0;
     for (auto& l : layers)
-      if (l.type == kDelta) need = std::max(need, (size_t)pegainfer_delta_rule_workspace((int32_t)rows, entries, l.dl.heads));
+      if (l.type == kDelta && delta_in_chunks(l)) need = std::max(need, (size_t)pegainfer_delta_rule_workspace((int32_t)rows, entries, l.dl.heads));
     return need > 0 && grow_scratch(delta_ws, need);
   }
   bool grow_scratch(pq::OptionalScratch& ws, size_t need) {
@@ -994,7 +995,7 @@ struct Model {
         if (single && !plain_kernels && pegainfer_recurrent_step_ok(&q)) {       // preparation, scan, norm and gate in one launch
           FZ_K(pegainfer_recurrent_step(&q, S()));
         } else {
-          if (delta_chunks && pegainfer_delta_rule_chunked_ok(d.dim, d.vdim, qkv32, c.conv_ch)) {
+          if (delta_chunks && delta_in_chunks(c)) {
             FZ_K(pegainfer_delta_rule_chunked(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
                                               o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, kDeltaScanMax, dtype, S()));
             if (delta_short)

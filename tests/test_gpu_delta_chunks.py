@@ -107,3 +107,22 @@ def test_an_entry_takes_the_form_of_its_own_length(lens, scan_max):
         own, own_st = qkv0[rows].clone(), mem[e:e + 1].clone()
         alone = B.delta_rule(own, proj[rows].clone(), 0, H, A, bias, own_st, H, G, d, dv, B.Ragged([length]), chunked=length > scan_max)
         assert torch.equal(got[rows], alone) and torch.equal(st[e], own_st[0]) and torch.equal(qkv[rows], own), e
+
+
+def test_a_long_step_in_runs_of_bounded_scratch():
+    """256 MB hold 455 chunks of 256 heads: the last entry's lie on both sides of the cut, and have the bits of a run of their own"""
+    from pegainfer_amd import ffi
+    from pegainfer_amd import ops_blocks as B
+    need = ffi.lib().pegainfer_delta_rule_workspace
+    assert need(10 ** 6, 1, 32) * 4 <= 256 << 20 and need(10 ** 6, 9, 32) == need(2 * 10 ** 6, 9, 32) and need(1, 1, 10 ** 6) >= 10 ** 6
+    H, G, d, dv, lens = 256, 1, 64, 16, [7000, 40, 900]
+    assert need(sum(lens), len(lens), H) < need(sum(lens), len(lens), H // 2) * 2
+    g = torch.Generator(device="cuda").manual_seed(1)
+    T = sum(lens)
+    qkv, proj = (torch.randn(T, w, device="cuda", generator=g) for w in (2 * G * d + H * dv, 2 * H))
+    A, bias, mem = torch.zeros(H, device="cuda"), torch.full((H,), -3.0, device="cuda"), torch.randn(3, H, d, dv, device="cuda", generator=g)
+    st, own_st = mem.clone(), mem[2:].clone()
+    own, own_proj = qkv[-900:].clone(), proj[-900:].clone()
+    got = B.delta_rule(qkv, proj, 0, H, A, bias, st, H, G, d, dv, B.Ragged(lens), chunked=True)
+    alone = B.delta_rule(own, own_proj, 0, H, A, bias, own_st, H, G, d, dv, B.Ragged([900]), chunked=True)
+    assert torch.equal(got[-900:], alone) and torch.equal(st[2], own_st[0])
