@@ -206,9 +206,10 @@ template <int N, int NB>
 struct RouteTail {
   static constexpr int kWaves = N / 64, P = N >= 1024 ? 4 : 8;      // pieces in flight per block; with 1024 threads a row has up to eight
   struct Shared {
-    uint16_t row[N * 4];
-    float part[kWaves][NB * 16];
+    alignas(16) uint16_t row[N * 4];                    // both are read or written 16 bytes at a time
+    alignas(16) float part[kWaves][NB * 16];
   };
+  static_assert(alignof(Shared) % 16 == 0 && sizeof(Shared::row) % 16 == 0 && sizeof(Shared::part[0]) % 16 == 0, "16-byte accesses");
   u32x4 w[P][NB];
   // a workgroup without a row (the first few have none either: they fill the round of XCDs that the rows begin)
   static __device__ __forceinline__ bool helps(const RouterTail& t, int d) {
