@@ -1412,8 +1412,9 @@ static pegainfer_status_t paged_attention(const float* q, const void* cache, int
   if (dtype == kDtBf16 && !plain) {   // bf16 cache: the matrix-core kernel; same tiles, same splits, same merge
     const int ncb = vdim <= 32 ? 2 : vdim <= 64 ? 4 : vdim <= 128 ? 8 : 16;
     const size_t lds = mfma_attention_lds(maps, dim, ncb);
-    auto launch_as = [&](auto kern, dim3 blocks, int threads, auto... more) {
-      if (lds > 48 * 1024 &&
+    // own: what the kernel has besides, at most; 64 KB in all need no request
+    auto launch_as = [&](auto kern, dim3 blocks, int threads, size_t own, auto... more) {
+      if (lds + own > 64 * 1024 &&
           hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         ok = false;
         return;
@@ -1423,10 +1424,10 @@ static pegainfer_status_t paged_attention(const float* q, const void* cache, int
                                                         tile_row0, tile_ntok, tile_qh0, tile_nqh, static_cast<uint16_t*>(out), out_stride, form,
                                                         n_split, workspace, more...);
     };
-    auto launch = [&](auto kern) { launch_as(kern, grid, 256); };
+    auto launch = [&](auto kern) { launch_as(kern, grid, 256, 16 * 1024); };
     if (const pegainfer_recurrent_step_desc* step = opt->beside) {
       const dim3 blocks((unsigned)((int64_t)n_tiles * kv_heads * n_split + (int64_t)step->heads * step->n_entries));
-      auto both = [&](auto kern) { launch_as(kern, blocks, kStepThreads, (int)n_tiles, *step); };
+      auto both = [&](auto kern) { launch_as(kern, blocks, kStepThreads, 16 * 1024, (int)n_tiles, *step); };
       if (ncb == 2) both(paged_attention_beside_kernel<2>);
       else if (ncb == 4) both(paged_attention_beside_kernel<4>);
       else if (ncb == 8) both(paged_attention_beside_kernel<8>);
@@ -1435,7 +1436,7 @@ static pegainfer_status_t paged_attention(const float* q, const void* cache, int
       const pegainfer_ssd_scan_desc& scan = *d->scan;
       const int nbx = ceil_div(scan.vdim, kRecCols);
       const dim3 blocks((unsigned)((int64_t)n_tiles * kv_heads * n_split + (int64_t)nbx * scan.heads * scan.n_entries));
-      auto both = [&](auto kern) { launch_as(kern, blocks, 256, (int)n_tiles, scan, nbx); };
+      auto both = [&](auto kern) { launch_as(kern, blocks, 256, 24 * 1024, (int)n_tiles, scan, nbx); };
       auto by_states = [&](auto cols) {
         constexpr int NCB = decltype(cols)::value;
         if (scan.n_state > 64) both(paged_attention_scan_kernel<NCB, 8>);
