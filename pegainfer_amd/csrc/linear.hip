@@ -614,17 +614,33 @@ static int small_tile_unsplit(int M, int T, int K) {
 }
 constexpr int kSplitKMaxRows = 16384;   // below this (< 128 row tiles) the 17..64-column GEMM splits K
 struct SplitKPlan { int ksplit, nk_slice, tt; };
+// A short K is over before its slices' sums would be: whole tiles of 128 rows x 64 tokens take 3.5 us + 7.3 us per 1024 of K while every one has a
+// compute unit (with more, a round of them), the split forms 9 - 13 us at 160 tokens, 13 - 20 at 300 and 19 - 26 from 1000 on, a third of it the
+// sum.  But a product that an addition and a norm follow (pegainfer_gemm_add_rms_norm and the like) has the same route, so as to have the same bits, and
+// there the sum's launch is the norm's: whole tiles cost it a launch more.  So the line lies where neither loses.  Cold weights, split / whole (us):
+//                                       the product alone    with addition and norm
+//   K <= 1024   1024 x 512, 160 tokens   8.2 / 7.2            9.1 / 10.3
+//               2560 x 512, 300         13.4 / 7.6           15.2 / 11.8
+//               1024 x 1024, 1024       18.5 / 11.0          20.9 / 14.6
+//               2560 x 1024, 200        1.04 x               0.81 x
+//               2560 x 1024, 300        15.1 / 11.0          16.9 / 15.3
+//               6144 x 1024, 300; 512   21.8 / 11.6; 1.78 x  24.9 / 22.6; 0.91 x
+//   K <= 2048   2048 x 2048, 300; 1024  1.00 x; 25.8 / 18.5  0.89 x; 27.2 / 23.7
+//               1280 x 2048, 512        19.8 / 17.8          20.9 / 21.4
+//               2560 x 2048, 256; 512   0.93 x; 23.3 / 18.2  0.79 x; 24.2 / 23.0
+//               3072 x 2048, 1024       0.99 x               0.87 x
+static bool short_k_whole(int M, int T, int K) {
+  const int m_tiles = ceil_div(M, BM);
+  const long tiles = (long)m_tiles * ceil_div(T, 64);
+  if (K <= 1024) return T > 256 && (K <= 512 || tiles >= 80) && (m_tiles <= 40 || tiles <= 320);
+  return K <= 2048 && T >= 512 && tiles >= (K <= 1536 ? 80 : 96) && (tiles <= 256 || m_tiles <= (K <= 1536 ? 24 : 16));
+}
 static SplitKPlan splitk_plan(int M, int T, int K, bool assume_ws = false) {
   static const bool enabled = [] { const char* e = getenv("PEGAINFER_SPLITK"); return !(e && e[0] == '0'); }();
   if (!enabled || (!g_splitk_ws && !assume_ws) || T <= 16) return {0, 0, 0};
   const int m_tiles = ceil_div(M, BM), nk_all = K / BK;
   if (T > 64) {
-    // A short K is over before its slices' sums would be: whole tiles of 128 rows x 64 tokens take 3.5 us + 7.3 us per 1024 of K while every one has a
-    // compute unit (with more, a round of them), the split forms 9 - 13 us at 160 tokens, 13 - 20 at 300 and 19 - 26 from 1000 on, a third of it the
-    // sum.  Split / whole, cold weights (us): 1024 x 512 and 160 tokens 8.7 / 7.6; 1024 x 1024 and 1024 18.6 / 11.0, and 3000 25.5 / 15.0; 2048 x 2048
-    // and 600 22.5 / 18.4, and 1024 24.2 / 19.2, and 2404 26.3 / 26.6; but 2048 x 1024 and 160 tokens (48 tiles) 9.9 / 11.0, 2048 x 2560 and 300
-    // 20.3 / 23.0, 2560 x 2560 and 1024 28.0 / 32.7.
-    if (K <= 512 || (K <= 2048 && (long)m_tiles * ceil_div(T, 64) >= 80)) return {0, 0, 0};
+    if (short_k_whole(M, T, K)) return {0, 0, 0};
     // long-K matrices at ~1.3-3 k tokens (down_proj: 50-128 tiles of 256 x 256): the 8-phase kernel over 2-5 K
     // slices, one workgroup per CU (tt == 256 marks this plan; PEGAINFER_SPLITK256=0 switches it off).  Same-box A/B of
     // TTFT: 2048 tokens 23.05 -> 21.4 ms; 1024 tokens (40 tiles, 6 slices: 63 MB of partials each way) 12.60 vs 12.56,

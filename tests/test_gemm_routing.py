@@ -155,3 +155,13 @@ def test_rows_behind_the_full_rounds_of_large_tiles():
     assert tail(6144, 4096, 2560) == (0, 0)            # 384: half a round more
     assert tail(6144, 10000, 2560) == (0, 0)
     assert tail(2560, 1024, 9728) == (0, 0)            # K split over workgroups
+
+
+@pytest.mark.parametrize("M,T,K,whole", [
+    (1024, 256, 512, False), (1024, 257, 512, True), (5120, 512, 512, True), (512, 1217, 1024, True), (512, 1216, 1024, False), (2560, 256, 1024, False),
+    (2560, 257, 1024, True), (5120, 512, 1024, True), (6144, 300, 1024, True), (6144, 512, 1024, False), (2560, 511, 1056, False), (2560, 512, 1056, True),
+    (3072, 777, 1536, True), (3200, 700, 1536, False), (1280, 512, 1536, True), (1280, 512, 2048, False), (1280, 577, 2048, True), (2048, 1024, 2048, True),
+    (2048, 1500, 2048, True), (2176, 1024, 2048, False), (2560, 640, 2048, True), (1024, 700, 2048, False), (2048, 1024, 2112, False)])
+def test_a_short_k_is_not_split_where_no_call_loses_by_it(route, M, T, K, whole):
+    """each line of the rule from both sides: 128-row x 64-token tiles in all, rows of them, tokens"""
+    assert (route(M, T, K)[1] == 1) == whole, route(M, T, K)
