@@ -1155,9 +1155,10 @@ int32_t pegainfer_latent_prep_absorb_ok(const pegainfer_latent_prep_desc* d, con
       g->groups <= 0 || g->groups > 65535 || g->epilogue != PEGAINFER_EPI_NONE || g->rows != d->n_tokens || g->x_dtype != d->dtype || g->w_dtype != d->dtype ||
       g->y_dtype != kDtF32 || !chunks_ok(*g))
     return 0;
-  // the forms that these rows take by themselves, so the same bits; of fp32 up to two outputs per wave (beyond, the product fills the chip by itself)
+  // the forms that these rows take by themselves, so the same bits; of fp32 up to four outputs per wave of the chip (beyond, the product fills it by
+  // itself)
   if (d->dtype == kDtBf16) return g->rows <= kRowsMax;
-  return d->dtype == kDtF32 && g->rows <= 4 && rows_direct_outputs(*g, g->rows == 3 ? 4 : g->rows, false) <= 2;
+  return d->dtype == kDtF32 && g->rows <= 4 && rows_direct_all(*g, g->rows == 3 ? 4 : g->rows) < 16L * device_cus();
 }
 
 pegainfer_status_t pegainfer_latent_prep_absorb(const pegainfer_latent_prep_desc* d, const pegainfer_gemm_desc* g, pegainfer_stream_t stream) {
@@ -1174,7 +1175,7 @@ pegainfer_status_t pegainfer_latent_prep_absorb(const pegainfer_latent_prep_desc
     if (f.ob == 2) go(latent_prep_absorb_kernel<2>);
     else go(latent_prep_absorb_kernel<1>);
   } else {
-    const int R = g->rows == 3 ? 4 : g->rows, mb = rows_direct_outputs(*g, R, false);
+    const int R = g->rows == 3 ? 4 : g->rows, mb = std::min(2, rows_direct_outputs(*g, R, false));
     const int gy = ceil_div(g->m, 4 * mb), n_gemm = gy * g->groups;
     auto go = [&](auto kern) { kern<<<n_gemm + n_prep, 256, 0, st>>>(latent_prep_parts<float>(d), place, static_cast<float*>(d->cache), ny, *g, gy, n_gemm); };
     auto by_outputs = [&](auto r) {

@@ -14,10 +14,10 @@ namespace pk {
 // No LDS and no barrier: a wave takes MB outputs (GLU: MB pairs of a gate row and its up row), lanes over k four values at a time, and fetches the rows
 // it multiplies with beside the weights, pieces of 512 k two ahead of the products.  An output's k order is fixed by K alone.
 // Bound by one memory latency behind the launch with few outputs and by the stream of weights with many.  With the rows in LDS first (a barrier
-// before any product, 32-byte strides between lanes), 1 / 2 / 4 rows: 1024 x 1024 3.3 / 4.1 / 5.3 -> 3.1 / 3.4 / 3.9 us, 1024 x 3072
-// 5.7 / 7.4 / 10.2 -> 4.9 / 6.1 / 7.0, 3072 x 1024 4.8 / 6.3 / 8.3 -> 4.5 / 4.9 / 6.3, 6144 x 1024 7.0 / 8.3 / 10.4 -> 7.3 / 8.0 / 9.7,
-// 32 768 x 1024 25.9 / 32.2 / 34.2 -> 25.3 / 25.8 / 28.2 (5.2 TB/s); on the fp32 matrix cores 2048 x 8192 takes 26.9 with two rows, 16.3 here.
-// Four outputs a wave where that leaves every SIMD a wave, then two, then one.
+// before any product, 32-byte strides between lanes), 1 / 2 / 4 rows and cold weights: 1024 x 1024 3.4 / 4.2 / 5.5 -> 3.3 / 3.3 / 3.7 us, 1024 x 2048
+// 4.2 / 5.4 / 7.4 -> 4.0 / 4.1 / 4.9, 3072 x 1024 5.1 / 6.3 / 8.3 -> 4.6 / 4.8 / 5.9, 6144 x 1024 7.3 / 8.2 / 10.3 -> 6.3 / 6.6 / 8.5,
+// 32 768 x 1024 25.9 / 31.3 / 32.2 -> 21.0 / 21.2 / 24.6 (6.4 TB/s); on the fp32 matrix cores 2048 x 8192 took 28.2 with two rows, 14.1 here.  One fp32
+// row against bf16 weights 65 536 x 2048: 54.9 -> 39.4.
 // a lane's eight values of a piece of 512, in one or two loads that are whole lines over the wave
 template <typename TW>
 struct DirectPiece;
@@ -126,31 +126,37 @@ __device__ __forceinline__ void gemm_rows_direct_block(const pegainfer_gemm_desc
     compute(p + CH, B);
     if (p + 3 * CH < np) issue(p + 3 * CH, B);
   }
+  // Sums over each 16 lanes, of which lane r MB + q keeps those of output q of row r: the way over the four runs of lanes, and what follows, is then one
+  // for all (each sum by itself as in wave_sum, whose steps these are, and stored by one lane: four rows of 65 536 x 256 24.9 -> 19.3 us).
+  static_assert(MB * R <= 16, "a lane of sixteen per sum");
+  float v = 0.f, u = 0.f;
 #pragma unroll
-  for (int q = 0; q < MB; ++q)
-#pragma unroll
-    for (int n = 0; n < NW; ++n)
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[q][n][r] = wave_sum(acc[q][n][r]);
-  if (lane != 0) return;
-  TY* Y = static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (r >= nrows) break;
-    const int yr = d.y_row_index ? d.y_row_index[row0 + r] : row0 + r;
+  for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int q = 0; q < MB; ++q) {
-      const int m = m0 + q;
-      if (m >= d.m) break;
-      float v = acc[q][0][r];
-      if constexpr (GLU) v = act_f(act, v) * acc[q][1][r];
-      else if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
-      else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
-      else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
-        v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)x_row(r) * d.gate_row_stride + g));
-      st(Y + (int64_t)yr * d.y_row_stride + m, v);
+      const bool mine = (lane & 15) == r * MB + q;
+      const float t = row16_sum(acc[q][0][r]);
+      v = mine ? t : v;
+      if constexpr (GLU) {
+        const float t2 = row16_sum(acc[q][1][r]);
+        u = mine ? t2 : u;
+      }
     }
+  v += __shfl_xor(v, 16, kWave);
+  v += __shfl_xor(v, 32, kWave);
+  if constexpr (GLU) {
+    u += __shfl_xor(u, 16, kWave);
+    u += __shfl_xor(u, 32, kWave);
   }
+  const int r = lane / MB, m = m0 + lane % MB;
+  if (r >= nrows || m >= d.m) return;
+  if constexpr (GLU) v = act_f(act, v) * u;
+  else if (d.epilogue == PEGAINFER_EPI_RELU_SQ) { v = fmaxf(v, 0.f); v *= v; }
+  else if (d.epilogue == PEGAINFER_EPI_GELU_ERF) v = gelu_erf_f(v);
+  else if (d.epilogue == PEGAINFER_EPI_SIGMOID_GATE)
+    v *= sigmoid_f(ld(static_cast<const TG*>(d.gate) + (int64_t)x_row(r) * d.gate_row_stride + g));
+  const int yr = d.y_row_index ? d.y_row_index[row0 + r] : row0 + r;
+  st(static_cast<TY*>(d.y) + (int64_t)g * d.y_group_stride + (int64_t)yr * d.y_row_stride + m, v);
 }
 
 // ------------------------------------------------------------------ few-rows form on the matrix cores (bf16 weights, decode)
@@ -470,11 +476,24 @@ inline RowsMfmaShape rows_mfma_shape(const pegainfer_gemm_desc& d) {
   const bool two = (long)row_tiles * groups * blocks >= 4L * device_cus();
   return {wk, two ? 2 : 1, dim3(row_tiles, two ? ceil_div(blocks, 2) : blocks, groups)};
 }
-// outputs of a wave of the direct form: four where that leaves every SIMD a wave, then two, then one
+inline long rows_direct_all(const pegainfer_gemm_desc& d, int R) {
+  return (long)(d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R)) * (d.tile_group ? 1 : d.groups) * d.m;
+}
+// Outputs of a wave of the direct form: the more, the fewer workgroups come and go and the more often a row's values are used; the fewer, the more
+// of a long row of weights is on its way.  So four from three outputs per wave of the chip on while a weight row is one piece (2 KB), for longer ones two, four
+// where three or four rows and many outputs use them, and one where a single row needs nothing but weights.  One / two / four (us):
+//   one row    16 384 x 256 9.9 / 7.0 / 5.3       16 384 x 1024 12.9 / 11.7 / 13.0   4096 x 8192 22.8 / 25.6 / 32.2
+//   two rows   16 384 x 256 10.9 / 8.6 / 5.8      16 384 x 1024 13.8 / 12.3 / 13.8   4096 x 8192 26.6 / 25.8 / 32.7
+//   four rows  16 384 x 256 15.4 / 12.7 / 7.5     16 384 x 1536 28.8 / 24.4 / 19.1   4096 x 8192 36.1 / 27.1 / 35.0
 inline int rows_direct_outputs(const pegainfer_gemm_desc& d, int R, bool glu) {
-  const int row_tiles = d.tile_group ? d.max_tiles | 1 : ceil_div(d.rows, R), groups = d.tile_group ? 1 : d.groups;
-  const long outputs = (long)row_tiles * groups * d.m, waves = 4L * device_cus();
-  return !glu && outputs >= 4 * waves ? 4 : outputs >= 2 * waves ? 2 : 1;
+  const long outputs = rows_direct_all(d, R), waves = 4L * device_cus();
+  if (glu) return outputs >= 2 * waves ? 2 : 1;
+  if (2 * outputs < 3 * waves) return 1;
+  const bool f32 = d.w_dtype == kDtF32;
+  const int words = f32 ? d.k : d.k / 2;                  // of a weight row
+  if (words <= 512) return outputs >= 3 * waves ? 4 : 2;
+  if (R == 1 && f32 && words >= 2048) return 1;
+  return R > 2 && words <= 4096 && outputs >= 8 * waves ? 4 : 2;
 }
 // operands in 16-byte chunks
 inline bool chunks_ok(const pegainfer_gemm_desc& d) {

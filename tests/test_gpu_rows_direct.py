@@ -52,6 +52,19 @@ def test_gated_unit_of_few_fp32_rows(act, T, M, K):
     assert float((y.double() - f(a) * u).abs().max()) <= 1e-6 * (K ** 0.5 + 8) * float(1 + z.abs().max()) * 2
 
 
+@pytest.mark.parametrize("wd,T", [(torch.float32, 1), (torch.float32, 2), (torch.float32, 4), (torch.bfloat16, 1)])
+@pytest.mark.parametrize("M,K", [(3200, 264), (5000, 512), (9000, 1040), (8500, 4104), (4200, 2056)])
+def test_an_output_does_not_depend_on_how_many_a_wave_makes(wd, T, M, K):
+    """one, two or four outputs a wave by their number, the row's length and the rows: the bits of a launch of a few (one a wave), and double precision"""
+    from pegainfer_amd import ops_blocks as B
+    g = torch.Generator(device="cuda").manual_seed(M + T)
+    x, w = torch.randn(T, K, device="cuda", generator=g), torch.randn(M, K, device="cuda", generator=g).to(wd)
+    y = B.linear(x, w, out_dtype=torch.float32)
+    for at in (0, M // 2, M - 77):
+        assert torch.equal(y[:, at:at + 77], B.linear(x, w[at:at + 77].contiguous(), out_dtype=torch.float32)), at
+    assert float((y.double() - x.double() @ w.double().T).abs().max()) <= 1e-6 * K
+
+
 def test_other_gated_units_are_refused():
     from pegainfer_amd import ops_blocks as B
     x, w, y = torch.zeros(5, 64, device="cuda"), torch.zeros(16, 64, device="cuda"), torch.zeros(5, 8, device="cuda")
