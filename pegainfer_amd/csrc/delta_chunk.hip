@@ -19,6 +19,7 @@
 #include "common.h"
 #include "typed.h"
 #include "sigmoid_power.h"
+#include "delta_scan.h"
 #include "pegainfer_kernels_blocks.h"
 
 namespace pk {
@@ -37,12 +38,19 @@ static int64_t delta_chunk_run(int64_t chunks, int heads) { return std::max<int6
 
 // A wave per (chunk, key head): k . k and q . k of the chunk's tokens, then, sixteen lanes per value head, the triangular matrix and its inverse
 // by forward substitution, a lane per column.
-template <typename A, int NB>
+// MIXED: the entries of up to scan_max rows are prepared for the token-by-token form, by workgroups of their own behind the chunks'.
+template <typename A, int NB, bool MIXED>
 __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                                int64_t proj_stride, int64_t b_off, int64_t a_off, const A* __restrict__ A_log,
                                                                const A* __restrict__ dt_bias, float* __restrict__ ws, int H, int G,
-                                                               const int32_t* __restrict__ entry_row0, int n_entries, int scan_max, int run0) {
+                                                               const int32_t* __restrict__ entry_row0, int n_entries, int scan_max, int run0, int run, float* gates) {
   constexpr int DIM = 64 * NB;
+  if (MIXED && (int)blockIdx.x >= run) {
+    const int row = blockIdx.x - run, e = entry_of_row(entry_row0, n_entries, row);
+    if (entry_row0[e + 1] - entry_row0[e] <= scan_max)
+      delta_prep_row<A>(row, blockIdx.y, gridDim.y, qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, H, G, DIM);
+    return;
+  }
   __shared__ float s_kk[4][kDc][kDc + 1], s_qk[4][kDc][kDc + 1];
   __shared__ __attribute__((aligned(16))) float s_l[4][4][kDc][kDc + 4], s_gb[4][4][kDc][2];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = lane & 15, j = lane >> 4;
@@ -149,10 +157,11 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(float* __restrict
 // the next product's operand in the same way.  Vector memory takes 16 cycles an instruction whatever it carries, so what all four waves need is
 // fetched by a fifth, which also makes the outputs; nothing waits for those.  Operands are asked for two chunks ahead.
 constexpr int kDcThreads = 320;
-template <int NB>
+// MIXED: the workgroups of entries of up to scan_max rows go token by token, four of their five waves (a launch of its own would follow this one).
+template <int NB, bool MIXED>
 __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qkv, int qkv_stride, const float* ws, float* __restrict__ state,
                                                                  int64_t slot_stride, float* __restrict__ o, int H, int G, int vdim,
-                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot, int scan_max, int run0, int run) {
+                                                                 const int32_t* __restrict__ entry_row0, const int32_t* __restrict__ entry_slot, int scan_max, int run0, int run, const float* gates) {
   constexpr int DIM = 64 * NB;
   __shared__ f32x4 s_part[2][4][2][64];        // K S0 and Q S0 over a wave's rows of S
   __shared__ f32x4 s_common[2][4][64];         // by lane: values, T', c, D[15][.]
@@ -160,7 +169,13 @@ __global__ __launch_bounds__(kDcThreads) void delta_chunk_kernel(const float* qk
   const int e = blockIdx.z, h = blockIdx.y, col = blockIdx.x * 16 + (threadIdx.x & 15);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l15 = lane & 15, j = lane >> 4;
   int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
-  if (len <= scan_max) return;                 // (0: empty ones)
+  if (len <= scan_max) {                       // (0: empty ones)
+    if (MIXED && run0 == 0 && len > 0 && wave < 4) {
+      constexpr int NS = NB == 1 ? 4 : NB == 2 ? 8 : 16;       // as by_slices does
+      delta_rule_block<NS, false>(blockIdx.x, h, e, qkv, qkv_stride, gates, state, slot_stride, o, H, G, DIM, vdim, entry_row0, entry_slot);
+    }
+    return;
+  }
   int place = delta_first_chunk(row0, e) - run0;               // of the entry's first chunk in this run
   {
     const int from = max(-place, 0), to = min((len + kDc - 1) / kDc, run - place);
@@ -344,10 +359,10 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
                                                 int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
                                                 int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
                                                 int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
-                                                int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
+                                                int32_t scan_max, float* gates, int32_t dtype, pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (n_entries <= 0 || n_rows <= 0) return 0;
-  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || scan_max < 0 || !workspace || !host_aligned16(workspace) ||
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || scan_max < 0 || (scan_max > 0 && !gates) || !workspace || !host_aligned16(workspace) ||
       !pegainfer_delta_rule_chunked_ok(dim, vdim, qkv, qkv_stride))
     return bad;
   hipStream_t st = as_stream(stream);
@@ -356,14 +371,19 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
     using A = std::remove_pointer_t<decltype(ptr)>;
     by_rows_of_s(dim, [&](auto nb) {
       constexpr int NB = decltype(nb)::value;
-      for (int c = 0; c < chunks; c += run) {
-        const int n = std::min(run, chunks - c);
-        delta_chunk_prep_kernel<A, NB><<<dim3(n, ceil_div(kv_heads, 4)), 256, 0, st>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off,
-                                                                                       static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace,
-                                                                                       heads, kv_heads, entry_row0, n_entries, scan_max, c);
-        delta_chunk_kernel<NB><<<dim3(vdim / 16, heads, n_entries), kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads, kv_heads,
-                                                                                         vdim, entry_row0, entry_slot, scan_max, c, n);
-      }
+      auto go = [&](auto mixed) {
+        constexpr bool MIXED = decltype(mixed)::value;
+        for (int c = 0; c < chunks; c += run) {
+          const int n = std::min(run, chunks - c), rows = MIXED && c == 0 ? n_rows : 0;
+          delta_chunk_prep_kernel<A, NB, MIXED><<<dim3(n + rows, ceil_div(kv_heads, 4)), 256, 0, st>>>(
+              qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off, a_off, static_cast<const A*>(A_log), static_cast<const A*>(dt_bias), workspace,
+              heads, kv_heads, entry_row0, n_entries, scan_max, c, n, gates);
+          delta_chunk_kernel<NB, MIXED><<<dim3(vdim / 16, heads, n_entries), kDcThreads, 0, st>>>(qkv, (int)qkv_stride, workspace, state, slot_stride, o, heads,
+                                                                                                  kv_heads, vdim, entry_row0, entry_slot, scan_max, c, n, gates);
+        }
+      };
+      if (scan_max > 0) go(std::true_type());
+      else go(std::false_type());
     });
   });
   return known ? (pegainfer_status_t)hipGetLastError() : bad;

@@ -83,9 +83,10 @@ constexpr float kGluAlpha = 1.702f;  // the clamp-GLU's sigmoid slope, fixed by 
 // longest entry whose matrix memory runs token by token: 8 heads of 128 x 256, scan / chunks 42 / 48 us at 96 tokens, 54 / 50 at 128,
 // 222 / 65 at 512; eight entries of 64 tokens 57 / 62, of 128 96 / 71
 constexpr int kScanMax = 112;
-// longest entry whose delta rule runs token by token: 32 heads of 128 x 128, one entry of 32 tokens 14.6 / 17.4, of 64 20 / 19, of 128 32 / 27, of 1024 196 / 89 us token
-// by token / 16 at a time
-constexpr int kDeltaScanMax = 64;
+// Longest entry whose delta rule runs token by token.  Token by token / 16 at a time: 32 heads of 128 x 128, one entry of 65 tokens 22 / 23, of 97 27 / 26, of 129
+// 33 / 30, of 400 83 / 48 us, sixteen entries of 97 168 / 165, of 113 188 / 183; 32 heads of 192 x 128 one of 65 31 / 29; 64 heads of 64 x 64, sixteen entries
+// of 129 140 / 161, of 257 264 / 277, of 400 410 / 396, one of 129 26 / 23.  Wider states gain more by chunks, narrow ones are over sooner.
+inline int delta_scan_max(int dim) { return dim <= 64 ? 256 : dim <= 128 ? 112 : 64; }
 constexpr int kAttRows = 16;         // (token, query head) rows of one attention workgroup
 
 enum { kDelta = 1, kParallel = 2 };
@@ -697,12 +698,14 @@ struct Model {
         if (l.mm.heads > 0) need = std::max(need, (size_t)pegainfer_gated_matrix_memory_workspace(n, l.mm.heads, l.mm.dim, l.mm.vdim));
     return grow_scratch(chunk_ws, need);
   }
-  bool delta_in_chunks(const LayerCfg& c) const { return pegainfer_delta_rule_chunked_ok(c.dl.dim, c.dl.vdim, qkv32, c.conv_ch); }
+  bool delta_in_chunks(const LayerCfg& c, int longest) const {
+    return c.type == kDelta && longest > delta_scan_max(c.dl.dim) && pegainfer_delta_rule_chunked_ok(c.dl.dim, c.dl.vdim, qkv32, c.conv_ch);
+  }
   // room for the delta rule of a step with prompts 16 tokens at a time; false: token by token
-  bool ensure_delta(int64_t rows, int entries) {
+  bool ensure_delta(int64_t rows, int entries, int longest) {
     size_t need = 0;
     for (auto& l : layers)
-      if (l.type == kDelta && delta_in_chunks(l)) need = std::max(need, (size_t)pegainfer_delta_rule_workspace((int32_t)rows, entries, l.dl.heads));
+      if (delta_in_chunks(l, longest)) need = std::max(need, (size_t)pegainfer_delta_rule_workspace((int32_t)rows, entries, l.dl.heads));
     return need > 0 && grow_scratch(delta_ws, need);
   }
   bool grow_scratch(pq::OptionalScratch& ws, size_t need) {
@@ -847,8 +850,8 @@ struct Model {
     ptiles::Chunks chunks = ptiles::chunks(ids, lens, n, PEGAINFER_DECAY_CHUNK, has_memory() && !plain_kernels ? kScanMax : INT32_MAX);
     if (!ensure_chunks((int)chunks.row0.size())) chunks = ptiles::Chunks();   // no memory: the scan, which needs none, takes every entry
     // the delta rule's long entries in chunks, each by its own length
-    const bool delta_chunks = !single && !plain_kernels && *std::max_element(lens, lens + n) > kDeltaScanMax && ensure_delta(T, n);
-    const bool delta_short = *std::min_element(lens, lens + n) <= kDeltaScanMax;
+    const int longest = *std::max_element(lens, lens + n), shortest = *std::min_element(lens, lens + n);
+    const bool delta_chunks = !single && !plain_kernels && ensure_delta(T, n, longest);
     const std::vector<int32_t>* chunk_cols[4] = {&chunks.row0, &chunks.rows, &chunks.first, &chunks.slot};
     size_t chunk_off[4];
     for (int k = 0; k < 4; ++k) { chunk_off[k] = words; words += chunk_cols[k]->size(); }
@@ -995,12 +998,10 @@ struct Model {
         if (single && !plain_kernels && pegainfer_recurrent_step_ok(&q)) {       // preparation, scan, norm and gate in one launch
           FZ_K(pegainfer_recurrent_step(&q, S()));
         } else {
-          if (delta_chunks && delta_in_chunks(c)) {
+          if (delta_chunks && delta_in_chunks(c, longest)) {
+            const int scan_max = shortest <= delta_scan_max(d.dim) ? delta_scan_max(d.dim) : 0;
             FZ_K(pegainfer_delta_rule_chunked(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
-                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, kDeltaScanMax, dtype, S()));
-            if (delta_short)
-              FZ_K(pegainfer_delta_rule_short(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
-                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, kDeltaScanMax, dtype, S()));
+                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, scan_max, gates32, dtype, S()));
           } else {
             FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
                                       o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));

@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "typed.h"
+#include "delta_scan.h"
 #include "head_rms_core.h"
 #include "qk_prep_core.h"
 #include "recurrent_core.h"
@@ -31,48 +32,15 @@ namespace pk {
 
 __device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
 
-// the entry that holds a row: the last one that begins at or before it
-__device__ __forceinline__ int entry_of_row(const int32_t* __restrict__ entry_row0, int n_entries, int row) {
-  int lo = 0, hi = n_entries - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (entry_row0[mid] <= row) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// Per row, before the recurrence: q and k heads made unit vectors in place (x / sqrt(sum(x^2) + 1e-6), q also * dim^-1/2),
-// gates[row] = [g: heads | beta: heads].  A wave per head; a row's heads and gates are dealt over gridDim.y workgroups (few rows: as many
-// as its heads fill - one workgroup took 10.0 us for a row of 32 heads of 128, eight take 4.2 us; from 256 rows on one).
-// scan_max > 0: the rows of entries of up to that many alone.
 template <typename A>
 __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ qkv, int64_t qkv_stride, const A* __restrict__ proj,
                                                          int64_t proj_stride, int64_t b_off, int64_t a_off,
                                                          const A* __restrict__ A_log, const A* __restrict__ dt_bias,
-                                                         float* __restrict__ gates, int H, int G, int dim,
-                                                         const int32_t* __restrict__ entry_row0, int n_entries, int scan_max) {
-  const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (scan_max > 0) {
-    const int e = entry_of_row(entry_row0, n_entries, row);
-    if (entry_row0[e + 1] - entry_row0[e] > scan_max) return;      // the chunk form has this entry
-  }
-  float* qk = qkv + (int64_t)row * qkv_stride;
-  const float qs = 1.0f / sqrtf((float)dim);
-  for (int hh = blockIdx.y * 4 + wave; hh < 2 * G; hh += 4 * gridDim.y) {
-    float* x = qk + (int64_t)hh * dim;
-    float ss = 0.f;
-    for (int d = lane; d < dim; d += 64) ss = fmaf(x[d], x[d], ss);
-    const float sc = (hh < G ? qs : 1.0f) / sqrtf(wave_sum(ss) + 1e-6f);
-    for (int d = lane; d < dim; d += 64) x[d] *= sc;
-  }
-  const A* pr = proj + (int64_t)row * proj_stride;
-  for (int h = blockIdx.y * 256 + threadIdx.x; h < H; h += 256 * gridDim.y) {
-    gates[(int64_t)row * 2 * H + h] = expf(-expf(ld(A_log + h)) * softplus_f(ld(pr + a_off + h) + ld(dt_bias + h)));
-    gates[(int64_t)row * 2 * H + H + h] = sigmoid_f(ld(pr + b_off + h));
-  }
+                                                         float* __restrict__ gates, int H, int G, int dim) {
+  delta_prep_row<A>(blockIdx.x, blockIdx.y, gridDim.y, qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, H, G, dim);
 }
 
-// The same for a decay per (head, key channel): gates[row] = [g: heads * dim | beta: heads], the decay inputs come as an fp32
+// What delta_prep_row does for a decay per (head, key channel): gates[row] = [g: heads * dim | beta: heads], the decay inputs come as an fp32
 // matrix `a` ([rows][heads * dim] at stride a_stride: the output of a low-rank projection pair), dt_bias has heads * dim values.
 template <typename A>
 __global__ __launch_bounds__(256) void delta_prep_channel_kernel(float* __restrict__ qkv, int64_t qkv_stride,
@@ -97,160 +65,13 @@ __global__ __launch_bounds__(256) void delta_prep_channel_kernel(float* __restri
   for (int h = blockIdx.y * 256 + threadIdx.x; h < H; h += 256 * gridDim.y) gr[(int64_t)H * dim + h] = sigmoid_f(ld(pr + b_off + h));
 }
 
-// CH: the decay is one number per (head, key channel) - it scales the ROWS of S - and the gates row is laid out as
-// delta_prep_channel_kernel leaves it; otherwise one number per head ([g: heads | beta: heads]).
-// A chain of dependent steps with one wave per SIMD: whatever a step waits for beside its own arithmetic is lost time, so a round's gates
-// come with its q | k | v (asked for when the round began, they held the chain up for a trip to memory), four values per load
-// where the layout allows it, and a token's values leave LDS while the token before it is worked on.  Lane r's NS values lie in groups of
-// four 64 floats apart, so that the lanes of a row read neighbouring 16 bytes.  1024 tokens of 32 heads of 128 x 128: 202 -> 180 us,
-// 8 portions of 700 tokens at most with channel decays 169 -> 145 us.
 template <int NS, bool CH>
 __global__ __launch_bounds__(256) void delta_rule_kernel(const float* __restrict__ qkv, int64_t qkv_stride,
                                                          const float* __restrict__ gates, float* __restrict__ state,
                                                          int64_t slot_stride, float* __restrict__ o, int H, int G, int dim,
                                                          int vdim, const int32_t* __restrict__ entry_row0,
-                                                         const int32_t* __restrict__ entry_slot, int scan_max) {
-  constexpr int DP = kRecSlices * NS;
-  constexpr int V = NS >= 4 ? 4 : 1, NV = NS / V;      // values per load, loads of a thread
-  __shared__ __attribute__((aligned(16))) float s_k[kRecTokens][DP], s_q[kRecTokens][DP];
-  __shared__ __attribute__((aligned(16))) float s_gb[kRecTokens][2];
-  __shared__ float s_v[kRecTokens][kRecCols];
-  __shared__ __attribute__((aligned(16))) float s_gc[CH ? kRecTokens : 1][CH ? DP : 1];
-  const int64_t gs = CH ? (int64_t)H * dim + H : (int64_t)2 * H;   // floats of one gates row
-  const int e = blockIdx.z, h = blockIdx.y, col0 = blockIdx.x * kRecCols;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, cl = wave * 4 + (lane >> 4);
-  const int col = col0 + cl;
-  const int g0 = h / (H / G);
-  const int row0 = entry_row0[e], len = entry_row0[e + 1] - row0;
-  if (scan_max > 0 && len > scan_max) return;      // the chunk form has this entry
-  float* S_g = state + (int64_t)entry_slot[e] * slot_stride + (int64_t)h * dim * vdim;
-  float S[NS];
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    const int d = r * NS + i;
-    S[i] = d < dim && col < vdim ? S_g[(int64_t)d * vdim + col] : 0.f;
-  }
-  const bool vec = V == 4 && (dim & 3) == 0 && (qkv_stride & 3) == 0 && aligned16(qkv);
-  const bool vec_g = V == 4 && (dim & 3) == 0 && (gs & 3) == 0 && aligned16(gates);
-  // thread t serves token t / 16 of a round: values V (t % 16 + 16 j) + 0 .. V of its query, key and decays, column t % 16 of its value
-  const int ft = tid >> 4, part = tid & 15;
-  struct Round { float q[NS], k[NS], gc[CH ? NS : 1], v, g, b; } nxt;
-  auto fetch = [&](int t0) {           // rows past the entry's end and values past dim: some that are there, dropped by land()
-    const int64_t row = row0 + min(t0 + ft, len - 1);
-    auto take = [&](const float* p, bool wide, float (&x)[NS]) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int d = V * (part + 16 * j);
-        if (V == 4 && wide) {
-          ld4(p + (d < dim ? d : 0), &x[V * j]);
-        } else {
-#pragma unroll
-          for (int u = 0; u < V; ++u) x[V * j + u] = p[d + u < dim ? d + u : 0];
-        }
-      }
-    };
-    const float* base = qkv + row * qkv_stride;
-    take(base + (int64_t)g0 * dim, vec, nxt.q);
-    take(base + (int64_t)(G + g0) * dim, vec, nxt.k);
-    nxt.v = base[(int64_t)2 * G * dim + (int64_t)h * vdim + min(col0 + part, vdim - 1)];
-    if constexpr (CH) take(gates + row * gs + (int64_t)h * dim, vec_g, nxt.gc);
-    const float* gr = gates + (int64_t)(row0 + min(t0 + part, len - 1)) * gs + h;    // token t % 16 here: the first 16 threads keep it
-    nxt.g = CH ? 1.f : gr[0];
-    nxt.b = gr[CH ? (int64_t)H * dim : H];
-  };
-  // where value d of a row lies: lane d / NS holds it, as number d % NS
-  auto place = [](int d) { return NS > 4 ? (d % NS / 4) * 64 + d / NS * 4 + d % 4 : d; };
-  auto land = [&](int tc) {
-    const bool live = ft < tc;
-    auto put = [&](const float (&x)[NS], float* dst, float none) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int d = V * (part + 16 * j);
-        if constexpr (V == 4) {
-          f32x4 t;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) t[u] = live && d + u < dim ? x[4 * j + u] : none;
-          *reinterpret_cast<f32x4*>(dst + place(d)) = t;
-        } else {
-          dst[d] = live && d < dim ? x[j] : none;
-        }
-      }
-    };
-    put(nxt.q, s_q[ft], 0.f);
-    put(nxt.k, s_k[ft], 0.f);
-    if constexpr (CH) put(nxt.gc, s_gc[ft], 1.f);
-    s_v[ft][part] = live && col0 + part < vdim ? nxt.v : 0.f;
-    if (tid < kRecTokens) {   // rows past the entry's end: g = 1, beta = 0, zero key - a step that leaves S as it is
-      s_gb[tid][0] = tid < tc ? nxt.g : 1.f;
-      s_gb[tid][1] = tid < tc ? nxt.b : 0.f;
-    }
-  };
-  struct Token { float k[NS], q[NS], gc[CH ? NS : 1], v, g, b; };
-  auto read = [&](int tt, Token& x) {
-    auto row = [&](const float* src, float (&y)[NS]) {
-      if constexpr (V == 4) {
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-          const f32x4 t = *reinterpret_cast<const f32x4*>(src + j * 64 + r * 4);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) y[4 * j + u] = t[u];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NS; ++i) y[i] = src[r * NS + i];
-      }
-    };
-    row(s_k[tt], x.k);
-    if constexpr (CH) row(s_gc[tt], x.gc);
-    x.v = s_v[tt][cl];
-    x.g = s_gb[tt][0];
-    x.b = s_gb[tt][1];
-    row(s_q[tt], x.q);
-    asm volatile("" ::: "memory");     // asked for here, not where it is used
-  };
-  if (len > 0) fetch(0);
-#pragma unroll
-  for (int i = 0; i < NS; ++i) asm volatile("" : "+v"(S[i]));   // the state is waited for here: its wait must not land in the loop
-  for (int t0 = 0; t0 < len; t0 += kRecTokens) {
-    const int tc = min(kRecTokens, len - t0);
-    __syncthreads();
-    land(tc);
-    __syncthreads();
-    if (t0 + kRecTokens < len) fetch(t0 + kRecTokens);
-    float okeep = 0.f;
-    auto step = [&](int tt, const Token& x) {
-      float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        if constexpr (CH) S[i] *= x.gc[i]; else S[i] *= x.g;
-        if (i & 1) a1 = fmaf(S[i], x.k[i], a1); else a0 = fmaf(S[i], x.k[i], a0);
-      }
-      const float u = x.b * (x.v - row16_sum(a0 + a1));
-      float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        S[i] = fmaf(x.k[i], u, S[i]);
-        if (i & 1) o1 = fmaf(S[i], x.q[i], o1); else o0 = fmaf(S[i], x.q[i], o0);
-      }
-      const float oa = row16_sum(o0 + o1);
-      okeep = tt == r ? oa : okeep;      // lane r of the column keeps token r of the round
-    };
-    // two tokens per trip: a token's first product starts while the read-out of the one before it is still being summed
-    Token x, y;
-    read(0, x);
-    for (int t2 = 0; t2 < tc; t2 += 2) {
-      read(t2 + 1, y);
-      step(t2, x);
-      read((t2 + 2) & (kRecTokens - 1), x);
-      step(t2 + 1, y);
-    }
-    if (r < tc && col < vdim) o[(int64_t)(row0 + t0 + r) * ((int64_t)H * vdim) + (int64_t)h * vdim + col] = okeep;
-  }
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    const int d = r * NS + i;
-    if (d < dim && col < vdim) S_g[(int64_t)d * vdim + col] = S[i];
-  }
+                                                         const int32_t* __restrict__ entry_slot) {
+  delta_rule_block<NS, CH>(blockIdx.x, blockIdx.y, blockIdx.z, qkv, qkv_stride, gates, state, slot_stride, o, H, G, dim, vdim, entry_row0, entry_slot);
 }
 
 // a token's log input and forget gate
@@ -548,11 +369,11 @@ using namespace pk;
 // workgroups per row of the launches before the recurrence
 static int prep_parts(int rows, int heads) { return rows >= 256 ? 1 : std::max(1, std::min(ceil_div(heads, 4), 1024 / rows)); }
 
-static pegainfer_status_t delta_rule_launch(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
                                         int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
                                         int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
                                         int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
-                                        int32_t n_entries, int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
+                                        int32_t n_entries, int32_t dtype, pegainfer_stream_t stream) {
   if (n_entries <= 0 || n_rows <= 0) return 0;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > 256 || vdim <= 0 || heads > 65535 || n_entries > 65535)
     return PK_BAD;
@@ -560,36 +381,17 @@ static pegainfer_status_t delta_rule_launch(float* qkv, int64_t qkv_stride, cons
         using A = std::remove_pointer_t<decltype(t)>;
         delta_prep_kernel<A><<<dim3(n_rows, prep_parts(n_rows, 2 * kv_heads)), 256, 0, as_stream(stream)>>>(qkv, qkv_stride, static_cast<const A*>(proj), proj_stride, b_off,
                                                                     a_off, static_cast<const A*>(A_log),
-                                                                    static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim, entry_row0, n_entries, scan_max);
+                                                                    static_cast<const A*>(dt_bias), gates, heads, kv_heads, dim);
       }))
     return PK_BAD;
   const dim3 grid(ceil_div(vdim, kRecCols), heads, n_entries);
   if (!by_slices(dim, [&](auto ns) {
         delta_rule_kernel<decltype(ns)::value, false><<<grid, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, gates, state, slot_stride, o,
                                                                                     heads, kv_heads, dim, vdim, entry_row0,
-                                                                                    entry_slot, scan_max);
+                                                                                    entry_slot);
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();
-}
-
-pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
-                                        int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
-                                        int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
-                                        int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
-                                        int32_t n_entries, int32_t dtype, pegainfer_stream_t stream) {
-  return delta_rule_launch(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, state, slot_stride, o, heads, kv_heads, dim, vdim, n_rows,
-                           entry_row0, entry_slot, n_entries, 0, dtype, stream);
-}
-
-pegainfer_status_t pegainfer_delta_rule_short(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
-                                              int64_t a_off, const void* A_log, const void* dt_bias, float* gates, float* state,
-                                              int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
-                                              int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
-                                              int32_t n_entries, int32_t scan_max, int32_t dtype, pegainfer_stream_t stream) {
-  if (scan_max <= 0) return PK_BAD;
-  return delta_rule_launch(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, gates, state, slot_stride, o, heads, kv_heads, dim, vdim, n_rows,
-                           entry_row0, entry_slot, n_entries, scan_max, dtype, stream);
 }
 
 pegainfer_status_t pegainfer_delta_rule_channel(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride,
@@ -612,7 +414,7 @@ pegainfer_status_t pegainfer_delta_rule_channel(float* qkv, int64_t qkv_stride, 
   if (!by_slices(dim, [&](auto ns) {
         delta_rule_kernel<decltype(ns)::value, true><<<grid, 256, 0, as_stream(stream)>>>(qkv, qkv_stride, gates, state, slot_stride, o,
                                                                                           heads, kv_heads, dim, vdim, entry_row0,
-                                                                                          entry_slot, 0);
+                                                                                          entry_slot);
       }))
     return PK_BAD;
   return (pegainfer_status_t)hipGetLastError();

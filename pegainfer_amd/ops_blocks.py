@@ -296,17 +296,14 @@ def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_hea
     o = torch.empty((T, heads * vdim), dtype=torch.float32, device=proj.device)
     first = (_p(qkv_f32), qkv_f32.stride(0), _p(proj), proj.stride(0), b_off, a_off, _p(A_log), _p(dt_bias))
     last = (_p(state), state.stride(0), _p(o), heads, kv_heads, dim, vdim, T, _p(rg.entry_row0), _p(rg.entry_slot), rg.n)
+    gates = torch.empty((T, 2 * heads), dtype=torch.float32, device=proj.device) if not chunked or scan_max > 0 else None
     if chunked:
         if not L.pegainfer_delta_rule_chunked_ok(dim, vdim, _p(qkv_f32), qkv_f32.stride(0)):
             return None
         ws = torch.empty(L.pegainfer_delta_rule_workspace(T, rg.n, heads), dtype=torch.float32, device=proj.device)
-        _chk(L.pegainfer_delta_rule_chunked(*first, _p(ws), *last, scan_max, _dt(proj), _stream()), "delta_rule_chunked")
-    if not chunked or scan_max > 0:
-        gates = torch.empty((T, 2 * heads), dtype=torch.float32, device=proj.device)
-        if chunked:
-            _chk(L.pegainfer_delta_rule_short(*first, _p(gates), *last, scan_max, _dt(proj), _stream()), "delta_rule_short")
-        else:
-            _chk(L.pegainfer_delta_rule(*first, _p(gates), *last, _dt(proj), _stream()), "delta_rule")
+        _chk(L.pegainfer_delta_rule_chunked(*first, _p(ws), *last, scan_max, _p(gates), _dt(proj), _stream()), "delta_rule_chunked")
+    else:
+        _chk(L.pegainfer_delta_rule(*first, _p(gates), *last, _dt(proj), _stream()), "delta_rule")
     return o
 
 

@@ -87,11 +87,12 @@ def test_chunks_let_nothing_reach_earlier_tokens(H, G, d, dv, what, bad):
                 assert float((a[ok] - b[ok]).abs().max()) < 2e-5 * float(a[ok].abs().max()), at
 
 
+@pytest.mark.parametrize("G,d,dv", [(2, 128, 32), (3, 64, 16), (6, 256, 16), (1, 192, 48)])
 @pytest.mark.parametrize("lens,scan_max", [([1, 30, 200, 64, 0, 65], 64), ([17, 3, 16], 16), ([5, 6], 64), ([70, 90], 64)])
-def test_an_entry_takes_the_form_of_its_own_length(lens, scan_max):
+def test_an_entry_takes_the_form_of_its_own_length(G, d, dv, lens, scan_max):
     """outputs, states and the rows made unit vectors: the bits that each entry has alone, token by token up to scan_max tokens and in chunks beyond"""
     from pegainfer_amd import ops_blocks as B
-    H, G, d, dv = 6, 2, 128, 32
+    H = 6
     gen = torch.Generator().manual_seed(len(lens))
     n, T = len(lens), sum(lens)
     A, bias = torch.randn(H, generator=gen).cuda(), torch.randn(H, generator=gen).cuda()
