@@ -40,7 +40,8 @@ pegainfer_status_t pegainfer_dyt_add_norm(float* x, const void* y, const void* p
                                           pegainfer_stream_t stream);
 /* The router of a feed-forward behind a row that a launch leaves (pegainfer_dyt_step_routed, pegainfer_row_step_routed, pegainfer_join_rms_routed): logits =
  * w row (the row as it is stored; w [experts, d], and one row more where gate_logit is given: its logit goes to gate_logit[row * gate_stride]), then the
- * selection of pegainfer_route_plan into out_expert / out_weight [rows, top].  For bf16 rows; the sizes it takes are router_tail_ok's. */
+ * selection of pegainfer_route_plan into out_expert / out_weight [rows, top].  For bf16 rows, up to 48 rows of w, d % 32 == 0, d <= 4096; router_tail_ok says where
+ * it also is the faster way. */
 typedef struct {
   const void* w;
   const void* correction;

@@ -238,7 +238,7 @@ extern "C" {
 using namespace pk;
 
 int32_t pegainfer_router_tail_ok(int32_t experts, int32_t has_gate, int32_t d, int32_t dtype) {
-  return router_tail_sizes(experts, has_gate, d, dtype);
+  return router_tail_pays(experts, has_gate, d, dtype);
 }
 
 // 64 or 128, or for few rows whatever no tile of the table may pass

@@ -188,8 +188,8 @@ __device__ __forceinline__ void route_select_lanes(float z, const A* __restrict_
 // Row, router product, selection and sort in three launches -> the row with its router in one (the experts' launches find their rows from the choices):
 // 8 rows of 1024, 17 router rows 14.0 -> 7.3 us; 8 of 2048, 41: 17.0 -> 9.9; 4 of 2048, 32: 17.2 -> 10.5; one of 2560, 32: 16.5 -> 8.5.  Without the
 // helping workgroups, and with conditional loads that kept 15 - 20 KB of instructions instead of 5: 10.8, 12.7, 13.3, 10.9.
-// Only while three blocks of 16 hold the experts, and a row a workgroup (d <= 4096): beyond that a compute unit's share of the router costs more
-// than the launches.
+// Only while three blocks of 16 hold the experts, and a row a workgroup (d <= 4096); and of those up to 240 KB of router: beyond that a compute unit's share of
+// it costs more than the launches.
 // The pieces of a wave in ascending order, then the waves in order: a logit's sum is fixed by the width alone.
 constexpr int kTailBlocks = 3;                          // experts and gate row: at most three blocks of 16 (NB: blocks of a launch, two or three)
 constexpr int kXcds = 8;
@@ -291,6 +291,12 @@ inline int tail_blocks(const RouterTail& t, int d) {
 }
 inline bool router_tail_sizes(int experts, int has_gate, int d, int dtype) {
   return dtype == kDtBf16 && experts > 0 && experts + (has_gate ? 1 : 0) <= 16 * kTailBlocks && d > 0 && d % 32 == 0 && d <= 4096;
+}
+// ... and where it is the faster way: up to 240 KB of router.  The row's launch, both products of the experts and, without the tail, the router's product and the plan,
+// cold weights, without / with (us): 48 rows of 2560 and 1 / 8 rows of a step 34.9 / 32.1, 67.4 / 68.8; 33 of 4096 41.7 / 39.1, 102.7 / 109.8; 48 of 4096
+// 43.5 / 44.1, 4 rows 71.3 / 78.3.
+inline bool router_tail_pays(int experts, int has_gate, int d, int dtype) {
+  return router_tail_sizes(experts, has_gate, d, dtype) && (experts + (has_gate ? 1 : 0)) * d <= 120 * 1024;
 }
 // the descriptor's form of it; false: that router stays a launch of its own
 inline bool router_tail(const pegainfer_router_tail_desc* q, int rows, int d, int dtype, RouterTail* t) {

@@ -88,6 +88,12 @@ def test_other_routers_stay_launches_of_their_own(rows, d, E, gate, dtype):
         B.join_rms(x, v, gain=v, y=row, router=t)
 
 
+def test_large_routers_are_left_to_a_product_of_their_own():
+    from pegainfer_amd import ffi
+    ok = lambda E, gate, d: ffi.lib().pegainfer_router_tail_ok(E, gate, d, 0)  # noqa: E731
+    assert ok(48, 0, 2560) and ok(47, 1, 2560) and not ok(48, 0, 2592) and ok(30, 0, 4096) and not ok(30, 1, 4096)
+
+
 @pytest.mark.parametrize("T,top,E,kind", [(1, 1, 1, "even"), (3, 4, 5, "even"), (16, 4, 64, "even"), (16, 16, 33, "even"), (16, 4, 7, "first"),
                                           (13, 5, 9, "beyond"), (2, 3, 6, "none")])
 @pytest.mark.parametrize("glu,slices,found", [(0, 0, False), (1, 2, False), (1, 1, True)])
