@@ -1,5 +1,5 @@
-"""Plain GEMMs whose rows behind the full rounds of 256 x 256 tiles run on smaller tiles: the same bits as those rows in a launch of their own,
-and the double-precision product within a sum of K products of about one in fp32 (1e-6 K) and the bf16 rounding of the result."""
+"""Plain GEMMs whose rows behind the full rounds of 256 x 256 tiles run on smaller tiles: the same bits as the same rows inside the full rounds
+have, the full rounds the bits of a launch without the others, and the double-precision product within a sum of K products of about one in fp32 (1e-6 K) and the bf16 rounding of the result."""
 import ctypes
 
 import pytest
@@ -29,9 +29,12 @@ def test_rows_behind_the_full_rounds(M, T, K, kernel, outputs):
         ys = [torch.full((T, m), float("nan"), device="cuda", dtype=torch.bfloat16) for m in (a, b, M - a - b)]
         P.gemm_split3_into(W, X, *ys)
         Y = torch.cat(ys, 1)
-    parts = [torch.empty((T, n), device="cuda", dtype=torch.bfloat16) for n in (cut, M - cut)]
-    P.gemm_into(W[:cut], X, parts[0])
-    assert torch.equal(Y[:, :cut], parts[0])
+    head = torch.empty((T, cut), device="cuda", dtype=torch.bfloat16)
+    P.gemm_into(W[:cut], X, head)
+    assert torch.equal(Y[:, :cut], head)
+    rolled = torch.empty((T, M), device="cuda", dtype=torch.bfloat16)
+    P.gemm_into(W.roll(M - cut, 0), X, rolled)   # the rows behind the cut come first: in the full rounds
+    assert torch.equal(Y[:, cut:], rolled[:, :M - cut])
     ref = X.double() @ W.double().T
     tol = 1e-6 * K * 4 + ref.abs() * 2.0 ** -8
     assert bool(((Y.double() - ref).abs() <= tol).all())
