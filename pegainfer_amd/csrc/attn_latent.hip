@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrep<A> a, Laten
 
 // Few rows (decoding): the prep and the product that carries the heads' queries into the latent space, which touch different values of qc and
 // read the same rows, in one grid - two launches that wait on chains of their own and leave most of the chip idle.  The product's workgroups
-// first.  4 rows, 16 heads, rank 512: 4.5 + 5.0 us one after the other, 5.1 in one; 16 steps of four such layers and their prompts
+// first.  4 rows, 16 heads, rank 512: 4.5 + 5.0 us one after the other, 5.2 in one (traced); 16 steps of four such layers and their prompts
 // 8.70 -> 8.43 ms.
 template <int OB>
 __global__ __launch_bounds__(256) void latent_prep_absorb_kernel(LatentPrep<uint16_t> a, LatentPlace p, uint16_t* __restrict__ cache, int ny,
@@ -1039,7 +1039,9 @@ struct LatentCall {
   }
   template <int ND>
   void wide() const {
-    // whole blocks of 32 values, eight neighbouring keys on one page: the form that shares LDS reads (both sides measured: at the kernel)
+    // The form that shares LDS reads, both sides measured at the kernel: ranks of 256 and 512 (its waves' eighths are two and four blocks of 16 dims), rotated
+    // parts of one and two blocks of 32 values, eight neighbouring keys on one page.  Its queries and values lie in registers, so every size is a kernel of its own;
+    // only these four are built and measured, any other size keeps the form below.
     if constexpr (ND >= 16) {
       if (r == ND * 16 && !(cut.dealt && sp > 1) && page_size % 8 == 0 && cut.grain % 8 == 0) {
         if (dr == 32) return tile_form<ND, ND / 2 + 1>();

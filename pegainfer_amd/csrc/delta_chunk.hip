@@ -8,7 +8,8 @@
 // delta_chunk_prep_kernel brings q and k to unit length and makes T', M and the factors for every (chunk, head) side by side; delta_chunk_kernel walks the chunks of an (entry,
 // head, 16 value columns), its four waves dim / 4 rows of S each.  All products are v_mfma_f32_16x16x4_f32 (plain fp32) and every decay is a product of
 // gates at most 1, never a quotient, so strong decays only underflow as they do one by one.
-// 1024 tokens of 32 heads of 128 x 128: 15 + 181 us (prep and token by token), 15 + 74 here; eight entries of 700 tokens, 8 heads 16 + 173 and 19 + 110.
+// 1024 tokens of 32 heads of 128 x 128 over 16 key heads, prep and all: 187 us token by token, 88 here (traced 18 + 75); eight entries of 700 tokens, 8 heads
+// over 4: 175 and 115.
 // Against 64 bits the read-outs are off by 2.0e-7 with slow decays (2.3e-7 token by token), by 0.85 - 1.0e-7 with fast ones (1.1 - 1.2e-7): lengths and the
 // products k . k, q . k are made in 64 bits and rounded once (in fp32 sums the fast ones were off by 1.2 - 1.4e-7).  fp32 logits of whole models are off by the
 // same either way (0.9 - 1.8e-6).
