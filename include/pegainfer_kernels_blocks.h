@@ -604,8 +604,7 @@ pegainfer_status_t pegainfer_delta_rule(float* qkv, int64_t qkv_stride, const vo
                                         int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim,
                                         int32_t vdim, int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot,
                                         int32_t n_entries, int32_t dtype, pegainfer_stream_t stream);
-/* The same for prompts, 16 tokens at a time on fp32 matrix-core products; entries of up to scan_max (>= 0) rows in the same launches token by token,
- * with the results of pegainfer_delta_rule, for which gates is as there (NULL with scan_max 0).  dim 64, 128, 192 or 256, vdim a multiple
+/* The same for prompts, 16 tokens at a time on fp32 matrix-core products.  dim 64, 128, 192 or 256, vdim a multiple
  * of 16, qkv on 16 bytes with a stride of a multiple of four (_ok).  workspace: _workspace floats, 16-byte aligned.  The results differ from the
  * token-by-token ones by rounding. */
 int64_t pegainfer_delta_rule_workspace(int32_t n_rows, int32_t n_entries, int32_t heads);
@@ -614,7 +613,14 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
                                                 int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
                                                 int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
                                                 int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
-                                                int32_t scan_max, float* gates, int32_t dtype, pegainfer_stream_t stream);
+                                                int32_t dtype, pegainfer_stream_t stream);
+/* ... with entries of up to scan_max (>= 0) rows in the same launches token by token, with the results of pegainfer_delta_rule, for which gates is as
+ * there (NULL with scan_max 0). */
+pegainfer_status_t pegainfer_delta_rule_by_length(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                                  int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
+                                                  int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
+                                                  int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
+                                                  int32_t scan_max, float* gates, int32_t dtype, pegainfer_stream_t stream);
 /* The gated delta rule with one decay per (head, key channel), acting on the rows of S:  g = exp(-exp(A_log[h]) *
  * softplus(a[row, h * dim + d] + dt_bias[h * dim + d])), a: fp32 [rows][heads * dim] at stride a_stride (the output of the decay
  * projection), dt_bias [heads * dim], A_log [heads]; gates: fp32 scratch [rows][heads * dim + heads].  Everything else as

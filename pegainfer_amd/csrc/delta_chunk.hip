@@ -356,11 +356,11 @@ int32_t pegainfer_delta_rule_chunked_ok(int32_t dim, int32_t vdim, const float* 
   return (dim == 64 || dim == 128 || dim == 192 || dim == 256) && vdim > 0 && vdim % 16 == 0 && qkv_stride % 4 == 0 && qkv_stride <= INT32_MAX && host_aligned16(qkv);
 }
 
-pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
-                                                int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
-                                                int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
-                                                int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
-                                                int32_t scan_max, float* gates, int32_t dtype, pegainfer_stream_t stream) {
+pegainfer_status_t pegainfer_delta_rule_by_length(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                                  int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
+                                                  int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
+                                                  int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
+                                                  int32_t scan_max, float* gates, int32_t dtype, pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (n_entries <= 0 || n_rows <= 0) return 0;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535 || (int64_t)heads * vdim > (1 << 24) || n_entries > 65535 || scan_max < 0 || (scan_max > 0 && !gates) || !workspace || !host_aligned16(workspace) ||
@@ -388,6 +388,15 @@ pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, 
     });
   });
   return known ? (pegainfer_status_t)hipGetLastError() : bad;
+}
+
+pegainfer_status_t pegainfer_delta_rule_chunked(float* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int64_t b_off,
+                                                int64_t a_off, const void* A_log, const void* dt_bias, float* workspace, float* state,
+                                                int64_t slot_stride, float* o, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim,
+                                                int32_t n_rows, const int32_t* entry_row0, const int32_t* entry_slot, int32_t n_entries,
+                                                int32_t dtype, pegainfer_stream_t stream) {
+  return pegainfer_delta_rule_by_length(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, workspace, state, slot_stride, o, heads, kv_heads,
+                                        dim, vdim, n_rows, entry_row0, entry_slot, n_entries, 0, nullptr, dtype, stream);
 }
 
 }  // extern "C"

@@ -1000,8 +1000,8 @@ struct Model {
         } else {
           if (delta_chunks && delta_in_chunks(c, longest)) {
             const int scan_max = shortest <= delta_scan_max(d.dim) ? delta_scan_max(d.dim) : 0;
-            FZ_K(pegainfer_delta_rule_chunked(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
-                                              o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, scan_max, gates32, dtype, S()));
+            FZ_K(pegainfer_delta_rule_by_length(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, delta_ws.p, state + c.st_mem, slot_stride,
+                                                o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, scan_max, gates32, dtype, S()));
           } else {
             FZ_K(pegainfer_delta_rule(qkv32, c.conv_ch, proj, Mp, c.o_b, c.o_a, w.A_log, w.dt_bias, gates32, state + c.st_mem, slot_stride,
                                       o32, d.heads, d.kv, d.dim, d.vdim, Ti, d_row0, d_slot, n, dtype, S()));

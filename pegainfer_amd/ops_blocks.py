@@ -301,7 +301,10 @@ def delta_rule(qkv_f32, proj, b_off, a_off, A_log, dt_bias, state, heads, kv_hea
         if not L.pegainfer_delta_rule_chunked_ok(dim, vdim, _p(qkv_f32), qkv_f32.stride(0)):
             return None
         ws = torch.empty(L.pegainfer_delta_rule_workspace(T, rg.n, heads), dtype=torch.float32, device=proj.device)
-        _chk(L.pegainfer_delta_rule_chunked(*first, _p(ws), *last, scan_max, _p(gates), _dt(proj), _stream()), "delta_rule_chunked")
+        if scan_max:
+            _chk(L.pegainfer_delta_rule_by_length(*first, _p(ws), *last, scan_max, _p(gates), _dt(proj), _stream()), "delta_rule_by_length")
+        else:
+            _chk(L.pegainfer_delta_rule_chunked(*first, _p(ws), *last, _dt(proj), _stream()), "delta_rule_chunked")
     else:
         _chk(L.pegainfer_delta_rule(*first, _p(gates), *last, _dt(proj), _stream()), "delta_rule")
     return o
