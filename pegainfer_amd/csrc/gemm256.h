@@ -1,26 +1,28 @@
-// Prefill GEMM, long prompts: 256 x 256 x 64 tiles, 8 waves (2 x 4), v_mfma_f32_16x16x32_bf16, 128 KiB of LDS.
+// Prefill GEMM, long prompts: 256 x 256 x 64 tiles, v_mfma_f32_16x16x32_bf16, 128 KiB of LDS.
 //
-//   Y[T, M] = X[T, K] . W[M, K]^T,  a workgroup owns 256 W rows x 256 token rows, wave (wr, wc) a 128 x 64 block of it
-//   as 8 x 4 MFMA tiles (128 accumulator VGPRs).
+//   Y[T, M] = X[T, K] . W[M, K]^T,  a workgroup owns 256 W rows x 256 token rows: four waves, one on each SIMD, wave (wr, wc) a
+//   128 x 128 block of it as 8 x 8 MFMA tiles (256 accumulator registers).
 //
-// The 128 x {128,64} kernel of linear.hip is LDS-read bound (two barriers per K tile, every fragment read serialised
-// behind the stage) and reaches 23-28 % of the dense bf16 peak.  This one follows the CDNA4 "8-phase" schedule:
-//   * a K tile is FOUR 16 KiB half-tiles - A_lo / A_hi = the rows of the wave's m-tiles 0-3 / 4-7 (both wave rows),
-//     B_lo / B_hi = the token rows of n-tiles 0-1 / 2-3 (all four wave columns) - and one phase computes one quadrant
-//     (4 m-tiles x 2 n-tiles x K 64 = 16 MFMAs) from one A half and one B half:
-//       phase 1: read A_lo + B_lo, quadrant (lo, lo)     phase 2: read B_hi, quadrant (lo, hi)
-//       phase 3: read A_hi,        quadrant (hi, hi)     phase 4: read B_lo, quadrant (hi, lo)
-//     so a K tile costs 24 ds_read_b128 per wave for 64 MFMAs (the 128-tile kernel: 16 for 32);
-//   * half-tiles travel global -> LDS by LDS-DMA (global_load_lds_dwordx4, XOR-swizzled through the SOURCE address),
-//     two instructions per thread per half-tile, ONE half-tile staged per phase into the slot whose last reader is two
-//     phases back: A_hi / B_lo of the next K tile in phases 1 / 2, A_lo / B_hi of the tile after that in phases 3 / 4.
-//     The only wait is a counted `s_waitcnt vmcnt(4)` at phases 4 and 8 (the two youngest half-tiles stay in flight
-//     across the barrier); a staged slot is first read one phase after the wait that retires it;
-//   * two raw s_barrier per phase, and the wave row wr = 1 runs one barrier behind wr = 0: while one half of the
-//     workgroup (one wave per SIMD) issues its 16 MFMAs, the other half does its fragment reads and its share of the
-//     DMA - the matrix pipe of every SIMD always has a wave in its MFMA segment.
+// Bound by the matrix cores, and by the power that they draw: with random operands the chip lowers its clock to 1.5 GHz, with zeros it stays at 2.2.
+// With eight waves of 128 x 64 (two a SIMD, one computing while the other reads, four phases a K tile) the bound was LDS: 28 ds_read_b128 a wave and K
+// tile, 224 KB, and 64 KB that the DMA writes are 2250 of its cycles for 2048 of the matrix cores.  Waves of 128 x 128 read 128 KB, so that
+//   * a wave has the matrix core of its SIMD to itself and everything else happens between two of its products (16 cycles each), a slot a product:
+//     128 slots a K tile, in the program's order (sched_barrier);
+//   * fragments are read one K step of 32 ahead, an instruction every second slot;
+//   * a K tile's place in LDS is free once every wave has read its second step (slot 36: barrier); from there the tile after the next is fetched
+//     into it by LDS-DMA (global_load_lds_dwordx4, XOR-swizzled through the SOURCE address), an instruction every eighth slot, as fast as
+//     addresses are taken without holding a wave up (every second or fourth slot: 13 / 5 % slower), its M0 one slot before;
+//   * the next tile has to be there at slot 96 (counted vmcnt: what the tile after it has been asked for stays in flight; barrier): 34 slots at
+//     least lie between a fetch and that;
+//   * results leave through LDS as whole lines: 8 bytes a lane in runs of 32, as the products leave them, took 8 us a tile, whole rows of 256 bytes 4.
+// Measured against the eight waves, same bits, random operands (us): 10 000 tokens: 19 456 x 2560 850 -> 750, 2560 x 9728 429 -> 386, 6144 x 2560
+// 277 -> 245; 5362 tokens: 2560 x 9728 221 -> 198, 2560 x 4096 100 -> 88; 2048 tokens, 24 576 x 4096 339 -> 300 (1375 TFLOP/s; 1900 with zeros).
+// The SwiGLU form, whose 128 gated units a lane are as long as eight K tiles' products, 10 000 tokens, 9728 x 2560: 821 -> 804; its results half as many.
 // Per-element K order (K tile by K tile, k-step 0 then 1) is that of the other tiled kernels: same bits.
 #pragma once
+
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 
@@ -33,15 +35,22 @@ enum { kHalfAlo = 0, kHalfAhi = 1, kHalfBlo = 2, kHalfBhi = 3 };
 
 struct G256Out { Half* Y; int ld; };
 
-template <bool SILU>
-__global__ __launch_bounds__(512) void mfma_gemm256_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
+template <int... I, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>()), ...); }
+// f(0), f(1), .. f(N - 1), the numbers as types
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
+
+// PART: a K slice's fp32 partials (the split-K launch)
+template <bool SILU, bool PART = false>
+__global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
                                                            Half* __restrict__ Y, int M, int T, int K, int m_tiles,
                                                            int t_tiles, SplitOut so, float* __restrict__ part = nullptr,
                                                            int nk_slice = 0) {
   extern __shared__ __attribute__((aligned(16))) u32x4 g256_smem[];
   const int ntiles = m_tiles * t_tiles;
   int tile = blockIdx.x, zslice = (int)blockIdx.y;
-  if (part && so.xcd_slices) {
+  if (PART && so.xcd_slices) {
     // K-split launches (round 6): one contiguous run of (slice, tile) work items per XCD in SLICE-major order, so an XCD pulls
     // one K slice of X through its L2 instead of all of X (see mfma_gemm128x256_kernel); same work items, same bits
     const int nitems = ntiles * (int)gridDim.y, id = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
@@ -74,226 +83,263 @@ __global__ __launch_bounds__(512) void mfma_gemm256_kernel(const Half* __restric
   }
   const int m0 = mt * G256_BM, t0 = tt * G256_BT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wr = wave >> 2, wc = wave & 3;
+  const int wr = wave >> 1, wc = wave & 1;
   const int l15 = lane & 15, g = lane >> 4;
 
-  // ---- DMA sources: piece j of a half-tile = LDS positions (j*8 + wave)*64 + lane: half-row hrow, 16-byte slot cpos;
-  //      the lane fetches global slot cpos ^ (hrow & 7) so that readers use lds_slot() ----
-  const Half* src[4][2];
+  // ---- DMA sources: piece p of an operand = its rows p * 32 + wave * 8 + (lane >> 3), LDS slot lane & 7: the lane fetches global slot
+  //      (lane & 7) ^ (row & 7) so that readers use lds_slot().  Offsets of 32 bits from the tile's first row; rows past the end repeat the last ----
+  const int kt_begin = PART ? zslice * nk_slice : 0;
+  const int nk_total = K / G256_BK;
+  // PART: a K slice of nk_slice K tiles (even, like the last, shorter one: the tiles are walked in pairs); the
+  // workgroup's fp32 tile goes to part[z][T][M] and a slice-sum launch adds the slices in z order (down_proj at 1-2 k tokens: 40-80 tiles
+  // of 256 x 256 for 256 CUs)
+  const int nk = PART ? (nk_total - kt_begin < nk_slice ? nk_total - kt_begin : nk_slice) : nk_total;
+  const int a_row0 = SILU ? so.silu_c0 + mt * 128 : m0;
+  const char* a_lo = reinterpret_cast<const char*>(W + (size_t)a_row0 * K + (size_t)kt_begin * G256_BK);
+  const char* a_hi = SILU ? a_lo + (size_t)so.silu_I * K * 2 : a_lo;      // pieces of the up rows
+  const char* b_at = reinterpret_cast<const char*>(X + (size_t)t0 * K + (size_t)kt_begin * G256_BK);
+  uint32_t va[8], vb[8];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int p = (j * 8 + wave) * 64 + lane, hrow = p >> 3, cs = (p & 7) ^ (hrow & 7);
-    // A halves: hrow = wr' * 64 + r  ->  tile row wr' * 128 (+ 64 for hi) + r
-    {
-      const int wr_ = hrow >> 6, r = hrow & 63;
-#pragma unroll
-      for (int hi = 0; hi < 2; ++hi) {
-        int row;
-        if (SILU) {  // tile = 128 gate rows + their 128 up rows: the wave's m-tiles 0-3 are gate rows, 4-7 the up rows
-          int gr = so.silu_c0 + mt * 128 + wr_ * 64 + r;
-          gr = gr < silu_cols_end(so) ? gr : silu_cols_end(so) - 1;
-          row = gr + (hi ? so.silu_I : 0);
-        } else {
-          row = m0 + wr_ * 128 + hi * 64 + r;
-          row = row < M ? row : M - 1;
-        }
-        src[hi ? kHalfAhi : kHalfAlo][j] = W + (size_t)row * K + cs * 8;
-      }
+  for (int p = 0; p < 8; ++p) {
+    const int r = p * 32 + wave * 8 + (lane >> 3), cs = (lane & 7) ^ (r & 7);
+    int ra, rb = t0 + r;
+    if (SILU) {  // tile = 128 gate rows + their 128 up rows: a wave's m-tiles 0-3 are gate rows, 4-7 the same up rows
+      ra = a_row0 + (r >> 7) * 64 + (r & 63);
+      ra = ra < silu_cols_end(so) ? ra : silu_cols_end(so) - 1;
+    } else {
+      ra = m0 + r;
+      ra = ra < M ? ra : M - 1;
     }
-    // B halves: hrow = wc' * 32 + r  ->  tile token wc' * 64 (+ 32 for hi) + r
-    {
-      const int wc_ = hrow >> 5, r = hrow & 31;
-#pragma unroll
-      for (int hi = 0; hi < 2; ++hi) {
-        int tr = t0 + wc_ * 64 + hi * 32 + r;
-        tr = tr < T ? tr : T - 1;
-        src[hi ? kHalfBhi : kHalfBlo][j] = X + (size_t)tr * K + cs * 8;
-      }
-    }
+    rb = rb < T ? rb : T - 1;
+    va[p] = (uint32_t)(ra - a_row0) * (uint32_t)(K * 2) + cs * 16;
+    vb[p] = (uint32_t)(rb - t0) * (uint32_t)(K * 2) + cs * 16;
   }
   typedef __attribute__((address_space(3))) void* lptr_t;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)&g256_smem[0];
-  // split-K form (part != null): blockIdx.y = K slice of nk_slice K tiles (even, like the last, shorter one: the
-  // tiles are walked in pairs); the workgroup's fp32 tile goes to part[z][T][M] and a slice-sum launch adds the slices
-  // in z order (down_proj at 1-2 k tokens: 40-80 tiles of 256 x 256 for 256 CUs)
-  const int kt_begin = part ? zslice * nk_slice : 0;
-  const int nk_total = K / G256_BK;
-  const int nk = part ? (nk_total - kt_begin < nk_slice ? nk_total - kt_begin : nk_slice) : nk_total;
-#pragma unroll
-  for (int w = 0; w < 4; ++w)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) src[w][j] += (size_t)kt_begin * G256_BK;
-  // stage half-tile `which` of K tile kt (clamped: past the end the slot is dead, the load only keeps vmcnt uniform)
-  auto stage = [&](int which, int kt) {
-    const int ktc = kt < nk ? kt : nk - 1;
-    const uint32_t slot = lds0 + (uint32_t)(((kt & 1) * 4 + which) * kG256HalfBytes);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t dst = __builtin_amdgcn_readfirstlane(slot + (uint32_t)(j * 8 + wave) * 1024u);
-      if ((which == kHalfAlo || which == kHalfAhi) && so.w_nt)   // a single token tile: W bytes have one reader (SplitOut::w_nt)
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                     :: "v"(src[which][j] + (size_t)ktc * G256_BK), "s"(dst) : "memory", "m0");
-      else
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                     :: "v"(src[which][j] + (size_t)ktc * G256_BK), "s"(dst) : "memory", "m0");
-    }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)&g256_smem[0] + wave * 1024u);
+  // piece q of a K tile (0-7: W, 8-15: X) in the place of parity par, `at` bytes behind the tile that a_lo, b_at point to: M0, then the load
+  auto aim = [&](auto q, auto par) {
+    const uint32_t to = lds0 + (uint32_t)(decltype(par)::value * 65536 + decltype(q)::value * 4096);
+    asm volatile("s_mov_b32 m0, %0" ::"s"(to) : "m0");
   };
-  auto half_ptr = [&](int par, int which) { return g256_smem + (size_t)(par * 4 + which) * (kG256HalfBytes / 16); };
+  auto fetch = [&](auto qc, int at) {
+    constexpr int q = decltype(qc)::value;
+    const char* base = (q >= 8 ? b_at : (q & 2) ? a_hi : a_lo) + at;
+    const uint32_t v = q < 8 ? va[q & 7] : vb[q & 7];
+    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(v), "s"(base) : "memory");
+  };
 
-  f32x4 acc[8][4];
+  f32x4 acc[8][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8_t a[4][2], b[2][2];
-  auto read_a = [&](int par, int which) {
-    const u32x4* h = half_ptr(par, which);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        a[i][ks] = __builtin_bit_cast(bf16x8_t, h[lds_slot(wr * 64 + i * 16 + l15, ks * 4 + g)]);
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8_t fa[2][8], fb[2][8];
+  // fragments of K step `ks` in the order of their first use: a0, b0 .. b7, a1 .. a7
+  auto read = [&](auto qc, auto ksc, auto parc) {
+    constexpr int q = decltype(qc)::value, ks = decltype(ksc)::value;
+    const u32x4* at = g256_smem + decltype(parc)::value * 4096;
+    if constexpr (q == 0 || q >= 9) {
+      constexpr int i = q == 0 ? 0 : q - 8;
+      fa[ks][i] = __builtin_bit_cast(bf16x8_t, at[lds_slot(wr * 128 + i * 16 + l15, ks * 4 + g)]);
+    } else {
+      fb[ks][q - 1] = __builtin_bit_cast(bf16x8_t, at[2048 + lds_slot(wc * 128 + (q - 1) * 16 + l15, ks * 4 + g)]);
+    }
   };
-  auto read_b = [&](int par, int which) {
-    const u32x4* h = half_ptr(par, which);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        b[j][ks] = __builtin_bit_cast(bf16x8_t, h[lds_slot(wc * 32 + j * 16 + l15, ks * 4 + g)]);
-  };
-  auto quad = [&](int ih, int jh) {   // 16 MFMAs: m-tiles ih*4.., n-tiles jh*2..
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[ih * 4 + i][jh * 2 + j] =
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][ks], b[j][ks], acc[ih * 4 + i][jh * 2 + j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
+  typedef std::integral_constant<int, 0> P0;
+  typedef std::integral_constant<int, 1> P1;
+  // the slots of a K tile (see above); a piece whose slot lies behind the last one is fetched by the next K tile
+  constexpr int kFree = 36, kLanded = 96, kEvery = 8, kReadEvery = 2;
+  constexpr int kBefore = (128 - kFree + kEvery - 1) / kEvery;       // pieces whose fetch begins in their own K tile's iteration
 
-  // ---- prologue: K tile 0 complete, A_lo / B_hi of K tile 1 in flight ----
-  stage(kHalfAlo, 0); stage(kHalfBlo, 0); stage(kHalfBhi, 0); stage(kHalfAhi, 0);
-  stage(kHalfAlo, 1); stage(kHalfBhi, 1);
-  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  // ---- prologue: K tile 0, and of K tile 1 what no iteration fetches ----
+  auto fetch_now = [&](auto q, auto par, int at) {
+    aim(q, par);
+    asm volatile("s_nop 0");
+    fetch(q, at);
+  };
+  static_for<16>([&](auto q) { fetch_now(q, P0(), 0); });
+  static_for<kBefore>([&](auto q) { fetch_now(q, P1(), 128); });
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kBefore) : "memory");
   __builtin_amdgcn_s_barrier();
-  if (wr == 1) __builtin_amdgcn_s_barrier();   // the second wave row runs one barrier behind the first
+  static_for<16>([&](auto q) { read(q, P0(), P0()); });
 
-  // one K tile = four phases; `kt` has parity `par`, the other slots belong to kt + 1
-  auto ktile = [&](int kt, int par) {
-    // phase 1: A_lo + B_lo -> (lo, lo); stage A_hi of kt + 1
-    read_b(par, kHalfBlo);
+  // one K tile in the place of parity par.  MORE: there is a tile after the next to fetch; NEXT: there is a next one
+  auto ktile = [&](auto parc, auto morec, auto nextc) {
+    constexpr int par = decltype(parc)::value;
+    constexpr bool MORE = decltype(morec)::value, NEXT = decltype(nextc)::value;
+    typedef std::integral_constant<int, par ^ 1> Other;
     __builtin_amdgcn_sched_barrier(0);
-    read_a(par, kHalfAlo);
-    stage(kHalfAhi, kt + 1);
-    __builtin_amdgcn_s_barrier();
-    quad(0, 0);
-    __builtin_amdgcn_s_barrier();
-    // phase 2: B_hi -> (lo, hi); stage B_lo of kt + 1
-    read_b(par, kHalfBhi);
-    stage(kHalfBlo, kt + 1);
-    __builtin_amdgcn_s_barrier();
-    quad(0, 1);
-    __builtin_amdgcn_s_barrier();
-    // phase 3: A_hi -> (hi, hi); stage A_lo of kt + 2
-    read_a(par, kHalfAhi);
-    stage(kHalfAlo, kt + 2);
-    __builtin_amdgcn_s_barrier();
-    quad(1, 1);
-    __builtin_amdgcn_s_barrier();
-    // phase 4: B_lo -> (hi, lo); stage B_hi of kt + 2; everything but the two youngest half-tiles has landed
-    read_b(par, kHalfBlo);
-    stage(kHalfBhi, kt + 2);
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    quad(1, 0);
-    __builtin_amdgcn_s_barrier();
+    static_for<128>([&](auto nc) {
+      constexpr int n = decltype(nc)::value, ks = n >> 6;
+      if constexpr (n % kReadEvery == 0 && n / kReadEvery < 16) read(std::integral_constant<int, n / kReadEvery>(), P1(), parc);
+      if constexpr (MORE && n == kFree) {        // every wave has its fragments of this tile
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (NEXT && n == kLanded) {      // the next tile is there; of the one after it, what has been asked for may be on its way
+        constexpr int asked = MORE ? (kLanded - 2 - kFree) / kEvery + 1 : 0;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(asked) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (NEXT && n >= kLanded && (n - kLanded) % kReadEvery == 0 && (n - kLanded) / kReadEvery < 16)
+        read(std::integral_constant<int, (n - kLanded) / kReadEvery>(), P0(), Other());
+      constexpr int own = n - kFree, late = n + 128 - kFree;
+      if constexpr (MORE && own >= 0 && own % kEvery == 0 && own / kEvery < 16) aim(std::integral_constant<int, own / kEvery>(), parc);
+      if constexpr (MORE && own >= 0 && own % kEvery == 1 && own / kEvery < 16) fetch(std::integral_constant<int, own / kEvery>(), 256);
+      if constexpr (NEXT && n < kFree && late % kEvery == 0 && late / kEvery < 16) aim(std::integral_constant<int, late / kEvery>(), Other());
+      if constexpr (NEXT && n < kFree && late % kEvery == 1 && late / kEvery < 16) fetch(std::integral_constant<int, late / kEvery>(), 128);
+      __builtin_amdgcn_sched_barrier(0);         // a product lies between M0 and the load that reads it
+      constexpr int i = (n & 63) >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    a_lo += 128;
+    a_hi += 128;
+    b_at += 128;
   };
-  for (int kt = 0; kt < nk; kt += 2) {
-    ktile(kt, 0);
-    ktile(kt + 1, 1);
+  static_assert(kFree % kEvery != 127 % kEvery, "an aim and its load lie in one iteration");
+  for (int kt = 0; kt + 2 < nk; kt += 2) {
+    ktile(P0(), std::true_type(), std::true_type());
+    ktile(P1(), std::true_type(), std::true_type());
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped tail loads must not outlive the workgroup's LDS
-  if (wr == 0) __builtin_amdgcn_s_barrier();
+  ktile(P0(), std::false_type(), std::true_type());
+  ktile(P1(), std::false_type(), std::false_type());
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
 
-  // ---- epilogue: lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15 ----
-  if (SILU) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = t0 + wc * 64 + j * 16 + l15;
-      if (t >= T) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = so.silu_c0 + mt * 128 + wr * 64 + i * 16 + g * 4;
-        float r[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {  // the GEMM output is bf16 before SwiGLU (fused_proj.cu:57-62)
-          const float sg = silu_f(bf16_round_f(acc[i][j][e]));
-          r[e] = (so.silu_round ? bf16_round_f(sg) : sg) * bf16_round_f(acc[i + 4][j][e]);
-        }
-        if (m + 3 < silu_cols_end(so)) {
-          u32x2 o;
-          o.x = pack_bf2(r[0], r[1]);
-          o.y = pack_bf2(r[2], r[3]);
-          *reinterpret_cast<u32x2*>(Y + (size_t)t * so.silu_I + m) = o;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (m + e < silu_cols_end(so)) Y[(size_t)t * so.silu_I + m + e] = f2bf(r[e]);
-        }
-      }
-    }
-    return;
-  }
-  if (part) {
+  // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 32 KB of LDS
+  //      (chunks of 16 bytes, XOR-swizzled by the token) and stores whole rows of a token.  `wide`: every row that is written begins on 16 bytes and the
+  //      segments are whole chunks of eight values; else a chunk leaves in halves or value by value ----
+  __syncthreads();                                 // every wave is through with the tiles
+  char* own = reinterpret_cast<char*>(g256_smem) + wave * 32768;
+  if constexpr (PART) {                             // 64 tokens of 512 bytes at a time
     float* pz = part + (size_t)zslice * T * M;
+    const bool wide = aligned16(pz) && (M & 3) == 0;
+    const int m = m0 + wr * 128 + (lane & 31) * 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = t0 + wc * 64 + j * 16 + l15;
-      if (t >= T) continue;
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int m = m0 + wr * 128 + i * 16 + g * 4;
-        if (m + 3 < M) {
-          *reinterpret_cast<f32x4*>(pz + (size_t)t * M + m) = acc[i][j];
-        } else {
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (m + e < M) pz[(size_t)t * M + m + e] = acc[i][j][e];
-        }
+        for (int i = 0; i < 8; ++i)
+          *reinterpret_cast<f32x4*>(own + (j * 16 + l15) * 512 + (((i * 4 + g) ^ l15) << 4)) = acc[i][h * 4 + j];
+      auto row = [&](int q, auto&& store) {
+        const int tl = q * 2 + (lane >> 5), t = t0 + wc * 128 + h * 64 + tl;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((lane & 31) ^ (tl & 15)) << 4));
+        if (t < T && m < M) store(pz + (size_t)t * M + m, v);
+      };
+      if (wide) {
+#pragma unroll 8
+        for (int q = 0; q < 32; ++q) row(q, [](float* to, const f32x4& v) { *reinterpret_cast<f32x4*>(to) = v; });
+      } else {
+#pragma unroll 1
+        for (int q = 0; q < 32; ++q)
+          row(q, [&](float* to, const f32x4& v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (m + e < M) to[e] = v[e];
+          });
       }
     }
     return;
   }
+  // the first `left` of four values; `whole` is one for the grid: all four, on 8 bytes, or none
+  auto leave = [&](Half* to, const u32x2& v, int left, bool whole) {
+    if (whole) {
+      if (left > 0) *reinterpret_cast<u32x2*>(to) = v;
+    } else {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int t = t0 + wc * 64 + j * 16 + l15;
-    if (t >= T) continue;
+      for (int e = 0; e < 4; ++e)
+        if (e < left) to[e] = (Half)(v[e >> 1] >> (16 * (e & 1)));
+    }
+  };
+  // rows of 256 bytes
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int m = m0 + wr * 128 + i * 16 + g * 4;
-      Half* dst = Y;
-      int ld = M, mm = m, mlim = M;
-      if (so.Y1) {
-        const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
-        if (m < so.M0) { ld = mlim = so.M0; }
-        else if (m < b1) { dst = so.Y1; ld = mlim = so.M1; mm = m - so.M0; }
-        else if (m < b2) { dst = so.Y2; ld = mlim = so.M2; mm = m - b1; }
-        else { dst = so.Y3; ld = mlim = M - b2; mm = m - b2; }
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      *reinterpret_cast<u32x2*>(own + (j * 16 + l15) * 256 + (((i * 2 + (g >> 1)) ^ l15) << 4) + (g & 1) * 8) =
+          u32x2{pack_bf2(acc[i][j][0], acc[i][j][1]), pack_bf2(acc[i][j][2], acc[i][j][3])};
+  auto chunk_of = [&](int tl, int c) { return *reinterpret_cast<const u32x4*>(own + tl * 256 + ((c ^ (tl & 15)) << 4)); };
+  if constexpr (SILU) {                            // 64 gate values and their 64 up values, bf16 as the GEMM's output is before SwiGLU (fused_proj.cu:57-62)
+    const int end = silu_cols_end(so), m = so.silu_c0 + mt * 128 + wr * 64 + (lane & 7) * 8;
+    const int odd = so.silu_I | so.silu_c0 | end;
+    const bool wide = aligned16(Y) && (odd & 7) == 0, fours = (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (odd & 3) == 0;
+    auto rows = [&](auto roundc) {
+#pragma unroll 2
+      for (int q = 0; q < 16; ++q) {
+        const int tl = q * 8 + (lane >> 3), t = t0 + wc * 128 + tl;
+        const u32x4 ga = chunk_of(tl, lane & 7), up = chunk_of(tl, 8 + (lane & 7));
+        float r[8];
+        auto values = [&](auto silu) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t gw = ga[e >> 1], uw = up[e >> 1];
+            const float sg = silu(e & 1 ? bf_hi(gw) : bf_lo(gw));
+            r[e] = (decltype(roundc)::value ? bf16_round_f(sg) : sg) * (e & 1 ? bf_hi(uw) : bf_lo(uw));
+          }
+        };
+        if (__all(silu_mid_ok(ga))) values([](float v) { return silu_mid_f(v); });
+        else values([](float v) { return silu_f(v); });
+        const u32x4 o{pack_bf2(r[0], r[1]), pack_bf2(r[2], r[3]), pack_bf2(r[4], r[5]), pack_bf2(r[6], r[7])};
+        Half* to = Y + (size_t)t * so.silu_I + m;
+        if (t >= T || m >= end) continue;
+        if (wide) {
+          *reinterpret_cast<u32x4*>(to) = o;
+        } else {
+          leave(to, u32x2{o.x, o.y}, end - m, fours);
+          leave(to + 4, u32x2{o.z, o.w}, end - m - 4, fours);
+        }
       }
-      if (mm + 3 < mlim) {
-        u32x2 o;
-        o.x = pack_bf2(acc[i][j][0], acc[i][j][1]);
-        o.y = pack_bf2(acc[i][j][2], acc[i][j][3]);
-        *reinterpret_cast<u32x2*>(dst + (size_t)t * ld + mm) = o;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (mm + e < mlim) dst[(size_t)t * ld + mm + e] = f2bf(acc[i][j][e]);
+    };
+    if (so.silu_round) rows(std::true_type());
+    else rows(std::false_type());
+  } else {
+    const bool whole = aligned16(Y) && (M & 7) == 0;
+    const bool wide = whole && (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
+    const int m = m0 + wr * 128 + l15 * 8;
+    struct Segment { Half* at; int ld, m, end; };
+    auto segment = [&](int r) {                    // where row r goes
+      if (!so.Y1) return Segment{Y, M, r, M};
+      const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
+      if (r < so.M0) return Segment{Y, so.M0, r, so.M0};
+      if (r < b1) return Segment{so.Y1, so.M1, r - so.M0, so.M1};
+      if (r < b2) return Segment{so.Y2, so.M2, r - b1, so.M2};
+      return Segment{so.Y3, M - b2, r - b2, M - b2};
+    };
+    const Segment sg = segment(m);
+    auto row = [&](int q, auto&& store) {
+      const int tl = q * 4 + g, t = t0 + wc * 128 + tl;
+      const u32x4 v = chunk_of(tl, l15);
+      if (t < T && m < M) store(t, v);
+    };
+    if (wide) {
+#pragma unroll 8
+      for (int q = 0; q < 32; ++q) row(q, [&](int t, const u32x4& v) { *reinterpret_cast<u32x4*>(sg.at + (size_t)t * sg.ld + sg.m) = v; });
+    } else if (!so.Y1) {                           // half a chunk a lane
+      const int mh = m0 + wr * 128 + (lane & 31) * 4;
+      const bool fours = (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (M & 3) == 0;
+#pragma unroll 4
+      for (int q = 0; q < 64; ++q) {
+        const int tl = q * 2 + (lane >> 5), t = t0 + wc * 128 + tl;
+        const u32x2 v = *reinterpret_cast<const u32x2*>(own + tl * 256 + ((((lane & 31) >> 1) ^ (tl & 15)) << 4) + (lane & 1) * 8);
+        if (t < T) leave(Y + (size_t)t * M + mh, v, M - mh, fours);
       }
+    } else {                                       // a chunk may lie across segments
+#pragma unroll 1
+      for (int q = 0; q < 32; ++q)
+        row(q, [&](int t, const u32x4& v) {
+#pragma unroll 1
+          for (int e = 0; e < 8; ++e) {
+            const Segment one = segment(m + e);
+            const uint32_t word = e < 4 ? (e < 2 ? v[0] : v[1]) : (e < 6 ? v[2] : v[3]);
+            if (m + e < M) one.at[(size_t)t * one.ld + one.m] = (Half)(word >> (16 * (e & 1)));
+          }
+        });
     }
   }
 }
@@ -309,7 +355,6 @@ inline bool gemm_t_major(int M, int T, const SplitOut& so) {   // PEGAINFER_GEMM
 inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, SplitOut so, hipStream_t s, int m_head = 0) {
   const bool silu = so.silu_I > 0;
   const int m_tiles = silu ? ceil_div(silu_cols_end(so) - so.silu_c0, 128) : m_head ? m_head : ceil_div(M, G256_BM), t_tiles = ceil_div(T, G256_BT);
-  so.w_nt = t_tiles == 1 && weights_nt_on();
   so.t_major = gemm_t_major(M, T, so);
   {  // PEGAINFER_GEMM_CHUNK=0: the plain order (A/B); N: chunks of N tiles
     static const int chunk = [] { const char* e = getenv("PEGAINFER_GEMM_CHUNK"); return e && *e ? atoi(e) : 8; }();
@@ -326,7 +371,7 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<true><<<m_tiles * t_tiles, 512, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<true><<<m_tiles * t_tiles, 256, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   } else {
     static const bool once = [] {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false>),
@@ -334,7 +379,7 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<false><<<m_tiles * t_tiles, 512, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<false><<<m_tiles * t_tiles, 256, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   }
 }
 
@@ -347,22 +392,24 @@ inline void gemm256_splitk_launch(const Half* W, const Half* X, int M, int T, in
                                   hipStream_t s) {
   const int m_tiles = ceil_div(M, G256_BM), t_tiles = ceil_div(T, G256_BT);
   static const bool once = [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false, true>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes);
     return true;
   }();
   (void)once;
-  mfma_gemm256_kernel<false><<<dim3(m_tiles * t_tiles, ksplit), 512, kG256LdsBytes, s>>>(
+  mfma_gemm256_kernel<false, true><<<dim3(m_tiles * t_tiles, ksplit), 256, kG256LdsBytes, s>>>(
       W, X, nullptr, M, T, K, m_tiles, t_tiles,
-      SplitOut{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0, t_tiles == 1 && weights_nt_on(), ksplit > 1 && splitk_xcd_on(), 0}, part, nk_slice);
+      SplitOut{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0, 0, ksplit > 1 && splitk_xcd_on(), 0}, part, nk_slice);
 }
 
-// ---- stream-K form of the 256 x 256 kernel (round 6) --------------------------------------------------------------------
+// ---- stream-K form of the 256 x 256 kernel, on the schedule of eight waves (2 x 4, blocks of 128 x 64) --------------------------------------------------------------------
 // The data-parallel launch above pays for tile quantisation: 304 tiles (gate_up at 1024 tokens) are one full round of the
 // 256 CUs plus 48 tiles that cost a second full tile time; 152 tiles (512 tokens) leave 104 CUs idle.  Here the launch is
 // PERSISTENT - one workgroup per CU - and the work is the linear sequence of (tile, K-tile pair) units, tile-major, dealt in
 // equal contiguous ranges: workgroup position p owns units [U p / G, U (p + 1) / G).  A range is cut at tile boundaries into
-// segments; each segment runs the 8-phase main loop over its K range and then
+// segments; each segment runs a main loop of eight phases per pair of K tiles - a K tile is four half-tiles (A_lo / A_hi: the rows of a wave's m-tiles 0-3 /
+// 4-7, B_lo / B_hi: the tokens of its n-tiles 0-1 / 2-3), a phase one quadrant of products and the DMA of one half-tile, the second wave row a barrier
+// behind the first - over its K range and then
 //   * covers the whole tile            -> the ordinary epilogue;
 //   * starts inside a tile             -> (only ever a workgroup's FIRST segment) the fp32 accumulators go to the workgroup's
 //                                         256 KiB slot of the split-K workspace, lane-contiguous, write-through (sc1) stores,

@@ -179,7 +179,7 @@ inline bool weights_nt_on() {
 }
 
 }  // namespace pk
-#include "gemm256.h"   // 256 x 256 tiles, 8 waves, 8-phase schedule (long prompts); uses SplitOut / lds_slot
+#include "gemm256.h"   // 256 x 256 tiles, a wave a SIMD (long prompts); uses SplitOut / lds_slot
 #include "gemm_stream.h"   // CU-count-sized row tiles for 17..64 token columns (round 4); uses SplitOut / lds_slot / BK
 namespace pk {
 
@@ -641,7 +641,7 @@ static SplitKPlan splitk_plan(int M, int T, int K, bool assume_ws = false) {
   const int m_tiles = ceil_div(M, BM), nk_all = K / BK;
   if (T > 64) {
     if (short_k_whole(M, T, K)) return {0, 0, 0};
-    // long-K matrices at ~1.3-3 k tokens (down_proj: 50-128 tiles of 256 x 256): the 8-phase kernel over 2-5 K
+    // long-K matrices at ~1.3-3 k tokens (down_proj: 50-128 tiles of 256 x 256): their kernel over 2-5 K
     // slices, one workgroup per CU (tt == 256 marks this plan; PEGAINFER_SPLITK256=0 switches it off).  Same-box A/B of
     // TTFT: 2048 tokens 23.05 -> 21.4 ms; 1024 tokens (40 tiles, 6 slices: 63 MB of partials each way) 12.60 vs 12.56,
     // 512 tokens (8 slices) 9.17 vs 9.33 - so only above 40 tiles.
@@ -752,7 +752,7 @@ static int plain_tail_kernel(int M, int T, int K, int m_head) {
 
 // Which tiled kernel a prefill-shaped GEMM (T > 64, not K-split) takes - by shape only.  kind: 259 = 256 with the rows behind its full rounds on a kernel
 // of smaller tiles (plain_tail_kernel; m_head = tiles of rows of the head), 12 / 13 / 22 / 23 = the
-// 128-row LDS-DMA kernel with 128- / 64-token tiles and that ring depth, 256 = the 256 x 256 8-phase kernel, 257 = its
+// 128-row LDS-DMA kernel with 128- / 64-token tiles and that ring depth, 256 = the 256 x 256 kernel, 257 = its
 // SwiGLU form with the thin last round handed to the 128-row kernel (m_head = activation-column tiles of the head), 1280 /
 // 1281 = the 128 x 256 kernel, plain / SwiGLU.  One function for the launcher and for pegainfer_debug_gemm_route (the
 // routing table is pinned by a CPU test: a threshold edit must not silently change what the GPU tests exercise).
@@ -766,7 +766,7 @@ static TiledRoute tiled_route(int M, int T, int K, const SplitOut& so, bool assu
   }
   if (so.silu_I == 0 && !force)
     if (const int kind = small_tile_unsplit(M, T, K)) return {kind, 0};
-  // long prompts: 256 x 256 tiles on the 8-phase schedule once they give every CU work (PEGAINFER_GEMM256 = 0 never,
+  // long prompts: 256 x 256 tiles once they give every CU work (PEGAINFER_GEMM256 = 0 never,
   // 1 whenever the shape allows, N = from N tiles on; A/B probe knob)
   // from 128 tiles on (half the CUs): one partly filled round of 256 x 256 tiles still beats the smaller tilings -
   // gate_up at 512 tokens (152 tiles) 100 -> 70 us, qkv at 1536 tokens (144 tiles) 80 -> 64 us, same bits
