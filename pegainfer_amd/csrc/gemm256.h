@@ -14,13 +14,16 @@
 //     addresses are taken without holding a wave up (every second or fourth slot: 13 / 5 % slower), its M0 one slot before;
 //   * the next tile has to be there at slot 96 (counted vmcnt: what the tile after it has been asked for stays in flight; barrier): 34 slots at
 //     least lie between a fetch and that;
-//   * results leave through LDS as whole lines: 8 bytes a lane in runs of 32, as the products leave them, took 8 us a tile, whole rows of 256 bytes 4.
-// Measured against the eight waves, same bits, random operands (us): 10 000 tokens: 19 456 x 2560 850 -> 750, 2560 x 9728 429 -> 386, 6144 x 2560
-// 277 -> 245; 5362 tokens: 2560 x 9728 221 -> 198, 2560 x 4096 100 -> 88; 2048 tokens, 24 576 x 4096 339 -> 300 (1375 TFLOP/s; 1900 with zeros).
-// The SwiGLU form, whose 128 gated units a lane are as long as eight K tiles' products, 10 000 tokens, 9728 x 2560: 821 -> 804; its results half as many.
+//   * results leave through LDS as whole lines: 8 bytes a lane in runs of 32, as the products leave them, took 8 us a tile, whole rows of 256 bytes 4;
+//   * a workgroup stays on its compute unit and takes every 256th tile: the next one's first two K tiles are asked for before the results are turned, and
+//     its products begin while they are still on their way out.  2 us of fetching and up to 4 of stores a tile of 60 to 75.
+// Measured against the eight waves, same bits, random operands (us): 10 000 tokens: 19 456 x 2560 926 -> 758, 2560 x 9728 487 -> 404, 6144 x 2560
+// 288 -> 242; 5362 tokens: 2560 x 9728 222 -> 197, 2560 x 4096 100 -> 88; 2048 tokens, 24 576 x 4096 330 -> 294.  The SwiGLU form, whose 128 gated
+// units a lane are as long as eight K tiles' products: 10 000 tokens, 9728 x 2560 862 -> 777 (804 of 821 with a workgroup a tile), 1024 tokens 99.5 -> 93.7.
 // Per-element K order (K tile by K tile, k-step 0 then 1) is that of the other tiled kernels: same bits.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -31,6 +34,7 @@ namespace pk {
 constexpr int G256_BM = 256, G256_BT = 256, G256_BK = 64;
 constexpr int kG256HalfBytes = 128 * 128;            // 128 rows x 128 B
 constexpr int kG256LdsBytes = 8 * kG256HalfBytes;    // 2 parities x {A_lo, A_hi, B_lo, B_hi}
+constexpr int kG256TurnBytes = 4 * 8192;             // where the waves turn their results
 enum { kHalfAlo = 0, kHalfAhi = 1, kHalfBlo = 2, kHalfBhi = 3 };
 
 struct G256Out { Half* Y; int ld; };
@@ -41,7 +45,7 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
 
-// PART: a K slice's fp32 partials (the split-K launch)
+// PART: a K slice's fp32 partials (the split-K launch), a work item a workgroup; else a workgroup takes every gridDim.x-th tile
 template <bool SILU, bool PART = false>
 __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
                                                            Half* __restrict__ Y, int M, int T, int K, int m_tiles,
@@ -49,90 +53,87 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
                                                            int nk_slice = 0) {
   extern __shared__ __attribute__((aligned(16))) u32x4 g256_smem[];
   const int ntiles = m_tiles * t_tiles;
-  int tile = blockIdx.x, zslice = (int)blockIdx.y;
-  if (PART && so.xcd_slices) {
-    // K-split launches (round 6): one contiguous run of (slice, tile) work items per XCD in SLICE-major order, so an XCD pulls
-    // one K slice of X through its L2 instead of all of X (see mfma_gemm128x256_kernel); same work items, same bits
-    const int nitems = ntiles * (int)gridDim.y, id = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
-    const int q = nitems / 8, r = nitems % 8, xcd = id % 8, idx = id / 8;
-    const int item = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-    zslice = item / ntiles;
-    tile = item - zslice * ntiles;
-  } else {  // XCD-aware order (block b runs on XCD b % 8): every XCD walks a contiguous run of tiles, token tile fastest
-    const int q = ntiles / 8, r = ntiles % 8, xcd = tile % 8, idx = tile / 8;
-    tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-  }
-  // (round 6) t_major: row tile fastest inside an XCD's run - for T > M (o_proj / down_proj / qkv at 10 k tokens) an XCD then pulls
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wr = wave >> 1, wc = wave & 1;
+  const int l15 = lane & 15, g = lane >> 4;
+  // the value as one that the loop over tiles does not know: what follows from it is computed where it is used, not kept across the products
+  auto again = [](int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  int zslice = (int)blockIdx.y;
+  // t_major: row tile fastest inside an XCD's run - for T > M (o_proj / down_proj / qkv at 10 k tokens) an XCD then pulls
   // 1/8 of X and all of W through its L2 instead of all of X and 1/8 of W
-  // (round 6) chunk: the slow dimension of the order is walked in chunks of `chunk` tiles, so the ~32 workgroups an XCD runs at a time
+  // chunk: the slow dimension of the order is walked in chunks of `chunk` tiles, so the ~32 workgroups an XCD runs at a time
   // are a (32 / chunk) x chunk block of tiles sharing 32 / chunk + chunk operand panels through its L2 instead of 1 + 32: gate_up at
   // 10 k tokens (76 x 40 tiles, token tile fastest) fetched 4.2 GB from the memory side per launch for 151 MB of operands - every X
   // panel once per row tile (FETCH_SIZE, profiles/r6c_ctx10000_pmc_fetch.csv)
   int mt, tt;
-  if (so.chunk > 0) {
-    const int fast_n = so.t_major ? m_tiles : t_tiles, slow_n = so.t_major ? t_tiles : m_tiles;   // fast = the inner dimension of the plain order
-    const int per_chunk = slow_n * so.chunk;                  // tiles of one full chunk of the FAST dimension
-    const int c = tile / per_chunk, rem = tile - c * per_chunk;
-    const int cw = fast_n - c * so.chunk < so.chunk ? fast_n - c * so.chunk : so.chunk;
-    const int slow = rem / cw, fast = c * so.chunk + rem - slow * cw;
-    mt = so.t_major ? fast : slow;
-    tt = so.t_major ? slow : fast;
-  } else {
-    mt = so.t_major ? tile % m_tiles : tile / t_tiles;
-    tt = so.t_major ? tile / m_tiles : tile - mt * t_tiles;
-  }
-  const int m0 = mt * G256_BM, t0 = tt * G256_BT;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int l15 = lane & 15, g = lane >> 4;
+  auto place = [&](int item) {
+    int tile = item;
+    if (PART && so.xcd_slices) {
+      // K-split launches: one contiguous run of (slice, tile) work items per XCD in SLICE-major order, so an XCD pulls
+      // one K slice of X through its L2 instead of all of X (see mfma_gemm128x256_kernel); same work items, same bits
+      const int nitems = ntiles * (int)gridDim.y, id = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
+      const int q = nitems / 8, r = nitems % 8, xcd = id % 8, idx = id / 8;
+      const int at = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+      zslice = at / ntiles;
+      tile = at - zslice * ntiles;
+    } else {  // XCD-aware order (block b runs on XCD b % 8): every XCD walks a contiguous run of tiles, token tile fastest
+      const int q = ntiles / 8, r = ntiles % 8, xcd = tile % 8, idx = tile / 8;
+      tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+    }
+    if (so.chunk > 0) {
+      const int fast_n = so.t_major ? m_tiles : t_tiles, slow_n = so.t_major ? t_tiles : m_tiles;   // fast = the inner dimension of the plain order
+      const int per_chunk = slow_n * so.chunk;                  // tiles of one full chunk of the FAST dimension
+      const int c = tile / per_chunk, rem = tile - c * per_chunk;
+      const int cw = fast_n - c * so.chunk < so.chunk ? fast_n - c * so.chunk : so.chunk;
+      const int slow = rem / cw, fast = c * so.chunk + rem - slow * cw;
+      mt = so.t_major ? fast : slow;
+      tt = so.t_major ? slow : fast;
+    } else {
+      mt = so.t_major ? tile % m_tiles : tile / t_tiles;
+      tt = so.t_major ? tile / m_tiles : tile - mt * t_tiles;
+    }
+  };
 
   // ---- DMA sources: piece p of an operand = its rows p * 32 + wave * 8 + (lane >> 3), LDS slot lane & 7: the lane fetches global slot
-  //      (lane & 7) ^ (row & 7) so that readers use lds_slot().  Offsets of 32 bits from the tile's first row; rows past the end repeat the last ----
-  const int kt_begin = PART ? zslice * nk_slice : 0;
-  const int nk_total = K / G256_BK;
-  // PART: a K slice of nk_slice K tiles (even, like the last, shorter one: the tiles are walked in pairs); the
-  // workgroup's fp32 tile goes to part[z][T][M] and a slice-sum launch adds the slices in z order (down_proj at 1-2 k tokens: 40-80 tiles
-  // of 256 x 256 for 256 CUs)
-  const int nk = PART ? (nk_total - kt_begin < nk_slice ? nk_total - kt_begin : nk_slice) : nk_total;
-  const int a_row0 = SILU ? so.silu_c0 + mt * 128 : m0;
-  const char* a_lo = reinterpret_cast<const char*>(W + (size_t)a_row0 * K + (size_t)kt_begin * G256_BK);
-  const char* a_hi = SILU ? a_lo + (size_t)so.silu_I * K * 2 : a_lo;      // pieces of the up rows
-  const char* b_at = reinterpret_cast<const char*>(X + (size_t)t0 * K + (size_t)kt_begin * G256_BK);
-  uint32_t va[8], vb[8];
+  //      (lane & 7) ^ (row & 7) so that readers use lds_slot().  The last tile of a direction begins
+  //      256 before the end (the kernel is taken from 256 rows and tokens on): what it shares with the tile before it, both leave with the same bits ----
+  const char *a_at, *b_at;
+  int m0, t0, nk = K / G256_BK;                    // SILU: m0 = the first of 128 activation columns
+  auto point = [&]() {
+    m0 = SILU ? std::min(so.silu_c0 + mt * 128, silu_cols_end(so) - 128) : std::min(mt * G256_BM, M - G256_BM);
+    t0 = std::min(tt * G256_BT, T - G256_BT);
+    // PART: a K slice of nk_slice K tiles (even and at least four, like the last, shorter one: the tiles are walked in pairs); the workgroup's fp32 tile goes to
+    // part[z][T][M] and a slice-sum launch adds the slices in z order (down_proj at 1-2 k tokens: 40-80 tiles of 256 x 256 for 256 CUs)
+    const int kt_begin = PART ? zslice * nk_slice : 0;
+    if (PART) nk = std::min(nk - kt_begin, nk_slice);
+    a_at = reinterpret_cast<const char*>(W + (size_t)m0 * K + (size_t)kt_begin * G256_BK);
+    b_at = reinterpret_cast<const char*>(X + (size_t)t0 * K + (size_t)kt_begin * G256_BK);
+  };
+  uint32_t piece_at[8];
 #pragma unroll
-  for (int p = 0; p < 8; ++p) {
-    const int r = p * 32 + wave * 8 + (lane >> 3), cs = (lane & 7) ^ (r & 7);
-    int ra, rb = t0 + r;
-    if (SILU) {  // tile = 128 gate rows + their 128 up rows: a wave's m-tiles 0-3 are gate rows, 4-7 the same up rows
-      ra = a_row0 + (r >> 7) * 64 + (r & 63);
-      ra = ra < silu_cols_end(so) ? ra : silu_cols_end(so) - 1;
-    } else {
-      ra = m0 + r;
-      ra = ra < M ? ra : M - 1;
-    }
-    rb = rb < T ? rb : T - 1;
-    va[p] = (uint32_t)(ra - a_row0) * (uint32_t)(K * 2) + cs * 16;
-    vb[p] = (uint32_t)(rb - t0) * (uint32_t)(K * 2) + cs * 16;
-  }
+  for (int p = 0; p < 8; ++p) piece_at[p] = (uint32_t)(p * 32 + wave * 8 + (lane >> 3)) * (uint32_t)(K * 2) + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16u;
+  const int64_t up_rows = SILU ? (int64_t)so.silu_I * K * 2 : 0;
   typedef __attribute__((address_space(3))) void* lptr_t;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)&g256_smem[0] + wave * 1024u);
-  // piece q of a K tile (0-7: W, 8-15: X) in the place of parity par, `at` bytes behind the tile that a_lo, b_at point to: M0, then the load
+  // piece q of a K tile (0-7: W, 8-15: X) in the place of parity par, `at` bytes behind the tile that a_at, b_at point to: M0, then the load
   auto aim = [&](auto q, auto par) {
     const uint32_t to = lds0 + (uint32_t)(decltype(par)::value * 65536 + decltype(q)::value * 4096);
     asm volatile("s_mov_b32 m0, %0" ::"s"(to) : "m0");
   };
-  auto fetch = [&](auto qc, int at) {
+  struct From { const char *a, *up, *b; };         // where a K tile lies in W (SILU: and the up rows) and in X
+  auto from = [&](int at) { return From{a_at + at, a_at + up_rows + at, b_at + at}; };
+  auto fetch = [&](auto qc, const From& f) {
     constexpr int q = decltype(qc)::value;
-    const char* base = (q >= 8 ? b_at : (q & 2) ? a_hi : a_lo) + at;
-    const uint32_t v = q < 8 ? va[q & 7] : vb[q & 7];
+    // SILU: a tile is 128 gate rows and their 128 up rows, a wave's m-tiles 0-3 gate rows, 4-7 the same up rows
+    const char* base = q >= 8 ? f.b : SILU && (q & 2) ? f.up : f.a;
+    const uint32_t v = piece_at[q >= 8 || !SILU ? q & 7 : (q >> 2) * 2 + (q & 1)];
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(v), "s"(base) : "memory");
   };
 
   f32x4 acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   bf16x8_t fa[2][8], fb[2][8];
   // fragments of K step `ks` in the order of their first use: a0, b0 .. b7, a1 .. a7
   auto read = [&](auto qc, auto ksc, auto parc) {
@@ -149,25 +150,24 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
   typedef std::integral_constant<int, 1> P1;
   // the slots of a K tile (see above); a piece whose slot lies behind the last one is fetched by the next K tile
   constexpr int kFree = 36, kLanded = 96, kEvery = 8, kReadEvery = 2;
-  constexpr int kBefore = (128 - kFree + kEvery - 1) / kEvery;       // pieces whose fetch begins in their own K tile's iteration
-
-  // ---- prologue: K tile 0, and of K tile 1 what no iteration fetches ----
-  auto fetch_now = [&](auto q, auto par, int at) {
-    aim(q, par);
-    asm volatile("s_nop 0");
-    fetch(q, at);
+  // K tiles 0 and 1 of the tile that point() was called for (the first iteration fetches the last pieces of K tile 1 again)
+  auto begin = [&]() {
+    auto fetch_now = [&](auto q, auto par, const From& f) {
+      aim(q, par);
+      asm volatile("s_nop 0");
+      fetch(q, f);
+    };
+    const From first = from(0), second = from(128);
+    static_for<16>([&](auto q) { fetch_now(q, P0(), first); });
+    static_for<16>([&](auto q) { fetch_now(q, P1(), second); });
   };
-  static_for<16>([&](auto q) { fetch_now(q, P0(), 0); });
-  static_for<kBefore>([&](auto q) { fetch_now(q, P1(), 128); });
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kBefore) : "memory");
-  __builtin_amdgcn_s_barrier();
-  static_for<16>([&](auto q) { read(q, P0(), P0()); });
 
-  // one K tile in the place of parity par.  MORE: there is a tile after the next to fetch; NEXT: there is a next one
-  auto ktile = [&](auto parc, auto morec, auto nextc) {
+  // one K tile in the place of parity par.  MORE: there is a tile after the next to fetch; NEXT: there is a next one.  there: it has landed already
+  auto ktile = [&](auto parc, auto morec, auto nextc, int there) {
     constexpr int par = decltype(parc)::value;
     constexpr bool MORE = decltype(morec)::value, NEXT = decltype(nextc)::value;
     typedef std::integral_constant<int, par ^ 1> Other;
+    const From next = from(128), after = from(256);
     __builtin_amdgcn_sched_barrier(0);
     static_for<128>([&](auto nc) {
       constexpr int n = decltype(nc)::value, ks = n >> 6;
@@ -179,7 +179,11 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
       }
       if constexpr (NEXT && n == kLanded) {      // the next tile is there; of the one after it, what has been asked for may be on its way
         constexpr int asked = MORE ? (kLanded - 2 - kFree) / kEvery + 1 : 0;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(asked) : "memory");
+        if constexpr (MORE && par == 0 && !PART)
+          asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lthere%=\n\ts_waitcnt vmcnt(%1)\n.Lthere%=:" ::"s"(__builtin_amdgcn_readfirstlane(there)), "i"(asked)
+                       : "memory", "scc");
+        else
+          asm volatile("s_waitcnt vmcnt(%0)" ::"i"(asked) : "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -187,164 +191,206 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
         read(std::integral_constant<int, (n - kLanded) / kReadEvery>(), P0(), Other());
       constexpr int own = n - kFree, late = n + 128 - kFree;
       if constexpr (MORE && own >= 0 && own % kEvery == 0 && own / kEvery < 16) aim(std::integral_constant<int, own / kEvery>(), parc);
-      if constexpr (MORE && own >= 0 && own % kEvery == 1 && own / kEvery < 16) fetch(std::integral_constant<int, own / kEvery>(), 256);
+      if constexpr (MORE && own >= 0 && own % kEvery == 1 && own / kEvery < 16) fetch(std::integral_constant<int, own / kEvery>(), after);
       if constexpr (NEXT && n < kFree && late % kEvery == 0 && late / kEvery < 16) aim(std::integral_constant<int, late / kEvery>(), Other());
-      if constexpr (NEXT && n < kFree && late % kEvery == 1 && late / kEvery < 16) fetch(std::integral_constant<int, late / kEvery>(), 128);
+      if constexpr (NEXT && n < kFree && late % kEvery == 1 && late / kEvery < 16) fetch(std::integral_constant<int, late / kEvery>(), next);
       __builtin_amdgcn_sched_barrier(0);         // a product lies between M0 and the load that reads it
       constexpr int i = (n & 63) >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
+      // as text, so that the sums stay in the accumulator registers between the products, which what reads them at a tile's end pulls them out of
+      // otherwise.  Operands come from LDS or from a product 64 slots before, so that no wait belongs between them and this one
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fa[ks][i]), "v"(fb[ks][j]));
       __builtin_amdgcn_sched_barrier(0);
     });
-    a_lo += 128;
-    a_hi += 128;
+    a_at += 128;
     b_at += 128;
   };
   static_assert(kFree % kEvery != 127 % kEvery, "an aim and its load lie in one iteration");
-  for (int kt = 0; kt + 2 < nk; kt += 2) {
-    ktile(P0(), std::true_type(), std::true_type());
-    ktile(P1(), std::true_type(), std::true_type());
-  }
-  ktile(P0(), std::false_type(), std::true_type());
-  ktile(P1(), std::false_type(), std::false_type());
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
 
-  // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 32 KB of LDS
-  //      (chunks of 16 bytes, XOR-swizzled by the token) and stores whole rows of a token.  `wide`: every row that is written begins on 16 bytes and the
-  //      segments are whole chunks of eight values; else a chunk leaves in halves or value by value ----
-  __syncthreads();                                 // every wave is through with the tiles
-  char* own = reinterpret_cast<char*>(g256_smem) + wave * 32768;
-  if constexpr (PART) {                             // 64 tokens of 512 bytes at a time
-    float* pz = part + (size_t)zslice * T * M;
-    const bool wide = aligned16(pz) && (M & 3) == 0;
-    const int m = m0 + wr * 128 + (lane & 31) * 4;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          *reinterpret_cast<f32x4*>(own + (j * 16 + l15) * 512 + (((i * 4 + g) ^ l15) << 4)) = acc[i][h * 4 + j];
-      auto row = [&](int q, auto&& store) {
-        const int tl = q * 2 + (lane >> 5), t = t0 + wc * 128 + h * 64 + tl;
-        const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((lane & 31) ^ (tl & 15)) << 4));
-        if (t < T && m < M) store(pz + (size_t)t * M + m, v);
-      };
-      if (wide) {
-#pragma unroll 8
-        for (int q = 0; q < 32; ++q) row(q, [](float* to, const f32x4& v) { *reinterpret_cast<f32x4*>(to) = v; });
-      } else {
-#pragma unroll 1
-        for (int q = 0; q < 32; ++q)
-          row(q, [&](float* to, const f32x4& v) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (m + e < M) to[e] = v[e];
-          });
-      }
-    }
-    return;
-  }
-  // the first `left` of four values; `whole` is one for the grid: all four, on 8 bytes, or none
-  auto leave = [&](Half* to, const u32x2& v, int left, bool whole) {
-    if (whole) {
-      if (left > 0) *reinterpret_cast<u32x2*>(to) = v;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (e < left) to[e] = (Half)(v[e >> 1] >> (16 * (e & 1)));
-    }
-  };
-  // rows of 256 bytes
-#pragma unroll
-  for (int j = 0; j < 8; ++j)
+  int item = (int)blockIdx.x;
+  place(item);
+  point();
+  begin();
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  for (bool later = false;; later = true) {
+    __builtin_amdgcn_s_barrier();                  // K tile 0 is there
+    static_for<16>([&](auto q) { read(q, P0(), P0()); });
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      *reinterpret_cast<u32x2*>(own + (j * 16 + l15) * 256 + (((i * 2 + (g >> 1)) ^ l15) << 4) + (g & 1) * 8) =
-          u32x2{pack_bf2(acc[i][j][0], acc[i][j][1]), pack_bf2(acc[i][j][2], acc[i][j][3])};
-  auto chunk_of = [&](int tl, int c) { return *reinterpret_cast<const u32x4*>(own + tl * 256 + ((c ^ (tl & 15)) << 4)); };
-  if constexpr (SILU) {                            // 64 gate values and their 64 up values, bf16 as the GEMM's output is before SwiGLU (fused_proj.cu:57-62)
-    const int end = silu_cols_end(so), m = so.silu_c0 + mt * 128 + wr * 64 + (lane & 7) * 8;
-    const int odd = so.silu_I | so.silu_c0 | end;
-    const bool wide = aligned16(Y) && (odd & 7) == 0, fours = (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (odd & 3) == 0;
-    auto rows = [&](auto roundc) {
-#pragma unroll 2
-      for (int q = 0; q < 16; ++q) {
-        const int tl = q * 8 + (lane >> 3), t = t0 + wc * 128 + tl;
-        const u32x4 ga = chunk_of(tl, lane & 7), up = chunk_of(tl, 8 + (lane & 7));
-        float r[8];
-        auto values = [&](auto silu) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t gw = ga[e >> 1], uw = up[e >> 1];
-            const float sg = silu(e & 1 ? bf_hi(gw) : bf_lo(gw));
-            r[e] = (decltype(roundc)::value ? bf16_round_f(sg) : sg) * (e & 1 ? bf_hi(uw) : bf_lo(uw));
+      for (int j = 0; j < 8; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[i][j]));
+      }
+    asm volatile("s_nop 7" ::: "memory");          // (a product's text tells nobody that a register just written must rest before it)
+    __builtin_amdgcn_sched_barrier(0);
+    int kt = 0;
+    do {
+      ktile(P0(), std::true_type(), std::true_type(), later && kt == 0);
+      ktile(P1(), std::true_type(), std::true_type(), 0);
+      kt += 2;
+    } while (kt + 2 < nk);
+    ktile(P0(), std::false_type(), std::true_type(), 0);
+    ktile(P1(), std::false_type(), std::false_type(), 0);
+    // the last products' way to their registers, which nothing reads before
+    asm volatile("s_nop 15\n\ts_nop 15"
+                 : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7])
+                 :
+                 : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the next tile's first K tiles are asked for before this one's results leave ----
+    const int mw = SILU ? m0 + wr * 64 : m0 + wr * 128, tw = t0 + wc * 128;      // the wave's block
+    item += (int)gridDim.x;
+    const bool more = !PART && item < ntiles;
+    if (more) {
+      __builtin_amdgcn_s_barrier();                // every wave is through with both places
+      place(item);
+      point();
+      begin();
+    }
+
+    // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 8 KB of LDS (chunks
+    //      of 16 bytes, XOR-swizzled by the token), 32 tokens at a time, and stores whole rows of a token.  `wide`: every row that is written begins on
+    //      16 bytes and the segments are whole chunks of eight values; else a chunk leaves in halves or value by value ----
+    const int ln = again(lane), e15 = ln & 15, eg = ln >> 4;
+    char* own = reinterpret_cast<char*>(g256_smem) + kG256LdsBytes + wave * 8192;
+    if constexpr (PART) {                          // 16 tokens of 512 bytes at a time
+      float* pz = part + (size_t)zslice * T * M;
+      const bool wide = aligned16(pz) && (M & 3) == 0;
+      static_for<8>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(own + e15 * 512 + (((i * 4 + eg) ^ e15) << 4)) = acc[i][j];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int tl = q * 2 + (ln >> 5);
+          const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((ln & 31) ^ tl) << 4));
+          float* to = pz + (size_t)(tw + j * 16 + tl) * M + mw + (ln & 31) * 4;
+          if (wide) {
+            *reinterpret_cast<f32x4*>(to) = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) to[e] = v[e];
           }
+        }
+      });
+    } else {
+      // what was asked for lands before the first store: loads and stores do not end in the order in which they were issued, and the next tile's
+      // products are not to wait for these stores
+      auto landed = [&]() {
+        if (more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      };
+      auto chunk_of = [&](int tl, int c) { return reinterpret_cast<u32x4*>(own + tl * 256 + ((c ^ (tl & 15)) << 4)); };
+      auto turn = [&](auto pc) {                   // tokens 32 p .. of the wave's block, rows of 256 bytes
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const f32x4& a = acc[i][decltype(pc)::value * 2 + h];
+            *reinterpret_cast<u32x2*>(own + (h * 16 + e15) * 256 + (((i * 2 + (eg >> 1)) ^ e15) << 4) + (eg & 1) * 8) =
+                u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
+          }
+        __builtin_amdgcn_wave_barrier();
+      };
+      if constexpr (SILU) {                        // 64 gate values and their 64 up values, bf16 as the GEMM's output is before SwiGLU (fused_proj.cu:57-62)
+        const bool wide = aligned16(Y) && ((so.silu_I | m0 | so.silu_c0 | silu_cols_end(so)) & 7) == 0;
+        auto rows = [&](auto roundc) {
+          auto unit = [&](float sg, float up) { return (decltype(roundc)::value ? bf16_round_f(sg) : sg) * up; };
+          Half* to = Y + (size_t)(tw + (ln >> 3)) * so.silu_I + mw + (ln & 7) * 8;
+          u32x4 o[2][4];                           // a pass's results wait while the next one's are made
+          auto leave = [&](auto p) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              Half* at = to + (size_t)(decltype(p)::value * 32 + q * 8) * so.silu_I;
+              const u32x4 v = o[decltype(p)::value & 1][q];
+              if (wide) {
+                *reinterpret_cast<u32x4*>(at) = v;
+              } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) at[e] = (Half)(v[e >> 1] >> (16 * (e & 1)));
+              }
+            }
+          };
+          static_for<4>([&](auto p) {
+            turn(p);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const int tl = q * 8 + (ln >> 3);
+              const u32x4 ga = *chunk_of(tl, ln & 7), up = *chunk_of(tl, 8 + (ln & 7));
+              u32x4& r = o[decltype(p)::value & 1][q];
+              if (__all(silu_mid_ok(ga))) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  r[e] = pack_bf2(unit(silu_mid_f(bf_lo(ga[e])), bf_lo(up[e])), unit(silu_mid_f(bf_hi(ga[e])), bf_hi(up[e])));
+              } else {                             // rare: value by value, in place
+                Half *at = reinterpret_cast<Half*>(chunk_of(tl, ln & 7)), *ua = reinterpret_cast<Half*>(chunk_of(tl, 8 + (ln & 7)));
+#pragma unroll 1
+                for (int e = 0; e < 8; ++e) at[e] = f2bf(unit(silu_f(bf2f(at[e])), bf2f(ua[e])));
+                r = *chunk_of(tl, ln & 7);
+              }
+            }
+            if constexpr (decltype(p)::value == 1) landed();
+            if constexpr (decltype(p)::value >= 1) leave(std::integral_constant<int, decltype(p)::value - 1>());
+          });
+          leave(std::integral_constant<int, 3>());
         };
-        if (__all(silu_mid_ok(ga))) values([](float v) { return silu_mid_f(v); });
-        else values([](float v) { return silu_f(v); });
-        const u32x4 o{pack_bf2(r[0], r[1]), pack_bf2(r[2], r[3]), pack_bf2(r[4], r[5]), pack_bf2(r[6], r[7])};
-        Half* to = Y + (size_t)t * so.silu_I + m;
-        if (t >= T || m >= end) continue;
+        if (so.silu_round) rows(std::true_type());
+        else rows(std::false_type());
+      } else {
+        const bool wide = aligned16(Y) && (M & 7) == 0 &&
+                          (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
+        const bool fours = !so.Y1 && (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (M & 3) == 0;
+        struct Segment { Half* at; int ld, m; };
+        auto segment = [&](int r) {                // where row r goes
+          if (!so.Y1) return Segment{Y, M, r};
+          const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
+          if (r < so.M0) return Segment{Y, so.M0, r};
+          if (r < b1) return Segment{so.Y1, so.M1, r - so.M0};
+          if (r < b2) return Segment{so.Y2, so.M2, r - b1};
+          return Segment{so.Y3, M - b2, r - b2};
+        };
+        const Segment sg = segment(mw + e15 * 8);
         if (wide) {
-          *reinterpret_cast<u32x4*>(to) = o;
+          u32x4 v[32];
+          static_for<4>([&](auto p) {
+            turn(p);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[decltype(p)::value * 8 + q] = *chunk_of(q * 4 + eg, e15);
+          });
+          landed();
+#pragma unroll
+          for (int q = 0; q < 32; ++q) *reinterpret_cast<u32x4*>(sg.at + (size_t)(tw + q * 4 + eg) * sg.ld + sg.m) = v[q];
         } else {
-          leave(to, u32x2{o.x, o.y}, end - m, fours);
-          leave(to + 4, u32x2{o.z, o.w}, end - m - 4, fours);
+          landed();
+          static_for<4>([&](auto p) {
+            turn(p);
+            const int tp = tw + decltype(p)::value * 32;
+            if (fours) {                           // half a chunk a lane
+#pragma unroll 4
+              for (int q = 0; q < 16; ++q) {
+                const int tl = q * 2 + (ln >> 5);
+                *reinterpret_cast<u32x2*>(Y + (size_t)(tp + tl) * M + mw + (ln & 31) * 4) = reinterpret_cast<const u32x2*>(chunk_of(tl, (ln & 31) >> 1))[ln & 1];
+              }
+            } else {                               // a chunk may lie across segments
+#pragma unroll 1
+              for (int v = ln; v < 32 * 128; v += 64) {
+                const int tl = v >> 7, r = v & 127;
+                const Segment one = segment(mw + r);
+                one.at[(size_t)(tp + tl) * one.ld + one.m] = reinterpret_cast<const Half*>(chunk_of(tl, r >> 3))[r & 7];
+              }
+            }
+          });
         }
       }
-    };
-    if (so.silu_round) rows(std::true_type());
-    else rows(std::false_type());
-  } else {
-    const bool whole = aligned16(Y) && (M & 7) == 0;
-    const bool wide = whole && (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
-    const int m = m0 + wr * 128 + l15 * 8;
-    struct Segment { Half* at; int ld, m, end; };
-    auto segment = [&](int r) {                    // where row r goes
-      if (!so.Y1) return Segment{Y, M, r, M};
-      const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
-      if (r < so.M0) return Segment{Y, so.M0, r, so.M0};
-      if (r < b1) return Segment{so.Y1, so.M1, r - so.M0, so.M1};
-      if (r < b2) return Segment{so.Y2, so.M2, r - b1, so.M2};
-      return Segment{so.Y3, M - b2, r - b2, M - b2};
-    };
-    const Segment sg = segment(m);
-    auto row = [&](int q, auto&& store) {
-      const int tl = q * 4 + g, t = t0 + wc * 128 + tl;
-      const u32x4 v = chunk_of(tl, l15);
-      if (t < T && m < M) store(t, v);
-    };
-    if (wide) {
-#pragma unroll 8
-      for (int q = 0; q < 32; ++q) row(q, [&](int t, const u32x4& v) { *reinterpret_cast<u32x4*>(sg.at + (size_t)t * sg.ld + sg.m) = v; });
-    } else if (!so.Y1) {                           // half a chunk a lane
-      const int mh = m0 + wr * 128 + (lane & 31) * 4;
-      const bool fours = (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (M & 3) == 0;
-#pragma unroll 4
-      for (int q = 0; q < 64; ++q) {
-        const int tl = q * 2 + (lane >> 5), t = t0 + wc * 128 + tl;
-        const u32x2 v = *reinterpret_cast<const u32x2*>(own + tl * 256 + ((((lane & 31) >> 1) ^ (tl & 15)) << 4) + (lane & 1) * 8);
-        if (t < T) leave(Y + (size_t)t * M + mh, v, M - mh, fours);
-      }
-    } else {                                       // a chunk may lie across segments
-#pragma unroll 1
-      for (int q = 0; q < 32; ++q)
-        row(q, [&](int t, const u32x4& v) {
-#pragma unroll 1
-          for (int e = 0; e < 8; ++e) {
-            const Segment one = segment(m + e);
-            const uint32_t word = e < 4 ? (e < 2 ? v[0] : v[1]) : (e < 6 ? v[2] : v[3]);
-            if (m + e < M) one.at[(size_t)t * one.ld + one.m] = (Half)(word >> (16 * (e & 1)));
-          }
-        });
     }
+    if (!more) return;
   }
 }
 
-// K must be a multiple of 128 (K tiles are processed in pairs); same alignment rules as the other LDS-DMA kernels
+// K must be a multiple of 128 (K tiles are processed in pairs, two pairs at least); same alignment rules as the other LDS-DMA kernels
 inline bool gemm256_ok(int M, int T, int K) { return (K % 128) == 0 && K >= 256 && M >= 256 && T >= 256; }
 
 inline bool gemm_t_major(int M, int T, const SplitOut& so) {   // PEGAINFER_GEMM_T_MAJOR=0: always row-tile-major runs (A/B)
@@ -364,22 +410,23 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
     const int nch = chunk > 0 ? ceil_div(fast_n, chunk) : 0;
     so.chunk = nch > 1 && (long)m_tiles * t_tiles > 256 ? ceil_div(fast_n, nch) : 0;
   }
+  const int blocks = std::min(m_tiles * t_tiles, device_cus());      // one a compute unit (LDS); a multiple of the XCDs where tiles are left over
   if (silu) {
     static const bool once = [] {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes);
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes + kG256TurnBytes);
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<true><<<m_tiles * t_tiles, 256, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<true><<<blocks, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   } else {
     static const bool once = [] {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes);
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes + kG256TurnBytes);
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<false><<<m_tiles * t_tiles, 256, kG256LdsBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<false><<<blocks, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   }
 }
 
@@ -393,11 +440,11 @@ inline void gemm256_splitk_launch(const Half* W, const Half* X, int M, int T, in
   const int m_tiles = ceil_div(M, G256_BM), t_tiles = ceil_div(T, G256_BT);
   static const bool once = [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false, true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes + kG256TurnBytes);
     return true;
   }();
   (void)once;
-  mfma_gemm256_kernel<false, true><<<dim3(m_tiles * t_tiles, ksplit), 256, kG256LdsBytes, s>>>(
+  mfma_gemm256_kernel<false, true><<<dim3(m_tiles * t_tiles, ksplit), 256, kG256LdsBytes + kG256TurnBytes, s>>>(
       W, X, nullptr, M, T, K, m_tiles, t_tiles,
       SplitOut{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0, 0, ksplit > 1 && splitk_xcd_on(), 0}, part, nk_slice);
 }

@@ -654,6 +654,7 @@ static SplitKPlan splitk_plan(int M, int T, int K, bool assume_ws = false) {
         want = want > 8 ? 8 : want;
         int nk_slice = (ceil_div(nk_all, want) + 1) & ~1;   // K tiles are walked in pairs
         nk_slice = nk_slice < 16 ? 16 : nk_slice;
+        while (nk_all % nk_slice == 2) nk_slice += 2;       // the kernel's slices are two pairs at least
         const int ksplit = ceil_div(nk_all, nk_slice);
         if (ksplit >= 2 && (size_t)ksplit * T * M * 4 <= kSplitKWorkspaceBytes) return {ksplit, nk_slice, 256};
       }

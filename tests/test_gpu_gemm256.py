@@ -24,9 +24,9 @@ def _close(Y, ref, K):
     return bool(((Y.double() - ref).abs() <= 4e-6 * K + ref.abs() * 2.0 ** -8).all())
 
 
-# one K tile pair and more, a row or a token more than whole tiles, rows that end inside a chunk of eight and of four
+# two K tile pairs and more, a row or a token more than whole tiles, rows that end inside a chunk of eight and of four; more tiles than workgroups
 @pytest.mark.parametrize("M,T,K", [(32768, 256, 256), (32768, 257, 384), (16385 + 255, 513, 256), (8193 + 511, 1023, 512), (16396, 511, 256), (5128, 2049, 640),
-                                   (5124, 2305, 256)])
+                                   (5124, 2305, 256), (12800, 2049, 384), (12804, 2100, 256), (2560, 9990, 768)])
 def test_plain(M, T, K):
     from pegainfer_amd import ops as P
     assert _route(M, T, K) in (256, 259)
@@ -48,7 +48,7 @@ def test_segments(parts):
     assert _close(torch.cat(ys, 1), X.double() @ W.double().T, K)
 
 
-@pytest.mark.parametrize("M,T,K", [(2560, 2047, 4096), (2568, 1500, 4224), (2562, 1793, 4096)])
+@pytest.mark.parametrize("M,T,K", [(2560, 2047, 4096), (2568, 1500, 4224), (2562, 1793, 4096), (2048, 1536, 4224)])
 def test_slices_of_k(M, T, K):
     from pegainfer_amd import ops as P
     assert _route(M, T, K) == 1256
@@ -58,7 +58,7 @@ def test_slices_of_k(M, T, K):
     assert _close(Y, X.double() @ W.double().T, K)
 
 
-@pytest.mark.parametrize("I,T,K", [(16384, 256, 256), (9224, 600, 256), (9220, 513, 256), (9219, 512, 384)])
+@pytest.mark.parametrize("I,T,K", [(16384, 256, 256), (9224, 600, 256), (9220, 513, 256), (9219, 512, 384), (12808, 1000, 256), (12801, 1000, 256)])
 def test_gated_unit_has_the_bits_of_product_and_unit(I, T, K):
     from pegainfer_amd import ops as P
     assert _route(0, T, K, I) in (256, 257)
