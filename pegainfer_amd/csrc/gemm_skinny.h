@@ -30,6 +30,8 @@
 // partial sums meet in LDS and are added in fixed wave order.
 #pragma once
 
+#include <type_traits>
+
 #include <cstdio>
 
 #include <cstdlib>
@@ -380,7 +382,8 @@ skinny_tiles_done:
 // ---------------------------------------------------------------------------------------------------
 constexpr int kSkinnyResidentBytes = 128 * 1024;   // o_proj at 16 columns (16 x 4096 x 2 B) is the largest resident x
 
-template <int NB, int EPI>
+// LONG: normed rows of 2560 < K <= 4096, at most 16 of them (an instance of its own: the registers of its prologue cost the others 0.5 us a launch)
+template <int NB, int EPI, bool LONG = false>
 __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const GemvFusedArgs a) {
   constexpr int NW = EPI == kEpiSilu ? 2 : 1;
   constexpr int CH = NW == 1 ? 4 : 2;  // pairs per chunk: 8 (store) / 2x4 (silu) weight loads in flight
@@ -436,16 +439,18 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
   //      trace), so wherever it fits the x side goes FIRST:
   //        plain x (o_proj, down_proj): rows -> swizzled LDS by LDS-DMA (lane l of piece q fetches chunk
   //          (64 q + l) ^ (t & 15), which is what the swizzled slot 64 q + l holds), weights behind, one counted wait;
-  //        add + RMSNorm (qkv, gate_up; K <= 2560, T <= 16): wave w's token rows w, w + 8 (+ residual, + norm weight)
+  //        add + RMSNorm (qkv, gate_up; K <= 4096, T <= 16): wave w's token rows w, w + 8 (+ residual, + norm weight)
   //          into registers first, weights behind; the wave holds its rows in the canonical distribution of
   //          norm_core.h (lane l: vectors l, l + 64, ...), so the sum of squares needs no second pass - same bits.
+  //          K = 4096, four rows (traced): 6144 outputs 19.5 -> 16.6 us, 2 x 12 288 with the gated unit 40.3 -> 37.1; with the rows behind
+  //          the weights and read twice they were there after a third of the launch.
   // kGemvRoundSum (the only flag these kernels take): "add, then norm" - hidden_out = bf16(X + residual) and the norm
   // runs over that ROUNDED sum (add_cuda then rms_norm_batched_cuda: the prefill residual chain, prefill.rs:183 + :89)
   const bool round_sum = (a.flags & kGemvRoundSum) != 0;
-  constexpr int XV = 5;   // 16-byte vectors per lane and row of the register-staged form (K <= 2560)
   const int nvec_row = K >> 3;
   const bool early_plain = !a.norm_w && (K & 511) == 0;
-  const bool early_norm = a.norm_w && nvec_row <= 64 * XV && T <= 2 * kSkinnyWaves;
+  constexpr int kStagedVec = LONG ? 8 : 5;   // 16-byte vectors per lane and row of the register-staged form
+  const bool early_norm = a.norm_w && nvec_row <= 64 * kStagedVec && T <= 2 * kSkinnyWaves;
   if (early_plain) {
     typedef __attribute__((address_space(3))) void* lds_ptr_t;
     const uint32_t xs_lds = (uint32_t)(uintptr_t)(lds_ptr_t)xs;
@@ -465,55 +470,71 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   } else if (early_norm) {
-    u32x4 hx[2][XV], rx[2][XV], gx[XV];
-#pragma unroll
-    for (int j = 0; j < XV; ++j) {
-      const int c = L.lane + 64 * j;
-      if (c < nvec_row) {
-        gx[j] = reinterpret_cast<const u32x4*>(a.norm_w)[c];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int t = L.wave + u * kSkinnyWaves;
-          if (t < T) {
-            hx[u][j] = reinterpret_cast<const u32x4*>(a.X + (size_t)t * K)[c];
-            if (a.residual) rx[u][j] = reinterpret_cast<const u32x4*>(a.residual + (size_t)t * K)[c];
-          }
-        }
-      }
-    }
-    asm volatile("" ::: "memory");   // the x-side loads stay in front of the weight loads
-    if (total > 0) issue(0, avA);
-    if (total > CH) issue(CH, avB);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int t = L.wave + u * kSkinnyWaves;
-      if (t >= T) continue;
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < XV; ++j) {
-        if (L.lane + 64 * j < nvec_row) {
-          if (a.residual && round_sum) add_round_sq8(hx[u][j], rx[u][j], ss);
-          else if (a.residual) add_sq8(hx[u][j], rx[u][j], ss);
-          else sq8(hx[u][j], ss);
-        }
-      }
-      ss = wave_sum(ss);
-      const float inv = rsqrtf(__fadd_rn(ss / (float)K, a.eps));
+    // XV vectors of U rows; LATE: the second chunk of weights is asked for once the first row has left its registers
+    auto stage_norm = [&](auto xv, auto rows, auto late) {
+      constexpr int XV = decltype(xv)::value, U = decltype(rows)::value;
+      constexpr bool LATE = decltype(late)::value;
+      u32x4 hx[U][XV], rx[U][XV], gx[XV];
 #pragma unroll
       for (int j = 0; j < XV; ++j) {
         const int c = L.lane + 64 * j;
         if (c < nvec_row) {
-          u32x4 v;
-          if (a.residual) {
-            u32x4 nh;
-            v = norm_scale8(hx[u][j], &rx[u][j], gx[j], inv, 0.f, &nh, round_sum);
-            if (blockIdx.x == 0) reinterpret_cast<u32x4*>(a.hidden_out + (size_t)t * K)[c] = nh;
-          } else {
-            v = norm_scale8(hx[u][j], nullptr, gx[j], inv, 0.f, nullptr);
+          gx[j] = reinterpret_cast<const u32x4*>(a.norm_w)[c];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int t = L.wave + u * kSkinnyWaves;
+            if (t < T) {
+              hx[u][j] = reinterpret_cast<const u32x4*>(a.X + (size_t)t * K)[c];
+              if (a.residual) rx[u][j] = reinterpret_cast<const u32x4*>(a.residual + (size_t)t * K)[c];
+            }
           }
-          xs[t * pitch + (c ^ (t & 15))] = v;
         }
       }
+      asm volatile("" ::: "memory");   // the x-side loads stay in front of the weight loads
+      if (total > 0) issue(0, avA);
+      if (!LATE && total > CH) issue(CH, avB);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = L.wave + u * kSkinnyWaves;
+        if (t < T) {
+          float ss = 0.f;
+#pragma unroll
+          for (int j = 0; j < XV; ++j) {
+            if (L.lane + 64 * j < nvec_row) {
+              if (a.residual && round_sum) add_round_sq8(hx[u][j], rx[u][j], ss);
+              else if (a.residual) add_sq8(hx[u][j], rx[u][j], ss);
+              else sq8(hx[u][j], ss);
+            }
+          }
+          ss = wave_sum(ss);
+          const float inv = rsqrtf(__fadd_rn(ss / (float)K, a.eps));
+#pragma unroll
+          for (int j = 0; j < XV; ++j) {
+            const int c = L.lane + 64 * j;
+            if (c < nvec_row) {
+              u32x4 v;
+              if (a.residual) {
+                u32x4 nh;
+                v = norm_scale8(hx[u][j], &rx[u][j], gx[j], inv, 0.f, &nh, round_sum);
+                if (blockIdx.x == 0) reinterpret_cast<u32x4*>(a.hidden_out + (size_t)t * K)[c] = nh;
+              } else {
+                v = norm_scale8(hx[u][j], nullptr, gx[j], inv, 0.f, nullptr);
+              }
+              xs[t * pitch + (c ^ (t & 15))] = v;
+            }
+          }
+        }
+        if (LATE && u == 0 && total > CH) issue(CH, avB);
+      }
+    };
+    typedef std::integral_constant<int, 1> One;
+    typedef std::integral_constant<int, 2> Two;
+    typedef std::integral_constant<int, kStagedVec> Vec;
+    if constexpr (LONG) {
+      if (T <= kSkinnyWaves) stage_norm(Vec(), One(), std::false_type());
+      else stage_norm(Vec(), Two(), std::true_type());
+    } else {
+      stage_norm(Vec(), Two(), std::false_type());
     }
     __syncthreads();
   } else {
@@ -721,7 +742,7 @@ inline SkinnyFlushPlan skinny_flush_plan(int nw, int nb, int T, int K, int rows)
   return p;
 }
 
-template <int NB, int EPI>
+template <int NB, int EPI, bool LONG = false>
 inline void skinny_launch_resident(GemvFusedArgs a, hipStream_t s) {
   constexpr int NW = EPI == kEpiSilu ? 2 : 1;
   a.KT = a.K;
@@ -732,7 +753,7 @@ inline void skinny_launch_resident(GemvFusedArgs a, hipStream_t s) {
   const int nrb = fp.nrb, bufs = fp.bufs;
   const int xs_bytes = (a.T * a.K * 2 + 15) & ~15, red_bytes = 8 * NW * NB * 64 * 16;
   const int lds = xs_bytes + bufs * red_bytes + 64 * 4 + 64;
-  auto kern = &skinny_resident_kernel<NB, EPI>;
+  auto kern = &skinny_resident_kernel<NB, EPI, LONG>;
   static const bool once = (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), true);
   (void)once;
@@ -796,7 +817,9 @@ inline bool skinny_dispatch(const GemvFusedArgs& a, hipStream_t s) {
   if (a.T < 2 || a.T > 64 || (a.K & 63) != 0 || (a.T > 8 && (a.K & 127) != 0)) return false;
   constexpr int NW = EPI == kEpiSilu ? 2 : 1;
   const bool resident = skinny_is_resident(NW, a.T, a.K);
-  if (a.T <= 16) { if (resident) skinny_launch_resident<1, EPI>(a, s); else skinny_launch<1, EPI>(a, s); }
+  const bool normed_long = a.norm_w && a.K > 2560 && a.K <= 4096;
+  if (a.T <= 16 && resident && normed_long) skinny_launch_resident<1, EPI, true>(a, s);
+  else if (a.T <= 16) { if (resident) skinny_launch_resident<1, EPI>(a, s); else skinny_launch<1, EPI>(a, s); }
   else if (a.T <= 32) { if (resident) skinny_launch_resident<2, EPI>(a, s); else skinny_launch<2, EPI>(a, s); }
   else { if (resident) skinny_launch_resident<4, EPI>(a, s); else skinny_launch<4, EPI>(a, s); }
   return true;
