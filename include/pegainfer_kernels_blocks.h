@@ -522,6 +522,8 @@ int32_t pegainfer_row_step_ok(int32_t d, int32_t groups, int32_t taps, int64_t s
 pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream);
 /* with the router behind conv_out's row (groups == 0) or xb_out's row (groups > 0); not with y_pairs */
 pegainfer_status_t pegainfer_row_step_routed(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream);
+/* groups == 0 with x_in NULL and row_index NULL: row r's x_in is embed[token_ids[r]] (dtype rows of d values); not with y_pairs */
+pegainfer_status_t pegainfer_row_step_embed(const pegainfer_row_step_desc* q, const void* embed, const uint32_t* token_ids, pegainfer_stream_t stream);
 /* out[row, i] = act(gate[row, i]) * up[row, i], i < I; gate and up are column ranges of rows with stride in_row_stride (elements of
  * dtype).  act 0 = silu, 1 = relu, 2 = gelu (tanh form), 3 = gelu (exact form) */
 enum { PEGAINFER_ACT_SILU = 0, PEGAINFER_ACT_RELU = 1, PEGAINFER_ACT_GELU_TANH = 2, PEGAINFER_ACT_GELU_ERF = 3 };

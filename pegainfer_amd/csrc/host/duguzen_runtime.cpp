@@ -131,8 +131,10 @@ struct Model {
   void* hw = nullptr;
   Half* logits16 = nullptr;      // bf16 image of the wanted rows' logits for the samplers
   struct GraphKey {
-    int n, want; bool tokens, plain; int keys;
-    bool operator==(const GraphKey& o) const { return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && keys == o.keys; }
+    int n, want; bool tokens, plain, every; int keys;
+    bool operator==(const GraphKey& o) const {
+      return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && every == o.every && keys == o.keys;
+    }
   };
   // captured decode steps, one per shape and context length rounded up to 256, 512, ... kGraphMaxKeys tokens.  A capture takes 0.6 - 0.9 ms, about two
   // steps: with bands of 256 tokens a batch met a new one every 256 steps and a few batch sizes filled the cache; so a batch size has six.
@@ -674,6 +676,7 @@ struct Model {
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
     const int32_t *d_pos = md + o_pos, *d_req = md + o_req, *d_ind = md + o_ind, *d_want = md + o_want, *d_pages = md + o_pages;
     const int Ti = (int)T;
+    const bool every = !plain_kernels && D % 4 == 0 && ptiles::all_wanted(want.data(), W, Ti);
     if (tap_on) {
       const size_t needf = layers.size() * T * D;
       if (needf > tap_cap) {
@@ -725,7 +728,7 @@ struct Model {
       const LayerW& w = weights[c.owner];
       const MixerCfg& m = c.mx;
       const int E = c.entry(), Mp = c.proj_rows(), qrow = m.heads * (m.nope + m.rot);
-      const Norm* next_pre = li + 1 < layers.size() ? &weights[layers[li + 1].owner].n1 : nullptr;
+      const Norm* next_pre = li + 1 < layers.size() ? &weights[layers[li + 1].owner].n1 : every ? &final_norm : nullptr;
       if (linear(w.proj, h, proj, Mp, Ti, D)) return -1;
       pegainfer_latent_prep_desc pr{};
       pr.dkv = static_cast<const uint8_t*>(proj) + (size_t)qrow * esize(); pr.dkv_stride = Mp; pr.c_norm_w = w.cnorm;
@@ -799,7 +802,8 @@ struct Model {
     }
     // ---- wanted rows: final norm + head
     if (W > 0) {
-      if (steps) {
+      if (every) {      // the last layer's closing launch has left them normed in h
+      } else if (steps) {
         pegainfer_dyt_step_desc q{};
         q.x = x; q.row_index = d_want; q.d = D; q.rows = W; q.dtype = dtype; q.out = hw;
         set_next(&q, &final_norm);
@@ -809,7 +813,7 @@ struct Model {
         DZ_K(pegainfer_dyt_norm(xw, final_norm.alpha, final_norm.w, final_norm.b, hw, D, W, dtype, S()));
       }
       void* lg = dtype == PEGAINFER_DTYPE_BF16 ? static_cast<void*>(logits16) : logits32;   // the output projection's own type
-      if (linear(head, hw, lg, V, W, D)) return -1;
+      if (linear(head, every ? h : hw, lg, V, W, D)) return -1;
       DZ_K(pegainfer_logits_finish(lg, dtype, logits32, logits16, 1.0f, 0.f, V, W, top1_state, out_tokens ? io.tokens() : nullptr, S()));
     }
     return 0;
@@ -817,7 +821,7 @@ struct Model {
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and replayed; steps with
     // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step at the time (45 now): 9.3 -> 9.05 ms for their prompts and 16 steps.
     if (captured) {
-      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, max_kv};
+      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, every, max_kv};
       hipGraphExec_t exec = graphs.find(key);
       if (!exec) {
         DZ_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));

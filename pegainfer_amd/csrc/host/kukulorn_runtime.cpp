@@ -189,8 +189,10 @@ struct Model {
   int mx_proj = 0, mx_mix = 0, mx_inner = 0, mx_conv = 0, mx_q = 0, mx_ff = 0, mx_vdim = 0;
 
   struct GraphKey {
-    int n, want; bool tokens, plain;
-    bool operator==(const GraphKey& o) const { return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain; }
+    int n, want; bool tokens, plain, every;
+    bool operator==(const GraphKey& o) const {
+      return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && every == o.every;
+    }
   };
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;   // captured decode steps, one per shape
   bool graphs_on = [] { const char* e = getenv("PEGAINFER_KUKULORN_GRAPH"); return !(e && e[0] == '0'); }();
@@ -872,7 +874,7 @@ struct Model {
       for (int k = 0; k < 4; ++k) std::copy(chunk_cols[k]->begin(), chunk_cols[k]->end(), mh + chunk_off[k]);
     }
     KK_HIP(hipEventRecord(ev0, stream));
-    const bool captured = single && graphs_on && !tap_on;
+    const bool captured = single && graphs_on && !tap_on, every = !plain_kernels && ptiles::all_wanted(want.data(), W, (int)T);
     KK_HIP(io.send(words, captured, stream));
     const int32_t* md = io.dev();
     const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(md + o_tok);
@@ -1036,19 +1038,24 @@ struct Model {
         if (linear(w.down, act, y3, D, Ti, c.ff)) return -1;
         terms[n_terms++] = pegainfer_sum_term{y3, D, nullptr, nullptr, 1.0f};
       }
-      // the closing launch also norms for the next run, unless that run opens a pass (its input projection comes first) or
-      // there is none (the final norm runs on the wanted rows only)
-      const bool next_plain = ri + 1 < runs.size() && runs[ri + 1].pass < 0;
-      KK_K(pegainfer_terms_rms_add(x, terms, n_terms, x, next_plain ? weights[(size_t)runs[ri + 1].layer].norm1 : nullptr, eps,
-                                   next_plain ? hb : nullptr, dtype, D, Ti, dtype, S()));
+      // the closing launch also norms for the next run, unless that run opens a pass (its input projection comes first), or behind
+      // the last run for the output table (not where only some rows are wanted: the final norm then runs on those)
+      const bool last = ri + 1 == runs.size(), next_plain = !last && runs[ri + 1].pass < 0;
+      if (last && every)
+        KK_K(pegainfer_terms_rms_add(x, terms, n_terms, x, final_norm, eps, hw, PEGAINFER_DTYPE_F32, D, Ti, dtype, S()));
+      else
+        KK_K(pegainfer_terms_rms_add(x, terms, n_terms, x, next_plain ? weights[(size_t)runs[ri + 1].layer].norm1 : nullptr, eps,
+                                     next_plain ? hb : nullptr, dtype, D, Ti, dtype, S()));
       if (tap_on) KK_HIP(hipMemcpyAsync(tap + ri * T * D, x, T * D * 4, hipMemcpyDeviceToDevice, stream));
     }
     // ---- wanted rows: final norm, logits over the embedding table in fp32, the soft cap
     if (W > 0) {
-      pegainfer_terms_rms_desc fin{};
-      fin.x_in = x; fin.row_index = d_want; fin.gain = final_norm; fin.eps = eps; fin.n_out = hw; fin.n_dtype = PEGAINFER_DTYPE_F32;
-      fin.d = D; fin.rows = W; fin.dtype = dtype;
-      KK_K(pegainfer_terms_rms(&fin, S()));
+      if (!every) {
+        pegainfer_terms_rms_desc fin{};
+        fin.x_in = x; fin.row_index = d_want; fin.gain = final_norm; fin.eps = eps; fin.n_out = hw; fin.n_dtype = PEGAINFER_DTYPE_F32;
+        fin.d = D; fin.rows = W; fin.dtype = dtype;
+        KK_K(pegainfer_terms_rms(&fin, S()));
+      }
       if (linear_strided(embed, hw, PEGAINFER_DTYPE_F32, D, logits32, PEGAINFER_DTYPE_F32, V, W, D)) return -1;
       KK_K(pegainfer_logits_finish(logits32, PEGAINFER_DTYPE_F32, logits32, logits16, 1.0f, logit_cap, V, W, top1_state,
                                    out_tokens ? io.tokens() : nullptr, S()));
@@ -1058,7 +1065,7 @@ struct Model {
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
     if (captured) {
-      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
+      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, every};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
         if (g.first == key) exec = g.second;

@@ -177,8 +177,10 @@ struct Model {
   int mx_proj = 0, mx_mix = 0, mx_conv = 0, mx_q = 0, mx_o = 0, mx_gates = 0, mx_a = 0, mx_ff = 0, mx_top = 0, mx_gu_e = 0, mx_experts = 0, mx_slices = 0, mx_sff = 0;
 
   struct GraphKey {
-    int n, want; bool tokens, plain;
-    bool operator==(const GraphKey& o) const { return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain; }
+    int n, want; bool tokens, plain, every;
+    bool operator==(const GraphKey& o) const {
+      return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && every == o.every;
+    }
   };
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;   // captured decode steps, one per shape
   bool graphs_on = [] { const char* e = getenv("PEGAINFER_RAMALIX_GRAPH"); return !(e && e[0] == '0'); }();
@@ -911,9 +913,10 @@ struct Model {
     // x <- x + mlt (yv + bias) + add_rows + add_vec; with a gain also the norm of the sublayer that follows and its input
     // convolution (hb = n + conv(n), the tail moved on)
     // routed (decode steps): the layer whose experts' rows are still to be summed, in place of yv
+    const bool every = row_steps && ptiles::all_wanted(want.data(), W, Ti);
     auto open_sublayer = [&](const void* yv, const void* bias, float mlt, const float* add_rows, const void* add_vec, bool write_x,
                              const void* gain, const void* conv_w, int64_t st_off, const MlpCfg* routed = nullptr,
-                             const pegainfer_router_tail_desc* router = nullptr) -> int {
+                             const pegainfer_router_tail_desc* router = nullptr, bool first = false, bool last = false) -> int {
       if (row_steps) {
         pegainfer_row_step_desc q{};
         q.x_in = x; q.x_out = write_x || !gain ? x : nullptr; q.y = yv; q.bias = yv ? bias : nullptr; q.mult = mlt;
@@ -927,9 +930,13 @@ struct Model {
           }
         }
         q.add_rows = add_rows; q.add_vec = add_vec; q.gain = gain; q.eps = eps;
-        if (gain) { q.conv_w = conv_w; q.conv_state = state + st_off; q.conv_slot_stride = slot_stride; q.conv_slot = d_slot; q.conv_out = hb; }
+        if (last) q.n_out = hw;
+        else if (gain) { q.conv_w = conv_w; q.conv_state = state + st_off; q.conv_slot_stride = slot_stride; q.conv_slot = d_slot; q.conv_out = hb; }
         q.d = D; q.rows = Ti; q.dtype = dtype;
-        if (router) RX_K(pegainfer_row_step_routed(&q, router, S()));
+        if (first) {
+          q.x_in = nullptr; q.x_out = x;
+          RX_K(pegainfer_row_step_embed(&q, embed, d_tok, S()));
+        } else if (router) RX_K(pegainfer_row_step_routed(&q, router, S()));
         else RX_K(pegainfer_row_step(&q, S()));
         return 0;
       }
@@ -951,7 +958,7 @@ struct Model {
     auto run_layers = [&]() -> int {
     if (std::any_of(runs.begin(), runs.end(), [](const Run& r) { return r.pass > 0; }))      // a later pass reads them again
       RX_K(pegainfer_embed_f32(embed, d_tok, emb, D, Ti, dtype, S()));
-    RX_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));
+    if (!row_steps) RX_K(pegainfer_embed_f32(embed, d_tok, x, D, Ti, dtype, S()));      // otherwise the first sublayer's opening launch reads them
     for (size_t ri = 0; ri < runs.size(); ++ri) {
       const Run& r = runs[ri];
       const LayerCfg& c = layers[(size_t)r.layer];
@@ -961,10 +968,10 @@ struct Model {
         // a pass over the repeated span begins: the embedding rows again (not before the first pass), this pass's own row,
         // and the first sublayer's norm and input convolution
         if (open_sublayer(nullptr, nullptr, 0.f, r.pass > 0 ? emb : nullptr, at(loop_step, (size_t)r.pass * D), true, w.norm1, w.canon1,
-                          r.st_canon1))
+                          r.st_canon1, nullptr, nullptr, ri == 0))
           return -1;
       } else if (ri == 0) {
-        if (open_sublayer(nullptr, nullptr, 0.f, nullptr, nullptr, false, w.norm1, w.canon1, r.st_canon1)) return -1;
+        if (open_sublayer(nullptr, nullptr, 0.f, nullptr, nullptr, false, w.norm1, w.canon1, r.st_canon1, nullptr, nullptr, true)) return -1;
       }   // otherwise the launch that closed the run before has left hb
       if (linear(w.proj, hb, proj, Mp, Ti, D)) return -1;
       if (c.type == kChannelDelta) {
@@ -1026,9 +1033,11 @@ struct Model {
       }
       if (linear(w.o, mix, y, D, Ti, c.mix_cols)) return -1;
       // what the launch that closes this run norms for: the next run's first sublayer, unless that run opens a pass (its own
-      // launch sums first) or there is none (the final norm runs on the wanted rows only)
-      const bool next_plain = ri + 1 < runs.size() && runs[ri + 1].pass < 0;
+      // launch sums first); behind the last run it norms for the output table (not where only some rows are wanted: the final
+      // norm then runs on those)
+      const bool last = ri + 1 == runs.size() && every, next_plain = ri + 1 < runs.size() && runs[ri + 1].pass < 0;
       const LayerW* nw = next_plain ? &weights[(size_t)runs[ri + 1].layer] : nullptr;
+      const void* next_gain = last ? final_norm : nw ? nw->norm1 : nullptr;
       const int64_t next_st = next_plain ? runs[ri + 1].st_canon1 : 0;
       if (c.mlp.kind) {
         // few rows: the launch that leaves a row's feed-forward input also routes it, and the experts' launches find their rows by the choices
@@ -1041,15 +1050,16 @@ struct Model {
         if (f.has_shared) { rt.gate_logit = route_logits + f.experts; rt.gate_stride = f.experts + 1; }
         if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, w.norm2, w.canon2, r.st_canon2, nullptr, chosen ? &rt : nullptr)) return -1;
         if (routed_ff(c, w, Ti, row_steps, chosen)) return -1;
-        if (open_sublayer(y, nullptr, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st, &c.mlp)) return -1;
-      } else if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, nw ? nw->norm1 : nullptr, nw ? nw->canon1 : nullptr, next_st)) {
+        if (open_sublayer(y, nullptr, mult, nullptr, nullptr, true, next_gain, nw ? nw->canon1 : nullptr, next_st, &c.mlp, nullptr, false, last)) return -1;
+      } else if (open_sublayer(y, w.o_bias, mult, nullptr, nullptr, true, next_gain, nw ? nw->canon1 : nullptr, next_st, nullptr, nullptr, false, last)) {
         return -1;
       }
       if (tap_on) RX_HIP(hipMemcpyAsync(tap + ri * T * D, x, T * D * 4, hipMemcpyDeviceToDevice, stream));
     }
     // ---- wanted rows: final norm, logits over the output table in fp32, the constant factor
     if (W > 0) {
-      if (!plain_kernels && pegainfer_row_step_ok(D, 0, 4, 0, 0)) {      // the wanted rows, normed
+      if (every) {      // the last run's closing launch has left them normed
+      } else if (!plain_kernels && pegainfer_row_step_ok(D, 0, 4, 0, 0)) {      // the wanted rows, normed
         pegainfer_row_step_desc q{};
         q.x_in = x; q.row_index = d_want; q.gain = final_norm; q.eps = eps; q.n_out = hw; q.d = D; q.rows = W; q.dtype = dtype;
         RX_K(pegainfer_row_step(&q, S()));
@@ -1066,7 +1076,7 @@ struct Model {
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
     if (captured) {
-      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
+      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, every};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
         if (g.first == key) exec = g.second;

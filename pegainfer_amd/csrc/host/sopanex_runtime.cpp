@@ -520,7 +520,7 @@ class Model : public StepModel {
     for (size_t i = 0; i < layers.size(); ++i) {
       const LayerCfg& c = layers[i];
       const LayerW& w = weights[i];
-      const void* next = i + 1 < layers.size() ? weights[i + 1].norm1 : nullptr;
+      const void* next = i + 1 < layers.size() ? weights[i + 1].norm1 : s.every ? final_norm : nullptr;
       if (linear(w.proj, h, proj, c.proj_rows, s.T, D) || mixer(s, c, w) || linear(w.o, mix, y, D, s.T, c.mix_cols)) return -1;
       const bool routed = c.moe.ff && routed_rows(s, c.moe);
       const pegainfer_router_tail_desc router = router_of(c.moe, w);
@@ -529,10 +529,12 @@ class Model : public StepModel {
       if (tap_on) PSTEP_HIP(hipMemcpyAsync(tap_at((int)i), x, (size_t)s.T * D * 4, hipMemcpyDeviceToDevice, stream));
     }
     if (s.W > 0) {
-      pegainfer_terms_rms_desc d = norm_desc(s.W);
-      d.x_in = x; d.row_index = s.want; d.gain = final_norm; d.n_out = hw;
-      PSTEP_K(pegainfer_terms_rms(&d, S()));
-      if (linear_strided(head, hw, dtype, D, logits32, PEGAINFER_DTYPE_F32, V, s.W, D)) return -1;
+      if (!s.every) {      // otherwise the last layer's closing launch has left them normed in h
+        pegainfer_terms_rms_desc d = norm_desc(s.W);
+        d.x_in = x; d.row_index = s.want; d.gain = final_norm; d.n_out = hw;
+        PSTEP_K(pegainfer_terms_rms(&d, S()));
+      }
+      if (linear_strided(head, s.every ? h : hw, dtype, D, logits32, PEGAINFER_DTYPE_F32, V, s.W, D)) return -1;
     }
     return 0;
   }

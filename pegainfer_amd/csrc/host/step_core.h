@@ -102,6 +102,7 @@ struct ChunkTable {
 struct StepCtx {
   int T = 0, n = 0, W = 0;         // token rows, entries, wanted rows
   bool single = false;             // every entry brings one token: decoding
+  bool every = false;              // every row is wanted, in order: the last layer's closing launch norms them for the output table
   const uint32_t* tokens = nullptr;
   const int32_t* prev = nullptr;   // a row's previous token in its sequence, -1 for the first
   const int32_t *pos = nullptr, *entry = nullptr, *row0 = nullptr, *slot = nullptr, *page_indptr = nullptr, *want = nullptr, *pages = nullptr;
@@ -321,6 +322,7 @@ class StepModel {
       mb[o_row0 + n] = (int32_t)t;
       mb[o_ind + n] = (int32_t)pg;
       for (int i = 0; i < W; ++i) mb[o_want + i] = want[i];
+      c.every = !plain_kernels && ptiles::all_wanted(want.data(), W, c.T);
     }
     std::vector<std::pair<size_t, int>> group_at, flat_at;    // (offset, tiles)
     std::vector<int> group_rows;
@@ -362,7 +364,7 @@ class StepModel {
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and
     // replayed; steps with prompt portions run eagerly
     if (captured) {
-      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels};
+      const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, c.every};
       hipGraphExec_t exec = nullptr;
       for (auto& g : graphs)
         if (g.first == key) exec = g.second;
@@ -607,8 +609,10 @@ class StepModel {
 
  private:
   struct GraphKey {
-    int n, want; bool tokens, plain;
-    bool operator==(const GraphKey& o) const { return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain; }
+    int n, want; bool tokens, plain, every;
+    bool operator==(const GraphKey& o) const {
+      return n == o.n && want == o.want && tokens == o.tokens && plain == o.plain && every == o.every;
+    }
   };
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;   // captured decode steps, one per shape
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -320,7 +320,8 @@ class Model : public StepModel {
     d.x_in = x; d.x_out = x;
     d.y = y; d.y_row_stride = D; d.mix = hc.mix; d.out_w = hc.out; d.mult = residual_mult;
     d.sum_out = sum_out;
-    if (next) { d.read_w = next->in; d.gain = next_norm; d.n_out = h; }
+    if (next) d.read_w = next->in;
+    if (next_norm) { d.gain = next_norm; d.n_out = h; }      // without a reading vector: of the plain sum
     PSTEP_K(pegainfer_stream_mix(&d, S()));
     return 0;
   }
@@ -444,13 +445,15 @@ class Model : public StepModel {
         }
         if (linear(w.down, act, y, D, s.T, c.ff)) return -1;
       }
-      if (join(s, w.hc[c.ff ? 1 : 0], nx ? &nx->hc[0] : nullptr, nx ? nx->norm[0] : nullptr, tap)) return -1;
+      if (join(s, w.hc[c.ff ? 1 : 0], nx ? &nx->hc[0] : nullptr, nx ? nx->norm[0] : s.every ? final_norm : nullptr, tap)) return -1;
     }
     if (s.W > 0) {
-      pegainfer_stream_mix_desc d = stream_desc(s.W);
-      d.x_in = x; d.row_index = s.want; d.gain = final_norm; d.n_out = hw;
-      PSTEP_K(pegainfer_stream_mix(&d, S()));
-      if (linear_strided(head, hw, dtype, D, logits32, PEGAINFER_DTYPE_F32, V, s.W, D)) return -1;
+      if (!s.every) {      // otherwise the last layer's closing launch has left them normed in h
+        pegainfer_stream_mix_desc d = stream_desc(s.W);
+        d.x_in = x; d.row_index = s.want; d.gain = final_norm; d.n_out = hw;
+        PSTEP_K(pegainfer_stream_mix(&d, S()));
+      }
+      if (linear_strided(head, s.every ? h : hw, dtype, D, logits32, PEGAINFER_DTYPE_F32, V, s.W, D)) return -1;
     }
     return 0;
   }

@@ -2,7 +2,8 @@
 //   row_scalar_step_kernel  residual sum with a constant factor (+ bias, + extra rows, + one extra vector), RMS norm with one number as its gain,
 //                           the input convolution of the sublayer that follows (four taps, tail moved on)
 //   row_group_step_kernel   RMS norm in groups of a sublayer's output, residual sum, weighted sum over earlier streams, the same convolution
-// The sublayer's output may be the weighted sum of routed experts, made on the way.
+// The sublayer's output may be the weighted sum of routed experts, made on the way.  A step's first row comes from the embedding table itself (in a
+// launch of its own: 3.7 us a step of 264), and the last is normed for the output table without a convolution.
 // Bound by latency and launches: a thread holds four neighbouring channels (NV times), everything that the row needs - output, stream, earlier
 // streams, weights, the convolution's tail - is requested before the first sum and stays in registers, so a row costs one memory latency, one or
 // two block sums and one round of stores.  8 rows of 1024: routed sum, residual with norm and convolution took 4.2 + 4.4 + 4.5 us in three launches,
@@ -21,6 +22,7 @@ constexpr int kStepGroups = 64;
 template <typename A>
 struct RowStep {
   const float* x_in; const int32_t* row_index; float* x_out;
+  const A* embed; const uint32_t* ids;                       // in place of x_in: a row is its token's embedding row
   const A* y; const A* bias; float mult;
   const float *pairs, *weight; int top;                      // routed: in place of y
   const A* add; const float* add_pairs; int n_add; const float* add_gate; int64_t add_gate_stride;
@@ -136,7 +138,12 @@ __global__ __launch_bounds__(N) void row_scalar_step_kernel(RowStep<A> p, Router
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int u = 0; u < 4; ++u) r[k][u] = 0.f;
-  each_chunk<N, NV>(p.d, [&](int k, int i) { ld4(p.x_in + src + i, r[k]); });
+  if (ROUTED || p.x_in) {
+    each_chunk<N, NV>(p.d, [&](int k, int i) { ld4(p.x_in + src + i, r[k]); });
+  } else {
+    const A* e = p.embed + (int64_t)p.ids[row] * p.d;
+    each_chunk<N, NV>(p.d, [&](int k, int i) { ld4(e + i, r[k]); });
+  }
   if (p.conv_w) conv.request(p, row);
   step_output<A, N, NV, ROUTED>(p, row, y);
   tail.request(router, p.d);
@@ -232,19 +239,20 @@ int32_t pegainfer_row_step_ok(int32_t d, int32_t groups, int32_t taps, int64_t s
          taps == kStepTaps && state_off % 4 == 0 && slot_stride % 4 == 0;
 }
 
-static pegainfer_status_t row_step_launch(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
+static pegainfer_status_t row_step_launch(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, const void* embed, const uint32_t* ids,
+                                          pegainfer_stream_t stream) {
   constexpr pegainfer_status_t bad = (pegainfer_status_t)hipErrorInvalidValue;
   if (!q) return bad;
   if (q->rows <= 0) return 0;
   const bool routed = q->y_pairs != nullptr, grouped = q->groups > 0;
   const void* vectors[] = {q->x_in, q->x_out, q->y, q->bias, q->y_pairs, q->add, q->add_pairs, q->add_rows, q->add_vec, q->n_out, q->xb_out, q->stack,
-                           q->mix_out, q->conv_w, q->conv_state, q->conv_out, grouped ? q->gain : nullptr};
+                           q->mix_out, q->conv_w, q->conv_state, q->conv_out, grouped ? q->gain : nullptr, embed};
   for (const void* v : vectors)
     if (reinterpret_cast<uintptr_t>(v) & (q->dtype == kDtF32 ? 15u : 7u)) return bad;       // fp32 rows: on 16 bytes, below
   const void* wide[] = {q->x_in, q->x_out, q->y_pairs, q->add_pairs, q->add_rows, q->n_out, q->stack, q->mix_out, q->conv_state};
   for (const void* v : wide)
     if (!host_aligned16(v)) return bad;
-  if (!pegainfer_row_step_ok(q->d, q->groups, kStepTaps, 0, q->conv_w ? q->conv_slot_stride : 0) || !q->x_in || (routed && (!q->weight || q->top <= 0 || q->y)) ||
+  if (!pegainfer_row_step_ok(q->d, q->groups, kStepTaps, 0, q->conv_w ? q->conv_slot_stride : 0) || (!q->x_in && !embed) || (routed && (!q->weight || q->top <= 0 || q->y)) ||
       q->n_add < 0 || (q->n_add > 0 && (!q->add_pairs || q->add || !routed)) || (q->add && !routed) ||
       (q->conv_w && (!q->conv_state || !q->conv_slot || !q->conv_out || !q->gain)) ||
       (grouped && (!q->gain || (!q->y && !routed) || q->n_mix < 0 || (q->n_mix > 0 && !q->coef) || (q->n_mix > 1 && !q->stack) ||
@@ -253,13 +261,14 @@ static pegainfer_status_t row_step_launch(const pegainfer_row_step_desc* q, cons
   // what the other form alone works on, and rows picked from a matrix that other workgroups write
   if (grouped ? q->row_index || q->add_rows || q->add_vec || q->n_out : q->stack || q->coef || q->mix_out || q->xb_out) return bad;
   if (q->bias && !q->y) return bad;
+  if (embed && (!ids || q->x_in || q->row_index || routed || grouped || router)) return bad;
   if (q->row_index && q->x_out == q->x_in) return bad;
   RouterTail tail{};
   if (router && (routed || (grouped ? !q->xb_out : !q->conv_w) || !router_tail(router, q->rows, q->d, q->dtype, &tail))) return bad;
   if (!by_dtype(q->dtype, [&](auto* t) {
         using A = std::remove_pointer_t<decltype(t)>;
         auto a = [](const void* p) { return static_cast<const A*>(p); };
-        const RowStep<A> p{q->x_in, q->row_index, q->x_out, a(q->y), a(q->bias), q->mult, q->y_pairs, q->weight, q->top, a(q->add), q->add_pairs, q->n_add,
+        const RowStep<A> p{q->x_in, q->row_index, q->x_out, a(embed), ids, a(q->y), a(q->bias), q->mult, q->y_pairs, q->weight, q->top, a(q->add), q->add_pairs, q->n_add,
                            q->add_gate, q->add_gate_stride, q->add_rows, a(q->add_vec), a(q->gain), q->groups, q->eps, q->n_out,
                            static_cast<A*>(q->xb_out), q->stack, q->stack_stride, a(q->coef), q->n_mix, q->mix_out, a(q->conv_w), q->conv_state,
                            q->conv_slot_stride, q->conv_slot, static_cast<A*>(q->conv_out), q->d, q->rows};
@@ -288,9 +297,12 @@ static pegainfer_status_t row_step_launch(const pegainfer_row_step_desc* q, cons
     return bad;
   return (pegainfer_status_t)hipGetLastError();
 }
-pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream) { return row_step_launch(q, nullptr, stream); }
+pegainfer_status_t pegainfer_row_step(const pegainfer_row_step_desc* q, pegainfer_stream_t stream) { return row_step_launch(q, nullptr, nullptr, nullptr, stream); }
 pegainfer_status_t pegainfer_row_step_routed(const pegainfer_row_step_desc* q, const pegainfer_router_tail_desc* router, pegainfer_stream_t stream) {
-  return router ? row_step_launch(q, router, stream) : (pegainfer_status_t)hipErrorInvalidValue;
+  return router ? row_step_launch(q, router, nullptr, nullptr, stream) : (pegainfer_status_t)hipErrorInvalidValue;
+}
+pegainfer_status_t pegainfer_row_step_embed(const pegainfer_row_step_desc* q, const void* embed, const uint32_t* token_ids, pegainfer_stream_t stream) {
+  return embed ? row_step_launch(q, nullptr, embed, token_ids, stream) : (pegainfer_status_t)hipErrorInvalidValue;
 }
 
 }  // extern "C"
