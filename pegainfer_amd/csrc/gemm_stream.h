@@ -5,13 +5,13 @@
 // 128-row tiles of mfma_gemm_glds_kernel give gate_up (19 456 rows) 152 workgroups - 152 of 256 CUs carry 655 KB each while
 // 104 idle (28 us at 32 columns for 99.6 MB = 3.6 TB/s) - and the small matrices (qkv 48 tiles, o_proj / down_proj 20) had
 // to split K over workgroups and pay fp32 partials + a slice-sum launch.  Here a tile is RT x 16 rows with
-// RT = ceil(ceil(M / CUs) / 16): gate_up 80 rows -> 244 workgroups, qkv 32 -> 192, every one walking the FULL K (no
+// RT = ceil(ceil(M / CUs) / 16), in steps of 8 rows: gate_up 80 rows -> 244 workgroups, qkv 24 -> 256, every one walking the FULL K (no
 // partials, no second launch), all token columns in the workgroup.  o_proj / down_proj (16-row tiles would re-read all of x
 // per 16 rows of W) keep their K slices and slice-sum launch, but the GEMM half is this kernel too (part != nullptr):
 // 256 / slices row tiles, so tiles x slices fill the chip.
 //
 // Structure: LDS-DMA rings of K tiles of 64 as in mfma_gemm_glds_kernel (source-side swizzle, counted vmcnt), but
-//  * four COMPUTE waves side by side along the token axis (TT / 4 tokens each, all RT row blocks): any RT works;
+//  * four COMPUTE waves (two for 32 tokens) side by side along the token axis (TT / 4 tokens each, all RT row blocks): any RT works;
 //  * separate FEEDER waves that only issue the DMAs, the W ring and the X ring each with its own waves and depth: a wave
 //    gets one 1 KB DMA instruction through its issue slot per ~93-133 cycles (18-26 GB/s per wave, however many it keeps in
 //    flight - tools/probes/ingest_probe) and issues nothing else meanwhile, and its loads retire in order (the L2-resident
@@ -35,14 +35,45 @@ namespace pk {
 // bytes cost (W from HBM at ~23 GB/s per CU, X from L2), not by issue + LDS reads + MFMAs of one wave in series.
 // part != nullptr: the K-split form - blockIdx.y = K slice z of nk_slice K tiles (the last one shorter), the workgroup's
 // fp32 tile goes to part[z][T][M] and a slice-sum launch adds the slices in z order (linear.hip, splitk_reduce kernels).
+// 17..32 columns: tiles of 32 tokens, two compute waves.  On the tiles of 64 half of the X pieces that pass a CU's DMA issue and LDS are copies of
+// the last row (stacked qkv: as many as W pieces), and half of the compute waves multiply them.
+// With row tiles in steps of 8 rows, further W feeders and waits that count to the end, cold weights, 64 -> 32 tokens a tile at 32 columns (us): stacked qkv
+// 6144 x 2560 11.7 -> 10.5, 6144 x 4096 16.1 -> 13.7, 11 264 x 2560 16.7 -> 14.3; K slices with their sum, add and norm 2560 x 4096 12.4 -> 11.7, 2560 x 9728
+// 17.0 -> 16.5; SwiGLU 9728 x 2560 22.2 -> 21.1, 12 288 x 4096 44.7 -> 44.2.  33 to 64 columns: 13.3 -> 12.6, 17.5 -> 16.6, 24.3 -> 24.0.  What is left is the
+// rate at which a compute unit takes weights (20 - 22 KB/us) behind 4 us of launch and first flight.
+constexpr int stream_compute_waves(int tt) { return tt == 32 ? 2 : 4; }
+// Waves that feed the W ring.  One for tiles of 32 and 48 rows held their K step to its own issue slot: stacked qkv of 6144 x 2560 over 32 columns 10.9 us
+// with one, 10.5 with two, 10.3 with four; 11 264 x 2560 16.1, 14.4, 14.3 (128-token tiles lose 0.8 - 3 us with more than they have).  For 96 rows over 32 columns a third
+// is worth 0.3 - 0.7 us of 22 and 45 and a fourth costs 1.7; with 80 rows (K slices) a third costs 0.5 - 0.8 of 12 and 17.
+constexpr int stream_w_feeders(int rt, int tt) { return tt == 128 ? (rt >= 4 ? 2 : 1) : rt == 1 ? 1 : rt == 6 && tt == 32 ? 3 : 2; }
+
+// Until at most `tiles` (TILES, or rounded down to a multiple of STEP) K tiles' worth of this wave's DMAs, PER each, are outstanding.  Near the end of K, and from
+// the start where a K slice is shorter than the ring, fewer tiles than the ring holds have been requested: waiting for all of them there
+// put the whole ring's flight in front of its first products (o_proj's slices are 8 tiles; 12.4 -> 11.7 us
+// with its slice sum, tiles of 32 tokens and all).
+template <int TILES, int STEP, int PER>
+__device__ __forceinline__ void wait_but(int tiles) {
+  if constexpr (TILES > 0) {
+    if (tiles >= TILES) {
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(TILES * PER) : "memory");
+      return;
+    }
+    wait_but<(TILES - 1) / STEP * STEP, STEP, PER>(tiles);
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
 template <int RT, int TT, int STW, int STX, int NLW, int NLX, int G>
-__global__ __launch_bounds__((4 + NLW + NLX) * 64) void stream_gemm_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
+__global__ __launch_bounds__((stream_compute_waves(TT) + NLW + NLX) * 64) void stream_gemm_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
                                                                       Half* __restrict__ Y, int M, int T, int K, int m_tiles,
                                                                       int t_tiles, int rows_per_tile, SplitOut so,
                                                                       float* __restrict__ part, int nk_slice) {
   constexpr int NW_ = NLW;                    // waves feeding the W ring
   constexpr int NX_ = NLX;                    // waves feeding the X ring
-  constexpr int TJ = TT / 64;                 // 16-token blocks per compute wave
+  constexpr int CW = stream_compute_waves(TT);
+  constexpr int TJ = TT / 16 / CW;            // 16-token blocks per compute wave
+  constexpr int WSTEP = TT == 128 ? 64 : G;   // (the tiles of 128 tokens gain nothing from counting at the end: 29.7 -> 29.9 us for gate_up)
   constexpr int NWG = RT * 2;                 // 8-row groups of the W tile
   constexpr int NXG = TT / 8;                 // 8-row groups of the X tile
   constexpr int DWW = (NWG + NW_ - 1) / NW_;  // W DMAs per W wave per K tile (groups past NWG re-send the last one)
@@ -68,9 +99,9 @@ __global__ __launch_bounds__((4 + NLW + NLX) * 64) void stream_gemm_kernel(const
   // of the next K step would wait behind W tiles requested for ten steps ahead.  Split by role, each ring has its own
   // depth: W (cold HBM, ~2 us away) 40-48 KB ahead per CU whatever RT is, X (L2-resident, shared by all workgroups) two
   // or more tiles ahead.
-  const int li = wave - 4;                    // feeder index (negative = compute wave)
-  const bool computes = wave < 4;
-  const bool feeds = wave >= 4;
+  const int li = wave - CW;                   // feeder index (negative = compute wave)
+  const bool computes = wave < CW;
+  const bool feeds = wave >= CW;
   const bool w_role = feeds && li < NW_;
   const int ww = w_role ? li : li - NW_;      // index among the feeders of this wave's ring
 
@@ -153,20 +184,17 @@ __global__ __launch_bounds__((4 + NLW + NLX) * 64) void stream_gemm_kernel(const
 #pragma unroll
     for (int p = 0; p < STW - G; ++p)
       if (p < nk) stage_w(p, p);
-    if (nk >= STW - G) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STW - 2 * G) * DWW) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_but<STW - 2 * G, WSTEP, DWW>(min(nk, STW - G) - G);
   } else if (feeds) {
 #pragma unroll
     for (int p = 0; p < STX - G; ++p)
       if (p < nk) stage_x(p, p);
-    if (nk >= STX - G) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STX - 2 * G) * DXX) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_but<STX - 2 * G, WSTEP, DXX>(min(nk, STX - G) - G);
   }
   __syncthreads();
-  const int wt = (wave & 3) * (TT / 4);
+  const int wt = (wave & (CW - 1)) * (TT / CW);
   int curw = 0, nxtw = STW - G, curx = 0, nxtx = STX - G;   // ring slots of tile it G and of the first tile staged during it
   for (int k0 = 0; k0 < nk; k0 += G) {
-    const bool full = w_role ? k0 + STW - 1 < nk : k0 + STX - 1 < nk;   // all G tiles this wave would stage exist
     if (feeds) {
 #pragma unroll
       for (int gi = 0; gi < G; ++gi) {
@@ -202,14 +230,8 @@ __global__ __launch_bounds__((4 + NLW + NLX) * 64) void stream_gemm_kernel(const
         }
       }
     }
-    // in the tail (not all G tiles left to stage) everything outstanding is simply waited for
-    if (w_role) {
-      if (full) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STW - 2 * G) * DWW) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else if (feeds) {
-      if (full) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STX - 2 * G) * DXX) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    if (w_role) wait_but<STW - 2 * G, WSTEP, DWW>(min(nk - k0, STW) - 2 * G);
+    else if (feeds) wait_but<STX - 2 * G, WSTEP, DXX>(min(nk - k0, STX) - 2 * G);
     __syncthreads();
     curw += G; curw = curw >= STW ? curw - STW : curw;
     nxtw += G; nxtw = nxtw >= STW ? nxtw - STW : nxtw;
@@ -307,9 +329,9 @@ inline StreamPlan stream_plan(int M, int silu_cols /* 0 = plain */) {
     if (half_blocks > 3) return {0, 0, 0};
     return {2 * half_blocks, c, ceil_div(silu_cols, c)};
   }
-  int r = ceil_div(ceil_div(M, kCus), 16) * 16;
+  const int r = ceil_div(ceil_div(M, kCus), 8) * 8;
   if (r > 96) return {0, 0, 0};
-  return {r / 16, r, ceil_div(M, r)};
+  return {ceil_div(r, 16), r, ceil_div(M, r)};
 }
 
 // Ring depths and K tiles per barrier.  W: ~2 us x 24 GB/s per CU = 40-48 KB beyond the 2 G tiles the barrier scheme itself
@@ -321,10 +343,13 @@ template <int RT, int TT = 64> struct StreamDepth {
   //                             4: 10 x 8 + 6 x 8 = 128       5: 10 x 10 + 6 x 8 = 148   6: 9 x 12 + 6 x 8 = 156
   // TT = 128 (X tile 16 KB): RT 3: 12 x 6 + 5 x 16 = 152      4: 9 x 8 + 5 x 16 = 152    5: 8 x 10 + 5 x 16 = 160
   //                             6: 6 x 12 + 5 x 16 = 152 (24-48 KB of W ahead; one tile per barrier with 48-60 KB ahead measured the same)
-  static constexpr int G = TT == 64 ? (RT <= 2 ? 4 : 2) : 2;
-  static constexpr int W = TT == 64 ? (RT == 1 ? 24 : RT == 2 ? 16 : RT == 3 ? 12 : RT == 4 ? 10 : RT == 5 ? 10 : 9)
+  // TT = 32 (X tile 4 KB):  RT  1: 24 x 2 + 12 x 4 = 96 KB    2: 22 x 4 + 12 x 4 = 136    3: 14 x 6 + 8 x 4 = 116
+  //                             4: 14 x 8 + 8 x 4 = 144       5: 12 x 10 + 8 x 4 = 152    6: 10 x 12 + 8 x 4 = 152
+  static constexpr int G = TT <= 64 && RT <= 2 ? 4 : 2;
+  static constexpr int W = TT == 32 ? (RT == 1 ? 24 : RT == 2 ? 22 : RT <= 4 ? 14 : RT == 5 ? 12 : 10)
+                         : TT == 64 ? (RT == 1 ? 24 : RT == 2 ? 16 : RT == 3 ? 12 : RT == 4 ? 10 : RT == 5 ? 10 : 9)
                                     : (RT <= 2 ? 16 : RT == 3 ? 12 : RT == 4 ? 9 : RT == 5 ? 8 : 6);   // RT 2: 16 x 4 + 5 x 16 = 144 KB
-  static constexpr int X = TT == 64 ? (RT <= 2 ? 12 : 6) : 5;
+  static constexpr int X = TT == 32 ? (RT <= 2 ? 12 : 8) : TT == 64 ? (RT <= 2 ? 12 : 6) : 5;
 };
 
 template <int RT, int TT, int NLW, int NLX>
@@ -344,14 +369,14 @@ inline void stream_gemm_launch_nl(const Half* W, const Half* X, Half* Y, int M, 
   const int t_tiles = ceil_div(T, TT);
   SplitOut sk = so;
   sk.w_nt = t_tiles == 1 && weights_nt_on();
-  stream_gemm_kernel<RT, TT, STW, STX, NLW, NLX, G><<<pl.m_tiles * t_tiles, (4 + NLW + NLX) * 64, kLds, s>>>(
+  stream_gemm_kernel<RT, TT, STW, STX, NLW, NLX, G><<<pl.m_tiles * t_tiles, (stream_compute_waves(TT) + NLW + NLX) * 64, kLds, s>>>(
       W, X, Y, M, T, K, pl.m_tiles, t_tiles, pl.rows_per_tile, sk, nullptr, 0);
 }
 // K-split launch (T <= TT): grid (row tiles, K slices), fp32 partials into part[ksplit][T][M]
 template <int RT, int TT>
 inline void stream_splitk_launch_rt(const Half* W, const Half* X, int M, int T, int K, const StreamPlan& pl, float* part,
                                     int ksplit, int nk_slice, hipStream_t s) {
-  constexpr int NLW = RT >= 4 ? 2 : 1, NLX = RT <= 2 ? TT / 16 : TT / 32;
+  constexpr int NLW = stream_w_feeders(RT, TT), NLX = RT <= 2 ? TT / 16 : TT / 32;
   constexpr int STW = StreamDepth<RT, TT>::W, STX = StreamDepth<RT, TT>::X, G = StreamDepth<RT, TT>::G;
   constexpr int kLds = (STW * RT * 16 + STX * TT) * 8 * 16;
   static const bool once = [] {
@@ -361,7 +386,7 @@ inline void stream_splitk_launch_rt(const Half* W, const Half* X, int M, int T, 
   }();
   (void)once;
   SplitOut sk{nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0, weights_nt_on()};
-  stream_gemm_kernel<RT, TT, STW, STX, NLW, NLX, G><<<dim3(pl.m_tiles, ksplit), (4 + NLW + NLX) * 64, kLds, s>>>(
+  stream_gemm_kernel<RT, TT, STW, STX, NLW, NLX, G><<<dim3(pl.m_tiles, ksplit), (stream_compute_waves(TT) + NLW + NLX) * 64, kLds, s>>>(
       W, X, nullptr, M, T, K, pl.m_tiles, 1, pl.rows_per_tile, sk, part, nk_slice);
 }
 // Row tiles of the K-split form: as many as fill the chip together with the K slices (256 / ksplit row tiles; o_proj /
@@ -385,15 +410,20 @@ inline bool stream_splitk_launch(const Half* W, const Half* X, int M, int T, int
       default: return false;
     }
   }
-  switch (pl.rt) {
-    case 1: stream_splitk_launch_rt<1, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    case 2: stream_splitk_launch_rt<2, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    case 3: stream_splitk_launch_rt<3, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    case 4: stream_splitk_launch_rt<4, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    case 5: stream_splitk_launch_rt<5, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    case 6: stream_splitk_launch_rt<6, 64>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
-    default: return false;
-  }
+  auto columns = [&](auto tt) {
+    constexpr int TT = decltype(tt)::value;
+    switch (pl.rt) {
+      case 1: stream_splitk_launch_rt<1, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      case 2: stream_splitk_launch_rt<2, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      case 3: stream_splitk_launch_rt<3, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      case 4: stream_splitk_launch_rt<4, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      case 5: stream_splitk_launch_rt<5, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      case 6: stream_splitk_launch_rt<6, TT>(W, X, M, T, K, pl, part, ksplit, nk_slice, s); return true;
+      default: return false;
+    }
+  };
+  if (T <= 32) return columns(std::integral_constant<int, 32>());
+  return columns(std::integral_constant<int, 64>());
 }
 
 // Feeder waves: a wave moves ~18 GB/s of 8-row x 128-B tile pieces through its DMA issue slot (ingest_probe, tile walk),
@@ -402,13 +432,18 @@ inline bool stream_splitk_launch(const Half* W, const Half* X, int M, int T, int
 template <int RT, int TT>
 inline void stream_gemm_launch_rt(const Half* W, const Half* X, Half* Y, int M, int T, int K, const StreamPlan& pl,
                                   const SplitOut& so, hipStream_t s) {
-  constexpr int NLW = RT >= 4 ? 2 : 1, NLX = RT <= 2 ? TT / 16 : TT / 32;   // X: 2 (x-dominated tiles; 1 measured no better) or 4 instructions per wave and K tile
+  constexpr int NLW = stream_w_feeders(RT, TT), NLX = RT <= 2 ? TT / 16 : TT / 32;   // X: 2 (x-dominated tiles; 1 measured no better) or 4 instructions per wave and K tile
   stream_gemm_launch_nl<RT, TT, NLW, NLX>(W, X, Y, M, T, K, pl, so, s);
 }
 template <int TT>
 inline bool stream_gemm_launch(const Half* W, const Half* X, Half* Y, int M, int T, int K, const SplitOut& so, hipStream_t s) {
-  const StreamPlan pl = stream_plan(M, so.silu_I > 0 ? silu_cols_end(so) - so.silu_c0 : 0);
-  if constexpr (TT == 64) {
+  StreamPlan pl = stream_plan(M, so.silu_I > 0 ? silu_cols_end(so) - so.silu_c0 : 0);
+  if (TT == 128 && so.silu_I <= 0) {           // whole blocks: every further workgroup pulls 128 rows of x past the same L2 (256 instead of 192: 18.8 -> 19.1 us)
+    pl.rows_per_tile = pl.rt * 16;
+    pl.m_tiles = ceil_div(M, pl.rows_per_tile);
+  }
+  if constexpr (TT <= 64) {
+    if (TT == 64 && T <= 32) return stream_gemm_launch<32>(W, X, Y, M, T, K, so, s);
     if (pl.rt == 1) { stream_gemm_launch_rt<1, TT>(W, X, Y, M, T, K, pl, so, s); return true; }
     if (pl.rt == 2) { stream_gemm_launch_rt<2, TT>(W, X, Y, M, T, K, pl, so, s); return true; }
   }
