@@ -37,6 +37,7 @@
 
 #include "graph_capture.h"
 #include "kv_pool.h"
+#include "pinned_word.h"
 #include "optional_scratch.h"
 #include "row_tiles.h"
 #include "seq_state.h"
@@ -177,7 +178,7 @@ struct Model {
   uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
-  int32_t* sample_out_d = nullptr;
+  PinnedWord sample_out;
   int last_rows = 0;
   std::vector<float> lp_row;
   bool tap_on = false;
@@ -409,7 +410,7 @@ struct Model {
     if (dalloc_a(&cache, (size_t)num_pages * (size_t)page_stride)) return -1;
     if (dalloc(&state, (size_t)max_requests * (size_t)std::max<int64_t>(1, state_layout.floats_per_slot()))) return -1;
     if (dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
-        dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1))
+        dalloc(&valid_scratch, 1) || (sample_out.alloc() && (set_error("no pinned memory for a sampled token"), true)))
       return -1;
     return 0;
   }
@@ -1097,14 +1098,15 @@ struct Model {
     if (row < 0 || row >= last_rows) return set_error("no logits for that row");
     const Half* lg = logits16 + (size_t)row * V;
     if ((temperature <= 0.0f || top_k == 1) && top_p >= 1.0f) {
-      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out_d, V, S());
+      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out.p, V, S());
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      KK_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
+      KK_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out.p, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
     }
     KK_HIP(hipStreamSynchronize(stream));
-    KK_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));
+    if (!out) { set_error("no place for the sampled token"); return -1; }
+    *out = *sample_out.p;
     return 0;
   }
   int logprobs(int row, uint32_t token, int top_k, float* out_lp, uint32_t* top_ids, float* top_lps) {

@@ -17,6 +17,7 @@
 
 #include "graph_capture.h"
 #include "kv_pool.h"
+#include "pinned_word.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_ext.h"
@@ -111,7 +112,7 @@ struct Model35 {
   uint8_t* sample_scratch = nullptr;
   Half* top1_value = nullptr;
   uint8_t *row_states = nullptr, *valid_scratch = nullptr;
-  int32_t* sample_out_d = nullptr;
+  PinnedWord sample_out;
   std::vector<uint16_t> lp_bits;
   std::vector<float> lp_row;
   uint8_t *meta_host = nullptr, *meta_dev = nullptr;
@@ -236,7 +237,7 @@ struct Model35 {
         dalloc(&gate_out, bs * I) || dalloc(&up_out, bs * I) || dalloc(&act_out, bs * I) ||
         dalloc(&mlp_out, bs * H) || dalloc(&logits, bs * (size_t)V) ||
         dalloc(&top1_state, bs * 16) || dalloc(&start_pos_d, 1) || dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) ||
-        dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1) ||
+        dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) || (sample_out.alloc() && (set_error("no pinned memory for a sampled token"), true)) ||
         dalloc(&wide, (size_t)kFusedBatch * std::max(C + Z + 2 * vh, 2 * q_dim + 2 * kv_dim)) ||
         dalloc(&split_tmp_v, bs * pq::kSplitMaxChunksPerRequest * q_dim) ||
         dalloc(&split_tmp_s, bs * pq::kSplitMaxChunksPerRequest * Hq) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&lin_ticket, bs * (size_t)kh) || dalloc(&pf_last, H) ||
@@ -913,15 +914,16 @@ struct Model35 {
     if (!last_logits || column < 0 || column >= last_rows) { set_error("no logits for that column"); return -1; }
     const Half* lg = last_logits + (size_t)column * V;
     if ((temperature <= 0.0f || top_k == 1) && top_p >= 1.0f) {
-      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out_d, V, S());
+      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out.p, V, S());
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      P35_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
+      P35_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out.p, V, 1.0f / temperature, top_k, top_p,
                                           (uint64_t)bits, S()));
     }
     P35_HIP(hipStreamSynchronize(stream));
-    P35_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));
+    if (!out) { set_error("no place for the sampled token"); return -1; }
+    *out = *sample_out.p;
     return 0;
   }
   // extract_logprobs (executor.rs:807-816 of the qwen3 crate; the qwen35 crate shares the engine types): row -> host f32 ->

@@ -19,6 +19,7 @@
 
 #include "graph_capture.h"
 #include "kv_pool.h"
+#include "pinned_word.h"
 #include "safetensors_loader.h"
 #include "pegainfer_kernels.h"
 #include "pegainfer_kernels_ext.h"
@@ -124,7 +125,7 @@ struct Model {
   Half* top1_value = nullptr;
   uint8_t* row_states = nullptr;
   uint8_t* valid_scratch = nullptr;
-  int32_t* sample_out_d = nullptr;
+  PinnedWord sample_out;
   // metadata
   MetaLayout ml;
   uint8_t* meta_host = nullptr;  // pinned
@@ -230,7 +231,7 @@ struct Model {
         dalloc(&logits, bs * (size_t)V) || dalloc(&split_tmp_v, slots * q_dim) || dalloc(&split_tmp_s, slots * Hq) ||
         dalloc(&top1_state, bs * 16) || dalloc(&merge_ctr, bs * (size_t)Hkv * 32) || dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) ||
         dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) || dalloc(&valid_scratch, 1) ||
-        dalloc(&sample_out_d, 1))
+        (sample_out.alloc() && (set_error("no pinned memory for a sampled token"), true)))
       return -1;
     // packed metadata block
     auto al = [](size_t x) { return (x + 63) & ~size_t(63); };
@@ -1350,15 +1351,16 @@ struct Model {
     if (!last_logits || column < 0 || column >= last_rows) { set_error("no logits for that column"); return -1; }
     const Half* lg = last_logits + (size_t)column * V;
     if ((temperature <= 0.0f || top_k == 1) && top_p >= 1.0f) {
-      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out_d, V, S());
+      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out.p, V, S());
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      PQ_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p,
+      PQ_HIP((hipError_t)pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out.p, V, 1.0f / temperature, top_k, top_p,
                                           (uint64_t)bits, S()));
     }
     PQ_HIP(hipStreamSynchronize(stream));
-    PQ_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));
+    if (!out) { set_error("no place for the sampled token"); return -1; }
+    *out = *sample_out.p;
     return 0;
   }
 

@@ -27,6 +27,7 @@
 
 #include "graph_capture.h"
 #include "kv_pool.h"
+#include "pinned_word.h"
 #include "row_tiles.h"
 #include "seq_state.h"
 #include "step_io.h"
@@ -175,7 +176,7 @@ class StepModel {
     if (dalloc_a(&cache, (size_t)num_pages * (size_t)page_stride)) return -1;
     if (dalloc(&state, (size_t)max_requests * (size_t)std::max<int64_t>(1, state_layout.floats_per_slot()))) return -1;
     return dalloc(&sample_scratch, (size_t)pegainfer_sample_scratch_bytes(V)) || dalloc(&top1_value, 1) || dalloc(&row_states, 1024 * 1024) ||
-           dalloc(&valid_scratch, 1) || dalloc(&sample_out_d, 1) ? -1 : 0;
+           dalloc(&valid_scratch, 1) || (sample_out.alloc() && (set_error("no pinned memory for a sampled token"), true)) ? -1 : 0;
   }
 
   // ------------------------------------------------------------------ weights
@@ -399,14 +400,15 @@ class StepModel {
     if (row < 0 || row >= last_rows) return set_error("no logits for that row");
     const Half* lg = logits16 + (size_t)row * V;
     if ((temperature <= 0.0f || top_k == 1) && top_p >= 1.0f) {
-      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out_d, V, S());
+      flashinfer_top1_cuda(lg, top1_value, row_states, sample_out.p, V, S());
     } else {
       uint32_t bits;
       std::memcpy(&bits, &random_val, 4);
-      PSTEP_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out_d, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
+      PSTEP_K(pegainfer_sample(lg, sample_scratch, valid_scratch, sample_out.p, V, 1.0f / temperature, top_k, top_p, (uint64_t)bits, S()));
     }
     PSTEP_HIP(hipStreamSynchronize(stream));
-    PSTEP_HIP(hipMemcpy(out, sample_out_d, 4, hipMemcpyDeviceToHost));
+    if (!out) { set_error("no place for the sampled token"); return -1; }
+    *out = *sample_out.p;
     return 0;
   }
   int logprobs(int row, uint32_t token, int top_k, float* out_lp, uint32_t* top_ids, float* top_lps) {
@@ -621,7 +623,7 @@ class StepModel {
   std::vector<int32_t> meta;
   pst::StepIo io;
   Half *logits16 = nullptr, *top1_value = nullptr;
-  int32_t* sample_out_d = nullptr;
+  PinnedWord sample_out;
   uint8_t *top1_state = nullptr, *row_states = nullptr, *valid_scratch = nullptr;
   float* tap = nullptr;
   uint8_t* sample_scratch = nullptr;
