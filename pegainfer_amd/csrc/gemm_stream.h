@@ -38,8 +38,8 @@ namespace pk {
 // 17..32 columns: tiles of 32 tokens, two compute waves.  On the tiles of 64 half of the X pieces that pass a CU's DMA issue and LDS are copies of
 // the last row (stacked qkv: as many as W pieces), and half of the compute waves multiply them.
 // With row tiles in steps of 8 rows, further W feeders and waits that count to the end, cold weights, 64 -> 32 tokens a tile at 32 columns (us): stacked qkv
-// 6144 x 2560 11.7 -> 10.5, 6144 x 4096 16.1 -> 13.7, 11 264 x 2560 16.7 -> 14.3; K slices with their sum, add and norm 2560 x 4096 12.4 -> 11.7, 2560 x 9728
-// 17.0 -> 16.5; SwiGLU 9728 x 2560 22.2 -> 21.1, 12 288 x 4096 44.7 -> 44.2.  33 to 64 columns: 13.3 -> 12.6, 17.5 -> 16.6, 24.3 -> 24.0.  What is left is the
+// 6144 x 2560 11.7 -> 10.5, 6144 x 4096 16.1 -> 13.7, 10 240 x 4096 (40 rows instead of 48) 24.4 -> 18.3, 11 264 x 2560 16.7 -> 14.3; K slices with their sum, add and norm 2560 x 4096 12.4 -> 11.7, 2560 x 9728
+// 17.0 -> 16.5; SwiGLU 9728 x 2560 22.2 -> 21.1, 12 288 x 4096 44.7 -> 44.2.  64 columns: 13.3 -> 12.6, 17.5 -> 16.6, 24.8 -> 22.4, 17.1 -> 17.0; SwiGLU 24.3 -> 24.0.  What is left is the
 // rate at which a compute unit takes weights (20 - 22 KB/us) behind 4 us of launch and first flight.
 constexpr int stream_compute_waves(int tt) { return tt == 32 ? 2 : 4; }
 // Waves that feed the W ring.  One for tiles of 32 and 48 rows held their K step to its own issue slot: stacked qkv of 6144 x 2560 over 32 columns 10.9 us
