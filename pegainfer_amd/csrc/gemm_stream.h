@@ -43,7 +43,7 @@ namespace pk {
 // rate at which a compute unit takes weights (20 - 22 KB/us) behind 4 us of launch and first flight.
 constexpr int stream_compute_waves(int tt) { return tt == 32 ? 2 : 4; }
 // Waves that feed the W ring.  One for tiles of 32 and 48 rows held their K step to its own issue slot: stacked qkv of 6144 x 2560 over 32 columns 10.9 us
-// with one, 10.5 with two, 10.3 with four; 11 264 x 2560 16.1, 14.4, 14.3 (128-token tiles lose 0.8 - 3 us with more than they have).  For 96 rows over 32 columns a third
+// with one, 10.5 with two, 10.3 with four; 11 264 x 2560 16.1, 14.4, 14.3 (128-token tiles lose 0.8 - 5 us of 22 - 33 with more than they have).  For 96 rows over 32 columns a third
 // is worth 0.3 - 0.7 us of 22 and 45 and a fourth costs 1.7; with 80 rows (K slices) a third costs 0.5 - 0.8 of 12 and 17.
 constexpr int stream_w_feeders(int rt, int tt) { return tt == 128 ? (rt >= 4 ? 2 : 1) : rt == 1 ? 1 : rt == 6 && tt == 32 ? 3 : 2; }
 
