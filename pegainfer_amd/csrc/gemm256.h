@@ -37,8 +37,6 @@ constexpr int kG256LdsBytes = 8 * kG256HalfBytes;    // 2 parities x {A_lo, A_hi
 constexpr int kG256TurnBytes = 4 * 8192;             // where the waves turn their results
 enum { kHalfAlo = 0, kHalfAhi = 1, kHalfBlo = 2, kHalfBhi = 3 };
 
-struct G256Out { Half* Y; int ld; };
-
 template <int... I, typename F>
 __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>()), ...); }
 // f(0), f(1), .. f(N - 1), the numbers as types
@@ -251,12 +249,14 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
 
     // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 8 KB of LDS (chunks
     //      of 16 bytes, XOR-swizzled by the token), 32 tokens at a time, and stores whole rows of a token.  `wide`: every row that is written begins on
-    //      16 bytes and the segments are whole chunks of eight values; else a chunk leaves in halves or value by value ----
+    //      16 bytes and the segments are whole chunks of eight values; else a chunk leaves in halves of four values, which no boundary cuts: rows of
+    //      outputs, segments and gated columns are multiples of four and begin on 8 bytes (glds_gemm_ok, pegainfer_gemm_split, gemm_silu_impl).  Value
+    //      by value such segments took 1.5 to 2.5 times as long (M 6144 in 4100 + 1020 + 1024, K 2560, 2048 tokens: 91 us, 56 in halves; 8192
+    //      in 4096 + 2052 + 2044, K 256, 4096 tokens: 89, 26) ----
     const int ln = again(lane), e15 = ln & 15, eg = ln >> 4;
     char* own = reinterpret_cast<char*>(g256_smem) + kG256LdsBytes + wave * 8192;
     if constexpr (PART) {                          // 16 tokens of 512 bytes at a time
-      float* pz = part + (size_t)zslice * T * M;
-      const bool wide = aligned16(pz) && (M & 3) == 0;
+      float* pz = part + (size_t)zslice * T * M;    // the workspace's own start, rows of fours: on 16 bytes
       static_for<8>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         __builtin_amdgcn_wave_barrier();
@@ -267,13 +267,7 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
         for (int q = 0; q < 8; ++q) {
           const int tl = q * 2 + (ln >> 5);
           const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((ln & 31) ^ tl) << 4));
-          float* to = pz + (size_t)(tw + j * 16 + tl) * M + mw + (ln & 31) * 4;
-          if (wide) {
-            *reinterpret_cast<f32x4*>(to) = v;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) to[e] = v[e];
-          }
+          *reinterpret_cast<f32x4*>(pz + (size_t)(tw + j * 16 + tl) * M + mw + (ln & 31) * 4) = v;
         }
       });
     } else {
@@ -309,8 +303,8 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
               if (wide) {
                 *reinterpret_cast<u32x4*>(at) = v;
               } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) at[e] = (Half)(v[e >> 1] >> (16 * (e & 1)));
+                *reinterpret_cast<u32x2*>(at) = u32x2{v[0], v[1]};
+                *reinterpret_cast<u32x2*>(at + 4) = u32x2{v[2], v[3]};
               }
             }
           };
@@ -342,7 +336,6 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
       } else {
         const bool wide = aligned16(Y) && (M & 7) == 0 &&
                           (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
-        const bool fours = !so.Y1 && (reinterpret_cast<uintptr_t>(Y) & 7) == 0 && (M & 3) == 0;
         struct Segment { Half* at; int ld, m; };
         auto segment = [&](int r) {                // where row r goes
           if (!so.Y1) return Segment{Y, M, r};
@@ -352,8 +345,8 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
           if (r < b2) return Segment{so.Y2, so.M2, r - b1};
           return Segment{so.Y3, M - b2, r - b2};
         };
-        const Segment sg = segment(mw + e15 * 8);
         if (wide) {
+          const Segment sg = segment(mw + e15 * 8);
           u32x4 v[32];
           static_for<4>([&](auto p) {
             turn(p);
@@ -364,23 +357,15 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
 #pragma unroll
           for (int q = 0; q < 32; ++q) *reinterpret_cast<u32x4*>(sg.at + (size_t)(tw + q * 4 + eg) * sg.ld + sg.m) = v[q];
         } else {
+          const Segment half = segment(mw + (ln & 31) * 4);
           landed();
           static_for<4>([&](auto p) {
             turn(p);
             const int tp = tw + decltype(p)::value * 32;
-            if (fours) {                           // half a chunk a lane
 #pragma unroll 4
-              for (int q = 0; q < 16; ++q) {
-                const int tl = q * 2 + (ln >> 5);
-                *reinterpret_cast<u32x2*>(Y + (size_t)(tp + tl) * M + mw + (ln & 31) * 4) = reinterpret_cast<const u32x2*>(chunk_of(tl, (ln & 31) >> 1))[ln & 1];
-              }
-            } else {                               // a chunk may lie across segments
-#pragma unroll 1
-              for (int v = ln; v < 32 * 128; v += 64) {
-                const int tl = v >> 7, r = v & 127;
-                const Segment one = segment(mw + r);
-                one.at[(size_t)(tp + tl) * one.ld + one.m] = reinterpret_cast<const Half*>(chunk_of(tl, r >> 3))[r & 7];
-              }
+            for (int q = 0; q < 16; ++q) {
+              const int tl = q * 2 + (ln >> 5);
+              *reinterpret_cast<u32x2*>(half.at + (size_t)(tp + tl) * half.ld + half.m) = reinterpret_cast<const u32x2*>(chunk_of(tl, (ln & 31) >> 1))[ln & 1];
             }
           });
         }

@@ -36,13 +36,22 @@ def test_plain(M, T, K):
     assert _close(Y, X.double() @ W.double().T, K)
 
 
-# segments on whole chunks, inside a chunk and inside a half
-@pytest.mark.parametrize("parts", [(4096, 1024, 1024), (4100, 1020, 1024), (4097, 1021, 1026), (8, 6128, 8)])
+# segments on whole chunks of eight, and inside a chunk (4 mod 8): the most that the entry point hands to these tiles
+@pytest.mark.parametrize("parts", [(4096, 1024, 1024), (4100, 1020, 1024), (4100, 1020, 1028), (8, 6128, 8), (4, 6136, 4)])
 def test_segments(parts):
     from pegainfer_amd import ops as P
     M, T, K = sum(parts), 1600, 256
-    assert _route(M, T, K) == 256
+    assert _route(M, T, K) == 256 and all(m % 4 == 0 for m in parts)
     W, X = _operands(M, T, K)
+    ys = [torch.full((T, m), float("nan"), device="cuda", dtype=torch.bfloat16) for m in parts]
+    P.gemm_split3_into(W, X, *ys)
+    assert _close(torch.cat(ys, 1), X.double() @ W.double().T, K)
+
+
+def test_segments_that_are_no_fours_run_as_products_of_their_own():
+    from pegainfer_amd import ops as P
+    parts, T, K = (4097, 1021, 1026), 1600, 256
+    W, X = _operands(sum(parts), T, K)
     ys = [torch.full((T, m), float("nan"), device="cuda", dtype=torch.bfloat16) for m in parts]
     P.gemm_split3_into(W, X, *ys)
     assert _close(torch.cat(ys, 1), X.double() @ W.double().T, K)

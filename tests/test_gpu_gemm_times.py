@@ -1,0 +1,39 @@
+"""Times of products that stand beside each other: what differs between the two of a pair is worth a few per cent, and a form that has lost its way out or its
+order of loads is a quarter slower or more.  The line lies between what was measured of both; a form is slower every time, so the best of three counts."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ratio(first, second, n, limit):
+    """median time of `first` over that of `second`, in turn; the best of three"""
+    best = float("inf")
+    for f in (first, second):
+        for i in range(n):
+            f(i)
+    for _ in range(3):
+        times = ([], [])
+        for _ in range(7):
+            for k, f in enumerate((first, second)):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in "ab")
+                a.record()
+                for i in range(n):
+                    f(i)
+                b.record()
+                b.synchronize()
+                times[k].append(a.elapsed_time(b))
+        best = min(best, sorted(times[0])[3] / sorted(times[1])[3])
+        if best < limit:
+            break
+    return best
+
+
+# 4 mod 8 against whole chunks: 1.0 where halves of a chunk leave in 8 bytes, 1.6 / 2.3 / 3.3 value by value
+@pytest.mark.parametrize("cut,whole,T,K", [((4100, 1020, 1024), (4096, 1024, 1024), 2048, 2560), ((8192, 1028, 1020), (8192, 1024, 1024), 2100, 1024),
+                                           ((4096, 2052, 2044), (4096, 2048, 2048), 4096, 256)])
+def test_segments_inside_a_chunk_cost_what_whole_ones_cost(cut, whole, T, K):
+    from pegainfer_amd import ops as P
+    W, X = torch.randn(sum(cut), K, device="cuda").bfloat16(), torch.randn(T, K, device="cuda").bfloat16()
+    ys = [[torch.empty(T, m, device="cuda", dtype=torch.bfloat16) for m in parts] for parts in (cut, whole)]
+    assert _ratio(lambda i: P.gemm_split3_into(W, X, *ys[0]), lambda i: P.gemm_split3_into(W, X, *ys[1]), 10, 1.3) < 1.3
