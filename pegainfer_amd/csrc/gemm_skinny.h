@@ -442,7 +442,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
   //        add + RMSNorm (qkv, gate_up; K <= 4096, T <= 16): wave w's token rows w, w + 8 (+ residual, + norm weight)
   //          into registers first, weights behind; the wave holds its rows in the canonical distribution of
   //          norm_core.h (lane l: vectors l, l + 64, ...), so the sum of squares needs no second pass - same bits.
-  //          K = 4096, four rows (traced): 6144 outputs 19.5 -> 16.6 us, 2 x 12 288 with the gated unit 40.3 -> 37.1; with the rows behind
+  //          K = 4096, three rows, cold weights: 6144 outputs 17.5 -> 15.7 us, 2 x 9728 with the gated unit 32.9 -> 30.9; with the rows behind
   //          the weights and read twice they were there after a third of the launch.
   // kGemvRoundSum (the only flag these kernels take): "add, then norm" - hidden_out = bf16(X + residual) and the norm
   // runs over that ROUNDED sum (add_cuda then rms_norm_batched_cuda: the prefill residual chain, prefill.rs:183 + :89)
@@ -470,18 +470,81 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   } else if (early_norm) {
-    // XV vectors of U rows; LATE: the second chunk of weights is asked for once the first row has left its registers
-    auto stage_norm = [&](auto xv, auto rows, auto late) {
-      constexpr int XV = decltype(xv)::value, U = decltype(rows)::value;
-      constexpr bool LATE = decltype(late)::value;
-      u32x4 hx[U][XV], rx[U][XV], gx[XV];
+    constexpr int XV = kStagedVec;
+    if constexpr (LONG) {
+      // U rows a wave; LATE: the second chunk of weights is asked for once the first row has left its registers.  The wait for the rows is written
+      // out: left to itself the compiler, which cannot count weights that are asked for under a condition, lets the norm wait for all of them
+      // (3072 x 6144, 3 and 9 rows: 13.9 and 16.3 us, 12.5 and 14.6 so; 1024 x 4096, 16 rows 17.0, 15.6)
+      auto stage_norm = [&](auto rows, auto late) {
+        constexpr int U = decltype(rows)::value;
+        constexpr bool LATE = decltype(late)::value;
+        u32x4 hx[U][XV], rx[U][XV], gx[XV];
+#pragma unroll
+        for (int j = 0; j < XV; ++j) {
+          const int c = L.lane + 64 * j;
+          if (c < nvec_row) {
+            gx[j] = reinterpret_cast<const u32x4*>(a.norm_w)[c];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int t = L.wave + u * kSkinnyWaves;
+              if (t < T) {
+                hx[u][j] = reinterpret_cast<const u32x4*>(a.X + (size_t)t * K)[c];
+                if (a.residual) rx[u][j] = reinterpret_cast<const u32x4*>(a.residual + (size_t)t * K)[c];
+              }
+            }
+          }
+        }
+        asm volatile("" ::: "memory");   // the x-side loads stay in front of the weight loads
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        if (total > 0) issue(0, avA);
+        if (!LATE && total > CH) issue(CH, avB);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int t = L.wave + u * kSkinnyWaves;
+          if (t < T) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < XV; ++j) {
+              if (L.lane + 64 * j < nvec_row) {
+                if (a.residual && round_sum) add_round_sq8(hx[u][j], rx[u][j], ss);
+                else if (a.residual) add_sq8(hx[u][j], rx[u][j], ss);
+                else sq8(hx[u][j], ss);
+              }
+            }
+            ss = wave_sum(ss);
+            const float inv = rsqrtf(__fadd_rn(ss / (float)K, a.eps));
+#pragma unroll
+            for (int j = 0; j < XV; ++j) {
+              const int c = L.lane + 64 * j;
+              if (c < nvec_row) {
+                u32x4 v;
+                if (a.residual) {
+                  u32x4 nh;
+                  v = norm_scale8(hx[u][j], &rx[u][j], gx[j], inv, 0.f, &nh, round_sum);
+                  if (blockIdx.x == 0) reinterpret_cast<u32x4*>(a.hidden_out + (size_t)t * K)[c] = nh;
+                } else {
+                  v = norm_scale8(hx[u][j], nullptr, gx[j], inv, 0.f, nullptr);
+                }
+                xs[t * pitch + (c ^ (t & 15))] = v;
+              }
+            }
+          }
+          if (LATE && u == 0 && total > CH) issue(CH, avB);
+        }
+      };
+      if (T <= kSkinnyWaves) stage_norm(std::integral_constant<int, 1>(), std::false_type());
+      else stage_norm(std::integral_constant<int, 2>(), std::true_type());
+    } else {
+      // straight, without the functor above: called for two rows of five vectors that cost 3 to 20 % of the launch (the norm behind all weights),
+      // with its wait written out still up to 5 (6144 x 2560, 9 rows 12.8 us, 14.9, 13.4; 6144 x 1024, 4 rows 5.9, 7.2, 5.8)
+      u32x4 hx[2][XV], rx[2][XV], gx[XV];
 #pragma unroll
       for (int j = 0; j < XV; ++j) {
         const int c = L.lane + 64 * j;
         if (c < nvec_row) {
           gx[j] = reinterpret_cast<const u32x4*>(a.norm_w)[c];
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
+          for (int u = 0; u < 2; ++u) {
             const int t = L.wave + u * kSkinnyWaves;
             if (t < T) {
               hx[u][j] = reinterpret_cast<const u32x4*>(a.X + (size_t)t * K)[c];
@@ -492,49 +555,38 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
       }
       asm volatile("" ::: "memory");   // the x-side loads stay in front of the weight loads
       if (total > 0) issue(0, avA);
-      if (!LATE && total > CH) issue(CH, avB);
+      if (total > CH) issue(CH, avB);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < 2; ++u) {
         const int t = L.wave + u * kSkinnyWaves;
-        if (t < T) {
-          float ss = 0.f;
+        if (t >= T) continue;
+        float ss = 0.f;
 #pragma unroll
-          for (int j = 0; j < XV; ++j) {
-            if (L.lane + 64 * j < nvec_row) {
-              if (a.residual && round_sum) add_round_sq8(hx[u][j], rx[u][j], ss);
-              else if (a.residual) add_sq8(hx[u][j], rx[u][j], ss);
-              else sq8(hx[u][j], ss);
-            }
-          }
-          ss = wave_sum(ss);
-          const float inv = rsqrtf(__fadd_rn(ss / (float)K, a.eps));
-#pragma unroll
-          for (int j = 0; j < XV; ++j) {
-            const int c = L.lane + 64 * j;
-            if (c < nvec_row) {
-              u32x4 v;
-              if (a.residual) {
-                u32x4 nh;
-                v = norm_scale8(hx[u][j], &rx[u][j], gx[j], inv, 0.f, &nh, round_sum);
-                if (blockIdx.x == 0) reinterpret_cast<u32x4*>(a.hidden_out + (size_t)t * K)[c] = nh;
-              } else {
-                v = norm_scale8(hx[u][j], nullptr, gx[j], inv, 0.f, nullptr);
-              }
-              xs[t * pitch + (c ^ (t & 15))] = v;
-            }
+        for (int j = 0; j < XV; ++j) {
+          if (L.lane + 64 * j < nvec_row) {
+            if (a.residual && round_sum) add_round_sq8(hx[u][j], rx[u][j], ss);
+            else if (a.residual) add_sq8(hx[u][j], rx[u][j], ss);
+            else sq8(hx[u][j], ss);
           }
         }
-        if (LATE && u == 0 && total > CH) issue(CH, avB);
+        ss = wave_sum(ss);
+        const float inv = rsqrtf(__fadd_rn(ss / (float)K, a.eps));
+#pragma unroll
+        for (int j = 0; j < XV; ++j) {
+          const int c = L.lane + 64 * j;
+          if (c < nvec_row) {
+            u32x4 v;
+            if (a.residual) {
+              u32x4 nh;
+              v = norm_scale8(hx[u][j], &rx[u][j], gx[j], inv, 0.f, &nh, round_sum);
+              if (blockIdx.x == 0) reinterpret_cast<u32x4*>(a.hidden_out + (size_t)t * K)[c] = nh;
+            } else {
+              v = norm_scale8(hx[u][j], nullptr, gx[j], inv, 0.f, nullptr);
+            }
+            xs[t * pitch + (c ^ (t & 15))] = v;
+          }
+        }
       }
-    };
-    typedef std::integral_constant<int, 1> One;
-    typedef std::integral_constant<int, 2> Two;
-    typedef std::integral_constant<int, kStagedVec> Vec;
-    if constexpr (LONG) {
-      if (T <= kSkinnyWaves) stage_norm(Vec(), One(), std::false_type());
-      else stage_norm(Vec(), Two(), std::true_type());
-    } else {
-      stage_norm(Vec(), Two(), std::false_type());
     }
     __syncthreads();
   } else {

@@ -37,3 +37,20 @@ def test_segments_inside_a_chunk_cost_what_whole_ones_cost(cut, whole, T, K):
     W, X = torch.randn(sum(cut), K, device="cuda").bfloat16(), torch.randn(T, K, device="cuda").bfloat16()
     ys = [[torch.empty(T, m, device="cuda", dtype=torch.bfloat16) for m in parts] for parts in (cut, whole)]
     assert _ratio(lambda i: P.gemm_split3_into(W, X, *ys[0]), lambda i: P.gemm_split3_into(W, X, *ys[1]), 10, 1.3) < 1.3
+
+
+# few rows with their norm in front against the product alone: 1.11 / 1.21 / 1.19 / 1.14 where the norm waits for its rows, 1.34 / 1.33 / 1.36 / 1.26 where it
+# waits for the weights behind them too
+@pytest.mark.parametrize("T,K,residual,limit", [(4, 1024, True, 1.24), (9, 2560, False, 1.27), (9, 3072, False, 1.28), (3, 3072, False, 1.20)])
+def test_norm_in_front_of_few_rows_does_not_wait_for_weights(T, K, residual, limit):
+    from pegainfer_amd import ffi
+    M, lib, s = 6144, ffi.lib(), torch.cuda.current_stream().cuda_stream
+    n = int(4e8 / (2 * M * K))                       # more weights than the last cache holds
+    W = torch.randn(n, M, K, device="cuda").bfloat16()
+    X, R, left, gain = (torch.randn(T, K, device="cuda").bfloat16() for _ in range(4))
+    Y = torch.empty(T, M, device="cuda", dtype=torch.bfloat16)
+
+    def run(i, norm):
+        assert lib.pegainfer_gemv_fused(W[i].data_ptr(), X.data_ptr(), Y.data_ptr(), M, T, K, R.data_ptr() if norm and residual else None, gain.data_ptr() if norm else None,
+                                        left.data_ptr() if norm and residual else None, 1e-6, 0, s) == 0
+    assert _ratio(lambda i: run(i, True), lambda i: run(i, False), n, limit) < limit
