@@ -344,9 +344,11 @@ template <int RT, int TT = 64> struct StreamDepth {
   // TT = 128 (X tile 16 KB): RT 3: 12 x 6 + 5 x 16 = 152      4: 9 x 8 + 5 x 16 = 152    5: 8 x 10 + 5 x 16 = 160
   //                             6: 6 x 12 + 5 x 16 = 152 (24-48 KB of W ahead; one tile per barrier with 48-60 KB ahead measured the same)
   // TT = 32 (X tile 4 KB):  RT  1: 24 x 2 + 12 x 4 = 96 KB    2: 22 x 4 + 12 x 4 = 136    3: 14 x 6 + 8 x 4 = 116
-  //                             4: 14 x 8 + 8 x 4 = 144       5: 12 x 10 + 8 x 4 = 152    6: 10 x 12 + 8 x 4 = 152
+  //                             4: 8 x 8 + 8 x 4 = 96         5: 12 x 10 + 8 x 4 = 152    6: 10 x 12 + 8 x 4 = 152
+  // A feeder requests its whole ring before its first wait.  64 rows over 32 columns, rings of 14 / 12 / 10 / 8 tiles (tiles of 64 columns: 10), us: 16 384 x
+  // 1024 9.4 / 9.0 / 8.6 / 8.2 (9.2), 16 384 x 4096 27.5 / 27.4 / 26.8 / 26.6 (27.9), gated 8192 x 1024 9.8 / 9.5 / 9.0 / 8.6 (9.5), slices of 2048 x 6144 10.4 / 10.2 / 9.9 / 9.6.
   static constexpr int G = TT <= 64 && RT <= 2 ? 4 : 2;
-  static constexpr int W = TT == 32 ? (RT == 1 ? 24 : RT == 2 ? 22 : RT <= 4 ? 14 : RT == 5 ? 12 : 10)
+  static constexpr int W = TT == 32 ? (RT == 1 ? 24 : RT == 2 ? 22 : RT == 3 ? 14 : RT == 4 ? 8 : RT == 5 ? 12 : 10)
                          : TT == 64 ? (RT == 1 ? 24 : RT == 2 ? 16 : RT == 3 ? 12 : RT == 4 ? 10 : RT == 5 ? 10 : 9)
                                     : (RT <= 2 ? 16 : RT == 3 ? 12 : RT == 4 ? 9 : RT == 5 ? 8 : 6);   // RT 2: 16 x 4 + 5 x 16 = 144 KB
   static constexpr int X = TT == 32 ? (RT <= 2 ? 12 : 8) : TT == 64 ? (RT <= 2 ? 12 : 6) : 5;

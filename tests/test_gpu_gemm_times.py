@@ -49,8 +49,20 @@ def test_norm_in_front_of_few_rows_does_not_wait_for_weights(T, K, residual, lim
     W = torch.randn(n, M, K, device="cuda").bfloat16()
     X, R, left, gain = (torch.randn(T, K, device="cuda").bfloat16() for _ in range(4))
     Y = torch.empty(T, M, device="cuda", dtype=torch.bfloat16)
+    w, x, y, plain = [v.data_ptr() for v in W], X.data_ptr(), Y.data_ptr(), (None, None, None)
+    normed = (R.data_ptr() if residual else None, gain.data_ptr(), left.data_ptr() if residual else None)
 
-    def run(i, norm):
-        assert lib.pegainfer_gemv_fused(W[i].data_ptr(), X.data_ptr(), Y.data_ptr(), M, T, K, R.data_ptr() if norm and residual else None, gain.data_ptr() if norm else None,
-                                        left.data_ptr() if norm and residual else None, 1e-6, 0, s) == 0
-    assert _ratio(lambda i: run(i, True), lambda i: run(i, False), n, limit) < limit
+    def run(i, before):
+        assert lib.pegainfer_gemv_fused(w[i], x, y, M, T, K, *before, 1e-6, 0, s) == 0
+    assert _ratio(lambda i: run(i, normed), lambda i: run(i, plain), n, limit) < limit
+
+
+# 32 columns (tiles of 32) against 33 (of 64): 0.92 with a ring of weights that is requested at once, 1.04 / 1.05 with one of 14 tiles
+@pytest.mark.parametrize("M", [16384, 12292])
+def test_32_columns_take_no_longer_than_33(M):
+    from pegainfer_amd import ffi
+    K, lib, s = 1024, ffi.lib(), torch.cuda.current_stream().cuda_stream
+    W, X = torch.randn(int(4e8 / (2 * M * K)), M, K, device="cuda").bfloat16(), torch.randn(33, K, device="cuda").bfloat16()
+    Y = torch.empty(33, M, device="cuda", dtype=torch.bfloat16)
+    w, x, y = [v.data_ptr() for v in W], X.data_ptr(), Y.data_ptr()
+    assert _ratio(lambda i: lib.gemm_cuda(w[i], x, y, M, 32, K, s), lambda i: lib.gemm_cuda(w[i], x, y, M, 33, K, s), len(w), 0.98) < 0.98
