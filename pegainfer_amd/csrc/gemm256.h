@@ -12,14 +12,16 @@
 //   * a K tile's place in LDS is free once every wave has read its second step (slot 36: barrier); from there the tile after the next is fetched
 //     into it by LDS-DMA (global_load_lds_dwordx4, XOR-swizzled through the SOURCE address), an instruction every eighth slot, as fast as
 //     addresses are taken without holding a wave up (every second or fourth slot: 13 / 5 % slower), its M0 one slot before;
-//   * the next tile has to be there at slot 96 (counted vmcnt: what the tile after it has been asked for stays in flight; barrier): 34 slots at
-//     least lie between a fetch and that;
+//   * the next tile has to be there at slot 96 (counted vmcnt: what the tile after it has been asked for stays in flight; barrier): its last piece is asked for
+//     at slot 29;
 //   * results leave through LDS as whole lines: 8 bytes a lane in runs of 32, as the products leave them, took 8 us a tile, whole rows of 256 bytes 4;
-//   * a workgroup stays on its compute unit and takes every 256th tile: the next one's first two K tiles are asked for before the results are turned, and
-//     its products begin while they are still on their way out.  2 us of fetching and up to 4 of stores a tile of 60 to 75.
-// Measured against the eight waves, same bits, random operands (us): 10 000 tokens: 19 456 x 2560 926 -> 758, 2560 x 9728 487 -> 404, 6144 x 2560
-// 288 -> 242; 5362 tokens: 2560 x 9728 222 -> 197, 2560 x 4096 100 -> 88; 2048 tokens, 24 576 x 4096 330 -> 294.  The SwiGLU form, whose 128 gated
-// units a lane are as long as eight K tiles' products: 10 000 tokens, 9728 x 2560 862 -> 777 (804 of 821 with a workgroup a tile), 1024 tokens 99.5 -> 93.7.
+//   * a workgroup takes one tile.  It has all of its compute unit's LDS and registers: what it does not give up nobody else gets.  Workgroups that stayed
+//     for every 256th tile hid 2 us of fetching and up to 4 of stores a tile, which made a launch alone 1 % faster (plain form; none the SwiGLU form), but one
+//     that found its unit held began only as the others were through: 10 000 tokens, 19 456 x 2560 beside 8 held units 1221 us of 802 (822 of 796 a tile a
+//     workgroup, 951 of 907 with eight waves), and another stream's launch waited 578 us for a unit (49, 61).
+// Measured against the eight waves, same bits, random operands, cold weights (us): 10 000 tokens: 19 456 x 2560 907 -> 796, 2560 x 9728 407 -> 371, 6144 x 2560
+// 268 -> 230; 5362 tokens: 2560 x 9728 217 -> 188, 2560 x 4096 96 -> 84.  The SwiGLU form, whose 128 gated units a lane are as long as eight K tiles'
+// products: 10 000 tokens, 9728 x 2560 800 -> 736, 2048 tokens, 12 288 x 4096 321 -> 290, 1024 tokens, 9728 x 2560 104 -> 99.
 // Per-element K order (K tile by K tile, k-step 0 then 1) is that of the other tiled kernels: same bits.
 #pragma once
 
@@ -43,7 +45,7 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
 
-// PART: a K slice's fp32 partials (the split-K launch), a work item a workgroup; else a workgroup takes every gridDim.x-th tile
+// PART: a K slice's fp32 partials (the split-K launch)
 template <bool SILU, bool PART = false>
 __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
                                                            Half* __restrict__ Y, int M, int T, int K, int m_tiles,
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wr = wave >> 1, wc = wave & 1;
   const int l15 = lane & 15, g = lane >> 4;
-  // the value as one that the loop over tiles does not know: what follows from it is computed where it is used, not kept across the products
+  // the value as one that nothing before knows: what follows from it is computed where it is used, not kept across the products
   auto again = [](int v) {
     asm volatile("" : "+v"(v));
     return v;
@@ -67,8 +69,8 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
   // 10 k tokens (76 x 40 tiles, token tile fastest) fetched 4.2 GB from the memory side per launch for 151 MB of operands - every X
   // panel once per row tile (FETCH_SIZE, profiles/r6c_ctx10000_pmc_fetch.csv)
   int mt, tt;
-  auto place = [&](int item) {
-    int tile = item;
+  {
+    int tile = (int)blockIdx.x;
     if (PART && so.xcd_slices) {
       // K-split launches: one contiguous run of (slice, tile) work items per XCD in SLICE-major order, so an XCD pulls
       // one K slice of X through its L2 instead of all of X (see mfma_gemm128x256_kernel); same work items, same bits
@@ -93,23 +95,19 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
       mt = so.t_major ? tile % m_tiles : tile / t_tiles;
       tt = so.t_major ? tile / m_tiles : tile - mt * t_tiles;
     }
-  };
+  }
 
   // ---- DMA sources: piece p of an operand = its rows p * 32 + wave * 8 + (lane >> 3), LDS slot lane & 7: the lane fetches global slot
   //      (lane & 7) ^ (row & 7) so that readers use lds_slot().  The last tile of a direction begins
   //      256 before the end (the kernel is taken from 256 rows and tokens on): what it shares with the tile before it, both leave with the same bits ----
-  const char *a_at, *b_at;
-  int m0, t0, nk = K / G256_BK;                    // SILU: m0 = the first of 128 activation columns
-  auto point = [&]() {
-    m0 = SILU ? std::min(so.silu_c0 + mt * 128, silu_cols_end(so) - 128) : std::min(mt * G256_BM, M - G256_BM);
-    t0 = std::min(tt * G256_BT, T - G256_BT);
-    // PART: a K slice of nk_slice K tiles (even and at least four, like the last, shorter one: the tiles are walked in pairs); the workgroup's fp32 tile goes to
-    // part[z][T][M] and a slice-sum launch adds the slices in z order (down_proj at 1-2 k tokens: 40-80 tiles of 256 x 256 for 256 CUs)
-    const int kt_begin = PART ? zslice * nk_slice : 0;
-    if (PART) nk = std::min(nk - kt_begin, nk_slice);
-    a_at = reinterpret_cast<const char*>(W + (size_t)m0 * K + (size_t)kt_begin * G256_BK);
-    b_at = reinterpret_cast<const char*>(X + (size_t)t0 * K + (size_t)kt_begin * G256_BK);
-  };
+  // SILU: m0 = the first of 128 activation columns
+  const int m0 = SILU ? std::min(so.silu_c0 + mt * 128, silu_cols_end(so) - 128) : std::min(mt * G256_BM, M - G256_BM);
+  const int t0 = std::min(tt * G256_BT, T - G256_BT);
+  // PART: a K slice of nk_slice K tiles (even and at least four, like the last, shorter one: the tiles are walked in pairs); the workgroup's fp32 tile goes to
+  // part[z][T][M] and a slice-sum launch adds the slices in z order (down_proj at 1-2 k tokens: 40-80 tiles of 256 x 256 for 256 CUs)
+  const int kt_begin = PART ? zslice * nk_slice : 0, nk = PART ? std::min(K / G256_BK - kt_begin, nk_slice) : K / G256_BK;
+  const char* a_at = reinterpret_cast<const char*>(W + (size_t)m0 * K + (size_t)kt_begin * G256_BK);
+  const char* b_at = reinterpret_cast<const char*>(X + (size_t)t0 * K + (size_t)kt_begin * G256_BK);
   uint32_t piece_at[8];
 #pragma unroll
   for (int p = 0; p < 8; ++p) piece_at[p] = (uint32_t)(p * 32 + wave * 8 + (lane >> 3)) * (uint32_t)(K * 2) + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16u;
@@ -148,20 +146,8 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
   typedef std::integral_constant<int, 1> P1;
   // the slots of a K tile (see above); a piece whose slot lies behind the last one is fetched by the next K tile
   constexpr int kFree = 36, kLanded = 96, kEvery = 8, kReadEvery = 2;
-  // K tiles 0 and 1 of the tile that point() was called for (the first iteration fetches the last pieces of K tile 1 again)
-  auto begin = [&]() {
-    auto fetch_now = [&](auto q, auto par, const From& f) {
-      aim(q, par);
-      asm volatile("s_nop 0");
-      fetch(q, f);
-    };
-    const From first = from(0), second = from(128);
-    static_for<16>([&](auto q) { fetch_now(q, P0(), first); });
-    static_for<16>([&](auto q) { fetch_now(q, P1(), second); });
-  };
-
-  // one K tile in the place of parity par.  MORE: there is a tile after the next to fetch; NEXT: there is a next one.  there: it has landed already
-  auto ktile = [&](auto parc, auto morec, auto nextc, int there) {
+  // one K tile in the place of parity par.  MORE: there is a tile after the next to fetch; NEXT: there is a next one
+  auto ktile = [&](auto parc, auto morec, auto nextc) {
     constexpr int par = decltype(parc)::value;
     constexpr bool MORE = decltype(morec)::value, NEXT = decltype(nextc)::value;
     typedef std::integral_constant<int, par ^ 1> Other;
@@ -177,11 +163,7 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
       }
       if constexpr (NEXT && n == kLanded) {      // the next tile is there; of the one after it, what has been asked for may be on its way
         constexpr int asked = MORE ? (kLanded - 2 - kFree) / kEvery + 1 : 0;
-        if constexpr (MORE && par == 0 && !PART)
-          asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lthere%=\n\ts_waitcnt vmcnt(%1)\n.Lthere%=:" ::"s"(__builtin_amdgcn_readfirstlane(there)), "i"(asked)
-                       : "memory", "scc");
-        else
-          asm volatile("s_waitcnt vmcnt(%0)" ::"i"(asked) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(asked) : "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -204,174 +186,161 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
   };
   static_assert(kFree % kEvery != 127 % kEvery, "an aim and its load lie in one iteration");
 
-  int item = (int)blockIdx.x;
-  place(item);
-  point();
-  begin();
+  // K tiles 0 and 1 (the first iteration fetches the last pieces of K tile 1 again)
+  {
+    auto fetch_now = [&](auto q, auto par, const From& f) {
+      aim(q, par);
+      asm volatile("s_nop 0");
+      fetch(q, f);
+    };
+    const From first = from(0), second = from(128);
+    static_for<16>([&](auto q) { fetch_now(q, P0(), first); });
+    static_for<16>([&](auto q) { fetch_now(q, P1(), second); });
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[i][j]));
+    }
   asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-  for (bool later = false;; later = true) {
-    __builtin_amdgcn_s_barrier();                  // K tile 0 is there
-    static_for<16>([&](auto q) { read(q, P0(), P0()); });
+  __builtin_amdgcn_s_barrier();                    // K tile 0 is there
+  static_for<16>([&](auto q) { read(q, P0(), P0()); });
+  asm volatile("s_nop 7" ::: "memory");            // (a product's text tells nobody that a register just written must rest before it)
+  __builtin_amdgcn_sched_barrier(0);
+  int kt = 0;
+  do {
+    ktile(P0(), std::true_type(), std::true_type());
+    ktile(P1(), std::true_type(), std::true_type());
+    kt += 2;
+  } while (kt + 2 < nk);
+  ktile(P0(), std::false_type(), std::true_type());
+  ktile(P1(), std::false_type(), std::false_type());
+  // The last products' way to their registers.  Nothing may read a sum before, and the compiler, which does not see that a product's text takes its time, is free
+  // to copy one right behind its last product: all of them pass through here as accumulator registers
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 8; ++i)
+    asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7]));
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int mw = SILU ? m0 + wr * 64 : m0 + wr * 128, tw = t0 + wc * 128;      // the wave's block
+  // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 8 KB of LDS (chunks
+  //      of 16 bytes, XOR-swizzled by the token), 32 tokens at a time, and stores whole rows of a token.  `wide`: every row that is written begins on
+  //      16 bytes and the segments are whole chunks of eight values; else a chunk leaves in halves of four values, which no boundary cuts: rows of
+  //      outputs, segments and gated columns are multiples of four and begin on 8 bytes (glds_gemm_ok, pegainfer_gemm_split, gemm_silu_impl).  Value
+  //      by value such segments took 1.5 to 2.5 times as long (M 6144 in 4100 + 1020 + 1024, K 2560, 2048 tokens: 91 us, 56 in halves; 8192
+  //      in 4096 + 2052 + 2044, K 256, 4096 tokens: 89, 26) ----
+  const int ln = again(lane), e15 = ln & 15, eg = ln >> 4;
+  char* own = reinterpret_cast<char*>(g256_smem) + kG256LdsBytes + wave * 8192;
+  if constexpr (PART) {                          // 16 tokens of 512 bytes at a time
+    float* pz = part + (size_t)zslice * T * M;    // the workspace's own start, rows of fours: on 16 bytes
+    static_for<8>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        asm volatile("" : "+a"(acc[i][j]));
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(own + e15 * 512 + (((i * 4 + eg) ^ e15) << 4)) = acc[i][j];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int tl = q * 2 + (ln >> 5);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((ln & 31) ^ tl) << 4));
+        *reinterpret_cast<f32x4*>(pz + (size_t)(tw + j * 16 + tl) * M + mw + (ln & 31) * 4) = v;
       }
-    asm volatile("s_nop 7" ::: "memory");          // (a product's text tells nobody that a register just written must rest before it)
-    __builtin_amdgcn_sched_barrier(0);
-    int kt = 0;
-    do {
-      ktile(P0(), std::true_type(), std::true_type(), later && kt == 0);
-      ktile(P1(), std::true_type(), std::true_type(), 0);
-      kt += 2;
-    } while (kt + 2 < nk);
-    ktile(P0(), std::false_type(), std::true_type(), 0);
-    ktile(P1(), std::false_type(), std::false_type(), 0);
-    // the last products' way to their registers, which nothing reads before
-    asm volatile("s_nop 15\n\ts_nop 15"
-                 : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7])
-                 :
-                 : "memory");
-    __builtin_amdgcn_sched_barrier(0);
-
-    // ---- the next tile's first K tiles are asked for before this one's results leave ----
-    const int mw = SILU ? m0 + wr * 64 : m0 + wr * 128, tw = t0 + wc * 128;      // the wave's block
-    item += (int)gridDim.x;
-    const bool more = !PART && item < ntiles;
-    if (more) {
-      __builtin_amdgcn_s_barrier();                // every wave is through with both places
-      place(item);
-      point();
-      begin();
-    }
-
-    // ---- epilogue.  A lane holds rows m = .. + g*4 + e (4 consecutive) of token t = .. + l15; the wave turns its block in its own 8 KB of LDS (chunks
-    //      of 16 bytes, XOR-swizzled by the token), 32 tokens at a time, and stores whole rows of a token.  `wide`: every row that is written begins on
-    //      16 bytes and the segments are whole chunks of eight values; else a chunk leaves in halves of four values, which no boundary cuts: rows of
-    //      outputs, segments and gated columns are multiples of four and begin on 8 bytes (glds_gemm_ok, pegainfer_gemm_split, gemm_silu_impl).  Value
-    //      by value such segments took 1.5 to 2.5 times as long (M 6144 in 4100 + 1020 + 1024, K 2560, 2048 tokens: 91 us, 56 in halves; 8192
-    //      in 4096 + 2052 + 2044, K 256, 4096 tokens: 89, 26) ----
-    const int ln = again(lane), e15 = ln & 15, eg = ln >> 4;
-    char* own = reinterpret_cast<char*>(g256_smem) + kG256LdsBytes + wave * 8192;
-    if constexpr (PART) {                          // 16 tokens of 512 bytes at a time
-      float* pz = part + (size_t)zslice * T * M;    // the workspace's own start, rows of fours: on 16 bytes
-      static_for<8>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        __builtin_amdgcn_wave_barrier();
+    });
+  } else {
+    auto chunk_of = [&](int tl, int c) { return reinterpret_cast<u32x4*>(own + tl * 256 + ((c ^ (tl & 15)) << 4)); };
+    auto turn = [&](auto pc) {                   // tokens 32 p .. of the wave's block, rows of 256 bytes
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(own + e15 * 512 + (((i * 4 + eg) ^ e15) << 4)) = acc[i][j];
-        __builtin_amdgcn_wave_barrier();
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int tl = q * 2 + (ln >> 5);
-          const f32x4 v = *reinterpret_cast<const f32x4*>(own + tl * 512 + (((ln & 31) ^ tl) << 4));
-          *reinterpret_cast<f32x4*>(pz + (size_t)(tw + j * 16 + tl) * M + mw + (ln & 31) * 4) = v;
+        for (int i = 0; i < 8; ++i) {
+          const f32x4& a = acc[i][decltype(pc)::value * 2 + h];
+          *reinterpret_cast<u32x2*>(own + (h * 16 + e15) * 256 + (((i * 2 + (eg >> 1)) ^ e15) << 4) + (eg & 1) * 8) =
+              u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
         }
-      });
-    } else {
-      // what was asked for lands before the first store: loads and stores do not end in the order in which they were issued, and the next tile's
-      // products are not to wait for these stores
-      auto landed = [&]() {
-        if (more) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      };
-      auto chunk_of = [&](int tl, int c) { return reinterpret_cast<u32x4*>(own + tl * 256 + ((c ^ (tl & 15)) << 4)); };
-      auto turn = [&](auto pc) {                   // tokens 32 p .. of the wave's block, rows of 256 bytes
-        __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_wave_barrier();
+    };
+    if constexpr (SILU) {                        // 64 gate values and their 64 up values, bf16 as the GEMM's output is before SwiGLU (fused_proj.cu:57-62)
+      const bool wide = aligned16(Y) && ((so.silu_I | m0 | so.silu_c0 | silu_cols_end(so)) & 7) == 0;
+      auto rows = [&](auto roundc) {
+        auto unit = [&](float sg, float up) { return (decltype(roundc)::value ? bf16_round_f(sg) : sg) * up; };
+        Half* to = Y + (size_t)(tw + (ln >> 3)) * so.silu_I + mw + (ln & 7) * 8;
+        u32x4 o[2][4];                           // a pass's results wait while the next one's are made
+        auto leave = [&](auto p) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const f32x4& a = acc[i][decltype(pc)::value * 2 + h];
-            *reinterpret_cast<u32x2*>(own + (h * 16 + e15) * 256 + (((i * 2 + (eg >> 1)) ^ e15) << 4) + (eg & 1) * 8) =
-                u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
+          for (int q = 0; q < 4; ++q) {
+            Half* at = to + (size_t)(decltype(p)::value * 32 + q * 8) * so.silu_I;
+            const u32x4 v = o[decltype(p)::value & 1][q];
+            if (wide) {
+              *reinterpret_cast<u32x4*>(at) = v;
+            } else {
+              *reinterpret_cast<u32x2*>(at) = u32x2{v[0], v[1]};
+              *reinterpret_cast<u32x2*>(at + 4) = u32x2{v[2], v[3]};
+            }
           }
-        __builtin_amdgcn_wave_barrier();
-      };
-      if constexpr (SILU) {                        // 64 gate values and their 64 up values, bf16 as the GEMM's output is before SwiGLU (fused_proj.cu:57-62)
-        const bool wide = aligned16(Y) && ((so.silu_I | m0 | so.silu_c0 | silu_cols_end(so)) & 7) == 0;
-        auto rows = [&](auto roundc) {
-          auto unit = [&](float sg, float up) { return (decltype(roundc)::value ? bf16_round_f(sg) : sg) * up; };
-          Half* to = Y + (size_t)(tw + (ln >> 3)) * so.silu_I + mw + (ln & 7) * 8;
-          u32x4 o[2][4];                           // a pass's results wait while the next one's are made
-          auto leave = [&](auto p) {
+        };
+        static_for<4>([&](auto p) {
+          turn(p);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              Half* at = to + (size_t)(decltype(p)::value * 32 + q * 8) * so.silu_I;
-              const u32x4 v = o[decltype(p)::value & 1][q];
-              if (wide) {
-                *reinterpret_cast<u32x4*>(at) = v;
-              } else {
-                *reinterpret_cast<u32x2*>(at) = u32x2{v[0], v[1]};
-                *reinterpret_cast<u32x2*>(at + 4) = u32x2{v[2], v[3]};
-              }
-            }
-          };
-          static_for<4>([&](auto p) {
-            turn(p);
+          for (int q = 0; q < 4; ++q) {
+            const int tl = q * 8 + (ln >> 3);
+            const u32x4 ga = *chunk_of(tl, ln & 7), up = *chunk_of(tl, 8 + (ln & 7));
+            u32x4& r = o[decltype(p)::value & 1][q];
+            if (__all(silu_mid_ok(ga))) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int tl = q * 8 + (ln >> 3);
-              const u32x4 ga = *chunk_of(tl, ln & 7), up = *chunk_of(tl, 8 + (ln & 7));
-              u32x4& r = o[decltype(p)::value & 1][q];
-              if (__all(silu_mid_ok(ga))) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  r[e] = pack_bf2(unit(silu_mid_f(bf_lo(ga[e])), bf_lo(up[e])), unit(silu_mid_f(bf_hi(ga[e])), bf_hi(up[e])));
-              } else {                             // rare: value by value, in place
-                Half *at = reinterpret_cast<Half*>(chunk_of(tl, ln & 7)), *ua = reinterpret_cast<Half*>(chunk_of(tl, 8 + (ln & 7)));
+              for (int e = 0; e < 4; ++e)
+                r[e] = pack_bf2(unit(silu_mid_f(bf_lo(ga[e])), bf_lo(up[e])), unit(silu_mid_f(bf_hi(ga[e])), bf_hi(up[e])));
+            } else {                             // rare: value by value, in place
+              Half *at = reinterpret_cast<Half*>(chunk_of(tl, ln & 7)), *ua = reinterpret_cast<Half*>(chunk_of(tl, 8 + (ln & 7)));
 #pragma unroll 1
-                for (int e = 0; e < 8; ++e) at[e] = f2bf(unit(silu_f(bf2f(at[e])), bf2f(ua[e])));
-                r = *chunk_of(tl, ln & 7);
-              }
+              for (int e = 0; e < 8; ++e) at[e] = f2bf(unit(silu_f(bf2f(at[e])), bf2f(ua[e])));
+              r = *chunk_of(tl, ln & 7);
             }
-            if constexpr (decltype(p)::value == 1) landed();
-            if constexpr (decltype(p)::value >= 1) leave(std::integral_constant<int, decltype(p)::value - 1>());
-          });
-          leave(std::integral_constant<int, 3>());
-        };
-        if (so.silu_round) rows(std::true_type());
-        else rows(std::false_type());
+          }
+          if constexpr (decltype(p)::value >= 1) leave(std::integral_constant<int, decltype(p)::value - 1>());
+        });
+        leave(std::integral_constant<int, 3>());
+      };
+      if (so.silu_round) rows(std::true_type());
+      else rows(std::false_type());
+    } else {
+      const bool wide = aligned16(Y) && (M & 7) == 0 &&
+                        (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
+      struct Segment { Half* at; int ld, m; };
+      auto segment = [&](int r) {                // where row r goes
+        if (!so.Y1) return Segment{Y, M, r};
+        const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
+        if (r < so.M0) return Segment{Y, so.M0, r};
+        if (r < b1) return Segment{so.Y1, so.M1, r - so.M0};
+        if (r < b2) return Segment{so.Y2, so.M2, r - b1};
+        return Segment{so.Y3, M - b2, r - b2};
+      };
+      if (wide) {
+        const Segment sg = segment(mw + e15 * 8);
+        u32x4 v[32];
+        static_for<4>([&](auto p) {
+          turn(p);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[decltype(p)::value * 8 + q] = *chunk_of(q * 4 + eg, e15);
+        });
+#pragma unroll
+        for (int q = 0; q < 32; ++q) *reinterpret_cast<u32x4*>(sg.at + (size_t)(tw + q * 4 + eg) * sg.ld + sg.m) = v[q];
       } else {
-        const bool wide = aligned16(Y) && (M & 7) == 0 &&
-                          (!so.Y1 || (aligned16(so.Y1) && aligned16(so.Y2) && aligned16(so.Y3) && ((so.M0 | so.M1 | so.M2) & 7) == 0));
-        struct Segment { Half* at; int ld, m; };
-        auto segment = [&](int r) {                // where row r goes
-          if (!so.Y1) return Segment{Y, M, r};
-          const int b1 = so.M0 + so.M1, b2 = b1 + so.M2;
-          if (r < so.M0) return Segment{Y, so.M0, r};
-          if (r < b1) return Segment{so.Y1, so.M1, r - so.M0};
-          if (r < b2) return Segment{so.Y2, so.M2, r - b1};
-          return Segment{so.Y3, M - b2, r - b2};
-        };
-        if (wide) {
-          const Segment sg = segment(mw + e15 * 8);
-          u32x4 v[32];
-          static_for<4>([&](auto p) {
-            turn(p);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[decltype(p)::value * 8 + q] = *chunk_of(q * 4 + eg, e15);
-          });
-          landed();
-#pragma unroll
-          for (int q = 0; q < 32; ++q) *reinterpret_cast<u32x4*>(sg.at + (size_t)(tw + q * 4 + eg) * sg.ld + sg.m) = v[q];
-        } else {
-          const Segment half = segment(mw + (ln & 31) * 4);
-          landed();
-          static_for<4>([&](auto p) {
-            turn(p);
-            const int tp = tw + decltype(p)::value * 32;
+        const Segment half = segment(mw + (ln & 31) * 4);
+        static_for<4>([&](auto p) {
+          turn(p);
+          const int tp = tw + decltype(p)::value * 32;
 #pragma unroll 4
-            for (int q = 0; q < 16; ++q) {
-              const int tl = q * 2 + (ln >> 5);
-              *reinterpret_cast<u32x2*>(half.at + (size_t)(tp + tl) * half.ld + half.m) = reinterpret_cast<const u32x2*>(chunk_of(tl, (ln & 31) >> 1))[ln & 1];
-            }
-          });
-        }
+          for (int q = 0; q < 16; ++q) {
+            const int tl = q * 2 + (ln >> 5);
+            *reinterpret_cast<u32x2*>(half.at + (size_t)(tp + tl) * half.ld + half.m) = reinterpret_cast<const u32x2*>(chunk_of(tl, (ln & 31) >> 1))[ln & 1];
+          }
+        });
       }
     }
-    if (!more) return;
   }
 }
 
@@ -395,7 +364,6 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
     const int nch = chunk > 0 ? ceil_div(fast_n, chunk) : 0;
     so.chunk = nch > 1 && (long)m_tiles * t_tiles > 256 ? ceil_div(fast_n, nch) : 0;
   }
-  const int blocks = std::min(m_tiles * t_tiles, device_cus());      // one a compute unit (LDS); a multiple of the XCDs where tiles are left over
   if (silu) {
     static const bool once = [] {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<true>),
@@ -403,7 +371,7 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<true><<<blocks, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<true><<<m_tiles * t_tiles, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   } else {
     static const bool once = [] {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false>),
@@ -411,7 +379,7 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<false><<<blocks, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+    mfma_gemm256_kernel<false><<<m_tiles * t_tiles, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
   }
 }
 

@@ -66,3 +66,38 @@ def test_32_columns_take_no_longer_than_33(M):
     Y = torch.empty(33, M, device="cuda", dtype=torch.bfloat16)
     w, x, y = [v.data_ptr() for v in W], X.data_ptr(), Y.data_ptr()
     assert _ratio(lambda i: lib.gemm_cuda(w[i], x, y, M, 32, K, s), lambda i: lib.gemm_cuda(w[i], x, y, M, 33, K, s), len(w), 0.98) < 0.98
+
+
+def test_ten_rounds_of_tiles_beside_a_held_unit():
+    """One wave of another stream keeps the 256 x 256 tiles off its compute unit: 1.1 of the time alone where a workgroup takes a tile, 1.4 and more where
+    workgroups stay for the whole launch and the one that found no unit begins as the others are through."""
+    import time
+    from pegainfer_amd import ffi, ops
+    M, T, K, lib = 19456, 8192, 512, ffi.lib()
+    W, X = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(T, K, device="cuda").bfloat16()
+    Y = torch.empty(T, M, device="cuda", dtype=torch.bfloat16)
+    here, there = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def timed(stream, f):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in "ab")
+        with torch.cuda.stream(stream):
+            a.record()
+            f()
+            b.record()
+        b.synchronize()
+        return a.elapsed_time(b)
+    ops.gemm_into(W, X, Y)
+    torch.cuda.synchronize()
+    gemm = lambda: lib.gemm_cuda(W.data_ptr(), X.data_ptr(), Y.data_ptr(), M, T, K, here.cuda_stream)  # noqa: E731
+    torch.cuda._sleep(1000)
+    cycles = 1000000 / timed(there, lambda: torch.cuda._sleep(1000000))      # a millisecond
+    alone, beside = sorted(timed(here, gemm) for _ in range(9))[4], []
+    while len(beside) < 5:
+        with torch.cuda.stream(there):
+            torch.cuda._sleep(int(cycles * (4 * alone + 3)))
+        time.sleep(0.001)
+        took = timed(here, gemm)
+        assert not there.query()                       # the unit was held all the time
+        beside.append(took)
+        there.synchronize()
+    assert sorted(beside)[2] / alone < 1.25
