@@ -45,8 +45,9 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
 
-// PART: a K slice's fp32 partials (the split-K launch)
-template <bool SILU, bool PART = false>
+// PART: a K slice's fp32 partials (the split-K launch).  NT: a single tile of tokens, so that this workgroup is the only reader of its W rows (SplitOut::w_nt); an
+// instance of its own, as a fetch has a slot.  256 tokens (us): 32 768 x 2560 63.1 -> 58.2, 65 536 x 4096 155 -> 126, SwiGLU of 16 384 x 2560 68.8 -> 62.4.
+template <bool SILU, bool PART = false, bool NT = false>
 __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __restrict__ W, const Half* __restrict__ X,
                                                            Half* __restrict__ Y, int M, int T, int K, int m_tiles,
                                                            int t_tiles, SplitOut so, float* __restrict__ part = nullptr,
@@ -126,7 +127,8 @@ __global__ __launch_bounds__(256, 1) void mfma_gemm256_kernel(const Half* __rest
     // SILU: a tile is 128 gate rows and their 128 up rows, a wave's m-tiles 0-3 gate rows, 4-7 the same up rows
     const char* base = q >= 8 ? f.b : SILU && (q & 2) ? f.up : f.a;
     const uint32_t v = piece_at[q >= 8 || !SILU ? q & 7 : (q >> 2) * 2 + (q & 1)];
-    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(v), "s"(base) : "memory");
+    if constexpr (NT && q < 8) asm volatile("global_load_lds_dwordx4 %0, %1 nt" ::"v"(v), "s"(base) : "memory");
+    else asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(v), "s"(base) : "memory");
   };
 
   f32x4 acc[8][8];
@@ -364,23 +366,21 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
     const int nch = chunk > 0 ? ceil_div(fast_n, chunk) : 0;
     so.chunk = nch > 1 && (long)m_tiles * t_tiles > 256 ? ceil_div(fast_n, nch) : 0;
   }
-  if (silu) {
+  const bool nt = t_tiles == 1 && weights_nt_on();
+  auto launch = [&](auto silu_form, auto nt_form) {
+    constexpr bool SILU = decltype(silu_form)::value, NT = decltype(nt_form)::value;
     static const bool once = [] {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<true>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<SILU, false, NT>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes + kG256TurnBytes);
       return true;
     }();
     (void)once;
-    mfma_gemm256_kernel<true><<<m_tiles * t_tiles, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
-  } else {
-    static const bool once = [] {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm256_kernel<false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kG256LdsBytes + kG256TurnBytes);
-      return true;
-    }();
-    (void)once;
-    mfma_gemm256_kernel<false><<<m_tiles * t_tiles, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
-  }
+    mfma_gemm256_kernel<SILU, false, NT><<<m_tiles * t_tiles, 256, kG256LdsBytes + kG256TurnBytes, s>>>(W, X, Y, M, T, K, m_tiles, t_tiles, so);
+  };
+  if (silu && nt) launch(std::true_type(), std::true_type());
+  else if (silu) launch(std::true_type(), std::false_type());
+  else if (nt) launch(std::false_type(), std::true_type());
+  else launch(std::false_type(), std::false_type());
 }
 
 // split-K launch of the plain form: fp32 partials into `part` ([ksplit][T][M]); the caller sums the slices

@@ -32,7 +32,7 @@ def test_sums_stay_in_their_registers_between_products(built_libs, tmp_path):
     path.write_bytes(code[0])
     text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], stdout=subprocess.PIPE, check=True, text=True).stdout
     kernels = [k for k in text.split("\n\n") if name.decode() in k.lstrip().split("\n")[0]]
-    assert len(kernels) == 3
+    assert len(kernels) == 5
     for k in kernels:
         lines = [line.split("//")[0].strip() for line in k.split("\n")]
         product = [i for i, line in enumerate(lines) if line.startswith("v_mfma_f32_16x16x32_bf16")]

@@ -101,3 +101,13 @@ def test_ten_rounds_of_tiles_beside_a_held_unit():
         beside.append(took)
         there.synchronize()
     assert sorted(beside)[2] / alone < 1.25
+
+
+# one tile of tokens against two: 0.65 where the weights, which have one reader, are loaded past the caches, 0.78 where they push each other out
+def test_weights_of_a_single_tile_of_tokens_pass_the_caches():
+    from pegainfer_amd import ffi
+    M, K, lib, s = 65536, 4096, ffi.lib(), torch.cuda.current_stream().cuda_stream
+    W, X = torch.randn(2, M, K, device="cuda").bfloat16(), torch.randn(257, K, device="cuda").bfloat16()
+    Y = torch.empty(257, M, device="cuda", dtype=torch.bfloat16)
+    w, x, y = [v.data_ptr() for v in W], X.data_ptr(), Y.data_ptr()
+    assert _ratio(lambda i: lib.gemm_cuda(w[i % 2], x, y, M, 256, K, s), lambda i: lib.gemm_cuda(w[i % 2], x, y, M, 257, K, s), 6, 0.71) < 0.71
