@@ -38,9 +38,11 @@ __device__ __forceinline__ float bf16_round_f(float f) { return bf2f(f2bf(f)); }
 // SiLU exactly as the reference writes it: g / (1 + expf(-g))  (csrc/fused_proj.cu:57-62)
 __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + expf(-g)); }
 
-// The same bits for a bf16 value of 0 < |g| <= 80 (compared over all of them): an exponential without the ends of its range, a quotient whose
+// The same fp32 bits for a bf16 value of 0 < |g| <= 80 (all 34 112 compared): an exponential without the ends of its range, a quotient whose
 // operands need no scaling (one residual step behind the hardware's reciprocal).  17 instructions, none of which keeps a second value's from
-// running beside them; silu_f takes 25 that share the one condition register.
+// running beside them; silu_f takes 25 that share the one condition register.  To have silu_f's bits the exponential is taken in the steps, and with
+// log2 e in the two parts, that hipcc makes of expf for gfx950 (assembly of silu_f): n = round(g log2 e), 2 to the fraction and its rounding rest, scaled by
+// n.  A compiler that expands expf otherwise would part the two; every finite gate of the fused unit is compared with the launches it stands for.
 __device__ __forceinline__ float silu_mid_f(float g) {
 #pragma clang fp contract(off)
   const float minus_log2e = __builtin_bit_cast(float, 0xBFB8AA3Bu), rest = __builtin_bit_cast(float, 0xB2A5705Fu);
