@@ -3,7 +3,8 @@
 //   Y[T, M] = X[T, K] . W[M, K]^T,  a workgroup owns 256 W rows x 256 token rows: four waves, one on each SIMD, wave (wr, wc) a
 //   128 x 128 block of it as 8 x 8 MFMA tiles (256 accumulator registers).
 //
-// Bound by the matrix cores, and by the power that they draw: with random operands the chip lowers its clock to 1.5 GHz, with zeros it stays at 2.2.
+// Bound by the matrix cores, which are busy 0.65 - 0.68 of all cycles of a launch (10 000 tokens, a last round that is not full among them), and by the power that
+// they draw: the plain form takes the same cycles with random operands and with zeros, at 1.85 GHz and at 2.3 (profiles/cases_pmc_sq.csv: gemm-random, gemm-zeros).
 // With eight waves of 128 x 64 (two a SIMD, one computing while the other reads, four phases a K tile) the bound was LDS: 28 ds_read_b128 a wave and K
 // tile, 224 KB, and 64 KB that the DMA writes are 2250 of its cycles for 2048 of the matrix cores.  Waves of 128 x 128 read 128 KB, so that
 //   * a wave has the matrix core of its SIMD to itself and everything else happens between two of its products (16 cycles each), a slot a product:
@@ -384,7 +385,7 @@ inline void gemm256_launch(const Half* W, const Half* X, Half* Y, int M, int T, 
 }
 
 // split-K launch of the plain form: fp32 partials into `part` ([ksplit][T][M]); the caller sums the slices
-inline bool splitk_xcd_on() {   // PEGAINFER_SPLITK_XCD=0: the slices of a tile on one XCD, as until round 6 (A/B)
+inline bool splitk_xcd_on() {   // PEGAINFER_SPLITK_XCD=0: the slices of a tile on one XCD (A/B)
   static const bool v = [] { const char* e = getenv("PEGAINFER_SPLITK_XCD"); return !(e && e[0] == '0'); }();
   return v;
 }
@@ -419,8 +420,8 @@ inline void gemm256_splitk_launch(const Half* W, const Half* X, int M, int T, in
 //                                         order (= ascending K), adds them to its accumulators, clears their flags, and runs
 //                                         the epilogue.  Those partials were published a whole range ago.
 // So the sum over K is taken in a FIXED order that depends on (M, T, K, G) only: deterministic, rerun- and graph-stable, but
-// not the K order of the data-parallel kernels - the cross-route bit identity of rounds 1-5 is given up for prefill GEMMs at
-// these sizes (VERDICT r5 item 2); the oracle comparison under the derived bar referees.  No deadlock: a publisher never waits,
+// not the K order of the data-parallel kernels - the bit identity across routes is given up for prefill GEMMs at
+// these sizes; the oracle comparison under the derived bar referees.  No deadlock: a publisher never waits,
 // an owner waits only for publishers, and all G <= CU-count workgroups are co-resident (one per CU by LDS).  Positions follow
 // the XCD-aware order of the other kernels (block b runs on XCD b % 8): neighbours in the unit order share an XCD's L2 except
 // at seven seams, so most partials are re-read from the L2 they were written through.
@@ -750,11 +751,11 @@ constexpr int G128_BM = 128;
 constexpr int kG128LdsBytes = 9 * kG256HalfBytes;
 enum { kG128A = 0, kG128Blo = 1, kG128Bhi = 2 };
 
-// NF = 4 (round 4): four more waves that do nothing but issue the DMAs (12 per K tile each), in the barrier rhythm of a
+// NF = 4: four more waves that do nothing but issue the DMAs (12 per K tile each), in the barrier rhythm of a
 // wave-row-0 wave; the eight compute waves issue none.  A DMA instruction costs its wave ~133 cycles of issue slot
 // (tools/probes/ingest_probe) - six per wave and K tile were 800 cycles next to 32 MFMAs = 512.  159 VGPRs: three waves
-// per SIMD fit.  NF = 0: the round-3 form (every wave stages its share), kept for the A/B (PEGAINFER_GEMM128X256_FEED=0).
-// MT (round 6) = 16-row MFMA tiles per wave row: 4 = the 128-row tile; 3 = a 96-row tile (plain NF = 4 form only) for
+// per SIMD fit.  NF = 0: the form in which every wave stages its share, kept for the A/B (PEGAINFER_GEMM128X256_FEED=0).
+// MT = 16-row MFMA tiles per wave row: 4 = the 128-row tile; 3 = a 96-row tile (plain NF = 4 form only) for
 // matrices whose 128-row tiling leaves CUs idle - the stacked qkv at 768 / 1024 tokens: 144 / 192 tiles of 128 rows, 192 / 256
 // of 96.  Same per-element K order: same bits.
 template <bool SILU, int NF, int MT = 4>
@@ -766,7 +767,7 @@ __global__ __launch_bounds__(512 + NF * 64) void mfma_gemm128x256_kernel(const H
   const int ntiles = m_tiles * t_tiles;
   int tile = blockIdx.x, zslice = (int)blockIdx.y;
   if (part && so.xcd_slices) {
-    // (round 6) K-split launches: the hardware deals workgroups to XCDs by their linear id; give every XCD one contiguous run of
+    // K-split launches: the hardware deals workgroups to XCDs by their linear id; give every XCD one contiguous run of
     // (slice, tile) work items in SLICE-major order, so an XCD works on (mostly) one K slice of a few row tiles.  With the slices
     // of a tile on one XCD (the 2-D grid's natural order: gridDim.x is a multiple of 8) every XCD pulled the WHOLE of X through
     // its L2 - down_proj at 1024 tokens fetched 209 MB from the memory side for 70 MB of operands (FETCH_SIZE, profiles/
@@ -881,7 +882,7 @@ __global__ __launch_bounds__(512 + NF * 64) void mfma_gemm128x256_kernel(const H
 
   constexpr int kTileDmas = PPA + 2 * PPW;  // DMAs per issuing wave and K tile: the counted wait leaves one tile in flight
   if (feeder) {
-    // the whole staging side, in the barrier rhythm of a wave-row-0 wave (the EARLIEST any wave of the round-3 form touched
+    // the whole staging side, in the barrier rhythm of a wave-row-0 wave (the EARLIEST any wave of the NF = 0 form touched
     // a ring slot, so the hazards are the ones argued above): A + B_lo of tile kt + 2 in phase 1, B_hi in phase 2
     stage(kG128A, 0, 0); stage(kG128Blo, 0, 0); stage(kG128Bhi, 0, 0);
     stage(kG128A, 1, 1); stage(kG128Blo, 1, 1); stage(kG128Bhi, 1, 1);

@@ -19,7 +19,7 @@
 // acc_even[i = 2 r] + acc_odd[i = 2 r + 1] - both in the same lane of the D layout, so no cross-lane traffic.
 // Half of the MFMA work is discarded on purpose: the op is priced against the HBM roofline, not the MFMA one.
 //
-// Row blocks are at most 16 rows high, but not necessarily 16 (round 4): a launch whose 16-row blocks would not deal
+// Row blocks are at most 16 rows high, but not necessarily 16: a launch whose 16-row blocks would not deal
 // evenly onto the 256 CUs takes the block height that does (2560 rows: 160 blocks of 16 -> 256 blocks of 10; a streaming
 // CU ingests ~24 GB/s, so 160 busy CUs cap the launch at 3.8 TB/s).  Rows past a block's height are clamped duplicates
 // of its last row in the loads (same cache lines, no extra HBM traffic) and never stored; a row's K order does not
@@ -435,8 +435,8 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
     }
   };
   // ---- prologue + one-time staging of x.  A wave's loads retire in order: x-side loads issued behind the first
-  //      weight chunks cannot be consumed before those have landed from cold HBM (the finding of the GEMV phase
-  //      trace), so wherever it fits the x side goes FIRST:
+  //      weight chunks cannot be consumed before those have landed from cold HBM (seen in the
+  //      GEMV's phase trace), so wherever it fits the x side goes FIRST:
   //        plain x (o_proj, down_proj): rows -> swizzled LDS by LDS-DMA (lane l of piece q fetches chunk
   //          (64 q + l) ^ (t & 15), which is what the swizzled slot 64 q + l holds), weights behind, one counted wait;
   //        add + RMSNorm (qkv, gate_up; K <= 4096, T <= 16): wave w's token rows w, w + 8 (+ residual, + norm weight)
@@ -616,8 +616,8 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_resident_kernel(const G
   zero();
 
   // Combine the 8 waves (fixed order), store, reset.  Four forms, same arithmetic per element:
-  //  * two barriers around a reduction by the first NB waves (rounds 1-4);
-  //  * one barrier (round 5): the partials of row block n go to buffer n & 1 and wave n & 7 ALONE adds and stores them
+  //  * two barriers around a reduction by the first NB waves;
+  //  * one barrier: the partials of row block n go to buffer n & 1 and wave n & 7 ALONE adds and stores them
   //    while the other seven walk on into block n + 1.  Buffer n & 1 is written again for block n + 2, i.e. after
   //    barrier n + 1, which the reducing wave reaches only after its reduction of block n.
   //  * no barrier (ticket form): a ring of buffers, block n -> buffer n % ring, its u-th use (u = n / ring).  A wave waits
@@ -743,7 +743,7 @@ inline int skinny_pick_rpb(int rows) {
 }
 
 // How the resident kernel combines its 8 waves per row block (bit-identical forms, profiles/r5_skinny_flush_ab.txt, T = 4 / 8 /
-// 16, cold weights): two barriers (rounds 1-4) -> gate_up 21.5-21.9 us, lm_head 131-143; one barrier -> 21.0-21.1, 129-142;
+// 16, cold weights): two barriers -> gate_up 21.5-21.9 us, lm_head 131-143; one barrier -> 21.0-21.1, 129-142;
 // tickets -> 20.2-20.7, 121-133, but qkv / o_proj (two / one row block per workgroup: nothing to overlap) +0.1 us.  A probe
 // without barriers and stores (FLUSH=2) measured 18.2 us: what is left is the reducing wave's own wait and the stores.
 // A ticket form in which the LAST ARRIVER adds (nobody waits; the slowest wave gets the extra work) measured worse than the
@@ -757,7 +757,7 @@ inline int skinny_pick_rpb(int rows) {
 extern int g_skinny_flush_override;   // linear.hip: pegainfer_debug_skinny_flush (tests compare the forms in one process); -1 = none
 // The timing probe (bit 1: partials written, nothing reduced or stored) exists only WITHOUT the ticket bit: with tickets its
 // early return would skip the arrival / done counters and every later use of a ring buffer would spin for ever on them - a GPU
-// hang, not garbage (ADVICE r5).  Modes 6 / 7 are therefore folded to 2; the probe is announced on stderr once.
+// hang, not garbage.  Modes 6 / 7 are therefore folded to 2; the probe is announced on stderr once.
 inline int skinny_flush_sanitise(int mode) {
   mode &= 7;
   if ((mode & 2) && (mode & 4)) mode = 2;

@@ -1,4 +1,4 @@
-// Weight-streaming GEMM for 17..128 token columns (round 4): Y[T, M] = X[T, K] . W[M, K]^T with the row tiles sized to the
+// Weight-streaming GEMM for 17..128 token columns: Y[T, M] = X[T, K] . W[M, K]^T with the row tiles sized to the
 // CU COUNT instead of to a power of two.
 //
 // At these widths the op is bound by how fast the chip INGESTS the weight matrix, and a streaming CU ingests ~24 GB/s: the
@@ -11,7 +11,7 @@
 // 256 / slices row tiles, so tiles x slices fill the chip.
 //
 // Structure: LDS-DMA rings of K tiles of 64 as in mfma_gemm_glds_kernel (source-side swizzle, counted vmcnt), but
-//  * four COMPUTE waves (two for 32 tokens) side by side along the token axis (TT / 4 tokens each, all RT row blocks): any RT works;
+//  * four COMPUTE waves (two for 32 tokens) side by side along the token axis (an equal share of the tokens each, all RT row blocks): any RT works;
 //  * separate FEEDER waves that only issue the DMAs, the W ring and the X ring each with its own waves and depth: a wave
 //    gets one 1 KB DMA instruction through its issue slot per ~93-133 cycles (18-26 GB/s per wave, however many it keeps in
 //    flight - tools/probes/ingest_probe) and issues nothing else meanwhile, and its loads retire in order (the L2-resident
@@ -28,7 +28,7 @@
 
 namespace pk {
 
-// Waves 0..3 compute only; then NLW waves that only feed the W ring and NLX that only feed the X ring.  (The first form of
+// The first four waves (two for tiles of 32 tokens) compute only; then NLW waves that only feed the W ring and NLX that only feed the X ring.  (The first form of
 // this kernel had four waves doing both - gate_up 28.9 us at 32 / 64 columns where this one takes 21.8 / 24.1.)  tools/probes/ingest_probe: a wave gets ~26 GB/s out of its
 // DMA issue slot (one 1 KB instruction per ~93 cycles) however many it keeps in flight, and while it sits there it issues
 // no MFMA; a CU takes ~125 GB/s when every SIMD has a wave issuing.  With loader waves the K step is bound by what the

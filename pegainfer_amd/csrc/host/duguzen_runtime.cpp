@@ -820,7 +820,7 @@ struct Model {
     return 0;
     };
     // a step of single tokens only (decoding) is launch-bound: its launches are captured once per shape as a hipGraph and replayed; steps with
-    // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step at the time (45 now): 9.3 -> 9.05 ms for their prompts and 16 steps.
+    // prompt portions run eagerly.  4 requests of ~900 tokens, 53 launches a step at the time (44 now): 9.3 -> 9.05 ms for their prompts and 16 steps.
     if (captured) {
       const GraphKey key{n, W, out_tokens != nullptr, plain_kernels, every, max_kv};
       hipGraphExec_t exec = graphs.find(key);

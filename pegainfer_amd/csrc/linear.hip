@@ -180,7 +180,7 @@ inline bool weights_nt_on() {
 
 }  // namespace pk
 #include "gemm256.h"   // 256 x 256 tiles, a wave a SIMD (long prompts); uses SplitOut / lds_slot
-#include "gemm_stream.h"   // CU-count-sized row tiles for 17..64 token columns (round 4); uses SplitOut / lds_slot / BK
+#include "gemm_stream.h"   // CU-count-sized row tiles for 17..64 token columns; uses SplitOut / lds_slot / BK
 namespace pk {
 
 // SPLITK: blockIdx.y = K slice z of `ksplit` (each nk_slice K tiles); the workgroup writes its fp32 partial tile to
@@ -418,7 +418,7 @@ static void splitk_reduce(const float* part, Half* Y, int M, int T, int ksplit, 
   }
 }
 
-// (round 6) un-split shapes of pegainfer_gemm_add_then_rms_norm: out = bf16(a + y), normed = rms_norm(out) * w in ONE pass over
+// un-split shapes of pegainfer_gemm_add_then_rms_norm: out = bf16(a + y), normed = rms_norm(out) * w in ONE pass over
 // the rows instead of add_cuda + rms_norm_batched_cuda (10 000 tokens: 25 + 22 us and 256 MB -> one launch, 205 MB).  One wave per
 // row, the canonical order of norm_core.h over the ROUNDED sum: the same bits as the two calls.  out may alias a.
 template <int VPL>   // 0: two passes over the row (any d); 5 / 8: the row in registers (d <= 2560 / 4096), one memory pass
@@ -460,13 +460,13 @@ __global__ __launch_bounds__(512) void splitk_reduce_add_norm_kernel(const float
                                                                      int d, int T, int ksplit, float eps, bool round_sum) {
   extern __shared__ __attribute__((aligned(16))) unsigned char rn_smem[];
   u32x4* rrow = reinterpret_cast<u32x4*>(rn_smem);              // [d / 8] bf16x8: the slice sum r
-  u32x4* hrow = reinterpret_cast<u32x4*>(rn_smem + (size_t)d * 2);   // [d / 8] bf16x8: the residual row (round 6)
+  u32x4* hrow = reinterpret_cast<u32x4*>(rn_smem + (size_t)d * 2);   // [d / 8] bf16x8: the residual row
   float* sm_inv = reinterpret_cast<float*>(rn_smem + (size_t)d * 4);
   const int t = blockIdx.x, nvec = d >> 3;
   const Half* hin = hidden_in + (size_t)t * d;
   Half* hr = hidden + (size_t)t * d;
   Half* orow = out + (size_t)t * d;
-  // (round 6) ONE memory round trip per thread instead of three dependent ones: the residual row and the norm weight leave
+  // ONE memory round trip per thread instead of three dependent ones: the residual row and the norm weight leave
   // with the partials; wave 0's canonical sum of squares reads both rows from LDS (same values, same order: same bits) and the
   // scale pass works from registers.  Rows of more than 512 vectors (d > 4096) keep the reloading loop for their tail.
   auto slice_sum = [&](int i) {
@@ -596,15 +596,15 @@ static bool gemm128x256_on() {
   static const bool v = [] { const char* e = getenv("PEGAINFER_GEMM128X256"); return !(e && e[0] == '0'); }();
   return v;
 }
-// (round 6) Plain prefill GEMMs of >= 512 tokens WITHOUT a K-split plan whose 128 x 256 tiling is ONE partly filled round: 1283 = the
+// Plain prefill GEMMs of >= 512 tokens WITHOUT a K-split plan whose 128 x 256 tiling is ONE partly filled round: 1283 = the
 // same round on 96 x 256 tiles (feeder kernel, gemm256.h) when those fill more of the chip, 0 = no.  The stacked qkv at 768 / 1024
-// tokens is 144 / 192 tiles of 128 rows, 192 / 256 of 96: 35.9 -> 31.5 / 37.8 -> 33.9 us, same bits; TTFT(768 / 1024) 7.90 -> 7.77 /
-// 9.85 -> 9.75 ms same-box (profiles/r6_gemm96_ab.txt, r6_small_tiles_ttft_ab2.txt).  PEGAINFER_GEMM_SMALL_TILES=0 switches it off.
+// tokens is 144 / 192 tiles of 128 rows, 192 / 256 of 96: 41.9 -> 37.9 / 41.4 -> 38.6 us cold, same bits (256 x 256 tiles: 53).  PEGAINFER_GEMM_SMALL_TILES=0
+// switches it off.
 // Two wider forms of the rule were measured and NOT kept - both look 10-30 % faster per GEMM with L2-hot weights
 // (tools/bench_prefill_gemm.py at 1 weight copy, profiles/r6_gemm_force_sweep.txt) and are slower in the model, where weights come
 // from HBM: (a) over the K-split plans of o_proj / down_proj at 1536 .. 3072 tokens (whose slice sum also carries the residual add +
-// RMSNorm): TTFT(1536 / 2048) +1 / +3 % (r6_small_tiles_ttft_ab.txt); (b) several rounds of small tiles instead of 1.1-1.5 rounds
-// of 256 x 256 (qkv at 3072 / 4096 tokens): TTFT +2.7 / +1.7 % (r6_small_tiles_ttft_ab2.txt).
+// RMSNorm): TTFT(1536 / 2048) +1 / +3 % (profiles/r6_small_tiles_ttft_ab.txt); (b) several rounds of small tiles instead of 1.1-1.5 rounds
+// of 256 x 256 (qkv at 3072 / 4096 tokens): 112 us of 97, 151 of 117.
 static int small_tile_unsplit(int M, int T, int K) {
   static const bool on = [] { const char* e = getenv("PEGAINFER_GEMM_SMALL_TILES"); return !(e && e[0] == '0'); }();
   if (!on || !gemm128x256_on() || !gemm128x256_feed_on() || !gemm128x256_ok(M, T, K) || T < 512) return 0;
@@ -642,9 +642,11 @@ static SplitKPlan splitk_plan(int M, int T, int K, bool assume_ws = false) {
   if (T > 64) {
     if (short_k_whole(M, T, K)) return {0, 0, 0};
     // long-K matrices at ~1.3-3 k tokens (down_proj: 50-128 tiles of 256 x 256): their kernel over 2-5 K
-    // slices, one workgroup per CU (tt == 256 marks this plan; PEGAINFER_SPLITK256=0 switches it off).  Same-box A/B of
-    // TTFT: 2048 tokens 23.05 -> 21.4 ms; 1024 tokens (40 tiles, 6 slices: 63 MB of partials each way) 12.60 vs 12.56,
-    // 512 tokens (8 slices) 9.17 vs 9.33 - so only above 40 tiles.
+    // slices, one workgroup per CU (tt == 256 marks this plan; PEGAINFER_SPLITK256=0 switches it off).  With sum, addition and norm, the smaller tilings /
+    // this plan (us, cold weights): 2560 x 9728 and 1300 tokens (60 tiles) 80 / 76, 2048 118 / 98, 3000 141 / 131; 4096 x 12 288 and 1024 (64) 101 / 95; 4096 x
+    // 4096 and 2048 84 / 77; 2560 x 4096 and 2048 58.2 / 57.3.  At 40 tiles (2560 x 9728 and 1024, 6 slices: 63 MB of partials each way) 64.3 / 62.1, 2560 x 4096 and 1024
+    // 38.2 / 37.7, at 20 (512 tokens, 8 slices) 44 / 47 - so only above 40 tiles.  (A slice is two pairs of K tiles at least: where two K tiles would
+    // be left over, the slices are a pair longer, which is another order of the sums than that of slices of the plain length.)
     static const bool s256 = [] { const char* e = getenv("PEGAINFER_SPLITK256"); return !(e && e[0] == '0'); }();
     static const int s256_mink = [] { const char* e = getenv("PEGAINFER_SPLITK256_MINK"); return e && *e ? atoi(e) : 4096; }();   // o_proj (K 4096) included: TTFT(2048) 21.72 -> 21.29 ms
     if (s256 && K >= s256_mink && gemm256_ok(M, T, K)) {
@@ -740,8 +742,8 @@ static void glds_splitk_launch(const Half* W, const Half* X, Half* Y, int M, int
 // The rows behind the full rounds of 256 x 256 tiles of a plain GEMM, when they would fill a small part of a further round: 64 = 128-row x 64-token
 // tiles, 96 = 96 x 256 tiles, 0 = they stay a round of their own.  The kernels keep the same per-element K order: the cut changes no bit.
 // A round of a few dozen tiles costs as much as a full one; measured with cold weights, whole / 64 / 96 (us): 17 408 x 2048 and 900
-// tokens (272 tiles) 100 / 79 / 84, 18 432 x 2560 and 1024 (288) 132 / 103 / 107, 6144 x 2560 and 3072 (288) 122 / 104 / 109, 8192 x 2048 and
-// 2100 (288) 100 / 83 / 84; 19 472 x 2048 and 1024 (308) 111 / 103 / 98, 8192 x 2048 and 2404 (320) 102 / 101 / 89.  The small tiles win while
+// tokens (272 tiles) 91 / 80 / 84, 18 432 x 2560 and 1024 (288) 115 / 93 / 98, 6144 x 2560 and 3072 (288) 105 / 97 / 101, 8192 x 2048 and
+// 2100 (288) 86 / 77 / 78; 19 472 x 2048 and 1024 (308) 91 / 83 / 80, 8192 x 2048 and 2404 (320) 91 / 94 / 80.  The small tiles win while
 // a quarter more than one workgroup per compute unit takes them, the 96-row ones (one workgroup per compute unit) while one round does.
 static int plain_tail_kernel(int M, int T, int K, int m_head) {
   const int rows = M - m_head * G256_BM;
@@ -770,13 +772,14 @@ static TiledRoute tiled_route(int M, int T, int K, const SplitOut& so, bool assu
   // long prompts: 256 x 256 tiles once they give every CU work (PEGAINFER_GEMM256 = 0 never,
   // 1 whenever the shape allows, N = from N tiles on; A/B probe knob)
   // from 128 tiles on (half the CUs): one partly filled round of 256 x 256 tiles still beats the smaller tilings -
-  // gate_up at 512 tokens (152 tiles) 100 -> 70 us, qkv at 1536 tokens (144 tiles) 80 -> 64 us, same bits
-  // (profiles/r3_gemm256_threshold_ab.txt); at 96 tiles (qkv at 1024 tokens) the 128 x 256 kernel wins (43 vs ~71 us)
+  // gate_up at 512 tokens (152 tiles) 92 -> 61 us, at 768 (228) 96 -> 67, qkv at 1536 tokens (144 tiles) 80 -> 54 us, same bits
+  // (at 300 tokens, where the second tile of tokens holds 44, the 128-row kernel takes 54 us to 61); at 96 and 120 tiles (qkv at 1024 and 1280 tokens) the
+  // 96 x 256 and 128 x 256 kernels win (38 and 43 us to 53)
   static const int g256_min = [] { const char* e = getenv("PEGAINFER_GEMM256"); return e && *e ? atoi(e) : 128; }();
   if (g256_min > 0 && gemm256_ok(M, T, K)) {
     const int mt256 = so.silu_I > 0 ? ceil_div(so.silu_I, 128) : ceil_div(M, G256_BM), tt256 = ceil_div(T, G256_BT);
     const long tiles256 = (long)mt256 * tt256;
-    // (round 6) stream-K, kind 258, OFF unless PEGAINFER_STREAMK=1: a PERSISTENT one-workgroup-per-CU launch over (row tile, K-tile
+    // stream-K, kind 258, OFF unless PEGAINFER_STREAMK=1: a PERSISTENT one-workgroup-per-CU launch over (row tile, K-tile
     // pair) units for shapes whose round of 256 x 256 tiles would leave >= 8 % of the CU-rounds idle (gate_up at 512 / 1024 /
     // 2048 tokens: 152 / 304 / 608 tiles on 256 CUs).  Built, correct, deterministic - and measured slower (gemm256.h).
     static const int sk_min = [] { const char* e = getenv("PEGAINFER_STREAMK_MIN_TILES"); return e && *e ? atoi(e) : 128; }();
@@ -786,7 +789,7 @@ static TiledRoute tiled_route(int M, int T, int K, const SplitOut& so, bool assu
       return {258, 0};
     if (tiles256 >= g256_min) {
       // A thin last round: 304 tiles (gate_up at 1024 tokens) are one full round of the 256 CUs plus 48 tiles that
-      // cost a second full tile time (127 us for 102 GFLOP).  The SwiGLU form can hand the activation columns of
+      // cost a second full tile time (124 us for 102 GFLOP, 111 handed over).  The SwiGLU form can hand the activation columns of
       // that remainder to the 128-row kernel (192 quarter-size tiles: one short round) - both kernels keep the same
       // per-element K order, so the result does not depend on the cut.  PEGAINFER_GEMM256_TAIL=0 switches it off.
       static const bool tail_on = [] { const char* e = getenv("PEGAINFER_GEMM256_TAIL"); return !(e && *e == '0'); }();
@@ -799,7 +802,7 @@ static TiledRoute tiled_route(int M, int T, int K, const SplitOut& so, bool assu
       return {256, 0};
     }
   }
-  // 65..128 tokens on a gate_up-sized matrix (round 4): the weight-streaming kernel with 128-token tiles - row tiles sized
+  // 65..128 tokens on a gate_up-sized matrix: the weight-streaming kernel with 128-token tiles - row tiles sized
   // to the CU count (244 workgroups instead of 152), same per-element K order as every un-split tiled kernel.  kind 3000 + RT.
   if (T <= 128 && so.silu_c1 == 0 && stream_gemm_on()) {
     const StreamPlan sp = stream_plan(M, so.silu_I > 0 ? so.silu_I : 0);
@@ -839,13 +842,14 @@ static void glds_gemm_launch(const Half* W, const Half* X, Half* Y, int M, int T
       gemm256_launch(W, X, Y, M, T, K, head, s);
       // the thin tail: 128-token tiles with a 2-deep ring (192 workgroups at 1024 tokens), or - PEGAINFER_GEMM256_TAIL_TT=64, A/B
       // knob - 64-token tiles with a 3-deep ring (384 workgroups, two per CU, all resident)
-      // (round 6, same-box A/B profiles/r6_reduce_and_tail_ttft.txt: TTFT(1024) 10.53 -> 10.33 ms, TTFT(2048) 18.25 -> 18.40):
+      // (same-box A/B profiles/r6_reduce_and_tail_ttft.txt: TTFT(1024) 10.53 -> 10.33 ms, TTFT(2048) 18.25 -> 18.40):
       // 64-token tiles exactly when the 128-token tiling would give the tail fewer tiles than there are CUs
       static const int tail_env = [] { const char* e = getenv("PEGAINFER_GEMM256_TAIL_TT"); return e && *e ? atoi(e) : 0; }();
       const long tail_tiles128 = (long)ceil_div(so.silu_I - r.m_head * 128, 64) * ceil_div(T, 128);
-      // (round 6, profiles/r6_tail_feeder_ab.txt) the feeder form of the 128 x 256 kernel takes the tail: (64 + 64)-row SwiGLU
-      // tiles (tail_tt 4), or (32 + 32)-row ones (tail_tt 2) while those still fit one round - TTFT(1024) 9.99 -> 9.76 ms (192
-      // tiles of 64 rows), TTFT(2048) 17.82 -> 17.24 (192 tiles of 128 rows); 64 / 128 = the round-5 kernels, kept for the A/B
+      // the feeder form of the 128 x 256 kernel takes the tail: (64 + 64)-row SwiGLU
+      // tiles (tail_tt 4), or (32 + 32)-row ones (tail_tt 2) while those still fit one round; 64 / 128 = the 128-row kernel's tiles, kept for the A/B.
+      // Head and tail, whole / tail 2 / 4 / 64 / 128 (us, cold weights): 9728 x 2560 and 1024 tokens 124 / 111 / 117 / 116 / 119, 2048 191 / 196 / 179 / 194 / 187, 5362
+      // 441 / 435 / 437 / 431 / 442; 9216 x 2560 and 1023 122 / 98 / 106 / 94 / 109, 6144 x 2048 and 1500 96 / 81 / 87 / 81 / 91
       const long tail_tiles4 = (long)ceil_div(so.silu_I - r.m_head * 128, 64) * ceil_div(T, G256_BT);
       const int tail_feeder = !gemm128x256_on() || !gemm128x256_feed_on() ? 0 : tail_tiles4 * 2 <= device_cus() ? 2 : 4;
       const int tail_tt = tail_env ? tail_env : tail_feeder ? tail_feeder : (tail_tiles128 < device_cus() ? 64 : 128);
@@ -868,7 +872,7 @@ static void glds_gemm_launch(const Half* W, const Half* X, Half* Y, int M, int T
     if (r.kind == 1283) { gemm96x256_launch(W, X, Y, M, T, K, so, s); return; }
     if (r.kind == 1280 || r.kind == 1281) { gemm128x256_launch(W, X, Y, M, T, K, so, nullptr, 1, 0, s); return; }
     // the plan said a 128-token stream tile exists; should a future plan / route change make the launcher refuse, fall
-    // through to the 128-row kernel (same per-element K order) instead of leaving Y unwritten (ADVICE r4)
+    // through to the 128-row kernel (same per-element K order) instead of leaving Y unwritten
     if (r.kind >= 3000 && stream_gemm_launch<128>(W, X, Y, M, T, K, so, s)) return;
     variant = r.kind >= 3000 ? 23 : r.kind;
   }
@@ -898,7 +902,7 @@ constexpr int kMidBatchMinRows = 5120;
 // 17..64 columns, plain (optionally row-segmented) output: 1 = tiled LDS-DMA GEMM, 2 = its split-K form, 0 = not
 // taken (skinny kernel / separate calls).  One decision for gemm_cuda, pegainfer_gemm_split and pegainfer_gemm_silu,
 // so that a stacked launch and the plain launch over the same matrix always run the same kernel.
-// 3 = the weight-streaming kernel of gemm_stream.h (round 4): row tiles sized to the CU count, full K per workgroup, feeder
+// 3 = the weight-streaming kernel of gemm_stream.h: row tiles sized to the CU count, full K per workgroup, feeder
 // waves.  Taken for tiles of >= 2 row blocks: gate_up 28.9 -> 21.8 us at 32 columns, 28.9 -> 24.1 at 64 (same bits as the
 // 128-row kernel); the stacked qkv matrix (32-row tiles, 192 workgroups) 13.8 -> 12.6 / 16.8 -> 13.7 us against its split-K
 // pair.  o_proj / down_proj (16-row tiles) keep the split-K route: with full K per workgroup they pull 0.5-1.2 MB of x per CU
